@@ -62,7 +62,12 @@ struct gh_ctx {
   // set while gh_submit_noalloc runs: the scratch is the library's fixed array and a
   // plan may not shrink to fit it (results must not depend on the scratch size)
   bool ws_strict = false;
-  bool sync_spin = false;  // gh_sync polls the stream instead of blocking in the runtime
+  // gh_sync's completion word: pinned host memory the stream writes `done_seq` to (gh_api.hip)
+  uint32_t* done_word = nullptr;
+  uint32_t done_seq = 0;
+  bool idle = true;         // nothing has been put on the stream since the last completed gh_sync
+  bool runtime_wait = false;  // a copy to or from pageable memory is under way: the runtime has its own part in finishing it
+  bool sync_block = false;  // gh_sync waits in the runtime only
   gh_llc_model llc;
   // pinned host buffers handed out by gh_host_alloc: [start, end)
   std::vector<std::pair<uint64_t, uint64_t>> host_ranges;
