@@ -87,6 +87,13 @@ int gh_check_hip(gh_ctx* ctx, hipError_t e, const char* what);
 // validated command.  Each returns GH_OK or a code with `msg` filled in.
 int gh_validate_cmd(const gh_cmd& c, std::string& msg);
 
+// whether the last-level cache has lost the buffer at p; whether a streaming kernel that moves `bytes`, all its
+// inputs lost (`cold`) or not, goes past the cache (k_elem.hip)
+bool gh_llc_cold(const gh_ctx* ctx, uint64_t p);
+bool gh_llc_stream(int64_t bytes, bool cold);
+// a run of elementwise commands in one pass (k_chain.hip): how many commands at the front of cmds (0 or >= 2), and the launch
+int gh_chain_length(const gh_cmd* cmds, int n);
+int gh_launch_chain(gh_ctx* ctx, const gh_cmd* cmds, int count);
 int gh_launch_elem_bin(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_elem_unary(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_bcast_bin(gh_ctx* ctx, const gh_cmd& c);
