@@ -166,7 +166,15 @@ class Tensor:
         return Tensor(self.mem, self.shape[::-1], self.dtype, not self.transposed, self.managed,
                       col_major=self.col_major)
 
+    def __setattr__(self, name, value):
+        object.__setattr__(self, name, value)
+        object.__setattr__(self, "_desc", None)   # built again for the next call
+
     def desc(self):
+        """The descriptor the library takes, kept until an attribute changes."""
+        d = self._desc
+        if d is not None:
+            return d
         d = GhhTensor()
         d.mem = self.mem
         d.dtype = DTYPES.get(self.dtype, 2)
@@ -175,7 +183,15 @@ class Tensor:
             d.shape[i] = s
         d.flags = ((0 if self.managed else T_NOT_MANAGED) | (T_TRANSPOSED if self.transposed else 0) |
                    (T_NEEDS_ITER if self.needs_iterator else 0) | (T_COL_MAJOR if self.col_major else 0))
+        object.__setattr__(self, "_desc", d)
+        object.__setattr__(self, "_ref", C.byref(d))
         return d
+
+    def ref(self):
+        """The descriptor as an argument of a call."""
+        if self._desc is None:
+            self.desc()
+        return self._ref
 
 
 BIN_FN = dict(_ffi.BIN_FN)
@@ -285,56 +301,52 @@ class Engine:
         n = int(np.prod(shape)) if len(shape) else 1
         return Tensor(self.Get(max(n * dtype.itemsize, 1)), shape, dtype)
 
-    # arith / cmp
-    def _binop(self, fn, a, b, reuse=None, unsafe=False, incr=False):
-        ret = C.c_uint64()
-        r = C.byref(reuse.desc()) if reuse is not None else None
-        self._check(self.lib.ghh_engine_binop(self.h, BIN_FN[fn], C.byref(a.desc()), C.byref(b.desc()), r,
-                                              0 if unsafe else 1, int(incr), C.byref(ret)))
-        return reuse if reuse is not None else a
-
-    def _binop_scalar(self, fn, a, b_mem, leftTensor, reuse=None, unsafe=False):
-        ret = C.c_uint64()
-        r = C.byref(reuse.desc()) if reuse is not None else None
-        b = b_mem.mem if isinstance(b_mem, Tensor) else (0 if b_mem is None else int(b_mem))
-        self._check(self.lib.ghh_engine_binop_scalar(self.h, BIN_FN[fn], C.byref(a.desc()), b,
-                                                     int(leftTensor), r, 0 if unsafe else 1, C.byref(ret)))
-        return reuse if reuse is not None else a
-
+    # arith / cmp: the methods made by _mk below
     def Unary(self, op_name, a, dst=None):
-        self._check(self.lib.ghh_engine_unary(self.h, op_name.encode(), C.byref(a.desc()),
+        self._check(self.lib.ghh_engine_unary(self.h, op_name.encode(), a.ref(),
                                               dst.mem if dst is not None else 0))
         return dst if dst is not None else a
 
     def MatMul(self, a, b, prealloc):
-        self._check(self.lib.ghh_engine_matmul(self.h, C.byref(a.desc()), C.byref(b.desc()),
-                                               C.byref(prealloc.desc())))
+        self._check(self.lib.ghh_engine_matmul(self.h, a.ref(), b.ref(),
+                                               prealloc.ref()))
 
     def MatVecMul(self, a, b, prealloc):
-        self._check(self.lib.ghh_engine_matvecmul(self.h, C.byref(a.desc()), C.byref(b.desc()),
-                                                  C.byref(prealloc.desc())))
+        self._check(self.lib.ghh_engine_matvecmul(self.h, a.ref(), b.ref(),
+                                                  prealloc.ref()))
 
     def Outer(self, a, b, prealloc):
-        self._check(self.lib.ghh_engine_outer(self.h, C.byref(a.desc()), C.byref(b.desc()),
-                                              C.byref(prealloc.desc())))
+        self._check(self.lib.ghh_engine_outer(self.h, a.ref(), b.ref(),
+                                              prealloc.ref()))
 
     def HasNaN(self, a):
         out = C.c_int()
-        self._check(self.lib.ghh_engine_has_nan(self.h, C.byref(a.desc()), C.byref(out)))
+        self._check(self.lib.ghh_engine_has_nan(self.h, a.ref(), C.byref(out)))
         return bool(out.value)
 
     def HasInf(self, a):
         out = C.c_int()
-        self._check(self.lib.ghh_engine_has_inf(self.h, C.byref(a.desc()), C.byref(out)))
+        self._check(self.lib.ghh_engine_has_inf(self.h, a.ref(), C.byref(out)))
         return bool(out.value)
 
 
 def _mk(fn):
+    code = BIN_FN[fn]
+
     def tt(self, a, b, reuse=None, unsafe=False, incr=False):
-        return self._binop(fn, a, b, reuse, unsafe, incr)
+        rc = self.lib.ghh_engine_binop(self.h, code, a.ref(), b.ref(), None if reuse is None else reuse.ref(),
+                                       0 if unsafe else 1, int(incr), None)
+        if rc:
+            self._check(rc)
+        return a if reuse is None else reuse
 
     def ts(self, a, b, leftTensor, reuse=None, unsafe=False):
-        return self._binop_scalar(fn, a, b, leftTensor, reuse, unsafe)
+        b_mem = b.mem if isinstance(b, Tensor) else (0 if b is None else int(b))
+        rc = self.lib.ghh_engine_binop_scalar(self.h, code, a.ref(), b_mem, int(leftTensor), None if reuse is None else reuse.ref(),
+                                              0 if unsafe else 1, None)
+        if rc:
+            self._check(rc)
+        return a if reuse is None else reuse
     return tt, ts
 
 

@@ -17,6 +17,10 @@ from .engine import Engine, EngineError, GhhOp, load_host
  K_BN_DIFF, K_SOFTMAX_DIFF, K_SET, K_SOLVER, K_RAND_UNIFORM, K_DROPOUT, K_DROPOUT_DIFF, K_RECTIFY_DIFF) = range(26)
 
 
+def _address(array):
+    return array.__array_interface__["data"][0]
+
+
 class Node:
     def __init__(self, g, nid):
         self.g, self.id = g, nid
@@ -36,7 +40,8 @@ class ExprGraph:
     def __init__(self):
         self.lib = load_host()
         self.h = self.lib.ghh_graph_new()
-        self._keep = []  # host arrays bound to nodes must outlive the graph
+        self._keep = []   # host arrays the graph writes into must outlive it
+        self._bound = {}  # node -> the host array it reads, kept until the node is bound to another
 
     def __del__(self):
         if getattr(self, "h", None):
@@ -80,13 +85,12 @@ def NewTensor(g, value, resident=False):
     value = np.asarray(value)
     if value.ndim:  # ascontiguousarray would turn a 0-d scalar into shape (1,)
         value = np.ascontiguousarray(value)
-    g._keep.append(value)
     shp = (C.c_int64 * max(value.ndim, 1))(*value.shape)
     dt = {np.dtype(np.float32): 0, np.dtype(np.float64): 1}.get(value.dtype, 2)
-    nid = g.lib.ghh_graph_new_tensor(g.h, shp, value.ndim, dt, value.ctypes.data_as(C.c_void_p),
-                                     int(resident))
+    nid = g.lib.ghh_graph_new_tensor(g.h, shp, value.ndim, dt, _address(value), int(resident))
     if nid < 0:
         raise EngineError(_ffi.GH_EINVAL, g.lib.ghh_graph_last_error(g.h).decode(errors="replace"))
+    g._bound[nid] = value
     node = Node(g, nid)
     node.dtype = value.dtype
     return node
@@ -98,8 +102,9 @@ def NewScalar(g, value, dtype=np.float32, resident=True):
 
 def Let(node, value):
     value = np.ascontiguousarray(value)
-    node.g._keep.append(value)
-    node.g._check(node.g.lib.ghh_graph_let(node.g.h, node.id, value.ctypes.data_as(C.c_void_p)))
+    g = node.g
+    g._check(g.lib.ghh_graph_let(g.h, node.id, _address(value)))
+    g._bound[node.id] = value
 
 
 def Read(node, dtype=None):

@@ -5,6 +5,7 @@
 namespace gorgonia {
 
 void BFC::reserve(uint64_t start, int64_t size) {
+  stamp_++;
   start_ = start;
   size_ = size - (size % block_size_);
   reserved_size_ = size;
@@ -12,6 +13,7 @@ void BFC::reserve(uint64_t start, int64_t size) {
 }
 
 uint64_t BFC::release() {
+  stamp_++;
   uint64_t r = start_;
   start_ = 0;
   size_ = 0;
@@ -51,6 +53,7 @@ void BFC::insert(uint64_t off, int64_t size) {
 }
 
 int BFC::alloc(int64_t size, uint64_t* addr, OomError* oom) {
+  stamp_++;
   if (size <= 0) return 1;  // "Cannot allocate memory with size 0 or less"
   const int64_t aligned = align(size);
   auto fit = [&]() {
@@ -80,6 +83,7 @@ int BFC::alloc(int64_t size, uint64_t* addr, OomError* oom) {
 }
 
 void BFC::free(uint64_t address) {
+  stamp_++;
   const uint64_t off = address - start_;
   auto it = used_.find(off);
   if (it == used_.end()) return;  // unknown address: silently ignored

@@ -61,6 +61,8 @@ class BFC {
   int used_count() const { return (int)used_.size(); }
   int allocs() const { return allocs_; }
   int frees() const { return frees_; }
+  // changes with every call that moves memory between free and used: equal stamps, equal arena
+  uint64_t stamp() const { return stamp_; }
 
  private:
   void insert(uint64_t off, int64_t size);
@@ -73,6 +75,7 @@ class BFC {
   int64_t allocated_ = 0;
   int allocs_ = 0;
   int frees_ = 0;
+  uint64_t stamp_ = 0;
 };
 
 }  // namespace gorgonia

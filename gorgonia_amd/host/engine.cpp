@@ -217,15 +217,19 @@ static Status handleFuncOpts(const Shape& expShape, Dtype expType, const FuncOpt
   return Status::OK();
 }
 
-static std::string binName(const char* fn, int mode, Dtype dt) {
+static const char* kFnNames[GH_BINFN__COUNT] = {"add", "sub", "mul", "div", "pow", "lt",
+                                                "lte", "gt",  "gte", "eq",  "ne",  "mod"};
+
+static std::string binName(int fn, int mode, Dtype dt) {
   static const char* modes[4] = {"vv", "vs", "sv", "ss"};
   char buf[96];
-  snprintf(buf, sizeof(buf), "elembinop.%s_%s_f%d", fn, modes[mode], (int)dtype_size(dt) * 8);
+  snprintf(buf, sizeof(buf), "elembinop.%s_%s_f%d", fn >= 0 && fn < GH_BINFN__COUNT ? kFnNames[fn] : "?", modes[mode], (int)dtype_size(dt) * 8);
   return buf;
 }
 
-static const char* kFnNames[GH_BINFN__COUNT] = {"add", "sub", "mul", "div", "pow", "lt",
-                                                "lte", "gt",  "gte", "eq",  "ne",  "mod"};
+// HasFunc(binName(...)) without spelling the name on every call: every function exists in every mode and both
+// float types (the Dtype is checked behind it).
+static bool hasBin(int fn) { return fn >= 0 && fn < GH_BINFN__COUNT; }
 
 // Destination selection shared by all arithmetic methods (cuda/arith.go:34-49):
 // with a reuse tensor the result lands there and a is left alone (the
@@ -257,10 +261,10 @@ Status Engine::prepBinary(const char* go_name, Tensor& a, const FuncOpts& o, uin
 Status Engine::BinOp(int fn, const char* go_name, Tensor& a, Tensor& b, const FuncOpts& o, Tensor** ret) {
   const int mode = a.shape.IsScalar() ? (b.shape.IsScalar() ? GH_SS : GH_SV)
                                       : (b.shape.IsScalar() ? GH_VS : GH_VV);  // constructName2
-  const std::string name = binName(kFnNames[fn], mode, a.dt);
-  if (!HasFunc(name))
+  if (!hasBin(fn))
     return Status::Err(GH_ENOFUNC, std::string("Unable to perform ") + go_name +
-                                       "(). The tensor engine does not have the function \"" + name + "\"");
+                                       "(). The tensor engine does not have the function \"" +
+                                       binName(fn, mode, a.dt) + "\"");
   Status st = binaryCheck(a, b);
   if (!st.ok()) return st.Wrap(std::string("Basic checks failed for ") + go_name);
   uint64_t mem; int64_t size;
@@ -277,10 +281,10 @@ Status Engine::BinOp(int fn, const char* go_name, Tensor& a, Tensor& b, const Fu
 Status Engine::BinOpScalar(int fn, const char* go_name, Tensor& a, uint64_t b_mem, bool left_tensor,
                            const FuncOpts& o, Tensor** ret) {
   const int mode = left_tensor ? GH_VS : GH_SV;  // constructName1
-  const std::string name = binName(kFnNames[fn], mode, a.dt);
-  if (!HasFunc(name))
+  if (!hasBin(fn))
     return Status::Err(GH_ENOFUNC, std::string("Unable to perform ") + go_name +
-                                       "(). The tensor engine does not have the function \"" + name + "\"");
+                                       "(). The tensor engine does not have the function \"" +
+                                       binName(fn, mode, a.dt) + "\"");
   if (!b_mem) return Status::Err(GH_EINVAL, "b has to be a tensor.Memory. Got <nil> instead");
   Status st = unaryCheck(a);
   if (!st.ok()) return st.Wrap(std::string("Basic checks failed for ") + go_name);

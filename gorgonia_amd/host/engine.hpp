@@ -177,6 +177,7 @@ class Engine {
   size_t PendingCommands() const { return segment_.size(); }
   const std::vector<gh_cmd>& Segment() const { return segment_; }
   void DropSegment() { segment_.clear(); }
+  void SetSegment(const std::vector<gh_cmd>& cmds) { segment_ = cmds; }
   int64_t SubmitCalls() const { return submit_calls_; }  // C-ABI crossings made by DoWork
   Status SubmitPending();                 // gh_submit of the segment, no wait
   Status Sync();                          // wait only

@@ -20,6 +20,10 @@ static constexpr int64_t kStageInTotal = 512ll << 20; // per machine
 static constexpr int64_t kPipelinedUpload = 4 << 20;
 static constexpr int64_t kUploadPiece = 2 << 20;
 
+// inputs up to this size are read where the host wrote them, in pinned memory: the copy kernel a few KB would
+// need costs 4 us on the device, an operand read over the bus about 1
+static constexpr int64_t kReadInPlace = 8 << 10;
+
 static Status bad(const std::string& m) { return Status::Err(GH_EINVAL, m); }
 
 static int64_t conv_out(int64_t in, int64_t k, int64_t pad, int64_t stride, int64_t dil) {
@@ -693,12 +697,12 @@ int Graph::FuseActivations() {
     if (n.is_input || n.fused_away || n.inputs.empty()) continue;
     const OpKind k = n.op.kind;
     if (k != OpKind::Rectify && k != OpKind::LeakyRelu && k != OpKind::BatchNorm && k != OpKind::MaxPool2D &&
-        k != OpKind::SoftMax && !(k == OpKind::BroadcastBin && n.op.fn == GH_ADD))
+        k != OpKind::SoftMax && !((k == OpKind::BroadcastBin || k == OpKind::ElemBin) && n.op.fn == GH_ADD))
       continue;
+    const bool add = k == OpKind::BroadcastBin || k == OpKind::ElemBin;
     // the producer: the first input, or for a broadcast add whichever input is the product
     int pi = n.inputs[0];
-    if (k == OpKind::BroadcastBin && n.inputs.size() == 2 && nodes_[(size_t)n.inputs[1]].op.kind == OpKind::MatMul &&
-        !nodes_[(size_t)n.inputs[1]].is_input)
+    if (add && n.inputs.size() == 2 && nodes_[(size_t)n.inputs[1]].op.kind == OpKind::MatMul && !nodes_[(size_t)n.inputs[1]].is_input)
       pi = n.inputs[1];
     Node& p = nodes_[(size_t)pi];
     if (p.is_input || p.fused_away || p.read_into || uses[(size_t)p.id] != 1) continue;
@@ -708,13 +712,14 @@ int Graph::FuseActivations() {
     std::vector<int> inputs = p.inputs;
     const bool has_act = op.fuse_act_relu || op.fuse_act_leaky;
     if (op.fuse_softmax) continue;   // nothing rides behind a softmax
-    if (k == OpKind::BroadcastBin) {
-      // Add(Mul(x, w), b) with b one value per column: a + b and b + a are the same bits
+    if (add) {
+      // Add(Mul(x, w), b) with b one value per column: a + b and b + a are the same bits.  For a single row
+      // that is the plain Add of two rows.
       if (op.kind != OpKind::MatMul || has_act || op.fuse_bias || n.inputs.size() != 2 || n.shape.Dims() != 2) continue;
       if (op.transA || op.transB) continue;   // the bias epilogue exists for untransposed products
       const Node& small = nodes_[(size_t)(pi == n.inputs[0] ? n.inputs[1] : n.inputs[0])];
       if (small.dt != Dtype::Float32 || small.shape.Dims() != 2 || small.shape[0] != 1 || small.shape[1] != n.shape[1] ||
-          n.shape[0] == 1)
+          small.id == pi)
         continue;
       op.fuse_bias = true;
       inputs.push_back(small.id);
@@ -986,6 +991,11 @@ Status TapeMachine::Compile() {
   }
   regs_.assign((size_t)nreg, Tensor());
   reg_live_.assign((size_t)nreg, 0);
+  reg_arena_.assign((size_t)nreg, 0);
+  in_pieces_.assign((size_t)N, 0);
+  lent_.assign((size_t)N, 0);
+  recorded_.clear();
+  steady_ = false;
   resident_done_.assign((size_t)N, 0);
   reg_bytes_.assign((size_t)nreg, 0);
   std::vector<int64_t>& reg_bytes = reg_bytes_;
@@ -1209,6 +1219,97 @@ Status TapeMachine::flush() {
   return eager();
 }
 
+Status TapeMachine::upload(const Instr& in, bool record) {
+  Node& n = g_->Nodes()[(size_t)in.node];
+  uint64_t& mem = regs_[(size_t)in.reg].mem;
+  if (void* pinned = stage_in_[(size_t)in.node]) {
+    // host value -> pinned buffer now, pinned buffer -> register as a command of
+    // the segment: the upload is captured and replayed with the operators
+    if (record) {
+      lent_[(size_t)in.node] = n.host_borrowed;
+      in_pieces_[(size_t)in.node] = !n.host_borrowed && in.size >= kPipelinedUpload && eng_.Segment().empty();
+    }
+    if (in_pieces_[(size_t)in.node] && !n.host_borrowed) {
+      // a large value at the front of its segment: piece by piece, the host copy of one
+      // piece runs while the copy engine moves the piece before it (stream order puts the
+      // segment's operators behind the last piece)
+      const char* src = static_cast<const char*>(n.host);
+      char* stg = static_cast<char*>(pinned);
+      for (int64_t off = 0; off < in.size; off += kUploadPiece) {
+        const int64_t len = std::min(kUploadPiece, in.size - off);
+        std::memcpy(stg + off, src + off, (size_t)len);
+        Status st = eng_.MemcpyHtoD(mem + (uint64_t)off, stg + off, len);
+        if (!st.ok()) return st;
+      }
+      return Status::OK();
+    }
+    if (!n.host_borrowed) std::memcpy(pinned, n.host, (size_t)in.size);
+    if (!record) return Status::OK();
+    const uint64_t arena = reg_memory((size_t)in.reg);
+    // (not a lent buffer: an operator may overwrite its input's register)
+    if (in.size <= kReadInPlace && !n.host_borrowed) {
+      reg_arena_[(size_t)in.reg] = arena;
+      mem = (uint64_t)(uintptr_t)pinned;
+    } else {
+      mem = arena;
+      eng_.RecordCopy(mem, (uint64_t)(uintptr_t)pinned, in.size);
+    }
+    return Status::OK();
+  }
+  // a borrowed input has no host value of its own (Node::host is a marker): without the machine's
+  // pinned buffer - LetBorrowed after Init, on an input this machine does not stage - there is
+  // nothing to upload
+  if (n.host_borrowed)
+    return Status::Err(GH_ESTATE, "input " + std::to_string(in.node) +
+                                      " was lent (LetBorrowed) but this machine holds no pinned buffer for it; "
+                                      "lend inputs before the machine is created");
+  return eng_.MemcpyHtoD(mem, n.host, in.size);
+}
+
+Status TapeMachine::read(const Instr& in, bool last) {
+  Node& n = g_->Nodes()[(size_t)in.node];
+  if (in.node < (int)stage_.size() && stage_[(size_t)in.node]) {
+    // the flush in front of the reads has waited for the staging copy; a borrowed
+    // read is finished with that
+    if (!n.read_borrowed) std::memcpy(n.read_into, stage_[(size_t)in.node], (size_t)in.size);
+    for (void* more : n.read_also) std::memcpy(more, stage_[(size_t)in.node], (size_t)in.size);
+    return Status::OK();
+  }
+  Status st = eng_.MemcpyDtoH(n.read_into, regs_[(size_t)in.reg].mem, in.size, false);
+  for (void* more : n.read_also)
+    if (st.ok()) st = eng_.MemcpyDtoH(more, regs_[(size_t)in.reg].mem, in.size, false);
+  if (!st.ok()) return st;
+  return last ? eng_.Sync() : Status::OK();
+}
+
+// A run of a settled machine: the commands are the recorded ones, because the program is fixed and the arena
+// hands out the same addresses again.  What is left of a run is to bring the inputs, submit (or replay), wait,
+// and hand the outputs over; walking the program, the arena and the operators' checks took 1-2 us of host time
+// per operator, which a network of small layers cannot hide.
+Status TapeMachine::run_steady() {
+  auto& nodes = g_->Nodes();
+  for (size_t pc = 0; pc < prog_.size(); pc++) {
+    const Instr& in = prog_[pc];
+    Status st;
+    if (in.kind == InstrKind::LoadArg && !nodes[(size_t)in.node].host)
+      return Status::Err(GH_EINVAL, "PC " + std::to_string(pc) + ": input node " + std::to_string(in.node) + " has no value bound");
+    if (in.kind == InstrKind::Transport && (!nodes[(size_t)in.node].resident || opt_.reupload_resident)) {
+      st = upload(in, false);
+      if (!st.ok()) return st.Wrap("PC " + std::to_string(pc) + ": devTrans");
+    }
+    if (in.kind == InstrKind::Flush) {
+      eng_.SetSegment(recorded_);
+      st = flush();
+      if (!st.ok()) return st.Wrap("PC " + std::to_string(pc) + ": flush");
+    }
+    if (in.kind == InstrKind::Read) {
+      st = read(in, pc + 1 >= prog_.size() || prog_[pc + 1].kind != InstrKind::Read);
+      if (!st.ok()) return st.Wrap("PC " + std::to_string(pc) + ": read");
+    }
+  }
+  return Status::OK();
+}
+
 Status TapeMachine::RunAll() {
   if (!eng_.Initialized()) return Status::Err(GH_ESTATE, "tape machine not initialised");
   auto& nodes = g_->Nodes();
@@ -1216,6 +1317,20 @@ Status TapeMachine::RunAll() {
   seg_index_ = 0;
   const int64_t t_run = now_ns();
   ns_launch_ = ns_wait_ = 0;
+  const bool watched = opt_.watch_nan || opt_.watch_inf;
+  for (const Instr& in : prog_)   // lent where it was bound before, or the other way round
+    if (in.kind == InstrKind::Transport && (bool)lent_[(size_t)in.node] != nodes[(size_t)in.node].host_borrowed) steady_ = false;
+  if (steady_ && !watched && arena_stamp_ == eng_.Allocator().stamp() && eng_.Segment().empty()) {
+    Status st = run_steady();
+    if (!st.ok()) steady_ = false;
+    runs_++;
+    ns_total_ = now_ns() - t_run;
+    return st;
+  }
+  steady_ = false;
+  bool settled = false;
+  const bool undisturbed = arena_stamp_ == eng_.Allocator().stamp();
+  const int64_t calls = eng_.SubmitCalls();
   for (size_t pc = 0; pc < prog_.size(); pc++) {
     const Instr& in = prog_[pc];
     Status st;
@@ -1231,47 +1346,16 @@ Status TapeMachine::RunAll() {
           st = eng_.Get(in.size, &mem);
           if (!st.ok()) return st.Wrap("PC " + std::to_string(pc) + ": alloc");
           regs_[(size_t)in.reg].mem = mem;
+          reg_arena_[(size_t)in.reg] = 0;
           reg_live_[(size_t)in.reg] = 1;
         }
         break;
-      case InstrKind::Transport: {
-        Node& n = nodes[(size_t)in.node];
-        if (n.resident && resident_done_[(size_t)in.node] && !opt_.reupload_resident) break;
-        if (void* pinned = stage_in_[(size_t)in.node]) {
-          // host value -> pinned buffer now, pinned buffer -> register as a command of
-          // the segment: the upload is captured and replayed with the operators
-          if (!n.host_borrowed && in.size >= kPipelinedUpload && eng_.Segment().empty()) {
-            // a large value at the front of its segment: piece by piece, the host copy of one
-            // piece runs while the copy engine moves the piece before it (stream order puts the
-            // segment's operators behind the last piece)
-            const char* src = static_cast<const char*>(n.host);
-            char* stg = static_cast<char*>(pinned);
-            for (int64_t off = 0; off < in.size; off += kUploadPiece) {
-              const int64_t len = std::min(kUploadPiece, in.size - off);
-              std::memcpy(stg + off, src + off, (size_t)len);
-              st = eng_.MemcpyHtoD(regs_[(size_t)in.reg].mem + (uint64_t)off, stg + off, len);
-              if (!st.ok()) return st.Wrap("PC " + std::to_string(pc) + ": devTrans");
-            }
-            resident_done_[(size_t)in.node] = 1;
-            break;
-          }
-          if (!n.host_borrowed) std::memcpy(pinned, n.host, (size_t)in.size);
-          eng_.RecordCopy(regs_[(size_t)in.reg].mem, (uint64_t)(uintptr_t)pinned, in.size);
-          resident_done_[(size_t)in.node] = 1;
-          break;
-        }
-        // a borrowed input has no host value of its own (Node::host is a marker): without the machine's
-        // pinned buffer - LetBorrowed after Init, on an input this machine does not stage - there is
-        // nothing to upload
-        if (n.host_borrowed)
-          return Status::Err(GH_ESTATE, "PC " + std::to_string(pc) + ": devTrans: input " + std::to_string(in.node) +
-                                            " was lent (LetBorrowed) but this machine holds no pinned buffer for it; "
-                                            "lend inputs before the machine is created");
-        st = eng_.MemcpyHtoD(regs_[(size_t)in.reg].mem, n.host, in.size);
+      case InstrKind::Transport:
+        if (nodes[(size_t)in.node].resident && resident_done_[(size_t)in.node] && !opt_.reupload_resident) break;
+        st = upload(in, true);
         if (!st.ok()) return st.Wrap("PC " + std::to_string(pc) + ": devTrans");
         resident_done_[(size_t)in.node] = 1;
         break;
-      }
       case InstrKind::ExecOp: {
         Node& n = nodes[(size_t)in.node];
         Tensor out;
@@ -1317,11 +1401,20 @@ Status TapeMachine::RunAll() {
       }
       case InstrKind::Free:
         if (reg_live_[(size_t)in.reg]) {
-          eng_.Put(regs_[(size_t)in.reg].mem, in.size);
+          eng_.Put(reg_memory((size_t)in.reg), in.size);
           reg_live_[(size_t)in.reg] = 0;
         }
         break;
       case InstrKind::Flush:
+        // nothing was submitted in front of it (but pieces of an upload): the run is this one segment
+        if (eng_.SubmitCalls() == calls && !watched && !opt_.node_at_a_time) {
+          const std::vector<gh_cmd>& cur = eng_.Segment();
+          settled = cur.size() == recorded_.size() &&
+                    (cur.empty() || std::memcmp(cur.data(), recorded_.data(), cur.size() * sizeof(gh_cmd)) == 0);
+          if (!settled) recorded_ = cur;
+        } else {
+          recorded_.clear();
+        }
         st = flush();
         if (!st.ok()) return st.Wrap("PC " + std::to_string(pc) + ": flush");
         break;
@@ -1331,26 +1424,10 @@ Status TapeMachine::RunAll() {
       case InstrKind::StageOut:
         eng_.RecordCopy((uint64_t)(uintptr_t)stage_[(size_t)in.node], regs_[(size_t)in.reg].mem, in.size);
         break;
-      case InstrKind::Read: {
-        Node& n = nodes[(size_t)in.node];
-        if (in.node < (int)stage_.size() && stage_[(size_t)in.node]) {
-          // the flush in front of the reads has waited for the staging copy; a borrowed
-          // read is finished with that
-          if (!n.read_borrowed) std::memcpy(n.read_into, stage_[(size_t)in.node], (size_t)in.size);
-          for (void* more : n.read_also) std::memcpy(more, stage_[(size_t)in.node], (size_t)in.size);
-          break;
-        }
-        st = eng_.MemcpyDtoH(n.read_into, regs_[(size_t)in.reg].mem, in.size, false);
-        for (void* more : n.read_also)
-          if (st.ok()) st = eng_.MemcpyDtoH(more, regs_[(size_t)in.reg].mem, in.size, false);
+      case InstrKind::Read:
+        st = read(in, pc + 1 >= prog_.size() || prog_[pc + 1].kind != InstrKind::Read);
         if (!st.ok()) return st.Wrap("PC " + std::to_string(pc) + ": read");
-        bool last = pc + 1 >= prog_.size() || prog_[pc + 1].kind != InstrKind::Read;
-        if (last) {
-          st = eng_.Sync();
-          if (!st.ok()) return st;
-        }
         break;
-      }
     }
   }
   Status st = eng_.DoWork();  // final DoWork (vm_tape.go:236)
@@ -1361,6 +1438,9 @@ Status TapeMachine::RunAll() {
   // segment stays replayable.
   eng_.Allocator().coalesce();
   eng_.Allocator().reset_stats();
+  // the same commands in two runs, and no run of other users of the arena in between
+  steady_ = st.ok() && settled && undisturbed;
+  arena_stamp_ = eng_.Allocator().stamp();
   ns_total_ = now_ns() - t_run;
   return st;
 }
@@ -1378,7 +1458,7 @@ void TapeMachine::drop_graphs() {
 void TapeMachine::release_registers() {
   for (size_t r = 0; r < reg_live_.size(); r++)
     if (reg_live_[r]) {
-      eng_.Put(regs_[r].mem, reg_bytes_[r]);
+      eng_.Put(reg_memory(r), reg_bytes_[r]);
       reg_live_[r] = 0;
     }
 }
@@ -1390,6 +1470,8 @@ Status TapeMachine::Reset() {
   else eng_.ResetAllocator();
   std::fill(reg_live_.begin(), reg_live_.end(), 0);
   std::fill(resident_done_.begin(), resident_done_.end(), 0);
+  steady_ = false;
+  recorded_.clear();
   return Status::OK();
 }
 

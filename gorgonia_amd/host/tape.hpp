@@ -219,8 +219,12 @@ class TapeMachine {
 
  private:
   Status flush();
+  Status upload(const Instr& in, bool record);   // Transport of an input that is not on the device yet
+  Status read(const Instr& in, bool last);
+  Status run_steady();
   void drop_graphs();   // destroy every captured segment graph
   void release_registers();
+  uint64_t reg_memory(size_t r) const { return reg_arena_[r] ? reg_arena_[r] : regs_[r].mem; }
   Graph* g_;
   TapeOptions opt_;
   Engine own_;
@@ -254,6 +258,14 @@ class TapeMachine {
     enum { Measuring, Plain, Replay } verdict = Measuring;
   };
   std::vector<SegCache> seg_cache_;
+  // What the last run recorded, and whether the runs have settled: two runs in a row recorded the same commands
+  // and nobody has touched the arena since, so the next run would record them again (run_steady).
+  std::vector<gh_cmd> recorded_;
+  std::vector<char> in_pieces_;    // per node: the last run uploaded it piece by piece in front of the segment
+  std::vector<char> lent_;         // per node: it was a lent input then
+  bool steady_ = false;
+  uint64_t arena_stamp_ = 0;
+  std::vector<uint64_t> reg_arena_;   // the register's arena memory while regs_ points at a pinned input buffer
   int seg_index_ = 0;
 };
 
