@@ -1,0 +1,350 @@
+// Filter gradient of Conv2d 3x3 / stride 1, float32 and float64, on the 16x16x4 MFMA with every operand
+// taken from memory straight into the lane that feeds it.
+//
+// dW[f][c][ky][kx] is a sum over (image, output row, output column) of dy[f] * x[c] shifted by the tap: a small
+// result summed over a long axis.  Tiled through LDS (64 x 64 results per workgroup, im2col gathers) a network's
+// first layers leave most of a tile empty and their gathers, not the matrix cores, set the time.  Measured, slab sum
+// included, against the kernels that took these shapes before: 3 -> 16 channels over 8 x 208 x 208 pixels 17.6 us
+// (274), 16 -> 32 over 8 x 104 x 104 21.9 (75), 128 -> 256 over 8 x 52 x 52 170 (213: 75 against 60 TFLOP/s), float64
+// 32 -> 64 over 50 x 14 x 14 19.8 (29.8).  Small ones are bound by what surrounds the MFMAs (first loads 1 us,
+// meeting of the wavefronts 3, slab sum 5), large ones by address and edge arithmetic between them.  Here
+//   * a wavefront owns 16 TM filters x 16 channels and all nine taps (TM * 9 accumulators) and walks chunks of
+//     4 P consecutive output columns of one row.  Lane (i, q) of a chunk holds P consecutive columns: of dy row i
+//     one P-wide load, of channel i the P + 2 values under each of the three filter rows.  MFMA step t of the
+//     chunk takes element t of dy and element t + kx of x, so three loads feed nine taps and P steps, nothing
+//     is staged, and no barrier stands in the loop; the loads of a chunk are issued before the MFMAs of the
+//     chunk in front of it.
+//   * with fewer than 16 channels the columns of a tile are (channel, tap) pairs instead, packed without gaps,
+//     and each has its own P-wide load (kPacked).
+//   * the long axis is cut among wavefronts and workgroups; the four wavefronts of a workgroup meet in LDS, the
+//     workgroups' slabs in k_slab_sum, both in a fixed order.
+// P is 4, or 2 where a row has at most eight columns.
+#include <algorithm>
+
+#include "gh_internal.h"
+
+namespace {
+
+constexpr int kWaves = 4, kThreads = kWaves * 64;
+
+template <class T> struct Mfma;
+template <> struct Mfma<float> {
+  typedef float acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc run(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+  static __device__ __forceinline__ int row(int q, int v) { return 4 * q + v; }   // result row of register v in lanes q
+};
+template <> struct Mfma<double> {
+  typedef double acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc run(double a, double b, acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+  static __device__ __forceinline__ int row(int q, int v) { return 4 * v + q; }
+};
+
+template <class T>
+struct Wg {
+  const T* x;
+  const T* dy;
+  T* out;                       // [slices][F][C * 9]
+  int x_total, dy_total;        // elements
+  int B, C, H, W, F, oh, ow, padH, padW;
+  int nch;                      // chunks of a row
+  int items, per;               // chunks in all, and per wavefront
+};
+
+// Waits for this wavefront's loads.  The compiler counts the loads in flight where paths meet by the worst of
+// them, so a path that leaves some in flight makes the others wait for the next chunk's as well.
+__device__ __forceinline__ void loads_done() { __builtin_amdgcn_s_waitcnt(0x0F70); }   // vmcnt(0), the other counters free
+
+// N consecutive elements from p + off, moved into [0, total) where they stick out: branch-free, so that a chunk's
+// loads stay in flight behind the chunk in front.  fix_n puts the elements right.
+template <int N, class T>
+__device__ __forceinline__ void load_n(const T* __restrict__ p, int off, int total, T* v) {
+  typedef T V2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+  typedef T V4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  const unsigned at = (unsigned)min(max(off, 0), total - N);
+  if constexpr (N >= 4 && sizeof(T) == 4) {
+    const V4 a = *(const V4*)(p + at);
+#pragma unroll
+    for (int t = 0; t < 4; t++) v[t] = a[t];
+    if constexpr (N == 6) {
+      const V2 b = *(const V2*)(p + at + 4);
+      v[4] = b[0]; v[5] = b[1];
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < N; t += 2) {
+      const V2 a = *(const V2*)(p + at + t);
+      v[t] = a[0]; v[t + 1] = a[1];
+    }
+  }
+}
+// The elements of a load_n that was moved (the tensor's first and last few), one by one; those outside the tensor
+// are whatever is inside (the caller drops them).
+template <int N, class T>
+__device__ __forceinline__ void fix_n(const T* __restrict__ p, int off, int total, T* v) {
+  if (__any(off < 0 || off + N > total)) {
+#pragma unroll
+    for (int t = 0; t < N; t++) v[t] = p[(unsigned)min(max(off + t, 0), total - 1)];
+    loads_done();   // here, not at the values' first use: that is where every chunk would wait
+  }
+}
+
+template <class T, int TM, int P, int NT, bool kPacked>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_conv3x3_wgrad(const Wg<T> g) {
+  static_assert(kPacked || NT == 9, "a channel tile has nine taps");
+  typedef typename Mfma<T>::acc Acc;
+  constexpr int NB = kPacked ? NT * P : 3 * (P + 2);
+  struct Frag { T a[TM][P]; T b[NB]; };
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = lane & 15, q = lane >> 4;
+  const int f0 = blockIdx.z * 16 * TM, c0 = kPacked ? 0 : blockIdx.y * 16;
+  const int CKK = g.C * 9, last_image = g.B - 1;
+
+  // element offsets: of a lane's dy rows and of its columns' channels inside an image, in 32 bits
+  int f_at[TM];
+#pragma unroll
+  for (int m = 0; m < TM; m++) f_at[m] = min(f0 + 16 * m + i, g.F - 1) * g.oh * g.ow;
+  const int f_image = g.F * g.oh * g.ow, c_image = g.C * g.H * g.W;
+  constexpr int NC = kPacked ? NT : 1;
+  int c_at[NC], ky[NC], kx[NC];
+#pragma unroll
+  for (int n = 0; n < NC; n++) {
+    const int col = kPacked ? min(n * 16 + i, CKK - 1) : min(c0 + i, g.C - 1) * 9;
+    const int c = col / 9, tap = col - c * 9;
+    c_at[n] = c * g.H * g.W;
+    ky[n] = tap / 3;
+    kx[n] = tap - ky[n] * 3;
+  }
+  // where operand k of a chunk starts: k < TM is a dy row, then one per packed column or per filter row
+  constexpr int NX = kPacked ? NT : 3, XN = kPacked ? P : P + 2;
+  auto dy_off = [&](int m, int b, int oy, int ch) { return b * f_image + f_at[m] + oy * g.ow + (ch * 4 + q) * P; };
+  auto x_off = [&](int n, int b, int oy, int ch) {
+    const int iy = oy + (kPacked ? ky[kPacked ? n : 0] : n) - g.padH, ix = (ch * 4 + q) * P + (kPacked ? kx[kPacked ? n : 0] : 0) - g.padW;
+    return b * c_image + c_at[kPacked ? n : 0] + min(max(iy, 0), g.H - 1) * g.W + ix;
+  };
+  // The values as they lie in memory: what is outside the row or the image is dropped in front of the MFMAs
+  // (touching a value here would make the wavefront wait for it, and nothing would be in flight under the MFMAs).
+  auto load = [&](int b, int oy, int ch, Frag& f) {
+#pragma unroll
+    for (int m = 0; m < TM; m++) load_n<P>(g.dy, dy_off(m, b, oy, ch), g.dy_total, f.a[m]);
+#pragma unroll
+    for (int n = 0; n < NX; n++) load_n<XN>(g.x, x_off(n, b, oy, ch), g.x_total, f.b + n * XN);
+  };
+  Acc acc[TM][NT];
+#pragma unroll
+  for (int m = 0; m < TM; m++)
+#pragma unroll
+    for (int n = 0; n < NT; n++) acc[m][n] = Acc{(T)0, (T)0, (T)0, (T)0};
+  auto multiply = [&](int b, int oy, int ch, Frag& f) {
+    const int ox = (ch * 4 + q) * P;
+    if (b == 0 || b == last_image) {   // the only images with loads that stick out of the tensors
+#pragma unroll
+      for (int m = 0; m < TM; m++) fix_n<P>(g.dy, dy_off(m, b, oy, ch), g.dy_total, f.a[m]);
+#pragma unroll
+      for (int n = 0; n < NX; n++) fix_n<XN>(g.x, x_off(n, b, oy, ch), g.x_total, f.b + n * XN);
+    }
+    // a chunk whose every value is inside its row and image has nothing to drop
+    const int left = ch * 4 * P - g.padW, right = (ch + 1) * 4 * P + 2 - g.padW;
+    if (left < 0 || right > g.W || (ch + 1) * 4 * P > g.ow || oy < g.padH || oy + 3 - g.padH > g.H) {
+#pragma unroll
+      for (int m = 0; m < TM; m++)
+#pragma unroll
+        for (int t = 0; t < P; t++) f.a[m][t] = ox + t < g.ow ? f.a[m][t] : (T)0;
+      if constexpr (kPacked) {
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+          const int iy = oy + ky[n] - g.padH, ix = ox + kx[n] - g.padW;
+          const bool row = iy >= 0 && iy < g.H;
+#pragma unroll
+          for (int t = 0; t < P; t++) f.b[n * P + t] = row && ix + t >= 0 && ix + t < g.W ? f.b[n * P + t] : (T)0;
+        }
+      } else {
+        const int ix = ox - g.padW;
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+          const bool row = oy + r - g.padH >= 0 && oy + r - g.padH < g.H;
+#pragma unroll
+          for (int t = 0; t < P + 2; t++)
+            f.b[r * (P + 2) + t] = row && ix + t >= 0 && ix + t < g.W ? f.b[r * (P + 2) + t] : (T)0;
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < P; t++)
+#pragma unroll
+      for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int m = 0; m < TM; m++) {
+          const T bv = kPacked ? f.b[n * P + t] : f.b[(n / 3) * (P + 2) + t + n % 3];
+          acc[m][n] = Mfma<T>::run(f.a[m][t], bv, acc[m][n]);
+        }
+  };
+
+  const int first = (int)min((int64_t)(blockIdx.x * kWaves + wave) * g.per, (int64_t)g.items);
+  const int count = min(g.per, g.items - first);
+  if (count > 0) {
+    int ch = first % g.nch, row = first / g.nch;   // row of the batch
+    int b = row / g.oh, oy = row - b * g.oh;
+    auto next = [&]() {
+      if (++ch == g.nch) {
+        ch = 0;
+        if (++oy == g.oh) { oy = 0; b++; }
+      }
+    };
+    Frag cur, ahead;
+    load(b, oy, ch, cur);
+    loads_done();
+    for (int k = 0; k < count; k++) {
+      const int b0 = b, oy0 = oy, ch0 = ch;
+      if (k + 1 < count) next();
+      load(b, oy, ch, ahead);   // (past the end the last chunk again: no branch around a load)
+      multiply(b0, oy0, ch0, cur);
+      cur = ahead;
+    }
+  }
+
+  // the wavefronts' sums, added in wavefront order and stored in the order of dW's rows
+  constexpr int COLS = 16 * NT;
+  __shared__ T red[kWaves][16 * COLS];
+  T* const slab = g.out + (int64_t)blockIdx.x * g.F * CKK;
+#pragma unroll
+  for (int m = 0; m < TM; m++) {
+    if (m) __syncthreads();
+    // column of dW: packed tiles hold them in order, a channel tile's tap n of channel i is column 9 i + n
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) red[wave][Mfma<T>::row(q, v) * COLS + (kPacked ? n * 16 + i : i * 9 + n)] = acc[m][n][v];
+    __syncthreads();
+    for (int e = threadIdx.x; e < 16 * COLS; e += kThreads) {
+      const int f = f0 + 16 * m + e / COLS, col = c0 * 9 + e % COLS;
+      if (f < g.F && col < CKK) slab[(int64_t)f * CKK + col] = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
+    }
+  }
+}
+
+// out[e] = sum over the slabs of ws[s][e]: a workgroup takes RW results, its 256 / RW thread groups every G-th
+// slab (reads of a slab are RW values wide), and the groups' sums are added pairwise, neighbours first.
+template <class T, int RW>
+__global__ __launch_bounds__(256) void k_slab_sum(const T* __restrict__ ws, int slabs, int64_t total, T* __restrict__ out) {
+  constexpr int G = 256 / RW;
+  __shared__ T sh[256];
+  const int grp = threadIdx.x / RW;
+  const int64_t e = (int64_t)blockIdx.x * RW + threadIdx.x % RW;
+  T sum = (T)0;
+  if (e < total) {
+    int s = grp;
+    for (; s + 3 * G < slabs; s += 4 * G) {   // four loads in flight
+      T v[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) v[u] = ws[(int64_t)(s + u * G) * total + e];
+#pragma unroll
+      for (int u = 0; u < 4; u++) sum = sum + v[u];
+    }
+    for (; s < slabs; s += G) sum = sum + ws[(int64_t)s * total + e];
+  }
+  sh[threadIdx.x] = sum;
+  for (int d = 1; d < G; d <<= 1) {
+    __syncthreads();
+    T v = (T)0;
+    const bool mine = grp % (2 * d) == 0;
+    if (mine) v = sh[threadIdx.x] + sh[threadIdx.x + d * RW];
+    __syncthreads();
+    if (mine) sh[threadIdx.x] = v;
+  }
+  if (grp == 0 && e < total) out[e] = sh[threadIdx.x];
+}
+
+template <class T>
+int slab_sum(gh_ctx* ctx, const T* ws, int slabs, int64_t total, T* out) {
+  // 64 results to a workgroup where that makes enough workgroups, else 16
+  if (total >= 64 * (int64_t)ctx->cu_count)
+    hipLaunchKernelGGL((k_slab_sum<T, 64>), dim3((unsigned)((total + 63) / 64)), dim3(256), 0, ctx->stream, ws, slabs, total, out);
+  else
+    hipLaunchKernelGGL((k_slab_sum<T, 16>), dim3((unsigned)((total + 15) / 16)), dim3(256), 0, ctx->stream, ws, slabs, total, out);
+  return gh_check_hip(ctx, hipGetLastError(), "slab sum launch");
+}
+
+template <class T>
+bool fill(const gh_cmd& c, Wg<T>* g) {
+  for (int i : {5, 6}) if (c.dim[i] != 3) return false;
+  for (int i : {9, 10, 11, 12}) if (c.dim[i] != 1) return false;
+  const int64_t B = c.dim[0], C = c.dim[1], H = c.dim[2], W = c.dim[3], F = c.dim[4];
+  const int64_t oh = gh_conv_out(H, 3, c.dim[7], 1, 1), ow = gh_conv_out(W, 3, c.dim[8], 1, 1);
+  if (B <= 0 || C <= 0 || F <= 0 || oh <= 0 || ow <= 0 || c.dim[7] > 1024 || c.dim[8] > 1024) return false;
+  if (H > (1 << 20) || W > (1 << 20) || C > (1 << 20) || F > 65535 * 16) return false;
+  g->x = (const T*)(uintptr_t)c.ptr[0];
+  g->dy = (const T*)(uintptr_t)c.ptr[1];
+  // 32-bit byte offsets; whole loads inside the tensors
+  const int64_t most = ((int64_t)1 << 31) / (int64_t)sizeof(T) - 64;
+  if (B * C * H > most / W || B * F * oh > most / ow || B * C * H * W < 6 || B * F * oh * ow < 4) return false;
+  g->x_total = (int)(B * C * H * W);
+  g->dy_total = (int)(B * F * oh * ow);
+  g->B = (int)B; g->C = (int)C; g->H = (int)H; g->W = (int)W; g->F = (int)F; g->oh = (int)oh; g->ow = (int)ow;
+  g->padH = (int)c.dim[7]; g->padW = (int)c.dim[8];
+  const int px = ow <= 8 ? 8 : 16;
+  g->nch = (int)((ow + px - 1) / px);
+  const int64_t items = B * oh * g->nch;
+  if (items > INT32_MAX / 2) return false;
+  g->items = (int)items;
+  return true;
+}
+
+template <class T, int TM, int P, int NT, bool kPacked>
+int launch(gh_ctx* ctx, Wg<T> g, T* dw) {
+  const int64_t ft = (g.F + 16 * TM - 1) / (16 * TM), ct = kPacked ? 1 : (g.C + 15) / 16;
+  const int64_t results = (int64_t)g.F * g.C * 9;
+  // Workgroups to a compute unit: what a wavefront does besides its MFMAs - the first loads, meeting the others, a
+  // slab to be summed - costs as much as some ten chunks of a channel tile, so one; packed tiles, three.
+  int64_t slices = std::max<int64_t>(1, (kPacked ? 3 : 1) * (int64_t)ctx->cu_count / (ft * ct));
+  slices = std::min<int64_t>(slices, std::max<int64_t>(1, g.items / (4 * kWaves)));
+  if (slices > 1 && slices * results * (int64_t)sizeof(T) > ctx->workspace_bytes) {
+    if (int rc = gh_ws_short(ctx, slices * results * (int64_t)sizeof(T))) return rc;
+    slices = std::max<int64_t>(1, ctx->workspace_bytes / (results * (int64_t)sizeof(T)));
+  }
+  g.per = (int)((g.items + slices * kWaves - 1) / (slices * kWaves));
+  slices = (g.items + (int64_t)g.per * kWaves - 1) / ((int64_t)g.per * kWaves);
+  g.out = slices > 1 ? (T*)ctx->workspace : dw;
+  hipLaunchKernelGGL((k_conv3x3_wgrad<T, TM, P, NT, kPacked>), dim3((unsigned)slices, (unsigned)ct, (unsigned)ft), dim3(kThreads), 0,
+                     ctx->stream, g);
+  const int rc = gh_check_hip(ctx, hipGetLastError(), "filter-gradient launch");
+  return rc || slices == 1 ? rc : slab_sum(ctx, (const T*)ctx->workspace, (int)slices, results, dw);
+}
+
+template <class T>
+int pick(gh_ctx* ctx, const Wg<T>& g, T* dw) {
+  // packed columns take fewer tiles than nine taps of a channel tile up to eight channels
+  if (g.C == 1) return launch<T, 1, 4, 1, true>(ctx, g, dw);
+  if (g.C <= 3) return launch<T, 1, 4, 2, true>(ctx, g, dw);
+  if (g.C <= 5) return launch<T, 1, 4, 3, true>(ctx, g, dw);
+  if (g.C <= 8) return launch<T, 1, 4, 5, true>(ctx, g, dw);
+  // two filter tiles share the loads of x; of float64 one fills the registers
+  if constexpr (sizeof(T) == 4) {
+    if (g.F > 16) return g.ow <= 8 ? launch<T, 2, 2, 9, false>(ctx, g, dw) : launch<T, 2, 4, 9, false>(ctx, g, dw);
+  }
+  return g.ow <= 8 ? launch<T, 1, 2, 9, false>(ctx, g, dw) : launch<T, 1, 4, 9, false>(ctx, g, dw);
+}
+
+}  // namespace
+
+// Whether k_conv3x3_wgrad takes a filter gradient: 3x3, stride 1.  Of float32, not the shapes the small-image and
+// the single-channel kernel hold in LDS, and up to four channels only where there are enough pixels to cut up
+// (below that the vector kernel's few workgroups do; of a single channel it wastes the least).
+bool gh_conv_wgrad_takes(const gh_cmd& c) {
+  Wg<double> g;   // (the narrower of the two in what its offsets reach)
+  if (!fill(c, &g) || g.F < 8) return false;
+  const int64_t pixels = g.dy_total / g.F;
+  if (g.C <= 8 && g.ow <= 8) return false;
+  if (gh_dtype_of(c.flags) == GH_F64) return pixels >= 256;
+  return pixels >= (g.C == 1 ? 65536 : g.C <= 4 ? 16384 : 256);
+}
+
+int gh_launch_conv_wgrad(gh_ctx* ctx, const gh_cmd& c) {
+  if (gh_dtype_of(c.flags) == GH_F64) {
+    Wg<double> g;
+    if (!fill(c, &g)) return gh_fail(ctx, GH_ESTATE, "filter gradient: not a shape of this kernel");
+    return pick<double>(ctx, g, (double*)(uintptr_t)c.ptr[2]);
+  }
+  Wg<float> g;
+  if (!fill(c, &g)) return gh_fail(ctx, GH_ESTATE, "filter gradient: not a shape of this kernel");
+  return pick<float>(ctx, g, (float*)(uintptr_t)c.ptr[2]);
+}

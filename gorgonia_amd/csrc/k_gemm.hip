@@ -2919,6 +2919,10 @@ bool gh_try_launch_conv2d_bwd_data_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
 // Float64 filter gradient on the matrix cores, pixel axis cut into slices.
 bool gh_try_launch_conv2d_bwd_filter_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
   ConvGeom64 g;
+  if (gh_conv_wgrad_takes(c)) {
+    gh_launch_conv_wgrad(ctx, c);   // an error is sticky on the context; the caller returns it
+    return true;
+  }
   if (!conv64_fill(c, &g)) return false;
   if ((int64_t)g.P * g.F * g.K < (int64_t)1 << 22 || g.P < 64) return false;
   constexpr int BM = 64, BN = 64, BK = 16;
@@ -3184,11 +3188,17 @@ static bool wgrad_c1_takes(const gh_cmd& c) {
   return img_bytes <= 60 * 1024 && g.oh * g.ow >= 64 && g.ow >= 2 && !getenv("GORGONIA_HIP_WGRAD_NO_C1");   // (tuning switch)
 }
 
+// ... and what is left to k_conv3x3_wgrad: neither the single-channel nor the small-image kernel's shapes.
+static bool wgrad_mfma_takes(const gh_cmd& c) {
+  return gh_conv_wgrad_takes(c) && !wgrad_c1_takes(c) && !gh_conv_wgrad_small_takes(c);
+}
+
 // dW = dY2d^T . col  (ptr[0] = x, ptr[1] = dy, ptr[2] = dw)
 int gh_launch_conv2d_bwd_filter(gh_ctx* ctx, const gh_cmd& c) {
   if (gh_dtype_of(c.flags) == GH_F64) return gh_launch_conv2d_bwd_filter_f64(ctx, c);
   const ConvGeom g = conv_geom(c);
   const int F = (int)c.dim[4], CKK = g.C * g.kh * g.kw;
+  if (wgrad_mfma_takes(c)) return gh_launch_conv_wgrad(ctx, c);
   if (conv_direct_shape(c) && F <= 65535) {
     const int B = (int)c.dim[0];
     int G = B < 64 ? B : 64;
@@ -3404,6 +3414,7 @@ extern "C" int gh_conv2d_bwd_filter_route(const gh_cmd* c) {
   if (!c || c->opcode != GH_OP_CONV2D_BWD_FILTER) return -1;
   if (gh_dtype_of(c->flags) == GH_F64) return GH_WGRAD_ROUTE_F64;
   if (wgrad_c1_takes(*c)) return GH_WGRAD_ROUTE_SINGLE_CHANNEL;
+  if (wgrad_mfma_takes(*c)) return GH_WGRAD_ROUTE_GEMM;
   if (conv_direct_shape(*c) && c->dim[4] <= 65535) return GH_WGRAD_ROUTE_DIRECT;
   if (gh_conv_wgrad_small_takes(*c)) return GH_WGRAD_ROUTE_SMALL;
   return GH_WGRAD_ROUTE_GEMM;

@@ -344,7 +344,7 @@ GH_API int gh_conv2d_route(const gh_cmd* conv);
 /* The same for a CONV2D_BWD_FILTER command (ConvolutionBackwardFilter,
  * ops/nn/convolution_cuda.go:230-267): GH_WGRAD_ROUTE_*, or -1. */
 enum gh_wgrad_route {
-  GH_WGRAD_ROUTE_DIRECT = 0,  /* 3x3, at most four channels: reduction on the vector ALUs     */
+  GH_WGRAD_ROUTE_DIRECT = 0,  /* 3x3, at most four channels, few pixels: on the vector ALUs   */
   GH_WGRAD_ROUTE_SMALL = 1,   /* 3x3 over images up to 16 x 16: dy and x in LDS, MFMA          */
   GH_WGRAD_ROUTE_GEMM = 2,    /* every other geometry: implicit GEMM over the output pixels    */
   GH_WGRAD_ROUTE_F64 = 3,     /* float64 (its own kernels)                                     */
