@@ -495,7 +495,8 @@ __global__ __launch_bounds__(256) void k_splitk_reduce_lanes(const float* __rest
 // - a fixed order, so results repeat bit for bit - and the epilogue is applied.
 // (Cutting K across workgroups as well, with the last one to arrive at a
 // per-tile counter adding the slices, was measured: the device-wide fences it
-// needs cost ~35 us per launch on this part, four times the whole kernel.)
+// needs cost ~35 us per launch on this part, four times the whole kernel.  Long
+// contractions are cut by grid.z and added by a second launch: skinny_slices.)
 template <int WV, bool VEC, bool VECB>
 __global__ __launch_bounds__(WV * 64) void k_gemm_skinny(const float* __restrict__ A,
                                                          const float* __restrict__ B,
@@ -515,7 +516,10 @@ __global__ __launch_bounds__(WV * 64) void k_gemm_skinny(const float* __restrict
   // bits from both (a column's sum does not depend on the tile it sits in).
   const int m0 = blockIdx.y * 32, n0 = VECB ? min((int)blockIdx.x * 32, N - 32) : blockIdx.x * 32;
   const int m = m0 + r, n = n0 + r;
-  const int nchunks = (K + 15) / 16;
+  // this slice's chunks [chunk0, nchunks); a slice's tile goes to a slab of its own
+  const int all_chunks = (K + 15) / 16, per = (all_chunks + (int)gridDim.z - 1) / (int)gridDim.z;
+  const int chunk0 = (int)blockIdx.z * per, nchunks = min(all_chunks, chunk0 + per);
+  C += (int64_t)blockIdx.z * M * N;
 
   // Lane (r, h) feeds k = 16*chunk + 8*h + t at MFMA step t of a chunk.  B comes
   // in that order straight from memory (32 consecutive columns per k).  A would
@@ -616,7 +620,7 @@ __global__ __launch_bounds__(WV * 64) void k_gemm_skinny(const float* __restrict
   // The MFMAs of one group form a dependent chain of 8*G*64 cycles; the next
   // group's loads are issued before it so their latency runs underneath.
   float a0[G][8], b0[G][8], a1[G][8], b1[G][8];
-  int c0 = wave;
+  int c0 = chunk0 + wave;
   if (c0 < nchunks) load_group(c0, a0, b0);
   while (c0 < nchunks) {
     const int c1 = c0 + G * WV;
@@ -723,7 +727,9 @@ __global__ __launch_bounds__(WV * 64) void k_gemm_skinny16(const float* __restri
     tile_y = nid - tile_x * gy;
   }
   const int m0 = min(tile_y * 16, M - 16), n0 = ragged_n ? 0 : min(tile_x * BN, N - BN);
-  const int nchunks = (K + 15) / 16;
+  const int all_chunks = (K + 15) / 16, per = (all_chunks + (int)gridDim.z - 1) / (int)gridDim.z;
+  const int chunk0 = (int)blockIdx.z * per, nchunks = min(all_chunks, chunk0 + per);   // as in k_gemm_skinny
+  C += (int64_t)blockIdx.z * M * N;
   int ncol[NT];   // this lane's columns (clamped when the tile is wider than the matrix)
 #pragma unroll
   for (int c = 0; c < NT; c++) ncol[c] = min(n0 + NT * i + c, N - 1);
@@ -797,7 +803,7 @@ __global__ __launch_bounds__(WV * 64) void k_gemm_skinny16(const float* __restri
       }
   };
   float a0[G][4], b0[G][4][NT], a1[G][4], b1[G][4][NT];
-  int c0 = wave;
+  int c0 = chunk0 + wave;
   if (c0 < nchunks) load_group(c0, a0, b0);
   while (c0 < nchunks) {
     const int c1 = c0 + G * WV;
@@ -851,6 +857,48 @@ __global__ __launch_bounds__(WV * 64) void k_gemm_skinny16(const float* __restri
     if (bias) sum = sum + bias[col];
     C[(int64_t)(m0 + e / BN) * ldc + col] = act_apply(sum, act, alpha);
   }
+}
+
+// Adds the slabs of a small-output product cut along K, in slab order, and applies the epilogue: bias, activation,
+// and the row softmax with the arithmetic of the softmax kernel (N <= 32: 32 lanes hold a row).
+__global__ __launch_bounds__(256) void k_skinny_sum(const float* __restrict__ ws, int slabs, int M, int N,
+                                                    float* __restrict__ C, int ldc, int act, float alpha,
+                                                    const float* __restrict__ bias, int softmax) {
+  const int64_t total = (int64_t)M * N;
+  const int width = softmax ? 32 : N;
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x, row = e / width;
+  const int col = (int)(e - row * width);
+  const bool mine = row < M && col < N;
+  float sum = 0.f;
+  if (mine) {
+    const float* p = ws + row * N + col;
+    int s = 0;
+    for (; s + 8 <= slabs; s += 8) {   // eight loads in flight
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = p[(int64_t)(s + u) * total];
+#pragma unroll
+      for (int u = 0; u < 8; u++) sum = sum + v[u];
+    }
+    for (; s < slabs; s++) sum = sum + p[(int64_t)s * total];
+    if (bias) sum = sum + bias[col];
+    sum = act_apply(sum, act, alpha);
+  }
+  if (softmax) {
+    __shared__ float x[8][33], ex[8][33];
+    const int r = threadIdx.x >> 5;
+    x[r][col] = sum;
+    __syncthreads();
+    float mx = -INFINITY;
+    for (int j = 0; j < N; j++) mx = fmaxf(mx, x[r][j]);
+    ex[r][col] = mine ? (float)exp((double)(sum - mx)) : 0.f;
+    __syncthreads();
+    float t = 0.f;
+    for (int j = 0; j < N; j++) t = t + ex[r][j];
+    const float inv = 1.0f / t;
+    sum = ex[r][col] * inv;
+  }
+  if (mine) C[row * ldc + col] = sum;
 }
 
 // ---- Conv2d 3x3 / stride 1 with the input staged in LDS -----------------------------
@@ -2760,8 +2808,41 @@ static bool gemm_skinny_takes(const gh_cmd& c, int cus) {
   return true;
 }
 
+// Slices of K for a small-output product: a tile is one workgroup's work, and one workgroup walks 1000 of K in about
+// 7 us, so a long contraction over few tiles is cut until the slices fill the device or are down to 512 (four chunks
+// for each of eight wavefronts); below 2048 the second launch (5 us) costs what the cut saves.
+static int skinny_slices(const gh_cmd& c, int cus) {
+  const int64_t M = c.dim[0], N = c.dim[1], K = c.dim[2];
+  if (K < 2048) return 1;
+  const int64_t tiles = cdiv(M, M >= 16 ? 16 : 32) * cdiv(N, 32);
+  return (int)std::max<int64_t>(1, std::min<int64_t>(cus / tiles, K / 512));
+}
+
+static int launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c, int slices);
+
 static int try_launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c) {
   if (!gemm_skinny_takes(c, ctx->cu_count)) return -1;
+  const int slices = skinny_slices(c, ctx->cu_count);
+  const int64_t M = c.dim[0], N = c.dim[1];
+  if (slices > 1 && (int64_t)slices * M * N * 4 > ctx->workspace_bytes) {
+    if (int rc = gh_ws_short(ctx, (int64_t)slices * M * N * 4)) return rc;
+    return launch_gemm_skinny(ctx, c, 1);
+  }
+  if (slices == 1) return launch_gemm_skinny(ctx, c, 1);
+  gh_cmd part = c;   // the bare product, slab after slab
+  part.flags &= ~(uint32_t)(GH_FLAG_ACT_RELU | GH_FLAG_ACT_LEAKY | GH_FLAG_GEMM_SOFTMAX | GH_FLAG_GEMM_BIAS);
+  part.ptr[2] = (uint64_t)(uintptr_t)ctx->workspace;
+  part.dim[5] = N;
+  if (int rc = launch_gemm_skinny(ctx, part, slices)) return rc;
+  const int softmax = (c.flags & GH_FLAG_GEMM_SOFTMAX) ? 1 : 0;
+  const int act = (c.flags & GH_FLAG_ACT_RELU) ? 1 : (c.flags & GH_FLAG_ACT_LEAKY) ? 2 : 0;
+  hipLaunchKernelGGL(k_skinny_sum, dim3((unsigned)cdiv(M * (softmax ? 32 : N), 256)), dim3(256), 0, ctx->stream,
+                     (const float*)ctx->workspace, slices, (int)M, (int)N, (float*)(uintptr_t)c.ptr[2], (int)c.dim[5], act, c.f[0],
+                     (c.flags & GH_FLAG_GEMM_BIAS) ? (const float*)(uintptr_t)c.ptr[3] : nullptr, softmax);
+  return gh_check_hip(ctx, hipGetLastError(), "skinny gemm slab sum launch");
+}
+
+static int launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c, int slices) {
   const bool ta = c.flags & GH_FLAG_TRANS_A, tb = c.flags & GH_FLAG_TRANS_B;
   const int M = (int)c.dim[0], N = (int)c.dim[1], K = (int)c.dim[2];
   const int64_t tiles = cdiv(M, 32) * cdiv(N, 32);
@@ -2790,7 +2871,7 @@ static int try_launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c) {
     const int64_t blocks_wide = cdiv(M, 16) * cdiv(N, 32);
     const bool narrow = N < 32 || (force ? !strcmp(force, "16x16") : blocks_wide * 2 <= ctx->cu_count);
     auto launch16 = [&](auto kernel, int bn) {
-      hipLaunchKernelGGL(kernel, dim3((N + bn - 1) / bn, (M + 15) / 16), dim3(WV * 64), 0, ctx->stream, A, B, C, M,
+      hipLaunchKernelGGL(kernel, dim3((N + bn - 1) / bn, (M + 15) / 16, slices), dim3(WV * 64), 0, ctx->stream, A, B, C, M,
                          N, K, lda, ldb, ldc, act, c.f[0], bias, softmax);
     };
     // Sixteen wavefronts share the K of a long contraction (a function of the shape alone, like the tile): each
@@ -2799,7 +2880,7 @@ static int try_launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c) {
     static const bool no16 = getenv("GORGONIA_HIP_SKINNY_WAVES8") != nullptr;   // tuning switch
     const bool wide16 = K >= 512 && !no16;
     auto launch16w = [&](auto kernel, int bn) {
-      hipLaunchKernelGGL(kernel, dim3((N + bn - 1) / bn, (M + 15) / 16), dim3(16 * 64), 0, ctx->stream, A, B, C, M,
+      hipLaunchKernelGGL(kernel, dim3((N + bn - 1) / bn, (M + 15) / 16, slices), dim3(16 * 64), 0, ctx->stream, A, B, C, M,
                          N, K, lda, ldb, ldc, act, c.f[0], bias, softmax);
     };
 #define GH_SKINNY16(TA_, TB_)                                                               \
@@ -2816,7 +2897,7 @@ static int try_launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c) {
     return gh_check_hip(ctx, hipGetLastError(), "skinny gemm launch");
   }
   const bool vec_a = al16(c.ptr[0]) && lda % 4 == 0 && K % 16 == 0;
-  const dim3 grid((N + 31) / 32, (M + 31) / 32);
+  const dim3 grid((N + 31) / 32, (M + 31) / 32, slices);
   const bool vec_b = N >= 32;   // whole column tiles (the last one moved left)
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(WV * 64), 0, ctx->stream, A, B, C, M, N, K, lda, ldb, ldc, act, c.f[0],
@@ -3040,7 +3121,10 @@ extern "C" int gh_gemm_route(const gh_cmd* c, int* splits) {
   gh_ctx probe;
   probe.workspace = &probe;   // never dereferenced: only "there is one" and its size are read
   probe.workspace_bytes = 64ll << 20;
-  if (gemm_skinny_takes(*c, probe.cu_count)) return GH_GEMM_ROUTE_SMALL_OUTPUT;
+  if (gemm_skinny_takes(*c, probe.cu_count)) {
+    if (splits) *splits = skinny_slices(*c, probe.cu_count);
+    return GH_GEMM_ROUTE_SMALL_OUTPUT;
+  }
   const TilePlan p = plan_tiles(&probe, c->dim[0], c->dim[1], c->dim[2], batch, false);
   if (splits) *splits = p.splits;
   return p.tile == kTile128 ? GH_GEMM_ROUTE_TILE128 : p.tile == kTile128x64 ? GH_GEMM_ROUTE_TILE128X64 : GH_GEMM_ROUTE_TILE64;
