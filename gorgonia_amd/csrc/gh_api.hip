@@ -264,23 +264,24 @@ __global__ __launch_bounds__(256) void k_copy_vec(uint4* __restrict__ dst, const
     ((uint32_t*)(dst + n16))[threadIdx.x] = ((const uint32_t*)(src + n16))[threadIdx.x];
 }
 
-static constexpr int64_t kKernelCopyLimit = 16 << 20;
-// From pinned host memory the copy engine asks the bus for larger pieces than a kernel's 64-byte
-// loads do: 16.6 MB in 299 us against 334 (55.6 / 49.8 GB/s); the kernel is ahead below about
-// 2.5 MB (0.4 MB: 10.7 us against 16.6), where the engine's 9 us of start-up count.
-static constexpr int64_t kHostDmaFrom = 4 << 20;
+static constexpr int64_t kKernelCopyLimit = 16 << 20;   // between device buffers
+// Workgroups of a copy out of pinned host memory.  The bus needs few requests in flight and serves them the better
+// the fewer workgroups interleave theirs: 16.6 MB take 355 us with 1024 workgroups, 308 with 64 to 128 (the copy
+// engine: 301, and 5 us more for the kernel behind it to see its signal), 2 MB 62 and 51.
+static constexpr int64_t kHostCopyBlocks = 96;
 
 int gh_memcpy_d2d(gh_ctx* ctx, gh_devptr dst, gh_devptr src, int64_t bytes) {
   if (!ctx || bytes < 0 || (bytes > 0 && (!dst || !src))) return GH_EINVAL;
   if (ctx->err) return ctx->err;
   if (bytes == 0) return GH_OK;
   ctx->idle = false;
-  const bool dma_from_host = bytes >= kHostDmaFrom && in_pinned_host(ctx, src);
-  if (!dma_from_host && bytes <= kKernelCopyLimit && ((dst | src | (uint64_t)bytes) & 3) == 0) {
+  const bool from_host = in_pinned_host(ctx, src);
+  if ((from_host || bytes <= kKernelCopyLimit) && ((dst | src | (uint64_t)bytes) & 3) == 0) {
     if (((dst | src) & 15) == 0 && bytes >= 4096) {
       const int64_t n16 = bytes / 16;
       int64_t blocks = (n16 + 511) / 512;
-      if (blocks > 1024) blocks = 1024;
+      const int64_t most = from_host ? kHostCopyBlocks : 1024;
+      if (blocks > most) blocks = most;
       hipLaunchKernelGGL(k_copy_vec, dim3((int)blocks), dim3(256), 0, ctx->stream, (uint4*)(uintptr_t)dst,
                          (const uint4*)(uintptr_t)src, n16, (bytes % 16) / 4);
     } else {

@@ -16,10 +16,11 @@ static constexpr int64_t kStageLimit = 8 << 20;
 // inputs re-uploaded on every run are staged through pinned memory up to these sizes
 static constexpr int64_t kStageInLimit = 16 << 20;    // per input (what one copy kernel moves)
 static constexpr int64_t kStageInTotal = 512ll << 20; // per machine
-// inputs from this size on are uploaded in pieces, the host copy into pinned memory overlapping the bus
-static constexpr int64_t kPipelinedUpload = 4 << 20;
-static constexpr int64_t kUploadPiece = 2 << 20;
-
+// inputs from this size on are uploaded in pieces, the host copy into pinned memory overlapping the bus.  A piece
+// costs a launch (some 5 us in front of the bus), so the pieces of a long upload are larger: host copy and upload
+// together take 72 us of 2 MB (109 in one piece), 124 of 4 MB (185), 392 of 16 MB (590).
+static constexpr int64_t kPipelinedUpload = 768 << 10;
+static constexpr int64_t kUploadPiece = 512 << 10, kUploadPieceLong = 2 << 20, kLongUpload = 8 << 20;
 // inputs up to this size are read where the host wrote them, in pinned memory: the copy kernel a few KB would
 // need costs 4 us on the device, an operand read over the bus about 1
 static constexpr int64_t kReadInPlace = 8 << 10;
@@ -1231,14 +1232,15 @@ Status TapeMachine::upload(const Instr& in, bool record) {
     }
     if (in_pieces_[(size_t)in.node] && !n.host_borrowed) {
       // a large value at the front of its segment: piece by piece, the host copy of one
-      // piece runs while the copy engine moves the piece before it (stream order puts the
+      // piece runs while the bus moves the piece before it (stream order puts the
       // segment's operators behind the last piece)
+      const int64_t piece = in.size >= kLongUpload ? kUploadPieceLong : kUploadPiece;
       const char* src = static_cast<const char*>(n.host);
       char* stg = static_cast<char*>(pinned);
-      for (int64_t off = 0; off < in.size; off += kUploadPiece) {
-        const int64_t len = std::min(kUploadPiece, in.size - off);
+      for (int64_t off = 0; off < in.size; off += piece) {
+        const int64_t len = std::min(piece, in.size - off);
         std::memcpy(stg + off, src + off, (size_t)len);
-        Status st = eng_.MemcpyHtoD(mem + (uint64_t)off, stg + off, len);
+        Status st = eng_.CopyNow(mem + (uint64_t)off, (uint64_t)(uintptr_t)(stg + off), len);
         if (!st.ok()) return st;
       }
       return Status::OK();
