@@ -66,8 +66,34 @@ static bool in_pinned_host(const gh_ctx* ctx, uint64_t p) {
   return false;
 }
 
+// The contexts' completion words: 64 of them, 64 bytes apart, in one pinned page that lives as long as the process
+// (allocating one costs more than the rest of a small context).  A context beyond the 64th has none and waits in
+// the runtime.
+static std::mutex g_words_mu;
+static unsigned char* g_words_page = nullptr;
+static uint64_t g_words_used = 0;
+
+static uint32_t* take_word() {
+  std::lock_guard<std::mutex> lock(g_words_mu);
+  if (!g_words_page && hipHostMalloc((void**)&g_words_page, 4096, hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();
+    g_words_page = nullptr;
+  }
+  if (!g_words_page || ~g_words_used == 0) return nullptr;
+  const int i = __builtin_ctzll(~g_words_used);
+  g_words_used |= 1ull << i;
+  uint32_t* const w = (uint32_t*)(g_words_page + 64 * i);
+  *w = 0;
+  return w;
+}
+static void give_word(uint32_t* w) {
+  if (!w) return;
+  std::lock_guard<std::mutex> lock(g_words_mu);
+  g_words_used &= ~(1ull << (((unsigned char*)w - g_words_page) / 64));
+}
+
 static void drop_ctx(gh_ctx* ctx) {
-  if (ctx->done_word) hipHostFree(ctx->done_word);
+  give_word(ctx->done_word);   // nothing is in flight any more
   if (ctx->workspace) hipFree(ctx->workspace);
   if (ctx->arena) hipFree(ctx->arena);
   hipStreamDestroy(ctx->stream);
@@ -103,13 +129,7 @@ int gh_init(int device, int64_t arena_bytes, gh_ctx** out) {
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) ctx->cu_count = prop.multiProcessorCount;
   if (const char* sm = getenv("GORGONIA_HIP_SYNC")) ctx->sync_block = strcmp(sm, "block") == 0;
-  // without the word gh_sync waits in the runtime
-  if (hipHostMalloc((void**)&ctx->done_word, 64, hipHostMallocDefault) != hipSuccess) {
-    (void)hipGetLastError();
-    ctx->done_word = nullptr;
-  } else {
-    *ctx->done_word = 0;
-  }
+  ctx->done_word = take_word();
   if (arena_bytes > 0) {
     size_t free_b = 0, total_b = 0;
     hipMemGetInfo(&free_b, &total_b);

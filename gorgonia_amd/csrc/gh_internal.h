@@ -114,6 +114,10 @@ int gh_launch_leaky_relu(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_fill(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_has_nan_inf(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_gemm(gh_ctx* ctx, const gh_cmd& c);
+// products with operands straight from memory (k_gemm_direct.hip)
+int gh_gemm_direct_form(const gh_cmd& c, int cus, double* us);   // -1: not taken
+int gh_gemm_direct_slices(const gh_cmd& c, int form, int cus);
+int gh_launch_gemm_direct(gh_ctx* ctx, const gh_cmd& c, int form);
 int gh_launch_gemv(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_outer(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_conv2d(gh_ctx* ctx, const gh_cmd& c);

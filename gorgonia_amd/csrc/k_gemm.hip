@@ -1402,52 +1402,6 @@ struct LoadKContig64 {
   }
 };
 
-// Operand stored [k][c] with c contiguous (B not transposed; A transposed): a
-// thread takes columns c, c+1 of rows k, k+1 and writes the two k-pairs.
-template <int R, int BK, bool VEC>
-struct LoadMnContig64 {
-  static constexpr int S2 = 2 * R + 8;
-  static constexpr int SIZE = (BK / 2) * S2;
-  static constexpr int TOTAL = (R / 2) * (BK / 2);   // 2x2 cells per tile
-  static constexpr int NV = (TOTAL + kThreads - 1) / kThreads;
-  const double* base; int ld; int rmax; int kmax;
-  f64x2 reg[NV][2];
-  __device__ __forceinline__ void load(int c0, int k0) {
-#pragma unroll
-    for (int j = 0; j < NV; j++) {
-      const int f = threadIdx.x + j * kThreads;
-      const int c = c0 + (f % (R / 2)) * 2;
-      const int k = k0 + (f / (R / 2)) * 2;
-      f64x2 v0 = {0.0, 0.0}, v1 = {0.0, 0.0};
-      if ((TOTAL % kThreads == 0 || f < TOTAL) && c < rmax) {
-        const double* p = base + (int64_t)k * ld + c;
-        if (VEC) {
-          if (k < kmax) v0 = *reinterpret_cast<const f64x2*>(p);
-          if (k + 1 < kmax) v1 = *reinterpret_cast<const f64x2*>(p + ld);
-        } else if (c + 1 < rmax) {
-          if (k < kmax) v0 = *reinterpret_cast<const f64x2_a8*>(p);
-          if (k + 1 < kmax) v1 = *reinterpret_cast<const f64x2_a8*>(p + ld);
-        } else {
-          if (k < kmax) v0[0] = p[0];
-          if (k + 1 < kmax) v1[0] = p[ld];
-        }
-      }
-      reg[j][0] = v0;
-      reg[j][1] = v1;
-    }
-  }
-  __device__ __forceinline__ void store(double* lds) const {
-#pragma unroll
-    for (int j = 0; j < NV; j++) {
-      const int f = threadIdx.x + j * kThreads;
-      if (TOTAL % kThreads != 0 && f >= TOTAL) continue;
-      double* d = &lds[(f / (R / 2)) * S2 + 4 * (f % (R / 2))];
-      *reinterpret_cast<f64x2*>(d) = f64x2{reg[j][0][0], reg[j][1][0]};
-      *reinterpret_cast<f64x2*>(d + 2) = f64x2{reg[j][0][1], reg[j][1][1]};
-    }
-  }
-};
-
 // The float64 MFMA core: 2x2 wavefronts over a BM x BN block, k-tiles [kt0, kt1).
 template <int BM, int BN, int BK, class LA, class LB>
 __device__ __forceinline__ void dmfma_tile_loop(double* lds, LA& la, LB& lb, int m0, int n0, int kt0, int kt1,
@@ -1597,38 +1551,6 @@ __device__ __forceinline__ void dmfma_tile_loop_auto(double* lds, LA& la, LB& lb
   dmfma_tile_loop<BM, BN, BK, LA, LB>(lds, la, lb, m0, n0, 0, nkt, acc);
 }
 
-template <int BM, int BN, int BK, bool TA, bool TB, bool VEC>
-__global__ __launch_bounds__(kThreads) void k_dgemm(const double* __restrict__ A,
-                                                    const double* __restrict__ B,
-                                                    double* __restrict__ C, int M, int N, int K,
-                                                    int lda, int ldb, int ldc, int64_t sA,
-                                                    int64_t sB, int64_t sC) {
-  using LA = typename std::conditional<TA, LoadMnContig64<BM, BK, VEC>, LoadKContig64<BM, BK, VEC>>::type;
-  using LB = typename std::conditional<TB, LoadKContig64<BN, BK, VEC>, LoadMnContig64<BN, BK, VEC>>::type;
-  constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
-  __shared__ double lds[2 * (LA::SIZE + LB::SIZE)];
-  int tile_m, tile_n, bz;
-  tile_coords(&tile_m, &tile_n, &bz, gridDim.z > 1);
-  const int m0 = tile_m * BM, n0 = tile_n * BN;
-  LA la; la.base = A + bz * sA; la.ld = lda; la.rmax = M; la.kmax = K;
-  LB lb; lb.base = B + bz * sB; lb.ld = ldb; lb.rmax = N; lb.kmax = K;
-  C += bz * sC;
-  f64x4 acc[TM][TN];
-  dmfma_tile_loop_auto<BM, BN, BK, LA, LB>(lds, la, lb, m0, n0, (K + BK - 1) / BK, acc);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
-  const int lr = lane & 15, lk = lane >> 4;
-#pragma unroll
-  for (int a = 0; a < TM; a++)
-#pragma unroll
-    for (int b = 0; b < TN; b++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int i = m0 + wm + a * 16 + 4 * v + lk, j = n0 + wn + b * 16 + lr;
-        if (i < M && j < N) C[(int64_t)i * ldc + j] = acc[a][b][v];
-      }
-}
-
 // Float64 product with a small result (a dense layer on a batch: too few 64x64
 // tiles to occupy the device, and a k loop of a thousand steps behind each).
 // One workgroup per 16x16 tile of C, its WV wavefronts each summing a slice of
@@ -1642,7 +1564,8 @@ __global__ __launch_bounds__(WV * 64) void k_dgemm_skinny(const double* __restri
                                                           const double* __restrict__ B,
                                                           double* __restrict__ C, int M, int N, int K,
                                                           int64_t sai, int64_t sak, int64_t sbk,
-                                                          int64_t sbj, int ldc) {
+                                                          int64_t sbj, int ldc, int64_t sA, int64_t sB, int64_t sC) {
+  A += blockIdx.z * sA; B += blockIdx.z * sB; C += blockIdx.z * sC;
   __shared__ double part[WV][256];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lr = lane & 15, lk = lane >> 4;
@@ -3033,53 +2956,24 @@ bool gh_try_launch_conv2d_bwd_filter_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
   return true;
 }
 
-template <int BM, int BN, int BK>
-static void launch_dgemm_cfg(gh_ctx* ctx, const gh_cmd& c, int M, int N, int K, int64_t batch) {
-  const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM, (unsigned)batch);
+// Float64: one 16x16 tile per workgroup (k_dgemm_skinny).  AV, BV: the operand is k-contiguous.
+static int launch_dgemm_skinny(gh_ctx* ctx, const gh_cmd& c) {
+  const int M = (int)c.dim[0], N = (int)c.dim[1], K = (int)c.dim[2];
+  const int64_t batch = c.dim[6] <= 0 ? 1 : c.dim[6];
+  const bool ta = c.flags & GH_FLAG_TRANS_A, tb = c.flags & GH_FLAG_TRANS_B;
+  const int64_t lda = c.dim[3], ldb = c.dim[4];
+  const int64_t sA = batch > 1 ? c.dim[7] : 0, sB = batch > 1 ? c.dim[8] : 0, sC = batch > 1 ? c.dim[9] : 0;
+  const dim3 grid((N + 15) / 16, (M + 15) / 16, (unsigned)batch);
   const double* A = (const double*)(uintptr_t)c.ptr[0];
   const double* B = (const double*)(uintptr_t)c.ptr[1];
   double* C = (double*)(uintptr_t)c.ptr[2];
-  const int lda = (int)c.dim[3], ldb = (int)c.dim[4], ldc = (int)c.dim[5];
-  const int64_t sA = batch > 1 ? c.dim[7] : 0, sB = batch > 1 ? c.dim[8] : 0, sC = batch > 1 ? c.dim[9] : 0;
-  const bool ta = c.flags & GH_FLAG_TRANS_A, tb = c.flags & GH_FLAG_TRANS_B;
-  const auto even = [](int64_t v) { return (v & 1) == 0; };
-  const bool vec = even(M) && even(N) && even(K) && even(lda) && even(ldb) && even(sA) && even(sB) &&
-                   ((c.ptr[0] | c.ptr[1]) & 15) == 0;
-#define GH_DGEMM_GO(TA, TB)                                                                                    \
-  do {                                                                                                         \
-    if (vec)                                                                                                   \
-      hipLaunchKernelGGL((k_dgemm<BM, BN, BK, TA, TB, true>), grid, dim3(kThreads), 0, ctx->stream, A, B, C, M, \
-                         N, K, lda, ldb, ldc, sA, sB, sC);                                                     \
-    else                                                                                                       \
-      hipLaunchKernelGGL((k_dgemm<BM, BN, BK, TA, TB, false>), grid, dim3(kThreads), 0, ctx->stream, A, B, C,  \
-                         M, N, K, lda, ldb, ldc, sA, sB, sC);                                                  \
-  } while (0)
-  if (ta && tb) GH_DGEMM_GO(true, true);
-  else if (ta) GH_DGEMM_GO(true, false);
-  else if (tb) GH_DGEMM_GO(false, true);
-  else GH_DGEMM_GO(false, false);
-#undef GH_DGEMM_GO
-}
-
-int gh_launch_gemm(gh_ctx* ctx, const gh_cmd& c) {
-  if (gh_dtype_of(c.flags) == GH_F64) {
-    const int M = (int)c.dim[0], N = (int)c.dim[1], K = (int)c.dim[2];
-    const int64_t batch = c.dim[6] <= 0 ? 1 : c.dim[6];
-    const int64_t tiles64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
-    if (batch == 1 && K >= 64 && tiles64 * 4 <= ctx->cu_count && M >= 1 && N >= 1) {
-      const bool ta = c.flags & GH_FLAG_TRANS_A, tb = c.flags & GH_FLAG_TRANS_B;
-      const int64_t lda = c.dim[3], ldb = c.dim[4];
-      const dim3 grid((N + 15) / 16, (M + 15) / 16, 1);
-      const double* A = (const double*)(uintptr_t)c.ptr[0];
-      const double* B = (const double*)(uintptr_t)c.ptr[1];
-      double* C = (double*)(uintptr_t)c.ptr[2];
-      // (which wavefront sums which k, and with AV which k shares an MFMA, depends on the shape and the operands'
-      // layout only: a product's bits repeat from run to run)
-      const bool pairs = K >= 2 && !getenv("GORGONIA_HIP_DGEMM_SKINNY_SCALAR");   // (tuning switch)
-      const bool av = pairs && !ta, bv = pairs && tb;
+  // (which wavefront sums which k, and with AV which k shares an MFMA, depends on the shape and the operands'
+  // layout only: a product's bits repeat from run to run)
+  const bool pairs = K >= 2 && !getenv("GORGONIA_HIP_DGEMM_SKINNY_SCALAR");   // (tuning switch)
+  const bool av = pairs && !ta, bv = pairs && tb;
 #define GH_DSK(WV_, AV_, BV_)                                                                                          \
   hipLaunchKernelGGL((k_dgemm_skinny<WV_, AV_, BV_>), grid, dim3(WV_ * 64), 0, ctx->stream, A, B, C, M, N, K,           \
-                     ta ? 1 : lda, ta ? lda : 1, tb ? 1 : ldb, tb ? ldb : 1, (int)c.dim[5])
+                     ta ? 1 : lda, ta ? lda : 1, tb ? 1 : ldb, tb ? ldb : 1, (int)c.dim[5], sA, sB, sC)
 #define GH_DSK_W(WV_)                                            \
   do {                                                           \
     if (av && bv) GH_DSK(WV_, true, true);                       \
@@ -3087,23 +2981,55 @@ int gh_launch_gemm(gh_ctx* ctx, const gh_cmd& c) {
     else if (bv) GH_DSK(WV_, false, true);                       \
     else GH_DSK(WV_, false, false);                              \
   } while (0)
-      if (K >= 256) GH_DSK_W(8);   // (sixteen wavefronts, as the float32 kernel has them from K = 512, are slower here: 15.7 us against 14.4)
-      else GH_DSK_W(4);
+  if (K >= 256) GH_DSK_W(8);   // (sixteen wavefronts, as the float32 kernel has them from K = 512, are slower here: 15.7 us against 14.4)
+  else GH_DSK_W(4);
 #undef GH_DSK_W
 #undef GH_DSK
-      return gh_check_hip(ctx, hipGetLastError(), "dgemm launch");
-    }
-    // 128x128 tiles once they fill the device, 64x64 with a longer k-tile below that
-    const int64_t tiles128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * batch;
-    if (tiles128 >= ctx->cu_count) launch_dgemm_cfg<128, 128, 8>(ctx, c, M, N, K, batch);
-    else launch_dgemm_cfg<64, 64, 16>(ctx, c, M, N, K, batch);
-    return gh_check_hip(ctx, hipGetLastError(), "dgemm launch");
+  return gh_check_hip(ctx, hipGetLastError(), "dgemm launch");
+}
+
+// Which kernel takes a float32 product that is none of the small-output ones: -1 for the LDS-tiled kernel under
+// plan_tiles, else a form of k_gemm_direct.
+static int direct_form(const gh_cmd& c, int cus) {
+  if (getenv("GORGONIA_HIP_GEMM_PLAN")) return -1;   // a forced tile plan means the tiled kernel
+  double us = 0;
+  const int form = gh_gemm_direct_form(c, cus, &us);
+  if (form < 0) return -1;
+  const int64_t M = c.dim[0], N = c.dim[1], K = c.dim[2], batch = c.dim[6] <= 0 ? 1 : c.dim[6];
+  const bool ta = c.flags & GH_FLAG_TRANS_A, tb = c.flags & GH_FLAG_TRANS_B;
+  const bool vec = ((c.ptr[0] | c.ptr[1]) & 15) == 0 && c.dim[3] % 4 == 0 && c.dim[4] % 4 == 0 && (ta ? M : K) % 4 == 0 && (tb ? K : N) % 4 == 0 &&
+                   (batch == 1 || (c.dim[7] % 4 == 0 && c.dim[8] % 4 == 0));
+  // Short contractions over many aligned 64x64 tiles: staging a tile once beats reading it per wavefront
+  // (1500 x 1500, K = 64: 9.2 us against 10.0; K = 100: equal; K = 130: 20 against 14).
+  if (vec && K <= 96 && cdiv(M, 64) * cdiv(N, 64) * batch >= 2 * cus) return -1;
+  // 128x128 tiles through LDS where they fill the device: 68 us per 1000 of K and round of tiles, half as much again
+  // with one workgroup per compute unit and nothing to run under its barriers.
+  const int64_t big = cdiv(M, 128) * cdiv(N, 128) * batch;
+  if (big >= cus && M > 64) {
+    const int64_t rounds = cdiv(big, cus);
+    const double est = 6.0 + (double)rounds * 64.0 * ((double)K * 1e-3 * 1.06 + 0.05) * (rounds == 1 ? 1.35 : 1.0) * (vec ? 1.0 : 1.25);
+    if (est < us) return -1;
+  }
+  return form;
+}
+
+int gh_launch_gemm(gh_ctx* ctx, const gh_cmd& c) {
+  const int64_t batch = c.dim[6] <= 0 ? 1 : c.dim[6];
+  if (gh_dtype_of(c.flags) == GH_F64) {
+    double us = 0;
+    const int form = gh_gemm_direct_form(c, ctx->cu_count, &us);
+    // one 16x16 tile per workgroup where larger tiles leave the device idle: 4.6 us per 1000 of K and 256 tiles
+    const double tiles16 = (double)cdiv(c.dim[0], 16) * (double)cdiv(c.dim[1], 16);
+    const double small = 4.0 + std::max(1.0, tiles16 / ctx->cu_count) * (double)c.dim[2] * 4.6e-3;
+    if (batch == 1 && c.dim[2] >= 64 && (form < 0 || small < us)) return launch_dgemm_skinny(ctx, c);
+    return form >= 0 ? gh_launch_gemm_direct(ctx, c, form) : launch_dgemm_skinny(ctx, c);
   }
   const int rs = try_launch_gemm_skinny(ctx, c);
   if (rs >= 0) return rs;
   if (c.flags & GH_FLAG_GEMM_SOFTMAX)
     return gh_fail(ctx, GH_EINVAL, "gemm: no fused softmax for this shape (see gh_gemm_can_softmax)");
-  const int64_t batch = c.dim[6] <= 0 ? 1 : c.dim[6];
+  const int form = direct_form(c, ctx->cu_count);
+  if (form >= 0) return gh_launch_gemm_direct(ctx, c, form);
   const TilePlan p = plan_tiles(ctx, c.dim[0], c.dim[1], c.dim[2], batch, false);
   if (ctx->err) return ctx->err;
   if (p.tile == kTile128) return launch_sgemm_cfg<128, 128, 2>(ctx, c, p.splits);
@@ -3124,6 +3050,11 @@ extern "C" int gh_gemm_route(const gh_cmd* c, int* splits) {
   if (gemm_skinny_takes(*c, probe.cu_count)) {
     if (splits) *splits = skinny_slices(*c, probe.cu_count);
     return GH_GEMM_ROUTE_SMALL_OUTPUT;
+  }
+  const int form = direct_form(*c, probe.cu_count);
+  if (form >= 0) {
+    if (splits) *splits = gh_gemm_direct_slices(*c, form, probe.cu_count);
+    return GH_GEMM_ROUTE_TILE64;
   }
   const TilePlan p = plan_tiles(&probe, c->dim[0], c->dim[1], c->dim[2], batch, false);
   if (splits) *splits = p.splits;
