@@ -142,6 +142,7 @@ bool gh_conv_rows1_takes(const gh_cmd& c);
 int gh_try_launch_conv_patch(gh_ctx* ctx, const gh_cmd& c);
 bool gh_conv_patch_takes(const gh_cmd& c);
 bool gh_conv_patch_can_pool(const gh_cmd& c);
+double gh_conv_patch_us(const gh_cmd& c, int cus);   // an estimate of its time
 // k_conv_wide.hip: 3x3 stride-1 convolution over large images with up to 64 channels
 int gh_try_launch_conv_wide(gh_ctx* ctx, const gh_cmd& c);
 bool gh_conv_wide_takes(const gh_cmd& c);
@@ -149,6 +150,9 @@ bool gh_conv_wide_can_pool(const gh_cmd& c);
 // k_conv_pointwise.hip: 1x1 stride-1 convolution whose result is too small for K-wide 64x64 tiles to fill the device
 int gh_try_launch_conv_pointwise(gh_ctx* ctx, const gh_cmd& c);
 bool gh_conv_pointwise_takes(const gh_cmd& c, int cus);
+// 3x3 stride-1 convolution with operands straight from memory, both float types; flip: of an image-gradient command (k_conv_lanes.hip)
+bool gh_conv_lanes_takes(const gh_cmd& c, bool flip, int cus, double other_us);
+int gh_launch_conv_lanes(gh_ctx* ctx, const gh_cmd& c, bool flip);
 int gh_launch_maxpool2d(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_bn_infer(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_softmax(gh_ctx* ctx, const gh_cmd& c);

@@ -395,6 +395,15 @@ bool gh_conv_patch_takes(const gh_cmd& c) {
   return patch_plan(c, false, &p);
 }
 
+// What a plain command takes here, in us (fitted to 1 to 8 images, 64 -> 128 at 52 x 52 to 512 -> 1024 at 13 x 13):
+// a workgroup walks its channels at 0.038 us per quad and 16 x 16 results.
+double gh_conv_patch_us(const gh_cmd& c, int cus) {
+  PatchPlan p;
+  if (!patch_plan(c, false, &p)) return 0;
+  const int64_t wgs = (int64_t)p.g.B * p.g.tiles_x * p.g.tiles_y * ((p.g.F + 16 * p.TM - 1) / (16 * p.TM));
+  return 3.2 + (double)((wgs + cus - 1) / cus) * (4.0 + 0.0377 * p.TM * p.TN * (p.g.C / 4));
+}
+
 // Pooling rides in the epilogue only where the even-sized patches it needs cost about the
 // same matrix work as the best plain patch grid; otherwise the separate pooling kernel is
 // cheaper than the extra MFMAs and halo.

@@ -2872,6 +2872,10 @@ bool gh_try_launch_conv2d_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
   if (!conv64_fill(c, &g)) return false;
   const int64_t P = g.P, K = g.K;
   if (g.F < 16 || P < 256 || K < 8 || P * g.F * K < (int64_t)1 << 22) return false;
+  if (gh_conv_lanes_takes(c, false, ctx->cu_count, 0)) {
+    gh_launch_conv_lanes(ctx, c, false);   // an error is sticky on the context; the caller returns it
+    return true;
+  }
   const int64_t tiles128 = (int64_t)((g.F + 127) / 128) * ((P + 127) / 128);
   // the smaller tiles do less per k-tile, so they take twice the k range per barrier
   const int64_t tiles64 = (int64_t)((g.F + 63) / 64) * ((P + 63) / 64);
@@ -2900,12 +2904,9 @@ bool gh_try_launch_conv2d_bwd_data_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
   const int64_t wcount = (int64_t)g.F * g.K;
   const int64_t wbytes = (wcount * 8 + 255) / 256 * 256;
   if (g.strideH != 1 || g.strideW != 1 || padH < 0 || padW < 0) return false;
-  if (wbytes > ctx->workspace_bytes) return gh_ws_short(ctx, wbytes) != GH_OK;   // true: the caller returns ctx->err
   gh_cmd f{};
   f.opcode = GH_OP_CONV2D;
   f.flags = c.flags;
-  double* wt = (double*)((char*)ctx->workspace + ctx->workspace_bytes - wbytes);
-  f.ptr[0] = c.ptr[0]; f.ptr[1] = (uint64_t)(uintptr_t)wt; f.ptr[2] = c.ptr[2];
   f.dim[0] = c.dim[0]; f.dim[1] = g.F; f.dim[2] = g.oh; f.dim[3] = g.ow; f.dim[4] = g.C;
   f.dim[5] = g.kh; f.dim[6] = g.kw; f.dim[7] = padH; f.dim[8] = padW;
   f.dim[9] = 1; f.dim[10] = 1; f.dim[11] = g.dilH; f.dim[12] = g.dilW;
@@ -2913,6 +2914,15 @@ bool gh_try_launch_conv2d_bwd_data_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
   ConvGeom64 gf;
   if (!conv64_fill(f, &gf)) return false;
   if (gf.F < 16 || gf.P < 256 || gf.K < 8 || (int64_t)gf.P * gf.F * gf.K < (int64_t)1 << 22) return false;
+  // (what a fixed scratch refuses does not depend on the kernel)
+  if (wbytes > ctx->workspace_bytes && gh_ws_short(ctx, wbytes) != GH_OK) return true;   // the caller returns ctx->err
+  if (gh_conv_lanes_takes(c, true, ctx->cu_count, 0)) {
+    gh_launch_conv_lanes(ctx, c, true);
+    return true;
+  }
+  if (wbytes > ctx->workspace_bytes) return false;
+  double* wt = (double*)((char*)ctx->workspace + ctx->workspace_bytes - wbytes);
+  f.ptr[0] = c.ptr[0]; f.ptr[1] = (uint64_t)(uintptr_t)wt; f.ptr[2] = c.ptr[2];
   int64_t blocks = cdiv(wcount, 256);
   if (blocks > (int64_t)ctx->cu_count * 8) blocks = (int64_t)ctx->cu_count * 8;
   hipLaunchKernelGGL(k_flip_filters<double>, dim3((int)blocks), dim3(256), 0, ctx->stream,
@@ -3079,6 +3089,34 @@ static bool conv_direct_takes(const gh_cmd& c) {
   return true;
 }
 
+// What the kernels that k_conv3x3_lanes competes with take for a plain command, in us.  The patch kernel's estimate is
+// its own; the wide-image and the tiled kernel are fitted from above their quickest (100 TFLOP/s past 10 us; 8 x 16 x
+// 104 x 104 -> 32 takes 23, 3 x 16 x 49 x 49 -> 32 13, 8 x 16 x 208 x 208 -> 32 40).
+static double conv_others_us(const gh_cmd& c, int cus) {
+  if (gh_conv_patch_takes(c)) return gh_conv_patch_us(c, cus);
+  const double oh = (double)(c.dim[2] + 2 * c.dim[7] - 2), ow = (double)(c.dim[3] + 2 * c.dim[8] - 2);
+  return 10.0 + 18.0 * (double)c.dim[0] * (double)c.dim[1] * (double)c.dim[4] * oh * ow * 1e-8;
+}
+// float32, behind the single-channel, few-channel and small-image kernels, which win where they take a shape.
+static bool conv_lanes_takes(const gh_cmd& c, int cus) {
+  if (c.dim[5] != 3 || c.dim[6] != 3 || gh_conv_rows1_takes(c) || conv_direct_takes(c) || gh_conv_small_takes(c)) return false;
+  return gh_conv_lanes_takes(c, false, cus, conv_others_us(c, cus));
+}
+// The image gradient: elsewhere that is a launch that mirrors the filters (4.7 us) and a forward one over dy.
+static bool conv_lanes_takes_gradient(const gh_cmd& c, int cus) {
+  if (c.dim[5] != 3 || c.dim[6] != 3 || c.dim[11] != 1 || c.dim[12] != 1) return false;
+  gh_cmd f{};
+  f.opcode = GH_OP_CONV2D;
+  f.dim[0] = c.dim[0]; f.dim[1] = c.dim[4]; f.dim[2] = gh_conv_out(c.dim[2], 3, c.dim[7], 1, 1); f.dim[3] = gh_conv_out(c.dim[3], 3, c.dim[8], 1, 1);
+  f.dim[4] = c.dim[1]; f.dim[5] = f.dim[6] = 3; f.dim[7] = 2 - c.dim[7]; f.dim[8] = 2 - c.dim[8];
+  f.dim[9] = f.dim[10] = f.dim[11] = f.dim[12] = 1;
+  if (gh_conv_rows1_takes(f) || conv_direct_takes(f)) return false;
+  // the small-image kernels run at 55 TFLOP/s past 6 us (128 x 32 x 14 x 14 -> 64: 12.8 us and the mirroring)
+  const double others = gh_conv_small_takes(f) ? 6.0 + 18.0 * (double)f.dim[0] * (double)f.dim[1] * (double)f.dim[4] * (double)f.dim[2] * (double)f.dim[3] / 55e6
+                                               : conv_others_us(f, cus);
+  return gh_conv_lanes_takes(c, true, cus, others + 4.7);
+}
+
 static int launch_conv_direct(gh_ctx* ctx, const gh_cmd& c) {
   const int B = (int)c.dim[0], C = (int)c.dim[1], H = (int)c.dim[2], W = (int)c.dim[3], F = (int)c.dim[4];
   const int pad = (int)c.dim[7];
@@ -3136,6 +3174,7 @@ int gh_launch_conv2d(gh_ctx* ctx, const gh_cmd& c) {
   if (conv_direct_takes(c)) return launch_conv_direct(ctx, c);
   const int rcs = gh_try_launch_conv_small(ctx, c);
   if (rcs >= 0) return rcs;
+  if (conv_lanes_takes(c, ctx->cu_count)) return gh_launch_conv_lanes(ctx, c, false);
   const int rcp = gh_try_launch_conv_patch(ctx, c);
   if (rcp >= 0) return rcp;
   const int rcw = gh_try_launch_conv_wide(ctx, c);
@@ -3311,7 +3350,8 @@ int gh_launch_conv2d_bwd_data(gh_ctx* ctx, const gh_cmd& c) {
   const int padH = g.dilH * (g.kh - 1) - g.padH, padW = g.dilW * (g.kw - 1) - g.padW;
   const bool mirror_shape = g.strideH == 1 && g.strideW == 1 && padH >= 0 && padW >= 0;
   if (mirror_shape && wbytes > ctx->workspace_bytes / 2)
-    if (int rc = gh_ws_short(ctx, 2 * wbytes)) return rc;
+    if (int rc = gh_ws_short(ctx, 2 * wbytes)) return rc;   // (what a fixed scratch refuses does not depend on the kernel)
+  if (mirror_shape && conv_lanes_takes_gradient(c, ctx->cu_count)) return gh_launch_conv_lanes(ctx, c, true);
   if (mirror_shape && wbytes <= ctx->workspace_bytes / 2) {
     // mirrored filters live at the top of the workspace; the forward launch
     // below may use what is left of it for its own split-K slabs

@@ -326,7 +326,9 @@ GH_API int gh_conv2d_can_keep(const gh_cmd* conv);
  * The three route queries take no context: where a launcher's choice depends on the number of
  * compute units (the 1x1 kernel, the small-output product, the K slices of a product) they
  * answer for 256 of them, the MI355X's count; on a device with another count gh_submit may
- * choose differently there. */
+ * choose differently there.  The answer names the family a shape belongs to: within PATCH, WIDE and
+ * TILED, 3x3 stride-1 commands whose tiles would leave most of the device idle run on one kernel
+ * with its operands straight from memory (k_conv3x3_lanes) where its estimate is the lowest. */
 enum gh_conv_route {
   GH_CONV_ROUTE_DIRECT = 0,     /* 3x3, at most four channels: vector ALUs               */
   GH_CONV_ROUTE_SMALL = 1,      /* 3x3 over images up to 16 x 16, K split over wavefronts */
