@@ -3026,6 +3026,7 @@ static int direct_form(const gh_cmd& c, int cus) {
 int gh_launch_gemm(gh_ctx* ctx, const gh_cmd& c) {
   const int64_t batch = c.dim[6] <= 0 ? 1 : c.dim[6];
   if (gh_dtype_of(c.flags) == GH_F64) {
+    if (gh_gemm_thin_takes(c)) return gh_launch_gemm_thin(ctx, c);
     double us = 0;
     const int form = gh_gemm_direct_form(c, ctx->cu_count, &us);
     // one 16x16 tile per workgroup where larger tiles leave the device idle: 4.6 us per 1000 of K and 256 tiles
@@ -3034,6 +3035,7 @@ int gh_launch_gemm(gh_ctx* ctx, const gh_cmd& c) {
     if (batch == 1 && c.dim[2] >= 64 && (form < 0 || small < us)) return launch_dgemm_skinny(ctx, c);
     return form >= 0 ? gh_launch_gemm_direct(ctx, c, form) : launch_dgemm_skinny(ctx, c);
   }
+  if (gh_gemm_thin_takes(c)) return gh_launch_gemm_thin(ctx, c);
   const int rs = try_launch_gemm_skinny(ctx, c);
   if (rs >= 0) return rs;
   if (c.flags & GH_FLAG_GEMM_SOFTMAX)
@@ -3057,6 +3059,7 @@ extern "C" int gh_gemm_route(const gh_cmd* c, int* splits) {
   gh_ctx probe;
   probe.workspace = &probe;   // never dereferenced: only "there is one" and its size are read
   probe.workspace_bytes = 64ll << 20;
+  if (gh_gemm_thin_takes(*c)) return GH_GEMM_ROUTE_SMALL_OUTPUT;
   if (gemm_skinny_takes(*c, probe.cu_count)) {
     if (splits) *splits = skinny_slices(*c, probe.cu_count);
     return GH_GEMM_ROUTE_SMALL_OUTPUT;
