@@ -105,7 +105,7 @@ int gh_launch_dropout_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_dropout_bwd_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_softmax_bwd_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_maxpool2d_bwd_f64(gh_ctx* ctx, const gh_cmd& c);
-int gh_launch_solver_step_f64(gh_ctx* ctx, const gh_cmd& c);
+int gh_launch_solver_steps_f64(gh_ctx* ctx, const gh_cmd* cmds, int count);
 int gh_launch_bn_train_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_bn_bwd_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_conv2d_bwd_data_f64(gh_ctx* ctx, const gh_cmd& c);

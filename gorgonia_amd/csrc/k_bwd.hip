@@ -669,10 +669,11 @@ int gh_launch_softmax_bwd(gh_ctx* ctx, const gh_cmd& c) {
 // SOLVER_STEP commands with the same solver, options and hyper-parameters.
 int gh_solver_run_length(const gh_cmd* cmds, int n) {
   if (n <= 0 || cmds[0].opcode != GH_OP_SOLVER_STEP) return 0;
-  if (gh_dtype_of(cmds[0].flags) == GH_F64) return 1;   // float64 steps go one tensor per launch
+  // (float64 settings are bit patterns in dim[1..10], float32 ones are in f)
   int len = 1;
   while (len < n && len < kSolverBatch && cmds[len].opcode == GH_OP_SOLVER_STEP && cmds[len].flags == cmds[0].flags &&
-         cmds[len].ptr[4] == cmds[0].ptr[4] && memcmp(cmds[len].f, cmds[0].f, sizeof(cmds[0].f)) == 0) {
+         cmds[len].ptr[4] == cmds[0].ptr[4] && memcmp(cmds[len].f, cmds[0].f, sizeof(cmds[0].f)) == 0 &&
+         memcmp(cmds[len].dim + 1, cmds[0].dim + 1, sizeof(cmds[0].dim) - sizeof(cmds[0].dim[0])) == 0) {
     // a tensor stepped twice keeps its two steps in order: the run ends before the repeat
     bool repeat = false;
     for (int j = 0; j < len; j++) repeat = repeat || cmds[j].ptr[0] == cmds[len].ptr[0];
@@ -685,6 +686,7 @@ int gh_solver_run_length(const gh_cmd* cmds, int n) {
 // One launch for cmds[0..count) (count from gh_solver_run_length).
 int gh_launch_solver_steps(gh_ctx* ctx, const gh_cmd* cmds, int count) {
   const gh_cmd& c = cmds[0];
+  if (gh_dtype_of(c.flags) == GH_F64) return gh_launch_solver_steps_f64(ctx, cmds, count);
   const int kind = (int)gh_fn(c.flags), use = (int)gh_mode(c.flags);
   SolverPar p{c.f[0], c.f[1], c.f[2], c.f[3], c.f[4], c.f[5], c.f[6], c.f[7], c.f[8], c.f[9]};
   SolverBatch sb{};
@@ -718,7 +720,6 @@ int gh_launch_solver_steps(gh_ctx* ctx, const gh_cmd* cmds, int count) {
 }
 
 int gh_launch_solver_step(gh_ctx* ctx, const gh_cmd& c) {
-  if (gh_dtype_of(c.flags) == GH_F64) return gh_launch_solver_step_f64(ctx, c);
   return gh_launch_solver_steps(ctx, &c, 1);
 }
 
