@@ -107,6 +107,54 @@ __global__ __launch_bounds__(kBlock) void k_maxpool2d_bwd_f64(const double* __re
   }
 }
 
+// 2x2 / stride 2 / no padding: windows do not overlap, so one thread owns one - its four values read once, not by each
+// of the four - and the last column's (row's) thread zeroes what an odd extent leaves outside every window.  The scan
+// order, strict > and "0 + dy" of the kernel above.  VEC: rows of 16-byte pairs.  HBM-bound where it is not the launch.
+template <bool VEC>
+__global__ __launch_bounds__(kBlock) void k_maxpool_2x2s2_bwd_f64(const double* __restrict__ x, const double* __restrict__ dy,
+                                                                  double* __restrict__ dx, int H, int W, int64_t windows) {
+  typedef double V2 __attribute__((ext_vector_type(2)));
+  const int64_t stride = (int64_t)gridDim.x * kBlock;
+  const int oh = H / 2, ow = W / 2;
+  for (int64_t idx = (int64_t)blockIdx.x * kBlock + threadIdx.x; idx < windows; idx += stride) {
+    const int64_t row = idx / ow;
+    const int pw = (int)(idx - row * ow);
+    const int64_t bc = row / oh;
+    const int ph = (int)(row - bc * oh);
+    const int64_t at = (bc * H + 2 * ph) * (int64_t)W + 2 * pw;
+    V2 r0, r1;
+    if (VEC) {
+      r0 = *reinterpret_cast<const V2*>(x + at);
+      r1 = *reinterpret_cast<const V2*>(x + at + W);
+    } else {
+      r0 = V2{x[at], x[at + 1]};
+      r1 = V2{x[at + W], x[at + W + 1]};
+    }
+    double best = -DBL_MAX;
+    int arg = -1;
+    if (r0[0] > best) { best = r0[0]; arg = 0; }
+    if (r0[1] > best) { best = r0[1]; arg = 1; }
+    if (r1[0] > best) { best = r1[0]; arg = 2; }
+    if (r1[1] > best) { best = r1[1]; arg = 3; }
+    const double v = 0.0 + dy[idx];
+    const V2 o0 = {arg == 0 ? v : 0.0, arg == 1 ? v : 0.0}, o1 = {arg == 2 ? v : 0.0, arg == 3 ? v : 0.0};
+    if (VEC) {
+      *reinterpret_cast<V2*>(dx + at) = o0;
+      *reinterpret_cast<V2*>(dx + at + W) = o1;
+    } else {
+      dx[at] = o0[0]; dx[at + 1] = o0[1];
+      dx[at + W] = o1[0]; dx[at + W + 1] = o1[1];
+    }
+    const bool right = (W & 1) && pw == ow - 1;
+    if (right) { dx[at + 2] = 0.0; dx[at + W + 2] = 0.0; }
+    if ((H & 1) && ph == oh - 1) {
+      dx[at + 2 * (int64_t)W] = 0.0;
+      dx[at + 2 * (int64_t)W + 1] = 0.0;
+      if (right) dx[at + 2 * (int64_t)W + 2] = 0.0;
+    }
+  }
+}
+
 // ---- BatchNorm training forward and gradient (op_nn.go:1489-1635, 1834-1943) -------------
 // One workgroup per channel: the channel's n = B*S values are summed by a fixed
 // tree (thread-strided partial sums, then a tree over the 256 threads), so
@@ -341,6 +389,17 @@ int gh_launch_maxpool2d_bwd_f64(gh_ctx* ctx, const gh_cmd& c) {
   g.padW = (int)(explicit_pad ? padE : padW);
   const int64_t total = B * C * g.H * g.W;
   if (total == 0) return GH_OK;
+  if (g.kh == 2 && g.kw == 2 && g.strideH == 2 && g.strideW == 2 && padN == 0 && padS == 0 && padW == 0 && padE == 0 && g.H >= 2 && g.W >= 2) {
+    const int64_t windows = B * C * (int64_t)g.oh * g.ow;
+    const bool vec = g.W % 2 == 0 && ((c.ptr[0] | c.ptr[2]) & 15) == 0;
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(blocks_for(ctx, windows)), dim3(kBlock), 0, ctx->stream, (const double*)(uintptr_t)c.ptr[0],
+                         (const double*)(uintptr_t)c.ptr[1], (double*)(uintptr_t)c.ptr[2], g.H, g.W, windows);
+    };
+    if (vec) go(k_maxpool_2x2s2_bwd_f64<true>);
+    else go(k_maxpool_2x2s2_bwd_f64<false>);
+    return gh_check_hip(ctx, hipGetLastError(), "maxpool backward launch");
+  }
   hipLaunchKernelGGL(k_maxpool2d_bwd_f64, dim3(blocks_for(ctx, total)), dim3(kBlock), 0, ctx->stream,
                      (const double*)(uintptr_t)c.ptr[0], (const double*)(uintptr_t)c.ptr[1],
                      (double*)(uintptr_t)c.ptr[2], g, total);
