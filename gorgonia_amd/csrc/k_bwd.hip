@@ -243,9 +243,9 @@ __global__ __launch_bounds__(kBlock) void k_bn_reduce(const float* __restrict__ 
 
 // y = x a + b with a = 1/sqrt(batch_var + eps), b = -mean a (op_nn.go:1573-1584, the inference kernel's arithmetic), one
 // (image, channel) plane per blockIdx.y.  Every workgroup adds its channel's partial sums up for itself, which costs less
-// than the launch that did it for all (8 x 16 x 208 x 208: 12.5 us for 8.8 + 4.9; 8 x 128 x 26 x 26: 4.9 for 3.8 + 4.9); the first workgroup of the channel's first plane keeps
-// save_mean, save_var (the SUM of squared deviations, as the reference keeps it) and the running statistics (momentum
-// weights the NEW value; unbiased variance, op_nn.go:1547-1550).
+// than the launch that did it for all (8 x 16 x 208 x 208: 12.5 us for 8.8 + 4.9; 8 x 128 x 26 x 26: 4.9 for 3.8 + 4.9);
+// the first workgroup of the channel's first plane keeps save_mean, save_var (the SUM of squared deviations, as the
+// reference keeps it) and the running statistics (momentum weights the NEW value; unbiased variance, op_nn.go:1547-1550).
 // (One pass for sums and squares, with the groups' deviations about their own means, was measured: another 9 us on four
 // layers of 8 images, for statistics that round differently from the two passes'.)
 template <bool VEC>

@@ -3093,12 +3093,14 @@ static bool conv_direct_takes(const gh_cmd& c) {
 }
 
 // What the kernels that k_conv3x3_lanes competes with take for a plain command, in us.  The patch kernel's estimate is
-// its own; the wide-image and the tiled kernel are fitted from above their quickest (100 TFLOP/s past 10 us; 8 x 16 x
-// 104 x 104 -> 32 takes 23, 3 x 16 x 49 x 49 -> 32 13, 8 x 16 x 208 x 208 -> 32 40).
+// its own; the wide-image kernel's is fitted from above its quickest (8 x 16 x 208 x 208 -> 32 takes 40, 8 x 16 x 104 x
+// 104 -> 32 23, 2 x 16 x 104 x 104 -> 32 11), the tiled one's to 23 for 8 x 32 x 52 x 52 -> 64, 17 for two such images,
+// 13 for 3 x 16 x 49 x 49 -> 32.
 static double conv_others_us(const gh_cmd& c, int cus) {
   if (gh_conv_patch_takes(c)) return gh_conv_patch_us(c, cus);
   const double oh = (double)(c.dim[2] + 2 * c.dim[7] - 2), ow = (double)(c.dim[3] + 2 * c.dim[8] - 2);
-  return 10.0 + 18.0 * (double)c.dim[0] * (double)c.dim[1] * (double)c.dim[4] * oh * ow * 1e-8;
+  const double flops = 18.0 * (double)c.dim[0] * (double)c.dim[1] * (double)c.dim[4] * oh * ow;
+  return gh_conv_wide_takes(c) ? 10.0 + flops * 1e-8 : 12.0 + flops / 75e6;
 }
 // float32, behind the single-channel, few-channel and small-image kernels, which win where they take a shape.
 static bool conv_lanes_takes(const gh_cmd& c, int cus) {
