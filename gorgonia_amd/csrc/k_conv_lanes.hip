@@ -305,6 +305,9 @@ static int quickest(const gh_cmd& c, bool flip, bool f64, int cus, double* us) {
   int best = -1;
   for (int i = 0; i < 3; i++) {
     const Form& f = (f64 ? kForms64 : kForms32)[i];
+    // an image gradient gains nothing from the form that halves the wavefronts (8 x 32 x 52 x 52 <- 64: 14.5 us, 14.0 with
+    // eight), and would add twice as many terms in a row
+    if (!f64 && flip && f.waves == 4) continue;
     const int64_t per = 16 * f.groups * (f.split ? 1 : f.waves);
     const int64_t tiles = (F + 16 * f.tm - 1) / (16 * f.tm) * ((lines * ((ow + f.v - 1) / f.v) + per - 1) / per);
     // one tile of four wavefronts to a compute unit waits for its loads
