@@ -1,4 +1,4 @@
-// Products of one to eight rows with a row-major matrix: y[m][:] = x[m][:] . B, float32 and float64.
+// Products of one to four rows (float64: one or two) with a row-major matrix: y[m][:] = x[m][:] . B, float32 and float64.
 //
 // A pass over B and nothing else, so a workgroup takes 16 columns (of float64 the same 16) and all of K: lane (kk, cg)
 // of a wavefront reads four neighbouring columns of every 128th row, 4 rows or more in flight, and the 128 partial sums
@@ -90,18 +90,23 @@ int launch(gh_ctx* ctx, const gh_cmd& c) {
   };
   if (M == 1) go(k_gemm_thin<T, 1>);
   else if (M == 2) go(k_gemm_thin<T, 2>);
-  else if (M <= 4) go(k_gemm_thin<T, 4>);
-  else go(k_gemm_thin<T, 8>);
+  else if constexpr (sizeof(T) == 4) go(k_gemm_thin<T, 4>);
   return gh_check_hip(ctx, hipGetLastError(), "thin gemm launch");
 }
 
 }  // namespace
 
-// One product of up to eight rows, operands as they lie, wider than a softmax in a product's epilogue (up to 32
-// columns: the fused and the separate softmax see the same product bits there), K long enough for a row per lane.
+// One product of up to four rows (two of float64: every row adds its partial sums' way through the wavefront, and at
+// eight rows, 8 x 300 x 100, that made 7.3 us of 4.9), operands as they lie, wider than a softmax in a product's epilogue
+// (up to 32 columns: the fused and the separate softmax see the same product bits there) and not so wide that 32-column
+// tiles fill the device (1 x 1000 x 8000: 14.3 us against 12.3), K long enough for a row per lane, with several rows for
+// two (4 x 64 x 100: 4.8 us against 3.9; 4 x 300 x 100 4.8 and 4.9; 4 x 784 x 300 5.4 against 8.4) and, where few
+// workgroups share the columns, not so long that cutting it over workgroups pays for a second launch.
 bool gh_gemm_thin_takes(const gh_cmd& c) {
   if (c.dim[6] > 1 || (c.flags & (GH_FLAG_TRANS_A | GH_FLAG_TRANS_B | GH_FLAG_GEMM_SOFTMAX))) return false;
-  return c.dim[0] >= 1 && c.dim[0] <= 8 && c.dim[1] > 32 && c.dim[1] <= 8192 && c.dim[2] >= 64 && !getenv("GORGONIA_HIP_GEMM_PLAN");
+  const int64_t rows = gh_dtype_of(c.flags) == GH_F64 ? 2 : 4;
+  return c.dim[0] >= 1 && c.dim[0] <= rows && c.dim[1] > 32 && c.dim[1] <= 4096 && c.dim[2] >= (c.dim[0] == 1 ? 64 : 256) && (c.dim[2] <= 4096 || c.dim[1] >= 2048) &&
+         !getenv("GORGONIA_HIP_GEMM_PLAN");
 }
 int gh_launch_gemm_thin(gh_ctx* ctx, const gh_cmd& c) {
   return gh_dtype_of(c.flags) == GH_F64 ? launch<double>(ctx, c) : launch<float>(ctx, c);

@@ -10,9 +10,9 @@ from tests.util import rel_frobenius
 
 pytestmark = pytest.mark.gpu
 
-# m, n, k: one tile and few, rows below and above sixteen, k one below and at the first cut, ragged, not a multiple of
+# m, n, k: one tile and few, rows below and above sixteen (up to four of wide products run elsewhere), k one below and at the first cut, ragged, not a multiple of
 # the slices' chunks, so long that the device is full
-SHAPES = [(8, 10, 21632), (1, 300, 2048), (1, 1, 2047), (20, 30, 4001), (64, 10, 4096), (16, 16, 2048), (33, 32, 2500), (7, 45, 5003),
+SHAPES = [(8, 10, 21632), (9, 300, 2048), (1, 1, 2047), (20, 30, 4001), (64, 10, 4096), (16, 16, 2048), (33, 32, 2500), (7, 45, 5003),
           (100, 17, 3333), (512, 32, 2064)]
 
 

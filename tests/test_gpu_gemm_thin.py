@@ -1,4 +1,4 @@
-"""k_gemm_thin: products of one to eight rows, at the edges of its column groups, rounds of K and row counts, against
+"""k_gemm_thin: products of one to four rows (and more, which it leaves), at the edges of its column groups, rounds of K and row counts, against
 float64 products."""
 import numpy as np
 import pytest
