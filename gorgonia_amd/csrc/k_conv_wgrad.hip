@@ -20,6 +20,7 @@
 //     workgroups' slabs in k_slab_sum, both in a fixed order.
 // P is 4, or 2 where a row has at most eight columns.
 #include <algorithm>
+#include <type_traits>
 
 #include "gh_internal.h"
 
@@ -134,7 +135,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   for (int m = 0; m < TM; m++)
 #pragma unroll
     for (int n = 0; n < NT; n++) acc[m][n] = Acc{(T)0, (T)0, (T)0, (T)0};
-  auto multiply = [&](int b, int oy, int ch, Frag& f) {
+  // A column past the row has to be zero on both sides: zero times an infinity or NaN of x is NaN.  A lane past the row
+  // holds zeros, but where a lane's columns reach past the row, x values that taps 1 and 2 of the row's last columns read
+  // meet the zero dy of the columns past it under another tap.  The walk notes whether there was one that was not finite
+  // (`odd` is NaN then), and if so the wavefront walks its chunks again, choosing x for every step.  (The choice takes 8 to
+  // 20 % of the kernel where every chunk makes it, 3 to 25 % where the rows' last ones do, the note 0 to 4 %: 128 -> 256
+  // over 8 x 52 x 52 170 us without either, 206, 192 and 171; 308 -> 66 over 26 x 29 x 29 148, 180, 175 and 153.)
+  T odd = (T)0;
+  auto multiply = [&](auto exact, int b, int oy, int ch, Frag& f) {
     const int ox = (ch * 4 + q) * P;
     if (b == 0 || b == last_image) {   // the only images with loads that stick out of the tensors
 #pragma unroll
@@ -154,34 +162,39 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         for (int n = 0; n < NT; n++) {
           const int iy = oy + ky[n] - g.padH, ix = ox + kx[n] - g.padW;
           const bool row = iy >= 0 && iy < g.H;
+          const int end = row ? min(g.W - ix, g.ow - ox) : 0;   // the image's and the row's
 #pragma unroll
-          for (int t = 0; t < P; t++) f.b[n * P + t] = row && ix + t >= 0 && ix + t < g.W ? f.b[n * P + t] : (T)0;
+          for (int t = 0; t < P; t++) f.b[n * P + t] = t >= -ix && t < end ? f.b[n * P + t] : (T)0;
         }
       } else {
         const int ix = ox - g.padW;
+        const int end = ox < g.ow ? g.W - ix : 0;   // the image's; a lane that is past the row has none
 #pragma unroll
         for (int r = 0; r < 3; r++) {
           const bool row = oy + r - g.padH >= 0 && oy + r - g.padH < g.H;
 #pragma unroll
-          for (int t = 0; t < P + 2; t++)
-            f.b[r * (P + 2) + t] = row && ix + t >= 0 && ix + t < g.W ? f.b[r * (P + 2) + t] : (T)0;
+          for (int t = 0; t < P + 2; t++) f.b[r * (P + 2) + t] = row && t >= -ix && t < end ? f.b[r * (P + 2) + t] : (T)0;
+        }
+        if (!decltype(exact)::value && g.ow % P != 0 && (ch + 1) * 4 * P > g.ow) {
+#pragma unroll
+          for (int k = 0; k < NB; k++) odd = odd + f.b[k] * (T)0;
         }
       }
     }
 #pragma unroll
     for (int t = 0; t < P; t++)
 #pragma unroll
-      for (int n = 0; n < NT; n++)
+      for (int n = 0; n < NT; n++) {
+        T bv = kPacked ? f.b[n * P + t] : f.b[(n / 3) * (P + 2) + t + n % 3];
+        if constexpr (decltype(exact)::value) bv = ox + t < g.ow ? bv : (T)0;
 #pragma unroll
-        for (int m = 0; m < TM; m++) {
-          const T bv = kPacked ? f.b[n * P + t] : f.b[(n / 3) * (P + 2) + t + n % 3];
-          acc[m][n] = Mfma<T>::run(f.a[m][t], bv, acc[m][n]);
-        }
+        for (int m = 0; m < TM; m++) acc[m][n] = Mfma<T>::run(f.a[m][t], bv, acc[m][n]);
+      }
   };
 
   const int first = (int)min((int64_t)(blockIdx.x * kWaves + wave) * g.per, (int64_t)g.items);
   const int count = min(g.per, g.items - first);
-  if (count > 0) {
+  auto walk = [&](auto exact) {
     int ch = first % g.nch, row = first / g.nch;   // row of the batch
     int b = row / g.oh, oy = row - b * g.oh;
     auto next = [&]() {
@@ -197,8 +210,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
       const int b0 = b, oy0 = oy, ch0 = ch;
       if (k + 1 < count) next();
       load(b, oy, ch, ahead);   // (past the end the last chunk again: no branch around a load)
-      multiply(b0, oy0, ch0, cur);
+      multiply(exact, b0, oy0, ch0, cur);
       cur = ahead;
+    }
+  };
+  if (count > 0) {
+    walk(std::false_type{});
+    if (!kPacked && __any(odd != odd)) {
+#pragma unroll
+      for (int m = 0; m < TM; m++)
+#pragma unroll
+        for (int n = 0; n < NT; n++) acc[m][n] = Acc{(T)0, (T)0, (T)0, (T)0};
+      walk(std::true_type{});
     }
   }
 

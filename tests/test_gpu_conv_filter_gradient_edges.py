@@ -1,0 +1,74 @@
+"""The 3x3 stride-1 filter gradient where a value must not be touched: infinities and NaN beside the columns a row
+does not have.  Against the sum over shifted, zero-padded images in float64, in which such a value reaches the taps that
+read it and no other."""
+import numpy as np
+import pytest
+
+from gorgonia_amd import _ffi
+from gorgonia_amd import device as D
+from tests.util import rel_frobenius
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = D.Context(0, 0)
+    yield c
+    c.close()
+
+
+def _reference(x, dy, pad):
+    B, C, H, W = x.shape
+    F, oh, ow = dy.shape[1:]
+    xp = np.zeros((B, C, H + 2 * pad[0], W + 2 * pad[1]))
+    xp[:, :, pad[0]:pad[0] + H, pad[1]:pad[1] + W] = x
+    out = np.empty((F, C, 3, 3))
+    d = dy.astype(np.float64).transpose(1, 0, 2, 3).reshape(F, -1)
+    for ky in range(3):
+        for kx in range(3):
+            out[:, :, ky, kx] = d @ xp[:, :, ky:ky + oh, kx:kx + ow].transpose(1, 0, 2, 3).reshape(C, -1).T
+    return out
+
+
+def _compare(ctx, x, dy, pad, code):
+    B, C, H, W = x.shape
+    F = dy.shape[1]
+    px, pg, pw = ctx.upload(x), ctx.upload(dy), ctx.upload(np.full((F, C, 3, 3), np.nan, x.dtype))
+    ctx.run(D.cmd_conv2d_bwd_filter(px, pg, pw, B, C, H, W, F, 3, 3, pad, dtype=code))
+    got = ctx.d2h(pw, (F, C, 3, 3), x.dtype)
+    for p in (px, pg, pw):
+        ctx.free(p)
+    with np.errstate(invalid="ignore"):
+        want = _reference(x, dy, pad)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], want[inf])
+    finite = np.isfinite(want)
+    # the bars of the engine's products (random signs leave the root of the chain length in units of 2^-24, 2^-53)
+    assert rel_frobenius(got[finite], want[finite]) <= (1e-5 if code == _ffi.F32 else 1e-13)
+
+
+# B, C, H, W, F, pad: rows that end inside a chunk of 16 (8) columns, by one and by several; packed columns (up to
+# eight channels) and channel tiles; no padding, and padding that puts the image's end before the row's
+RAGGED = [(2, 16, 26, 26, 32, 1), (2, 20, 20, 18, 40, 0), (1, 16, 40, 52, 16, 1), (2, 17, 24, 17, 24, 2), (3, 12, 30, 19, 48, 3),
+          (2, 8, 40, 37, 16, 1), (2, 5, 60, 35, 24, 0)]
+RAGGED_F64 = RAGGED + [(12, 32, 7, 7, 16, 1), (4, 64, 14, 14, 32, 1), (2, 1, 28, 28, 32, 1), (12, 16, 9, 9, 16, 0)]
+
+
+@pytest.mark.parametrize("where", ["x", "dy"])
+@pytest.mark.parametrize("dt,cfg", [("f32", c) for c in RAGGED] + [("f64", c) for c in RAGGED_F64])
+def test_infinities_and_nan_at_the_ends_of_rows(ctx, dt, cfg, where):
+    np_dt, code = (np.float32, _ffi.F32) if dt == "f32" else (np.float64, _ffi.F64)
+    B, C, H, W, F, pad = cfg
+    oh, ow = H + 2 * pad - 2, W + 2 * pad - 2
+    rng = np.random.default_rng(W * 10 + pad)
+    x = rng.uniform(-1, 1, (B, C, H, W)).astype(np_dt)
+    dy = rng.uniform(-1, 1, (B, F, oh, ow)).astype(np_dt)
+    if where == "x":   # a channel each: the last column, the one before it, the first; the other channels stay finite
+        for c, (col, v) in enumerate(((W - 1, np.inf), (W - 2, -np.inf), (0, np.nan), (W - 1, np.nan))[:max(1, C - 1)]):
+            x[(c + 1) % B, c, H // 2 + c, col] = v
+    else:              # a filter each: the ends of a row, and the first column, which lies behind the row above
+        for f, (col, v) in enumerate(((ow - 1, np.inf), (0, np.nan), (0, -np.inf))):
+            dy[(f + 1) % B, f, oh // 2, col] = v
+    _compare(ctx, x, dy, (pad, pad), code)
