@@ -297,9 +297,9 @@ bool fill(const gh_cmd& c, Wg<T>* g) {
   if (H > (1 << 20) || W > (1 << 20) || C > (1 << 20) || F > 65535 * 16) return false;
   g->x = (const T*)(uintptr_t)c.ptr[0];
   g->dy = (const T*)(uintptr_t)c.ptr[1];
-  // 32-bit byte offsets; whole loads inside the tensors
+  // 32-bit byte offsets; an image holds a whole load, so that none but the first and last image's stick out of a tensor
   const int64_t most = ((int64_t)1 << 31) / (int64_t)sizeof(T) - 64;
-  if (B * C * H > most / W || B * F * oh > most / ow || B * C * H * W < 6 || B * F * oh * ow < 4) return false;
+  if (B * C * H > most / W || B * F * oh > most / ow || C * H * W < 6 || F * oh * ow < 4) return false;
   g->x_total = (int)(B * C * H * W);
   g->dy_total = (int)(B * F * oh * ow);
   g->B = (int)B; g->C = (int)C; g->H = (int)H; g->W = (int)W; g->F = (int)F; g->oh = (int)oh; g->ow = (int)ow;

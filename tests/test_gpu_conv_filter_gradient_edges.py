@@ -1,6 +1,6 @@
 """The 3x3 stride-1 filter gradient where a value must not be touched: infinities and NaN beside the columns a row
-does not have.  Against the sum over shifted, zero-padded images in float64, in which such a value reaches the taps that
-read it and no other."""
+does not have, and images of a handful of values.  Against the sum over shifted, zero-padded images in float64, in
+which such a value reaches the taps that read it and no other."""
 import numpy as np
 import pytest
 
@@ -72,3 +72,22 @@ def test_infinities_and_nan_at_the_ends_of_rows(ctx, dt, cfg, where):
         for f, (col, v) in enumerate(((ow - 1, np.inf), (0, np.nan), (0, -np.inf))):
             dy[(f + 1) % B, f, oh // 2, col] = v
     _compare(ctx, x, dy, (pad, pad), code)
+
+
+# B, C, H, W, F, padH, padW: up to six values in an image, rows made of padding
+TINY = [(40, 1, 1, 2, 8, 1, 5), (40, 2, 1, 2, 8, 1, 5), (40, 1, 2, 2, 9, 1, 6), (40, 1, 1, 3, 16, 1, 5), (60, 3, 1, 1, 8, 1, 5),
+        (60, 4, 1, 1, 8, 1, 8), (40, 1, 1, 5, 8, 1, 4), (40, 1, 2, 3, 8, 1, 5), (40, 5, 1, 1, 8, 1, 6), (30, 1, 2, 1, 8, 3, 7)]
+
+
+@pytest.mark.parametrize("dt", ["f32", "f64"])
+@pytest.mark.parametrize("cfg", TINY)
+def test_images_of_a_few_values(ctx, cfg, dt):
+    np_dt, code = (np.float32, _ffi.F32) if dt == "f32" else (np.float64, _ffi.F64)
+    B, C, H, W, F, padH, padW = cfg
+    oh, ow = H + 2 * padH - 2, W + 2 * padW - 2
+    if dt == "f32":   # enough pixels for the matrix-core kernel
+        B = -(-70000 // (oh * ow))
+    rng = np.random.default_rng(B + W)
+    x = rng.uniform(-1, 1, (B, C, H, W)).astype(np_dt)
+    dy = rng.uniform(-1, 1, (B, F, oh, ow)).astype(np_dt)
+    _compare(ctx, x, dy, (padH, padW), code)
