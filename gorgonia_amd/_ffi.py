@@ -91,6 +91,7 @@ SYMBOLS = {
     "gh_submit": (C.c_int, [_P, C.POINTER(GhCmd), C.c_int]),
     "gh_submit_noalloc": (C.c_int, [_P, C.POINTER(GhCmd), C.c_int]),
     "gh_validate": (C.c_int, [C.POINTER(GhCmd), C.c_int, C.c_char_p, C.c_int]),
+    "gh_elementwise_run": (C.c_int, [C.POINTER(GhCmd), C.c_int]),
     "gh_conv2d_can_pool": (C.c_int, [C.POINTER(GhCmd)]),
     "gh_conv2d_can_pre": (C.c_int, [C.POINTER(GhCmd)]),
     "gh_conv2d_can_keep": (C.c_int, [C.POINTER(GhCmd)]),

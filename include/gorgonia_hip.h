@@ -304,6 +304,11 @@ GH_API int gh_submit(gh_ctx* ctx, const gh_cmd* cmds, int n);
 GH_API int gh_submit_noalloc(gh_ctx* ctx, const gh_cmd* cmds, int n);
 /* Validate only: same checks as gh_submit, touches no device. */
 GH_API int gh_validate(const gh_cmd* cmds, int n, char* msg, int msg_len);
+/* How many of the n commands, from the first on, gh_submit executes as one pass: 1, or the length of a run
+ * of elementwise commands on tensors of one size and type (the bits are those of the commands one by one).
+ * Host only, and for valid commands.  The reference launches a kernel per operator (cuda/arith.go:62); a
+ * caller that times one operator by submitting it several times asks here whether it still does. */
+GH_API int gh_elementwise_run(const gh_cmd* cmds, int n);
 /* 1 when this CONV2D command may carry GH_FLAG_CONV_POOL2 (a convolution whose
  * kernel keeps a whole pooling window in one thread), else 0.  Host only.  The
  * reference has no fused form: this folds maxpool.CUDADo
