@@ -352,7 +352,31 @@ bool plan(const Elem* e, int count, int item, Chain* c) {
 // what the other wrote, save a quarter: 36 against 45 us; two that only read the same tensor: 42 against 41).
 constexpr int64_t kLaunchBound = 16 << 20;
 
+// What a command earns by joining a run, in percent of the launch (of large tensors: the pass over memory) that a run
+// costs.  A function of few instructions earns the whole of its own launch or pass.  One of many costs more in the run than
+// by itself, a call for each of a thread's elements in turn, and the long ones as much as they save: two in one launch
+// against two launches, float32, 2^10 to 2^24 elements: sin, cos, ln, log2 0.87 to 1.0 times as fast, log1p 0.80 to 1.0,
+// softplus 0.65 to 1.06, pow 0.52 to 0.96, exp and expm1 1.14 to 1.07 below 4 MiB and 0.90 to 1.0 from there;
+// float64: pow 0.79 to 0.98, softplus 0.90 to 1.15, tanh 0.98 to 1.1, the others above 1.06.  With one command of few
+// instructions all gain (1.0 to 1.7) but float32 pow below 16 MiB (x * y, then pow: 0.81 to 0.95), which two of them carry.
+// A scalar exponent is 2 more often than not, which makes pow a product: only the kernel knows.
+int earns(const Elem& x, int item) {
+  const bool f64 = item == 8, small = x.n * item < (4 << 20), large = x.n * item >= (16 << 20);
+  switch (x.fn) {
+    case GH_POW: return x.scalar_b ? 50 : f64 ? 10 : large ? 27 : -55;
+    case kUnary + GH_SOFTPLUS: return f64 ? (small ? 45 : 55) : large ? 55 : small ? 0 : 45;
+    case kUnary + GH_TANH: return f64 ? 55 : 105;
+    case kUnary + GH_EXP: case kUnary + GH_EXPM1: return f64 ? 105 : small ? 75 : 45;
+    case kUnary + GH_LOG1P: return f64 ? 60 : small ? 28 : 45;
+    case kUnary + GH_SIN: case kUnary + GH_COS: case kUnary + GH_LN: case kUnary + GH_LOG2: return f64 ? 105 : 45;
+    default: return 105;
+  }
+}
+
 bool pays(const Elem* e, int count, int item, const Chain& c) {
+  int earned = 0;
+  for (int k = 0; k < count; k++) earned += earns(e[k], item);
+  if (earned <= 100) return false;
   if (e[0].n * item <= (count >= 4 ? 2 : 1) * kLaunchBound) return true;
   int apart = 0, together = 0;   // tensors read and written
   for (int k = 0; k < count; k++) {

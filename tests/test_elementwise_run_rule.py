@@ -58,3 +58,31 @@ def test_what_is_no_run():
     assert _run([neg, D.cmd_unary("neg", y + 4, n, dst=z)]) == 1                     # no whole vectors
     assert _run([neg, D.cmd_softmax(y, z, 64, 64)]) == 1
     assert _ffi.load().gh_elementwise_run(None, 0) == 0
+
+
+@pytest.mark.parametrize("dtype,item", [(_ffi.F32, 4), (_ffi.F64, 8)])
+@pytest.mark.parametrize("mib", [0.01, 1, 4, 16, 64])
+def test_long_functions(dtype, item, mib):
+    """Functions of many instructions cost a run as much as the launch they save: two of them do not make one."""
+    n = int(mib * MIB) // item
+    x, y, z, t, two = _tensors(5, n, item)
+    f32 = dtype == _ffi.F32
+
+    def twice(fn, times=2):
+        return [D.cmd_unary(fn, x, n, dtype=dtype, dst=z)] + [D.cmd_unary(fn, z, n, dtype=dtype)] * (times - 1)
+    for fn in ("sin", "cos", "ln", "log2", "log1p"):
+        assert _run(twice(fn)) == (1 if f32 else 2), fn
+    for fn in ("exp", "expm1"):
+        assert _run(twice(fn)) == (1 if f32 and mib >= 4 else 2), fn
+    assert _run(twice("softplus")) == (1 if mib < (16 if f32 else 4) else 2)
+    for fn in ("neg", "sqrt", "inverse", "sigmoid", "tanh"):
+        assert _run(twice(fn)) == 2, fn
+    assert _run(twice("sin", 3)) == 3 and _run(twice("exp", 3)) == 3
+    for fn in ("sin", "exp", "softplus", "log1p"):   # with one of few instructions all of them do
+        assert _run([D.cmd_unary("abs", x, n, dtype=dtype, dst=z), D.cmd_unary(fn, z, n, dtype=dtype)]) == 2, fn
+    mul, add = D.cmd_bin("mul", "vv", x, y, n, dtype=dtype, dst=z), D.cmd_bin("add", "vv", z, y, n, dtype=dtype)
+    power, square = D.cmd_bin("pow", "vv", z, y, n, dtype=dtype), D.cmd_bin("pow", "vs", z, two, n, dtype=dtype)
+    assert _run([mul, power]) == (1 if f32 and mib < 16 else 2)
+    assert _run([mul, add, power]) == 3
+    assert _run([power, power]) == 1
+    assert _run([mul, square]) == 2 and _run([square, square]) == 1
