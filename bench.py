@@ -14,6 +14,7 @@ as a reported baseline.  Prints ONE JSON line.
 from __future__ import annotations
 
 import argparse
+import ctypes as C
 import json
 import os
 import sys
@@ -57,7 +58,16 @@ SUSTAIN_MS = 40.0   # a kernel is timed after this much back-to-back work of its
 IN_FLIGHT = 32      # graph replays queued between two host waits of the sustained loop
 
 
-def time_cmds(ctx, cmds, iters, warm=3):
+def submit_passes(ctx, cmds, passes, as_one):
+    """`passes` times the commands, each in a submit of its own - elementwise commands of one submit may be
+    executed as one pass over memory, and then it is not the named kernel that runs - or, with as_one, a
+    submit per pass, the way a program issues them."""
+    for _ in range(passes):
+        for part in ([cmds] if as_one else [[c] for c in cmds]):
+            ctx.submit(part)
+
+
+def time_cmds(ctx, cmds, iters, warm=3, as_one=False):
     """Average milliseconds per pass over `cmds`: `iters` passes are captured into one hipGraph
     (so host enqueue time is out of the picture) and replays are bracketed by HIP events on the
     engine's stream.
@@ -68,16 +78,16 @@ def time_cmds(ctx, cmds, iters, warm=3):
     case, so the graph is first replayed for SUSTAIN_MS, then timed over at least SUSTAIN_MS.
     The first replay after the capture - the short-burst figure - is kept in
     time_cmds.last_burst_ms."""
-    ctx.submit(list(cmds) * warm)
+    submit_passes(ctx, cmds, warm, as_one)
     ctx.sync()
     if EAGER_TIMING:
         ctx.event(0)
-        ctx.submit(list(cmds) * iters)
+        submit_passes(ctx, cmds, iters, as_one)
         ctx.event(1)
         time_cmds.last_burst_ms = ctx.elapsed_ms(0, 1) / iters
         return time_cmds.last_burst_ms
     ctx.graph_begin()
-    ctx.submit(list(cmds) * iters)
+    submit_passes(ctx, cmds, iters, as_one)
     gid = ctx.graph_end()
     ctx.graph_launch(gid)
     ctx.sync()
@@ -173,12 +183,17 @@ def bench_elementwise(ctx, iters):
     no_arith = {"us": round(ms_neg * 1e3, 2), "GBps": round(2 * 4 * N / ms_neg / 1e6, 1),
                 "frac_hbm": round(2 * 4 * N / ms_neg / 1e6 / HBM_PEAK_GBPS, 4), "bytes": 2 * 4 * N,
                 "kernel": "Neg, same tensors and rotation as Sigmoid"}
-    # the chain as configuration 2 issues it - five launches in order on one set of tensors
-    # (x, y, z, t, p: 320 MiB, intermediates re-read straight after they were written)
+    # the chain as configuration 2 issues it - five commands in one submit on one set of tensors, which the
+    # library executes in chain_in_sequence_launches passes: x, y and the bias in, z, t and p out, once each
     z, t, p = ys[1], ps[0], ps[1]
     seq = [D.cmd_bin("mul", "vv", xs[0], ys[0], N, dst=z), D.cmd_bcast("add", z, z, b, 4096, 4096, 1),
            D.cmd_unary("sigmoid", z, N), D.cmd_unary("tanh", z, N, dst=t), D.cmd_bin("pow", "vs", z, two, N, dst=p)]
-    ms_seq = time_cmds(ctx, seq, max(4, iters // 3))
+    ms_seq = time_cmds(ctx, seq, max(4, iters // 3), as_one=True)
+    seq_bytes = 5 * 4 * N + 4 * 4096
+    seq_array, seq_launches, at = (D.GhCmd * len(seq))(*seq), 0, 0
+    while at < len(seq):
+        at += ctx.lib.gh_elementwise_run(C.cast(C.byref(seq_array, at * C.sizeof(D.GhCmd)), C.POINTER(D.GhCmd)), len(seq) - at)
+        seq_launches += 1
     # tensors no cache can hold (8192 x 8192, 256 MiB each): the kernels' streaming form
     big = [ctx.malloc(16 * N) for _ in range(3)]
     ctx.run([D.cmd_fill(q, 4 * N, 1.5) for q in big[:2]])
@@ -200,7 +215,8 @@ def bench_elementwise(ctx, iters):
     return {"chain_GBps": round(total_bytes / total_ms / 1e6, 1), "chain_bytes": total_bytes,
             "chain_us": round(total_ms * 1e3, 1), "frac_hbm": round(total_bytes / total_ms / 1e6 / HBM_PEAK_GBPS, 4),
             "frac_llc_assisted": round(total_bytes / total_ms_warm / 1e6 / HBM_PEAK_GBPS, 4),
-            "chain_in_sequence_us": round(ms_seq * 1e3, 1), "chain_in_sequence_GBps": round(total_bytes / ms_seq / 1e6, 1),
+            "chain_in_sequence_us": round(ms_seq * 1e3, 1), "chain_in_sequence_GBps": round(seq_bytes / ms_seq / 1e6, 1),
+            "chain_in_sequence_bytes": seq_bytes, "chain_in_sequence_launches": seq_launches,
             "streaming_8192": streaming, "operand_sets": S, "footprint_bytes": 3 * S * 4 * N,
             "device_copy_GBps": round(copy_gbps, 1), "device_copy_GBps_llc_assisted": round(copy_gbps_warm, 1),
             "kernels": out, "one_read_one_write_without_arithmetic": no_arith}
