@@ -1362,6 +1362,10 @@ Status TapeMachine::RunAll() {
         Node& n = nodes[(size_t)in.node];
         Tensor out;
         out.mem = regs_[(size_t)in.reg].mem;
+        // overwriting an input that lies in pinned memory: the result goes to the register's device memory, or every
+        // operator behind this one would read it over the bus
+        const bool moves = reg_arena_[(size_t)in.reg] && n.alias_of < 0;
+        if (moves) out.mem = reg_arena_[(size_t)in.reg];
         out.dt = n.dt;
         out.shape = n.shape;
         std::vector<Tensor> ins(n.inputs.size());
@@ -1375,6 +1379,10 @@ Status TapeMachine::RunAll() {
         }
         st = CUDADo(eng_, n.op, out, inp);
         if (!st.ok()) return st.Wrap("PC " + std::to_string(pc) + ": " + op_name(n.op));
+        if (moves) {
+          regs_[(size_t)in.reg].mem = out.mem;
+          reg_arena_[(size_t)in.reg] = 0;
+        }
         if (opt_.node_at_a_time) {
           st = flush();  // DoWork after every node (vm_genera.go:144)
           if (!st.ok()) return st.Wrap("PC " + std::to_string(pc) + ": " + op_name(n.op) + ": DoWork failed");
