@@ -21,9 +21,9 @@ static constexpr int64_t kStageInTotal = 512ll << 20; // per machine
 // together take 72 us of 2 MB (109 in one piece), 124 of 4 MB (185), 392 of 16 MB (590).
 static constexpr int64_t kPipelinedUpload = 768 << 10;
 static constexpr int64_t kUploadPiece = 512 << 10, kUploadPieceLong = 2 << 20, kLongUpload = 8 << 20;
-// inputs up to this size are read where the host wrote them, in pinned memory: the copy kernel a few KB would
-// need costs 4 us on the device, an operand read over the bus about 1
+// inputs up to this size may be read where the host wrote them, in pinned memory (reads_in_place)
 static constexpr int64_t kReadInPlace = 8 << 10;
+static constexpr int64_t kWalkInPlace = 2 << 10;
 
 static Status bad(const std::string& m) { return Status::Err(GH_EINVAL, m); }
 
@@ -922,6 +922,37 @@ int Graph::fuse_pooled_rectify() {
 
 // ---- TapeMachine --------------------------------------------------------------------
 
+// Whether n reads its k-th input from pinned memory as quickly as from the device.  A copy kernel in front costs 1.6 to
+// 2.5 us; over the bus a reader waits about 1 us for a load instead, once where its loads are in flight together.  How many
+// workgroups read the operand does not matter, they find it in the caches (a row of 2048 values added to 4 rows 22.3
+// against 24.1 us with the copy, to 4096 rows 38.2 against 40.1; 64 x 32 as the right factor of 65536 rows 40.7 and 42.7).
+// What does is a walk along it in steps, round after round over the bus: the K of a product (256 values of a row 15 to 17 us
+// against 16 to 18, 784 18.7 against 17.8, 2000 25.6 against 19.6, both with 300 columns; with 4000 the reading of the
+// matrix hides it, 784 19.5 against 22.3, 2000 29.1 against 32.1; a matrix-vector product of 200 values 12.2 against 14.3,
+// of 1000 18.2 against 16.9), the rows of a single-channel image (28 x 28 18.9 against 17.6, 44 x 44 23.8 against 19.2;
+// several channels gain).  Operators that pass over their input more than once, or were not measured, get the copy.
+static bool reads_in_place(const Node& n, size_t k, const std::vector<Node>& nodes) {
+  const Node& x = nodes[(size_t)n.inputs[k]];
+  const int64_t item = dtype_size(x.dt);
+  switch (n.op.kind) {
+    case OpKind::ElemBin: case OpKind::ElemUnary: case OpKind::BroadcastBin: case OpKind::Rectify: case OpKind::LeakyRelu:
+    case OpKind::RectifyDiff: case OpKind::MaxPool2D: case OpKind::BatchNorm:
+      return true;
+    case OpKind::MatMul: case OpKind::MatVecMul: case OpKind::BatchedMatMul: {
+      if (k >= 2) return true;   // a folded bias
+      const Shape& a = nodes[(size_t)n.inputs[0]].shape;
+      const bool wide = k == 0 && n.op.kind == OpKind::MatMul && n.shape.Dims() == 2 && n.shape[1] > 2048;
+      return a.Dims() >= 2 && (wide || a[a.Dims() - (n.op.transA ? 2 : 1)] * item <= kWalkInPlace);
+    }
+    case OpKind::Conv2d:
+      return k > 0 || (x.shape.Dims() == 4 && (x.shape[1] > 1 || x.shape[2] * x.shape[3] * item <= kWalkInPlace));
+    case OpKind::SolverStep:
+      return k == 4;   // Adam's two corrections; the others are written as well
+    default:
+      return false;
+  }
+}
+
 TapeMachine::~TapeMachine() { Close(); }
 
 Status TapeMachine::Compile() {
@@ -989,6 +1020,18 @@ Status TapeMachine::Compile() {
     for (int j = 0; j < N; j++)
       if (j != i && (root[(size_t)j] == i || node_reg_[(size_t)j] == node_reg_[(size_t)i])) shared = true;
     if (!shared) host_out[(size_t)i] = 1;
+  }
+  // small inputs that every reader reads in place
+  in_place_.assign((size_t)N, 0);
+  for (int i = 0; i < N; i++) {
+    const Node& n = nodes[(size_t)i];
+    in_place_[(size_t)i] = n.is_input && n.alias_of < 0 && !n.read_into && bytes_of(n) <= kReadInPlace;
+  }
+  for (int i = 0; i < N; i++) {
+    const Node& n = nodes[(size_t)i];
+    if (n.fused_away || n.is_input || (n.alias_of >= 0 && n.op.kind == OpKind::Reshape)) continue;   // a view's readers count
+    for (size_t k = 0; k < n.inputs.size(); k++)
+      if (!reads_in_place(n, k, nodes)) in_place_[(size_t)root[(size_t)n.inputs[k]]] = 0;
   }
   regs_.assign((size_t)nreg, Tensor());
   reg_live_.assign((size_t)nreg, 0);
@@ -1248,8 +1291,7 @@ Status TapeMachine::upload(const Instr& in, bool record) {
     if (!n.host_borrowed) std::memcpy(pinned, n.host, (size_t)in.size);
     if (!record) return Status::OK();
     const uint64_t arena = reg_memory((size_t)in.reg);
-    // (not a lent buffer: an operator may overwrite its input's register)
-    if (in.size <= kReadInPlace && !n.host_borrowed) {
+    if (in_place_[(size_t)in.node] && !n.host_borrowed) {   // (a lent buffer is the caller's, and its address theirs)
       reg_arena_[(size_t)in.reg] = arena;
       mem = (uint64_t)(uintptr_t)pinned;
     } else {
@@ -1518,6 +1560,9 @@ std::string TapeMachine::ProgramString() const {
     if (in.kind == InstrKind::ExecOp)
       os << " " << op_name(nodes[(size_t)in.node].op) << (in.use_unsafe ? " [unsafe]" : " [reuse]");
     if (in.size) os << " " << in.size << "B";
+    if (in.kind == InstrKind::Transport && in_place_[(size_t)in.node] && !nodes[(size_t)in.node].host_borrowed &&
+        (!nodes[(size_t)in.node].resident || opt_.reupload_resident))
+      os << " [in place]";
     os << "\n";
   }
   os << "GPU Memories: " << gpumem_ << "\n";

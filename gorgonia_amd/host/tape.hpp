@@ -263,6 +263,7 @@ class TapeMachine {
   std::vector<gh_cmd> recorded_;
   std::vector<char> in_pieces_;    // per node: the last run uploaded it piece by piece in front of the segment
   std::vector<char> lent_;         // per node: it was a lent input then
+  std::vector<char> in_place_;     // per node: a small input that its readers read in pinned memory (if it is not lent)
   bool steady_ = false;
   uint64_t arena_stamp_ = 0;
   std::vector<uint64_t> reg_arena_;   // the register's arena memory while regs_ points at a pinned input buffer
