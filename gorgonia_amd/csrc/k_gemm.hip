@@ -2384,6 +2384,23 @@ inline int clamp_splits(gh_ctx* ctx, int64_t splits, int64_t M, int64_t N, int64
   return splits < 1 ? 1 : (int)splits;
 }
 
+// K slices of a matrix product on 64x64 tiles: a compute unit works through its workgroups' k-tiles
+// at about 0.8 us each however many share it, and a second launch to add the slabs costs 3.5 us plus
+// 1 us per slab and million results (1152 x 625 results, K = 128 ... 2048: this picks the
+// measured best count, one slice up to K = 256 and four from 512 on, where
+// cdiv(2 cus, blocks) = 3 lost 8-25 %).
+inline int64_t gemm_tile64_slices(int64_t M, int64_t N, int64_t K, int64_t cus) {
+  const int64_t nk = cdiv(K, 16), blocks = cdiv(M, 64) * cdiv(N, 64);
+  const double slab_us = (double)M * (double)N * 1e-6;
+  double best = 0;
+  int64_t sp = 1;
+  for (int64_t s = 1; s <= 16 && (s == 1 || 2 * s <= nk); s++) {
+    const double est = (double)(cdiv(blocks * s, cus) * cdiv(nk, s)) * 0.8 + (s > 1 ? 3.5 + slab_us * (double)s : 0.0);
+    if (s == 1 || est < best) { best = est; sp = s; }
+  }
+  return sp;
+}
+
 TilePlan plan_tiles(gh_ctx* ctx, int64_t M, int64_t N, int64_t K, int64_t batch, bool allow_32x256) {
   TilePlan p{kTile128, 1};
   if (const char* env = getenv("GORGONIA_HIP_GEMM_PLAN")) {  // tuning override: "tile,splits"
@@ -2401,21 +2418,11 @@ TilePlan plan_tiles(gh_ctx* ctx, int64_t M, int64_t N, int64_t K, int64_t batch,
   else p.tile = kTile64;
   const int64_t blocks = p.tile == kTile64 ? cdiv(M, 64) * cdiv(N, 64) * batch : cdiv(M, 32) * cdiv(N, 256);
   if (batch == 1 && blocks < 2 * cus) {
-    const int64_t nk = cdiv(K, 16);
     int64_t sp = 1;
     if (!allow_32x256) {
-      // matrix product on 64x64 tiles: a compute unit works through its workgroups' k-tiles at about
-      // 0.8 us each however many share it, and a second launch to add the slabs costs 3.5 us plus
-      // 1 us per slab and million results (1152 x 625 results, K = 128 ... 2048: this picks the
-      // measured best count, one slice up to K = 256 and four from 512 on, where
-      // cdiv(2 cus, blocks) = 3 lost 8-25 %)
-      double best = 0;
-      const double slab_us = (double)M * (double)N * 1e-6;
-      for (int64_t s = 1; s <= 16 && (s == 1 || 2 * s <= nk); s++) {
-        const double est = (double)(cdiv(blocks * s, cus) * cdiv(nk, s)) * 0.8 + (s > 1 ? 3.5 + slab_us * (double)s : 0.0);
-        if (s == 1 || est < best) { best = est; sp = s; }
-      }
+      sp = gemm_tile64_slices(M, N, K, cus);
     } else {
+      const int64_t nk = cdiv(K, 16);
       sp = cdiv(2 * cus, blocks);
       const int64_t max_sp = nk / 4 > 0 ? nk / 4 : 1;  // at least 4 k-tiles per slice
       if (sp > max_sp) sp = max_sp;
@@ -3012,6 +3019,17 @@ static int direct_form(const gh_cmd& c, int cus) {
   // Short contractions over many aligned 64x64 tiles: staging a tile once beats reading it per wavefront
   // (1500 x 1500, K = 64: 9.2 us against 10.0; K = 100: equal; K = 130: 20 against 14).
   if (vec && K <= 96 && cdiv(M, 64) * cdiv(N, 64) * batch >= 2 * cus) return -1;
+  // Long contractions into few tiles: k_gemm_direct splits K among the wavefronts of a tile's one workgroup, slabs of
+  // 64x64 tiles among workgroups (transposed 6 x 103, K = 9561: 30 us against 98; 468 x 24, K = 1430: 12.1 against 18.4;
+  // 10 x 65, K = 441: 8.7 against 7.4).  A k-tile takes 0.8 us, 0.5 with 16-byte loads, four fifths of that each with two
+  // workgroups to a compute unit; for so few tiles the other estimate is up to 4 us high.  (Only slabs that any scratch
+  // holds: what a caller may not enlarge refuses no more than before.)
+  if (batch == 1 && cdiv(M, 64) * cdiv(N, 64) < 2 * cus) {
+    const int64_t slices = gemm_tile64_slices(M, N, K, cus), rounds = cdiv(cdiv(M, 64) * cdiv(N, 64) * slices, cus);
+    const double slabs = 6.0 + (double)(rounds * cdiv(cdiv(K, 16), slices)) * (vec ? 0.5 : 0.8) * (rounds > 1 ? 0.78 : 1.0) +
+                         (double)(M * N * slices) * 1e-6;
+    if (slices > 1 && slices * M * N * 4 <= GH_NOALLOC_SCRATCH_BYTES && slabs + 4.0 < us && slabs < 0.95 * us) return -1;
+  }
   // 128x128 tiles through LDS where they fill the device: 68 us per 1000 of K and round of tiles, half as much again
   // with one workgroup per compute unit and nothing to run under its barriers.
   const int64_t big = cdiv(M, 128) * cdiv(N, 128) * batch;
@@ -3023,16 +3041,21 @@ static int direct_form(const gh_cmd& c, int cus) {
   return form;
 }
 
+// Which kernel takes a float64 product of more than two rows: a form of k_gemm_direct, or -1 for one 16x16 tile per
+// workgroup (k_dgemm_skinny) where larger tiles leave the device idle: 4.6 us per 1000 of K and 256 tiles.
+static int gemm64_form(const gh_cmd& c, int cus) {
+  double us = 0;
+  const int form = gh_gemm_direct_form(c, cus, &us);
+  const double tiles16 = (double)cdiv(c.dim[0], 16) * (double)cdiv(c.dim[1], 16);
+  const double small = 4.0 + std::max(1.0, tiles16 / cus) * (double)c.dim[2] * 4.6e-3;
+  return c.dim[6] <= 1 && c.dim[2] >= 64 && small < us ? -1 : form;
+}
+
 int gh_launch_gemm(gh_ctx* ctx, const gh_cmd& c) {
   const int64_t batch = c.dim[6] <= 0 ? 1 : c.dim[6];
   if (gh_dtype_of(c.flags) == GH_F64) {
     if (gh_gemm_thin_takes(c)) return gh_launch_gemm_thin(ctx, c);
-    double us = 0;
-    const int form = gh_gemm_direct_form(c, ctx->cu_count, &us);
-    // one 16x16 tile per workgroup where larger tiles leave the device idle: 4.6 us per 1000 of K and 256 tiles
-    const double tiles16 = (double)cdiv(c.dim[0], 16) * (double)cdiv(c.dim[1], 16);
-    const double small = 4.0 + std::max(1.0, tiles16 / ctx->cu_count) * (double)c.dim[2] * 4.6e-3;
-    if (batch == 1 && c.dim[2] >= 64 && (form < 0 || small < us)) return launch_dgemm_skinny(ctx, c);
+    const int form = gemm64_form(c, ctx->cu_count);
     return form >= 0 ? gh_launch_gemm_direct(ctx, c, form) : launch_dgemm_skinny(ctx, c);
   }
   if (gh_gemm_thin_takes(c)) return gh_launch_gemm_thin(ctx, c);
@@ -3072,6 +3095,14 @@ extern "C" int gh_gemm_route(const gh_cmd* c, int* splits) {
   const TilePlan p = plan_tiles(&probe, c->dim[0], c->dim[1], c->dim[2], batch, false);
   if (splits) *splits = p.splits;
   return p.tile == kTile128 ? GH_GEMM_ROUTE_TILE128 : p.tile == kTile128x64 ? GH_GEMM_ROUTE_TILE128X64 : GH_GEMM_ROUTE_TILE64;
+}
+
+extern "C" int gh_gemm_straight(const gh_cmd* c) {
+  if (!c || c->opcode != GH_OP_GEMM) return 0;
+  const int cus = gh_ctx{}.cu_count;   // the MI355X's
+  if (gh_gemm_thin_takes(*c)) return 1;
+  if (gh_dtype_of(c->flags) == GH_F64) return gemm64_form(*c, cus) >= 0;
+  return !gemm_skinny_takes(*c, cus) && direct_form(*c, cus) >= 0;
 }
 
 // The direct kernel's shapes: 3x3, stride 1, no dilation, square padding, at
