@@ -2740,12 +2740,18 @@ static bool gemm_skinny_takes(const gh_cmd& c, int cus) {
 
 // Slices of K for a small-output product: a tile is one workgroup's work, and one workgroup walks 1000 of K in about
 // 7 us, so a long contraction over few tiles is cut until the slices fill the device or are down to 512 (four chunks
-// for each of eight wavefronts); below 2048 the second launch (5 us) costs what the cut saves.
+// for each of eight wavefronts); below 2048 the second launch (5 us) costs what the cut saves.  Tiles that leave the
+// device only two slices are not cut, as so many workgroups already share the memory, and of the 16-row kernel's those
+// that leave three or four only from a longer K on (two: 36 x 907, K = 2696 10.5 us in one piece, 12.9 cut; 116 x 402,
+// K = 13586 49.4 and 53.1; three: 60 x 560, K = 2300 8.7 and 10.0, 343 x 73, K = 5249 22.8 and 20.2; four: 44 x 612,
+// K = 2104 8.5 and 10.0, 61 x 451, K = 2913 13.2 and 12.1, but 324 x 4, K = 2408 8.7 and 6.6).
 static int skinny_slices(const gh_cmd& c, int cus) {
   const int64_t M = c.dim[0], N = c.dim[1], K = c.dim[2];
   if (K < 2048) return 1;
   const int64_t tiles = cdiv(M, M >= 16 ? 16 : 32) * cdiv(N, 32);
-  return (int)std::max<int64_t>(1, std::min<int64_t>(cus / tiles, K / 512));
+  const int64_t slices = std::min<int64_t>(cus / tiles, K / 512);
+  const int64_t from = slices < 3 ? INT64_MAX : M < 16 || tiles <= 32 ? 2048 : slices == 3 ? 4800 : 2800;
+  return K >= from ? (int)slices : 1;
 }
 
 static int launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c, int slices);
