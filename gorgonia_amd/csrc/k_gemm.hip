@@ -2750,7 +2750,7 @@ static int skinny_slices(const gh_cmd& c, int cus) {
   if (K < 2048) return 1;
   const int64_t tiles = cdiv(M, M >= 16 ? 16 : 32) * cdiv(N, 32);
   const int64_t slices = std::min<int64_t>(cus / tiles, K / 512);
-  const int64_t from = slices < 3 ? INT64_MAX : M < 16 || tiles <= 32 ? 2048 : slices == 3 ? 4800 : 2800;
+  const int64_t from = slices < 3 ? INT64_MAX : M < 16 || tiles <= 32 || slices > 4 ? 2048 : slices == 3 ? 4800 : 2800;
   return K >= from ? (int)slices : 1;
 }
 

@@ -46,6 +46,6 @@ def test_slabs_fit_any_scratch():
                                                 (116, 402, 13586, False, False, 1), (60, 560, 2300, False, False, 1), (48, 836, 2648, False, True, 1),
                                                 (51, 641, 12494, False, False, 3), (424, 77, 20171, False, True, 3), (61, 451, 2913, False, True, 4),
                                                 (343, 73, 5249, False, True, 3), (44, 612, 2104, True, False, 1),
-                                                (324, 4, 2408, False, False, 4), (12, 1336, 2496, False, False, 4), (12, 12, 7808, False, False, 15)])
+                                                (324, 4, 2408, False, False, 4), (537, 1, 2784, True, False, 5), (12, 1336, 2496, False, False, 4), (12, 12, 7808, False, False, 15)])
 def test_small_outputs_are_cut_where_slices_fill_an_idle_device(m, n, k, ta, tb, slices):
     assert _slices(m, n, k, ta, tb) == slices
