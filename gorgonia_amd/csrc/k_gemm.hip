@@ -3011,6 +3011,33 @@ static int launch_dgemm_skinny(gh_ctx* ctx, const gh_cmd& c) {
   return gh_check_hip(ctx, hipGetLastError(), "dgemm launch");
 }
 
+// Short contractions whose tiles are better staged in LDS than read by every wavefront.  vec: the tiled kernel stages with
+// 16-byte loads.  Times as staged / straight, us:
+//   * more tiles than compute units: 1952 x 1716, K = 24 8.2 / 11.9, K = 256 20.1 / 22.8 transposed; 4096 x 4096, K = 5 18.7 / 30.
+//     Without vec the staging itself is slow, and it is so only up to K = 28, of very many tiles 48 (1954 x 1715, K = 24
+//     9.5 / 11.8, K = 64 20 / 15; 4001 x 3001, K = 40 24.4 / 30).
+//   * the right operand transposed: half a 128-byte line to a load of the straight kernel, and its last chunk, where K
+//     is no multiple of 16, comes value by value (505 x 274 x 9, K = 24 6.0 / 8.6).  For few tiles that matters where K
+//     is a multiple of 4 and not an odd one of 16, which its loads pair up (500 x 500, K = 8 4.2 / 5.6, K = 16 4.2 / 4.0), and
+//     not for narrow results (2000 x 8, K = 8 4.2 / 3.4).
+//   * up to 8 rows and K below 32 the same by 0.2 to 0.5 us of 3.4.
+// Batches of two to eight rounds of tiles without vec, and results of few rows or columns, which fill no 64 x 64 tile,
+// are quicker straight (338 x 182 x 64, K = 2 11.3 / 8.7; 4012 x 7 x 8, K = 3 6.8 / 4.0; but 230 x 2495 x 24, K = 7 17.5 / 25.7).
+// The estimates below are no help here: fixed costs make these times, and vary by a third.
+static bool gemm_short_k_staged(int64_t M, int64_t N, int64_t K, int64_t batch, bool ta, bool tb, bool vec, int cus) {
+  const int64_t tiles = cdiv(M, 64) * cdiv(N, 64) * batch;
+  const bool many = tiles > cus, paired = K % 32 == 16;
+  if (M <= 8 && K < 32 && batch == 1 && N >= 128) return true;
+  if (N < 48 || (many && M <= 32) || (!vec && batch > 1 && tiles >= 2 * cus && tiles < 8 * cus)) return false;
+  if (K <= 128) {
+    if (tb && ta) return K < 32 ? K != 16 : vec && !paired;
+    if (tb) return many || (vec && !paired && N >= 64);
+    return many && (vec || K <= (tiles >= 8 * cus ? 48 : 28));
+  }
+  if (!vec || ta == tb) return false;
+  return tb ? K <= 300 && 5 * tiles >= 9 * cus : K <= 256 && tiles >= 3 * cus;
+}
+
 // Which kernel takes a float32 product that is none of the small-output ones: -1 for the LDS-tiled kernel under
 // plan_tiles, else a form of k_gemm_direct.
 static int direct_form(const gh_cmd& c, int cus) {
@@ -3022,9 +3049,7 @@ static int direct_form(const gh_cmd& c, int cus) {
   const bool ta = c.flags & GH_FLAG_TRANS_A, tb = c.flags & GH_FLAG_TRANS_B;
   const bool vec = ((c.ptr[0] | c.ptr[1]) & 15) == 0 && c.dim[3] % 4 == 0 && c.dim[4] % 4 == 0 && (ta ? M : K) % 4 == 0 && (tb ? K : N) % 4 == 0 &&
                    (batch == 1 || (c.dim[7] % 4 == 0 && c.dim[8] % 4 == 0));
-  // Short contractions over many aligned 64x64 tiles: staging a tile once beats reading it per wavefront
-  // (1500 x 1500, K = 64: 9.2 us against 10.0; K = 100: equal; K = 130: 20 against 14).
-  if (vec && K <= 96 && cdiv(M, 64) * cdiv(N, 64) * batch >= 2 * cus) return -1;
+  if (gemm_short_k_staged(M, N, K, batch, ta, tb, vec, cus)) return -1;
   // Long contractions into few tiles: k_gemm_direct splits K among the wavefronts of a tile's one workgroup, slabs of
   // 64x64 tiles among workgroups (transposed 6 x 103, K = 9561: 30 us against 98; 468 x 24, K = 1430: 12.1 against 18.4;
   // 10 x 65, K = 441: 8.7 against 7.4).  A k-tile takes 0.8 us, 0.5 with 16-byte loads, four fifths of that each with two

@@ -49,3 +49,25 @@ def test_slabs_fit_any_scratch():
                                                 (324, 4, 2408, False, False, 4), (537, 1, 2784, True, False, 5), (12, 1336, 2496, False, False, 4), (12, 12, 7808, False, False, 15)])
 def test_small_outputs_are_cut_where_slices_fill_an_idle_device(m, n, k, ta, tb, slices):
     assert _slices(m, n, k, ta, tb) == slices
+
+
+@pytest.mark.parametrize("m,n,batch", [(1952, 1716, 1), (248, 164, 24), (4096, 4096, 1), (3060, 632, 1)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("k", [4, 24, 96, 128])
+def test_short_contractions_over_many_aligned_tiles_are_staged(m, n, batch, ta, tb, k):
+    assert _straight(m, n, k, ta, tb, batch) == 0
+
+
+@pytest.mark.parametrize("m,n,k,ta,tb,batch,straight", [
+    (1954, 1715, 24, False, False, 1, 0), (1954, 1715, 64, False, False, 1, 1),      # rows that 16-byte loads cannot take
+    (4001, 3001, 40, True, False, 1, 0), (505, 274, 48, True, False, 9, 1),
+    (505, 274, 24, False, True, 9, 0), (500, 500, 8, False, True, 4, 0), (500, 500, 16, False, True, 4, 1),
+    (2000, 8, 8, False, True, 4, 1), (128, 128, 12, False, False, 32, 1), (128, 128, 9, True, False, 32, 1),
+    (200, 200, 24, True, True, 1, 0), (200, 200, 16, True, True, 1, 1), (200, 200, 48, True, True, 1, 1),
+    (4, 3008, 8, True, True, 1, 0), (7, 194, 5, True, False, 1, 0),
+    (1952, 1716, 256, True, False, 1, 0), (1952, 1716, 256, False, True, 1, 0), (249, 164, 256, False, True, 23, 1),
+    (1952, 1716, 400, False, False, 1, 1), (1676, 2628, 192, False, False, 1, 1),
+    (338, 182, 2, False, True, 64, 1), (230, 2495, 7, True, False, 24, 0), (1408, 260, 3, True, True, 8, 1), (4012, 7, 3, False, True, 8, 1), (24, 1260, 76, False, False, 24, 1),
+    (12, 9, 27, False, True, 24, 1)])
+def test_short_contractions(m, n, k, ta, tb, batch, straight):
+    assert _straight(m, n, k, ta, tb, batch) == straight
