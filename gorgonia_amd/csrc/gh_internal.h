@@ -129,7 +129,8 @@ int gh_try_launch_conv_small(gh_ctx* ctx, const gh_cmd& c);
 int gh_try_launch_conv_wgrad_small(gh_ctx* ctx, const gh_cmd& c, int* splits);
 bool gh_conv_wgrad_small_takes(const gh_cmd& c);
 // 3x3 stride-1 filter gradient with operands straight from memory, both float types (k_conv_wgrad.hip)
-bool gh_conv_wgrad_takes(const gh_cmd& c);
+bool gh_conv_wgrad_takes(const gh_cmd& c, int cus);
+int64_t gh_conv_wgrad_slab_limit(const gh_cmd& c, int64_t slab_bytes);
 int gh_launch_conv_wgrad(gh_ctx* ctx, const gh_cmd& c);
 bool gh_conv_small_takes(const gh_cmd& c);
 bool gh_conv_small_can_pool(const gh_cmd& c);

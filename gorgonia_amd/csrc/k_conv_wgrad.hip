@@ -312,14 +312,18 @@ bool fill(const gh_cmd& c, Wg<T>* g) {
   return true;
 }
 
+// Workgroups along the long axis.  To a compute unit: what a wavefront does besides its MFMAs - the first loads, meeting the
+// others, a slab to be summed - costs as much as some ten chunks of a channel tile, so one; packed tiles, three.
+int64_t slices_of(int64_t tiles, int64_t items, int cus, bool packed) {
+  const int64_t slices = std::max<int64_t>(1, (packed ? 3 : 1) * (int64_t)cus / tiles);
+  return std::min<int64_t>(slices, std::max<int64_t>(1, items / (4 * kWaves)));
+}
+
 template <class T, int TM, int P, int NT, bool kPacked>
 int launch(gh_ctx* ctx, Wg<T> g, T* dw) {
   const int64_t ft = (g.F + 16 * TM - 1) / (16 * TM), ct = kPacked ? 1 : (g.C + 15) / 16;
   const int64_t results = (int64_t)g.F * g.C * 9;
-  // Workgroups to a compute unit: what a wavefront does besides its MFMAs - the first loads, meeting the others, a
-  // slab to be summed - costs as much as some ten chunks of a channel tile, so one; packed tiles, three.
-  int64_t slices = std::max<int64_t>(1, (kPacked ? 3 : 1) * (int64_t)ctx->cu_count / (ft * ct));
-  slices = std::min<int64_t>(slices, std::max<int64_t>(1, g.items / (4 * kWaves)));
+  int64_t slices = slices_of(ft * ct, g.items, ctx->cu_count, kPacked);
   if (slices > 1 && slices * results * (int64_t)sizeof(T) > ctx->workspace_bytes) {
     if (int rc = gh_ws_short(ctx, slices * results * (int64_t)sizeof(T))) return rc;
     slices = std::max<int64_t>(1, ctx->workspace_bytes / (results * (int64_t)sizeof(T)));
@@ -349,16 +353,48 @@ int pick(gh_ctx* ctx, const Wg<T>& g, T* dw) {
 
 }  // namespace
 
+// Whether a channel tile's walk is the slower one.  Its tiles hold 16 channels, 16 or 32 filters and chunks of 16 (8)
+// columns of a row, so few channels over a multiple of 16, or rows little longer than a chunk, leave much of it empty; the
+// tiled kernel pads filters and (channel, tap) columns to 64 and no row.  Both are so many us per round of their tiles'
+// chunks over the compute units, and per million slab values; fitted to 320 shapes in float32 and 277 in float64 of 1 to 64
+// images of 3 x 3 to 208 x 208, 9 to 400 channels, 8 to 300 filters, within 10 % for most.  By it 55 x 21 x 90 x 3 -> 157 in
+// float64 takes 54 us (120 here), 12 x 249 x 20 x 20 -> 376 119 (161), 11 x 198 x 21 x 21 -> 173 63 (77).
+static bool tiled_is_quicker(const gh_cmd& c, const Wg<double>& g, int cus) {
+  const bool f64 = gh_dtype_of(c.flags) == GH_F64;
+  auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const int64_t results = (int64_t)g.F * g.C * 9, pixels = g.dy_total / g.F;
+  const int64_t ft64 = cdiv(g.F, 64) * cdiv(g.C * 9, 64), nk = cdiv(pixels, f64 ? 16 : 32);
+  int64_t slabs = std::min<int64_t>(std::min<int64_t>(cdiv(5 * (int64_t)cus / 2, ft64), nk / 4), f64 ? 512 : 64);
+  slabs = std::max<int64_t>(1, std::min<int64_t>(slabs, GH_NOALLOC_SCRATCH_BYTES / (results * (f64 ? 8 : 4))));
+  if (f64 && pixels * results < (int64_t)1 << 22) return false;   // the tiled kernel leaves these to one thread a result
+  const int tm = !f64 && g.F > 16 ? 2 : 1;
+  const int64_t tiles = cdiv(g.F, 16 * tm) * cdiv(g.C, 16), slices = slices_of(tiles, g.items, cus, false);
+  const double chunks = (double)(cdiv(slices * tiles, cus) * cdiv(g.items, slices * kWaves)) * tm * (g.ow <= 8 ? 0.5 : 1.0);
+  const double here = f64 ? 7.3 + 1.55 * chunks + 5.4e-6 * (double)(slices * results) : 6.6 + 0.80 * chunks + 4.5e-6 * (double)(slices * results);
+  const double there = f64 ? 12.3 + 1.26 * (double)(ft64 * nk) / cus + 0.8e-6 * (double)(slabs * results)
+                           : 11.0 + 1.06 * (double)(ft64 * nk) / cus + 1.0e-6 * (double)(slabs * results);
+  return here > (f64 ? 1.06 : 1.0) * there;
+}
+
 // Whether k_conv3x3_wgrad takes a filter gradient: 3x3, stride 1.  Of float32, not the shapes the small-image and
 // the single-channel kernel hold in LDS, and up to four channels only where there are enough pixels to cut up
 // (below that the vector kernel's few workgroups do; of a single channel it wastes the least).
-bool gh_conv_wgrad_takes(const gh_cmd& c) {
-  Wg<double> g;   // (the narrower of the two in what its offsets reach)
-  if (!fill(c, &g) || g.F < 8) return false;
-  const int64_t pixels = g.dy_total / g.F;
-  if (g.C <= 8 && g.ow <= 8) return false;
+static bool can_take(const gh_cmd& c, Wg<double>* g) {   // (the narrower of the two in what its offsets reach)
+  if (!fill(c, g) || g->F < 8) return false;
+  const int64_t pixels = g->dy_total / g->F;
+  if (g->C <= 8 && g->ow <= 8) return false;
   if (gh_dtype_of(c.flags) == GH_F64) return pixels >= 256;
-  return pixels >= (g.C == 1 ? 65536 : g.C <= 4 ? 16384 : 256);
+  return pixels >= (g->C == 1 ? 65536 : g->C <= 4 ? 16384 : 256);
+}
+bool gh_conv_wgrad_takes(const gh_cmd& c, int cus) {
+  Wg<double> g;
+  return can_take(c, &g) && (g.C <= 8 || !tiled_is_quicker(c, g, cus));
+}
+// Slabs that the tiled kernels may use for a command: those of a shape that this one could take, and without scratch, fit
+// any scratch, so that the choice refuses nothing.
+int64_t gh_conv_wgrad_slab_limit(const gh_cmd& c, int64_t slab_bytes) {
+  Wg<double> g;
+  return can_take(c, &g) ? std::max<int64_t>(1, GH_NOALLOC_SCRATCH_BYTES / slab_bytes) : INT64_MAX;
 }
 
 int gh_launch_conv_wgrad(gh_ctx* ctx, const gh_cmd& c) {

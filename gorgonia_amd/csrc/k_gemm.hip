@@ -2878,13 +2878,17 @@ static bool conv64_fill(const gh_cmd& c, ConvGeom64* out) {
   return true;
 }
 
-// Float64 Conv2d on the matrix cores; false = not taken (few filters or a tiny
-// problem: the one-thread-per-result kernel stays).
+// Whether the matrix cores take a float64 Conv2d: not of few filters, nor a tiny problem (the one-thread-per-result
+// kernel stays).
+static bool conv64_mfma_takes(const gh_cmd& c, ConvGeom64* g) {
+  return conv64_fill(c, g) && g->F >= 16 && g->P >= 256 && g->K >= 8 && (int64_t)g->P * g->F * g->K >= (int64_t)1 << 22;
+}
+
+// Float64 Conv2d on the matrix cores; false = not taken.
 bool gh_try_launch_conv2d_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
   ConvGeom64 g;
-  if (!conv64_fill(c, &g)) return false;
-  const int64_t P = g.P, K = g.K;
-  if (g.F < 16 || P < 256 || K < 8 || P * g.F * K < (int64_t)1 << 22) return false;
+  if (!conv64_mfma_takes(c, &g)) return false;
+  const int64_t P = g.P;
   if (gh_conv_lanes_takes(c, false, ctx->cu_count, 0)) {
     gh_launch_conv_lanes(ctx, c, false);   // an error is sticky on the context; the caller returns it
     return true;
@@ -2908,25 +2912,30 @@ bool gh_try_launch_conv2d_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
   return true;
 }
 
-// Float64 image gradient of a stride-1 convolution: the forward kernel over dy
-// with mirrored, transposed filters (held at the top of the workspace).
-bool gh_try_launch_conv2d_bwd_data_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
+// The forward command that a float64 image gradient of stride 1 is, over dy with mirrored, transposed filters (its
+// pointers are the caller's to fill); false where the matrix cores do not take that.
+static bool conv64_mirror(const gh_cmd& c, gh_cmd* out) {
   ConvGeom64 g;
   if (!conv64_fill(c, &g)) return false;
   const int padH = g.dilH * (g.kh - 1) - g.padH, padW = g.dilW * (g.kw - 1) - g.padW;
-  const int64_t wcount = (int64_t)g.F * g.K;
-  const int64_t wbytes = (wcount * 8 + 255) / 256 * 256;
   if (g.strideH != 1 || g.strideW != 1 || padH < 0 || padW < 0) return false;
-  gh_cmd f{};
+  gh_cmd& f = *out;
+  f = gh_cmd{};
   f.opcode = GH_OP_CONV2D;
   f.flags = c.flags;
   f.dim[0] = c.dim[0]; f.dim[1] = g.F; f.dim[2] = g.oh; f.dim[3] = g.ow; f.dim[4] = g.C;
   f.dim[5] = g.kh; f.dim[6] = g.kw; f.dim[7] = padH; f.dim[8] = padW;
   f.dim[9] = 1; f.dim[10] = 1; f.dim[11] = g.dilH; f.dim[12] = g.dilW;
-  // decide before mirroring whether the forward kernel takes the shape (same tests as above)
   ConvGeom64 gf;
-  if (!conv64_fill(f, &gf)) return false;
-  if (gf.F < 16 || gf.P < 256 || gf.K < 8 || (int64_t)gf.P * gf.F * gf.K < (int64_t)1 << 22) return false;
+  return conv64_mfma_takes(f, &gf);
+}
+
+// Float64 image gradient of a stride-1 convolution: the forward kernel (mirrored filters at the top of the workspace).
+bool gh_try_launch_conv2d_bwd_data_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
+  gh_cmd f;
+  if (!conv64_mirror(c, &f)) return false;
+  const int F = (int)c.dim[4], C = (int)c.dim[1], kh = (int)c.dim[5], kw = (int)c.dim[6];
+  const int64_t wcount = (int64_t)F * C * kh * kw, wbytes = (wcount * 8 + 255) / 256 * 256;
   // (what a fixed scratch refuses does not depend on the kernel)
   if (wbytes > ctx->workspace_bytes && gh_ws_short(ctx, wbytes) != GH_OK) return true;   // the caller returns ctx->err
   if (gh_conv_lanes_takes(c, true, ctx->cu_count, 0)) {
@@ -2939,14 +2948,14 @@ bool gh_try_launch_conv2d_bwd_data_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
   int64_t blocks = cdiv(wcount, 256);
   if (blocks > (int64_t)ctx->cu_count * 8) blocks = (int64_t)ctx->cu_count * 8;
   hipLaunchKernelGGL(k_flip_filters<double>, dim3((int)blocks), dim3(256), 0, ctx->stream,
-                     (const double*)(uintptr_t)c.ptr[1], wt, g.F, g.C, g.kh, g.kw);
+                     (const double*)(uintptr_t)c.ptr[1], wt, F, C, kh, kw);
   return gh_try_launch_conv2d_f64_mfma(ctx, f);
 }
 
 // Float64 filter gradient on the matrix cores, pixel axis cut into slices.
 bool gh_try_launch_conv2d_bwd_filter_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
   ConvGeom64 g;
-  if (gh_conv_wgrad_takes(c)) {
+  if (gh_conv_wgrad_takes(c, ctx->cu_count)) {
     gh_launch_conv_wgrad(ctx, c);   // an error is sticky on the context; the caller returns it
     return true;
   }
@@ -2959,6 +2968,7 @@ bool gh_try_launch_conv2d_bwd_filter_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
   if (splits > nk / 4) splits = nk / 4;
   if (splits > 512) splits = 512;
   const int64_t slab = (int64_t)g.F * g.K * 8;
+  splits = std::min(splits, gh_conv_wgrad_slab_limit(c, slab));
   if (splits > 1 && ctx->workspace_bytes / slab < splits) {
     if (gh_ws_short(ctx, splits * slab)) return true;   // the caller returns ctx->err
     splits = ctx->workspace_bytes / slab;
@@ -3126,14 +3136,6 @@ extern "C" int gh_gemm_route(const gh_cmd* c, int* splits) {
   const TilePlan p = plan_tiles(&probe, c->dim[0], c->dim[1], c->dim[2], batch, false);
   if (splits) *splits = p.splits;
   return p.tile == kTile128 ? GH_GEMM_ROUTE_TILE128 : p.tile == kTile128x64 ? GH_GEMM_ROUTE_TILE128X64 : GH_GEMM_ROUTE_TILE64;
-}
-
-extern "C" int gh_gemm_straight(const gh_cmd* c) {
-  if (!c || c->opcode != GH_OP_GEMM) return 0;
-  const int cus = gh_ctx{}.cu_count;   // the MI355X's
-  if (gh_gemm_thin_takes(*c)) return 1;
-  if (gh_dtype_of(c->flags) == GH_F64) return gemm64_form(*c, cus) >= 0;
-  return !gemm_skinny_takes(*c, cus) && direct_form(*c, cus) >= 0;
 }
 
 // The direct kernel's shapes: 3x3, stride 1, no dilation, square padding, at
@@ -3310,8 +3312,8 @@ static bool wgrad_c1_takes(const gh_cmd& c) {
 }
 
 // ... and what is left to k_conv3x3_wgrad: neither the single-channel nor the small-image kernel's shapes.
-static bool wgrad_mfma_takes(const gh_cmd& c) {
-  return gh_conv_wgrad_takes(c) && !wgrad_c1_takes(c) && !gh_conv_wgrad_small_takes(c);
+static bool wgrad_mfma_takes(const gh_cmd& c, int cus) {
+  return gh_conv_wgrad_takes(c, cus) && !wgrad_c1_takes(c) && !gh_conv_wgrad_small_takes(c);
 }
 
 // dW = dY2d^T . col  (ptr[0] = x, ptr[1] = dy, ptr[2] = dw)
@@ -3319,7 +3321,7 @@ int gh_launch_conv2d_bwd_filter(gh_ctx* ctx, const gh_cmd& c) {
   if (gh_dtype_of(c.flags) == GH_F64) return gh_launch_conv2d_bwd_filter_f64(ctx, c);
   const ConvGeom g = conv_geom(c);
   const int F = (int)c.dim[4], CKK = g.C * g.kh * g.kw;
-  if (wgrad_mfma_takes(c)) return gh_launch_conv_wgrad(ctx, c);
+  if (wgrad_mfma_takes(c, ctx->cu_count)) return gh_launch_conv_wgrad(ctx, c);
   if (conv_direct_shape(c) && F <= 65535) {
     const int B = (int)c.dim[0];
     int G = B < 64 ? B : 64;
@@ -3388,6 +3390,7 @@ int gh_launch_conv2d_bwd_filter(gh_ctx* ctx, const gh_cmd& c) {
   if (splits > nk / 4) splits = nk / 4;
   if (splits > 64) splits = 64;
   const int64_t slab = (int64_t)F * CKK * 4;
+  splits = std::min(splits, gh_conv_wgrad_slab_limit(c, slab));
   if (splits > 1 && ctx->workspace_bytes / slab < splits) {
     if (int rc = gh_ws_short(ctx, splits * slab)) return rc;
     splits = ctx->workspace_bytes / slab;
@@ -3536,10 +3539,34 @@ extern "C" int gh_conv2d_bwd_filter_route(const gh_cmd* c) {
   if (!c || c->opcode != GH_OP_CONV2D_BWD_FILTER) return -1;
   if (gh_dtype_of(c->flags) == GH_F64) return GH_WGRAD_ROUTE_F64;
   if (wgrad_c1_takes(*c)) return GH_WGRAD_ROUTE_SINGLE_CHANNEL;
-  if (wgrad_mfma_takes(*c)) return GH_WGRAD_ROUTE_GEMM;
+  if (wgrad_mfma_takes(*c, 256)) return GH_WGRAD_ROUTE_GEMM;
   if (conv_direct_shape(*c) && c->dim[4] <= 65535) return GH_WGRAD_ROUTE_DIRECT;
   if (gh_conv_wgrad_small_takes(*c)) return GH_WGRAD_ROUTE_SMALL;
   return GH_WGRAD_ROUTE_GEMM;
+}
+
+extern "C" int gh_runs_straight(const gh_cmd* c) {
+  if (!c) return 0;
+  const int cus = gh_ctx{}.cu_count;   // the MI355X's
+  const bool f64 = gh_dtype_of(c->flags) == GH_F64;
+  switch (c->opcode) {
+    case GH_OP_GEMM:
+      if (gh_gemm_thin_takes(*c)) return 1;
+      return f64 ? gemm64_form(*c, cus) >= 0 : !gemm_skinny_takes(*c, cus) && direct_form(*c, cus) >= 0;
+    case GH_OP_CONV2D: {
+      ConvGeom64 g;
+      if (f64) return conv64_mfma_takes(*c, &g) && gh_conv_lanes_takes(*c, false, cus, 0);
+      return !(c->flags & GH_FLAG_CONV_PRE) && conv_lanes_takes(*c, cus);
+    }
+    case GH_OP_CONV2D_BWD_DATA: {
+      gh_cmd f;
+      if (f64) return conv64_mirror(*c, &f) && gh_conv_lanes_takes(*c, true, cus, 0);
+      const ConvGeom g = conv_geom(*c);
+      return g.strideH == 1 && g.strideW == 1 && g.dilH * (g.kh - 1) >= g.padH && g.dilW * (g.kw - 1) >= g.padW && conv_lanes_takes_gradient(*c, cus);
+    }
+    case GH_OP_CONV2D_BWD_FILTER: return f64 ? gh_conv_wgrad_takes(*c, cus) : wgrad_mfma_takes(*c, cus);
+  }
+  return 0;
 }
 
 extern "C" int gh_conv2d_can_keep(const gh_cmd* c) {

@@ -364,15 +364,16 @@ GH_API int gh_conv2d_bwd_filter_route(const gh_cmd* conv_bwd_filter);
 enum gh_gemm_route {
   GH_GEMM_ROUTE_SMALL_OUTPUT = 0, /* few output tiles: K split over the wavefronts of a workgroup */
   GH_GEMM_ROUTE_TILE128 = 1,      /* 128 x 128 tiles through LDS                                 */
-  GH_GEMM_ROUTE_TILE64 = 2,       /* tiles of 32 to 128 rows x 64 (see gh_gemm_straight)          */
+  GH_GEMM_ROUTE_TILE64 = 2,       /* tiles of 32 to 128 rows x 64 (see gh_runs_straight)          */
   GH_GEMM_ROUTE_TILE128X64 = 3,
   GH_GEMM_ROUTE_F64 = 4           /* float64 (its own kernels)                                   */
 };
 GH_API int gh_gemm_route(const gh_cmd* gemm, int* splits);
-/* 1 when gh_submit runs this GEMM command, of either type, on a kernel whose operands go from memory
- * straight to the matrix cores or the vector units (k_gemm_direct, k_gemm_thin), 0 where tiles are staged
- * in LDS or a workgroup holds one small tile.  Host only; 256 compute units, as above. */
-GH_API int gh_gemm_straight(const gh_cmd* gemm);
+/* 1 when gh_submit runs this GEMM, CONV2D, CONV2D_BWD_DATA or CONV2D_BWD_FILTER command, of either type, on a kernel
+ * whose operands go from memory straight to the matrix cores or the vector units (k_gemm_direct, k_gemm_thin,
+ * k_conv3x3_lanes, k_conv3x3_wgrad), 0 where they are staged in LDS or by a kernel of another kind, and for every
+ * other command.  Host only; 256 compute units, as above. */
+GH_API int gh_runs_straight(const gh_cmd* cmd);
 
 /* 1 when this GEMM command may carry GH_FLAG_GEMM_SOFTMAX: a float32 product of
  * untransposed operands with at most 32 columns and at most 2048 rows, whose

@@ -10,7 +10,7 @@ from gorgonia_amd import device as D
 
 def _straight(m, n, k, ta=False, tb=False, batch=1):
     cmd = D.cmd_gemm(0x10000, 0x20000, 0x30000, m, n, k, trans_a=ta, trans_b=tb, batch=batch, stride_a=m * k, stride_b=k * n, stride_c=m * n)
-    return _ffi.load().gh_gemm_straight(C.byref(cmd))
+    return _ffi.load().gh_runs_straight(C.byref(cmd))
 
 
 def _slices(m, n, k, ta=False, tb=False):
@@ -39,7 +39,7 @@ def test_slabs_fit_any_scratch():
     assert _slices(600, 850, 9000, True, True) * 600 * 850 * 4 <= 16 << 20 or _straight(600, 850, 9000, True, True) == 1
     assert _straight(64, 64, 64) == 0      # one small tile
     assert _straight(1, 300, 784) == 1     # one row
-    assert _ffi.load().gh_gemm_straight(C.byref(D.cmd_relu(0x1000, 0x2000, 16))) == 0
+    assert _ffi.load().gh_runs_straight(C.byref(D.cmd_relu(0x1000, 0x2000, 16))) == 0
 
 
 @pytest.mark.parametrize("m,n,k,ta,tb,slices", [(36, 907, 2696, False, False, 1), (300, 160, 4580, False, False, 1), (199, 280, 2287, True, False, 1),
