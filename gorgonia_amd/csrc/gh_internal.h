@@ -115,7 +115,7 @@ int gh_launch_fill(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_has_nan_inf(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_gemm(gh_ctx* ctx, const gh_cmd& c);
 // products with operands straight from memory (k_gemm_direct.hip)
-int gh_gemm_direct_form(const gh_cmd& c, int cus, double* us);   // -1: not taken
+int gh_gemm_direct_form(const gh_cmd& c, int cus, double* us, int* rounds);   // -1: not taken
 int gh_gemm_direct_slices(const gh_cmd& c, int form, int cus);
 int gh_launch_gemm_direct(gh_ctx* ctx, const gh_cmd& c, int form);
 // products of one to four rows (k_gemm_thin.hip)

@@ -1402,6 +1402,52 @@ struct LoadKContig64 {
   }
 };
 
+// Operand stored [k][c] with c contiguous (B not transposed; A transposed): a
+// thread takes columns c, c+1 of rows k, k+1 and writes the two k-pairs.
+template <int R, int BK, bool VEC>
+struct LoadMnContig64 {
+  static constexpr int S2 = 2 * R + 8;
+  static constexpr int SIZE = (BK / 2) * S2;
+  static constexpr int TOTAL = (R / 2) * (BK / 2);   // 2x2 cells per tile
+  static constexpr int NV = (TOTAL + kThreads - 1) / kThreads;
+  const double* base; int ld; int rmax; int kmax;
+  f64x2 reg[NV][2];
+  __device__ __forceinline__ void load(int c0, int k0) {
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+      const int f = threadIdx.x + j * kThreads;
+      const int c = c0 + (f % (R / 2)) * 2;
+      const int k = k0 + (f / (R / 2)) * 2;
+      f64x2 v0 = {0.0, 0.0}, v1 = {0.0, 0.0};
+      if ((TOTAL % kThreads == 0 || f < TOTAL) && c < rmax) {
+        const double* p = base + (int64_t)k * ld + c;
+        if (VEC) {
+          if (k < kmax) v0 = *reinterpret_cast<const f64x2*>(p);
+          if (k + 1 < kmax) v1 = *reinterpret_cast<const f64x2*>(p + ld);
+        } else if (c + 1 < rmax) {
+          if (k < kmax) v0 = *reinterpret_cast<const f64x2_a8*>(p);
+          if (k + 1 < kmax) v1 = *reinterpret_cast<const f64x2_a8*>(p + ld);
+        } else {
+          if (k < kmax) v0[0] = p[0];
+          if (k + 1 < kmax) v1[0] = p[ld];
+        }
+      }
+      reg[j][0] = v0;
+      reg[j][1] = v1;
+    }
+  }
+  __device__ __forceinline__ void store(double* lds) const {
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+      const int f = threadIdx.x + j * kThreads;
+      if (TOTAL % kThreads != 0 && f >= TOTAL) continue;
+      double* d = &lds[(f / (R / 2)) * S2 + 4 * (f % (R / 2))];
+      *reinterpret_cast<f64x2*>(d) = f64x2{reg[j][0][0], reg[j][1][0]};
+      *reinterpret_cast<f64x2*>(d + 2) = f64x2{reg[j][0][1], reg[j][1][1]};
+    }
+  }
+};
+
 // The float64 MFMA core: 2x2 wavefronts over a BM x BN block, k-tiles [kt0, kt1).
 template <int BM, int BN, int BK, class LA, class LB>
 __device__ __forceinline__ void dmfma_tile_loop(double* lds, LA& la, LB& lb, int m0, int n0, int kt0, int kt1,
@@ -1549,6 +1595,38 @@ __device__ __forceinline__ void dmfma_tile_loop_auto(double* lds, LA& la, LB& lb
     }
   }
   dmfma_tile_loop<BM, BN, BK, LA, LB>(lds, la, lb, m0, n0, 0, nkt, acc);
+}
+
+template <int BM, int BN, int BK, bool TA, bool TB, bool VEC>
+__global__ __launch_bounds__(kThreads) void k_dgemm(const double* __restrict__ A,
+                                                    const double* __restrict__ B,
+                                                    double* __restrict__ C, int M, int N, int K,
+                                                    int lda, int ldb, int ldc, int64_t sA,
+                                                    int64_t sB, int64_t sC) {
+  using LA = typename std::conditional<TA, LoadMnContig64<BM, BK, VEC>, LoadKContig64<BM, BK, VEC>>::type;
+  using LB = typename std::conditional<TB, LoadKContig64<BN, BK, VEC>, LoadMnContig64<BN, BK, VEC>>::type;
+  constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
+  __shared__ double lds[2 * (LA::SIZE + LB::SIZE)];
+  int tile_m, tile_n, bz;
+  tile_coords(&tile_m, &tile_n, &bz, gridDim.z > 1);
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  LA la; la.base = A + bz * sA; la.ld = lda; la.rmax = M; la.kmax = K;
+  LB lb; lb.base = B + bz * sB; lb.ld = ldb; lb.rmax = N; lb.kmax = K;
+  C += bz * sC;
+  f64x4 acc[TM][TN];
+  dmfma_tile_loop_auto<BM, BN, BK, LA, LB>(lds, la, lb, m0, n0, (K + BK - 1) / BK, acc);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
+  const int lr = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for (int a = 0; a < TM; a++)
+#pragma unroll
+    for (int b = 0; b < TN; b++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int i = m0 + wm + a * 16 + 4 * v + lk, j = n0 + wn + b * 16 + lr;
+        if (i < M && j < N) C[(int64_t)i * ldc + j] = acc[a][b][v];
+      }
 }
 
 // Float64 product with a small result (a dense layer on a batch: too few 64x64
@@ -2989,6 +3067,35 @@ bool gh_try_launch_conv2d_bwd_filter_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
   return true;
 }
 
+template <int BM, int BN, int BK>
+static void launch_dgemm_cfg(gh_ctx* ctx, const gh_cmd& c, int64_t batch) {
+  const int M = (int)c.dim[0], N = (int)c.dim[1], K = (int)c.dim[2];
+  const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM, (unsigned)batch);
+  const double* A = (const double*)(uintptr_t)c.ptr[0];
+  const double* B = (const double*)(uintptr_t)c.ptr[1];
+  double* C = (double*)(uintptr_t)c.ptr[2];
+  const int lda = (int)c.dim[3], ldb = (int)c.dim[4], ldc = (int)c.dim[5];
+  const int64_t sA = batch > 1 ? c.dim[7] : 0, sB = batch > 1 ? c.dim[8] : 0, sC = batch > 1 ? c.dim[9] : 0;
+  const bool ta = c.flags & GH_FLAG_TRANS_A, tb = c.flags & GH_FLAG_TRANS_B;
+  const auto even = [](int64_t v) { return (v & 1) == 0; };
+  const bool vec = even(M) && even(N) && even(K) && even(lda) && even(ldb) && even(sA) && even(sB) &&
+                   ((c.ptr[0] | c.ptr[1]) & 15) == 0;
+#define GH_DGEMM_GO(TA, TB)                                                                                    \
+  do {                                                                                                         \
+    if (vec)                                                                                                   \
+      hipLaunchKernelGGL((k_dgemm<BM, BN, BK, TA, TB, true>), grid, dim3(kThreads), 0, ctx->stream, A, B, C, M, \
+                         N, K, lda, ldb, ldc, sA, sB, sC);                                                     \
+    else                                                                                                       \
+      hipLaunchKernelGGL((k_dgemm<BM, BN, BK, TA, TB, false>), grid, dim3(kThreads), 0, ctx->stream, A, B, C,  \
+                         M, N, K, lda, ldb, ldc, sA, sB, sC);                                                  \
+  } while (0)
+  if (ta && tb) GH_DGEMM_GO(true, true);
+  else if (ta) GH_DGEMM_GO(true, false);
+  else if (tb) GH_DGEMM_GO(false, true);
+  else GH_DGEMM_GO(false, false);
+#undef GH_DGEMM_GO
+}
+
 // Float64: one 16x16 tile per workgroup (k_dgemm_skinny).  AV, BV: the operand is k-contiguous.
 static int launch_dgemm_skinny(gh_ctx* ctx, const gh_cmd& c) {
   const int M = (int)c.dim[0], N = (int)c.dim[1], K = (int)c.dim[2];
@@ -3053,7 +3160,7 @@ static bool gemm_short_k_staged(int64_t M, int64_t N, int64_t K, int64_t batch, 
 static int direct_form(const gh_cmd& c, int cus) {
   if (getenv("GORGONIA_HIP_GEMM_PLAN")) return -1;   // a forced tile plan means the tiled kernel
   double us = 0;
-  const int form = gh_gemm_direct_form(c, cus, &us);
+  const int form = gh_gemm_direct_form(c, cus, &us, nullptr);
   if (form < 0) return -1;
   const int64_t M = c.dim[0], N = c.dim[1], K = c.dim[2], batch = c.dim[6] <= 0 ? 1 : c.dim[6];
   const bool ta = c.flags & GH_FLAG_TRANS_A, tb = c.flags & GH_FLAG_TRANS_B;
@@ -3082,14 +3189,27 @@ static int direct_form(const gh_cmd& c, int cus) {
   return form;
 }
 
-// Which kernel takes a float64 product of more than two rows: a form of k_gemm_direct, or -1 for one 16x16 tile per
-// workgroup (k_dgemm_skinny) where larger tiles leave the device idle: 4.6 us per 1000 of K and 256 tiles.
+// Which kernel takes a float64 product of more than two rows: a form of k_gemm_direct, kStaged64 for tiles staged in LDS
+// (k_dgemm), or -1 for one 16x16 tile per workgroup (k_dgemm_skinny) where larger tiles leave the device idle: 4.6 us per
+// 1000 of K and 256 tiles, and 0.1 us for each 256 (without that it took 2000 x 2000, K = 64: 31 us against 24 and staged 23).
+constexpr int kStaged64 = 100;
 static int gemm64_form(const gh_cmd& c, int cus) {
+  const int64_t M = c.dim[0], N = c.dim[1], K = c.dim[2], batch = std::max<int64_t>(1, c.dim[6]);
   double us = 0;
-  const int form = gh_gemm_direct_form(c, cus, &us);
-  const double tiles16 = (double)cdiv(c.dim[0], 16) * (double)cdiv(c.dim[1], 16);
-  const double small = 4.0 + std::max(1.0, tiles16 / cus) * (double)c.dim[2] * 4.6e-3;
-  return c.dim[6] <= 1 && c.dim[2] >= 64 && small < us ? -1 : form;
+  int rounds = 0;
+  const int form = gh_gemm_direct_form(c, cus, &us, &rounds);
+  // Short contractions: a large tile of k_gemm_direct passes its results through LDS in steps of 16 rows, which is then
+  // most of its time (560 x 1680, K = 12: 7.5 us against 4.7 staged; 104 x 936 x 24, K = 8 11.8 and 7.5; K = 32 1.2 to 1.5 times,
+  // K = 48 1.0 to 1.5 where 16-byte loads stage), as is the start of many small ones (255 x 3906 x 8, K = 12 1.2 times; 1543 x
+  // 777 in five rounds, K = 24 0.9).  Fewer tiles than half the compute units do not fill the staged kernel (300 x 1868, K = 4,
+  // 150 tiles, 5.1 us against 4.4; 128 x 128 x 32, 128 tiles, 4.1 against 4.5).
+  if (form >= 0 && cdiv(M, 64) * cdiv(N, 64) * batch >= 140) {
+    const bool even = ((M | N | K | c.dim[3] | c.dim[4] | (batch > 1 ? c.dim[7] | c.dim[8] : 0)) & 1) == 0 && ((c.ptr[0] | c.ptr[1]) & 15) == 0;
+    if (form > 0 ? K <= 32 || (K <= 48 && even && form > 1) : K <= 16 && rounds > 10) return kStaged64;
+  }
+  const double tiles16 = (double)cdiv(M, 16) * (double)cdiv(N, 16);
+  const double small = 4.0 + std::max(1.0, tiles16 / cus) * ((double)K * 4.6e-3 + 0.1);
+  return batch == 1 && K >= 64 && small < us ? -1 : form;
 }
 
 int gh_launch_gemm(gh_ctx* ctx, const gh_cmd& c) {
@@ -3097,6 +3217,12 @@ int gh_launch_gemm(gh_ctx* ctx, const gh_cmd& c) {
   if (gh_dtype_of(c.flags) == GH_F64) {
     if (gh_gemm_thin_takes(c)) return gh_launch_gemm_thin(ctx, c);
     const int form = gemm64_form(c, ctx->cu_count);
+    if (form == kStaged64) {
+      // 128x128 tiles once they fill the device, 64x64 with a longer k-tile below that
+      if (cdiv(c.dim[0], 128) * cdiv(c.dim[1], 128) * batch >= ctx->cu_count) launch_dgemm_cfg<128, 128, 8>(ctx, c, batch);
+      else launch_dgemm_cfg<64, 64, 16>(ctx, c, batch);
+      return gh_check_hip(ctx, hipGetLastError(), "dgemm launch");
+    }
     return form >= 0 ? gh_launch_gemm_direct(ctx, c, form) : launch_dgemm_skinny(ctx, c);
   }
   if (gh_gemm_thin_takes(c)) return gh_launch_gemm_thin(ctx, c);
@@ -3552,7 +3678,7 @@ extern "C" int gh_runs_straight(const gh_cmd* c) {
   switch (c->opcode) {
     case GH_OP_GEMM:
       if (gh_gemm_thin_takes(*c)) return 1;
-      return f64 ? gemm64_form(*c, cus) >= 0 : !gemm_skinny_takes(*c, cus) && direct_form(*c, cus) >= 0;
+      return f64 ? gemm64_form(*c, cus) >= 0 && gemm64_form(*c, cus) != kStaged64 : !gemm_skinny_takes(*c, cus) && direct_form(*c, cus) >= 0;
     case GH_OP_CONV2D: {
       ConvGeom64 g;
       if (f64) return conv64_mfma_takes(*c, &g) && gh_conv_lanes_takes(*c, false, cus, 0);

@@ -236,8 +236,8 @@ static const Form kForms64[] = {{2, 2, true, 2.28, 0.17}, {2, 4, true, 2.00, 0.1
                                 {5, 4, true, 1.90, 0.17}};
 
 // Whether k_gemm_direct takes a product - at least one whole group of rows and columns, a tile's offsets in 32 bits -
-// and the quickest form for it: its number, and its time in *us.
-int gh_gemm_direct_form(const gh_cmd& c, int cus, double* us) {
+// and the quickest form for it: its number, its time in *us and its rounds of tiles over the compute units.
+int gh_gemm_direct_form(const gh_cmd& c, int cus, double* us, int* rounds) {
   const bool f64 = gh_dtype_of(c.flags) == GH_F64;
   const int64_t M = c.dim[0], N = c.dim[1], K = c.dim[2], batch = c.dim[6] <= 0 ? 1 : c.dim[6];
   const int v = f64 ? 2 : 4;
@@ -252,7 +252,10 @@ int gh_gemm_direct_form(const gh_cmd& c, int cus, double* us) {
     const int64_t tiles = (M + 16 * f.tm - 1) / (16 * f.tm) * ((N + 16 * f.tn - 1) / (16 * f.tn)) * batch;
     const double per_k = f.per_k * (f64 && along_k && f.tm == 2 ? (f.tn == 2 ? 1.5 : 1.3) : 1.0);
     const double est = 4.0 + (double)((tiles + cus - 1) / cus) * f.tm * f.tn * ((double)K * 1e-3 * per_k + f.per_tile);
-    if (best < 0 || est < *us) { *us = est; best = i; }
+    if (best >= 0 && est >= *us) continue;
+    *us = est;
+    best = i;
+    if (rounds) *rounds = (int)((tiles + cus - 1) / cus);
   }
   return best;
 }

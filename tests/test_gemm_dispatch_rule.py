@@ -1,4 +1,4 @@
-"""Which float32 products take their operands straight from memory and which are staged through LDS tiles, at shapes
+"""Which products take their operands straight from memory and which are staged through LDS tiles, at shapes
 where either was measured to be the slower by a tenth and more."""
 import ctypes as C
 
@@ -71,3 +71,14 @@ def test_short_contractions_over_many_aligned_tiles_are_staged(m, n, batch, ta, 
     (12, 9, 27, False, True, 24, 1)])
 def test_short_contractions(m, n, k, ta, tb, batch, straight):
     assert _straight(m, n, k, ta, tb, batch) == straight
+
+
+@pytest.mark.parametrize("m,n,k,batch,straight", [
+    (560, 1680, 12, 1, 0), (104, 936, 8, 24, 0), (1416, 3936, 16, 5, 0), (2000, 2000, 32, 1, 0), (2000, 2000, 48, 1, 0), (160, 499, 16, 16, 0),
+    (255, 3906, 12, 8, 0), (300, 1868, 4, 1, 0),                                                     # staged
+    (160, 499, 48, 16, 1), (128, 128, 5, 32, 1), (2000, 2000, 64, 1, 1), (1416, 3936, 64, 1, 1), (1543, 777, 24, 1, 1), (500, 500, 8, 1, 1), (300, 40, 12, 5, 1),
+    (777, 1543, 1021, 1, 1),
+    (64, 64, 64, 1, 0), (100, 100, 500, 1, 0)])                                # a tile a workgroup
+def test_float64(m, n, k, batch, straight):
+    cmd = D.cmd_gemm(0x10000, 0x20000, 0x30000, m, n, k, batch=batch, stride_a=m * k, stride_b=k * n, stride_c=m * n, dtype=_ffi.F64)
+    assert _ffi.load().gh_runs_straight(C.byref(cmd)) == straight
