@@ -128,7 +128,10 @@ int gh_init(int device, int64_t arena_bytes, gh_ctx** out) {
   }
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) ctx->cu_count = prop.multiProcessorCount;
-  if (const char* sm = getenv("GORGONIA_HIP_SYNC")) ctx->sync_block = strcmp(sm, "block") == 0;
+  if (const char* sm = getenv("GORGONIA_HIP_SYNC")) {
+    ctx->sync_block = strcmp(sm, "block") == 0;
+    ctx->sync_spin = strcmp(sm, "spin") == 0;
+  }
   ctx->done_word = take_word();
   if (arena_bytes > 0) {
     size_t free_b = 0, total_b = 0;
@@ -453,7 +456,13 @@ int gh_sync(gh_ctx* ctx) {
   }
   ctx->done_seq = seq;
   if (!seen) {
-    const hipError_t e = hipStreamSynchronize(ctx->stream);
+    hipError_t e;
+    if (ctx->sync_spin) {   // the thread keeps its core however long it takes
+      while ((e = hipStreamQuery(ctx->stream)) == hipErrorNotReady) {
+      }
+    } else {
+      e = hipStreamSynchronize(ctx->stream);
+    }
     if (e != hipSuccess) {
       gh_check_hip(ctx, e, "hipStreamSynchronize");
       return ctx->err;

@@ -68,6 +68,7 @@ struct gh_ctx {
   bool idle = true;         // nothing has been put on the stream since the last completed gh_sync
   bool runtime_wait = false;  // a copy to or from pageable memory is under way: the runtime has its own part in finishing it
   bool sync_block = false;  // gh_sync waits in the runtime only
+  bool sync_spin = false;   // gh_sync never gives up its core: where it would leave the wait to the runtime it asks the stream again and again
   gh_llc_model llc;
   // pinned host buffers handed out by gh_host_alloc: [start, end)
   std::vector<std::pair<uint64_t, uint64_t>> host_ranges;
