@@ -92,7 +92,8 @@ int gh_validate_cmd(const gh_cmd& c, std::string& msg);
 // inputs lost (`cold`) or not, goes past the cache (k_elem.hip)
 bool gh_llc_cold(const gh_ctx* ctx, uint64_t p);
 bool gh_llc_stream(int64_t bytes, bool cold);
-// a run of elementwise commands in one pass (k_chain.hip): how many commands at the front of cmds (0 or >= 2), and the launch
+// a run of elementwise commands in one pass (k_chain.hip): how many commands at the front of cmds one pass can take and is
+// quicker for (0 or >= 2; gh_elementwise_run asks the same), and the launch
 int gh_chain_length(const gh_cmd* cmds, int n);
 int gh_launch_chain(gh_ctx* ctx, const gh_cmd* cmds, int count);
 int gh_launch_elem_bin(gh_ctx* ctx, const gh_cmd& c);

@@ -3,7 +3,7 @@
 // A pass over B and nothing else, so a workgroup takes 16 columns (of float64 the same 16) and all of K: lane (kk, cg)
 // of a wavefront reads four neighbouring columns of every 128th row, 4 rows or more in flight, and the 128 partial sums
 // of a result meet in the wavefront and then in LDS, in a fixed order.  The MFMA kernels give 32 columns to a workgroup
-// and all rows of a 16- or 32-row tile to the matrix cores, of which one to eight hold anything; their walk over K is
+// and all rows of a 16- or 32-row tile to the matrix cores, of which one to four hold anything; their walk over K is
 // eight times as long.  Bound by the latency of its two or three rounds of loads and the launch.
 // 1 x 784 . 784 x 300 with x in pinned host memory: 8.6 us (14.2); 1 x 300 . 300 x 100: 3.8 (4.7).
 #include <cstdlib>

@@ -1,5 +1,7 @@
-"""k_conv3x3_wgrad: the 3x3 stride-1 filter gradient whose operands go from memory straight to the matrix cores,
-at the edges of its chunks, tiles and slices, against a float64 sum over shifted images."""
+"""3x3 stride-1 filter gradients at the edges of the chunks, tiles and slices of k_conv3x3_wgrad, whose operands go from
+memory straight to the matrix cores, against a float64 sum over shifted images.  Each shape runs on the kernel that the
+dispatch finds the quicker; the shapes that must run on the one or the other are in
+tests/test_gpu_conv_filter_gradient_edges.py."""
 import numpy as np
 import pytest
 
