@@ -3155,7 +3155,15 @@ static bool gemm_short_k_staged(int64_t M, int64_t N, int64_t K, int64_t batch, 
   return tb ? K <= 300 && 5 * tiles >= 9 * cus : K <= 256 && tiles >= 3 * cus;
 }
 
-// Which kernel takes a float32 product that is none of the small-output ones: -1 for the LDS-tiled kernel under
+// 128x128 tiles through LDS where they fill the device: 68 us per 1000 of K and round of tiles, half as much again
+// with one workgroup per compute unit and nothing to run under its barriers.
+static double tile128_us(const gh_cmd& c, bool vec, int cus) {
+  const int64_t tiles = cdiv(c.dim[0], 128) * cdiv(c.dim[1], 128) * std::max<int64_t>(1, c.dim[6]), rounds = cdiv(tiles, cus);
+  if (tiles < cus || c.dim[0] <= 64) return 1e30;
+  return 6.0 + (double)rounds * 64.0 * ((double)c.dim[2] * 1e-3 * 1.06 + 0.05) * (rounds == 1 ? 1.35 : 1.0) * (vec ? 1.0 : 1.25);
+}
+
+// Which float32-instruction kernel takes a product that is none of the small-output ones: -1 for the LDS-tiled kernel under
 // plan_tiles, else a form of k_gemm_direct.
 static int direct_form(const gh_cmd& c, int cus) {
   if (getenv("GORGONIA_HIP_GEMM_PLAN")) return -1;   // a forced tile plan means the tiled kernel
@@ -3178,15 +3186,14 @@ static int direct_form(const gh_cmd& c, int cus) {
                          (double)(M * N * slices) * 1e-6;
     if (slices > 1 && slices * M * N * 4 <= GH_NOALLOC_SCRATCH_BYTES && slabs + 4.0 < us && slabs < 0.95 * us) return -1;
   }
-  // 128x128 tiles through LDS where they fill the device: 68 us per 1000 of K and round of tiles, half as much again
-  // with one workgroup per compute unit and nothing to run under its barriers.
-  const int64_t big = cdiv(M, 128) * cdiv(N, 128) * batch;
-  if (big >= cus && M > 64) {
-    const int64_t rounds = cdiv(big, cus);
-    const double est = 6.0 + (double)rounds * 64.0 * ((double)K * 1e-3 * 1.06 + 0.05) * (rounds == 1 ? 1.35 : 1.0) * (vec ? 1.0 : 1.25);
-    if (est < us) return -1;
-  }
-  return form;
+  return tile128_us(c, vec, cus) < us ? -1 : form;
+}
+
+// The form of k_gemm_split that takes a float32 product that is none of the small-output ones, or -1.
+static int split_form(const gh_cmd& c, int cus) {
+  if (getenv("GORGONIA_HIP_GEMM_PLAN") || getenv("GORGONIA_HIP_NO_SPLIT")) return -1;
+  double us = 0;
+  return gh_gemm_direct_form(c, cus, &us, nullptr) < 0 ? -1 : gh_gemm_split_form(c, cus, std::min(us, tile128_us(c, true, cus)));
 }
 
 // Which kernel takes a float64 product of more than two rows: a form of k_gemm_direct, kStaged64 for tiles staged in LDS
@@ -3230,6 +3237,8 @@ int gh_launch_gemm(gh_ctx* ctx, const gh_cmd& c) {
   if (rs >= 0) return rs;
   if (c.flags & GH_FLAG_GEMM_SOFTMAX)
     return gh_fail(ctx, GH_EINVAL, "gemm: no fused softmax for this shape (see gh_gemm_can_softmax)");
+  const int split = split_form(c, ctx->cu_count);
+  if (split >= 0) return gh_launch_gemm_split(ctx, c, split);
   const int form = direct_form(c, ctx->cu_count);
   if (form >= 0) return gh_launch_gemm_direct(ctx, c, form);
   const TilePlan p = plan_tiles(ctx, c.dim[0], c.dim[1], c.dim[2], batch, false);
@@ -3669,6 +3678,13 @@ extern "C" int gh_conv2d_bwd_filter_route(const gh_cmd* c) {
   if (conv_direct_shape(*c) && c->dim[4] <= 65535) return GH_WGRAD_ROUTE_DIRECT;
   if (gh_conv_wgrad_small_takes(*c)) return GH_WGRAD_ROUTE_SMALL;
   return GH_WGRAD_ROUTE_GEMM;
+}
+
+extern "C" int gh_runs_split(const gh_cmd* c) {
+  if (!c || gh_dtype_of(c->flags) != GH_F32) return 0;
+  const int cus = gh_ctx{}.cu_count;   // the MI355X's
+  if (c->opcode == GH_OP_GEMM) return !gh_gemm_thin_takes(*c) && !gemm_skinny_takes(*c, cus) && split_form(*c, cus) >= 0;
+  return 0;
 }
 
 extern "C" int gh_runs_straight(const gh_cmd* c) {

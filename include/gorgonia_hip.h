@@ -374,6 +374,10 @@ GH_API int gh_gemm_route(const gh_cmd* gemm, int* splits);
  * k_conv3x3_lanes, k_conv3x3_wgrad), 0 where they are staged in LDS or by a kernel of another kind, and for every
  * other command.  Host only; 256 compute units, as above. */
 GH_API int gh_runs_straight(const gh_cmd* cmd);
+/* 1 when gh_submit runs this float32 GEMM command on the bf16 matrix instructions, its
+ * values split into three bf16 parts each (k_gemm_split); the queries above then name the kernel of the float32
+ * instructions that it would run on otherwise.  Host only; 256 compute units, as above. */
+GH_API int gh_runs_split(const gh_cmd* cmd);
 
 /* 1 when this GEMM command may carry GH_FLAG_GEMM_SOFTMAX: a float32 product of
  * untransposed operands with at most 32 columns and at most 2048 rows, whose

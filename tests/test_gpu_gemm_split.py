@@ -1,0 +1,121 @@
+"""k_gemm_split: float32 products on the bf16 matrix instructions, values split into three bf16 parts.  Every form
+at edges of its tiles, steps and parts of K, transposes, leading dimensions, operands that are only 4-byte aligned, batches,
+epilogues, and the values the split cannot hold (infinities, NaN, the largest), against float64 products."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from gorgonia_amd import _ffi
+from gorgonia_amd import device as D
+from tests.util import rel_frobenius
+
+pytestmark = pytest.mark.gpu
+
+# 256 x 256; 128 x 128; the same in two parts of K; 64 x 64 in two parts; in four
+SHAPES = [(3800, 4001, 131, 1), (640, 650, 18, 40), (2047, 2049, 95, 1), (2000, 2000, 47, 1), (2176, 1900, 64, 1), (1025, 1023, 129, 4),
+          (255, 513, 97, 30), (1200, 2100, 333, 1), (500, 500, 500, 8), (1000, 1000, 1025, 1), (1024, 1024, 1024, 1)]
+
+
+def _cmd(pa, pb, pc, m, n, k, batch, **kw):
+    cmd = D.cmd_gemm(pa, pb, pc, m, n, k, batch=batch, **kw)
+    assert _ffi.load().gh_runs_split(C.byref(cmd)) == 1, (m, n, k, batch)
+    return cmd
+
+
+def _run(ctx, a, b, m, n, k, batch=1, ta=False, tb=False, pad=0, shift=0, **kw):
+    """a, b: what lies in memory, (batch, rows, columns + pad); shift: floats in front of each tensor."""
+    front = np.full(shift, np.nan, np.float32)
+    held = [ctx.upload(np.concatenate([front, t.ravel()]) if shift else t) for t in (a, b)]
+    pc = ctx.upload(np.full(batch * m * (n + pad) + shift, np.nan, np.float32))
+    o = 4 * shift
+    ctx.run(_cmd(held[0] + o, held[1] + o, pc + o, m, n, k, batch, trans_a=ta, trans_b=tb, lda=a.shape[2], ldb=b.shape[2], ldc=n + pad,
+                 stride_a=a[0].size, stride_b=b[0].size, stride_c=m * (n + pad), **kw))
+    got = ctx.d2h(pc + o, (batch, m, n + pad))
+    for p in held + [pc]:
+        ctx.free(p)
+    assert pad == 0 or np.isnan(got[:, :, n:]).all()   # nothing is stored past the columns
+    return got[:, :, :n]
+
+
+def _inputs(m, n, k, batch, ta, tb, pad=0, seed=0):
+    rng = np.random.default_rng(m * 7 + n * 3 + k + batch + seed)
+    a = rng.standard_normal((batch, k if ta else m, (m if ta else k) + pad), np.float32)
+    b = rng.standard_normal((batch, n if tb else k, (k if tb else n) + pad), np.float32)
+    x, y = a[:, :, :a.shape[2] - pad].astype(np.float64), b[:, :, :b.shape[2] - pad].astype(np.float64)
+    return a, b, (x.transpose(0, 2, 1) if ta else x), (y.transpose(0, 2, 1) if tb else y)
+
+
+# 16 k are summed exactly but for one rounding of the sum, 2^-24 of its size at most, a third of that on average, and the roundings
+# add up as their root: K = 1025 gives sqrt(65) * 2^-24 / sqrt(3) * sqrt(1/2) = 2.0e-7; six times that with all six products in
+# one sum, where K is at most 131 here.
+@pytest.mark.parametrize("m,n,k,batch", SHAPES)
+def test_product(ctx, m, n, k, batch):
+    for ta, tb in ((False, False), (True, False), (False, True), (True, True)):
+        a, b, x, y = _inputs(m, n, k, batch, ta, tb)
+        assert rel_frobenius(_run(ctx, a, b, m, n, k, batch, ta, tb), np.matmul(x, y)) <= 3e-7, (ta, tb)
+
+
+@pytest.mark.parametrize("m,n,k,batch", [(2176, 1900, 64, 1), (500, 500, 500, 8)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+def test_wider_leading_dimensions_at_any_float(ctx, m, n, k, batch, ta, tb):
+    a, b, x, y = _inputs(m, n, k, batch, ta, tb, pad=3)
+    assert rel_frobenius(_run(ctx, a, b, m, n, k, batch, ta, tb, pad=3, shift=1), np.matmul(x, y)) <= 3e-7
+
+
+def test_whole_numbers_are_exact(ctx):
+    rng = np.random.default_rng(3)
+    a, b = (rng.integers(-60, 61, s).astype(np.float32) for s in ((1, 1024, 1024), (1, 1024, 1024)))
+    assert np.array_equal(_run(ctx, a, b, 1024, 1024, 1024), np.matmul(a.astype(np.float64), b.astype(np.float64)))
+
+
+def test_bias_and_activation(ctx):
+    m, n, k = 2000, 2000, 47
+    a, b, _, _ = _inputs(m, n, k, 1, False, False)
+    bias = np.random.default_rng(1).standard_normal(n, np.float32)
+    bare, pb = _run(ctx, a, b, m, n, k), ctx.upload(bias)
+    z = bare + bias
+    assert np.array_equal(_run(ctx, a, b, m, n, k, bias=pb, act="relu"), z * (z >= 0))
+    assert np.array_equal(_run(ctx, a, b, m, n, k, act="leaky", alpha=0.1), bare * (bare >= 0) + (bare * (bare < 0)) * np.float32(0.1))
+    ctx.free(pb)
+
+
+@pytest.mark.parametrize("m,n,k,batch", [(640, 650, 18, 40), (500, 500, 500, 8)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
+def test_values_the_split_cannot_hold(ctx, m, n, k, batch, ta, tb):
+    """Infinities, NaN, values and sums that only float32 itself can hold: their tiles come from the float32 instructions."""
+    a, b, x, y = _inputs(m, n, k, batch, ta, tb)
+    x, y = np.ascontiguousarray(x), np.ascontiguousarray(y)
+    x[0, 3, 1], x[1, m - 1, k - 1], y[1, 2, 77] = np.inf, np.nan, -np.inf
+    x[2, 40], y[2, :, 9] = 2e38 / k, 1.0        # a row of the largest values, a column that keeps their sum in range
+    y[3, :, n - 1] *= np.float32(1e30)
+    x, y = x.astype(np.float32), y.astype(np.float32)
+    a = np.ascontiguousarray(x.transpose(0, 2, 1) if ta else x)
+    b = np.ascontiguousarray(y.transpose(0, 2, 1) if tb else y)
+    got = _run(ctx, a, b, m, n, k, batch, ta, tb)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = np.matmul(x.astype(np.float64), y.astype(np.float64))
+        # a sum beyond float32 is an infinity wherever its partial sums overflow, which is a matter of order: left out near the limit
+        sure = ~(np.abs(want) > 1e38) | np.isinf(want)
+        sure[2, 40] = False
+        sure[2, 40, 9] = True
+        want32 = want.astype(np.float32)
+        assert np.array_equal(np.isnan(got[sure]), np.isnan(want32[sure]))
+        assert np.array_equal(np.where(np.isinf(got), got, 0)[sure], np.where(np.isinf(want32), want32, 0)[sure])
+    fin = sure & np.isfinite(want32)
+    assert abs(got[2, 40, 9] / want[2, 40, 9] - 1) <= 1e-6
+    for z in range(4):
+        for cols in (slice(0, n - 1), slice(n - 1, n)):
+            f = fin[z, :, cols].copy()
+            f[40] &= z != 2
+            assert rel_frobenius(got[z, :, cols][f], want[z, :, cols][f]) <= 1e-6
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e-36, 1e-39])
+def test_small_and_denormal_values_keep_their_bits(ctx, scale):
+    m, n, k = 1024, 1024, 1024
+    a, b, _, _ = _inputs(m, n, k, 1, False, False)
+    a = (a.astype(np.float64) * scale).astype(np.float32)
+    want = np.matmul(a.astype(np.float64), b.astype(np.float64))
+    # results below 2^-126 are rounded to multiples of 2^-149
+    assert np.abs(_run(ctx, a, b, m, n, k) - want).max() <= 2e-6 * np.abs(want).max() + 2.0 ** -149
