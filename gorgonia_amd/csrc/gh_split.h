@@ -15,6 +15,8 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
+#include <utility>
 
 namespace gh_split {
 
@@ -29,26 +31,35 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr float kUp = 65536.0f;                          // of each operand
 constexpr float kDown = 1.0f / (65536.0f * 65536.0f);   // of a product
 
-// two values to their three parts, each part of the two in one register
-__device__ __forceinline__ void pair(float x0, float x1, uint32_t* h, uint32_t* m, uint32_t* l) {
-  f32x2 r = {x0 * kUp, x1 * kUp};
-  uint32_t* const out[3] = {h, m, l};
-#pragma unroll
-  for (int p = 0; p < 3; p++) {
-    const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
-    *out[p] = u;
-    r[0] -= __builtin_bit_cast(float, u << 16);
-    r[1] -= __builtin_bit_cast(float, u & 0xffff0000u);
+// f(0), f(1), ... f(N - 1), each with its number as a constant
+template <class F, int... I>
+__device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, class F>
+__device__ __forceinline__ void each(F&& f) { each_of(f, std::make_integer_sequence<int, (N > 0 ? N : 0)>{}); }
+
+// Two values to their parts, a part of both in one register, in eight stages of one or two vector instructions.  An
+// instruction that waits for the one before it costs a wavefront eight cycles; so the stages of a pair go behind one
+// matrix instruction each, next to other stages of other pairs.
+struct Pair {
+  f32x2 rest, top;
+  uint32_t part[3];
+  template <int STAGE>
+  __device__ __forceinline__ void stage(float x0, float x1) {
+    if constexpr (STAGE == 0) rest = f32x2{x0 * kUp, x1 * kUp};
+    if constexpr (STAGE == 1 || STAGE == 4 || STAGE == 7) part[STAGE / 3] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, bf16x2));
+    if constexpr (STAGE == 2 || STAGE == 5) top = f32x2{__builtin_bit_cast(float, part[STAGE / 3] << 16), __builtin_bit_cast(float, part[STAGE / 3] & 0xffff0000u)};
+    if constexpr (STAGE == 3 || STAGE == 6) { rest[0] -= top[0]; rest[1] -= top[1]; }
   }
-}
+};
+constexpr int kStages = 8;
 
 // eight values that follow each other in k: one operand register group per part
 __device__ __forceinline__ void eight(const float* x, u32x4* h, u32x4* m, u32x4* l) {
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    uint32_t a, b, c;
-    pair(x[2 * i], x[2 * i + 1], &a, &b, &c);
-    (*h)[i] = a; (*m)[i] = b; (*l)[i] = c;
+    Pair p;
+    each<kStages>([&](auto k) { p.template stage<decltype(k)::value>(x[2 * i], x[2 * i + 1]); });
+    (*h)[i] = p.part[0]; (*m)[i] = p.part[1]; (*l)[i] = p.part[2];
   }
 }
 

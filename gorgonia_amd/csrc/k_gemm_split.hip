@@ -3,10 +3,12 @@
 //
 // A workgroup owns a tile of the result; the operands' values are split into their bf16 parts on the way from memory to
 // LDS, once per workgroup that needs them.  That is what the tile's size buys: at 256 x 256 a lane converts 16 values
-// (104 vector instructions, which the SIMD does not issue under a matrix instruction of another wavefront)
-// for 48 matrix instructions, at 64 x 64 for 12.  Smaller products have too few such tiles for the compute units: theirs
-// are smaller, and K is cut into parts inside the workgroup, each with wavefronts and LDS buffers of its own, whose
-// sums are added in LDS at the end.  Which form runs depends on the shape only.
+// (104 vector instructions) for 48 matrix instructions, at 64 x 64 for 12.  A wavefront issues a vector instruction every
+// five cycles under its matrix instructions, if it does not wait for the one before: the stages of several pairs of values
+// are interleaved, one to a matrix instruction (in a row, pair by pair: 622 us for 4096 x 4096 x 4096, 108 for 2048).
+// Smaller products have too few such tiles for the compute units: theirs are smaller, and K is cut into parts inside the
+// workgroup, each with wavefronts and LDS buffers of its own, whose sums are added in LDS at the end.  Which form runs
+// depends on the shape only.
 //
 // Error against 64-bit sums, next to the float32 kernels': 4096 x 4096 x 4096 normal values 1.00e-6 (1.15e-6), uniform
 // ones 5.3e-7 (8.4e-7).  All forms but the 256 x 256 one, which has no registers for it, sum the five smaller products
@@ -14,7 +16,6 @@
 // 1.9e-7 (4.0e-7 on k_gemm_direct, which cuts K four ways); with one sum it was 4.9e-7.
 #include <algorithm>
 #include <type_traits>
-#include <utility>
 
 #include "gh_conv_common.h"
 #include "gh_internal.h"
@@ -81,26 +82,20 @@ struct Operand {
       reg[j][e] = past ? 0.0f : v;
     }
   }
-  // two of a thread's values to their parts; the last two of a unit write it
+  // stage K of pair I of a thread's values; the last stage of a unit's last pair stores the unit
   static constexpr int kPairs = 4 * kPer;
-  u32x4 part[3];
-  __device__ __forceinline__ void convert(int i, u32x4* lds) {
-    const int j = i / 4, e = i % 4;
-    uint32_t h, m, l;
-    pair(reg[j][2 * e], reg[j][2 * e + 1], &h, &m, &l);
-    part[0][e] = h; part[1][e] = m; part[2][e] = l;
-    if (e == 3) {
-#pragma unroll
-      for (int p = 0; p < 3; p++) lds[p * kPart + slot[j]] = part[p];
+  u32x4 part[kPer][3];
+  Pair pairs[kPairs];
+  template <int I, int K>
+  __device__ __forceinline__ void convert(u32x4* lds) {
+    constexpr int j = I / 4, e = I % 4;
+    pairs[I].template stage<K>(reg[j][2 * e], reg[j][2 * e + 1]);
+    if constexpr (K == 1 || K == 4 || K == 7) {
+      part[j][K / 3][e] = pairs[I].part[K / 3];
+      if constexpr (e == 3) lds[(K / 3) * kPart + slot[j]] = part[j][K / 3];
     }
   }
 };
-
-// f(0), f(1), ... f(N - 1), each with its number as a constant
-template <class F, int... I>
-__device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
-template <int N, class F>
-__device__ __forceinline__ void each(F&& f) { each_of(f, std::make_integer_sequence<int, (N > 0 ? N : 0)>{}); }
 
 // sixteen results of a 32 x 32 tile: the rows i, i + 1, i + 2, i + 3, i + 8, ... of column j
 __device__ __forceinline__ void put(const Args& g, float* C, int i, int j, f32x16 v, float scale, float bias) {
@@ -193,10 +188,8 @@ __global__ __launch_bounds__(WM * WN * KS * 64, 2) void k_gemm_split(Args g) {
   };
   for (int s = 0; s < 2 && s < steps; s++) {
     load(s);
-#pragma unroll
-    for (int i = 0; i < OA::kPairs; i++) oa.convert(i, lds + s * kBuf);
-#pragma unroll
-    for (int i = 0; i < OB::kPairs; i++) ob.convert(i, lds + s * kBuf + OA::kUnits);
+    each<OA::kPairs * kStages>([&](auto i) { oa.template convert<decltype(i)::value / kStages, decltype(i)::value % kStages>(lds + s * kBuf); });
+    each<OB::kPairs * kStages>([&](auto i) { ob.template convert<decltype(i)::value / kStages, decltype(i)::value % kStages>(lds + s * kBuf + OA::kUnits); });
   }
   if (steps > 2) load(2);
   __syncthreads();
@@ -237,18 +230,20 @@ __global__ __launch_bounds__(WM * WN * KS * 64, 2) void k_gemm_split(Args g) {
       if constexpr (i >= 4 * T && i < 4 * T + TN) fb[2][i - 4 * T] = read_b(next, 2, i - 4 * T);
       if constexpr (i >= 5 * T && i < 5 * T + TN) { fb[1][i - 5 * T] = read_b(next, 1, i - 5 * T); nb[i - 5 * T] = read_b(next, 0, i - 5 * T); }
       if constexpr (CONV) {
-        constexpr int c0 = i * kPairs / (NM - 1), c1 = (i + 1) * kPairs / (NM - 1);
-        each<(c1 < kPairs ? c1 : kPairs) - c0>([&](auto n) {
-          constexpr int c = c0 + decltype(n)::value;
-          if constexpr (c < OA::kPairs) {
-            oa.convert(c, then);
-            if constexpr (c % 4 == 3 && LOAD == 1) oa.load(c / 4, k_of(s + 3));
-            if constexpr (c % 4 == 3 && LOAD == 2) oa.load_end(c / 4, k_of(s + 3), g.K);
-          } else {
-            constexpr int d = c - OA::kPairs;
-            ob.convert(d, then + OA::kUnits);
-            if constexpr (d % 4 == 3 && LOAD == 1) ob.load(d / 4, k_of(s + 3));
-            if constexpr (d % 4 == 3 && LOAD == 2) ob.load_end(d / 4, k_of(s + 3), g.K);
+        // pair c begins behind instruction c kLast / (kPairs - 1), a stage to an instruction; the last stores have some
+        // instructions to go before the barrier waits for them
+        constexpr int kLast = NM - kStages - (NM >= 24 ? 4 : 0);
+        each<kPairs>([&](auto n) {
+          constexpr int c = decltype(n)::value, k = i - c * kLast / (kPairs - 1), d = c - OA::kPairs;
+          if constexpr (k >= 0 && k < kStages) {
+            if constexpr (c < OA::kPairs) oa.template convert<c, k>(then);
+            else ob.template convert<d, k>(then + OA::kUnits);
+          }
+          if constexpr (k == 0 && c % 4 == 3) {   // a unit's values are taken: the loads of the step behind
+            if constexpr (c < OA::kPairs && LOAD == 1) oa.load(c / 4, k_of(s + 3));
+            if constexpr (c < OA::kPairs && LOAD == 2) oa.load_end(c / 4, k_of(s + 3), g.K);
+            if constexpr (c >= OA::kPairs && LOAD == 1) ob.load(d / 4, k_of(s + 3));
+            if constexpr (c >= OA::kPairs && LOAD == 2) ob.load_end(d / 4, k_of(s + 3), g.K);
           }
         });
       }
@@ -329,18 +324,18 @@ void launch(hipStream_t stream, const Args& g, int batch, bool ta, bool tb) {
 // unit, and their times in us: per tile and step of 16 k (of each part) with a compute unit full of workgroups, the
 // same for those that do not fill one (per_odd once, and for each of them), and per tile.  Fitted to 600 products of 16 to
 // 4096 a side and batches of up to 64; nine in ten of the estimates are within 9 % of the times.  4096 x 4096 x 4096
-// takes 610 us on the 256 x 256 tiles (float32 instructions 1122; 1.35 PFLOP/s of bf16 products at the clock the chip
-// holds under them: the same inputs all zero 476), 720 on 128 x 128 and 950 on 64 x 64, where every wavefront
-// converts more of what it multiplies; 2048 x 2048 x 2048 95 with K in two parts, 107 in one (float32 145); 64 of
-// 512 x 512 x 512 85 (150); 1024 x 1024 x 1024 21 with K in four parts (25).
+// takes 575 us on the 256 x 256 tiles (float32 instructions 1122; 1.43 PFLOP/s of bf16 products at the clock the chip
+// holds under them: where it need not save power a step takes 1.53 us, the matrix instructions alone 1.57), 675 on 128 x 128
+// and 950 on 64 x 64, where every wavefront converts more of what it multiplies; 2048 x 2048 x 2048 91 with K in two parts,
+// 95 in one (float32 145); 64 of 512 x 512 x 512 82 (150); 1024 x 1024 x 1024 19 with K in four parts (25).
 struct Form { int rows, cols, parts, share; double per_step, per_odd, per_tile, start; };
-static const Form kForms[] = {{256, 256, 1, 1, 1.69, 0, 4.28, 4.3}, {128, 128, 1, 2, 0.583, 0.349, 3.5, 2.4}, {128, 128, 2, 1, 1.09, 0, 7.6, 0},
-                              {64, 64, 2, 2, 0.444, 0.306, 1.58, 3.2}, {64, 64, 4, 1, 0.931, 0, 4.5, 1.1}};
+static const Form kForms[] = {{256, 256, 1, 1, 1.53, 0, 4.5, 4.5}, {128, 128, 1, 2, 0.604, 0.312, 2.75, 3.3}, {128, 128, 2, 1, 1.07, 0, 7.3, 0},
+                              {64, 64, 2, 2, 0.438, 0.274, 1.54, 3.4}, {64, 64, 4, 1, 0.895, 0, 4.6, 1.1}};
 
 // The form for a float32 product whose quickest kernel on the float32 instructions takes other_us by its estimate, or -1.
 // Below 9 us the launch and the first loads are what either kernel takes, and the estimates no help (1241 x 199,
-// K = 90 6.4 us against 6.0); of 376 products offered to
-// the rule none that it took, at 0.93 of that estimate and less, was slower by 3 %, and together they took 0.92 of the time.
+// K = 90 6.4 us against 6.0); of 450 products offered to the rule one that it took, at 0.93 of that estimate and less,
+// was slower, by 4 %, and together they took 0.92 of the time.
 int gh_gemm_split_form(const gh_cmd& c, int cus, double other_us) {
   const int64_t M = c.dim[0], N = c.dim[1], K = c.dim[2], batch = c.dim[6] <= 0 ? 1 : c.dim[6];
   // at least one whole step; offsets inside a tile in 32 bits; a launch of one dimension
