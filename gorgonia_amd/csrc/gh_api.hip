@@ -395,8 +395,11 @@ static int submit_cmds(gh_ctx* ctx, const gh_cmd* cmds, int n) {
       i += run - 1;
       continue;
     }
-    rc = dispatch(ctx, cmds[i]);
+    // two commands of which the second reads what the first writes are one launch where a kernel takes both
+    const bool pair = gh_is_pair(cmds + i, n - i);
+    rc = pair ? gh_launch_pair(ctx, cmds + i) : dispatch(ctx, cmds[i]);
     if (rc) return rc;
+    if (pair) i++;
   }
   return GH_OK;
 }

@@ -96,6 +96,9 @@ bool gh_llc_stream(int64_t bytes, bool cold);
 // quicker for (0 or >= 2; gh_elementwise_run asks the same), and the launch
 int gh_chain_length(const gh_cmd* cmds, int n);
 int gh_launch_chain(gh_ctx* ctx, const gh_cmd* cmds, int count);
+// two commands in one launch (k_pairs.hip)
+bool gh_is_pair(const gh_cmd* cmds, int n);
+int gh_launch_pair(gh_ctx* ctx, const gh_cmd* cmds);
 int gh_launch_elem_bin(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_elem_unary(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_bcast_bin(gh_ctx* ctx, const gh_cmd& c);
