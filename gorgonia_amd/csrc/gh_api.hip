@@ -151,12 +151,14 @@ int gh_init(int device, int64_t arena_bytes, gh_ctx** out) {
   // filters.  Mandatory: the launchers index it without asking again.
   ctx->workspace_bytes = 64ll << 20;
   void* fixed = nullptr;
-  if (hipMalloc(&ctx->workspace, (size_t)ctx->workspace_bytes) != hipSuccess ||
+  if (hipMalloc(&ctx->workspace, (size_t)(ctx->workspace_bytes + kBnHeldPage)) != hipSuccess ||
+      hipMemset((char*)ctx->workspace + ctx->workspace_bytes, 0, (size_t)kBnHeldPage) != hipSuccess || hipDeviceSynchronize() != hipSuccess ||
       static_scratch(device, &fixed) != hipSuccess) {
     (void)hipGetLastError();
     drop_ctx(ctx);
     return GH_EOOM;
   }
+  ctx->bn_page = (char*)ctx->workspace + ctx->workspace_bytes;
   *out = ctx;
   return GH_OK;
 }
@@ -396,8 +398,8 @@ static int submit_cmds(gh_ctx* ctx, const gh_cmd* cmds, int n) {
       continue;
     }
     // two commands of which the second reads what the first writes are one launch where a kernel takes both
-    const bool pair = gh_is_pair(cmds + i, n - i);
-    rc = pair ? gh_launch_pair(ctx, cmds + i) : dispatch(ctx, cmds[i]);
+    const bool held = gh_bn_held_pair(ctx, cmds + i, n - i), pair = held || gh_is_pair(cmds + i, n - i);
+    rc = held ? gh_launch_bn_held_pair(ctx, cmds + i) : pair ? gh_launch_pair(ctx, cmds + i) : dispatch(ctx, cmds[i]);
     if (rc) return rc;
     if (pair) i++;
   }

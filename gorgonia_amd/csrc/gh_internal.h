@@ -45,6 +45,9 @@ struct gh_llc_model {
   }
 };
 
+constexpr int kBnHeldSlots = 512;
+constexpr int64_t kBnHeldPage = kBnHeldSlots * (8 + 8 + 4);
+
 struct gh_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -59,6 +62,9 @@ struct gh_ctx {
   // scratch owned by the context (split-K partials, reduction flags)
   void* workspace = nullptr;
   int64_t workspace_bytes = 0;
+  // what the workgroups of k_bn_held.hip pass to each other: two slots of 8 bytes and one count of 4 for each of
+  // kBnHeldSlots, behind the workspace (no plan reaches them), zero whenever no kernel runs
+  void* bn_page = nullptr;
   // set while gh_submit_noalloc runs: the scratch is the library's fixed array and a
   // plan may not shrink to fit it (results must not depend on the scratch size)
   bool ws_strict = false;
@@ -92,6 +98,9 @@ int gh_validate_cmd(const gh_cmd& c, std::string& msg);
 // inputs lost (`cold`) or not, goes past the cache (k_elem.hip)
 bool gh_llc_cold(const gh_ctx* ctx, uint64_t p);
 bool gh_llc_stream(int64_t bytes, bool cold);
+// {BN_TRAIN, MAXPOOL2D} and {MAXPOOL2D_BWD, BN_BWD} in one launch that reads a channel once (k_bn_held.hip)
+bool gh_bn_held_pair(const gh_ctx* ctx, const gh_cmd* cmds, int n);
+int gh_launch_bn_held_pair(gh_ctx* ctx, const gh_cmd* cmds);
 // a run of elementwise commands in one pass (k_chain.hip): how many commands at the front of cmds one pass can take and is
 // quicker for (0 or >= 2; gh_elementwise_run asks the same), and the launch
 int gh_chain_length(const gh_cmd* cmds, int n);
