@@ -4,6 +4,7 @@
 // kernel launch (cuda/arith.go:62) and DoWork/Signal (cuda/external.go:223).
 #include <immintrin.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cstdio>
 #include <cstring>
@@ -84,6 +85,7 @@ static uint32_t* take_word() {
   g_words_used |= 1ull << i;
   uint32_t* const w = (uint32_t*)(g_words_page + 64 * i);
   *w = 0;
+  ((uint64_t*)w)[1] = 0;
   return w;
 }
 static void give_word(uint32_t* w) {
@@ -322,6 +324,95 @@ int gh_memcpy_d2d(gh_ctx* ctx, gh_devptr dst, gh_devptr src, int64_t bytes) {
                       hipMemcpyAsync((void*)(uintptr_t)dst, (const void*)(uintptr_t)src,
                                      (size_t)bytes, hipMemcpyDefault, ctx->stream),
                       "hipMemcpyAsync(D2D)");
+}
+
+// A value on its way from pageable memory: the host copies it into pinned memory and says after each `say` bytes how far it
+// is, and the workgroups of one kernel, launched in front of that, read what is there.  Bound: the bus (56 GB/s) and the
+// first bytes' way.  us with the wait: 392 KB 20 (24 copied, then moved), 2 MB 54 (70 in pieces of 512 KB, whose launches cost
+// some 4 us each until their first bytes came), 4 MB 92 (123), 8 MB 173 (217), 16 MB 320 (385); the bus alone 7, 37, 74, 150
+// and 296.  More workgroups read the host's word and the value against each other: 4 MB 97 with 96 of them, 108 with 192.
+//
+// A workgroup has ranges of kRange bytes and waits for the host's word to pass the end of the next one.  It gives up after
+// kGiveUp of the device's clock: the host, which never waits for the kernel, then took longer than three quarters of that by
+// its own clock (it looks at it before the launch and behind its last word) and enqueues an ordinary copy of everything.
+static constexpr int64_t kRange = 16384, kFollowers = 32;
+static constexpr int64_t kGiveUp = 400000;   // ticks of 10 ns (GORGONIA_HIP_STAGED_TICKS: fewer)
+// A long value is copied in parts that memcpy stores past the host's caches: 16 MB 320 us, 358 in parts of 128 KB (which are
+// quicker up to 12 MB: 253 for 261).
+static int64_t say_after(int64_t bytes) { return bytes > (14 << 20) ? 1 << 20 : 128 << 10; }
+__global__ __launch_bounds__(256) void k_copy_following(uint4* __restrict__ dst, const uint4* src, int64_t n16, int64_t tail_words, const uint64_t* said,
+                                                        uint64_t base, int64_t give_up) {
+  __shared__ uint64_t word;
+  constexpr int kRange16 = kRange / 16;
+  const int64_t t0 = wall_clock64();
+  uint64_t known = base;
+  bool there = true;
+  // waits for `bytes` of the value, in all threads
+  auto wait = [&](int64_t bytes) {
+    if ((int64_t)(known - base) >= bytes) return;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      uint64_t now;
+      while ((int64_t)((now = __hip_atomic_load(said, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_SYSTEM)) - base) < bytes && (int64_t)wall_clock64() - t0 < give_up)
+        __builtin_amdgcn_s_sleep(8);
+      word = now;
+    }
+    __syncthreads();
+    known = word;
+    there = (int64_t)(known - base) >= bytes;
+  };
+  const int64_t ranges = (n16 + kRange16 - 1) / kRange16;
+  for (int64_t r = blockIdx.x; r < ranges; r += gridDim.x) {
+    const int64_t from = r * kRange16, to = from + kRange16 < n16 ? from + kRange16 : n16;
+    wait(to * 16);
+    if (!there) return;
+    int64_t i = from + threadIdx.x;
+    if (to - from == kRange16) {
+      const uint4 a = src[i], b = src[i + 256], c = src[i + 512], d = src[i + 768];
+      dst[i] = a;
+      dst[i + 256] = b;
+      dst[i + 512] = c;
+      dst[i + 768] = d;
+    } else {
+      for (; i < to; i += 256) dst[i] = src[i];
+    }
+  }
+  if (blockIdx.x == 0 && tail_words) {
+    wait(n16 * 16 + tail_words * 4);
+    if (there && (int64_t)threadIdx.x < tail_words) ((uint32_t*)(dst + n16))[threadIdx.x] = ((const uint32_t*)(src + n16))[threadIdx.x];
+  }
+}
+
+int gh_memcpy_staged(gh_ctx* ctx, gh_devptr dst, void* stage, const void* src, int64_t bytes) {
+  if (!ctx || bytes < 0 || (bytes > 0 && (!dst || !stage || !src))) return GH_EINVAL;
+  if (ctx->err) return ctx->err;
+  if (bytes == 0) return GH_OK;
+  const uint64_t from = (uint64_t)(uintptr_t)stage;
+  if (!in_pinned_host(ctx, from) || !in_pinned_host(ctx, from + (uint64_t)bytes - 1)) return gh_fail(ctx, GH_EINVAL, "gh_memcpy_staged: the staging memory is not of gh_host_alloc");
+  if (!ctx->done_word || ctx->capturing || bytes < GH_STAGED_FROM || ((dst | from) & 15) || (bytes & 3)) {
+    memcpy(stage, src, (size_t)bytes);
+    return gh_memcpy_d2d(ctx, dst, from, bytes);
+  }
+  ctx->idle = false;
+  uint64_t* const said = (uint64_t*)ctx->done_word + 1;   // behind the completion word, on its cache line
+  const uint64_t base = *said;
+  const int64_t ranges = (bytes / 16 + kRange / 16 - 1) / (kRange / 16), say = say_after(bytes);
+  int64_t give_up = kGiveUp;
+  if (const char* ticks = getenv("GORGONIA_HIP_STAGED_TICKS")) give_up = std::max<int64_t>(0, std::min<int64_t>(kGiveUp, atoll(ticks)));
+  const auto before = std::chrono::steady_clock::now();
+  hipLaunchKernelGGL(k_copy_following, dim3((unsigned)std::min(ranges, kFollowers)), dim3(256), 0, ctx->stream, (uint4*)(uintptr_t)dst, (const uint4*)stage, bytes / 16,
+                     (bytes % 16) / 4, said, base, give_up);
+  const hipError_t e = hipGetLastError();
+  for (int64_t at = 0; at < bytes; at += say) {
+    const int64_t len = std::min(say, bytes - at);
+    memcpy((char*)stage + at, (const char*)src + at, (size_t)len);
+    _mm_sfence();   // memcpy may have stored past the cache
+    __atomic_store_n(said, base + (uint64_t)(at + len), __ATOMIC_RELEASE);
+  }
+  if (e != hipSuccess) return gh_check_hip(ctx, e, "copy launch");
+  const auto took = std::chrono::steady_clock::now() - before;
+  if (took >= std::chrono::nanoseconds(give_up * 10 * 3 / 4)) return gh_memcpy_d2d(ctx, dst, from, bytes);
+  return GH_OK;
 }
 
 static int dispatch(gh_ctx* ctx, const gh_cmd& c) {

@@ -181,10 +181,10 @@ void Engine::HostFree(void* p) {
   if (ctx_ && p) gh_host_free(ctx_, p);
 }
 
-Status Engine::CopyNow(uint64_t dst, uint64_t src, int64_t bytes) {
+Status Engine::StagedCopy(uint64_t dst, void* stage, const void* src, int64_t bytes) {
   if (!ctx_) return Status::Err(GH_ESTATE, "engine not initialised");
-  const int rc = gh_memcpy_d2d(ctx_, dst, src, bytes);
-  return rc == GH_OK ? Status::OK() : fail(rc, "CopyNow");
+  const int rc = gh_memcpy_staged(ctx_, dst, stage, src, bytes);
+  return rc == GH_OK ? Status::OK() : fail(rc, "StagedCopy");
 }
 
 void Engine::RecordCopy(uint64_t dst, uint64_t src, int64_t bytes) {

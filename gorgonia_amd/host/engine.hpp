@@ -121,7 +121,8 @@ class Engine {
   Status HostAlloc(int64_t bytes, void** out);
   void HostFree(void* p);
   void RecordCopy(uint64_t dst, uint64_t src, int64_t bytes);
-  Status CopyNow(uint64_t dst, uint64_t src, int64_t bytes);   // queued at once, in front of the segment being recorded
+  // host memory to the device by way of a pinned buffer, queued at once, in front of the segment being recorded
+  Status StagedCopy(uint64_t dst, void* stage, const void* src, int64_t bytes);
 
   // ---- arithmetic and comparison (cuda/arith.go, cuda/cmp.go) -----------------------
   // fn is a gh_binfn.  Tensor-tensor form: Add/Sub/Mul/Div/Pow/Lt/Lte/Gt/Gte/ElEq/ElNe.

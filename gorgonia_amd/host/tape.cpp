@@ -16,11 +16,8 @@ static constexpr int64_t kStageLimit = 8 << 20;
 // inputs re-uploaded on every run are staged through pinned memory up to these sizes
 static constexpr int64_t kStageInLimit = 16 << 20;    // per input (what one copy kernel moves)
 static constexpr int64_t kStageInTotal = 512ll << 20; // per machine
-// inputs from this size on are uploaded in pieces, the host copy into pinned memory overlapping the bus.  A piece
-// costs a launch (some 5 us in front of the bus), so the pieces of a long upload are larger: host copy and upload
-// together take 72 us of 2 MB (109 in one piece), 124 of 4 MB (185), 392 of 16 MB (590).
-static constexpr int64_t kPipelinedUpload = 768 << 10;
-static constexpr int64_t kUploadPiece = 512 << 10, kUploadPieceLong = 2 << 20, kLongUpload = 8 << 20;
+// inputs from this size on are uploaded while the host copies them into pinned memory
+static constexpr int64_t kFollowedUpload = 256 << 10;
 // inputs up to this size may be read where the host wrote them, in pinned memory (reads_in_place)
 static constexpr int64_t kReadInPlace = 8 << 10;
 static constexpr int64_t kWalkInPlace = 2 << 10;
@@ -1036,7 +1033,7 @@ Status TapeMachine::Compile() {
   regs_.assign((size_t)nreg, Tensor());
   reg_live_.assign((size_t)nreg, 0);
   reg_arena_.assign((size_t)nreg, 0);
-  in_pieces_.assign((size_t)N, 0);
+  followed_.assign((size_t)N, 0);
   lent_.assign((size_t)N, 0);
   recorded_.clear();
   steady_ = false;
@@ -1271,23 +1268,10 @@ Status TapeMachine::upload(const Instr& in, bool record) {
     // the segment: the upload is captured and replayed with the operators
     if (record) {
       lent_[(size_t)in.node] = n.host_borrowed;
-      in_pieces_[(size_t)in.node] = !n.host_borrowed && in.size >= kPipelinedUpload && eng_.Segment().empty();
+      followed_[(size_t)in.node] = !n.host_borrowed && in.size >= kFollowedUpload && eng_.Segment().empty();
     }
-    if (in_pieces_[(size_t)in.node] && !n.host_borrowed) {
-      // a large value at the front of its segment: piece by piece, the host copy of one
-      // piece runs while the bus moves the piece before it (stream order puts the
-      // segment's operators behind the last piece)
-      const int64_t piece = in.size >= kLongUpload ? kUploadPieceLong : kUploadPiece;
-      const char* src = static_cast<const char*>(n.host);
-      char* stg = static_cast<char*>(pinned);
-      for (int64_t off = 0; off < in.size; off += piece) {
-        const int64_t len = std::min(piece, in.size - off);
-        std::memcpy(stg + off, src + off, (size_t)len);
-        Status st = eng_.CopyNow(mem + (uint64_t)off, (uint64_t)(uintptr_t)(stg + off), len);
-        if (!st.ok()) return st;
-      }
-      return Status::OK();
-    }
+    // a large value at the front of its segment (stream order puts the segment's operators behind it)
+    if (followed_[(size_t)in.node] && !n.host_borrowed) return eng_.StagedCopy(mem, pinned, n.host, in.size);
     if (!n.host_borrowed) std::memcpy(pinned, n.host, (size_t)in.size);
     if (!record) return Status::OK();
     const uint64_t arena = reg_memory((size_t)in.reg);
@@ -1458,7 +1442,7 @@ Status TapeMachine::RunAll() {
         }
         break;
       case InstrKind::Flush:
-        // nothing was submitted in front of it (but pieces of an upload): the run is this one segment
+        // nothing was submitted in front of it (but an upload): the run is this one segment
         if (eng_.SubmitCalls() == calls && !watched && !opt_.node_at_a_time) {
           const std::vector<gh_cmd>& cur = eng_.Segment();
           settled = cur.size() == recorded_.size() &&

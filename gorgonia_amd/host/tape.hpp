@@ -261,7 +261,7 @@ class TapeMachine {
   // What the last run recorded, and whether the runs have settled: two runs in a row recorded the same commands
   // and nobody has touched the arena since, so the next run would record them again (run_steady).
   std::vector<gh_cmd> recorded_;
-  std::vector<char> in_pieces_;    // per node: the last run uploaded it piece by piece in front of the segment
+  std::vector<char> followed_;    // per node: the last run uploaded it in front of the segment, behind the host's copy
   std::vector<char> lent_;         // per node: it was a lent input then
   std::vector<char> in_place_;     // per node: a small input that its readers read in pinned memory (if it is not lent)
   bool steady_ = false;

@@ -279,6 +279,11 @@ GH_API int gh_host_free(gh_ctx* ctx, void* p);
 GH_API int gh_memcpy_h2d(gh_ctx* ctx, gh_devptr dst, const void* src, int64_t bytes);
 GH_API int gh_memcpy_d2h(gh_ctx* ctx, void* dst, gh_devptr src, int64_t bytes);
 GH_API int gh_memcpy_d2d(gh_ctx* ctx, gh_devptr dst, gh_devptr src, int64_t bytes);
+/* src (any host memory) to dst by way of `stage` (memory of gh_host_alloc, `bytes` of it): the bus moves what has been
+ * copied while the host copies the rest.  Returns when src has been read; `stage` must stay untouched until the next
+ * gh_sync(). */
+#define GH_STAGED_FROM (128 << 10) /* below, one copy after the other */
+GH_API int gh_memcpy_staged(gh_ctx* ctx, gh_devptr dst, void* stage, const void* src, int64_t bytes);
 
 /* ---- work submission --------------------------------------------------- */
 
