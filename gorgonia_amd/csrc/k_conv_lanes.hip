@@ -169,6 +169,18 @@ __global__ __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(WV == 8
 #pragma unroll
         for (int n = 0; n < TN; n++) acc[m][n] = U::run(f.a[m][kFlip ? 8 - t : t], f.b[n / V][t / 3][n % V + t % 3], acc[m][n]);
   };
+  // The filters' BatchNorm constants go into a table, loaded here and worked out behind the channels: 1 / sqrt for each result
+  // was up to half of a pooled layer's time (8 x 16 x 112 x 112 -> 32 with all of its channels in a wavefront 24.3 us, with
+  // the table filled here 15.3, behind the channels 14.6).
+  const int tf = f0 + (int)threadIdx.x;
+  const bool fills = sizeof(T) == 4 && !kFlip && tail.mean && (int)threadIdx.x < 16 * TM && tf < g.F;
+  float bn_mean = 0.0f, bn_var = 1.0f, bn_gamma = 1.0f, bn_beta = -0.0f;   // (as conv_tail_table has absent ones)
+  if (fills) {
+    bn_mean = tail.mean[tf];
+    bn_var = tail.var[tf];
+    if (tail.gamma) bn_gamma = tail.gamma[tf];
+    if (tail.beta) bn_beta = tail.beta[tf];
+  }
   const int quads = g.C >> 2;
   constexpr int step = kSplit ? WV : 1;
   const int first = kSplit ? wave : 0;
@@ -183,24 +195,71 @@ __global__ __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(WV == 8
     }
   }
 
-  // The sums go through LDS, 16 filter rows at a time, in the order of the results: wavefront order where they split
-  // the channels, else each wavefront its own.
-  __shared__ __attribute__((aligned(16))) T red[WV][TN * 256];
-  const int tid = kSplit ? (int)threadIdx.x : lane;
-  constexpr int nthreads = kSplit ? WV * 64 : 64;
-  auto value = [&](int e) {
-    if constexpr (kSplit) {
-      T sum = red[0][e];
+  __shared__ float tab[sizeof(T) == 4 ? 4 * 16 * TM : 1];
+  if (fills) {
+    const float a = 1.0f / sqrtf(bn_var + tail.eps);
+    const int i = threadIdx.x;
+    tab[i] = a;
+    tab[16 * TM + i] = -bn_mean * a;
+    tab[2 * 16 * TM + i] = bn_gamma;
+    tab[3 * 16 * TM + i] = bn_beta;
+  }
+  __shared__ __attribute__((aligned(16))) T red[kSplit ? WV : 1][kSplit ? TN * 256 : 1];
+  auto store = [&](auto epilogue) __attribute__((always_inline)) {
+  if constexpr (!kSplit) {
+    // A lane holds V neighbours of its group for four filters of each tile and stores them as they are.
+    typedef T Row __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+    typedef T Half __attribute__((ext_vector_type(V / 2), aligned(sizeof(T))));
 #pragma unroll
-      for (int v = 1; v < WV; v++) sum = sum + red[v][e];
-      return sum;
-    } else {
-      return red[wave][e];
+    for (int n = 0; n < G; n++) {
+      const int grp = g0 + 16 * n + i;
+      if (grp >= g.groups) continue;   // (the groups of a pair are both inside or both outside)
+      int b, oy, ox;
+      place(grp, &b, &oy, &ox);
+#pragma unroll
+      for (int m = 0; m < TM; m++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const int f = f0 + 16 * m + U::row(q, v);
+          T own[V];
+#pragma unroll
+          for (int e = 0; e < V; e++) own[e] = epilogue(16 * m + U::row(q, v), acc[m][n * V + e][v]);
+          if constexpr (kPool) {
+            T best[V / 2];
+            T below[V];
+#pragma unroll
+            for (int e = 0; e < V; e++) below[e] = __shfl_xor(own[e], 1, 64);
+#pragma unroll
+            for (int k = 0; k < V / 2; k++) {
+              best[k] = (T)-3.402823466e+38f;   // scan order and strict > of the pooling kernel
+              if (own[2 * k] > best[k]) best[k] = own[2 * k];
+              if (own[2 * k + 1] > best[k]) best[k] = own[2 * k + 1];
+              if (below[2 * k] > best[k]) best[k] = below[2 * k];
+              if (below[2 * k + 1] > best[k]) best[k] = below[2 * k + 1];
+            }
+            if (f < g.F && !(i & 1)) {
+              Half h;
+#pragma unroll
+              for (int k = 0; k < V / 2; k++) h[k] = best[k];
+              *(Half*)(g.y + (((int64_t)b * g.F + f) * (g.rows >> 1) + (oy >> 1)) * (g.cols >> 1) + (ox >> 1)) = h;
+            }
+          } else if (f < g.F) {
+            Row r;
+#pragma unroll
+            for (int e = 0; e < V; e++) r[e] = own[e];
+            *(Row*)(g.y + (((int64_t)b * g.F + f) * g.oh + oy) * g.ow + ox) = r;
+          }
+        }
     }
-  };
-  auto epilogue = [&](int f, T v) -> T {
-    if constexpr (sizeof(T) == 4) return tail_apply(tail, f, v);
-    else return v;
+  } else {
+  // The sums go through LDS, 16 filter rows at a time, and are added in wavefront order.
+  const int tid = (int)threadIdx.x;
+  constexpr int nthreads = WV * 64;
+  auto value = [&](int e) {
+    T sum = red[0][e];
+#pragma unroll
+    for (int v = 1; v < WV; v++) sum = sum + red[v][e];
+    return sum;
   };
 #pragma unroll
   for (int m = 0; m < TM; m++) {
@@ -221,7 +280,7 @@ __global__ __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(WV == 8
         T best = (T)-3.402823466e+38f;   // scan order and strict > of the pooling kernel
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-          const T v = epilogue(f, value(at + (u >> 1) * V + (u & 1)));
+          const T v = epilogue(16 * m + r, value(at + (u >> 1) * V + (u & 1)));
           if (v > best) best = v;
         }
         int b, oy, ox;
@@ -234,9 +293,17 @@ __global__ __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(WV == 8
         if (f >= g.F || grp >= g.groups) continue;
         int b, oy, ox;
         place(grp, &b, &oy, &ox);
-        g.y[(((int64_t)b * g.F + f) * g.oh + oy) * g.ow + ox + col % V] = epilogue(f, value(e));
+        g.y[(((int64_t)b * g.F + f) * g.oh + oy) * g.ow + ox + col % V] = epilogue(16 * m + r, value(e));
       }
     }
+  }
+  }
+  };
+  if constexpr (sizeof(T) == 8 || kFlip) {
+    store([](int, T v) { return v; });
+  } else {
+    if (!kSplit) __syncthreads();   // the table
+    conv_tail_dispatch(tail, [&](auto BN, auto ACT) { store([&](int r, float v) { return tail_apply_fixed<BN(), ACT()>(tab, 16 * TM, r, v, tail.alpha); }); });
   }
 }
 
@@ -294,49 +361,61 @@ bool fill(const gh_cmd& c, bool flip, bool pool, Lanes<T>* g) {
 // channels.  Fitted to 50 shapes of 1 to 256 images of 7 x 7 to 104 x 104, 16 to 512 channels, forward and gradient;
 // the estimates are mostly within 15 % of the times.
 struct Form { int tm, v, waves, groups; bool split; double per_tile, per_quad; };
-static const Form kForms32[] = {{1, 4, 8, 1, true, 1.9, 0.160}, {2, 4, 8, 1, true, 3.2, 0.263}, {2, 4, 4, 1, true, 2.4, 0.24}};
+static const Form kForms32[] = {{1, 4, 8, 1, true, 1.9, 0.160}, {2, 4, 8, 1, true, 3.2, 0.263}, {2, 4, 4, 1, true, 2.4, 0.24}, {2, 4, 4, 1, false, 2.6, 1.05}, {1, 4, 4, 1, false, 1.8, 0.52}};
 static const Form kForms64[] = {{1, 2, 4, 1, true, 0.8, 0.17}, {2, 2, 4, 2, true, 3.4, 0.47}, {2, 2, 4, 2, false, 4.0, 2.2}};
 
-// The quickest form and its time: a function of the plain command (a pooled one takes the same form and so sums in the
-// same order).
-static int quickest(const gh_cmd& c, bool flip, bool f64, int cus, double* us) {
+// The quickest of the forms from..to - 1 and its time: a function of the plain command (a pooled one takes the same form
+// and so sums in the same order).
+static int quickest(const gh_cmd& c, bool flip, bool f64, int cus, int from, int to, double* us) {
   const int64_t B = c.dim[0], oh = c.dim[2] + 2 * c.dim[7] - 2, ow = c.dim[3];
   const int64_t K = flip ? c.dim[4] : c.dim[1], F = flip ? c.dim[1] : c.dim[4], lines = B * (flip ? c.dim[2] : oh);
   int best = -1;
-  for (int i = 0; i < 3; i++) {
+  for (int i = from; i < to; i++) {
     const Form& f = (f64 ? kForms64 : kForms32)[i];
     // an image gradient gains nothing from the form that halves the wavefronts (8 x 32 x 52 x 52 <- 64: 14.5 us, 14.0 with
     // eight), and would add twice as many terms in a row
-    if (!f64 && flip && f.waves == 4) continue;
+    if (!f64 && flip && f.split && f.waves == 4) continue;
     const int64_t per = 16 * f.groups * (f.split ? 1 : f.waves);
     const int64_t tiles = (F + 16 * f.tm - 1) / (16 * f.tm) * ((lines * ((ow + f.v - 1) / f.v) + per - 1) / per);
     // one tile of four wavefronts to a compute unit waits for its loads
-    const double per_quad = !f64 && f.waves == 4 && tiles <= cus ? 0.33 : f.per_quad;
+    const bool lone = !f64 && f.waves == 4 && tiles <= cus;
+    const double per_quad = !lone ? f.per_quad : f.split ? 0.33 : 1.27 * f.per_quad;
     const double est = 3.2 + (double)((tiles + cus - 1) / cus) * (f.per_tile + per_quad * (double)(K / 4));
     if (best < 0 || est < *us) { best = i; *us = est; }
   }
   return best;
 }
 
-// Whether this kernel takes a convolution (flip: an image gradient) that `other_us` is what the others would take for;
-// 0 asks only whether it can.  It has to be a sixth quicker by the estimates, which are that good.
-bool gh_conv_lanes_takes(const gh_cmd& c, bool flip, int cus, double other_us) {
-  if (getenv("GORGONIA_HIP_CONV_NO_LANES")) return false;   // tuning switch: the other kernels only
+// Which form takes a convolution (flip: an image gradient) that `other_us` is what the other kernels would take for, -1
+// where they keep it; other_us 0: any shape that a form can take.  It has to be a sixth quicker by the estimates, which
+// are that good.
+//
+// float32 where that is not so: a wavefront with a tile of its own and all channels, for few channels and many pixels, where
+// the split forms have one or two quads to a wavefront and the wide-image kernel stages as much as it multiplies.  Not in
+// place of a split form or of the patch kernel, which split the channels: its sums are longer (the gradient of 4 x 128 x 60 x
+// 60 -> 64 would be off by 4.3e-7 of its norm instead of 1.6e-7).  us, before / now: 8 x 16 x 104 x 104 -> 32 22.9 / 15.9, pooled 17.9 / 13.6, its gradient 24.2 / 13.6; 8 x 16 x 104 x 104 -> 16
+// 15.8 / 10.0 and its gradient 17.8 / 8.7; 8 x 32 x 104 x 104 -> 64 46.7 / 39.7 (80 TFLOP/s); 8 x 16 x 208 x 208 -> 32's
+// gradient 45.8 / 36.1; 1 x 16 x 208 x 208 -> 32 pooled 11.0 / 8.7.
+int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, bool patch) {
+  if (getenv("GORGONIA_HIP_CONV_NO_LANES")) return -1;   // tuning switch: the other kernels only
   const bool f64 = gh_dtype_of(c.flags) == GH_F64;
   Lanes<double> g;   // (the narrower of the two in what its offsets reach)
-  if (!fill(c, flip, false, &g) || g.F < 8 || g.C < 8 || g.oh < 2) return false;
+  if (!fill(c, flip, false, &g) || g.F < 8 || g.C < 8 || g.oh < 2) return -1;
   double us;
-  return quickest(c, flip, f64, cus, &us) >= 0 && (other_us <= 0 || us < other_us / 1.17);
+  const int split = quickest(c, flip, f64, cus, 0, 3, &us);
+  if (other_us <= 0 || us < other_us / 1.17) return split;
+  if (f64 || patch) return -1;
+  const int whole = quickest(c, flip, false, cus, 3, 5, &us);
+  return us < other_us / 1.1 ? whole : -1;
 }
 
-int gh_launch_conv_lanes(gh_ctx* ctx, const gh_cmd& c, bool flip) {
+int gh_launch_conv_lanes(gh_ctx* ctx, const gh_cmd& c, bool flip, int form) {
   const bool pool = !flip && (c.flags & GH_FLAG_CONV_POOL2);
-  double us;
   if (gh_dtype_of(c.flags) == GH_F64) {
     Lanes<double> g;
     if (!fill(c, flip, false, &g)) return gh_fail(ctx, GH_ESTATE, "conv3x3: not a shape of this kernel");
     const ConvTail t{};
-    switch (quickest(c, flip, true, ctx->cu_count, &us)) {
+    switch (form) {
       case 0: return launch<double, 4, 1, 2, 1, true>(ctx, g, t, flip, false);
       case 1: return launch<double, 4, 2, 2, 2, true>(ctx, g, t, flip, false);
       default: return launch<double, 4, 2, 2, 2, false>(ctx, g, t, flip, false);
@@ -345,9 +424,11 @@ int gh_launch_conv_lanes(gh_ctx* ctx, const gh_cmd& c, bool flip) {
   Lanes<float> g;
   if (!fill(c, flip, pool, &g)) return gh_fail(ctx, GH_ESTATE, "conv3x3: not a shape of this kernel");
   const ConvTail t = flip ? ConvTail{} : conv_tail(c);
-  switch (quickest(c, flip, false, ctx->cu_count, &us)) {
+  switch (form) {
     case 0: return launch<float, 8, 1, 4, 1, true>(ctx, g, t, flip, pool);
     case 1: return launch<float, 8, 2, 4, 1, true>(ctx, g, t, flip, pool);
+    case 3: return launch<float, 4, 2, 4, 1, false>(ctx, g, t, flip, pool);
+    case 4: return launch<float, 4, 1, 4, 1, false>(ctx, g, t, flip, pool);
     default: return launch<float, 4, 2, 4, 1, true>(ctx, g, t, flip, pool);
   }
 }

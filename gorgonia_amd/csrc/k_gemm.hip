@@ -2967,8 +2967,8 @@ bool gh_try_launch_conv2d_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
   ConvGeom64 g;
   if (!conv64_mfma_takes(c, &g)) return false;
   const int64_t P = g.P;
-  if (gh_conv_lanes_takes(c, false, ctx->cu_count, 0)) {
-    gh_launch_conv_lanes(ctx, c, false);   // an error is sticky on the context; the caller returns it
+  if (const int form = gh_conv_lanes_form(c, false, ctx->cu_count, 0); form >= 0) {
+    gh_launch_conv_lanes(ctx, c, false, form);   // an error is sticky on the context; the caller returns it
     return true;
   }
   const int64_t tiles128 = (int64_t)((g.F + 127) / 128) * ((P + 127) / 128);
@@ -3016,8 +3016,8 @@ bool gh_try_launch_conv2d_bwd_data_f64_mfma(gh_ctx* ctx, const gh_cmd& c) {
   const int64_t wcount = (int64_t)F * C * kh * kw, wbytes = (wcount * 8 + 255) / 256 * 256;
   // (what a fixed scratch refuses does not depend on the kernel)
   if (wbytes > ctx->workspace_bytes && gh_ws_short(ctx, wbytes) != GH_OK) return true;   // the caller returns ctx->err
-  if (gh_conv_lanes_takes(c, true, ctx->cu_count, 0)) {
-    gh_launch_conv_lanes(ctx, c, true);
+  if (const int form = gh_conv_lanes_form(c, true, ctx->cu_count, 0); form >= 0) {
+    gh_launch_conv_lanes(ctx, c, true, form);
     return true;
   }
   if (wbytes > ctx->workspace_bytes) return false;
@@ -3295,30 +3295,34 @@ static bool conv_direct_takes(const gh_cmd& c) {
 // its own; the wide-image kernel's is fitted from above its quickest (8 x 16 x 208 x 208 -> 32 takes 40, 8 x 16 x 104 x
 // 104 -> 32 23, 2 x 16 x 104 x 104 -> 32 11), the tiled one's to 23 for 8 x 32 x 52 x 52 -> 64, 17 for two such images,
 // 13 for 3 x 16 x 49 x 49 -> 32.
-static double conv_others_us(const gh_cmd& c, int cus) {
-  if (gh_conv_patch_takes(c)) return gh_conv_patch_us(c, cus);
+static double conv_others_us(const gh_cmd& c, int cus, bool* patch) {
+  const double us = gh_conv_patch_us(c, cus);   // 0 where it does not take the shape
+  if ((*patch = us > 0)) return us;
   const double oh = (double)(c.dim[2] + 2 * c.dim[7] - 2), ow = (double)(c.dim[3] + 2 * c.dim[8] - 2);
   const double flops = 18.0 * (double)c.dim[0] * (double)c.dim[1] * (double)c.dim[4] * oh * ow;
   return gh_conv_wide_takes(c) ? 10.0 + flops * 1e-8 : 12.0 + flops / 75e6;
 }
 // float32, behind the single-channel, few-channel and small-image kernels, which win where they take a shape.
-static bool conv_lanes_takes(const gh_cmd& c, int cus) {
-  if (c.dim[5] != 3 || c.dim[6] != 3 || gh_conv_rows1_takes(c) || conv_direct_takes(c) || gh_conv_small_takes(c)) return false;
-  return gh_conv_lanes_takes(c, false, cus, conv_others_us(c, cus));
+static int conv_lanes_form(const gh_cmd& c, int cus) {
+  if (c.dim[5] != 3 || c.dim[6] != 3 || gh_conv_rows1_takes(c) || conv_direct_takes(c) || gh_conv_small_takes(c)) return -1;
+  bool patch;
+  const double others = conv_others_us(c, cus, &patch);
+  return gh_conv_lanes_form(c, false, cus, others, patch);
 }
 // The image gradient: elsewhere that is a launch that mirrors the filters (4.7 us) and a forward one over dy.
-static bool conv_lanes_takes_gradient(const gh_cmd& c, int cus) {
-  if (c.dim[5] != 3 || c.dim[6] != 3 || c.dim[11] != 1 || c.dim[12] != 1) return false;
+static int conv_lanes_gradient_form(const gh_cmd& c, int cus) {
+  if (c.dim[5] != 3 || c.dim[6] != 3 || c.dim[11] != 1 || c.dim[12] != 1) return -1;
   gh_cmd f{};
   f.opcode = GH_OP_CONV2D;
   f.dim[0] = c.dim[0]; f.dim[1] = c.dim[4]; f.dim[2] = gh_conv_out(c.dim[2], 3, c.dim[7], 1, 1); f.dim[3] = gh_conv_out(c.dim[3], 3, c.dim[8], 1, 1);
   f.dim[4] = c.dim[1]; f.dim[5] = f.dim[6] = 3; f.dim[7] = 2 - c.dim[7]; f.dim[8] = 2 - c.dim[8];
   f.dim[9] = f.dim[10] = f.dim[11] = f.dim[12] = 1;
-  if (gh_conv_rows1_takes(f) || conv_direct_takes(f)) return false;
+  if (gh_conv_rows1_takes(f) || conv_direct_takes(f)) return -1;
   // the small-image kernels run at 55 TFLOP/s past 6 us (128 x 32 x 14 x 14 -> 64: 12.8 us and the mirroring)
+  bool patch = false;
   const double others = gh_conv_small_takes(f) ? 6.0 + 18.0 * (double)f.dim[0] * (double)f.dim[1] * (double)f.dim[4] * (double)f.dim[2] * (double)f.dim[3] / 55e6
-                                               : conv_others_us(f, cus);
-  return gh_conv_lanes_takes(c, true, cus, others + 4.7);
+                                               : conv_others_us(f, cus, &patch);
+  return gh_conv_lanes_form(c, true, cus, others + 4.7, patch);
 }
 
 static int launch_conv_direct(gh_ctx* ctx, const gh_cmd& c) {
@@ -3378,7 +3382,7 @@ int gh_launch_conv2d(gh_ctx* ctx, const gh_cmd& c) {
   if (conv_direct_takes(c)) return launch_conv_direct(ctx, c);
   const int rcs = gh_try_launch_conv_small(ctx, c);
   if (rcs >= 0) return rcs;
-  if (conv_lanes_takes(c, ctx->cu_count)) return gh_launch_conv_lanes(ctx, c, false);
+  if (const int form = conv_lanes_form(c, ctx->cu_count); form >= 0) return gh_launch_conv_lanes(ctx, c, false, form);
   const int rcp = gh_try_launch_conv_patch(ctx, c);
   if (rcp >= 0) return rcp;
   const int rcw = gh_try_launch_conv_wide(ctx, c);
@@ -3556,7 +3560,7 @@ int gh_launch_conv2d_bwd_data(gh_ctx* ctx, const gh_cmd& c) {
   const bool mirror_shape = g.strideH == 1 && g.strideW == 1 && padH >= 0 && padW >= 0;
   if (mirror_shape && wbytes > ctx->workspace_bytes / 2)
     if (int rc = gh_ws_short(ctx, 2 * wbytes)) return rc;   // (what a fixed scratch refuses does not depend on the kernel)
-  if (mirror_shape && conv_lanes_takes_gradient(c, ctx->cu_count)) return gh_launch_conv_lanes(ctx, c, true);
+  if (const int form = mirror_shape ? conv_lanes_gradient_form(c, ctx->cu_count) : -1; form >= 0) return gh_launch_conv_lanes(ctx, c, true, form);
   if (mirror_shape && wbytes <= ctx->workspace_bytes / 2) {
     // mirrored filters live at the top of the workspace; the forward launch
     // below may use what is left of it for its own split-K slabs
@@ -3697,14 +3701,14 @@ extern "C" int gh_runs_straight(const gh_cmd* c) {
       return f64 ? gemm64_form(*c, cus) >= 0 && gemm64_form(*c, cus) != kStaged64 : !gemm_skinny_takes(*c, cus) && direct_form(*c, cus) >= 0;
     case GH_OP_CONV2D: {
       ConvGeom64 g;
-      if (f64) return conv64_mfma_takes(*c, &g) && gh_conv_lanes_takes(*c, false, cus, 0);
-      return !(c->flags & GH_FLAG_CONV_PRE) && conv_lanes_takes(*c, cus);
+      if (f64) return conv64_mfma_takes(*c, &g) && gh_conv_lanes_form(*c, false, cus, 0) >= 0;
+      return !(c->flags & GH_FLAG_CONV_PRE) && conv_lanes_form(*c, cus) >= 0;
     }
     case GH_OP_CONV2D_BWD_DATA: {
       gh_cmd f;
-      if (f64) return conv64_mirror(*c, &f) && gh_conv_lanes_takes(*c, true, cus, 0);
+      if (f64) return conv64_mirror(*c, &f) && gh_conv_lanes_form(*c, true, cus, 0) >= 0;
       const ConvGeom g = conv_geom(*c);
-      return g.strideH == 1 && g.strideW == 1 && g.dilH * (g.kh - 1) >= g.padH && g.dilW * (g.kw - 1) >= g.padW && conv_lanes_takes_gradient(*c, cus);
+      return g.strideH == 1 && g.strideW == 1 && g.dilH * (g.kh - 1) >= g.padH && g.dilW * (g.kw - 1) >= g.padW && conv_lanes_gradient_form(*c, cus) >= 0;
     }
     case GH_OP_CONV2D_BWD_FILTER: return f64 ? gh_conv_wgrad_takes(*c, cus) : wgrad_mfma_takes(*c, cus);
   }
