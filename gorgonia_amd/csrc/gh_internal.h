@@ -45,7 +45,7 @@ struct gh_llc_model {
   }
 };
 
-constexpr int kBnHeldSlots = 512;
+constexpr int kBnHeldSlots = 2048;
 constexpr int64_t kBnHeldPage = kBnHeldSlots * (8 + 8 + 4);
 
 struct gh_ctx {
@@ -99,6 +99,7 @@ int gh_validate_cmd(const gh_cmd& c, std::string& msg);
 bool gh_llc_cold(const gh_ctx* ctx, uint64_t p);
 bool gh_llc_stream(int64_t bytes, bool cold);
 // {BN_TRAIN, MAXPOOL2D} and {MAXPOOL2D_BWD, BN_BWD} in one launch that reads a channel once (k_bn_held.hip)
+int gh_bn_groups(int64_t n, int64_t S);   // the groups of 256 threads that k_bn_reduce cuts a channel of n values in planes of S into (k_bwd.hip)
 bool gh_bn_held_pair(const gh_ctx* ctx, const gh_cmd* cmds, int n);
 int gh_launch_bn_held_pair(gh_ctx* ctx, const gh_cmd* cmds);
 // a run of elementwise commands in one pass (k_chain.hip): how many commands at the front of cmds one pass can take and is

@@ -1,18 +1,19 @@
-// Batch statistics and the 2x2 pooling behind them, a channel held in registers.
+// Batch statistics and the 2x2 pooling behind them in one launch, and their gradients in another.
 //
-// Training mode needs a channel's mean before its deviations and both before a value can be written: three passes over the
-// tensor, then the pooling's.  The gradient needs two sums before it can be written.  A convolution's result of 22 MB fits
-// the chip's registers (128 MB), so that here a channel's values are read once: C channels times G workgroups of up to 1024
-// threads, one workgroup on a compute unit, each with its share of a channel in registers.  The workgroups of a channel
-// pass their sums to each other through memory and wait for each other's.
+// Training mode needs a channel's mean before its deviations and both before a value can be written, and a launch for each
+// of these and for the pooling; the gradient needs two sums before it can be written.  Here C channels times G workgroups of
+// up to 1024 threads, one workgroup on a compute unit, have a share of a channel each.  They pass their sums to each other
+// through memory and wait for each other's.  A 22 MB tensor fits the chip's registers (128 MB): between its sums and the
+// values it writes the gradient keeps what it has read, the forward its values between its two passes.
 //
 // A wait ends whether or not the others come: a workgroup that has asked kPolls times reads the missing shares and adds
 // them up itself, in the same order, to the same bits.  Nothing depends on all workgroups being on the chip at once.
 //
 // Bound: HBM and the caches for large planes, the launch and the waits (some 1.5 us each) for small ones.  us, four launches
-// or three / one, forward and gradient: 8 x 16 x 208 x 208 (22 MB) 30.9 / 14.8 and 33.8 / 20.7 (5.3 TB/s of the 110 MB that
-// the gradient moves), 8 x 32 x 104 x 104 20.6 / 9.9 and 23.0 / 12.0, 8 x 128 x 26 x 26 14.2 / 7.3 and 13.5 / 6.7,
-// 8 x 16 x 207 x 207 (single loads) 46.8 / 18.9 and 46.8 / 25.2, 2 x 3 x 4 x 4 11.7 / 5.4 and 9.3 / 4.3.
+// or three / one, forward and gradient: 8 x 16 x 208 x 208 30.9 / 18.7 and 33.8 / 21.1 (5.2 TB/s of the 110 MB that the
+// gradient moves), 8 x 32 x 104 x 104 20.5 / 11.8 and 22.9 / 12.3, 8 x 128 x 26 x 26 14.2 / 8.9 and 13.4 / 7.0,
+// 8 x 16 x 207 x 207 (single loads) 46.6 / 20.8 and 47.3 / 25.8, 2 x 3 x 4 x 4 12.1 / 7.5 and 10.0 / 4.9.  (The forward as the
+// gradient is, its values kept as the pooling's windows lie: 14.8, 9.9 and 7.3, and other sums.)
 #include <algorithm>
 #include <cfloat>
 
@@ -21,6 +22,7 @@
 namespace {
 
 constexpr int kThreads = 1024;
+constexpr int kHeld = 6;   // groups of four values that a thread of the forward keeps
 constexpr int kPolls = 2000;   // about a millisecond (GORGONIA_HIP_BN_POLLS: another number)
 typedef unsigned long long u64;
 
@@ -161,9 +163,9 @@ __device__ __forceinline__ void total(u64* const (&slots)[2], int kinds, int G, 
 
 // The channel's slots are zero again when its last workgroup is through.  (No order with the tensors' values is needed, and a
 // release here would write the cache back: 16 us instead of 10 for 8 x 128 x 26 x 26.)
-__device__ __forceinline__ void leave(u64* const (&slots)[2], unsigned* count, int G) {
-  if (threadIdx.x == 0 && __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)G - 1) {
-    for (int g = 0; g < G; g++) {
+__device__ __forceinline__ void leave(u64* const (&slots)[2], unsigned* count, int shares, int workgroups) {
+  if (threadIdx.x == 0 && __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)workgroups - 1) {
+    for (int g = 0; g < shares; g++) {
       __hip_atomic_store(slots[0] + g, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(slots[1] + g, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -176,60 +178,105 @@ struct BnOut {
   float eps, momentum;
 };
 
-// N: units of a thread.
-template <int COLS, bool EDGES, int N>
-__global__ __launch_bounds__(kThreads) void k_bn_train_pool(const float* __restrict__ x, float* __restrict__ y, float* __restrict__ pooled, Planes g, int64_t n, BnOut o,
-                                                            u64* page) {
+// How k_bn_reduce cuts a channel: `groups` groups of 256 threads, thread t of group k with the values k * 256 + t, then every
+// groups * 256-th of a plane, of all images - or, in planes of fewer values than a group has threads, whole planes.  A
+// workgroup here does the work of `own` of them.
+struct Cut {
+  int S, groups, own;
+};
+
+// The forward sums are k_bn_reduce's to the bit: where one order of additions sends a value to one side of a rectifier's
+// step or a window's maximum and another order to the other, a whole gradient element goes with it.
+// HELD: groups of four images that a thread keeps in registers between its two passes (0: it reads them again).
+template <int COLS, bool EDGES, int HELD>
+__global__ __launch_bounds__(kThreads) void k_bn_train_pool(const float* __restrict__ x, float* __restrict__ y, float* __restrict__ pooled, Planes g, Cut cut, int64_t n,
+                                                            BnOut o, u64* page) {
   __shared__ Sums sh;
   const int c = blockIdx.x % g.C, w = blockIdx.x / g.C;
-  u64* const slots[2] = {page + c * g.G, page + kBnHeldSlots + c * g.G};
-  float v[N][2][COLS];
-  // a share's sum (pass 0) or squared deviations (pass 1), loaded where it is not the one in registers
-  auto share = [&](int who, float mean, bool sq, bool load, float (&hold)[N][2][COLS]) __attribute__((always_inline)) {
-    float acc = 0.0f;
-#pragma unroll
-    for (int k = 0; k < N; k++) {
-      const int u = who * g.per + k * (int)blockDim.x + (int)threadIdx.x;
-      const bool mine = k * (int)blockDim.x + (int)threadIdx.x < g.per && u < g.units;
-      const Unit<COLS, EDGES> t(g, mine ? u : 0);
-      if (load && mine) t.load(g, x + t.at(g, c), hold[k]);
-      float s[2][COLS];
-#pragma unroll
-      for (int r = 0; r < 2; r++)
-#pragma unroll
-        for (int e = 0; e < COLS; e++) {
-          const float d = hold[k][r][e] - mean;
-          s[r][e] = !mine || !t.has(r, e) ? 0.0f : sq ? d * d : hold[k][r][e];
-        }
-      float q = 0.0f;
-#pragma unroll
-      for (int e = 0; e < COLS; e += 2) q = q + ((s[0][e] + s[0][e + 1]) + (s[1][e] + s[1][e + 1]));
-      acc = acc + q;
-    }
-    return group_sum(acc, sh.waves);
+  u64* const slots[2] = {page + c * cut.groups, page + kBnHeldSlots + c * cut.groups};
+  const int quarter = threadIdx.x >> 8, t = threadIdx.x & 255, mine = w * cut.own + quarter;
+  const bool works = quarter < cut.own && mine < cut.groups;
+  const int B = (int)(n / cut.S), img = g.C * cut.S, step = cut.groups * 256;
+  float v[HELD > 0 ? HELD : 1][4];
+  auto term = [&](float x_, float mean, bool sq) {
+    if (!sq) return x_;
+    const float d = x_ - mean;
+    return d * d;
   };
-  float sum[2];
-  {
-    const float mine = share(w, 0.0f, false, true, v);
-    if (threadIdx.x == 0) publish(slots[0], w, mine);
-    u64* const s0[2] = {slots[0], slots[0]};
-    total(s0, 1, g.G, g.polls, sh, sum, [&](int who, float (&r)[2]) {
-      float other[N][2][COLS];
-      r[0] = share(who, 0.0f, false, true, other);
+  // thread t's sum of group k: of values (mean 0) or of squared deviations
+  auto walk = [&](int k, float mean, bool sq) {
+    if (cut.S < 256) {
+      float acc = 0.0f;
+      for (int b = k * 256 + t; b < B; b += step) {
+        const float* const p = x + (b * g.C + c) * cut.S;
+        for (int d = 0; d < cut.S; d++) acc = acc + term(p[d], mean, sq);
+      }
+      return acc;
+    }
+    float a4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int d = k * 256 + t; d < cut.S; d += step) {
+      const float* const p = x + c * cut.S + d;
+      int b = 0;
+      for (; b + 4 <= B; b += 4) {
+        const float v0 = p[b * img], v1 = p[(b + 1) * img], v2 = p[(b + 2) * img], v3 = p[(b + 3) * img];
+        a4[0] = a4[0] + term(v0, mean, sq);
+        a4[1] = a4[1] + term(v1, mean, sq);
+        a4[2] = a4[2] + term(v2, mean, sq);
+        a4[3] = a4[3] + term(v3, mean, sq);
+      }
+      for (; b < B; b++) a4[0] = a4[0] + term(p[b * img], mean, sq);
+    }
+    return (a4[0] + a4[1]) + (a4[2] + a4[3]);
+  };
+  // the same from and to registers: whole groups of four images only, HELD of them at most
+  const int fours = B >> 2;
+  auto hold = [&](auto&& f) __attribute__((always_inline)) {   // f(slot, first value's place) for each group of four that thread t has
+    int b4 = 0, d = mine * 256 + t;
+#pragma unroll
+    for (int j = 0; j < HELD; j++) {
+      if (d < cut.S) f(j, c * cut.S + d + 4 * b4 * img);
+      if (++b4 == fours) { b4 = 0; d += step; }
+    }
+  };
+  auto held = [&](float mean, bool sq) __attribute__((always_inline)) {
+    float a4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    hold([&](int j, int) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) a4[e] = a4[e] + term(v[j][e], mean, sq);
     });
+    return (a4[0] + a4[1]) + (a4[2] + a4[3]);
+  };
+  // a group's sum, in all of its threads: block_sum of k_bn_reduce
+  auto group = [&](float acc) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) sh.waves[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    const float* const four = sh.waves + 4 * quarter;
+    return (four[0] + four[1]) + (four[2] + four[3]);
+  };
+  float mean = 0.0f, var = 0.0f, sum[2];
+  if constexpr (HELD > 0) {
+    if (works)
+      hold([&](int j, int at) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[j][e] = x[at + e * img];
+      });
   }
-  const float mean = sum[0] / (float)n;
-  __syncthreads();
-  {
-    const float mine = share(w, mean, true, false, v);
-    if (threadIdx.x == 0) publish(slots[1], w, mine);
-    u64* const s1[2] = {slots[1], slots[1]};
-    total(s1, 1, g.G, g.polls, sh, sum, [&](int who, float (&r)[2]) {
-      float other[N][2][COLS];
-      r[0] = share(who, mean, true, true, other);
-    });
+#pragma unroll
+  for (int pass = 0; pass < 2; pass++) {
+    const bool sq = pass == 1;
+    float acc = 0.0f;
+    if (works) acc = HELD > 0 ? held(mean, sq) : walk(mine, mean, sq);
+    const float s = group(acc);
+    if (works && t == 0) publish(slots[pass], mine, s);
+    u64* const both[2] = {slots[pass], slots[pass]};
+    total(both, 1, cut.groups, g.polls, sh, sum, [&](int k, float (&r)[2]) { r[0] = group(walk(k, mean, sq)); });
+    if (!sq) mean = sum[0] / (float)n;
+    else var = sum[0];
+    __syncthreads();   // the sums have been read
   }
-  const float var = sum[0];
   if (w == 0 && threadIdx.x == 0) {
     o.save_mean[c] = mean;
     o.save_var[c] = var;
@@ -241,36 +288,37 @@ __global__ __launch_bounds__(kThreads) void k_bn_train_pool(const float* __restr
   }
   const float a = 1.0f / sqrtf(var / (float)n + o.eps);
   const float b = -mean * a;
-#pragma unroll
-  for (int k = 0; k < N; k++) {
-    const int u = w * g.per + k * (int)blockDim.x + (int)threadIdx.x;
-    if (k * (int)blockDim.x + (int)threadIdx.x >= g.per || u >= g.units) break;
-    const Unit<COLS, EDGES> t(g, u);
+  // the values again, from the caches, as the pooling's windows lie
+  const int end = min(g.units, (w + 1) * g.per);
+#pragma unroll 2
+  for (int u = w * g.per + threadIdx.x; u < end; u += blockDim.x) {
+    const Unit<COLS, EDGES> q(g, u);
     float z[2][COLS];
+    q.load(g, x + q.at(g, c), z);
 #pragma unroll
     for (int r = 0; r < 2; r++)
 #pragma unroll
       for (int e = 0; e < COLS; e++) {
-        const float m = v[k][r][e] * a;
+        const float m = z[r][e] * a;
         z[r][e] = m + b;
       }
-    t.store(g, y + t.at(g, c), z);
-    if (EDGES && !(t.right && t.below)) continue;
+    q.store(g, y + q.at(g, c), z);
+    if (EDGES && !(q.right && q.below)) continue;
     float best[COLS / 2];
 #pragma unroll
     for (int e = 0; e < COLS / 2; e++) {
       best[e] = -FLT_MAX;
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const float r = relu_of(z[q >> 1][2 * e + (q & 1)]);
+      for (int k = 0; k < 4; k++) {
+        const float r = relu_of(z[k >> 1][2 * e + (k & 1)]);
         if (r > best[e]) best[e] = r;
       }
     }
-    float* const p = pooled + t.pooled(g, c);
+    float* const p = pooled + q.pooled(g, c);
     if constexpr (COLS == 4) *(Vec<2>::T*)p = Vec<2>::T{best[0], best[1]};
     else *p = best[0];
   }
-  leave(slots, (unsigned*)(page + 2 * kBnHeldSlots) + c, g.G);
+  leave(slots, (unsigned*)(page + 2 * kBnHeldSlots) + c, cut.groups, g.G);
 }
 
 // x: the tensor that was rectified and pooled; dp: the pooled tensor's gradient; dx: the gradient of x; z: the tensor that was
@@ -384,7 +432,7 @@ __global__ __launch_bounds__(kThreads) void k_pool_bn_bwd(const float* x, const 
       }
     t.store(g, dz + t.at(g, c), gv[k]);
   }
-  leave(slots, (unsigned*)(page + 2 * kBnHeldSlots) + c, g.G);
+  leave(slots, (unsigned*)(page + 2 * kBnHeldSlots) + c, g.G, g.G);
 }
 
 // ---- which commands ---------------------------------------------------------------------
@@ -399,43 +447,71 @@ bool pools(const gh_cmd& c) {
   return c.dim[0] > 0 && c.dim[1] > 0 && c.dim[2] >= 2 && c.dim[3] >= 2;
 }
 
-constexpr int kMost = 3;   // units of a thread, of four columns each: 24 values
+constexpr int kMost = 3;   // units of a thread in the gradient, of four columns each: 24 values, and as many of the other tensor
 
-// How the planes go to workgroups: false where a channel does not fit them.
-bool split(const gh_cmd& pool, uint64_t wide, uint64_t narrow, int cus, Planes& g, int& cols, int& threads, int& N) {
-  const int64_t B = pool.dim[0], C = pool.dim[1], H = pool.dim[2], W = pool.dim[3];
-  if (C > cus || C > kBnHeldSlots || B * C * H * W > INT32_MAX || B * H * W < 2) return false;
-  cols = W % 4 == 0 && H % 2 == 0 && wide % 16 == 0 && narrow % 8 == 0 ? 4 : W % 2 == 0 && H % 2 == 0 && wide % 8 == 0 ? 2 : 1;
-  const int64_t across = cols == 4 ? W / 4 : (W + 1) / 2, units = B * ((H + 1) / 2) * across;
-  // a compute unit for each workgroup, and half of its threads' work at least: a channel of 8 x 26 x 26 takes 7.9 and 7.9 us
-  // (forward and gradient) with one workgroup, 7.3 and 6.7 with two
-  int64_t G = std::min<int64_t>({(int64_t)cus / C, 64, kBnHeldSlots / C, (units + 511) / 512});
-  if (G < 1) G = 1;
+struct Plan {
+  Planes g;
+  Cut cut;
+  int cols, threads, N;   // N: units of a thread (the gradient)
+  bool held;              // the forward's values stay in registers
+};
+
+// How the planes go to workgroups, one to a compute unit: false where a channel does not fit them.
+bool plan(const gh_cmd& pool, bool fwd, uint64_t wide, uint64_t narrow, int cus, Plan& p) {
+  const int64_t B = pool.dim[0], C = pool.dim[1], H = pool.dim[2], W = pool.dim[3], S = H * W, n = B * S;
+  if (C > cus || B * C * S > INT32_MAX || n < 2) return false;
+  p.cols = W % 4 == 0 && H % 2 == 0 && wide % 16 == 0 && narrow % 8 == 0 ? 4 : W % 2 == 0 && H % 2 == 0 && wide % 8 == 0 ? 2 : 1;
+  const int64_t across = p.cols == 4 ? W / 4 : (W + 1) / 2, units = B * ((H + 1) / 2) * across;
+  // half of a workgroup's threads have work at least: the gradient of 8 x 128 x 26 x 26 takes 7.9 us with one workgroup to a
+  // channel, 6.7 with two
+  int64_t G = std::min<int64_t>({(int64_t)cus / C, 64, (units + 511) / 512});
+  p.cut = {(int)S, 0, 0};
+  if (fwd) {
+    const int64_t groups = gh_bn_groups(n, S);
+    G = std::max(G, (groups + 3) / 4);
+    if (C * G > cus || C * groups > kBnHeldSlots) return false;
+    p.cut.groups = (int)groups;
+    p.cut.own = (int)((groups + G - 1) / G);
+  }
   const int64_t per = (units + G - 1) / G;
-  N = (int)((per + kThreads - 1) / kThreads);
-  if (N > kMost * (cols == 4 ? 1 : 2)) return false;
-  threads = (int)(((per + N - 1) / N + 63) / 64 * 64);
-  g = {(int)H, (int)W, (int)across, (int)((H + 1) / 2 * across), (int)units, (int)per, (int)C, (int)((units + per - 1) / per), kPolls};
-  if (const char* asks = getenv("GORGONIA_HIP_BN_POLLS")) g.polls = std::max(0, std::min(kPolls, atoi(asks)));
+  p.g = {(int)H, (int)W, (int)across, (int)((H + 1) / 2 * across), (int)units, (int)per, (int)C, (int)G, kPolls};
+  if (fwd) {
+    p.N = 0;
+    p.threads = (int)std::max<int64_t>(256 * p.cut.own, std::min<int64_t>(kThreads, (per + 255) / 256 * 256));
+    // (a thread's strips of 256 values, of whole groups of four images)
+    p.held = S >= 256 && B % 4 == 0 && ((S + 255) / 256 + p.cut.groups - 1) / p.cut.groups * (B / 4) <= kHeld;
+  } else {
+    p.g.G = (int)((units + per - 1) / per);
+    p.N = (int)((per + kThreads - 1) / kThreads);
+    if (C * p.g.G > kBnHeldSlots || p.N > kMost * (p.cols == 4 ? 1 : 2)) return false;
+    p.threads = (int)(((per + p.N - 1) / p.N + 63) / 64 * 64);
+  }
+  if (const char* asks = getenv("GORGONIA_HIP_BN_POLLS")) p.g.polls = std::max(0, std::min(kPolls, atoi(asks)));
   return true;
 }
 
-// f(kernel arguments' types): the form for cols and N
+// f(columns, edges, units of a thread): the gradient's form
 template <class F>
-void with_form(int cols, int N, F&& f) {
-  if (cols == 4) {
-    if (N == 1) f(std::integral_constant<int, 4>(), std::false_type(), std::integral_constant<int, 1>());
-    else if (N == 2) f(std::integral_constant<int, 4>(), std::false_type(), std::integral_constant<int, 2>());
-    else f(std::integral_constant<int, 4>(), std::false_type(), std::integral_constant<int, 3>());
-  } else if (cols == 2) {
-    if (N == 1) f(std::integral_constant<int, 2>(), std::false_type(), std::integral_constant<int, 1>());
-    else if (N == 2) f(std::integral_constant<int, 2>(), std::false_type(), std::integral_constant<int, 2>());
-    else f(std::integral_constant<int, 2>(), std::false_type(), std::integral_constant<int, 6>());
-  } else {
-    if (N == 1) f(std::integral_constant<int, 2>(), std::true_type(), std::integral_constant<int, 1>());
-    else if (N == 2) f(std::integral_constant<int, 2>(), std::true_type(), std::integral_constant<int, 2>());
-    else f(std::integral_constant<int, 2>(), std::true_type(), std::integral_constant<int, 6>());
-  }
+void with_form(const Plan& p, F&& f) {
+  auto of = [&](auto cols, auto edges, auto most) {
+    if (p.N == 1) f(cols, edges, std::integral_constant<int, 1>());
+    else if (p.N == 2) f(cols, edges, std::integral_constant<int, 2>());
+    else f(cols, edges, most);
+  };
+  if (p.cols == 4) of(std::integral_constant<int, 4>(), std::false_type(), std::integral_constant<int, kMost>());
+  else if (p.cols == 2) of(std::integral_constant<int, 2>(), std::false_type(), std::integral_constant<int, 2 * kMost>());
+  else of(std::integral_constant<int, 2>(), std::true_type(), std::integral_constant<int, 2 * kMost>());
+}
+// f(columns, edges, held): the forward's
+template <class F>
+void with_held(const Plan& p, F&& f) {
+  auto of = [&](auto cols, auto edges) {
+    if (p.held) f(cols, edges, std::integral_constant<int, kHeld>());
+    else f(cols, edges, std::integral_constant<int, 0>());
+  };
+  if (p.cols == 4) of(std::integral_constant<int, 4>(), std::false_type());
+  else if (p.cols == 2) of(std::integral_constant<int, 2>(), std::false_type());
+  else of(std::integral_constant<int, 2>(), std::true_type());
 }
 
 template <class T> T* at(uint64_t p) { return (T*)(uintptr_t)p; }
@@ -486,9 +562,8 @@ bool gh_bn_held_pair(const gh_ctx* ctx, const gh_cmd* c, int n) {
   if (!fwd && !(c[0].opcode == GH_OP_MAXPOOL2D_BWD && c[1].opcode == GH_OP_BN_BWD)) return false;
   std::string m;
   Tensors t;
-  Planes g;
-  int cols, threads, N;
-  return gh_validate_cmd(c[1], m) == GH_OK && fits(c, t) && split(c[fwd ? 1 : 0], t.wide, t.narrow, ctx->cu_count, g, cols, threads, N);
+  Plan p;
+  return gh_validate_cmd(c[1], m) == GH_OK && fits(c, t) && plan(c[fwd ? 1 : 0], fwd, t.wide, t.narrow, ctx->cu_count, p);
 }
 
 int gh_launch_bn_held_pair(gh_ctx* ctx, const gh_cmd* c) {
@@ -496,22 +571,23 @@ int gh_launch_bn_held_pair(gh_ctx* ctx, const gh_cmd* c) {
   for (int k = 0; k < 2; k++)
     for (uint64_t p : c[k].ptr) ctx->llc.touch(p, 0, false);
   Tensors t;
-  Planes g;
-  int cols, threads, N;
-  if (!fits(c, t) || !split(c[fwd ? 1 : 0], t.wide, t.narrow, ctx->cu_count, g, cols, threads, N)) return gh_fail(ctx, GH_EINVAL, "not a pair of commands that one launch takes");
+  Plan p;
+  if (!fits(c, t) || !plan(c[fwd ? 1 : 0], fwd, t.wide, t.narrow, ctx->cu_count, p)) return gh_fail(ctx, GH_EINVAL, "not a pair of commands that one launch takes");
   const gh_cmd &pool = fwd ? c[1] : c[0], &bn = fwd ? c[0] : c[1];
   const int64_t count = bn.dim[0] * bn.dim[2];
-  const dim3 grid((unsigned)(g.C * g.G)), block((unsigned)threads);
+  const dim3 grid((unsigned)(p.g.C * p.g.G)), block((unsigned)p.threads);
   u64* const page = (u64*)ctx->bn_page;
-  with_form(cols, N, [&](auto COLS, auto EDGES, auto UNITS) {
-    if (fwd) {
-      const BnOut o{at<float>(bn.ptr[2]), at<float>(bn.ptr[3]), at<float>(bn.ptr[4]), at<float>(bn.ptr[5]), bn.f[0], bn.f[1]};
-      hipLaunchKernelGGL((k_bn_train_pool<COLS(), EDGES(), UNITS()>), grid, block, 0, ctx->stream, at<const float>(bn.ptr[0]), at<float>(bn.ptr[1]), at<float>(pool.ptr[1]), g,
-                         count, o, page);
-    } else {
+  if (fwd) {
+    const BnOut o{at<float>(bn.ptr[2]), at<float>(bn.ptr[3]), at<float>(bn.ptr[4]), at<float>(bn.ptr[5]), bn.f[0], bn.f[1]};
+    with_held(p, [&](auto COLS, auto EDGES, auto HELD) {
+      hipLaunchKernelGGL((k_bn_train_pool<COLS(), EDGES(), HELD()>), grid, block, 0, ctx->stream, at<const float>(bn.ptr[0]), at<float>(bn.ptr[1]), at<float>(pool.ptr[1]), p.g,
+                         p.cut, count, o, page);
+    });
+  } else {
+    with_form(p, [&](auto COLS, auto EDGES, auto UNITS) {
       hipLaunchKernelGGL((k_pool_bn_bwd<COLS(), EDGES(), UNITS()>), grid, block, 0, ctx->stream, at<const float>(pool.ptr[0]), at<const float>(pool.ptr[1]),
-                         at<float>(pool.ptr[2]), at<const float>(bn.ptr[0]), at<float>(bn.ptr[2]), g, count, at<const float>(bn.ptr[3]), at<const float>(bn.ptr[4]), bn.f[0], page);
-    }
-  });
+                         at<float>(pool.ptr[2]), at<const float>(bn.ptr[0]), at<float>(bn.ptr[2]), p.g, count, at<const float>(bn.ptr[3]), at<const float>(bn.ptr[4]), bn.f[0], page);
+    });
+  }
   return gh_check_hip(ctx, hipGetLastError(), fwd ? "batchnorm statistics launch" : "batchnorm backward launch");
 }

@@ -549,15 +549,15 @@ __global__ __launch_bounds__(kBlock) void k_dropout_bwd(const float* __restrict_
 }
 
 // how many workgroups share one channel's reduction
-int bn_groups(int64_t n, int64_t S) {
+}  // namespace
+
+int gh_bn_groups(int64_t n, int64_t S) {
   // wide planes: two 256-wide strips of every image per workgroup; else 1024 images per workgroup
   int64_t g = S >= kBlock ? (S + kBlock - 1) / kBlock / 2 : (n / S) / 1024;
   if (g < 1) g = 1;
   if (g > 64) g = 64;
   return (int)g;
 }
-
-}  // namespace
 
 int gh_launch_maxpool2d_bwd(gh_ctx* ctx, const gh_cmd& c) {
   if (gh_dtype_of(c.flags) == GH_F64) return gh_launch_maxpool2d_bwd_f64(ctx, c);
@@ -620,7 +620,7 @@ int gh_launch_maxpool2d_bwd(gh_ctx* ctx, const gh_cmd& c) {
 int gh_launch_bn_train(gh_ctx* ctx, const gh_cmd& c) {
   if (gh_dtype_of(c.flags) == GH_F64) return gh_launch_bn_train_f64(ctx, c);
   const int64_t B = c.dim[0], C = c.dim[1], S = c.dim[2], n = B * S;
-  const int G = bn_groups(n, S);
+  const int G = gh_bn_groups(n, S);
   const int64_t need = (2 * C * G + C) * 4;   // [C][G] sums, [C][G] squared deviations (and C more, as ever)
   if (need > ctx->workspace_bytes) {
     // under gh_submit_noalloc: the refusal that names the need; there is no smaller plan to fall back to
@@ -653,7 +653,7 @@ int gh_launch_bn_train(gh_ctx* ctx, const gh_cmd& c) {
 int gh_launch_bn_bwd(gh_ctx* ctx, const gh_cmd& c) {
   if (gh_dtype_of(c.flags) == GH_F64) return gh_launch_bn_bwd_f64(ctx, c);
   const int64_t B = c.dim[0], C = c.dim[1], S = c.dim[2], n = B * S;
-  const int G = bn_groups(n, S);
+  const int G = gh_bn_groups(n, S);
   if (2 * C * G * 4 > ctx->workspace_bytes) {
     if (const int rc = gh_ws_short(ctx, 2 * C * G * 4)) return rc;
     return gh_fail(ctx, GH_ESTATE, "batchnorm: reduction scratch does not fit the workspace");

@@ -1,6 +1,7 @@
 """Batch statistics with the pooling behind them and their gradients in one launch (k_bn_held.hip): every tensor that the two
-commands write.  The saved statistics are held to a float64 sum, what is computed from them to the bit; the gradient's two sums
-are not stored, so that its result is held to the bound their rounding leaves."""
+commands write.  The forward's are those of the two commands apart, to the bit; the saved statistics are held to a float64 sum,
+what is computed from them to the bit; the gradient's two sums are not stored, so that its result is held to the bound that
+their rounding leaves."""
 import numpy as np
 import pytest
 
@@ -11,8 +12,8 @@ from tests.util import assert_bits_equal
 pytestmark = pytest.mark.gpu
 
 EPS, MOMENTUM = 1e-5, 0.1
-# a value passes at most 3 + 6 additions in its thread, 6 in its wavefront, 16 and 64 behind it
-DEPTH = 100
+# a value passes at most 72 additions in its thread (of the shapes below), 6 in its wavefront, 3 and 64 behind it
+DEPTH = 150
 U = 2.0 ** -24
 # four columns a load with one to three units a thread, two columns with one to six, single loads (an odd size), one workgroup a
 # channel and sixty-four, a window for each channel, more channels than half of the compute units
@@ -68,14 +69,15 @@ def _commands(m, shape, z="x", dz="dz"):
     return [bn, pool], [back, D.cmd_bn_bwd(m[z], m["t"], m[dz], m["sm"], m["sv"], B, C, H * W, EPS)]
 
 
-def _run(ctx, shape, seed, shift=0, dz="dz", polls=None, monkeypatch=None, together=True):
+def _run(ctx, shape, seed, shift=0, dz="dz", polls=None, monkeypatch=None, together=True, forward=True):
     x, rm, rv, dp = _inputs(shape, seed)
     nan = np.full_like(x, np.nan)
     m = _Place(ctx, shift, x=x, y=nan, p=np.full_like(dp, np.nan), rm=rm, rv=rv, sm=np.full_like(rm, np.nan), sv=np.full_like(rm, np.nan), dp=dp, t=nan, dz=nan)
     if polls is not None:
         monkeypatch.setenv("GORGONIA_HIP_BN_POLLS", str(polls))
     fwd, bwd = _commands(m, shape, dz=dz)
-    ctx.run(fwd)
+    for group in ([fwd] if forward else [[c] for c in fwd]):
+        ctx.run(group)
     for group in ([bwd] if together else [[c] for c in bwd]):
         ctx.run(group)
     return (x, rm, rv, dp), m.all()
@@ -102,9 +104,9 @@ def _check(shape, given, got, dz="dz"):
     if dz != "y":
         assert_bits_equal(got["y"], y)
     win = _windows(_relu(y))
-    assert_bits_equal(got["p"], win.max(0))
-    # MaxPool2DDiff behind Rectify: the first of the largest takes dy where y >= 0
+    # the first of the largest; MaxPool2DDiff behind Rectify gives it dy where y >= 0
     first = win.argmax(0)
+    assert_bits_equal(got["p"], np.take_along_axis(win, first[None], 0)[0])
     t = np.zeros_like(y)
     for k in range(4):
         hit = np.where(first == k, np.float32(0) + dp, np.float32(0))
@@ -129,6 +131,10 @@ def test_one_launch(ctx, shape):
     for dz in ("dz", "y"):   # the normalised tensor's gradient in a place of its own, or over the pooled tensor's source
         given, got = _run(ctx, shape, 5, dz=dz)
         _check(shape, given, got, dz)
+    _, apart = _run(ctx, shape, 5, forward=False)
+    for k in ("y", "p", "sm", "sv", "rm", "rv", "t"):
+        if k != "y":   # (the last gradient lies over it)
+            assert_bits_equal(got[k], apart[k])
 
 
 @pytest.mark.parametrize("shift", [1, 2])
