@@ -94,8 +94,36 @@ static void give_word(uint32_t* w) {
   g_words_used &= ~(1ull << (((unsigned char*)w - g_words_page) / 64));
 }
 
+// The contexts' pages for k_bn_held.hip, 64 on a device, part of the library's device image as `scratch` is: zero from load
+// time on, and again whenever no kernel runs.  A context beyond the 64th has none and runs those commands apart.
+static constexpr int kBnPages = 64;
+static __device__ __align__(256) unsigned char bn_pages[kBnPages][kBnHeldPage];
+static std::mutex g_pages_mu;
+static unsigned char* g_pages[kMaxDevices] = {};
+static uint64_t g_pages_used[kMaxDevices] = {};
+
+static void* take_page(int device) {   // `device` is current
+  if (device < 0 || device >= kMaxDevices) return nullptr;
+  std::lock_guard<std::mutex> lock(g_pages_mu);
+  if (!g_pages[device]) {
+    void* p = nullptr;
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(bn_pages)) != hipSuccess) (void)hipGetLastError();
+    g_pages[device] = (unsigned char*)p;
+  }
+  if (!g_pages[device] || ~g_pages_used[device] == 0) return nullptr;
+  const int i = __builtin_ctzll(~g_pages_used[device]);
+  g_pages_used[device] |= 1ull << i;
+  return g_pages[device] + i * kBnHeldPage;
+}
+static void give_page(const gh_ctx* ctx) {
+  if (!ctx->bn_page || ctx->err == GH_EDEVICE) return;   // (a kernel that did not end may have left it as it was)
+  std::lock_guard<std::mutex> lock(g_pages_mu);
+  g_pages_used[ctx->device] &= ~(1ull << (((unsigned char*)ctx->bn_page - g_pages[ctx->device]) / kBnHeldPage));
+}
+
 static void drop_ctx(gh_ctx* ctx) {
   give_word(ctx->done_word);   // nothing is in flight any more
+  give_page(ctx);
   if (ctx->workspace) hipFree(ctx->workspace);
   if (ctx->arena) hipFree(ctx->arena);
   hipStreamDestroy(ctx->stream);
@@ -153,14 +181,13 @@ int gh_init(int device, int64_t arena_bytes, gh_ctx** out) {
   // filters.  Mandatory: the launchers index it without asking again.
   ctx->workspace_bytes = 64ll << 20;
   void* fixed = nullptr;
-  if (hipMalloc(&ctx->workspace, (size_t)(ctx->workspace_bytes + kBnHeldPage)) != hipSuccess ||
-      hipMemset((char*)ctx->workspace + ctx->workspace_bytes, 0, (size_t)kBnHeldPage) != hipSuccess || hipDeviceSynchronize() != hipSuccess ||
+  if (hipMalloc(&ctx->workspace, (size_t)ctx->workspace_bytes) != hipSuccess ||
       static_scratch(device, &fixed) != hipSuccess) {
     (void)hipGetLastError();
     drop_ctx(ctx);
     return GH_EOOM;
   }
-  ctx->bn_page = (char*)ctx->workspace + ctx->workspace_bytes;
+  ctx->bn_page = take_page(device);
   *out = ctx;
   return GH_OK;
 }

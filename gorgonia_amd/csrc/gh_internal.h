@@ -63,7 +63,7 @@ struct gh_ctx {
   void* workspace = nullptr;
   int64_t workspace_bytes = 0;
   // what the workgroups of k_bn_held.hip pass to each other: two slots of 8 bytes and one count of 4 for each of
-  // kBnHeldSlots, behind the workspace (no plan reaches them), zero whenever no kernel runs
+  // kBnHeldSlots, zero whenever no kernel runs; null where the device's pages were all taken
   void* bn_page = nullptr;
   // set while gh_submit_noalloc runs: the scratch is the library's fixed array and a
   // plan may not shrink to fit it (results must not depend on the scratch size)

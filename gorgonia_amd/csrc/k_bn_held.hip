@@ -557,7 +557,7 @@ bool fits(const gh_cmd* c, Tensors& t) {
 
 // (c[0] is a valid command; c[1] is looked at where its opcode makes it a candidate)
 bool gh_bn_held_pair(const gh_ctx* ctx, const gh_cmd* c, int n) {
-  if (n < 2) return false;
+  if (n < 2 || !ctx->bn_page) return false;
   const bool fwd = c[0].opcode == GH_OP_BN_TRAIN && c[1].opcode == GH_OP_MAXPOOL2D;
   if (!fwd && !(c[0].opcode == GH_OP_MAXPOOL2D_BWD && c[1].opcode == GH_OP_BN_BWD)) return false;
   std::string m;

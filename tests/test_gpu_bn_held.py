@@ -184,3 +184,26 @@ def test_replays(ctx):
         ctx.run(fwd + bwd)
     ctx.graph_destroy(graph)
     m.all()
+
+
+def test_two_contexts_at_once(ctx):
+    """Each has places of its own for the sums that its workgroups exchange."""
+    shape = (8, 16, 104, 104)
+    x, rm, rv, dp = _inputs(shape, 10)
+    nan = np.full_like(x, np.nan)
+    _, want = _run(ctx, shape, 10)
+    with D.Context() as other:
+        both = []
+        for c in (ctx, other):
+            m = _Place(c, 0, x=x, y=nan, p=np.full_like(dp, np.nan), rm=rm, rv=rv, sm=rm * 0, sv=rm * 0, dp=dp, t=nan, dz=nan)
+            both.append((c, m, sum(_commands(m, shape), [])))
+        for _ in range(20):
+            for c, m, cmds in both:
+                c.h2d(m["rm"], rm)
+                c.h2d(m["rv"], rv)
+                c.submit(cmds)
+        for c, m, cmds in both:
+            c.sync()
+            got = m.all()
+            for k in want:
+                assert_bits_equal(got[k], want[k])
