@@ -3282,7 +3282,8 @@ static bool conv_direct_shape(const gh_cmd& c) {
 
 // The direct kernel's shapes, less those the wide-image kernel runs quicker: three or four
 // channels fill most of a quad of its K steps, and on images with enough pixels its matrix
-// cores then beat the vector units (3 -> 16 at 416 x 416: 42 us against 53).  Only where it can
+// cores then beat the vector units (3 -> 16 at 416 x 416: 42 us against 53; k_conv3x3_strip, which
+// runs those with even rows and columns, 30).  Only where it can
 // also pool, so that a shape's plain and pooled commands stay with one kernel and one summing
 // order.
 static bool conv_direct_takes(const gh_cmd& c) {
@@ -3382,6 +3383,7 @@ int gh_launch_conv2d(gh_ctx* ctx, const gh_cmd& c) {
   if (conv_direct_takes(c)) return launch_conv_direct(ctx, c);
   const int rcs = gh_try_launch_conv_small(ctx, c);
   if (rcs >= 0) return rcs;
+  if (gh_conv_strip_takes(c) && gh_conv_wide_takes(c)) return gh_launch_conv_strip(ctx, c);
   if (const int form = conv_lanes_form(c, ctx->cu_count); form >= 0) return gh_launch_conv_lanes(ctx, c, false, form);
   const int rcp = gh_try_launch_conv_patch(ctx, c);
   if (rcp >= 0) return rcp;
