@@ -181,12 +181,13 @@ int gh_init(int device, int64_t arena_bytes, gh_ctx** out) {
   // filters.  Mandatory: the launchers index it without asking again.
   ctx->workspace_bytes = 64ll << 20;
   void* fixed = nullptr;
-  if (hipMalloc(&ctx->workspace, (size_t)ctx->workspace_bytes) != hipSuccess ||
+  if (hipMalloc(&ctx->workspace, (size_t)(ctx->workspace_bytes + kSlabSpace)) != hipSuccess ||
       static_scratch(device, &fixed) != hipSuccess) {
     (void)hipGetLastError();
     drop_ctx(ctx);
     return GH_EOOM;
   }
+  ctx->slab_space = (char*)ctx->workspace + ctx->workspace_bytes;
   ctx->bn_page = take_page(device);
   *out = ctx;
   return GH_OK;
@@ -495,12 +496,13 @@ int gh_validate(const gh_cmd* cmds, int n, char* msg, int msg_len) {
   return GH_OK;
 }
 
-static int submit_cmds(gh_ctx* ctx, const gh_cmd* cmds, int n) {
+static int submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
   ctx->idle = false;
   for (int i = 0; i < n; i++) {
     std::string m;
     int rc = gh_validate_cmd(cmds[i], m);
     if (rc) return gh_fail(ctx, rc, "cmd " + std::to_string(i) + ": " + m);
+    if ((rc = gh_flush_sums_before(ctx, cmds[i]))) return rc;
     // a run of solver steps with the same settings (a model's weight tensors) is one launch, and so is a run of
     // elementwise commands on tensors of one size
     const int solver = gh_solver_run_length(cmds + i, n - i);
@@ -517,11 +519,21 @@ static int submit_cmds(gh_ctx* ctx, const gh_cmd* cmds, int n) {
     }
     // two commands of which the second reads what the first writes are one launch where a kernel takes both
     const bool held = gh_bn_held_pair(ctx, cmds + i, n - i), pair = held || gh_is_pair(cmds + i, n - i);
+    if (pair && (rc = gh_flush_sums_before(ctx, cmds[i + 1]))) return rc;
     rc = held ? gh_launch_bn_held_pair(ctx, cmds + i) : pair ? gh_launch_pair(ctx, cmds + i) : dispatch(ctx, cmds[i]);
     if (rc) return rc;
     if (pair) i++;
   }
   return GH_OK;
+}
+
+// Sums of filter-gradient slabs may wait for the commands behind them (k_slab_sums.hip); none waits past the submission.
+static int submit_cmds(gh_ctx* ctx, const gh_cmd* cmds, int n) {
+  ctx->defer_sums = n > 1 && !ctx->ws_strict;
+  const int rc = submit_each(ctx, cmds, n);
+  ctx->defer_sums = false;
+  const int late = gh_flush_sums(ctx);
+  return rc ? rc : late;
 }
 
 int gh_submit(gh_ctx* ctx, const gh_cmd* cmds, int n) {

@@ -48,6 +48,17 @@ struct gh_llc_model {
 constexpr int kBnHeldSlots = 2048;
 constexpr int64_t kBnHeldPage = kBnHeldSlots * (8 + 8 + 4);
 
+// One sum of slabs (k_slab_sums.hip): out[e] = the sum over the slabs of ws[s][e], in one of these orders.
+enum { kSumGroups64, kSumGroups16, kSumGroups64F64, kSumGroups16F64, kSumLanes16, kSumLanes4, kSumPlain };
+struct gh_slab_sum {
+  const void* ws;
+  void* out;
+  int64_t total;
+  int slabs, how;
+};
+constexpr int kSlabSums = 8;
+constexpr int64_t kSlabSpace = 16ll << 20;   // (the larger allocation makes opening a context some 10 us slower)
+
 struct gh_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -65,6 +76,12 @@ struct gh_ctx {
   // what the workgroups of k_bn_held.hip pass to each other: two slots of 8 bytes and one count of 4 for each of
   // kBnHeldSlots, zero whenever no kernel runs; null where the device's pages were all taken
   void* bn_page = nullptr;
+  // slabs whose sums gh_submit has put off, behind the workspace (no other plan reaches them), and those sums
+  void* slab_space = nullptr;
+  int64_t slabs_used = 0;
+  gh_slab_sum sums[kSlabSums];
+  int pending = 0;
+  bool defer_sums = false;
   // set while gh_submit_noalloc runs: the scratch is the library's fixed array and a
   // plan may not shrink to fit it (results must not depend on the scratch size)
   bool ws_strict = false;
@@ -99,6 +116,10 @@ int gh_validate_cmd(const gh_cmd& c, std::string& msg);
 bool gh_llc_cold(const gh_ctx* ctx, uint64_t p);
 bool gh_llc_stream(int64_t bytes, bool cold);
 // {BN_TRAIN, MAXPOOL2D} and {MAXPOOL2D_BWD, BN_BWD} in one launch that reads a channel once (k_bn_held.hip)
+void* gh_slab_space(gh_ctx* ctx, int64_t bytes);
+int gh_sum_slabs(gh_ctx* ctx, const gh_slab_sum& s);
+int gh_flush_sums(gh_ctx* ctx);
+int gh_flush_sums_before(gh_ctx* ctx, const gh_cmd& c);
 int gh_bn_groups(int64_t n, int64_t S);   // the groups of 256 threads that k_bn_reduce cuts a channel of n values in planes of S into (k_bwd.hip)
 bool gh_bn_held_pair(const gh_ctx* ctx, const gh_cmd* cmds, int n);
 int gh_launch_bn_held_pair(gh_ctx* ctx, const gh_cmd* cmds);
@@ -144,7 +165,7 @@ int gh_launch_outer(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_conv2d(gh_ctx* ctx, const gh_cmd& c);
 // small-image 3x3 convolution (k_conv_small.hip): -1 when the shape is not one it takes
 int gh_try_launch_conv_small(gh_ctx* ctx, const gh_cmd& c);
-int gh_try_launch_conv_wgrad_small(gh_ctx* ctx, const gh_cmd& c, int* splits);
+int gh_try_launch_conv_wgrad_small(gh_ctx* ctx, const gh_cmd& c, int* splits, float** slabs);
 bool gh_conv_wgrad_small_takes(const gh_cmd& c);
 // 3x3 stride-1 filter gradient with operands straight from memory, both float types (k_conv_wgrad.hip)
 bool gh_conv_wgrad_takes(const gh_cmd& c, int cus);

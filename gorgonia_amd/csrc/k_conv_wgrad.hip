@@ -17,7 +17,7 @@
 //   * with fewer than 16 channels the columns of a tile are (channel, tap) pairs instead, packed without gaps,
 //     and each has its own P-wide load (kPacked).
 //   * the long axis is cut among wavefronts and workgroups; the four wavefronts of a workgroup meet in LDS, the
-//     workgroups' slabs in k_slab_sum, both in a fixed order.
+//     workgroups' slabs in k_slab_sums, both in a fixed order.
 // P is 4, or 2 where a row has at most eight columns.
 #include <algorithm>
 #include <type_traits>
@@ -245,48 +245,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   }
 }
 
-// out[e] = sum over the slabs of ws[s][e]: a workgroup takes RW results, its 256 / RW thread groups every G-th
-// slab (reads of a slab are RW values wide), and the groups' sums are added pairwise, neighbours first.
-template <class T, int RW>
-__global__ __launch_bounds__(256) void k_slab_sum(const T* __restrict__ ws, int slabs, int64_t total, T* __restrict__ out) {
-  constexpr int G = 256 / RW;
-  __shared__ T sh[256];
-  const int grp = threadIdx.x / RW;
-  const int64_t e = (int64_t)blockIdx.x * RW + threadIdx.x % RW;
-  T sum = (T)0;
-  if (e < total) {
-    int s = grp;
-    for (; s + 3 * G < slabs; s += 4 * G) {   // four loads in flight
-      T v[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) v[u] = ws[(int64_t)(s + u * G) * total + e];
-#pragma unroll
-      for (int u = 0; u < 4; u++) sum = sum + v[u];
-    }
-    for (; s < slabs; s += G) sum = sum + ws[(int64_t)s * total + e];
-  }
-  sh[threadIdx.x] = sum;
-  for (int d = 1; d < G; d <<= 1) {
-    __syncthreads();
-    T v = (T)0;
-    const bool mine = grp % (2 * d) == 0;
-    if (mine) v = sh[threadIdx.x] + sh[threadIdx.x + d * RW];
-    __syncthreads();
-    if (mine) sh[threadIdx.x] = v;
-  }
-  if (grp == 0 && e < total) out[e] = sh[threadIdx.x];
-}
-
-template <class T>
-int slab_sum(gh_ctx* ctx, const T* ws, int slabs, int64_t total, T* out) {
-  // 64 results to a workgroup where that makes enough workgroups, else 16
-  if (total >= 64 * (int64_t)ctx->cu_count)
-    hipLaunchKernelGGL((k_slab_sum<T, 64>), dim3((unsigned)((total + 63) / 64)), dim3(256), 0, ctx->stream, ws, slabs, total, out);
-  else
-    hipLaunchKernelGGL((k_slab_sum<T, 16>), dim3((unsigned)((total + 15) / 16)), dim3(256), 0, ctx->stream, ws, slabs, total, out);
-  return gh_check_hip(ctx, hipGetLastError(), "slab sum launch");
-}
-
 template <class T>
 bool fill(const gh_cmd& c, Wg<T>* g) {
   for (int i : {5, 6}) if (c.dim[i] != 3) return false;
@@ -330,11 +288,14 @@ int launch(gh_ctx* ctx, Wg<T> g, T* dw) {
   }
   g.per = (int)((g.items + slices * kWaves - 1) / (slices * kWaves));
   slices = (g.items + (int64_t)g.per * kWaves - 1) / ((int64_t)g.per * kWaves);
-  g.out = slices > 1 ? (T*)ctx->workspace : dw;
+  g.out = slices > 1 ? (T*)gh_slab_space(ctx, slices * results * (int64_t)sizeof(T)) : dw;
   hipLaunchKernelGGL((k_conv3x3_wgrad<T, TM, P, NT, kPacked>), dim3((unsigned)slices, (unsigned)ct, (unsigned)ft), dim3(kThreads), 0,
                      ctx->stream, g);
   const int rc = gh_check_hip(ctx, hipGetLastError(), "filter-gradient launch");
-  return rc || slices == 1 ? rc : slab_sum(ctx, (const T*)ctx->workspace, (int)slices, results, dw);
+    if (rc || slices == 1) return rc;
+  // 64 results to a workgroup of the sum where that makes enough workgroups, else 16
+  const bool many = results >= 64 * (int64_t)ctx->cu_count;
+  return gh_sum_slabs(ctx, {g.out, dw, results, (int)slices, sizeof(T) == 8 ? (many ? kSumGroups64F64 : kSumGroups16F64) : many ? kSumGroups64 : kSumGroups16});
 }
 
 template <class T>

@@ -313,9 +313,9 @@ bool gh_conv_wgrad_small_takes(const gh_cmd& c) {
 }
 
 // Returns -1 when the shape is not one this kernel takes (or its slabs do not fit the
-// workspace); otherwise the partial sums are in the workspace as *splits slabs of F x C*9
+// workspace); otherwise the partial sums are at *slabs, *splits slabs of F x C*9
 // (or, with *splits == 1, dW is complete).
-int gh_try_launch_conv_wgrad_small(gh_ctx* ctx, const gh_cmd& c, int* splits) {
+int gh_try_launch_conv_wgrad_small(gh_ctx* ctx, const gh_cmd& c, int* splits, float** slabs) {
   WgPlan p;
   if (!wgrad_small_plan(ctx, c, &p)) return -1;
   const int64_t slab = (int64_t)p.g.F * p.g.CKK;
@@ -333,7 +333,8 @@ int gh_try_launch_conv_wgrad_small(gh_ctx* ctx, const gh_cmd& c, int* splits) {
                                   160 * 1024);
   });
   if (attr_rc != hipSuccess) return gh_check_hip(ctx, attr_rc, "hipFuncSetAttribute(conv3x3 wgrad small)");
-  float* const dst = p.splits > 1 ? (float*)ctx->workspace : (float*)(uintptr_t)c.ptr[2];
+  float* const dst = p.splits > 1 ? (float*)gh_slab_space(ctx, slab * 4 * p.splits) : (float*)(uintptr_t)c.ptr[2];
+  *slabs = dst;
   const dim3 grid((unsigned)p.splits, (unsigned)(p.g.C / kCT), (unsigned)((p.g.F + kBM - 1) / kBM));
   hipLaunchKernelGGL(k_conv3x3_wgrad_small, grid, dim3(kThreads), p.lds, ctx->stream,
                      (const float*)(uintptr_t)c.ptr[0], (const float*)(uintptr_t)c.ptr[1], dst, p.g, slab);

@@ -455,36 +455,6 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(const float* __restrict__
   }
 }
 
-// Many slabs, few results (filter gradients): L lanes share one result (4, or 16 from 64
-// slabs up).  Lane q adds slabs q, q+L, q+2L, ... in that order, then the L sums are
-// combined pairwise, neighbours first: (s0 + s1) + (s2 + s3), ... - a fixed order, so
-// results repeat.
-template <class SC, int L>
-__global__ __launch_bounds__(256) void k_splitk_reduce_lanes(const float* __restrict__ ws, int splits, int M,
-                                                        int N, SC sc, int act, float alpha) {
-  const int64_t total = (int64_t)M * N;
-  const int q = threadIdx.x & (L - 1);
-  const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) / L;
-  float acc = 0.f;
-  if (e < total) {
-    const float* p = ws + (int64_t)q * total + e;
-    int s = q;
-    for (; s + 3 * L < splits; s += 4 * L) {   // four loads in flight
-      const float v0 = p[0], v1 = p[(int64_t)L * total], v2 = p[2 * (int64_t)L * total], v3 = p[3 * (int64_t)L * total];
-      acc = acc + v0; acc = acc + v1; acc = acc + v2; acc = acc + v3;
-      p += 4 * (int64_t)L * total;
-    }
-    for (; s < splits; s += L) { acc = acc + p[0]; p += (int64_t)L * total; }
-  }
-  float sum = acc;
-#pragma unroll
-  for (int d = 1; d < L; d <<= 1) sum = sum + __shfl_xor(sum, d, 64);   // commutative per level: every lane ends with the total
-  if (e < total && q == 0) {
-    const int i = (int)(e / N), j = (int)(e - (int64_t)i * N);
-    sc.put(i, j, act_apply(sc.pre(j, sum), act, alpha));
-  }
-}
-
 // ---- small-output GEMM: the K range is split across the wavefronts of one block ------
 // C(M x N) = A(M x K) B(K x N), both row-major, for products whose output has
 // too few 32x32 tiles to fill the chip when each tile walks all of K.  One
@@ -3425,22 +3395,9 @@ static ConvGeom conv_geom(const gh_cmd& c) {
   return g;
 }
 
-// Sum `splits` slabs of F x CKK partial filter gradients from the workspace into dw, in slab order.
+// Sum `splits` slabs of F x CKK partial filter gradients at ws into dw, in slab order.
 static int launch_slab_reduce(gh_ctx* ctx, const float* ws, int splits, int F, int CKK, float* dw) {
-  const int64_t total = (int64_t)F * CKK;
-  if (splits >= 64) {
-    hipLaunchKernelGGL((k_splitk_reduce_lanes<StoreRowMajor, 16>), dim3((int)cdiv(total * 16, 256)), dim3(256), 0,
-                       ctx->stream, ws, splits, F, CKK, StoreRowMajor{dw, CKK}, 0, 0.f);
-  } else if (splits >= 8) {
-    hipLaunchKernelGGL((k_splitk_reduce_lanes<StoreRowMajor, 4>), dim3((int)cdiv(total * 4, 256)), dim3(256), 0,
-                       ctx->stream, ws, splits, F, CKK, StoreRowMajor{dw, CKK}, 0, 0.f);
-  } else {
-    int64_t blocks = cdiv(total, 256);
-    if (blocks > (int64_t)ctx->cu_count * 8) blocks = (int64_t)ctx->cu_count * 8;
-    hipLaunchKernelGGL((k_splitk_reduce<StoreRowMajor>), dim3((int)blocks), dim3(256), 0, ctx->stream, ws, splits, F,
-                       CKK, StoreRowMajor{dw, CKK}, 0, 0.f);
-  }
-  return gh_check_hip(ctx, hipGetLastError(), "split-K reduce launch");
+  return gh_sum_slabs(ctx, {ws, dw, (int64_t)F * CKK, splits, splits >= 64 ? kSumLanes16 : splits >= 8 ? kSumLanes4 : kSumPlain});
 }
 
 // The direct kernel's shapes that k_conv3x3_wgrad_c1 takes: one channel, a padded image of at most 60 KB, at least
@@ -3472,7 +3429,6 @@ int gh_launch_conv2d_bwd_filter(gh_ctx* ctx, const gh_cmd& c) {
       if ((int64_t)G * F * CKK * 4 > ctx->workspace_bytes)
         return gh_fail(ctx, GH_ESTATE, "conv2d filter gradient: partial sums do not fit the workspace");
     }
-    float* wsd = (float*)ctx->workspace;
     const float* xd = (const float*)(uintptr_t)c.ptr[0];
     const float* dyd = (const float*)(uintptr_t)c.ptr[1];
     const size_t img_bytes = (size_t)(g.H + 2 * g.padH) * (g.W + 2 * g.padH) * 4;
@@ -3491,17 +3447,17 @@ int gh_launch_conv2d_bwd_filter(gh_ctx* ctx, const gh_cmd& c) {
       // exact while i * d < 2^32: ceil(2^32 / d)
       auto magic = [](int d) { return (unsigned)((0x100000000ull + (unsigned)d - 1) / (unsigned)d); };
       const int PW = g.W + 2 * g.padH;
+      float* const wsd = (float*)gh_slab_space(ctx, (int64_t)G1 * F * CKK * 4);
       hipLaunchKernelGGL(k_conv3x3_wgrad_c1, dim3((unsigned)G1, (unsigned)fby), dim3(256), img_bytes, ctx->stream, xd, dyd,
                          wsd, B, g.H, g.W, F, g.padH, g.oh, g.ow, magic(g.ow), magic(PW));
       int rc1 = gh_check_hip(ctx, hipGetLastError(), "single-channel filter-gradient launch");
       if (rc1) return rc1;
-      hipLaunchKernelGGL((k_splitk_reduce_lanes<StoreRowMajor, 4>), dim3((int)cdiv((int64_t)F * CKK * 4, 256)), dim3(256),
-                         0, ctx->stream, wsd, G1, F, CKK, StoreRowMajor{(float*)(uintptr_t)c.ptr[2], CKK}, 0, 0.f);
-      return gh_check_hip(ctx, hipGetLastError(), "split-K reduce launch");
+      return gh_sum_slabs(ctx, {wsd, (void*)(uintptr_t)c.ptr[2], (int64_t)F * CKK, G1, kSumLanes4});
     }
 #define GH_WGRAD_DIRECT(C_, FB_)                                                                             \
   hipLaunchKernelGGL((k_conv3x3_wgrad_direct<C_, FB_>), dim3((unsigned)G, (unsigned)cdiv(F, FB_)), dim3(256), 0, \
                      ctx->stream, xd, dyd, wsd, B, g.H, g.W, F, g.padH, g.oh, g.ow)
+    float* const wsd = (float*)gh_slab_space(ctx, (int64_t)G * F * CKK * 4);
     // two filters per workgroup pay for one channel (28x28, 32 filters, 128 images: 15.8 us
     // against 17.4); four filters, or more channels, spend the gain on the longer fold
     switch (g.C) {
@@ -3513,16 +3469,15 @@ int gh_launch_conv2d_bwd_filter(gh_ctx* ctx, const gh_cmd& c) {
 #undef GH_WGRAD_DIRECT
     int rc = gh_check_hip(ctx, hipGetLastError(), "direct filter-gradient launch");
     if (rc) return rc;
-    hipLaunchKernelGGL((k_splitk_reduce_lanes<StoreRowMajor, 4>), dim3((int)cdiv((int64_t)F * CKK * 4, 256)), dim3(256),
-                       0, ctx->stream, wsd, G, F, CKK, StoreRowMajor{(float*)(uintptr_t)c.ptr[2], CKK}, 0, 0.f);
-    return gh_check_hip(ctx, hipGetLastError(), "split-K reduce launch");
+    return gh_sum_slabs(ctx, {wsd, (void*)(uintptr_t)c.ptr[2], (int64_t)F * CKK, G, kSumLanes4});
   }
   {
     // small images: the kernel that keeps dy and x of a few images in LDS; slabs summed as below
     int sp = 0;
-    const int rcs = gh_try_launch_conv_wgrad_small(ctx, c, &sp);
+    float* slabs = nullptr;
+    const int rcs = gh_try_launch_conv_wgrad_small(ctx, c, &sp, &slabs);
     if (rcs > 0 || (rcs == 0 && sp <= 1)) return rcs;
-    if (rcs == 0) return launch_slab_reduce(ctx, (const float*)ctx->workspace, sp, F, CKK, (float*)(uintptr_t)c.ptr[2]);
+    if (rcs == 0) return launch_slab_reduce(ctx, slabs, sp, F, CKK, (float*)(uintptr_t)c.ptr[2]);
   }
   constexpr int BM = 64, BN = 64, BK = 32;
   const int64_t tiles = cdiv(F, BM) * cdiv(CKK, BN);
@@ -3540,7 +3495,7 @@ int gh_launch_conv2d_bwd_filter(gh_ctx* ctx, const gh_cmd& c) {
   const float* x = (const float*)(uintptr_t)c.ptr[0];
   const float* dy = (const float*)(uintptr_t)c.ptr[1];
   float* dw = (float*)(uintptr_t)c.ptr[2];
-  float* ws = (float*)ctx->workspace;
+  float* ws = splits > 1 ? (float*)gh_slab_space(ctx, splits * slab) : nullptr;
   const dim3 grid((unsigned)cdiv(CKK, BN), (unsigned)cdiv(F, BM), (unsigned)splits);
   hipLaunchKernelGGL((k_conv2d_wgrad<BM, BN, BK, 2>), grid, dim3(kThreads), 0, ctx->stream, x, dy, dw, g, F,
                      CKK, (int)splits, ws);

@@ -1,0 +1,207 @@
+// Sums of filter-gradient slabs, several gradients in one launch.
+//
+// A filter gradient's long axis is cut among workgroups, whose slabs of partial results a second launch adds up: some 5 us
+// each, of which the additions take one or two.  A training step has one for each layer, and nobody reads a gradient before
+// the solver.  So the sums are put off while the commands behind the gradient, of the kinds that stand between the layers of
+// a backward pass, neither read nor write its result: the slabs lie in a part of the workspace that no other plan reaches,
+// and the next command of another kind, one that touches a result, or the end of the submission has them added in one launch.
+// us of a training step, a launch for each sum / one: the convnet at batch 128 in float32 229 / 224, the four-block network at
+// batch 8 431 / 425.
+#include <algorithm>
+
+#include "gh_internal.h"
+
+namespace {
+
+struct Batch {
+  const void* ws[kSlabSums];
+  void* out[kSlabSums];
+  int64_t total[kSlabSums];
+  int slabs[kSlabSums], how[kSlabSums], first[kSlabSums + 1];
+};
+
+// RW results to a workgroup; its 256 / RW thread groups take every G-th slab (reads of a slab are RW values wide), and the
+// groups' sums are added pairwise, neighbours first.
+template <class T, int RW>
+__device__ __forceinline__ void by_groups(const T* __restrict__ ws, int slabs, int64_t total, T* __restrict__ out, int block, T* sh) {
+  constexpr int G = 256 / RW;
+  const int grp = threadIdx.x / RW;
+  const int64_t e = (int64_t)block * RW + threadIdx.x % RW;
+  T sum = (T)0;
+  if (e < total) {
+    int s = grp;
+    for (; s + 3 * G < slabs; s += 4 * G) {   // four loads in flight
+      T v[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) v[u] = ws[(int64_t)(s + u * G) * total + e];
+#pragma unroll
+      for (int u = 0; u < 4; u++) sum = sum + v[u];
+    }
+    for (; s < slabs; s += G) sum = sum + ws[(int64_t)s * total + e];
+  }
+  sh[threadIdx.x] = sum;
+  for (int d = 1; d < G; d <<= 1) {
+    __syncthreads();
+    T v = (T)0;
+    const bool mine = grp % (2 * d) == 0;
+    if (mine) v = sh[threadIdx.x] + sh[threadIdx.x + d * RW];
+    __syncthreads();
+    if (mine) sh[threadIdx.x] = v;
+  }
+  if (grp == 0 && e < total) out[e] = sh[threadIdx.x];
+}
+
+// Many slabs, few results: L lanes share one result.  Lane q adds slabs q, q + L, q + 2 L, ... in that order, then the L
+// sums are combined pairwise, neighbours first.
+template <int L>
+__device__ __forceinline__ void by_lanes(const float* __restrict__ ws, int slabs, int64_t total, float* __restrict__ out, int block) {
+  const int q = threadIdx.x & (L - 1);
+  const int64_t e = ((int64_t)block * 256 + threadIdx.x) / L;
+  float acc = 0.f;
+  if (e < total) {
+    const float* p = ws + (int64_t)q * total + e;
+    int s = q;
+    for (; s + 3 * L < slabs; s += 4 * L) {   // four loads in flight
+      const float v0 = p[0], v1 = p[(int64_t)L * total], v2 = p[2 * (int64_t)L * total], v3 = p[3 * (int64_t)L * total];
+      acc = acc + v0; acc = acc + v1; acc = acc + v2; acc = acc + v3;
+      p += 4 * (int64_t)L * total;
+    }
+    for (; s < slabs; s += L) { acc = acc + p[0]; p += (int64_t)L * total; }
+  }
+  float sum = acc;
+#pragma unroll
+  for (int d = 1; d < L; d <<= 1) sum = sum + __shfl_xor(sum, d, 64);   // commutative per level: every lane ends with the total
+  if (e < total && q == 0) out[e] = sum;
+}
+
+__global__ __launch_bounds__(256) void k_slab_sums(const Batch b) {
+  __shared__ double sh[256];
+  int t = 0;
+#pragma unroll
+  for (int q = 1; q < kSlabSums; q++)
+    if ((int)blockIdx.x >= b.first[q]) t = q;
+  const int block = blockIdx.x - b.first[t], slabs = b.slabs[t];
+  const int64_t total = b.total[t];
+  const float* const ws = (const float*)b.ws[t];
+  float* const out = (float*)b.out[t];
+  switch (b.how[t]) {
+    case kSumGroups64: by_groups<float, 64>(ws, slabs, total, out, block, (float*)sh); break;
+    case kSumGroups16: by_groups<float, 16>(ws, slabs, total, out, block, (float*)sh); break;
+    case kSumGroups64F64: by_groups<double, 64>((const double*)ws, slabs, total, (double*)out, block, sh); break;
+    case kSumGroups16F64: by_groups<double, 16>((const double*)ws, slabs, total, (double*)out, block, sh); break;
+    case kSumLanes16: by_lanes<16>(ws, slabs, total, out, block); break;
+    case kSumLanes4: by_lanes<4>(ws, slabs, total, out, block); break;
+    default: {
+      const int64_t e = (int64_t)block * 256 + threadIdx.x;
+      if (e >= total) break;
+      float acc = ws[e];
+      for (int s = 1; s < slabs; s++) acc = acc + ws[(int64_t)s * total + e];
+      out[e] = acc;
+    }
+  }
+}
+
+int results_of_block(int how) {
+  switch (how) {
+    case kSumGroups64: case kSumGroups64F64: case kSumLanes4: return 64;
+    case kSumGroups16: case kSumGroups16F64: case kSumLanes16: return 16;
+    default: return 256;
+  }
+}
+
+int64_t item(int how) { return how == kSumGroups64F64 || how == kSumGroups16F64 ? 8 : 4; }
+
+int launch(gh_ctx* ctx, const gh_slab_sum* sums, int n) {
+  Batch b{};
+  int blocks = 0;
+  for (int i = 0; i < n; i++) {
+    b.ws[i] = sums[i].ws;
+    b.out[i] = sums[i].out;
+    b.total[i] = sums[i].total;
+    b.slabs[i] = sums[i].slabs;
+    b.how[i] = sums[i].how;
+    b.first[i] = blocks;
+    const int r = results_of_block(sums[i].how);
+    blocks += (int)((sums[i].total + r - 1) / r);
+  }
+  for (int i = n; i <= kSlabSums; i++) b.first[i] = blocks;
+  hipLaunchKernelGGL(k_slab_sums, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, b);
+  return gh_check_hip(ctx, hipGetLastError(), "slab sum launch");
+}
+
+struct Range {
+  uint64_t from, to;
+};
+
+// What a command of a backward pass reads and writes; 0 for other commands.
+int ranges_of(const gh_cmd& c, Range (&r)[8]) {
+  const int64_t size = gh_dtype_of(c.flags) == GH_F64 ? 8 : 4;
+  int n = 0;
+  auto add = [&](int slot, int64_t values) { r[n++] = {c.ptr[slot], c.ptr[slot] + (uint64_t)(values * size)}; };
+  const int64_t B = c.dim[0], C = c.dim[1];
+  switch (c.opcode) {
+    case GH_OP_CONV2D_BWD_DATA: case GH_OP_CONV2D_BWD_FILTER: {
+      const int64_t x = B * C * c.dim[2] * c.dim[3], w = c.dim[4] * C * c.dim[5] * c.dim[6];
+      const int64_t dy = B * c.dim[4] * gh_conv_out(c.dim[2], c.dim[5], c.dim[7], c.dim[9], c.dim[11]) * gh_conv_out(c.dim[3], c.dim[6], c.dim[8], c.dim[10], c.dim[12]);
+      const bool data = c.opcode == GH_OP_CONV2D_BWD_DATA;   // dy, w, dx; else x, dy, dw
+      add(0, data ? dy : x);
+      add(1, data ? w : dy);
+      add(2, data ? x : w);
+      return n;
+    }
+    case GH_OP_MAXPOOL2D_BWD: {
+      const int64_t x = B * C * c.dim[2] * c.dim[3];
+      add(0, x);
+      add(1, B * C * gh_pool_out(c.dim[2], c.dim[4], c.dim[6], c.dim[7], c.dim[10]) * gh_pool_out(c.dim[3], c.dim[5], c.dim[8], c.dim[9], c.dim[11]));
+      add(2, x);
+      return n;
+    }
+    case GH_OP_BN_BWD:
+      for (int k = 0; k < 3; k++) add(k, B * C * c.dim[2]);
+      add(3, C);
+      add(4, C);
+      return n;
+    case GH_OP_RELU_BWD:
+      for (int k = 0; k < 3; k++) add(k, c.dim[0]);
+      return n;
+  }
+  return 0;
+}
+
+}  // namespace
+
+// Where a filter gradient puts its slabs: behind the workspace if its sum may be put off, else in the workspace.
+void* gh_slab_space(gh_ctx* ctx, int64_t bytes) {
+  if (!ctx->defer_sums || ctx->pending == kSlabSums || ctx->slabs_used + bytes > kSlabSpace) return ctx->workspace;
+  void* const p = (char*)ctx->slab_space + ctx->slabs_used;
+  ctx->slabs_used += (bytes + 255) / 256 * 256;
+  return p;
+}
+
+int gh_sum_slabs(gh_ctx* ctx, const gh_slab_sum& s) {
+  const char *p = (const char*)s.ws, *base = (const char*)ctx->slab_space;
+  if (!base || p < base || p >= base + kSlabSpace) return launch(ctx, &s, 1);
+  ctx->sums[ctx->pending++] = s;
+  return GH_OK;
+}
+
+int gh_flush_sums(gh_ctx* ctx) {
+  const int n = ctx->pending;
+  ctx->pending = 0;
+  ctx->slabs_used = 0;
+  return n ? launch(ctx, ctx->sums, n) : GH_OK;
+}
+
+// The sums that were put off, in front of a command that may have to do with their results.  (c is a valid command.)
+int gh_flush_sums_before(gh_ctx* ctx, const gh_cmd& c) {
+  if (!ctx->pending) return GH_OK;
+  Range r[8];
+  const int n = ranges_of(c, r);
+  bool meets = n == 0;
+  for (int i = 0; i < ctx->pending; i++) {
+    const gh_slab_sum& s = ctx->sums[i];
+    const uint64_t from = (uint64_t)(uintptr_t)s.out, to = from + (uint64_t)(s.total * item(s.how));
+    for (int k = 0; k < n; k++) meets = meets || (r[k].from < to && from < r[k].to);
+  }
+  return meets ? gh_flush_sums(ctx) : GH_OK;
+}
