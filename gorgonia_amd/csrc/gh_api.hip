@@ -506,13 +506,14 @@ static int submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
     // a run of solver steps with the same settings (a model's weight tensors) is one launch, and so is a run of
     // elementwise commands on tensors of one size
     const int solver = gh_solver_run_length(cmds + i, n - i);
-    const int run = solver > 1 ? solver : gh_chain_length(cmds + i, n - i);
+    const bool copy = solver && gh_solver_copy_rides(cmds + i, solver, n - i);
+    const int run = solver > 1 || copy ? solver + copy : gh_chain_length(cmds + i, n - i);
     if (run > 1) {
       for (int j = 1; j < run; j++) {
         rc = gh_validate_cmd(cmds[i + j], m);
         if (rc) return gh_fail(ctx, rc, "cmd " + std::to_string(i + j) + ": " + m);
       }
-      rc = solver > 1 ? gh_launch_solver_steps(ctx, cmds + i, run) : gh_launch_chain(ctx, cmds + i, run);
+      rc = solver ? gh_launch_solver_steps(ctx, cmds + i, solver, copy) : gh_launch_chain(ctx, cmds + i, run);
       if (rc) return rc;
       i += run - 1;
       continue;

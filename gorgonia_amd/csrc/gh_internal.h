@@ -141,7 +141,7 @@ int gh_launch_dropout_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_dropout_bwd_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_softmax_bwd_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_maxpool2d_bwd_f64(gh_ctx* ctx, const gh_cmd& c);
-int gh_launch_solver_steps_f64(gh_ctx* ctx, const gh_cmd* cmds, int count);
+int gh_launch_solver_steps_f64(gh_ctx* ctx, const gh_cmd* cmds, int count, bool copy);
 int gh_launch_bn_train_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_bn_bwd_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_conv2d_bwd_data_f64(gh_ctx* ctx, const gh_cmd& c);
@@ -210,7 +210,15 @@ int gh_launch_bn_bwd(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_softmax_bwd(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_solver_step(gh_ctx* ctx, const gh_cmd& c);
 int gh_solver_run_length(const gh_cmd* cmds, int n);
-int gh_launch_solver_steps(gh_ctx* ctx, const gh_cmd* cmds, int count);
+int gh_launch_solver_steps(gh_ctx* ctx, const gh_cmd* cmds, int count, bool copy);   // copy: cmds[count] rides along
+// whether the command behind a run of `count` solver steps is a small copy that has nothing to do with their tensors
+bool gh_solver_copy_rides(const gh_cmd* cmds, int count, int n);
+// a copy of words by the workgroups behind a launch's own
+struct gh_small_copy {
+  const uint32_t* src;
+  uint32_t* dst;
+  int words;
+};
 int gh_launch_rand_uniform(gh_ctx* ctx, const gh_cmd& c);
 // float64 twins of the forward neural-network operators (k_nn64.hip)
 int gh_launch_relu_f64(gh_ctx* ctx, const gh_cmd& c, bool leaky);

@@ -457,7 +457,12 @@ struct SolverBatch {
 
 template <int KIND>
 __global__ __launch_bounds__(kBlock) void k_solver_step(SolverBatch sb, int use, SolverPar p,
-                                                        const float* __restrict__ corr) {
+                                                        const float* __restrict__ corr, gh_small_copy copy) {
+  if ((int)blockIdx.x >= sb.first[kSolverBatch]) {
+    const int i = ((int)blockIdx.x - sb.first[kSolverBatch]) * kBlock + (int)threadIdx.x;
+    if (i < copy.words) copy.dst[i] = copy.src[i];
+    return;
+  }
   // Adam's two bias corrections from device memory when the command names it: they change
   // every step, and as command constants they would make every step a new command
   if (KIND == GH_SOLVER_ADAM && corr) { p.corr1 = corr[0]; p.corr2 = corr[1]; }
@@ -708,10 +713,28 @@ int gh_solver_run_length(const gh_cmd* cmds, int n) {
   return len;
 }
 
-// One launch for cmds[0..count) (count from gh_solver_run_length).
-int gh_launch_solver_steps(gh_ctx* ctx, const gh_cmd* cmds, int count) {
+// The network's result leaves the device behind the solver's steps: of up to 64 KB, by more workgroups of their launch (a
+// launch of its own some 3 us).
+bool gh_solver_copy_rides(const gh_cmd* cmds, int count, int n) {
+  if (count >= n || cmds[count].opcode != GH_OP_MEMCPY_D2D) return false;
+  const gh_cmd& c = cmds[count];
+  const int64_t bytes = c.dim[0];
+  if (bytes <= 0 || bytes > 65536 || ((c.ptr[0] | c.ptr[1] | (uint64_t)bytes) & 3) || !c.ptr[0] || !c.ptr[1]) return false;
+  auto meets = [&](uint64_t p, int64_t size, uint64_t q) { return q && q < p + (uint64_t)bytes && p < q + (uint64_t)size; };
+  if (meets(c.ptr[0], bytes, c.ptr[1])) return false;
+  for (int i = 0; i < count; i++) {
+    const int64_t size = cmds[i].dim[0] * (gh_dtype_of(cmds[i].flags) == GH_F64 ? 8 : 4);
+    for (int k = 0; k < 4; k++)
+      if (meets(c.ptr[0], size, cmds[i].ptr[k]) || (k != 1 && meets(c.ptr[1], size, cmds[i].ptr[k]))) return false;
+    if (meets(c.ptr[0], 16, cmds[i].ptr[4])) return false;   // the corrections
+  }
+  return true;
+}
+
+// One launch for cmds[0..count) (count from gh_solver_run_length), and for the copy behind them.
+int gh_launch_solver_steps(gh_ctx* ctx, const gh_cmd* cmds, int count, bool copy) {
   const gh_cmd& c = cmds[0];
-  if (gh_dtype_of(c.flags) == GH_F64) return gh_launch_solver_steps_f64(ctx, cmds, count);
+  if (gh_dtype_of(c.flags) == GH_F64) return gh_launch_solver_steps_f64(ctx, cmds, count, copy);
   const int kind = (int)gh_fn(c.flags), use = (int)gh_mode(c.flags);
   SolverPar p{c.f[0], c.f[1], c.f[2], c.f[3], c.f[4], c.f[5], c.f[6], c.f[7], c.f[8], c.f[9]};
   SolverBatch sb{};
@@ -730,22 +753,24 @@ int gh_launch_solver_steps(gh_ctx* ctx, const gh_cmd* cmds, int count) {
     blocks_total += (int)blocks;
     nt++;
   }
-  if (nt == 0) return GH_OK;
+  if (nt == 0 && !copy) return GH_OK;
   for (int i = nt; i <= kSolverBatch; i++) sb.first[i] = blocks_total;
   sb.count = nt;
-  const dim3 grid(blocks_total), block(kBlock);
+  gh_small_copy tail{};
+  if (copy) tail = {(const uint32_t*)(uintptr_t)cmds[count].ptr[1], (uint32_t*)(uintptr_t)cmds[count].ptr[0], (int)(cmds[count].dim[0] / 4)};
+  const dim3 grid(blocks_total + (tail.words + kBlock - 1) / kBlock), block(kBlock);
   const float* corr = (const float*)(uintptr_t)c.ptr[4];
   if (kind == GH_SOLVER_VANILLA)
-    hipLaunchKernelGGL((k_solver_step<GH_SOLVER_VANILLA>), grid, block, 0, ctx->stream, sb, use, p, corr);
+    hipLaunchKernelGGL((k_solver_step<GH_SOLVER_VANILLA>), grid, block, 0, ctx->stream, sb, use, p, corr, tail);
   else if (kind == GH_SOLVER_RMSPROP)
-    hipLaunchKernelGGL((k_solver_step<GH_SOLVER_RMSPROP>), grid, block, 0, ctx->stream, sb, use, p, corr);
+    hipLaunchKernelGGL((k_solver_step<GH_SOLVER_RMSPROP>), grid, block, 0, ctx->stream, sb, use, p, corr, tail);
   else
-    hipLaunchKernelGGL((k_solver_step<GH_SOLVER_ADAM>), grid, block, 0, ctx->stream, sb, use, p, corr);
+    hipLaunchKernelGGL((k_solver_step<GH_SOLVER_ADAM>), grid, block, 0, ctx->stream, sb, use, p, corr, tail);
   return gh_check_hip(ctx, hipGetLastError(), "solver step launch");
 }
 
 int gh_launch_solver_step(gh_ctx* ctx, const gh_cmd& c) {
-  return gh_launch_solver_steps(ctx, &c, 1);
+  return gh_launch_solver_steps(ctx, &c, 1, false);
 }
 
 static int stream_blocks(gh_ctx* ctx, int64_t n) {

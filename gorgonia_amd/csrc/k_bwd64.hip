@@ -282,7 +282,12 @@ struct SolverBatch64 {
 };
 
 template <int KIND>
-__global__ __launch_bounds__(kBlock) void k_solver_step_f64(SolverBatch64 sb, int use, SolverPar64 p, const double* __restrict__ corr) {
+__global__ __launch_bounds__(kBlock) void k_solver_step_f64(SolverBatch64 sb, int use, SolverPar64 p, const double* __restrict__ corr, gh_small_copy copy) {
+  if ((int)blockIdx.x >= sb.first[kSolverBatch64]) {
+    const int i = ((int)blockIdx.x - sb.first[kSolverBatch64]) * kBlock + (int)threadIdx.x;
+    if (i < copy.words) copy.dst[i] = copy.src[i];
+    return;
+  }
   if (KIND == GH_SOLVER_ADAM && corr) { p.corr1 = corr[0]; p.corr2 = corr[1]; }   // see k_solver_step
   int t = 0;
 #pragma unroll
@@ -425,8 +430,8 @@ int gh_launch_bn_bwd_f64(gh_ctx* ctx, const gh_cmd& c) {
   return gh_check_hip(ctx, hipGetLastError(), "batchnorm backward launch");
 }
 
-// One launch for cmds[0..count) (count from gh_solver_run_length).
-int gh_launch_solver_steps_f64(gh_ctx* ctx, const gh_cmd* cmds, int count) {
+// One launch for cmds[0..count) (count from gh_solver_run_length), and for the copy behind them.
+int gh_launch_solver_steps_f64(gh_ctx* ctx, const gh_cmd* cmds, int count, bool copy) {
   const gh_cmd& c = cmds[0];
   const int kind = (int)gh_fn(c.flags), use = (int)gh_mode(c.flags);
   SolverPar64 p{bits_to_double(c.dim[1]), bits_to_double(c.dim[2]), bits_to_double(c.dim[3]),
@@ -447,16 +452,18 @@ int gh_launch_solver_steps_f64(gh_ctx* ctx, const gh_cmd* cmds, int count) {
     blocks += blocks_for(ctx, n);
     nt++;
   }
-  if (nt == 0) return GH_OK;
+  if (nt == 0 && !copy) return GH_OK;
   for (int i = nt; i <= kSolverBatch64; i++) sb.first[i] = blocks;
   sb.count = nt;
-  const dim3 grid((unsigned)blocks), block(kBlock);
+  gh_small_copy tail{};
+  if (copy) tail = {(const uint32_t*)(uintptr_t)cmds[count].ptr[1], (uint32_t*)(uintptr_t)cmds[count].ptr[0], (int)(cmds[count].dim[0] / 4)};
+  const dim3 grid((unsigned)(blocks + (tail.words + kBlock - 1) / kBlock)), block(kBlock);
   const double* corr = (const double*)(uintptr_t)c.ptr[4];
   if (kind == GH_SOLVER_VANILLA)
-    hipLaunchKernelGGL((k_solver_step_f64<GH_SOLVER_VANILLA>), grid, block, 0, ctx->stream, sb, use, p, corr);
+    hipLaunchKernelGGL((k_solver_step_f64<GH_SOLVER_VANILLA>), grid, block, 0, ctx->stream, sb, use, p, corr, tail);
   else if (kind == GH_SOLVER_RMSPROP)
-    hipLaunchKernelGGL((k_solver_step_f64<GH_SOLVER_RMSPROP>), grid, block, 0, ctx->stream, sb, use, p, corr);
+    hipLaunchKernelGGL((k_solver_step_f64<GH_SOLVER_RMSPROP>), grid, block, 0, ctx->stream, sb, use, p, corr, tail);
   else
-    hipLaunchKernelGGL((k_solver_step_f64<GH_SOLVER_ADAM>), grid, block, 0, ctx->stream, sb, use, p, corr);
+    hipLaunchKernelGGL((k_solver_step_f64<GH_SOLVER_ADAM>), grid, block, 0, ctx->stream, sb, use, p, corr, tail);
   return gh_check_hip(ctx, hipGetLastError(), "solver step launch");
 }
