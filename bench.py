@@ -235,6 +235,7 @@ def bench_linalg(ctx, iters):
         fl = 2.0 * m * n * k * batch
         res[name] = {"us": round(ms * 1e3, 1), "TFLOPs": round(fl / ms / 1e9, 2),
                      "frac_mfma": round(fl / ms / 1e9 / MFMA_F32_PEAK_TFLOPS, 4), "flop": fl,
+                     "matrix_instructions": "bf16, each float32 value in three parts" if ctx.lib.gh_runs_split(C.byref(cmd)) else "float32",
                      "us_short_burst": round(time_cmds.last_burst_ms * 1e3, 1)}
         for q in (A, B, Cm):
             ctx.free(q)
