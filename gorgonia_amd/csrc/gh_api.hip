@@ -125,6 +125,7 @@ static void drop_ctx(gh_ctx* ctx) {
   give_word(ctx->done_word);   // nothing is in flight any more
   give_page(ctx);
   if (ctx->workspace) hipFree(ctx->workspace);
+  if (ctx->slab_space) hipFree(ctx->slab_space);
   if (ctx->arena) hipFree(ctx->arena);
   hipStreamDestroy(ctx->stream);
   delete ctx;
@@ -181,13 +182,12 @@ int gh_init(int device, int64_t arena_bytes, gh_ctx** out) {
   // filters.  Mandatory: the launchers index it without asking again.
   ctx->workspace_bytes = 64ll << 20;
   void* fixed = nullptr;
-  if (hipMalloc(&ctx->workspace, (size_t)(ctx->workspace_bytes + kSlabSpace)) != hipSuccess ||
+  if (hipMalloc(&ctx->workspace, (size_t)ctx->workspace_bytes) != hipSuccess ||
       static_scratch(device, &fixed) != hipSuccess) {
     (void)hipGetLastError();
     drop_ctx(ctx);
     return GH_EOOM;
   }
-  ctx->slab_space = (char*)ctx->workspace + ctx->workspace_bytes;
   ctx->bn_page = take_page(device);
   *out = ctx;
   return GH_OK;
@@ -528,9 +528,27 @@ static int submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
   return GH_OK;
 }
 
+// The memory for slabs whose sums wait: made for the first submission of several commands with a filter gradient among them
+// (none while a graph is captured: the sums are then launched where they stand).
+static bool slab_space(gh_ctx* ctx, const gh_cmd* cmds, int n) {
+  if (ctx->slab_space || ctx->no_slab_space || ctx->capturing) return ctx->slab_space;
+  bool any = false;
+  for (int i = 0; i < n; i++) any = any || cmds[i].opcode == GH_OP_CONV2D_BWD_FILTER;
+  if (!any) return false;
+  int before = ctx->device;
+  (void)hipGetDevice(&before);
+  if (hipSetDevice(ctx->device) != hipSuccess || hipMalloc(&ctx->slab_space, (size_t)kSlabSpace) != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->slab_space = nullptr;
+    ctx->no_slab_space = true;
+  }
+  (void)hipSetDevice(before);
+  return ctx->slab_space;
+}
+
 // Sums of filter-gradient slabs may wait for the commands behind them (k_slab_sums.hip); none waits past the submission.
 static int submit_cmds(gh_ctx* ctx, const gh_cmd* cmds, int n) {
-  ctx->defer_sums = n > 1 && !ctx->ws_strict;
+  ctx->defer_sums = n > 1 && !ctx->ws_strict && slab_space(ctx, cmds, n);
   const int rc = submit_each(ctx, cmds, n);
   ctx->defer_sums = false;
   const int late = gh_flush_sums(ctx);

@@ -57,7 +57,7 @@ struct gh_slab_sum {
   int slabs, how;
 };
 constexpr int kSlabSums = 8;
-constexpr int64_t kSlabSpace = 16ll << 20;   // (the larger allocation makes opening a context some 10 us slower)
+constexpr int64_t kSlabSpace = 24ll << 20;
 
 struct gh_ctx {
   int device = 0;
@@ -76,8 +76,9 @@ struct gh_ctx {
   // what the workgroups of k_bn_held.hip pass to each other: two slots of 8 bytes and one count of 4 for each of
   // kBnHeldSlots, zero whenever no kernel runs; null where the device's pages were all taken
   void* bn_page = nullptr;
-  // slabs whose sums gh_submit has put off, behind the workspace (no other plan reaches them), and those sums
+  // slabs whose sums gh_submit has put off, in memory of their own (kSlabSpace, or null so far), and those sums
   void* slab_space = nullptr;
+  bool no_slab_space = false;   // there was none to be had
   int64_t slabs_used = 0;
   gh_slab_sum sums[kSlabSums];
   int pending = 0;

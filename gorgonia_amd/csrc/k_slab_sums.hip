@@ -5,8 +5,8 @@
 // the solver.  So the sums are put off while the commands behind the gradient, of the kinds that stand between the layers of
 // a backward pass, neither read nor write its result: the slabs lie in a part of the workspace that no other plan reaches,
 // and the next command of another kind, one that touches a result, or the end of the submission has them added in one launch.
-// us of a training step, a launch for each sum / one: the convnet at batch 128 in float32 229 / 224, the four-block network at
-// batch 8 431 / 425.
+// us of a training step, a launch for each sum / one: the convnet at batch 128 in float32 229 / 222, the four-block network at
+// batch 8 431 / 424.
 #include <algorithm>
 
 #include "gh_internal.h"
@@ -170,7 +170,7 @@ int ranges_of(const gh_cmd& c, Range (&r)[8]) {
 
 }  // namespace
 
-// Where a filter gradient puts its slabs: behind the workspace if its sum may be put off, else in the workspace.
+// Where a filter gradient puts its slabs: in memory of its own if its sum may be put off, else in the workspace.
 void* gh_slab_space(gh_ctx* ctx, int64_t bytes) {
   if (!ctx->defer_sums || ctx->pending == kSlabSums || ctx->slabs_used + bytes > kSlabSpace) return ctx->workspace;
   void* const p = (char*)ctx->slab_space + ctx->slabs_used;
