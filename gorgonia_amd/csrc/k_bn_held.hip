@@ -10,7 +10,7 @@
 // them up itself, in the same order, to the same bits.  Nothing depends on all workgroups being on the chip at once.
 //
 // Bound: HBM and the caches for large planes, the launch and the waits (some 1.5 us each) for small ones.  us, four launches
-// or three / one, forward and gradient: 8 x 16 x 208 x 208 30.9 / 18.7 and 33.8 / 21.1 (5.2 TB/s of the 110 MB that the
+// or three / one, forward and gradient: 8 x 16 x 208 x 208 30.9 / 18.7 and 33.8 / 21.1 (4.4 TB/s of the 94 MB that the
 // gradient moves), 8 x 32 x 104 x 104 20.5 / 11.8 and 22.9 / 12.3, 8 x 128 x 26 x 26 14.2 / 8.9 and 13.4 / 7.0,
 // 8 x 16 x 207 x 207 (single loads) 46.6 / 20.8 and 47.3 / 25.8, 2 x 3 x 4 x 4 12.1 / 7.5 and 10.0 / 4.9.  (The forward as the
 // gradient is, its values kept as the pooling's windows lie: 14.8, 9.9 and 7.3, and other sums.)
