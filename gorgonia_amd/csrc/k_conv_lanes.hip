@@ -362,7 +362,13 @@ bool fill(const gh_cmd& c, bool flip, bool pool, Lanes<T>* g) {
 // the estimates are mostly within 15 % of the times.
 struct Form { int tm, v, waves, groups; bool split; double per_tile, per_quad; };
 static const Form kForms32[] = {{1, 4, 8, 1, true, 1.9, 0.160}, {2, 4, 8, 1, true, 3.2, 0.263}, {2, 4, 4, 1, true, 2.4, 0.24}, {2, 4, 4, 1, false, 2.6, 1.05}, {1, 4, 4, 1, false, 1.8, 0.52}};
-static const Form kForms64[] = {{1, 2, 4, 1, true, 0.8, 0.17}, {2, 2, 4, 2, true, 3.4, 0.47}, {2, 2, 4, 2, false, 4.0, 2.2}};
+// float64, where a forward pass's fragments of a quad come from rows C filters apart: its small forms take longer than a
+// gradient's.  The last is one filter tile by two groups, between the first two in loads for a product, with their sums in
+// their order: us, without it / with, 50 x 32 x 14 x 14 -> 64 16.4 / 14.3; 20 x 64 x 7 x 7 -> 128 10.8 / 9.0; 96 x 64 x 7 x 7 ->
+// 128 29.5 / 22.2; 8 x 64 x 26 x 26 -> 128 29.1 / 22.0 (36 TFLOP/s); 64 x 32 x 14 x 14 -> 64, a little past
+// three rounds of it, 16.6 in the second and 18.8 in it.  A gradient gains nothing from it.
+static const Form kForward64[] = {{1, 2, 4, 1, true, 0.7, 0.20}, {2, 2, 4, 2, true, 3.4, 0.47}, {2, 2, 4, 2, false, 4.0, 2.2}, {1, 2, 4, 2, true, 1.15, 0.32}};
+static const Form kGradient64[] = {{1, 2, 4, 1, true, 0.8, 0.17}, {2, 2, 4, 2, true, 3.4, 0.47}, {2, 2, 4, 2, false, 4.0, 2.2}};
 
 // The quickest of the forms from..to - 1 and its time: a function of the plain command (a pooled one takes the same form
 // and so sums in the same order).
@@ -371,7 +377,7 @@ static int quickest(const gh_cmd& c, bool flip, bool f64, int cus, int from, int
   const int64_t K = flip ? c.dim[4] : c.dim[1], F = flip ? c.dim[1] : c.dim[4], lines = B * (flip ? c.dim[2] : oh);
   int best = -1;
   for (int i = from; i < to; i++) {
-    const Form& f = (f64 ? kForms64 : kForms32)[i];
+    const Form& f = (!f64 ? kForms32 : flip ? kGradient64 : kForward64)[i];
     // an image gradient gains nothing from the form that halves the wavefronts (8 x 32 x 52 x 52 <- 64: 14.5 us, 14.0 with
     // eight), and would add twice as many terms in a row
     if (!f64 && flip && f.split && f.waves == 4) continue;
@@ -402,7 +408,7 @@ int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, boo
   Lanes<double> g;   // (the narrower of the two in what its offsets reach)
   if (!fill(c, flip, false, &g) || g.F < 8 || g.C < 8 || g.oh < 2) return -1;
   double us;
-  const int split = quickest(c, flip, f64, cus, 0, 3, &us);
+  const int split = quickest(c, flip, f64, cus, 0, f64 && !flip ? 4 : 3, &us);
   if (other_us <= 0 || us < other_us / 1.17) return split;
   if (f64 || patch) return -1;
   const int whole = quickest(c, flip, false, cus, 3, 5, &us);
@@ -418,6 +424,7 @@ int gh_launch_conv_lanes(gh_ctx* ctx, const gh_cmd& c, bool flip, int form) {
     switch (form) {
       case 0: return launch<double, 4, 1, 2, 1, true>(ctx, g, t, flip, false);
       case 1: return launch<double, 4, 2, 2, 2, true>(ctx, g, t, flip, false);
+      case 3: return launch<double, 4, 1, 2, 2, true>(ctx, g, t, flip, false);   // (forward)
       default: return launch<double, 4, 2, 2, 2, false>(ctx, g, t, flip, false);
     }
   }
