@@ -512,6 +512,7 @@ static int submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
       for (int j = 1; j < run; j++) {
         rc = gh_validate_cmd(cmds[i + j], m);
         if (rc) return gh_fail(ctx, rc, "cmd " + std::to_string(i + j) + ": " + m);
+        if ((rc = gh_flush_sums_before(ctx, cmds[i + j]))) return rc;
       }
       rc = solver ? gh_launch_solver_steps(ctx, cmds + i, solver, copy) : gh_launch_chain(ctx, cmds + i, run);
       if (rc) return rc;

@@ -92,6 +92,27 @@ def test_a_result_that_the_next_command_reads_or_writes(ctx):
         _same(ctx, build)
 
 
+@pytest.mark.parametrize("code,np_dt", [(_ffi.F32, np.float32), (_ffi.F64, np.float64)])
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("member", [1, 2])
+def test_a_result_inside_a_run_of_elementwise_commands(ctx, code, np_dt, in_place, member):
+    """The run's first command has nothing to do with the result; its second or third reads it, or writes over it."""
+    layer = (64, 32, 14, 14, 64)
+    n = 64 * 32 * 9
+    counts = []
+
+    def build(t):
+        g = _gradient(t, layer, code)
+        run = [D.cmd_relu_bwd(t.make(n), t.make(n), t.make(n), n, dtype=code)]
+        if member == 2:
+            run.append(D.cmd_relu(t.make(n), t.make(n), n, dtype=code))
+        run.append(D.cmd_relu(g.ptr[2], g.ptr[2] if in_place else t.make(n), n, dtype=code))
+        counts.append(_ffi.load().gh_elementwise_run((_ffi.GhCmd * len(run))(*run), len(run)))
+        return [g] + run
+    _same(ctx, build, np_dt)
+    assert counts[0] == member + 1   # one run
+
+
 def test_replays(ctx):
     layer = (8, 16, 52, 52, 32)
     t = _Tensors(ctx, np.float32)
