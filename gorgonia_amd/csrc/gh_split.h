@@ -1,11 +1,13 @@
 // float32 contractions on the bf16 matrix instructions.
 //
 // A float32 has 24 significant bits, a bf16 eight and the same exponents: x = h + m + l with three bf16 numbers, exactly
-// (h is x rounded to nearest, m what is left rounded to nearest, l the rest).  Of the nine products of two such sums six are
-// added up, a.h b.h, a.h b.m, a.m b.h, a.m b.m, a.h b.l and a.l b.h; each is exact in the multiplier.  The other three are
-// at most 2^-25 of the product (a.m <= 2^-8 a, b.l <= 2^-17 b), half of what rounding the product to float32 may cost.
-// The sums are float32, as on the float32 instructions, rounded to nearest once per instruction.  Six
-// instructions of 16 k take 98 ns on a SIMD where the eight float32 ones of 2 k take 217.
+// (h is x rounded to nearest, m what is left rounded to nearest, l the rest).  Of the nine products of two such sums all but
+// a.l b.l are added up, each exact in the multiplier; that one is at most 2^-34 of the product (|m| <= 2^-8 |x|, |l| <= 2^-17 |x|).
+// (Without a.m b.l and a.l b.m as well, 2^-25 of the product each, a result of one product was off by up to 0.96 of its last
+// place.)  The sums are float32, as on the float32 instructions, rounded once per instruction.  The seven products behind
+// a.h b.h, at most 2^-7 of it together, have sums of their own: the large sum is rounded once per 16 k, and a result of one
+// product (a diagonal, a scaling, a sparse row) is off by at most 0.51 of its last place, 0.5 on the float32 instructions.
+// Eight instructions of 16 k take 130 ns on a SIMD where the eight float32 ones of 2 k take 217.
 //
 // Range: the inputs are scaled by 2^16, so that every bit of the smallest denormal stays inside bf16's (denormal) range
 // and the split is exact for all inputs below 2^112; results are scaled back.  Larger, infinite and NaN inputs, and

@@ -1,19 +1,20 @@
-// Large float32 products on the bf16 matrix instructions (gh_split.h): six of their instructions do the work of eight
-// float32 ones that take twice the time.
+// Large float32 products on the bf16 matrix instructions (gh_split.h): eight of their instructions do the work of eight
+// float32 ones that take nearly twice the time.
 //
 // A workgroup owns a tile of the result; the operands' values are split into their bf16 parts on the way from memory to
-// LDS, once per workgroup that needs them.  That is what the tile's size buys: at 256 x 256 a lane converts 16 values
-// (104 vector instructions) for 48 matrix instructions, at 64 x 64 for 12.  A wavefront issues a vector instruction every
+// LDS, once per workgroup that needs them.  That is what the tile's size buys: at 128 x 128 a lane converts 16 values
+// (104 vector instructions) for 32 matrix instructions, at 64 x 64 for 16.  A wavefront issues a vector instruction every
 // five cycles under its matrix instructions, if it does not wait for the one before: the stages of several pairs of values
-// are interleaved, one to a matrix instruction (in a row, pair by pair: 622 us for 4096 x 4096 x 4096, 108 for 2048).
+// are interleaved, one to a matrix instruction.  (256 x 256 has no registers for the two sums of a result; 256 x 128 with
+// one wavefront to a SIMD takes 1023 us for 4096 x 4096 x 4096, 128 x 128 843.)
 // Smaller products have too few such tiles for the compute units: theirs are smaller, and K is cut into parts inside the
 // workgroup, each with wavefronts and LDS buffers of its own, whose sums are added in LDS at the end.  Which form runs
 // depends on the shape only.
 //
-// Error against 64-bit sums, next to the float32 kernels': 4096 x 4096 x 4096 normal values 1.00e-6 (1.15e-6), uniform
-// ones 5.3e-7 (8.4e-7).  All forms but the 256 x 256 one, which has no registers for it, sum the five smaller products
-// apart from the first, so that the large sum is rounded once per 16 k: 2048 x 2048 x 2048 1.9e-7 (8.1e-7), 576 x 2549 x 1991
-// 1.9e-7 (4.0e-7 on k_gemm_direct, which cuts K four ways); with one sum it was 4.9e-7.
+// Error against 64-bit sums, of normal / of uniform values in [0, 1), next to the float32 kernel that the shape would run
+// on: 4096 x 4096 x 4096 4.0e-7 / 3.0e-7 (k_sgemm 1.14e-6 / 8.4e-7); 2321 x 3480, K = 2049 1.9e-7 / 1.2e-7 (k_gemm_direct in
+// four slices 4.1e-7 / 1.6e-7); 1000 x 1000, K = 4000 1.9e-7 / 8.3e-8 (in eight 4.0e-7 / 1.1e-7).  One, two and sixteen
+// products to a result 2.53e-8, 2.56e-8 and 3.4e-8 (2.53e-8, 3.1e-8 and 6.0e-8).
 #include <algorithm>
 #include <type_traits>
 
@@ -137,7 +138,7 @@ __device__ __forceinline__ void redo(const Args& g, const float* pa, const float
   }
 }
 
-template <int WM, int WN, int TM, int TN, int KS, bool APART, bool TA, bool TB>
+template <int WM, int WN, int TM, int TN, int KS, bool TA, bool TB>
 __global__ __launch_bounds__(WM * WN * KS * 64, 2) void k_gemm_split(Args g) {
   constexpr int NT = WM * WN * 64, BM = WM * TM * 32, BN = WN * TN * 32;
   using OA = Operand<BM, NT, !TA>;
@@ -166,16 +167,11 @@ __global__ __launch_bounds__(WM * WN * KS * 64, 2) void k_gemm_split(Args g) {
   oa.prep(pa, g.lda, m0, g.M, tid);
   ob.prep(pb, g.ldb, n0, g.N, tid);
 
-  f32x16 acc[TM][TN], low[APART ? TM : 1][APART ? TN : 1];   // APART: the five smaller products of the six, in sums of their own
+  f32x16 acc[TM][TN], low[TM][TN];   // the products of the first parts; the seven smaller ones
 #pragma unroll
   for (int a = 0; a < TM; a++)
 #pragma unroll
-    for (int b = 0; b < TN; b++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) {
-        acc[a][b][v] = 0.0f;
-        if constexpr (APART) low[a][b][v] = 0.0f;
-      }
+    for (int b = 0; b < TN; b++) acc[a][b] = low[a][b] = f32x16{};
 
   // the parts take the steps in turn: this one's step s is the product's step s KS + part (zeros behind the last one)
   const int full = g.K / kStep / KS, steps = (g.K + kStep * KS - 1) / (kStep * KS);
@@ -212,23 +208,23 @@ __global__ __launch_bounds__(WM * WN * KS * 64, 2) void k_gemm_split(Args g) {
   auto step = [&](int s, auto load_kind, auto conv) {
     constexpr int LOAD = decltype(load_kind)::value;
     constexpr bool CONV = decltype(conv)::value;
-    constexpr int T = TM * TN, NM = 6 * T, kPairs = OA::kPairs + OB::kPairs;
+    constexpr int T = TM * TN, NM = 8 * T, kPairs = OA::kPairs + OB::kPairs;
 #pragma unroll
     for (int a = 0; a < TM; a++) fa[2][a] = na[a];
 #pragma unroll
     for (int b = 0; b < TN; b++) fb[0][b] = nb[b];
     each<NM>([&](auto at) {
       constexpr int i = decltype(at)::value;
-      // smaller products first: part 2 of A with 0 of B, 1 with 1 and 0, 0 with 2, 1 and 0
-      constexpr int p = i < T ? 2 : i < 3 * T ? 1 : 0, in = i - (p == 2 ? 0 : p == 1 ? T : 3 * T), q = 2 - p - in / T, t = in % T, a = t / TN, b = t % TN;
-      if constexpr (APART && p + q > 0) low[a][b] = mfma(fa[p][a], fb[q][b], low[a][b]);
+      // smaller products first: part 2 of A with 1 and 0 of B, 1 with 2, 1 and 0, 0 with 2, 1 and 0
+      constexpr int p = i < 2 * T ? 2 : i < 5 * T ? 1 : 0, in = i - (p == 2 ? 0 : p == 1 ? 2 * T : 5 * T), q = (p == 2 ? 1 : 2) - in / T, t = in % T, a = t / TN, b = t % TN;
+      if constexpr (p + q > 0) low[a][b] = mfma(fa[p][a], fb[q][b], low[a][b]);
       else acc[a][b] = mfma(fa[p][a], fb[q][b], acc[a][b]);
       if constexpr (i < TM) fa[1][i] = read_a(cur, 1, i);
       if constexpr (i >= T && i < T + TM) fa[0][i - T] = read_a(cur, 0, i - T);
       // operands of the next step as their registers fall free (behind the last step: whatever LDS holds, unused)
-      if constexpr (i >= 3 * T && i < 3 * T + TM) na[i - 3 * T] = read_a(next, 2, i - 3 * T);
-      if constexpr (i >= 4 * T && i < 4 * T + TN) fb[2][i - 4 * T] = read_b(next, 2, i - 4 * T);
-      if constexpr (i >= 5 * T && i < 5 * T + TN) { fb[1][i - 5 * T] = read_b(next, 1, i - 5 * T); nb[i - 5 * T] = read_b(next, 0, i - 5 * T); }
+      if constexpr (i >= 4 * T && i < 4 * T + TM) na[i - 4 * T] = read_a(next, 2, i - 4 * T);
+      if constexpr (i >= 6 * T && i < 6 * T + TN) fb[2][i - 6 * T] = read_b(next, 2, i - 6 * T);
+      if constexpr (i >= 7 * T && i < 7 * T + TN) { fb[1][i - 7 * T] = read_b(next, 1, i - 7 * T); nb[i - 7 * T] = read_b(next, 0, i - 7 * T); }
       if constexpr (CONV) {
         // pair c begins behind instruction c kLast / (kPairs - 1), a stage to an instruction; the last stores have some
         // instructions to go before the barrier waits for them
@@ -260,12 +256,10 @@ __global__ __launch_bounds__(WM * WN * KS * 64, 2) void k_gemm_split(Args g) {
   for (; s + 2 < steps; s++) step(s, std::integral_constant<int, 0>{}, Yes{});
   for (; s < steps; s++) step(s, std::integral_constant<int, 0>{}, No{});
 
-  if constexpr (APART) {
 #pragma unroll
-    for (int a = 0; a < TM; a++)
+  for (int a = 0; a < TM; a++)
 #pragma unroll
-      for (int b = 0; b < TN; b++) acc[a][b] += low[a][b];
-  }
+    for (int b = 0; b < TN; b++) acc[a][b] += low[a][b];
   if constexpr (KS > 1) {   // the parts' sums, in the order of the parts (behind the last step's barrier LDS is free)
     static_assert((KS - 1) * BM * BN * 4 <= (int)sizeof(shared), "the parts' sums fit");
     float* const sums = (float*)shared;
@@ -308,40 +302,39 @@ __global__ __launch_bounds__(WM * WN * KS * 64, 2) void k_gemm_split(Args g) {
   }
 }
 
-template <int WM, int WN, int TM, int TN, int KS, bool APART>
+template <int WM, int WN, int TM, int TN, int KS>
 void launch(hipStream_t stream, const Args& g, int batch, bool ta, bool tb) {
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
   const dim3 grid((unsigned)((int64_t)((g.N + BN - 1) / BN) * ((g.M + BM - 1) / BM) * batch)), block(WM * WN * KS * 64);
-  if (ta && tb) hipLaunchKernelGGL((k_gemm_split<WM, WN, TM, TN, KS, APART, true, true>), grid, block, 0, stream, g);
-  else if (ta) hipLaunchKernelGGL((k_gemm_split<WM, WN, TM, TN, KS, APART, true, false>), grid, block, 0, stream, g);
-  else if (tb) hipLaunchKernelGGL((k_gemm_split<WM, WN, TM, TN, KS, APART, false, true>), grid, block, 0, stream, g);
-  else hipLaunchKernelGGL((k_gemm_split<WM, WN, TM, TN, KS, APART, false, false>), grid, block, 0, stream, g);
+  if (ta && tb) hipLaunchKernelGGL((k_gemm_split<WM, WN, TM, TN, KS, true, true>), grid, block, 0, stream, g);
+  else if (ta) hipLaunchKernelGGL((k_gemm_split<WM, WN, TM, TN, KS, true, false>), grid, block, 0, stream, g);
+  else if (tb) hipLaunchKernelGGL((k_gemm_split<WM, WN, TM, TN, KS, false, true>), grid, block, 0, stream, g);
+  else hipLaunchKernelGGL((k_gemm_split<WM, WN, TM, TN, KS, false, false>), grid, block, 0, stream, g);
 }
 
 }  // namespace
 
 // The forms: rows and columns of a workgroup's tile, parts of K inside the workgroup, workgroups that share a compute
 // unit, and their times in us: per tile and step of 16 k (of each part) with a compute unit full of workgroups, the
-// same for those that do not fill one (per_odd once, and for each of them), and per tile.  Fitted to 600 products of 16 to
-// 4096 a side and batches of up to 64; nine in ten of the estimates are within 9 % of the times.  4096 x 4096 x 4096
-// takes 575 us on the 256 x 256 tiles (float32 instructions 1122; 1.43 PFLOP/s of bf16 products at the clock the chip
-// holds under them: where it need not save power a step takes 1.53 us, the matrix instructions alone 1.57), 675 on 128 x 128
-// and 950 on 64 x 64, where every wavefront converts more of what it multiplies; 2048 x 2048 x 2048 91 with K in two parts,
-// 95 in one (float32 145); 64 of 512 x 512 x 512 82 (150); 1024 x 1024 x 1024 19 with K in four parts (25).
+// same for those that do not fill one (per_odd once, and for each of them), per tile, and once.  Fitted to 318 products of 64 to
+// 4096 a side and batches of up to 64, each run for 12 ms; nine in ten of the estimates are between 0.87 and 1.11 of the times,
+// those above 200 us, where the clock comes down, between 0.81 and 0.99.  4096 x 4096 x 4096 takes 843 us on 128 x 128 tiles
+// (float32 instructions 1202) and 1082 on 64 x 64, where every wavefront converts more of what it multiplies; 2048 x 2048 x 2048
+// 115 with K in two parts, 123 in one (float32 153); 64 of 512 x 512 x 512 116 (151); 1024 x 1024 x 1024 22 with K in four parts (26).
 struct Form { int rows, cols, parts, share; double per_step, per_odd, per_tile, start; };
-static const Form kForms[] = {{256, 256, 1, 1, 1.53, 0, 4.5, 4.5}, {128, 128, 1, 2, 0.604, 0.312, 2.75, 3.3}, {128, 128, 2, 1, 1.07, 0, 7.3, 0},
-                              {64, 64, 2, 2, 0.438, 0.274, 1.54, 3.4}, {64, 64, 4, 1, 0.895, 0, 4.6, 1.1}};
+static const Form kForms[] = {{128, 128, 1, 2, 0.69, 0.38, 2.8, 3.5}, {128, 128, 2, 1, 1.41, 0, 7.3, 0}, {64, 64, 2, 2, 0.495, 0.34, 1.75, 2.6},
+                              {64, 64, 4, 1, 1.01, 0, 4.6, 1.0}};
 
 // The form for a float32 product whose quickest kernel on the float32 instructions takes other_us by its estimate, or -1.
 // Below 9 us the launch and the first loads are what either kernel takes, and the estimates no help (1241 x 199,
-// K = 90 6.4 us against 6.0); of 450 products offered to the rule one that it took, at 0.93 of that estimate and less,
-// was slower, by 4 %, and together they took 0.92 of the time.
+// K = 90 6.4 us against 6.0).  Of 318 products offered to the rule it takes 214, together in 0.75 of the time; at 0.95 of the other
+// estimate and less eight of them are slower, by 1 to 4 %.
 int gh_gemm_split_form(const gh_cmd& c, int cus, double other_us) {
   const int64_t M = c.dim[0], N = c.dim[1], K = c.dim[2], batch = c.dim[6] <= 0 ? 1 : c.dim[6];
   // at least one whole step; offsets inside a tile in 32 bits; a launch of one dimension
   if (K < kStep || std::max(c.dim[3], c.dim[4]) >= (int64_t)1 << 21 || std::max(M, N) >= (int64_t)1 << 30 || (M + 63) / 64 * ((N + 63) / 64) * batch >= (int64_t)1 << 30) return -1;
   int best = -1;
-  double us = 0.93 * other_us;
+  double us = 0.95 * other_us;
   if (us < 9.0) return -1;
   for (int i = 0; i < (int)(sizeof(kForms) / sizeof(kForms[0])); i++) {
     const Form& f = kForms[i];
@@ -365,11 +358,10 @@ int gh_launch_gemm_split(gh_ctx* ctx, const gh_cmd& c, int form) {
   g.alpha = c.f[0];
   const bool ta = c.flags & GH_FLAG_TRANS_A, tb = c.flags & GH_FLAG_TRANS_B;
   switch (form) {
-    case 0: launch<2, 4, 4, 2, 1, false>(ctx->stream, g, batch, ta, tb); break;
-    case 1: launch<2, 2, 2, 2, 1, true>(ctx->stream, g, batch, ta, tb); break;
-    case 2: launch<2, 2, 2, 2, 2, true>(ctx->stream, g, batch, ta, tb); break;
-    case 3: launch<1, 2, 2, 1, 2, true>(ctx->stream, g, batch, ta, tb); break;
-    default: launch<1, 2, 2, 1, 4, true>(ctx->stream, g, batch, ta, tb); break;
+    case 0: launch<2, 2, 2, 2, 1>(ctx->stream, g, batch, ta, tb); break;
+    case 1: launch<2, 2, 2, 2, 2>(ctx->stream, g, batch, ta, tb); break;
+    case 2: launch<1, 2, 2, 1, 2>(ctx->stream, g, batch, ta, tb); break;
+    default: launch<1, 2, 2, 1, 4>(ctx->stream, g, batch, ta, tb); break;
   }
   return gh_check_hip(ctx, hipGetLastError(), "gemm launch");
 }

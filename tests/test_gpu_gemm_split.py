@@ -12,7 +12,7 @@ from tests.util import rel_frobenius
 
 pytestmark = pytest.mark.gpu
 
-# 256 x 256; 128 x 128; the same in two parts of K; 64 x 64 in two parts; in four
+# 128 x 128; the same in two parts of K; 64 x 64 in two parts; in four
 SHAPES = [(3800, 4001, 131, 1), (640, 650, 18, 40), (2047, 2049, 95, 1), (2000, 2000, 47, 1), (2176, 1900, 64, 1), (1025, 1023, 129, 4),
           (255, 513, 97, 30), (1200, 2100, 333, 1), (500, 500, 500, 8), (1000, 1000, 1025, 1), (1024, 1024, 1024, 1)]
 
@@ -47,8 +47,7 @@ def _inputs(m, n, k, batch, ta, tb, pad=0, seed=0):
 
 
 # 16 k are summed exactly but for one rounding of the sum, 2^-24 of its size at most, a third of that on average, and the roundings
-# add up as their root: K = 1025 gives sqrt(65) * 2^-24 / sqrt(3) * sqrt(1/2) = 2.0e-7; six times that with all six products in
-# one sum, where K is at most 131 here.
+# add up as their root: K = 1025 gives sqrt(65) * 2^-24 / sqrt(3) * sqrt(1/2) = 2.0e-7.
 @pytest.mark.parametrize("m,n,k,batch", SHAPES)
 def test_product(ctx, m, n, k, batch):
     for ta, tb in ((False, False), (True, False), (False, True), (True, True)):
@@ -61,6 +60,19 @@ def test_product(ctx, m, n, k, batch):
 def test_wider_leading_dimensions_at_any_float(ctx, m, n, k, batch, ta, tb):
     a, b, x, y = _inputs(m, n, k, batch, ta, tb, pad=3)
     assert rel_frobenius(_run(ctx, a, b, m, n, k, batch, ta, tb, pad=3, shift=1), np.matmul(x, y)) <= 3e-7
+
+
+# 0.5 for rounding the sum, and of the seven smaller products, 2^-7 of the first, three roundings of half their last place at most
+@pytest.mark.parametrize("m,n,k,batch", [(2000, 2000, 47, 1), (1200, 2100, 333, 1), (500, 500, 500, 8), (1024, 1024, 1024, 1)])
+def test_one_product_to_a_result(ctx, m, n, k, batch):
+    rng = np.random.default_rng(m + k)
+    a, b = np.zeros((batch, m, k), np.float32), rng.standard_normal((batch, k, n), np.float32)
+    at = rng.integers(0, k, (batch, m))
+    scale = rng.standard_normal((batch, m), np.float32)
+    np.put_along_axis(a, at[:, :, None], scale[:, :, None], 2)
+    want = scale[:, :, None].astype(np.float64) * np.take_along_axis(b, np.repeat(at[:, :, None], n, 2), 1)
+    last = np.spacing(np.abs(want).astype(np.float32)).astype(np.float64)
+    assert (np.abs(_run(ctx, a, b, m, n, k, batch) - want) / last).max() <= 0.5 + 1.5 / 128
 
 
 def test_whole_numbers_are_exact(ctx):
