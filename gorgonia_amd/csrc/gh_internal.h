@@ -156,7 +156,7 @@ int gh_gemm_direct_form(const gh_cmd& c, int cus, double* us, int* rounds);   //
 int gh_gemm_direct_slices(const gh_cmd& c, int form, int cus);
 int gh_launch_gemm_direct(gh_ctx* ctx, const gh_cmd& c, int form);
 // float32 products on the bf16 matrix instructions (k_gemm_split.hip)
-int gh_gemm_split_form(const gh_cmd& c, int cus, double other_us);   // -1: not taken
+int gh_gemm_split_form(const gh_cmd& c, int cus, double other_us, int other_slices);   // -1: not taken; the other kernel's time and its slices of K
 int gh_launch_gemm_split(gh_ctx* ctx, const gh_cmd& c, int form);
 // products of one to four rows (k_gemm_thin.hip)
 bool gh_gemm_thin_takes(const gh_cmd& c);

@@ -3163,7 +3163,12 @@ static int direct_form(const gh_cmd& c, int cus) {
 static int split_form(const gh_cmd& c, int cus) {
   if (getenv("GORGONIA_HIP_GEMM_PLAN") || getenv("GORGONIA_HIP_NO_SPLIT")) return -1;
   double us = 0;
-  return gh_gemm_direct_form(c, cus, &us, nullptr) < 0 ? -1 : gh_gemm_split_form(c, cus, std::min(us, tile128_us(c, true, cus)));
+  if (gh_gemm_direct_form(c, cus, &us, nullptr) < 0) return -1;
+  us = std::min(us, tile128_us(c, true, cus));
+  if (gh_gemm_split_form(c, cus, us, 1) < 0) return -1;   // (its slices are asked for only where they matter)
+  int slices = 1;
+  gh_gemm_route(&c, &slices);
+  return gh_gemm_split_form(c, cus, us, slices);
 }
 
 // Which kernel takes a float64 product of more than two rows: a form of k_gemm_direct, kStaged64 for tiles staged in LDS

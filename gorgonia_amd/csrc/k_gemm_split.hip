@@ -325,11 +325,18 @@ struct Form { int rows, cols, parts, share; double per_step, per_odd, per_tile, 
 static const Form kForms[] = {{128, 128, 1, 2, 0.69, 0.38, 2.8, 3.5}, {128, 128, 2, 1, 1.41, 0, 7.3, 0}, {64, 64, 2, 2, 0.495, 0.34, 1.75, 2.6},
                               {64, 64, 4, 1, 1.01, 0, 4.6, 1.0}};
 
-// The form for a float32 product whose quickest kernel on the float32 instructions takes other_us by its estimate, or -1.
+// The form for a float32 product whose quickest kernel on the float32 instructions takes other_us by its estimate and cuts K
+// into other_slices sums, or -1.
+//
+// A sum of n roundings is off by about sqrt(n) of one, cut into p parts by sqrt(n) / p: 2.0e-8 sqrt(n) / p for uniform values
+// on either kind of instruction.  Here n is K / 16, there K / 2, so that p has to be 0.35 of the other's slices at least for an
+// error below the other kernel's (2321 x 3480, K = 2049 of uniform values: 2.2e-7 in one part, 1.2e-7 in two, 1.6e-7 on
+// k_gemm_direct in four).
+//
 // Below 9 us the launch and the first loads are what either kernel takes, and the estimates no help (1241 x 199,
 // K = 90 6.4 us against 6.0).  Of 318 products offered to the rule it takes 214, together in 0.75 of the time; at 0.95 of the other
 // estimate and less eight of them are slower, by 1 to 4 %.
-int gh_gemm_split_form(const gh_cmd& c, int cus, double other_us) {
+int gh_gemm_split_form(const gh_cmd& c, int cus, double other_us, int other_slices) {
   const int64_t M = c.dim[0], N = c.dim[1], K = c.dim[2], batch = c.dim[6] <= 0 ? 1 : c.dim[6];
   // at least one whole step; offsets inside a tile in 32 bits; a launch of one dimension
   if (K < kStep || std::max(c.dim[3], c.dim[4]) >= (int64_t)1 << 21 || std::max(M, N) >= (int64_t)1 << 30 || (M + 63) / 64 * ((N + 63) / 64) * batch >= (int64_t)1 << 30) return -1;
@@ -338,6 +345,7 @@ int gh_gemm_split_form(const gh_cmd& c, int cus, double other_us) {
   if (us < 9.0) return -1;
   for (int i = 0; i < (int)(sizeof(kForms) / sizeof(kForms[0])); i++) {
     const Form& f = kForms[i];
+    if (8 * f.parts * f.parts < other_slices * other_slices) continue;
     const int64_t tiles = (M + f.rows - 1) / f.rows * ((N + f.cols - 1) / f.cols) * batch, steps = (K + kStep * f.parts - 1) / (kStep * f.parts);
     const int64_t each = (tiles + cus - 1) / cus, odd = each % f.share, whole = each - odd;
     const double est = f.start + (double)steps * ((double)whole * f.per_step + (odd ? (1.0 + (double)odd) * f.per_odd : 0.0)) + (double)each * f.per_tile;

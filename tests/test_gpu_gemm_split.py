@@ -75,6 +75,18 @@ def test_one_product_to_a_result(ctx, m, n, k, batch):
     assert (np.abs(_run(ctx, a, b, m, n, k, batch) - want) / last).max() <= 0.5 + 1.5 / 128
 
 
+@pytest.mark.parametrize("m,n,k", [(4096, 4096, 4096), (2048, 2048, 2048), (2321, 3480, 2049), (2649, 3563, 3143), (1000, 1000, 4000)])
+@pytest.mark.parametrize("values", ["normal", "uniform"])
+def test_error_is_no_larger_than_on_the_float32_instructions(ctx, monkeypatch, m, n, k, values):
+    rng = np.random.default_rng(k)
+    a, b = (rng.standard_normal(s, np.float32) if values == "normal" else rng.random(s, np.float32) for s in ((1, m, k), (1, k, n)))
+    want = np.matmul(a[0].astype(np.float64), b[0].astype(np.float64))
+    split = rel_frobenius(_run(ctx, a, b, m, n, k)[0], want)
+    monkeypatch.setitem(globals(), "_cmd", lambda pa, pb, pc, m, n, k, batch, **kw: D.cmd_gemm(pa, pb, pc, m, n, k, batch=batch, **kw))
+    monkeypatch.setenv("GORGONIA_HIP_NO_SPLIT", "1")
+    assert split <= rel_frobenius(_run(ctx, a, b, m, n, k)[0], want)
+
+
 def test_whole_numbers_are_exact(ctx):
     rng = np.random.default_rng(3)
     a, b = (rng.integers(-60, 61, s).astype(np.float32) for s in ((1, 1024, 1024), (1, 1024, 1024)))
