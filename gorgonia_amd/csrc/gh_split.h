@@ -11,8 +11,8 @@
 //
 // Range: the inputs are scaled by 2^16, so that every bit of the smallest denormal stays inside bf16's (denormal) range
 // and the split is exact for all inputs below 2^112; results are scaled back.  Larger, infinite and NaN inputs, and
-// sums above 2^96, come out as an infinity or a NaN: a kernel tests what it summed (split_finite) and computes such a tile
-// again with the float32 instructions.
+// sums above 2^96, come out as an infinity or a NaN: a kernel tests what it summed and computes such a tile again with the
+// float32 instructions.
 #pragma once
 #include <hip/hip_runtime.h>
 

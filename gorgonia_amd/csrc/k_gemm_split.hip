@@ -15,6 +15,11 @@
 // on: 4096 x 4096 x 4096 4.0e-7 / 3.0e-7 (k_sgemm 1.14e-6 / 8.4e-7); 2321 x 3480, K = 2049 1.9e-7 / 1.2e-7 (k_gemm_direct in
 // four slices 4.1e-7 / 1.6e-7); 1000 x 1000, K = 4000 1.9e-7 / 8.3e-8 (in eight 4.0e-7 / 1.1e-7).  One, two and sixteen
 // products to a result 2.53e-8, 2.56e-8 and 3.4e-8 (2.53e-8, 3.1e-8 and 6.0e-8).
+//
+// Values that the split cannot hold: a workgroup whose sums are not finite computes its tile on the float32 instructions, from
+// the step on where it finds that out.  It looks in its third step, every 32 steps, and at the end.  us, beside k_sgemm or
+// k_gemm_direct: 4096 x 4096 x 4096 of NaN 1230 (1102), with one row of -FLT_MAX 1372 (1157), with a triangle of it or infinities
+// in the last k 2010 and 2131 (1138); 1024 x 1024 x 1024 31, 33, 44 and 45 (25); 64 of 512 x 512 x 512 180, 200, 274 and 304 (160).
 #include <algorithm>
 #include <type_traits>
 
@@ -83,6 +88,16 @@ struct Operand {
       reg[j][e] = past ? 0.0f : v;
     }
   }
+  // the values as they are, as [k][row] with rows kRows floats long
+  static constexpr int kRows = R + 4;
+  __device__ __forceinline__ void put32(float* lds) const {
+#pragma unroll
+    for (int j = 0; j < kPer; j++) {
+      float* const p = lds + k_at[j] * kRows + slot[j] - k_at[j] / 8 * kHalf;
+#pragma unroll
+      for (int e = 0; e < 8; e++) p[e * kRows] = reg[j][e];
+    }
+  }
   // stage K of pair I of a thread's values; the last stage of a unit's last pair stores the unit
   static constexpr int kPairs = 4 * kPer;
   u32x4 part[kPer][3];
@@ -116,28 +131,6 @@ __device__ __forceinline__ void put(const Args& g, float* C, int i, int j, f32x1
     if (i + 8 * (e / 4) + e % 4 < g.M) p[(int64_t)(8 * (e / 4) + e % 4) * g.ldc] = v[e];
 }
 
-// A wavefront's TM x TN tiles at row i0 and column j0 with the float32 instructions, one after the other.
-template <int TM, int TN, bool TA, bool TB>
-__device__ __forceinline__ void redo(const Args& g, const float* pa, const float* pb, float* C, int i0, int j0) {
-  const int lr = (int)threadIdx.x & 31, lh = ((int)threadIdx.x & 63) >> 5;
-  const int64_t ka = TA ? g.lda : 1, kb = TB ? 1 : g.ldb;
-  for (int t = 0; t < TM * TN; t++) {
-    const int i = i0 + t / TN * 32, j = j0 + t % TN * 32;
-    if (i >= g.M || j >= g.N) continue;
-    const float* const ra = pa + (int64_t)min(i + lr, g.M - 1) * (TA ? 1 : g.lda);
-    const float* const rb = pb + (int64_t)min(j + lr, g.N - 1) * (TB ? g.ldb : 1);
-    f32x16 acc[4] = {};
-    for (int k0 = 0; k0 < g.K; k0 += 8)
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int k = k0 + 2 * u + lh, kc = min(k, g.K - 1);
-        const float xa = ra[kc * ka], xb = rb[kc * kb];
-        acc[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(k < g.K ? xa : 0.0f, k < g.K ? xb : 0.0f, acc[u], 0, 0, 0);
-      }
-    put(g, C, i + 4 * lh, j + lr, (acc[0] + acc[1]) + (acc[2] + acc[3]), 1.0f, g.bias && j + lr < g.N ? g.bias[j + lr] : -0.0f);
-  }
-}
-
 template <int WM, int WN, int TM, int TN, int KS, bool TA, bool TB>
 __global__ __launch_bounds__(WM * WN * KS * 64, 2) void k_gemm_split(Args g) {
   constexpr int NT = WM * WN * 64, BM = WM * TM * 32, BN = WN * TN * 32;
@@ -168,10 +161,33 @@ __global__ __launch_bounds__(WM * WN * KS * 64, 2) void k_gemm_split(Args g) {
   ob.prep(pb, g.ldb, n0, g.N, tid);
 
   f32x16 acc[TM][TN], low[TM][TN];   // the products of the first parts; the seven smaller ones
+  auto clear = [&](f32x16 (&v)[TM][TN]) {
 #pragma unroll
-  for (int a = 0; a < TM; a++)
+    for (int a = 0; a < TM; a++)
 #pragma unroll
-    for (int b = 0; b < TN; b++) acc[a][b] = low[a][b] = f32x16{};
+      for (int b = 0; b < TN; b++) v[a][b] = f32x16{};
+  };
+  auto fold = [&] {
+#pragma unroll
+    for (int a = 0; a < TM; a++)
+#pragma unroll
+      for (int b = 0; b < TN; b++) acc[a][b] += low[a][b];
+  };
+  clear(acc);
+  clear(low);
+  // whether a sum of this wavefront is infinite or NaN, for the whole workgroup behind its next barrier
+  __shared__ int lost;
+  if (threadIdx.x == 0) lost = 0;
+  auto look = [&] {
+    float zero = 0.0f;   // stays 0 where every sum is finite
+#pragma unroll
+    for (int a = 0; a < TM; a++)
+#pragma unroll
+      for (int b = 0; b < TN; b++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) zero = __builtin_fmaf(acc[a][b][v], 0.0f, zero);
+    if (__any(zero != 0.0f) && lane == 0) lost = 1;
+  };
 
   // the parts take the steps in turn: this one's step s is the product's step s KS + part (zeros behind the last one)
   const int full = g.K / kStep / KS, steps = (g.K + kStep * KS - 1) / (kStep * KS);
@@ -251,46 +267,88 @@ __global__ __launch_bounds__(WM * WN * KS * 64, 2) void k_gemm_split(Args g) {
   };
   using Yes = std::true_type; using No = std::false_type;
   int s = 0;
-  for (; s + 3 < full; s++) step(s, std::integral_constant<int, 1>{}, Yes{});
-  for (; s + 3 < steps; s++) step(s, std::integral_constant<int, 2>{}, Yes{});
-  for (; s + 2 < steps; s++) step(s, std::integral_constant<int, 0>{}, Yes{});
-  for (; s < steps; s++) step(s, std::integral_constant<int, 0>{}, No{});
-
-#pragma unroll
-  for (int a = 0; a < TM; a++)
-#pragma unroll
-    for (int b = 0; b < TN; b++) acc[a][b] += low[a][b];
-  if constexpr (KS > 1) {   // the parts' sums, in the order of the parts (behind the last step's barrier LDS is free)
-    static_assert((KS - 1) * BM * BN * 4 <= (int)sizeof(shared), "the parts' sums fit");
-    float* const sums = (float*)shared;
-    if (part) {
-#pragma unroll
-      for (int a = 0; a < TM; a++)
-#pragma unroll
-        for (int b = 0; b < TN; b++)
-#pragma unroll
-          for (int v = 0; v < 16; v++) sums[((((part - 1) * TM + a) * TN + b) * 16 + v) * NT + tid] = acc[a][b][v];
-    }
-    __syncthreads();
-    if (part) return;
-#pragma unroll
-    for (int p = 0; p < KS - 1; p++)
-#pragma unroll
-      for (int a = 0; a < TM; a++)
-#pragma unroll
-        for (int b = 0; b < TN; b++)
-#pragma unroll
-          for (int v = 0; v < 16; v++) acc[a][b][v] += sums[(((p * TM + a) * TN + b) * 16 + v) * NT + tid];
+  bool again = false;
+  for (; s + 3 < full && !again; s++) {
+    // (early, for operands that are infinite or NaN throughout, and now and then; 1 % of the time)
+    const bool looks = s % 32 == 2;
+    if (looks) look();
+    step(s, std::integral_constant<int, 1>{}, Yes{});
+    if (looks) again = lost;
+  }
+  if (!again) {
+    for (; s + 3 < steps; s++) step(s, std::integral_constant<int, 2>{}, Yes{});
+    for (; s + 2 < steps; s++) step(s, std::integral_constant<int, 0>{}, Yes{});
+    for (; s < steps; s++) step(s, std::integral_constant<int, 0>{}, No{});
   }
 
-  float zero = 0.0f;   // stays 0 where every sum is finite
+  // the parts' sums, in the order of the parts, to those of part 0
+  static_assert((KS - 1) * BM * BN * 4 <= (int)sizeof(shared), "the parts' sums fit");
+  auto gather = [&] {
+    if constexpr (KS > 1) {
+      __syncthreads();   // LDS is free
+      float* const sums = (float*)shared;
+      if (part) {
 #pragma unroll
-  for (int a = 0; a < TM; a++)
+        for (int a = 0; a < TM; a++)
 #pragma unroll
-    for (int b = 0; b < TN; b++)
+          for (int b = 0; b < TN; b++)
 #pragma unroll
-      for (int v = 0; v < 16; v++) zero = __builtin_fmaf(acc[a][b][v], 0.0f, zero);
-  if (__any(zero != 0.0f)) return redo<TM, TN, TA, TB>(g, pa, pb, g.C + bz * g.sC, m0 + wm, n0 + wn);
+            for (int v = 0; v < 16; v++) sums[((((part - 1) * TM + a) * TN + b) * 16 + v) * NT + tid] = acc[a][b][v];
+      }
+      __syncthreads();
+      if (!part) {
+#pragma unroll
+        for (int p = 0; p < KS - 1; p++)
+#pragma unroll
+          for (int a = 0; a < TM; a++)
+#pragma unroll
+            for (int b = 0; b < TN; b++)
+#pragma unroll
+              for (int v = 0; v < 16; v++) acc[a][b][v] += sums[(((p * TM + a) * TN + b) * 16 + v) * NT + tid];
+      }
+    }
+  };
+  if (!again) {
+    fold();
+    gather();
+    look();
+    __syncthreads();
+    again = lost;
+  }
+  float scale = kDown;
+  if (again) {
+    // The tile with the float32 instructions, its operands staged as they are, in two buffers; a chain of 256 k at a time.
+    constexpr int kTile = kStep * (OA::kRows + OB::kRows);
+    static_assert(2 * kTile <= 4 * 3 * kBuf, "two steps of float32 operands fit");
+    float* const mine = (float*)lds;
+    scale = 1.0f;
+    clear(acc);
+    clear(low);
+    load(0);
+    for (int r = 0; r < steps; r++) {
+      float* const buf = mine + (r & 1) * kTile;
+      oa.put32(buf);
+      ob.put32(buf + kStep * OA::kRows);
+      if (r + 1 < steps) load(r + 1);
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < kStep; k += 2) {
+        float xa[TM], xb[TN];
+#pragma unroll
+        for (int a = 0; a < TM; a++) xa[a] = buf[(k + lh) * OA::kRows + wm + a * 32 + lr];
+#pragma unroll
+        for (int b = 0; b < TN; b++) xb[b] = buf[(kStep * OA::kRows) + (k + lh) * OB::kRows + wn + b * 32 + lr];
+#pragma unroll
+        for (int a = 0; a < TM; a++)
+#pragma unroll
+          for (int b = 0; b < TN; b++) low[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[a], xb[b], low[a][b], 0, 0, 0);
+      }
+      if (r % 16 == 15) { fold(); clear(low); }
+    }
+    fold();
+    gather();
+  }
+  if (part) return;
 
   float* const C = g.C + bz * g.sC;
 #pragma unroll
@@ -298,7 +356,7 @@ __global__ __launch_bounds__(WM * WN * KS * 64, 2) void k_gemm_split(Args g) {
     const int j = n0 + wn + b * 32 + lr;
     const float bias = g.bias && j < g.N ? g.bias[j] : -0.0f;
 #pragma unroll
-    for (int a = 0; a < TM; a++) put(g, C, m0 + wm + a * 32 + 4 * lh, j, acc[a][b], kDown, bias);
+    for (int a = 0; a < TM; a++) put(g, C, m0 + wm + a * 32 + 4 * lh, j, acc[a][b], scale, bias);
   }
 }
 

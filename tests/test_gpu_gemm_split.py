@@ -135,6 +135,50 @@ def test_values_the_split_cannot_hold(ctx, m, n, k, batch, ta, tb):
             assert rel_frobenius(got[z, :, cols][f], want[z, :, cols][f]) <= 1e-6
 
 
+# the places where a workgroup looks at its sums: early, on the way (from 560 k in one part) and at the end
+@pytest.mark.parametrize("m,n,k,batch", [(640, 650, 18, 40), (3000, 3001, 700, 1), (1200, 2100, 333, 1), (500, 500, 500, 8), (1024, 1024, 1024, 1)])
+@pytest.mark.parametrize("place", [0.0, 0.6, 1.0])
+@pytest.mark.parametrize("value", [np.nan, np.inf, -3.4e38])
+def test_one_value_that_the_split_cannot_hold(ctx, m, n, k, batch, place, value):
+    a, b, x, y = _inputs(m, n, k, batch, False, False)
+    row, at = m - 2, int(place * (k - 1))
+    a[batch - 1, row, at] = value
+    b[:, at] = np.where(np.abs(b[:, at]) > 0.5, 0.5, b[:, at])   # (a product of the largest value stays a float32)
+    got = _run(ctx, a, b, m, n, k, batch)
+    want = np.matmul(a.astype(np.float64), b.astype(np.float64)) if np.isfinite(value) else None
+    if want is None:
+        bad = np.float32(value) * b[batch - 1, at]
+        assert np.array_equal(got[batch - 1, row], bad, equal_nan=True)
+        a[batch - 1, row] = 0.0
+        want = np.matmul(a.astype(np.float64), b.astype(np.float64))
+        got[batch - 1, row] = 0.0
+    else:
+        assert rel_frobenius(got[batch - 1, row], want[batch - 1, row]) <= 1e-6
+        got[batch - 1, row] = want[batch - 1, row] = 0.0
+    assert rel_frobenius(got, want) <= 3e-7
+
+
+# A tile that is computed twice takes both kernels' times (less than twice the slower one's), and some more where a compute
+# unit has one tile.
+@pytest.mark.parametrize("m,n,k,batch", [(2048, 2048, 2048, 1), (1024, 1024, 1024, 1), (512, 512, 512, 64)])
+def test_time_of_values_that_the_split_cannot_hold(ctx, monkeypatch, m, n, k, batch):
+    a = np.full((batch, m, k), np.nan, np.float32)
+    p = [ctx.upload(a), ctx.upload(a), ctx.malloc(4 * batch * m * n)]
+    cmd = _cmd(*p, m, n, k, batch, stride_a=m * k, stride_b=k * n, stride_c=m * n)
+
+    def ms():
+        ctx.run([cmd] * 20)
+        ctx.event(0)
+        ctx.submit([cmd] * 20)
+        ctx.event(1)
+        return ctx.elapsed_ms(0, 1)
+    split = min(ms() for _ in range(5))
+    monkeypatch.setenv("GORGONIA_HIP_NO_SPLIT", "1")
+    assert split <= 3 * min(ms() for _ in range(5))
+    for q in p:
+        ctx.free(q)
+
+
 @pytest.mark.parametrize("scale", [1e-30, 1e-36, 1e-39])
 def test_small_and_denormal_values_keep_their_bits(ctx, scale):
     m, n, k = 1024, 1024, 1024
