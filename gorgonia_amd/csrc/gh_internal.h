@@ -46,7 +46,7 @@ struct gh_llc_model {
 };
 
 constexpr int kBnHeldSlots = 2048;
-constexpr int64_t kBnHeldPage = kBnHeldSlots * (8 + 8 + 4);
+constexpr int64_t kBnHeldPage = kBnHeldSlots * (8 + 8 + 4 + 4);
 
 // One sum of slabs (k_slab_sums.hip): out[e] = the sum over the slabs of ws[s][e], in one of these orders.
 enum { kSumGroups64, kSumGroups16, kSumGroups64F64, kSumGroups16F64, kSumLanes16, kSumLanes4, kSumPlain };
@@ -73,7 +73,7 @@ struct gh_ctx {
   // scratch owned by the context (split-K partials, reduction flags)
   void* workspace = nullptr;
   int64_t workspace_bytes = 0;
-  // what the workgroups of k_bn_held.hip pass to each other: two slots of 8 bytes and one count of 4 for each of
+  // what the workgroups of k_bn_held.hip pass to each other: two slots of 8 bytes, a claim and a count of 4 for each of
   // kBnHeldSlots, zero whenever no kernel runs; null where the device's pages were all taken
   void* bn_page = nullptr;
   // slabs whose sums gh_submit has put off, in memory of their own (kSlabSpace, or null so far), and those sums

@@ -6,13 +6,18 @@
 // through memory and wait for each other's.  A 22 MB tensor fits the chip's registers (128 MB): between its sums and the
 // values it writes the gradient keeps what it has read, the forward its values between its two passes.
 //
-// A wait ends whether or not the others come: a workgroup that has asked kPolls times reads the missing shares and adds
-// them up itself, in the same order, to the same bits.  Nothing depends on all workgroups being on the chip at once.
+// Nobody waits for a workgroup that has not begun: a share belongs to the workgroup that claims it, its own at first, and one
+// that has asked kPolls times for the missing sums claims shares that nobody has begun.  So a share that is waited for is being
+// worked on, by a workgroup that waits for nothing meanwhile, however few of them the chip has room for; one that begins when
+// its share is taken leaves.  The sums are added in the order of the shares, to the same bits whoever brings them.
+// us of a forward pair in one context and in each of two, three and four at once, 8 x 16 x 208 x 208: 20, 35, 57 and 74 (the
+// commands apart 33, 47, 61 and 77; waiting for every workgroup, with the missing shares added up again by all: 20, 61, 8900 and
+// 13800); a training step of the four-block network 430, 660, 910 and 1310 (apart 500, 750, 990 and 1460).
 //
 // Bound: HBM and the caches for large planes, the launch and the waits (some 1.5 us each) for small ones.  us, four launches
-// or three / one, forward and gradient: 8 x 16 x 208 x 208 30.9 / 18.7 and 33.8 / 21.1 (4.4 TB/s of the 94 MB that the
-// gradient moves), 8 x 32 x 104 x 104 20.5 / 11.8 and 22.9 / 12.3, 8 x 128 x 26 x 26 14.2 / 8.9 and 13.4 / 7.0,
-// 8 x 16 x 207 x 207 (single loads) 46.6 / 20.8 and 47.3 / 25.8, 2 x 3 x 4 x 4 12.1 / 7.5 and 10.0 / 4.9.  (The forward as the
+// or three / one, forward and gradient: 8 x 16 x 208 x 208 30.9 / 19.6 and 33.8 / 22.5 (4.2 TB/s of the 94 MB that the
+// gradient moves), 8 x 32 x 104 x 104 20.5 / 12.6 and 22.9 / 13.1, 8 x 128 x 26 x 26 14.2 / 9.8 and 13.4 / 7.7,
+// 8 x 16 x 207 x 207 (single loads) 46.6 / 20.9 and 47.3 / 25.9, 2 x 3 x 4 x 4 12.1 / 8.9 and 10.0 / 5.7.  (The forward as the
 // gradient is, its values kept as the pooling's windows lie: 14.8, 9.9 and 7.3, and other sums.)
 #include <algorithm>
 #include <cfloat>
@@ -23,7 +28,8 @@ namespace {
 
 constexpr int kThreads = 1024;
 constexpr int kHeld = 6;   // groups of four values that a thread of the forward keeps
-constexpr int kPolls = 2000;   // about a millisecond (GORGONIA_HIP_BN_POLLS: another number)
+constexpr int kPolls = 8;   // some 5 us (GORGONIA_HIP_BN_POLLS: another number; 0: every second workgroup is taken to come too late)
+constexpr int kGiveUp = 1 << 22;   // polls, seconds: never reached; the sums are NaN then
 typedef unsigned long long u64;
 
 __device__ __forceinline__ float relu_of(float v) { return v * (v >= 0.0f ? 1.0f : 0.0f); }
@@ -35,7 +41,7 @@ template <int K> struct Vec { typedef float T __attribute__((ext_vector_type(K))
 // a workgroup has `per` of a channel's units.
 struct Planes {
   int H, W, uw, plane_units, units, per, C, G;
-  int polls;   // how often a workgroup asks for the others' sums
+  int polls;   // how often a workgroup asks for the others' sums before it claims shares
 };
 
 // Two rows of COLS values; EDGES: H or W is odd, or rows lie where only single values can be loaded.
@@ -102,74 +108,71 @@ __device__ __forceinline__ float group_sum(float v, float* sh) {
 __device__ __forceinline__ void publish(u64* slots, int g, float v) {
   __hip_atomic_store(slots + g, (1ull << 32) | __builtin_bit_cast(unsigned, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// the same, and back when every compute unit sees it
-__device__ __forceinline__ void publish_and_wait(u64* slots, int g, float v) {
-  const u64 old = __hip_atomic_exchange(slots + g, (1ull << 32) | __builtin_bit_cast(unsigned, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  asm volatile("" ::"v"((unsigned)old) : "memory");
-}
 __device__ __forceinline__ u64 look(const u64* slots, int g) { return __hip_atomic_load(slots + g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 struct Sums {
   float part[2][64];
-  u64 missing;
   float waves[kThreads / 64];
+  int mine;   // a claim came first
+  int next;   // the share to do next, or -1
 };
 
-// Wavefront 0 waits for the G shares of `kinds` sums and leaves them in LDS; a share that has not come is in `missing`.
-__device__ __forceinline__ void gather(u64* const (&slots)[2], int kinds, int G, int polls, Sums& sh) {
+// What a channel's workgroups share: G sums of two kinds (forward: one after the other), a claim for each share, and a count.
+struct Channel {
+  u64* slots[2];
+  unsigned *claims, *count;
+  __device__ __forceinline__ Channel(u64* page, int c, int sums, int shares)
+      : slots{page + c * sums, page + kBnHeldSlots + c * sums}, claims((unsigned*)(page + 2 * kBnHeldSlots) + c * shares), count((unsigned*)(page + 2 * kBnHeldSlots) + kBnHeldSlots + c) {}
+};
+__device__ __forceinline__ bool claim(const Channel& ch, int share) { return !__hip_atomic_exchange(ch.claims + share, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// Waits for the G sums of kinds `first`..`last` and leaves them in LDS: -1.  Or the number of a share (of the first `shares`)
+// that nobody has begun and that is this workgroup's now.
+__device__ __forceinline__ int gather(const Channel& ch, int first, int last, int G, int shares, int polls, Sums& sh) {
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
+    int next = -1;
     u64 v[2] = {1ull << 32, 1ull << 32};
-    u64 miss = G < 64 ? (1ull << G) - 1 : ~0ull;
-    for (int asked = 0; asked < polls; asked++) {
+    for (int asked = 0;; asked++) {
       if (lane < G)
-        for (int k = 0; k < kinds; k++) v[k] = look(slots[k], lane);
-      miss = __ballot(!(v[0] >> 32) || !(v[1] >> 32));
-      if (!miss) break;
+        for (int k = first; k <= last; k++) v[k] = look(ch.slots[k], lane);
+      if (!__ballot(!(v[0] >> 32) || !(v[1] >> 32)) || asked == kGiveUp) break;
+      if (asked >= polls && shares) {
+        const u64 open = __ballot(lane < shares && !__hip_atomic_load(ch.claims + (lane < shares ? lane : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        if (open) {
+          const int s = __builtin_ctzll(open);
+          const int got = lane == 0 && claim(ch, s);
+          if (__shfl(got, 0, 64)) { next = s; break; }
+          continue;
+        }
+      }
       __builtin_amdgcn_s_sleep(1);
     }
-    for (int k = 0; k < kinds; k++) sh.part[k][lane] = __builtin_bit_cast(float, (unsigned)v[k]);
-    if (lane == 0) sh.missing = miss;
+    for (int k = first; k <= last; k++) sh.part[k][lane] = v[k] >> 32 ? __builtin_bit_cast(float, (unsigned)v[k]) : __builtin_nanf("");
+    if (lane == 0) sh.next = next;
   }
   __syncthreads();
+  const int next = sh.next;
+  __syncthreads();   // before the next one is written
+  return next;
+}
+__device__ __forceinline__ float total(const Sums& sh, int kind, int G) {
+  float s = 0.0f;
+  for (int g = 0; g < G; g++) s = s + sh.part[kind][g];
+  return s;
 }
 
-// The G shares, the missing ones added up here by `share(g)`, in order.  A share that has come meanwhile is taken as it came:
-// its workgroup may already be writing over what share(g) has read.
-template <class F>
-__device__ __forceinline__ void total(u64* const (&slots)[2], int kinds, int G, int polls, Sums& sh, float (&out)[2], F&& share) {
-  gather(slots, kinds, G, polls, sh);
-  u64 miss = sh.missing;
-  while (miss) {
-    const int g = __builtin_ctzll(miss);
-    miss &= miss - 1;
-    float v[2];
-    share(g, v);
-    __threadfence();
-    __syncthreads();
-    if (threadIdx.x == 0)
-      for (int k = 0; k < kinds; k++) {
-        const u64 now = look(slots[k], g);
-        sh.part[k][g] = now >> 32 ? __builtin_bit_cast(float, (unsigned)now) : v[k];
-      }
-    __syncthreads();
-  }
-  for (int k = 0; k < kinds; k++) {
-    float s = 0.0f;
-    for (int g = 0; g < G; g++) s = s + sh.part[k][g];
-    out[k] = s;
-  }
-}
-
-// The channel's slots are zero again when its last workgroup is through.  (No order with the tensors' values is needed, and a
-// release here would write the cache back: 16 us instead of 10 for 8 x 128 x 26 x 26.)
-__device__ __forceinline__ void leave(u64* const (&slots)[2], unsigned* count, int shares, int workgroups) {
-  if (threadIdx.x == 0 && __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)workgroups - 1) {
-    for (int g = 0; g < shares; g++) {
-      __hip_atomic_store(slots[0] + g, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(slots[1] + g, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Everything of the channel is zero again when its last workgroup is through.  (A workgroup that has published a sum has seen
+// it, with all the others, before it comes here.  No order with the tensors' values is needed, and a release here would write
+// the cache back: 16 us instead of 10 for 8 x 128 x 26 x 26.)
+__device__ __forceinline__ void leave(const Channel& ch, int sums, int shares) {
+  if (threadIdx.x == 0 && __hip_atomic_fetch_add(ch.count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)shares - 1) {
+    for (int g = 0; g < sums; g++) {
+      __hip_atomic_store(ch.slots[0] + g, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(ch.slots[1] + g, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int g = 0; g < shares; g++) __hip_atomic_store(ch.claims + g, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(ch.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -193,7 +196,10 @@ __global__ __launch_bounds__(kThreads) void k_bn_train_pool(const float* __restr
                                                             BnOut o, u64* page) {
   __shared__ Sums sh;
   const int c = blockIdx.x % g.C, w = blockIdx.x / g.C;
-  u64* const slots[2] = {page + c * cut.groups, page + kBnHeldSlots + c * cut.groups};
+  const Channel ch(page, c, cut.groups, g.G);
+  const int shares = (cut.groups + cut.own - 1) / cut.own;   // those with sums; the others only write
+  bool claimed = false;
+  if (threadIdx.x == 0 && !(g.polls == 0 && (w & 1) && w < shares)) claimed = claim(ch, w);
   const int quarter = threadIdx.x >> 8, t = threadIdx.x & 255, mine = w * cut.own + quarter;
   const bool works = quarter < cut.own && mine < cut.groups;
   const int B = (int)(n / cut.S), img = g.C * cut.S, step = cut.groups * 256;
@@ -256,7 +262,7 @@ __global__ __launch_bounds__(kThreads) void k_bn_train_pool(const float* __restr
     const float* const four = sh.waves + 4 * quarter;
     return (four[0] + four[1]) + (four[2] + four[3]);
   };
-  float mean = 0.0f, var = 0.0f, sum[2];
+  float mean = 0.0f, var = 0.0f;
   if constexpr (HELD > 0) {
     if (works)
       hold([&](int j, int at) {
@@ -264,20 +270,36 @@ __global__ __launch_bounds__(kThreads) void k_bn_train_pool(const float* __restr
         for (int e = 0; e < 4; e++) v[j][e] = x[at + e * img];
       });
   }
+  if (threadIdx.x == 0) sh.mine = claimed;   // (asked for in front of the loads)
+  __syncthreads();
+  if (!sh.mine) return leave(ch, cut.groups, g.G);
+  u64 more = 0;   // shares that were claimed behind the first
+  auto again = [&](int share, int pass) {   // from memory
+    const int k = share * cut.own + quarter;
+    const bool has = quarter < cut.own && k < cut.groups;
+    const float s = group(has ? walk(k, mean, pass == 1) : 0.0f);
+    if (has && t == 0) publish(ch.slots[pass], k, s);
+  };
 #pragma unroll
   for (int pass = 0; pass < 2; pass++) {
     const bool sq = pass == 1;
     float acc = 0.0f;
     if (works) acc = HELD > 0 ? held(mean, sq) : walk(mine, mean, sq);
     const float s = group(acc);
-    if (works && t == 0) publish(slots[pass], mine, s);
-    u64* const both[2] = {slots[pass], slots[pass]};
-    total(both, 1, cut.groups, g.polls, sh, sum, [&](int k, float (&r)[2]) { r[0] = group(walk(k, mean, sq)); });
-    if (!sq) mean = sum[0] / (float)n;
-    else var = sum[0];
+    if (works && t == 0) publish(ch.slots[pass], mine, s);
+    if (sq)
+      for (u64 left = more; left; left &= left - 1) again(__builtin_ctzll(left), pass);
+    for (int share; (share = gather(ch, pass, pass, cut.groups, sq ? 0 : shares, g.polls, sh)) >= 0;) {
+      more |= 1ull << share;
+      again(share, pass);
+    }
+    const float sum = total(sh, pass, cut.groups);
+    if (!sq) mean = sum / (float)n;
+    else var = sum;
     __syncthreads();   // the sums have been read
   }
-  if (w == 0 && threadIdx.x == 0) {
+  more |= 1ull << w;
+  if ((more & 1) && threadIdx.x == 0) {
     o.save_mean[c] = mean;
     o.save_var[c] = var;
     const float m1 = o.momentum * mean, m2 = (1.0f - o.momentum) * o.run_mean[c];
@@ -289,36 +311,38 @@ __global__ __launch_bounds__(kThreads) void k_bn_train_pool(const float* __restr
   const float a = 1.0f / sqrtf(var / (float)n + o.eps);
   const float b = -mean * a;
   // the values again, from the caches, as the pooling's windows lie
-  const int end = min(g.units, (w + 1) * g.per);
+  for (; more; more &= more - 1) {
+    const int from = __builtin_ctzll(more) * g.per, end = min(g.units, from + g.per);
 #pragma unroll 2
-  for (int u = w * g.per + threadIdx.x; u < end; u += blockDim.x) {
-    const Unit<COLS, EDGES> q(g, u);
-    float z[2][COLS];
-    q.load(g, x + q.at(g, c), z);
+    for (int u = from + threadIdx.x; u < end; u += blockDim.x) {
+      const Unit<COLS, EDGES> q(g, u);
+      float z[2][COLS];
+      q.load(g, x + q.at(g, c), z);
 #pragma unroll
-    for (int r = 0; r < 2; r++)
+      for (int r = 0; r < 2; r++)
 #pragma unroll
-      for (int e = 0; e < COLS; e++) {
-        const float m = z[r][e] * a;
-        z[r][e] = m + b;
+        for (int e = 0; e < COLS; e++) {
+          const float m = z[r][e] * a;
+          z[r][e] = m + b;
+        }
+      q.store(g, y + q.at(g, c), z);
+      if (EDGES && !(q.right && q.below)) continue;
+      float best[COLS / 2];
+#pragma unroll
+      for (int e = 0; e < COLS / 2; e++) {
+        best[e] = -FLT_MAX;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const float r = relu_of(z[k >> 1][2 * e + (k & 1)]);
+          if (r > best[e]) best[e] = r;
+        }
       }
-    q.store(g, y + q.at(g, c), z);
-    if (EDGES && !(q.right && q.below)) continue;
-    float best[COLS / 2];
-#pragma unroll
-    for (int e = 0; e < COLS / 2; e++) {
-      best[e] = -FLT_MAX;
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const float r = relu_of(z[k >> 1][2 * e + (k & 1)]);
-        if (r > best[e]) best[e] = r;
-      }
+      float* const p = pooled + q.pooled(g, c);
+      if constexpr (COLS == 4) *(Vec<2>::T*)p = Vec<2>::T{best[0], best[1]};
+      else *p = best[0];
     }
-    float* const p = pooled + q.pooled(g, c);
-    if constexpr (COLS == 4) *(Vec<2>::T*)p = Vec<2>::T{best[0], best[1]};
-    else *p = best[0];
   }
-  leave(slots, (unsigned*)(page + 2 * kBnHeldSlots) + c, cut.groups, g.G);
+  leave(ch, cut.groups, g.G);
 }
 
 // x: the tensor that was rectified and pooled; dp: the pooled tensor's gradient; dx: the gradient of x; z: the tensor that was
@@ -328,111 +352,140 @@ __global__ __launch_bounds__(kThreads) void k_pool_bn_bwd(const float* x, const 
                                                           int64_t n, const float* __restrict__ save_mean, const float* __restrict__ save_var, float eps, u64* page) {
   __shared__ Sums sh;
   const int c = blockIdx.x % g.C, w = blockIdx.x / g.C;
-  u64* const slots[2] = {page + c * g.G, page + kBnHeldSlots + c * g.G};
+  const Channel ch(page, c, g.G, g.G);
+  bool claimed = false;
+  if (threadIdx.x == 0 && !(g.polls == 0 && (w & 1))) claimed = claim(ch, w);
   const float mean = save_mean[c], vb = save_var[c] / (float)n;
   float zv[N][2][COLS], gv[N][2][COLS];
-  auto share = [&](int who, bool own, float (&hz)[N][2][COLS], float (&hg)[N][2][COLS], float (&out)[2]) __attribute__((always_inline)) {
-    float s = 0.0f, dot = 0.0f;
+  // unit k of a thread in share `who`
+  auto has = [&](int who, int k) { return k * (int)blockDim.x + (int)threadIdx.x < g.per && who * g.per + k * (int)blockDim.x + (int)threadIdx.x < g.units; };
+  auto unit = [&](int who, int k) { return Unit<COLS, EDGES>(g, who * g.per + k * (int)blockDim.x + (int)threadIdx.x); };
+  auto load = [&](int who, int k, float (&hz)[2][COLS], float (&hg)[2][COLS], float (&d)[COLS / 2]) __attribute__((always_inline)) {
+    if (!has(who, k)) return;
+    const Unit<COLS, EDGES> t = unit(who, k);
+    t.load(g, x + t.at(g, c), hg);
+    t.load(g, z + t.at(g, c), hz);
+    const float* const p = dp + t.pooled(g, c);
+    if constexpr (COLS == 4) {
+      const auto pv = *(const Vec<2>::T*)p;
+      d[0] = pv[0];
+      d[1] = pv[1];
+    } else {
+      d[0] = t.right && t.below ? *p : 0.0f;
+    }
+  };
+  float s, dot;
+  auto add = [&](int who, int k, const float (&hz)[2][COLS], float (&hg)[2][COLS], const float (&d)[COLS / 2]) __attribute__((always_inline)) {
+    if (!has(who, k)) return;
+    const Unit<COLS, EDGES> t = unit(who, k);
+    const bool whole = t.right && t.below;
+#pragma unroll
+    for (int e = 0; e < COLS / 2; e++) {
+      float best = -FLT_MAX;
+      int arg = -1;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const float r = relu_of(hg[q >> 1][2 * e + (q & 1)]);
+        if (r > best) { best = r; arg = q; }
+      }
+      const float v = 0.0f + d[e];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        float& h = hg[q >> 1][2 * e + (q & 1)];
+        const float o = arg == q ? v : 0.0f;
+        h = whole ? o * relu_mask(h) : 0.0f;
+      }
+    }
+    t.store(g, dx + t.at(g, c), hg);
+    float s4[2][COLS], d4[2][COLS];
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int e = 0; e < COLS; e++) {
+        const float t1 = hz[r][e] * hg[r][e], t2 = mean * hg[r][e];
+        s4[r][e] = t.has(r, e) ? hg[r][e] : 0.0f;
+        d4[r][e] = t.has(r, e) ? t1 - t2 : 0.0f;
+      }
+    float qs = 0.0f, qd = 0.0f;
+#pragma unroll
+    for (int e = 0; e < COLS; e += 2) {
+      qs = qs + ((s4[0][e] + s4[0][e + 1]) + (s4[1][e] + s4[1][e + 1]));
+      qd = qd + ((d4[0][e] + d4[0][e + 1]) + (d4[1][e] + d4[1][e + 1]));
+    }
+    s = s + qs;
+    dot = dot + qd;
+  };
+  float sum[2];
+  auto say = [&](int who) {
+    sum[0] = group_sum(s, sh.waves);
+    sum[1] = group_sum(dot, sh.waves);
+    if (threadIdx.x == 0) {
+      publish(ch.slots[0], who, sum[0]);
+      publish(ch.slots[1], who, sum[1]);
+    }
+  };
+  {
     // everything a thread needs is on its way before the first value is looked at
     float d[N][COLS / 2];
 #pragma unroll
-    for (int k = 0; k < N; k++) {
-      const int u = who * g.per + k * (int)blockDim.x + (int)threadIdx.x;
-      const bool mine = k * (int)blockDim.x + (int)threadIdx.x < g.per && u < g.units;
-      if (!mine) continue;
-      const Unit<COLS, EDGES> t(g, u);
-      t.load(g, x + t.at(g, c), hg[k]);
-      t.load(g, z + t.at(g, c), hz[k]);
-      const float* const p = dp + t.pooled(g, c);
-      if constexpr (COLS == 4) {
-        const auto pv = *(const Vec<2>::T*)p;
-        d[k][0] = pv[0];
-        d[k][1] = pv[1];
-      } else {
-        d[k][0] = t.right && t.below ? *p : 0.0f;
-      }
-    }
+    for (int k = 0; k < N; k++) load(w, k, zv[k], gv[k], d[k]);
+    if (threadIdx.x == 0) sh.mine = claimed;   // (asked for in front of the loads)
+    __syncthreads();
+    if (!sh.mine) return leave(ch, g.G, g.G);
+    s = dot = 0.0f;
 #pragma unroll
-    for (int k = 0; k < N; k++) {
-      const int u = who * g.per + k * (int)blockDim.x + (int)threadIdx.x;
-      const bool mine = k * (int)blockDim.x + (int)threadIdx.x < g.per && u < g.units;
-      if (!mine) continue;
-      const Unit<COLS, EDGES> t(g, u);
-      const bool whole = t.right && t.below;
-#pragma unroll
-      for (int e = 0; e < COLS / 2; e++) {
-        float best = -FLT_MAX;
-        int arg = -1;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const float r = relu_of(hg[k][q >> 1][2 * e + (q & 1)]);
-          if (r > best) { best = r; arg = q; }
-        }
-        const float v = 0.0f + d[k][e];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          float& h = hg[k][q >> 1][2 * e + (q & 1)];
-          const float o = arg == q ? v : 0.0f;
-          h = whole ? o * relu_mask(h) : 0.0f;
-        }
-      }
-      if (own) t.store(g, dx + t.at(g, c), hg[k]);
-      float s4[2][COLS], d4[2][COLS];
-#pragma unroll
-      for (int r = 0; r < 2; r++)
-#pragma unroll
-        for (int e = 0; e < COLS; e++) {
-          const float t1 = hz[k][r][e] * hg[k][r][e], t2 = mean * hg[k][r][e];
-          s4[r][e] = t.has(r, e) ? hg[k][r][e] : 0.0f;
-          d4[r][e] = t.has(r, e) ? t1 - t2 : 0.0f;
-        }
-      float qs = 0.0f, qd = 0.0f;
-#pragma unroll
-      for (int e = 0; e < COLS; e += 2) {
-        qs = qs + ((s4[0][e] + s4[0][e + 1]) + (s4[1][e] + s4[1][e + 1]));
-        qd = qd + ((d4[0][e] + d4[0][e + 1]) + (d4[1][e] + d4[1][e + 1]));
-      }
-      s = s + qs;
-      dot = dot + qd;
-    }
-    out[0] = group_sum(s, sh.waves);
-    out[1] = group_sum(dot, sh.waves);
-  };
-  float sum[2];
-  share(w, true, zv, gv, sum);
-  if (threadIdx.x == 0) {
-    // before dz is written (behind the barrier in total): a workgroup that adds up this share in this one's place and reads
-    // values of dz finds the slots filled
-    publish_and_wait(slots[0], w, sum[0]);
-    publish_and_wait(slots[1], w, sum[1]);
+    for (int k = 0; k < N; k++) add(w, k, zv[k], gv[k], d[k]);
+    say(w);
   }
-  total(slots, 2, g.G, g.polls, sh, sum, [&](int who, float (&r)[2]) {
-    float oz[N][2][COLS], og[N][2][COLS];
-    share(who, false, oz, og, r);
-  });
+  u64 more = 0;   // shares that were claimed behind the first
+  for (int who; (who = gather(ch, 0, 1, g.G, g.G, g.polls, sh)) >= 0;) {
+    more |= 1ull << who;
+    s = dot = 0.0f;
+#pragma unroll 1
+    for (int k = 0; k < N; k++) {
+      float hz[2][COLS], hg[2][COLS], d[COLS / 2];
+      load(who, k, hz, hg, d);
+      add(who, k, hz, hg, d);
+    }
+    say(who);
+  }
+  sum[0] = total(sh, 0, g.G);
+  sum[1] = total(sh, 1, g.G);
   const float invstd = 1.0f / sqrtf(vb + eps);
   float f = sum[1] * invstd;
   f = f * invstd;
   f = f / (float)n;
   const float grad_mean = sum[0] / (float)n;
-#pragma unroll
-  for (int k = 0; k < N; k++) {
-    const int u = w * g.per + k * (int)blockDim.x + (int)threadIdx.x;
-    if (k * (int)blockDim.x + (int)threadIdx.x >= g.per || u >= g.units) break;
-    const Unit<COLS, EDGES> t(g, u);
+  auto finish = [&](const Unit<COLS, EDGES>& t, const float (&hz)[2][COLS], float (&hg)[2][COLS]) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < 2; r++)
 #pragma unroll
       for (int e = 0; e < COLS; e++) {
-        float m = zv[k][r][e] - mean;
+        float m = hz[r][e] - mean;
         m = m * f;
-        float q = gv[k][r][e] - grad_mean;
+        float q = hg[r][e] - grad_mean;
         q = q - m;
-        gv[k][r][e] = q * invstd;
+        hg[r][e] = q * invstd;
       }
-    t.store(g, dz + t.at(g, c), gv[k]);
+    t.store(g, dz + t.at(g, c), hg);
+  };
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    if (!has(w, k)) break;
+    finish(unit(w, k), zv[k], gv[k]);
   }
-  leave(slots, (unsigned*)(page + 2 * kBnHeldSlots) + c, g.G, g.G);
+  for (; more; more &= more - 1) {   // (a thread reads the gradient that it has written)
+    const int who = __builtin_ctzll(more);
+#pragma unroll 1
+    for (int k = 0; k < N && has(who, k); k++) {
+      const Unit<COLS, EDGES> t = unit(who, k);
+      float hz[2][COLS], hg[2][COLS];
+      t.load(g, z + t.at(g, c), hz);
+      t.load(g, dx + t.at(g, c), hg);
+      finish(t, hz, hg);
+    }
+  }
+  leave(ch, g.G, g.G);
 }
 
 // ---- which commands ---------------------------------------------------------------------
@@ -486,7 +539,7 @@ bool plan(const gh_cmd& pool, bool fwd, uint64_t wide, uint64_t narrow, int cus,
     if (C * p.g.G > kBnHeldSlots || p.N > kMost * (p.cols == 4 ? 1 : 2)) return false;
     p.threads = (int)(((per + p.N - 1) / p.N + 63) / 64 * 64);
   }
-  if (const char* asks = getenv("GORGONIA_HIP_BN_POLLS")) p.g.polls = std::max(0, std::min(kPolls, atoi(asks)));
+  if (const char* asks = getenv("GORGONIA_HIP_BN_POLLS")) p.g.polls = std::max(0, std::min(1000, atoi(asks)));
   return true;
 }
 

@@ -2,6 +2,9 @@
 commands write.  The forward's are those of the two commands apart, to the bit; the saved statistics are held to a float64 sum,
 what is computed from them to the bit; the gradient's two sums are not stored, so that its result is held to the bound that
 their rounding leaves."""
+import threading
+import time
+
 import numpy as np
 import pytest
 
@@ -184,6 +187,40 @@ def test_replays(ctx):
         ctx.run(fwd + bwd)
     ctx.graph_destroy(graph)
     m.all()
+
+
+@pytest.mark.parametrize("shape", [(8, 16, 208, 208), (8, 32, 104, 104)])
+def test_time_of_three_contexts_at_once(shape):
+    """Each launch has a workgroup for every compute unit: together they find room for some of each.  Three take three times as
+    long as one, and some more where they load what another has put out of the caches."""
+    x, rm, rv, dp = _inputs(shape, 11)
+    nan = np.full_like(x, np.nan)
+
+    def seconds(ctxs):
+        work = []
+        for c in ctxs:
+            m = _Place(c, 0, x=x, y=nan, p=np.full_like(dp, np.nan), rm=rm, rv=rv, sm=rm * 0, sv=rm * 0, dp=dp, t=nan, dz=nan)
+            work.append((c, sum(_commands(m, shape), []) * 10))
+            c.run(work[-1][1])
+        gate = threading.Barrier(len(work) + 1)
+
+        def run(c, cmds):
+            gate.wait()
+            for _ in range(10):
+                c.run(cmds)
+            gate.wait()
+        threads = [threading.Thread(target=run, args=w) for w in work]
+        for t in threads:
+            t.start()
+        gate.wait()
+        start = time.perf_counter()
+        gate.wait()
+        took = time.perf_counter() - start
+        for t in threads:
+            t.join()
+        return took
+    with D.Context() as a, D.Context() as b, D.Context() as c:
+        assert min(seconds([a, b, c]) for _ in range(2)) <= 10 * min(seconds([a]) for _ in range(2))
 
 
 def test_two_contexts_at_once(ctx):
