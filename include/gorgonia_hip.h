@@ -291,7 +291,11 @@ GH_API int gh_memcpy_staged(gh_ctx* ctx, gh_devptr dst, void* stage, const void*
  * BatchedContext.LaunchAndSync of cuda/arith.go:62, the cuBLAS calls at
  * cuda/linalg.go:102,223,282 and the cuDNN calls in ops/nn/ *_cuda.go files).
  * A command that fails validation enqueues nothing from that command on and
- * returns GH_EINVAL/GH_ENOFUNC with the index in gh_last_error(). */
+ * returns GH_EINVAL/GH_ENOFUNC with the index in gh_last_error().  Commands
+ * that run in one launch have the bits of the commands one by one, but for a
+ * BN_BWD right behind the MAXPOOL2D_BWD whose result it takes: its two sums are
+ * added in another order than when it is submitted apart (or in a context
+ * beyond a device's 64th), so that the gradient's last bits are others. */
 GH_API int gh_submit(gh_ctx* ctx, const gh_cmd* cmds, int n);
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory around a submit - code under HIP graph capture, tight serving loops,

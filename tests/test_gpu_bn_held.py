@@ -10,7 +10,7 @@ import pytest
 
 from gorgonia_amd import _ffi
 from gorgonia_amd import device as D
-from tests.util import assert_bits_equal
+from tests.util import assert_bits_equal, rel_frobenius
 
 pytestmark = pytest.mark.gpu
 
@@ -138,6 +138,17 @@ def test_one_launch(ctx, shape):
     for k in ("y", "p", "sm", "sv", "rm", "rv", "t"):
         if k != "y":   # (the last gradient lies over it)
             assert_bits_equal(got[k], apart[k])
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_gradient_next_to_the_commands_apart(ctx, shape):
+    """Two orders of adding the same terms: both within the bound, and apart by less than the rounding of a result."""
+    given, got = _run(ctx, shape, 5)
+    _, apart = _run(ctx, shape, 5, together=False)
+    _check(shape, given, apart)
+    for k in ("y", "p", "sm", "sv", "rm", "rv", "t"):
+        assert_bits_equal(got[k], apart[k])
+    assert rel_frobenius(got["dz"], apart["dz"].astype(np.float64)) <= U
 
 
 @pytest.mark.parametrize("shift", [1, 2])
