@@ -198,7 +198,7 @@ bool gh_conv_pointwise_takes(const gh_cmd& c, int cus);
 // 3x3 / padding 1 over three or four channels, in place of the wide-image kernel (k_conv_strip.hip)
 bool gh_conv_strip_takes(const gh_cmd& c);
 int gh_launch_conv_strip(gh_ctx* ctx, const gh_cmd& c);
-int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, bool patch = false);   // -1: not taken; patch: the patch kernel is the other
+int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, bool whole = false);   // -1: not taken; whole: the other's sums run over all channels
 int gh_launch_conv_lanes(gh_ctx* ctx, const gh_cmd& c, bool flip, int form);
 int gh_launch_maxpool2d(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_bn_infer(gh_ctx* ctx, const gh_cmd& c);

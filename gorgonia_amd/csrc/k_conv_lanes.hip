@@ -397,12 +397,14 @@ static int quickest(const gh_cmd& c, bool flip, bool f64, int cus, int from, int
 // are that good.
 //
 // float32 where that is not so: a wavefront with a tile of its own and all channels, for few channels and many pixels, where
-// the split forms have one or two quads to a wavefront and the wide-image kernel stages as much as it multiplies.  Not in
-// place of a split form or of the patch kernel, which split the channels: its sums are longer (the gradient of 4 x 128 x 60 x
-// 60 -> 64 would be off by 4.3e-7 of its norm instead of 1.6e-7).  us, before / now: 8 x 16 x 104 x 104 -> 32 22.9 / 15.9, pooled 17.9 / 13.6, its gradient 24.2 / 13.6; 8 x 16 x 104 x 104 -> 16
+// the split forms have one or two quads to a wavefront and the wide-image kernel stages as much as it multiplies.  Only in place
+// of a kernel whose sums run over all channels too (`whole`), since its own are longer than those of one that splits them: the
+// gradient of 4 x 128 x 60 x 60 -> 64 would be off by 4.3e-7 of its norm instead of 1.6e-7, that of 13 x 96 x 45 x 45 -> 48, which
+// runs as a split form over dy, by 2.9e-7 instead of 8.1e-8, that of 234 x 8 x 15 x 15 -> 32 by 2.5e-7, on the small-image
+// kernel 2.0e-7.  us, before / now: 8 x 16 x 104 x 104 -> 32 22.9 / 15.9, pooled 17.9 / 13.6, its gradient 24.2 / 13.6; 8 x 16 x 104 x 104 -> 16
 // 15.8 / 10.0 and its gradient 17.8 / 8.7; 8 x 32 x 104 x 104 -> 64 46.7 / 39.7 (80 TFLOP/s); 8 x 16 x 208 x 208 -> 32's
 // gradient 45.8 / 36.1; 1 x 16 x 208 x 208 -> 32 pooled 11.0 / 8.7.
-int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, bool patch) {
+int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, bool whole) {
   if (getenv("GORGONIA_HIP_CONV_NO_LANES")) return -1;   // tuning switch: the other kernels only
   const bool f64 = gh_dtype_of(c.flags) == GH_F64;
   Lanes<double> g;   // (the narrower of the two in what its offsets reach)
@@ -410,9 +412,9 @@ int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, boo
   double us;
   const int split = quickest(c, flip, f64, cus, 0, f64 && !flip ? 4 : 3, &us);
   if (other_us <= 0 || us < other_us / 1.17) return split;
-  if (f64 || patch) return -1;
-  const int whole = quickest(c, flip, false, cus, 3, 5, &us);
-  return us < other_us / 1.1 ? whole : -1;
+  if (f64 || !whole) return -1;
+  const int form = quickest(c, flip, false, cus, 3, 5, &us);
+  return us < other_us / 1.1 ? form : -1;
 }
 
 int gh_launch_conv_lanes(gh_ctx* ctx, const gh_cmd& c, bool flip, int form) {

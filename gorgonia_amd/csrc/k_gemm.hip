@@ -3271,19 +3271,27 @@ static bool conv_direct_takes(const gh_cmd& c) {
 // its own; the wide-image kernel's is fitted from above its quickest (8 x 16 x 208 x 208 -> 32 takes 40, 8 x 16 x 104 x
 // 104 -> 32 23, 2 x 16 x 104 x 104 -> 32 11), the tiled one's to 23 for 8 x 32 x 52 x 52 -> 64, 17 for two such images,
 // 13 for 3 x 16 x 49 x 49 -> 32.
-static double conv_others_us(const gh_cmd& c, int cus, bool* patch) {
+static double conv_others_us(const gh_cmd& c, int cus) {
   const double us = gh_conv_patch_us(c, cus);   // 0 where it does not take the shape
-  if ((*patch = us > 0)) return us;
+  if (us > 0) return us;
   const double oh = (double)(c.dim[2] + 2 * c.dim[7] - 2), ow = (double)(c.dim[3] + 2 * c.dim[8] - 2);
   const double flops = 18.0 * (double)c.dim[0] * (double)c.dim[1] * (double)c.dim[4] * oh * ow;
   return gh_conv_wide_takes(c) ? 10.0 + flops * 1e-8 : 12.0 + flops / 75e6;
 }
+// Whether the sums of the kernel that would run a 3x3 convolution go over all channels in one chain: the wide-image kernel's, the
+// tiled one's below 64 channels, where it does not cut them among workgroups, and the gathering one's where it does not.
+static bool conv_sums_whole(const gh_cmd& c) {
+  const int route = gh_conv2d_route(&c);
+  if (route != GH_CONV_ROUTE_GATHER) return route == GH_CONV_ROUTE_WIDE || (route == GH_CONV_ROUTE_TILED && c.dim[1] < 64);
+  gh_ctx probe;
+  probe.workspace = &probe;   // never dereferenced
+  probe.workspace_bytes = 64ll << 20;
+  return plan_tiles(&probe, c.dim[4], c.dim[0] * gh_conv_out(c.dim[2], 3, c.dim[7], 1, 1) * gh_conv_out(c.dim[3], 3, c.dim[8], 1, 1), 9 * c.dim[1], 1, true).splits == 1;
+}
 // float32, behind the single-channel, few-channel and small-image kernels, which win where they take a shape.
 static int conv_lanes_form(const gh_cmd& c, int cus) {
   if (c.dim[5] != 3 || c.dim[6] != 3 || gh_conv_rows1_takes(c) || conv_direct_takes(c) || gh_conv_small_takes(c)) return -1;
-  bool patch;
-  const double others = conv_others_us(c, cus, &patch);
-  return gh_conv_lanes_form(c, false, cus, others, patch);
+  return gh_conv_lanes_form(c, false, cus, conv_others_us(c, cus), conv_sums_whole(c));
 }
 // The image gradient: elsewhere that is a launch that mirrors the filters (4.7 us) and a forward one over dy.
 static int conv_lanes_gradient_form(const gh_cmd& c, int cus) {
@@ -3295,10 +3303,11 @@ static int conv_lanes_gradient_form(const gh_cmd& c, int cus) {
   f.dim[9] = f.dim[10] = f.dim[11] = f.dim[12] = 1;
   if (gh_conv_rows1_takes(f) || conv_direct_takes(f)) return -1;
   // the small-image kernels run at 55 TFLOP/s past 6 us (128 x 32 x 14 x 14 -> 64: 12.8 us and the mirroring)
-  bool patch = false;
   const double others = gh_conv_small_takes(f) ? 6.0 + 18.0 * (double)f.dim[0] * (double)f.dim[1] * (double)f.dim[4] * (double)f.dim[2] * (double)f.dim[3] / 55e6
-                                               : conv_others_us(f, cus, &patch);
-  return gh_conv_lanes_form(c, true, cus, others + 4.7, patch);
+                                               : conv_others_us(f, cus);
+  // (a forward form of 3 and more has whole sums as well)
+  const int forward = conv_lanes_form(f, cus);
+  return gh_conv_lanes_form(c, true, cus, others + 4.7, conv_sums_whole(f) && (forward < 0 || forward >= 3));
 }
 
 static int launch_conv_direct(gh_ctx* ctx, const gh_cmd& c) {
