@@ -116,12 +116,13 @@ int gh_validate_cmd(const gh_cmd& c, std::string& msg);
 // inputs lost (`cold`) or not, goes past the cache (k_elem.hip)
 bool gh_llc_cold(const gh_ctx* ctx, uint64_t p);
 bool gh_llc_stream(int64_t bytes, bool cold);
-// {BN_TRAIN, MAXPOOL2D} and {MAXPOOL2D_BWD, BN_BWD} in one launch that reads a channel once (k_bn_held.hip)
+// sums of filter-gradient slabs, put off where gh_submit allows it (k_slab_sums.hip)
 void* gh_slab_space(gh_ctx* ctx, int64_t bytes);
 int gh_sum_slabs(gh_ctx* ctx, const gh_slab_sum& s);
 int gh_flush_sums(gh_ctx* ctx);
 int gh_flush_sums_before(gh_ctx* ctx, const gh_cmd& c);
 int gh_bn_groups(int64_t n, int64_t S);   // the groups of 256 threads that k_bn_reduce cuts a channel of n values in planes of S into (k_bwd.hip)
+// {BN_TRAIN, MAXPOOL2D} and {MAXPOOL2D_BWD, BN_BWD} in one launch (k_bn_held.hip)
 bool gh_bn_held_pair(const gh_ctx* ctx, const gh_cmd* cmds, int n);
 int gh_launch_bn_held_pair(gh_ctx* ctx, const gh_cmd* cmds);
 // a run of elementwise commands in one pass (k_chain.hip): how many commands at the front of cmds one pass can take and is
@@ -194,10 +195,10 @@ bool gh_conv_wide_can_pool(const gh_cmd& c);
 // k_conv_pointwise.hip: 1x1 stride-1 convolution whose result is too small for K-wide 64x64 tiles to fill the device
 int gh_try_launch_conv_pointwise(gh_ctx* ctx, const gh_cmd& c);
 bool gh_conv_pointwise_takes(const gh_cmd& c, int cus);
-// 3x3 stride-1 convolution with operands straight from memory, both float types; flip: of an image-gradient command (k_conv_lanes.hip)
 // 3x3 / padding 1 over three or four channels, in place of the wide-image kernel (k_conv_strip.hip)
 bool gh_conv_strip_takes(const gh_cmd& c);
 int gh_launch_conv_strip(gh_ctx* ctx, const gh_cmd& c);
+// 3x3 stride-1 convolution with operands straight from memory, both float types; flip: of an image-gradient command (k_conv_lanes.hip)
 int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, bool whole = false);   // -1: not taken; whole: the other's sums run over all channels
 int gh_launch_conv_lanes(gh_ctx* ctx, const gh_cmd& c, bool flip, int form);
 int gh_launch_maxpool2d(gh_ctx* ctx, const gh_cmd& c);

@@ -55,16 +55,6 @@ struct Pair {
 };
 constexpr int kStages = 8;
 
-// eight values that follow each other in k: one operand register group per part
-__device__ __forceinline__ void eight(const float* x, u32x4* h, u32x4* m, u32x4* l) {
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    Pair p;
-    each<kStages>([&](auto k) { p.template stage<decltype(k)::value>(x[2 * i], x[2 * i + 1]); });
-    (*h)[i] = p.part[0]; (*m)[i] = p.part[1]; (*l)[i] = p.part[2];
-  }
-}
-
 __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }

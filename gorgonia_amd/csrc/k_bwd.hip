@@ -553,9 +553,9 @@ __global__ __launch_bounds__(kBlock) void k_dropout_bwd(const float* __restrict_
     dx[i] = (prob != 0.0f && y[i] != 0.0f) ? dy[i] / prob : 0.0f;
 }
 
-// how many workgroups share one channel's reduction
 }  // namespace
 
+// how many workgroups share one channel's reduction
 int gh_bn_groups(int64_t n, int64_t S) {
   // wide planes: two 256-wide strips of every image per workgroup; else 1024 images per workgroup
   int64_t g = S >= kBlock ? (S + kBlock - 1) / kBlock / 2 : (n / S) / 1024;

@@ -292,7 +292,7 @@ int launch(gh_ctx* ctx, Wg<T> g, T* dw) {
   hipLaunchKernelGGL((k_conv3x3_wgrad<T, TM, P, NT, kPacked>), dim3((unsigned)slices, (unsigned)ct, (unsigned)ft), dim3(kThreads), 0,
                      ctx->stream, g);
   const int rc = gh_check_hip(ctx, hipGetLastError(), "filter-gradient launch");
-    if (rc || slices == 1) return rc;
+  if (rc || slices == 1) return rc;
   // 64 results to a workgroup of the sum where that makes enough workgroups, else 16
   const bool many = results >= 64 * (int64_t)ctx->cu_count;
   return gh_sum_slabs(ctx, {g.out, dw, results, (int)slices, sizeof(T) == 8 ? (many ? kSumGroups64F64 : kSumGroups16F64) : many ? kSumGroups64 : kSumGroups16});
