@@ -2,14 +2,14 @@
 //
 // Elementwise commands that follow each other on tensors of one size read what the command before them wrote:
 // each is a pass over memory (or, for small tensors, a launch) that exists only to hand a value on.  gh_submit
-// gives such a run to this kernel: every thread takes its vectors through all the steps, reads each tensor
+// gives such a run to this kernel: every thread takes its values through all the steps, reads each tensor
 // where it is first needed, keeps intermediate values in registers and LDS, and stores only what is still
 // there when the run ends - a tensor that a later step of the run overwrites is not stored twice.  The steps
 // apply the functions of gh_elem_fn.h in the order of the commands, so the stored bits are theirs.
 // Which commands make a run is decided by earns() and pays() below.
 //
 // Bound: HBM for large tensors (sigmoid, tanh and pow(., 2) of x * y + b on 4096 x 4096 float32: 336 MB instead
-// of 738, 66 us instead of 117), the launch for small ones (five launches become one: 12.5 us become 3).
+// of 738, 66 us instead of 117), for small ones the launch and a thread's walk from step to step (five launches become one).
 #include <algorithm>
 #include <cstring>
 
@@ -19,7 +19,6 @@
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kU = 2;         // vectors of 16 bytes per thread and pass
 constexpr int kMaxSteps = 8;
 constexpr int kSlots = 2;     // values kept past the step behind theirs
 
@@ -49,10 +48,9 @@ __device__ __forceinline__ uint32_t fast_div(uint32_t n, uint32_t mul, uint32_t 
   return sh ? (t + ((n - t) >> 1)) >> (sh - 1) : n;
 }
 
-template <class T, bool STREAM>
+template <class T, bool STREAM, int N>
 struct Lane {
-  typedef typename VecOf<T>::type V;
-  static constexpr int N = VecOf<T>::N;
+  typedef T V __attribute__((ext_vector_type(N)));
 
   // vector i of a tensor of n elements: the last one may be partial
   static __device__ __forceinline__ V load(const void* p, int64_t i, int64_t n) {
@@ -99,11 +97,15 @@ __device__ __attribute__((noinline)) T unary_call(T x) { return unary_apply<F>(x
 template <int F, class T>
 __device__ __attribute__((noinline)) T bin_call(T x, T y) { return bin_apply<F, T>(x, y); }
 
-template <class T, bool STREAM>
+template <class T, bool STREAM, int N, int kU>
 __global__ __launch_bounds__(kBlock) void k_chain(const Chain c) {
-  typedef Lane<T, STREAM> L;
+  typedef Lane<T, STREAM, N> L;
   typedef typename L::V V;
-  constexpr int N = L::N;
+  // the arguments' lines into the scalar cache, all at once: a step's own loads would each wait for theirs
+  uint32_t lines = 0;
+#pragma unroll
+  for (int l = 0; l < (int)(sizeof(Chain) / 64); l++) lines |= ((const uint32_t*)&c)[16 * l];
+  asm volatile("" ::"s"(lines));
   __shared__ V slots[kSlots][kU][kBlock];
   __shared__ V scratch[2][kBlock];
   const int64_t nv = (c.n + N - 1) / N;
@@ -407,12 +409,31 @@ int find_run(const gh_cmd* cmds, int n, Chain* c) {
   return count >= 2 ? count : 0;
 }
 
+template <class T, bool STREAM, int N, int U>
+void launch_as(gh_ctx* ctx, const Chain& c, int64_t most) {
+  const int64_t nv = (c.n + N - 1) / N, blocks = (nv + kBlock * U - 1) / (kBlock * U);
+  hipLaunchKernelGGL((k_chain<T, STREAM, N, U>), dim3((unsigned)std::min(blocks, most)), dim3(kBlock), 0, ctx->stream, c);
+}
+
+// A thread's share.  What a run of few elements takes is a thread's way through the steps, so as long as that leaves a compute
+// unit no more than five workgroups a thread has one element; above, one vector, and the whole run a launch of that many
+// workgroups.  The pow-free chain at the head of this file, us with the wait, two vectors a thread and at most sixteen
+// workgroups to a compute unit / as here: float32 1024 values 20.1 / 15.1, 131072 21.1 / 15.8, 262144 21.2 / 17.0, 524288
+// 17.8 / 17.0 (one element 19.8, one vector 19.5 where the power is no product), 2097152 21.6 / 20.8, 16777216 74.3 / 71.2,
+// 33554432 138 / 128.  float64 keeps two vectors and the bounded launch for tensors beyond 16 MiB (8388608 values 106, one
+// vector 114 to 124; 2097152 36 either way, 524288 21.4 / 20.0, 10001 20.0 / 15.6).
 template <class T>
 void launch(gh_ctx* ctx, const Chain& c, bool stream) {
-  const int64_t nv = (c.n + VecOf<T>::N - 1) / VecOf<T>::N;
-  const int64_t blocks = std::min<int64_t>((nv + kBlock * kU - 1) / (kBlock * kU), (int64_t)ctx->cu_count * 16);
-  if (stream) hipLaunchKernelGGL((k_chain<T, true>), dim3((int)blocks), dim3(kBlock), 0, ctx->stream, c);
-  else hipLaunchKernelGGL((k_chain<T, false>), dim3((int)blocks), dim3(kBlock), 0, ctx->stream, c);
+  constexpr int N = VecOf<T>::N;
+  if (c.n <= 5 * (int64_t)ctx->cu_count * kBlock) return launch_as<T, false, 1, 1>(ctx, c, INT32_MAX);
+  if constexpr (sizeof(T) == 8) {
+    const int64_t most = 16 * (int64_t)ctx->cu_count;
+    if (stream) return launch_as<T, true, N, 2>(ctx, c, most);
+    if (c.n * (int64_t)sizeof(T) > (16 << 20)) return launch_as<T, false, N, 2>(ctx, c, most);
+  } else if (stream) {
+    return launch_as<T, true, N, 1>(ctx, c, INT32_MAX);
+  }
+  launch_as<T, false, N, 1>(ctx, c, INT32_MAX);
 }
 
 }  // namespace

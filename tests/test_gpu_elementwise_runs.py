@@ -110,3 +110,21 @@ def test_random_runs(ctx, seed):
                 cmds.append(D.cmd_bin(fn, "vs", z, x + item * int(r.integers(n)), n, dtype=code))
         return cmds
     _same(_both(ctx, make, tensors))
+
+
+# the last size whose threads take one element each, the first of one vector each, tails of a vector; float64 past 16 MiB
+@pytest.mark.parametrize("dt,mid,rows", [("f32", 640, 512), ("f32", 641, 512), ("f32", 327683, 1), ("f64", 640, 512), ("f64", 327681, 1),
+                                         ("f64", 1048577, 2), ("f64", 2097153, 1)])
+def test_runs_around_a_threads_share(ctx, dt, mid, rows):
+    np_dt, code = (np.float32, _ffi.F32) if dt == "f32" else (np.float64, _ffi.F64)
+    n = rows * mid
+    heavy = ["exp", "softplus", "ln", "tanh"]
+
+    def make(p):
+        return [D.cmd_bin("mul", "vv", p["a"], p["b"], n, dtype=code, dst=p["c"]),
+                D.cmd_bcast("add", p["c"], p["c"], p["m"], rows, mid, 1, dtype=code),
+                D.cmd_unary(heavy[rows % 4], p["c"], n, dtype=code),
+                D.cmd_bin("pow", "vs", p["c"], p["s"], n, dtype=code, dst=p["a"]),
+                D.cmd_bin("sub", "vv", p["a"], p["b"], n, dtype=code, dst=p["d"]),
+                D.cmd_relu(p["d"], p["d"], n, dtype=code)]
+    _same(_both(ctx, make, _tensors(np.random.default_rng(n), (rows, mid), mid, np_dt)))
