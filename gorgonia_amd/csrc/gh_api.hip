@@ -519,6 +519,19 @@ static int submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
       i += run - 1;
       continue;
     }
+    // a filter gradient and the image gradient beside it, in one launch where a kernel has both
+    if (gh_gradient_pair(cmds + i, n - i)) {
+      if ((rc = gh_flush_sums_before(ctx, cmds[i + 1]))) return rc;
+      const bool first = cmds[i].opcode == GH_OP_CONV2D_BWD_FILTER;
+      ctx->hold_filter = true;
+      rc = dispatch(ctx, cmds[first ? i : i + 1]);
+      ctx->hold_filter = false;
+      if (!rc) rc = dispatch(ctx, cmds[first ? i + 1 : i]);
+      const int alone = gh_launch_held(ctx);
+      if (rc || alone) return rc ? rc : alone;
+      i++;
+      continue;
+    }
     // two commands of which the second reads what the first writes are one launch where a kernel takes both
     const bool held = gh_bn_held_pair(ctx, cmds + i, n - i), pair = held || gh_is_pair(cmds + i, n - i);
     if (pair && (rc = gh_flush_sums_before(ctx, cmds[i + 1]))) return rc;

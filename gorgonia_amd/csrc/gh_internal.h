@@ -56,6 +56,15 @@ struct gh_slab_sum {
   int64_t total;
   int slabs, how;
 };
+// A filter gradient whose launch waits for the image gradient beside it (k_conv_gradients.hip): which kernel, its grid, its
+// dynamic LDS and its argument.
+enum { kHeldNone, kHeldSmall, kHeldSmallNarrow, kHeldF32, kHeldF64, kHeldF64Narrow };
+struct gh_held_filter {
+  int kind = kHeldNone;
+  dim3 grid;
+  size_t lds = 0;
+  alignas(16) unsigned char args[192];
+};
 constexpr int kSlabSums = 8;
 constexpr int64_t kSlabSpace = 24ll << 20;
 
@@ -83,6 +92,8 @@ struct gh_ctx {
   gh_slab_sum sums[kSlabSums];
   int pending = 0;
   bool defer_sums = false;
+  bool hold_filter = false;   // the next filter gradient may be held
+  gh_held_filter held;
   // set while gh_submit_noalloc runs: the scratch is the library's fixed array and a
   // plan may not shrink to fit it (results must not depend on the scratch size)
   bool ws_strict = false;
@@ -173,6 +184,13 @@ bool gh_conv_wgrad_small_takes(const gh_cmd& c);
 bool gh_conv_wgrad_takes(const gh_cmd& c, int cus);
 int64_t gh_conv_wgrad_slab_limit(const gh_cmd& c, int64_t slab_bytes);
 int gh_launch_conv_wgrad(gh_ctx* ctx, const gh_cmd& c);
+// both gradients of a 3x3 convolution in one launch (k_conv_gradients.hip)
+bool gh_gradient_pair(const gh_cmd* cmds, int n);
+int gh_launch_held(gh_ctx* ctx);
+int gh_launch_held_wgrad(gh_ctx* ctx);         // k_conv_wgrad.hip
+int gh_launch_held_wgrad_small(gh_ctx* ctx);   // k_conv_wgrad_small.hip
+// whether a filter gradient that writes `out` (slabs, or the result itself) may be held: not where it uses the workspace
+static inline bool gh_may_hold(const gh_ctx* ctx, const void* out) { return ctx->hold_filter && out != ctx->workspace; }
 bool gh_conv_small_takes(const gh_cmd& c);
 bool gh_conv_small_can_pool(const gh_cmd& c);
 // its 32- and 64-channel kernel (k_conv_rows.hip), same conventions

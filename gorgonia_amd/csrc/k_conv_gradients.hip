@@ -1,0 +1,156 @@
+// A 3x3 convolution's filter gradient and its image gradient in one launch.
+//
+// The two read the same dy and neither reads what the other writes.  Each is some 12 to 20 us in a training step, of which its
+// matrix instructions are a third: first loads, the wavefronts' meeting, a last round of few workgroups.  Here the filter
+// gradient's workgroups, the longer ones, come first in the grid and the image gradient's behind them, so that one's waits run
+// under the other's instructions.  Both are the workgroups of the kernels they have alone (gh_conv_wgrad.h,
+// gh_conv_wgrad_small.h, gh_conv_lanes.h): the stored bits are theirs.
+//
+// Bound: the matrix instructions of both and, of small ones, the launch; where both kernels fill the device by themselves one
+// launch takes what two do.  us, slab sum included, apart / together: float32 128 x 32 x 14 x 14 -> 64 38.7 / 36.5, 128 x 64 x 7 x 7
+// -> 128 34.9 / 31.3, three times as many images 90.6 / 80.2 and 82.8 / 72.6, 8 x 64 x 26 x 26 -> 128 34.9 / 32.9, 8 x 16 x 52 x 52 -> 32
+// 23.4 / 19.3, 8 x 16 x 104 x 104 -> 32 34.5 / 33.8; float64 50 x 64 x 7 x 7 -> 128 31.0 / 28.1, 96 x 32 x 14 x 14 -> 64 47.1 / 40.3,
+// 8 x 32 x 26 x 26 -> 64 23.9 / 20.0.  Of 350 drawn shapes of 1 to 360 images of 4 x 4 to 110 x 110 (float64 to 32 x 32) none was
+// slower by more than 2.4 % and the 249 that a kernel here has both of took 0.85 of their time, so there is no rule but that.  (Registers
+// for a third workgroup to a compute unit, float64's by two meetings of half the LDS, spill and lose what they gain: 96 x 32 x 14 x 14
+// 48.7.  The float32 form that had two filter-gradient workgroups side by side in eight wavefronts spilled, 57 for 35.)
+//
+// gh_submit holds a filter gradient back (gh_held_filter) where an image gradient that has nothing to do with its result
+// stands beside it; the image gradient's launch takes it along, or it is launched by itself behind that.
+#include <algorithm>
+#include <cstdlib>
+#include <mutex>
+
+#include "gh_conv_lanes.h"
+#include "gh_conv_wgrad.h"
+#include "gh_conv_wgrad_small.h"
+
+namespace {
+
+using conv_lanes::Lanes;
+using conv_wgrad::Wg;
+
+// The filter gradient's grid: x, y and all workgroups.
+struct Grid {
+  int x, y, all;
+  __device__ __forceinline__ void at(int b, int* bx, int* by, int* bz) const {
+    const int r = b / x;
+    *bx = b - r * x;
+    *bz = r / y;
+    *by = r - *bz * y;
+  }
+};
+
+template <int kRowPitch, int TM>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_conv3x3_gradients_small(const gh_wgrad_small_args w, const Grid grid, const Lanes<float> g) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int b = (int)blockIdx.x;
+  if (b < grid.all) {
+    int bx, by, bz;
+    grid.at(b, &bx, &by, &bz);
+    conv_wgrad_small::workgroup<kRowPitch>(w.x, w.dy, w.out, w.g, w.slab, bx, by, bz, (float*)lds);
+  } else {
+    conv_lanes::workgroup<float, 8, TM, 4, 1, true, true, false>(g, ConvTail{}, b - grid.all, (int)gridDim.x - grid.all, lds);
+  }
+}
+
+// (Where the image gradient's workgroups have eight wavefronts, the filter gradient's use the first four of theirs.)
+template <class T, int TMW, int P, int WV, int TM, int V, bool kSplit>
+__global__ __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 2 : 3))) void k_conv3x3_gradients(const Wg<T> w, const Grid grid, const Lanes<T> g) {
+  constexpr int wl = conv_wgrad::lds_of<T, 9>(), ll = conv_lanes::lds_of<T, WV, TM, V, 1, kSplit>(true);
+  __shared__ __attribute__((aligned(16))) char lds[wl > ll ? wl : ll];
+  const int b = (int)blockIdx.x;
+  if (b < grid.all) {
+    if (WV > conv_wgrad::kWaves && (int)threadIdx.x >= conv_wgrad::kThreads) return;
+    int bx, by, bz;
+    grid.at(b, &bx, &by, &bz);
+    conv_wgrad::workgroup<T, TMW, P, 9, false>(w, bx, by, bz, lds);
+  } else {
+    conv_lanes::workgroup<T, WV, TM, V, 1, kSplit, true, false>(g, ConvTail{}, b - grid.all, (int)gridDim.x - grid.all, lds);
+  }
+}
+
+Grid grid_of(const gh_held_filter& h) { return {(int)h.grid.x, (int)h.grid.y, (int)(h.grid.x * h.grid.y * h.grid.z)}; }
+
+template <int kRowPitch, int TM>
+int go_small(gh_ctx* ctx, const Lanes<float>& g, int blocks) {
+  static std::once_flag once;
+  static hipError_t attr_rc = hipSuccess;
+  std::call_once(once, [] { attr_rc = hipFuncSetAttribute((const void*)k_conv3x3_gradients_small<kRowPitch, TM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); });
+  if (attr_rc != hipSuccess) return gh_check_hip(ctx, attr_rc, "hipFuncSetAttribute(conv3x3 gradients)");
+  const Grid grid = grid_of(ctx->held);
+  gh_wgrad_small_args w;
+  memcpy(&w, ctx->held.args, sizeof w);
+  const size_t lds = std::max<size_t>(ctx->held.lds, conv_lanes::lds_of<float, 8, TM, 4, 1, true>(true));
+  hipLaunchKernelGGL((k_conv3x3_gradients_small<kRowPitch, TM>), dim3((unsigned)(grid.all + blocks)), dim3(512), lds, ctx->stream, w, grid, g);
+  return GH_OK;
+}
+
+template <class T, int TMW, int P, int WV, int TM, int V, bool kSplit>
+int go(gh_ctx* ctx, const Lanes<T>& g, int blocks) {
+  const Grid grid = grid_of(ctx->held);
+  Wg<T> w;
+  memcpy(&w, ctx->held.args, sizeof w);
+  hipLaunchKernelGGL((k_conv3x3_gradients<T, TMW, P, WV, TM, V, kSplit>), dim3((unsigned)(grid.all + blocks)), dim3(WV * 64), 0, ctx->stream, w, grid, g);
+  return GH_OK;
+}
+
+int done(gh_ctx* ctx, int rc) {
+  ctx->held.kind = kHeldNone;
+  return rc ? rc : gh_check_hip(ctx, hipGetLastError(), "convolution gradients launch");
+}
+
+bool apart(uint64_t a, int64_t na, uint64_t b, int64_t nb) { return a + (uint64_t)na <= b || b + (uint64_t)nb <= a; }
+
+}  // namespace
+
+int gh_try_launch_gradients(gh_ctx* ctx, const conv_lanes::Lanes<float>& g, int waves, int tm, bool split, int blocks) {
+  using namespace conv_wgrad_small;
+  if ((waves == 8) != split || getenv("GORGONIA_HIP_CONV_APART")) return -1;   // tuning switch: a launch each
+  switch (ctx->held.kind) {
+    case kHeldSmall: return !split ? -1 : done(ctx, tm == 1 ? go_small<kWide, 1>(ctx, g, blocks) : go_small<kWide, 2>(ctx, g, blocks));
+    case kHeldSmallNarrow: return !split ? -1 : done(ctx, tm == 1 ? go_small<kNarrow, 1>(ctx, g, blocks) : go_small<kNarrow, 2>(ctx, g, blocks));
+    case kHeldF32:
+      if (split) return done(ctx, tm == 1 ? go<float, 2, 4, 8, 1, 4, true>(ctx, g, blocks) : go<float, 2, 4, 8, 2, 4, true>(ctx, g, blocks));
+      return done(ctx, tm == 1 ? go<float, 2, 4, 4, 1, 4, false>(ctx, g, blocks) : go<float, 2, 4, 4, 2, 4, false>(ctx, g, blocks));
+  }
+  return -1;
+}
+
+int gh_try_launch_gradients(gh_ctx* ctx, const conv_lanes::Lanes<double>& g, int waves, int tm, bool split, int blocks) {
+  if (waves != 4 || tm != 1 || !split || getenv("GORGONIA_HIP_CONV_APART")) return -1;
+  switch (ctx->held.kind) {
+    case kHeldF64: return done(ctx, go<double, 1, 4, 4, 1, 2, true>(ctx, g, blocks));
+    case kHeldF64Narrow: return done(ctx, go<double, 1, 2, 4, 1, 2, true>(ctx, g, blocks));
+  }
+  return -1;
+}
+
+// The filter gradient that no image gradient took along.
+int gh_launch_held(gh_ctx* ctx) {
+  if (ctx->held.kind == kHeldNone) return GH_OK;
+  const int rc = ctx->held.kind == kHeldSmall || ctx->held.kind == kHeldSmallNarrow ? gh_launch_held_wgrad_small(ctx) : gh_launch_held_wgrad(ctx);
+  ctx->held.kind = kHeldNone;
+  return rc;
+}
+
+// Whether cmds[0] and cmds[1] are the two gradients of 3x3 convolutions, in either order, and neither meets the other's result.
+// (The first command is a valid one.)
+bool gh_gradient_pair(const gh_cmd* cmds, int n) {
+  if (n < 2) return false;
+  const uint32_t a = cmds[0].opcode, b = cmds[1].opcode;
+  if (!(a == GH_OP_CONV2D_BWD_FILTER && b == GH_OP_CONV2D_BWD_DATA) && !(a == GH_OP_CONV2D_BWD_DATA && b == GH_OP_CONV2D_BWD_FILTER)) return false;
+  std::string m;
+  if (gh_validate_cmd(cmds[1], m) != GH_OK) return false;
+  const gh_cmd &f = a == GH_OP_CONV2D_BWD_FILTER ? cmds[0] : cmds[1], &d = a == GH_OP_CONV2D_BWD_FILTER ? cmds[1] : cmds[0];
+  if (f.dim[5] != 3 || f.dim[6] != 3 || d.dim[5] != 3 || d.dim[6] != 3 || gh_dtype_of(f.flags) != gh_dtype_of(d.flags)) return false;
+  const int64_t item = gh_dtype_of(f.flags) == GH_F64 ? 8 : 4;
+  auto x_of = [&](const gh_cmd& c) { return c.dim[0] * c.dim[1] * c.dim[2] * c.dim[3] * item; };
+  auto w_of = [&](const gh_cmd& c) { return c.dim[4] * c.dim[1] * 9 * item; };
+  auto y_of = [&](const gh_cmd& c) {
+    return c.dim[0] * c.dim[4] * gh_conv_out(c.dim[2], 3, c.dim[7], c.dim[9], c.dim[11]) * gh_conv_out(c.dim[3], 3, c.dim[8], c.dim[10], c.dim[12]) * item;
+  };
+  const uint64_t dw = f.ptr[2], dx = d.ptr[2];
+  return apart(dx, x_of(d), f.ptr[0], x_of(f)) && apart(dx, x_of(d), f.ptr[1], y_of(f)) && apart(dx, x_of(d), dw, w_of(f)) && apart(dw, w_of(f), d.ptr[0], y_of(d)) &&
+         apart(dw, w_of(f), d.ptr[1], w_of(d));
+}
