@@ -532,6 +532,15 @@ static int submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
       i++;
       continue;
     }
+    // and so with a dense layer's two gradients
+    if (gh_gemm_gradient_pair(cmds + i, n - i)) {
+      if ((rc = gh_flush_sums_before(ctx, cmds[i + 1]))) return rc;
+      if ((rc = gh_try_launch_gemm_gradients(ctx, cmds + i)) >= 0) {
+        if (rc) return rc;
+        i++;
+        continue;
+      }
+    }
     // two commands of which the second reads what the first writes are one launch where a kernel takes both
     const bool held = gh_bn_held_pair(ctx, cmds + i, n - i), pair = held || gh_is_pair(cmds + i, n - i);
     if (pair && (rc = gh_flush_sums_before(ctx, cmds[i + 1]))) return rc;

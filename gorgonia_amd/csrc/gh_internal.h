@@ -167,6 +167,12 @@ int gh_launch_gemm(gh_ctx* ctx, const gh_cmd& c);
 int gh_gemm_direct_form(const gh_cmd& c, int cus, double* us, int* rounds);   // -1: not taken
 int gh_gemm_direct_slices(const gh_cmd& c, int form, int cus);
 int gh_launch_gemm_direct(gh_ctx* ctx, const gh_cmd& c, int form);
+// a dense layer's two gradients in one launch (k_gemm_gradients.hip)
+enum { kGemmOther, kGemmDirect, kGemmSkinny };
+struct gh_gemm_choice { int kind = kGemmOther, form = 0, waves = 0, columns = 0; };   // form: k_gemm_direct's; waves, columns: the small-output kernels'; waves: float32 k_gemm_direct's that share K
+gh_gemm_choice gh_choose_gemm(const gh_ctx* ctx, const gh_cmd& c);
+bool gh_gemm_gradient_pair(const gh_cmd* cmds, int n);
+int gh_try_launch_gemm_gradients(gh_ctx* ctx, const gh_cmd* cmds);   // -1: no kernel has both
 // float32 products on the bf16 matrix instructions (k_gemm_split.hip)
 int gh_gemm_split_form(const gh_cmd& c, int cus, double other_us, int other_slices);   // -1: not taken; the other kernel's time and its slices of K
 int gh_launch_gemm_split(gh_ctx* ctx, const gh_cmd& c, int form);

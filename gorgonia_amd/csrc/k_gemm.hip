@@ -26,6 +26,7 @@
 
 #include "gh_internal.h"
 #include "gh_conv_common.h"
+#include "gh_gemm_skinny.h"
 
 namespace {
 
@@ -648,185 +649,12 @@ __global__ __launch_bounds__(WV * 64) void k_gemm_skinny(const float* __restrict
   }
 }
 
-// ---- small-output GEMM on 16-row tiles -----------------------------------------------
-// A compute unit keeps only so many cache lines in flight, which holds one
-// workgroup to ~40 GB/s of operand fill however its loads are written (measured
-// on the 32x32 kernel above), so a product whose 32x32 tiles cover a fraction of
-// the chip is bounded by the number of compute units it touches.  This kernel
-// cuts the output into tiles of 16 rows by 16*NT columns (two to four times as
-// many workgroups) on the 16x16x4 MFMA; the K split over the wavefronts of a
-// block and the fixed-order sum of their partial tiles are those of
-// k_gemm_skinny.  Lane l = (i = l % 16, q = l / 16) owns k = 16*chunk + 4*q + t
-// at MFMA step t: its four A values are one 128-bit load of row i, already in
-// MFMA order; of B it takes, per k, the NT adjacent columns n0 + NT*i + c (one
-// load of NT floats; with NT = 2 sixteen lanes cover one whole 128-byte line)
-// and column set c feeds accumulator c.  The last tile in each direction is
-// moved back to end at the matrix edge (M >= 16, N >= 16*NT), so no row or
-// column is ever masked; k past K is clamped in the address and zeroed before
-// the MFMA.
-// TA / TB: the operand is a transposed view (A stored k x m, B stored n x k, as
-// for k_sgemm); the lane's four k-values are then four loads for A and one
-// 128-bit load for B instead of the other way round.  N < 16 (NT = 1 only;
-// transposed views alone reach here with so few columns): one column tile,
-// column indices clamped in the loads and masked in the store.
+// ---- small-output GEMM on 16-row tiles (gh_gemm_skinny.h) ------------------------------
 template <int WV, int NT, bool TA, bool TB>
-__global__ __launch_bounds__(WV * 64) void k_gemm_skinny16(const float* __restrict__ A,
-                                                           const float* __restrict__ B,
-                                                           float* __restrict__ C, int M, int N, int K,
-                                                           int lda, int ldb, int ldc, int act, float alpha,
-                                                           const float* __restrict__ bias, int softmax) {
-  constexpr int G = NT == 1 ? 5 : 4;
-  constexpr int BN = 16 * NT, TILE = 16 * BN;
-  typedef float bvec __attribute__((ext_vector_type(NT), aligned(4)));
-  __shared__ float part[WV * TILE];
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int i = lane & 15, q = lane >> 4;
-  const bool ragged_n = N < BN;
-  // Workgroup ids are dealt round-robin over the 8 XCDs, each with its own L2.
-  // Regroup them so that one XCD gets a contiguous run of ids, and walk a run
-  // row-tile fastest: every row tile of a column tile then reads that strip of
-  // B (the weights, the big operand of a dense layer) through the same L2, once
-  // from memory, instead of once per XCD.
-  int tile_x, tile_y;
-  {
-    const int gx = gridDim.x, gy = gridDim.y, total = gx * gy;
-    const int id = blockIdx.y * gx + blockIdx.x;
-    const int xcd = id & 7, per = total >> 3, extra = total & 7;
-    const int nid = xcd * per + min(xcd, extra) + (id >> 3);
-    tile_x = nid / gy;
-    tile_y = nid - tile_x * gy;
-  }
-  const int m0 = min(tile_y * 16, M - 16), n0 = ragged_n ? 0 : min(tile_x * BN, N - BN);
-  const int all_chunks = (K + 15) / 16, per = (all_chunks + (int)gridDim.z - 1) / (int)gridDim.z;
-  const int chunk0 = (int)blockIdx.z * per, nchunks = min(all_chunks, chunk0 + per);   // as in k_gemm_skinny
-  C += (int64_t)blockIdx.z * M * N;
-  int ncol[NT];   // this lane's columns (clamped when the tile is wider than the matrix)
-#pragma unroll
-  for (int c = 0; c < NT; c++) ncol[c] = min(n0 + NT * i + c, N - 1);
-  // k runs along the row of an untransposed A and of a transposed B
-  const float* const a_base = TA ? A + m0 + i : A + (int64_t)(m0 + i) * lda;
-  // The lane's quad of chunk `chunk` starts at k0 = 16*chunk + 4*q; a quad that
-  // would stick out past K starts at K-4 instead, and its elements below k0
-  // (which the quad before it already covers) are zeroed before the MFMA.  So
-  // element t always stands for k = kb + t with kb = min(k0, K-4): every load is
-  // unconditional, k-contiguous operands are one 128-bit load at any 4-byte
-  // aligned address, and no loaded value is touched under a branch (which would
-  // make each load wait for the one before it).
-  auto load_k4 = [&](const float* row, int kb, float (&dst)[4]) {
-    const f32x4 v = *reinterpret_cast<const f32x4_a4*>(row + kb);
-#pragma unroll
-    for (int t = 0; t < 4; t++) dst[t] = v[t];
-  };
-  auto load = [&](int chunk, float (&a)[4], float (&b)[4][NT]) {
-    const int kb = min(chunk * 16 + 4 * q, K - 4);
-    if constexpr (TA) {
-#pragma unroll
-      for (int t = 0; t < 4; t++) a[t] = a_base[(int64_t)(kb + t) * lda];
-    } else {
-      load_k4(a_base, kb, a);
-    }
-    if constexpr (TB) {
-#pragma unroll
-      for (int c = 0; c < NT; c++) {
-        float col[4];
-        load_k4(B + (int64_t)ncol[c] * ldb, kb, col);
-#pragma unroll
-        for (int t = 0; t < 4; t++) b[t][c] = col[t];
-      }
-    } else {
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const float* src = B + (int64_t)(kb + t) * ldb;
-        if constexpr (NT == 1) {
-          b[t][0] = src[ncol[0]];
-        } else {
-          const bvec v = *reinterpret_cast<const bvec*>(src + ncol[0]);
-#pragma unroll
-          for (int c = 0; c < NT; c++) b[t][c] = v[c];
-        }
-      }
-    }
-  };
-  auto load_group = [&](int c, float (&a)[G][4], float (&b)[G][4][NT]) {
-#pragma unroll
-    for (int g = 0; g < G; g++)
-      if (c + g * WV < nchunks) load(c + g * WV, a[g], b[g]);
-  };
-  f32x4 acc[NT];
-#pragma unroll
-  for (int c = 0; c < NT; c++) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto mfma_group = [&](int c, float (&a)[G][4], float (&b)[G][4][NT]) {
-#pragma unroll
-    for (int g = 0; g < G; g++)
-      if (c + g * WV < nchunks) {
-        const int k0 = (c + g * WV) * 16 + 4 * q;
-        const int first = k0 - min(k0, K - 4);   // elements below this index belong to the quad before
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-          const float av = t >= first ? a[g][t] : 0.f;
-#pragma unroll
-          for (int cs = 0; cs < NT; cs++) {
-            const float bv = t >= first ? b[g][t][cs] : 0.f;
-            acc[cs] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc[cs], 0, 0, 0);
-          }
-        }
-      }
-  };
-  float a0[G][4], b0[G][4][NT], a1[G][4], b1[G][4][NT];
-  int c0 = chunk0 + wave;
-  if (c0 < nchunks) load_group(c0, a0, b0);
-  while (c0 < nchunks) {
-    const int c1 = c0 + G * WV;
-    if (c1 < nchunks) load_group(c1, a1, b1);
-    mfma_group(c0, a0, b0);
-    if (c1 >= nchunks) break;
-    c0 = c1 + G * WV;
-    if (c0 < nchunks) load_group(c0, a0, b0);
-    mfma_group(c1, a1, b1);
-  }
-  // element v of accumulator c in lane (i, q) is C[m0 + 4*q + v][n0 + NT*i + c]
-#pragma unroll
-  for (int c = 0; c < NT; c++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) part[wave * TILE + (4 * q + v) * BN + NT * i + c] = acc[c][v];
-  __syncthreads();
-  if (NT == 1 && softmax) {
-    // Row softmax (N <= 16: the one column tile holds whole rows) with the
-    // arithmetic of the softmax kernel: max, exp(x - max) in float64 rounded
-    // once, the sum taken in column order, one rounded reciprocal.
-    __shared__ float sm_x[16 * 17], sm_e[16 * 17];
-    const int e = threadIdx.x, row = (e >> 4) & 15, col = e & 15;
-    if (e < TILE) {
-      float sum = part[e];
-#pragma unroll
-      for (int w = 1; w < WV; w++) sum = sum + part[w * TILE + e];
-      if (bias && col < N) sum = sum + bias[col];
-      sm_x[row * 17 + col] = act_apply(sum, act, alpha);
-    }
-    __syncthreads();
-    if (e < TILE) {
-      float mx = -INFINITY;
-      for (int j = 0; j < N; j++) mx = fmaxf(mx, sm_x[row * 17 + j]);
-      sm_e[row * 17 + col] = col < N ? (float)exp((double)(sm_x[row * 17 + col] - mx)) : 0.f;
-    }
-    __syncthreads();
-    if (e < TILE && col < N) {
-      float sum = 0.f;
-      for (int j = 0; j < N; j++) sum = sum + sm_e[row * 17 + j];
-      const float inv = 1.0f / sum;
-      C[(int64_t)(m0 + row) * ldc + col] = sm_e[row * 17 + col] * inv;
-    }
-    return;
-  }
-  for (int e = threadIdx.x; e < TILE; e += WV * 64) {
-    float sum = part[e];
-#pragma unroll
-    for (int w = 1; w < WV; w++) sum = sum + part[w * TILE + e];
-    const int col = n0 + e % BN;
-    if (col >= N) continue;
-    if (bias) sum = sum + bias[col];
-    C[(int64_t)(m0 + e / BN) * ldc + col] = act_apply(sum, act, alpha);
-  }
+__global__ __launch_bounds__(WV * 64) void k_gemm_skinny16(const gemm_skinny::Args32 g) {
+  __shared__ __attribute__((aligned(16))) char lds[gemm_skinny::lds16<WV, NT>()];
+  gemm_skinny::workgroup16<WV, NT, TA, TB, false>(g, (int)(blockIdx.y * gridDim.x + blockIdx.x), (int)gridDim.x, (int)gridDim.y, (int)blockIdx.z,
+                                                  (int)gridDim.z, lds);
 }
 
 // Adds the slabs of a small-output product cut along K, in slab order, and applies the epilogue: bias, activation,
@@ -1599,96 +1427,11 @@ __global__ __launch_bounds__(kThreads) void k_dgemm(const double* __restrict__ A
       }
 }
 
-// Float64 product with a small result (a dense layer on a batch: too few 64x64
-// tiles to occupy the device, and a k loop of a thousand steps behind each).
-// One workgroup per 16x16 tile of C, its WV wavefronts each summing a slice of
-// K straight from global memory into one MFMA accumulator (element (i, k) of
-// op(A) at A[i*sai + k*sak], (k, j) of op(B) at B[k*sbk + j*sbj], so every
-// transpose is the same code); loads are unconditional at clamped addresses and
-// masked afterwards, so they all stay in flight.  The slices are added in LDS in
-// wavefront order: the result does not depend on scheduling.
+// Float64, one 16x16 tile per workgroup (gh_gemm_skinny.h)
 template <int WV, bool AV, bool BV>
-__global__ __launch_bounds__(WV * 64) void k_dgemm_skinny(const double* __restrict__ A,
-                                                          const double* __restrict__ B,
-                                                          double* __restrict__ C, int M, int N, int K,
-                                                          int64_t sai, int64_t sak, int64_t sbk,
-                                                          int64_t sbj, int ldc, int64_t sA, int64_t sB, int64_t sC) {
-  A += blockIdx.z * sA; B += blockIdx.z * sB; C += blockIdx.z * sC;
-  __shared__ double part[WV][256];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int lr = lane & 15, lk = lane >> 4;
-  const int m0 = blockIdx.y * 16, n0 = blockIdx.x * 16;
-  const double* ap = A + (int64_t)min(m0 + lr, M - 1) * sai;
-  const double* bp = B + (int64_t)min(n0 + lr, N - 1) * sbj;
-  const int kper = (((K + WV - 1) / WV) + 7) & ~7;
-  const int k0 = wave * kper, k1 = min(K, k0 + kper);
-  f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-  if constexpr (AV || BV) {
-    // An operand that is k-contiguous: a lane fetches two consecutive k of its row or column in one load (the
-    // sixteen k of a step are then two 64-byte pieces instead of sixteen 8-byte ones; 8-byte alignment is all
-    // the load needs); which k a lane group multiplies in which MFMA is the same for both operands -
-    // k0 + 8 u + 2 lk + e.  The pair that would start at the last k of an odd K starts one earlier and is
-    // shifted into place.
-    for (int k = k0; k < k1; k += 16) {
-      f64x2 a[2], b[2];
-#pragma unroll
-      for (int u = 0; u < 2; u++) {
-        const int kk = k + 8 * u + 2 * lk;
-        const bool last = kk > K - 2;   // kk == K - 1 (its second k does not exist), or past the end (masked below)
-        if constexpr (AV) {
-          const f64x2 v = *reinterpret_cast<const f64x2_a8*>(ap + min(kk, K - 2));
-          a[u] = last ? f64x2{v[1], 0.0} : v;
-        }
-        if constexpr (BV) {
-          const f64x2 v = *reinterpret_cast<const f64x2_a8*>(bp + min(kk, K - 2));
-          b[u] = last ? f64x2{v[1], 0.0} : v;
-        }
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-          if constexpr (!AV) a[u][e] = ap[(int64_t)min(kk + e, K - 1) * sak];
-          if constexpr (!BV) b[u][e] = bp[(int64_t)min(kk + e, K - 1) * sbk];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 2; u++)
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-          const bool ok = k + 8 * u + 2 * lk + e < k1;
-          const double av = ok ? a[u][e] : 0.0, bv = ok ? b[u][e] : 0.0;
-          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc, 0, 0, 0);
-        }
-    }
-  } else {
-    for (int k = k0; k < k1; k += 16) {
-      double a[4], b[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int kc = min(k + 4 * u + lk, K - 1);
-        a[u] = ap[kc * sak];
-        b[u] = bp[kc * sbk];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const bool ok = k + 4 * u + lk < k1;
-        a[u] = ok ? a[u] : 0.0;
-        b[u] = ok ? b[u] : 0.0;
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b[u], acc, 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int v = 0; v < 4; v++) part[wave][v * 64 + lane] = acc[v];
-  __syncthreads();
-  if (wave == 0) {
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      double sum = part[0][v * 64 + lane];
-      for (int w = 1; w < WV; w++) sum = sum + part[w][v * 64 + lane];
-      const int i = m0 + 4 * v + lk, j = n0 + lr;
-      if (i < M && j < N) C[(int64_t)i * ldc + j] = sum;
-    }
-  }
+__global__ __launch_bounds__(WV * 64) void k_dgemm_skinny(const gemm_skinny::Args64 g) {
+  __shared__ __attribute__((aligned(16))) char lds[gemm_skinny::lds64<WV>()];
+  gemm_skinny::workgroup64<WV, AV, BV>(g, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, lds);
 }
 
 // ---- float64 Conv2d as an implicit GEMM on the matrix cores ---------------------------
@@ -2826,6 +2569,22 @@ static int try_launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c) {
   return gh_check_hip(ctx, hipGetLastError(), "skinny gemm slab sum launch");
 }
 
+// The 16-row kernel's wavefronts and tiles of 16 columns.
+struct Skinny16 { int waves, columns; };
+static Skinny16 skinny16_form(const gh_cmd& c, int cus) {
+  // 16x32 tiles read whole 128-byte lines of B; when even those leave half the
+  // chip without a tile, 16x16 (measured on MI355X, 8 wavefronts per block:
+  // 128x625x1152 11.0 us on 32x32, 8.4 on 16x32, 9.8 on 16x16; 64x1000x4096
+  // 33 / 21.8 / 19.5 us)
+  const char* force = force_tile();
+  const bool narrow = c.dim[1] < 32 || (force ? !strcmp(force, "16x16") : cdiv(c.dim[0], 16) * cdiv(c.dim[1], 32) * 2 <= cus);
+  // Sixteen wavefronts share the K of a long contraction (a function of the shape alone, like the tile): each
+  // wavefront's chain of grouped loads is half as long (measured: 128x1152x625 7.8 -> 7.2 us, 256x784x300
+  // 5.8 -> 5.3, 128x625x10 4.3 -> 4.1; nothing below K = 512, where a wavefront has four chunks or fewer).
+  static const bool no16 = getenv("GORGONIA_HIP_SKINNY_WAVES8") != nullptr;   // tuning switch
+  return {c.dim[2] >= 512 && !no16 ? 16 : 8, narrow ? 1 : 2};
+}
+
 static int launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c, int slices) {
   const bool ta = c.flags & GH_FLAG_TRANS_A, tb = c.flags & GH_FLAG_TRANS_B;
   const int M = (int)c.dim[0], N = (int)c.dim[1], K = (int)c.dim[2];
@@ -2848,24 +2607,14 @@ static int launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c, int slices) {
   const bool transposed = ta || tb;
   const bool tiles16 = N <= 16 || (N > 32 && tiles * 2 <= ctx->cu_count);
   if (transposed || (M >= 16 && tiles16 && !(force && !strcmp(force, "32")))) {
-    // 16x32 tiles read whole 128-byte lines of B; when even those leave half the
-    // chip without a tile, 16x16 (measured on MI355X, 8 wavefronts per block:
-    // 128x625x1152 11.0 us on 32x32, 8.4 on 16x32, 9.8 on 16x16; 64x1000x4096
-    // 33 / 21.8 / 19.5 us)
-    const int64_t blocks_wide = cdiv(M, 16) * cdiv(N, 32);
-    const bool narrow = N < 32 || (force ? !strcmp(force, "16x16") : blocks_wide * 2 <= ctx->cu_count);
+    const Skinny16 f = skinny16_form(c, ctx->cu_count);
+    const bool narrow = f.columns == 1, wide16 = f.waves == 16;
+    const gemm_skinny::Args32 g = gemm_skinny::args32_of(c);
     auto launch16 = [&](auto kernel, int bn) {
-      hipLaunchKernelGGL(kernel, dim3((N + bn - 1) / bn, (M + 15) / 16, slices), dim3(WV * 64), 0, ctx->stream, A, B, C, M,
-                         N, K, lda, ldb, ldc, act, c.f[0], bias, softmax);
+      hipLaunchKernelGGL(kernel, dim3((N + bn - 1) / bn, (M + 15) / 16, slices), dim3(WV * 64), 0, ctx->stream, g);
     };
-    // Sixteen wavefronts share the K of a long contraction (a function of the shape alone, like the tile): each
-    // wavefront's chain of grouped loads is half as long (measured: 128x1152x625 7.8 -> 7.2 us, 256x784x300
-    // 5.8 -> 5.3, 128x625x10 4.3 -> 4.1; nothing below K = 512, where a wavefront has four chunks or fewer).
-    static const bool no16 = getenv("GORGONIA_HIP_SKINNY_WAVES8") != nullptr;   // tuning switch
-    const bool wide16 = K >= 512 && !no16;
     auto launch16w = [&](auto kernel, int bn) {
-      hipLaunchKernelGGL(kernel, dim3((N + bn - 1) / bn, (M + 15) / 16, slices), dim3(16 * 64), 0, ctx->stream, A, B, C, M,
-                         N, K, lda, ldb, ldc, act, c.f[0], bias, softmax);
+      hipLaunchKernelGGL(kernel, dim3((N + bn - 1) / bn, (M + 15) / 16, slices), dim3(16 * 64), 0, ctx->stream, g);
     };
 #define GH_SKINNY16(TA_, TB_)                                                               \
   do {                                                                                      \
@@ -3066,24 +2815,19 @@ static void launch_dgemm_cfg(gh_ctx* ctx, const gh_cmd& c, int64_t batch) {
 #undef GH_DGEMM_GO
 }
 
+static bool skinny64_pairs(const gh_cmd& c) { return c.dim[2] >= 2 && !getenv("GORGONIA_HIP_DGEMM_SKINNY_SCALAR"); }   // (tuning switch)
+
 // Float64: one 16x16 tile per workgroup (k_dgemm_skinny).  AV, BV: the operand is k-contiguous.
 static int launch_dgemm_skinny(gh_ctx* ctx, const gh_cmd& c) {
   const int M = (int)c.dim[0], N = (int)c.dim[1], K = (int)c.dim[2];
-  const int64_t batch = c.dim[6] <= 0 ? 1 : c.dim[6];
   const bool ta = c.flags & GH_FLAG_TRANS_A, tb = c.flags & GH_FLAG_TRANS_B;
-  const int64_t lda = c.dim[3], ldb = c.dim[4];
-  const int64_t sA = batch > 1 ? c.dim[7] : 0, sB = batch > 1 ? c.dim[8] : 0, sC = batch > 1 ? c.dim[9] : 0;
-  const dim3 grid((N + 15) / 16, (M + 15) / 16, (unsigned)batch);
-  const double* A = (const double*)(uintptr_t)c.ptr[0];
-  const double* B = (const double*)(uintptr_t)c.ptr[1];
-  double* C = (double*)(uintptr_t)c.ptr[2];
+  const dim3 grid((N + 15) / 16, (M + 15) / 16, (unsigned)std::max<int64_t>(1, c.dim[6]));
+  const gemm_skinny::Args64 g = gemm_skinny::args64_of(c);
   // (which wavefront sums which k, and with AV which k shares an MFMA, depends on the shape and the operands'
   // layout only: a product's bits repeat from run to run)
-  const bool pairs = K >= 2 && !getenv("GORGONIA_HIP_DGEMM_SKINNY_SCALAR");   // (tuning switch)
+  const bool pairs = skinny64_pairs(c);
   const bool av = pairs && !ta, bv = pairs && tb;
-#define GH_DSK(WV_, AV_, BV_)                                                                                          \
-  hipLaunchKernelGGL((k_dgemm_skinny<WV_, AV_, BV_>), grid, dim3(WV_ * 64), 0, ctx->stream, A, B, C, M, N, K,           \
-                     ta ? 1 : lda, ta ? lda : 1, tb ? 1 : ldb, tb ? ldb : 1, (int)c.dim[5], sA, sB, sC)
+#define GH_DSK(WV_, AV_, BV_) hipLaunchKernelGGL((k_dgemm_skinny<WV_, AV_, BV_>), grid, dim3(WV_ * 64), 0, ctx->stream, g)
 #define GH_DSK_W(WV_)                                            \
   do {                                                           \
     if (av && bv) GH_DSK(WV_, true, true);                       \
@@ -3221,6 +2965,28 @@ int gh_launch_gemm(gh_ctx* ctx, const gh_cmd& c) {
   if (p.tile == kTile128) return launch_sgemm_cfg<128, 128, 2>(ctx, c, p.splits);
   if (p.tile == kTile128x64) return launch_sgemm_cfg<128, 64, 2>(ctx, c, p.splits);
   return launch_sgemm_cfg<64, 64, 2>(ctx, c, p.splits);
+}
+
+// The choice of gh_launch_gemm where it is a kernel that k_gemm_gradients.hip has beside another, for a transposed view of one
+// operand and nothing behind the product.
+gh_gemm_choice gh_choose_gemm(const gh_ctx* ctx, const gh_cmd& c) {
+  const int cus = ctx->cu_count;
+  if (gh_dtype_of(c.flags) == GH_F64) {
+    const int form = gemm64_form(c, cus);
+    if (form == kStaged64) return {};
+    if (form >= 0) return {kGemmDirect, form, 0, 0};
+    if (!skinny64_pairs(c)) return {};
+    return {kGemmSkinny, 0, c.dim[2] >= 256 ? 8 : 4, 1};
+  }
+  if (gemm_skinny_takes(c, cus)) {
+    if (skinny_slices(c, cus) > 1) return {};
+    const Skinny16 f = skinny16_form(c, cus);
+    return {kGemmSkinny, 0, f.waves, f.columns};
+  }
+  if (split_form(c, cus) >= 0) return {};
+  const int form = direct_form(c, cus);
+  if (form < 0) return {};
+  return {kGemmDirect, form, gh_gemm_direct_slices(c, form, cus), 0};
 }
 
 // The choices of gh_launch_gemm for a float32 product, asked without launching (MI355X's

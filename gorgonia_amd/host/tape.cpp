@@ -1005,15 +1005,19 @@ Status TapeMachine::Compile() {
     reg_last[(size_t)r] = std::max(reg_last[(size_t)r], std::max(i, last_reader[(size_t)root[(size_t)i]]));
     if (value_kept[(size_t)root[(size_t)i]]) reg_kept[(size_t)r] = 1;
   }
-  // The two gradients of a convolution, one behind the other, run in one launch where neither's result lies in what the
-  // other reads: what dies with the first is kept until the second is done.
+  // The two gradients of a convolution or of a dense layer, one behind the other, run in one launch where neither's result
+  // lies in what the other reads: what dies with the first is kept until the second is done.
   if (!opt_.node_at_a_time) {
     int before = -1;
     for (int i = 0; i < N; i++) {
       const Node& n = nodes[(size_t)i];
       if (n.fused_away || n.is_input || n.deferred || (n.alias_of >= 0 && n.op.kind != OpKind::Set && n.op.kind != OpKind::SolverStep)) continue;
-      const OpKind first = before >= 0 ? nodes[(size_t)before].op.kind : OpKind::Set, second = n.op.kind;
-      if ((first == OpKind::Conv2dDiffFilter && second == OpKind::Conv2dDiffData) || (first == OpKind::Conv2dDiffData && second == OpKind::Conv2dDiffFilter))
+      const auto &second = n.op, &first = before >= 0 ? nodes[(size_t)before].op : second;
+      const bool convolution = (first.kind == OpKind::Conv2dDiffFilter && second.kind == OpKind::Conv2dDiffData) ||
+                               (first.kind == OpKind::Conv2dDiffData && second.kind == OpKind::Conv2dDiffFilter);
+      const bool dense = first.kind == OpKind::MatMul && second.kind == OpKind::MatMul && first.transA != first.transB &&
+                         second.transA == first.transB && second.transB == first.transA;
+      if (convolution || dense)
         for (int& last : reg_last)
           if (last == before) last = i;
       before = i;
