@@ -502,6 +502,18 @@ static int submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
     std::string m;
     int rc = gh_validate_cmd(cmds[i], m);
     if (rc) return gh_fail(ctx, rc, "cmd " + std::to_string(i) + ": " + m);
+    // solver steps take the sums that wait along where they are their gradients
+    if (ctx->pending && cmds[i].opcode == GH_OP_SOLVER_STEP) {
+      const int steps = gh_solver_run_length(cmds + i, n - i);
+      const bool copy = gh_solver_copy_rides(cmds + i, steps, n - i);
+      bool valid = true;
+      for (int j = 1; j < steps + copy; j++) valid = valid && gh_validate_cmd(cmds[i + j], m) == GH_OK;
+      if (valid && (rc = gh_try_launch_solver_sums(ctx, cmds + i, steps, copy)) >= 0) {
+        if (rc) return rc;
+        i += steps + copy - 1;
+        continue;
+      }
+    }
     if ((rc = gh_flush_sums_before(ctx, cmds[i]))) return rc;
     // a run of solver steps with the same settings (a model's weight tensors) is one launch, and so is a run of
     // elementwise commands on tensors of one size

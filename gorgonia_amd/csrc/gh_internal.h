@@ -154,7 +154,6 @@ int gh_launch_dropout_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_dropout_bwd_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_softmax_bwd_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_maxpool2d_bwd_f64(gh_ctx* ctx, const gh_cmd& c);
-int gh_launch_solver_steps_f64(gh_ctx* ctx, const gh_cmd* cmds, int count, bool copy);
 int gh_launch_bn_train_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_bn_bwd_f64(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_conv2d_bwd_data_f64(gh_ctx* ctx, const gh_cmd& c);
@@ -237,6 +236,7 @@ int gh_launch_softmax_bwd(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_solver_step(gh_ctx* ctx, const gh_cmd& c);
 int gh_solver_run_length(const gh_cmd* cmds, int n);
 int gh_launch_solver_steps(gh_ctx* ctx, const gh_cmd* cmds, int count, bool copy);   // copy: cmds[count] rides along
+int gh_try_launch_solver_sums(gh_ctx* ctx, const gh_cmd* cmds, int count, bool copy);   // with the sums that wait; -1: not together
 // whether the command behind a run of `count` solver steps is a small copy that has nothing to do with their tensors
 bool gh_solver_copy_rides(const gh_cmd* cmds, int count, int n);
 // a copy of words by the workgroups behind a launch's own

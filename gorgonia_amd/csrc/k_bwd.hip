@@ -427,98 +427,6 @@ __global__ __launch_bounds__(kBlock) void k_softmax_bwd(const float* __restrict_
   }
 }
 
-// ---- solver steps ---------------------------------------------------------------------
-// One fused pass per tensor instead of the reference's 6-15 tensor ops
-// (solvers.go:273-372, 461-640, 780-870); every intermediate is rounded where
-// a tensor op of the reference would round it, so the weights and caches get
-// the reference's bits.
-struct SolverPar { float eta, eps, l1reg, l2reg, clip, one_per_batch, a, b, corr1, corr2; };
-
-__device__ __forceinline__ float clampf(float v, float lo, float hi) { return v < lo ? lo : (v > hi ? hi : v); }
-
-__device__ __forceinline__ float prep_grad(float g, float w, int use, const SolverPar& p) {
-  if (use & 1) { const float t = p.l1reg * (float)((w > 0.0f) - (w < 0.0f)); g = g + t; }
-  if (use & 2) { const float t = w * p.l2reg; g = g + t; }
-  if (use & 8) g = g * p.one_per_batch;
-  if ((use & 4) && p.clip > 0.0f) g = clampf(g, -p.clip, p.clip);
-  return g;
-}
-
-// Up to kSolverBatch weight tensors per launch: a model's solver steps are many
-// small tensors, and one launch per tensor costs more than the arithmetic.
-// Tensor t owns workgroups [first[t], first[t + 1]).
-constexpr int kSolverBatch = 8;
-struct SolverBatch {
-  float* w[kSolverBatch]; const float* g[kSolverBatch]; float* c1[kSolverBatch]; float* c2[kSolverBatch];
-  int64_t n[kSolverBatch];
-  int first[kSolverBatch + 1];
-  int count;
-};
-
-template <int KIND>
-__global__ __launch_bounds__(kBlock) void k_solver_step(SolverBatch sb, int use, SolverPar p,
-                                                        const float* __restrict__ corr, gh_small_copy copy) {
-  if ((int)blockIdx.x >= sb.first[kSolverBatch]) {
-    const int i = ((int)blockIdx.x - sb.first[kSolverBatch]) * kBlock + (int)threadIdx.x;
-    if (i < copy.words) copy.dst[i] = copy.src[i];
-    return;
-  }
-  // Adam's two bias corrections from device memory when the command names it: they change
-  // every step, and as command constants they would make every step a new command
-  if (KIND == GH_SOLVER_ADAM && corr) { p.corr1 = corr[0]; p.corr2 = corr[1]; }
-  int t = 0;
-#pragma unroll
-  for (int q = 1; q < kSolverBatch; q++)
-    if (q < sb.count && (int)blockIdx.x >= sb.first[q]) t = q;
-  float* __restrict__ w = sb.w[t];
-  const float* __restrict__ g = sb.g[t];
-  float* __restrict__ c1 = sb.c1[t];
-  float* __restrict__ c2 = sb.c2[t];
-  const int64_t n = sb.n[t];
-  const int64_t nblk = sb.first[t + 1] - sb.first[t];
-  const float neg_eta = -p.eta;
-  for (int64_t i = (int64_t)(blockIdx.x - sb.first[t]) * kBlock + threadIdx.x; i < n; i += nblk * kBlock) {
-    if (KIND == GH_SOLVER_VANILLA) {
-      float gi = prep_grad(g[i], w[i], use, p);
-      gi = gi * neg_eta;
-      w[i] = w[i] + gi;
-    } else if (KIND == GH_SOLVER_RMSPROP) {
-      float gi = g[i];
-      float gt2 = gi * gi;
-      float cw = c1[i] * p.a;
-      gt2 = gt2 * p.b;
-      cw = cw + gt2;
-      c1[i] = cw;
-      if (use & 4) gi = clampf(gi, -p.clip, p.clip);
-      float upd = cw + p.eps;
-      upd = 1.0f / sqrtf(upd);
-      gi = gi * neg_eta;
-      upd = upd * gi;
-      if (use & 2) { const float reg = w[i] * p.l2reg; upd = upd - reg; }
-      w[i] = w[i] + upd;
-    } else {
-      const float gi = prep_grad(g[i], w[i], use, p);
-      const float omb1 = 1.0f - p.a, omb2 = 1.0f - p.b;
-      float t1 = gi * omb1;
-      float g2 = gi * gi;
-      g2 = g2 * omb2;
-      const float mb = c1[i] * p.a;
-      t1 = t1 + mb;
-      const float vb = c2[i] * p.b;
-      g2 = g2 + vb;
-      c1[i] = t1;
-      c2[i] = g2;
-      float mh = t1 * p.corr1;
-      float vh = g2 * p.corr2;
-      vh = sqrtf(vh);
-      vh = vh + p.eps;
-      mh = mh * neg_eta;
-      mh = mh / vh;
-      w[i] = w[i] + mh;
-    }
-  }
-}
-
 // ---- dropout and its random source -------------------------------------------------------
 // Counter-based: element i is a pure function of (seed, offset + i), so the
 // numbers do not depend on the launch shape and a CPU twin can reproduce them.
@@ -693,84 +601,6 @@ int gh_launch_softmax_bwd(gh_ctx* ctx, const gh_cmd& c) {
                      (const float*)(uintptr_t)c.ptr[0], (const float*)(uintptr_t)c.ptr[1],
                      (float*)(uintptr_t)c.ptr[2], rows, cols);
   return gh_check_hip(ctx, hipGetLastError(), "softmax backward launch");
-}
-
-// How many of the commands cmds[0..n) form one solver launch: consecutive
-// SOLVER_STEP commands with the same solver, options and hyper-parameters.
-int gh_solver_run_length(const gh_cmd* cmds, int n) {
-  if (n <= 0 || cmds[0].opcode != GH_OP_SOLVER_STEP) return 0;
-  // (float64 settings are bit patterns in dim[1..10], float32 ones are in f)
-  int len = 1;
-  while (len < n && len < kSolverBatch && cmds[len].opcode == GH_OP_SOLVER_STEP && cmds[len].flags == cmds[0].flags &&
-         cmds[len].ptr[4] == cmds[0].ptr[4] && memcmp(cmds[len].f, cmds[0].f, sizeof(cmds[0].f)) == 0 &&
-         memcmp(cmds[len].dim + 1, cmds[0].dim + 1, sizeof(cmds[0].dim) - sizeof(cmds[0].dim[0])) == 0) {
-    // a tensor stepped twice keeps its two steps in order: the run ends before the repeat
-    bool repeat = false;
-    for (int j = 0; j < len; j++) repeat = repeat || cmds[j].ptr[0] == cmds[len].ptr[0];
-    if (repeat) break;
-    len++;
-  }
-  return len;
-}
-
-// The network's result leaves the device behind the solver's steps: of up to 64 KB, by more workgroups of their launch (a
-// launch of its own some 3 us).
-bool gh_solver_copy_rides(const gh_cmd* cmds, int count, int n) {
-  if (count >= n || cmds[count].opcode != GH_OP_MEMCPY_D2D) return false;
-  const gh_cmd& c = cmds[count];
-  const int64_t bytes = c.dim[0];
-  if (bytes <= 0 || bytes > 65536 || ((c.ptr[0] | c.ptr[1] | (uint64_t)bytes) & 3) || !c.ptr[0] || !c.ptr[1]) return false;
-  auto meets = [&](uint64_t p, int64_t size, uint64_t q) { return q && q < p + (uint64_t)bytes && p < q + (uint64_t)size; };
-  if (meets(c.ptr[0], bytes, c.ptr[1])) return false;
-  for (int i = 0; i < count; i++) {
-    const int64_t size = cmds[i].dim[0] * (gh_dtype_of(cmds[i].flags) == GH_F64 ? 8 : 4);
-    for (int k = 0; k < 4; k++)
-      if (meets(c.ptr[0], size, cmds[i].ptr[k]) || (k != 1 && meets(c.ptr[1], size, cmds[i].ptr[k]))) return false;
-    if (meets(c.ptr[0], 16, cmds[i].ptr[4])) return false;   // the corrections
-  }
-  return true;
-}
-
-// One launch for cmds[0..count) (count from gh_solver_run_length), and for the copy behind them.
-int gh_launch_solver_steps(gh_ctx* ctx, const gh_cmd* cmds, int count, bool copy) {
-  const gh_cmd& c = cmds[0];
-  if (gh_dtype_of(c.flags) == GH_F64) return gh_launch_solver_steps_f64(ctx, cmds, count, copy);
-  const int kind = (int)gh_fn(c.flags), use = (int)gh_mode(c.flags);
-  SolverPar p{c.f[0], c.f[1], c.f[2], c.f[3], c.f[4], c.f[5], c.f[6], c.f[7], c.f[8], c.f[9]};
-  SolverBatch sb{};
-  int nt = 0, blocks_total = 0;
-  for (int i = 0; i < count; i++) {
-    const int64_t n = cmds[i].dim[0];
-    if (n == 0) continue;
-    sb.w[nt] = (float*)(uintptr_t)cmds[i].ptr[0];
-    sb.g[nt] = (const float*)(uintptr_t)cmds[i].ptr[1];
-    sb.c1[nt] = (float*)(uintptr_t)cmds[i].ptr[2];
-    sb.c2[nt] = (float*)(uintptr_t)cmds[i].ptr[3];
-    sb.n[nt] = n;
-    int64_t blocks = (n + kBlock - 1) / kBlock;
-    if (blocks > (int64_t)ctx->cu_count * 32) blocks = (int64_t)ctx->cu_count * 32;
-    sb.first[nt] = blocks_total;
-    blocks_total += (int)blocks;
-    nt++;
-  }
-  if (nt == 0 && !copy) return GH_OK;
-  for (int i = nt; i <= kSolverBatch; i++) sb.first[i] = blocks_total;
-  sb.count = nt;
-  gh_small_copy tail{};
-  if (copy) tail = {(const uint32_t*)(uintptr_t)cmds[count].ptr[1], (uint32_t*)(uintptr_t)cmds[count].ptr[0], (int)(cmds[count].dim[0] / 4)};
-  const dim3 grid(blocks_total + (tail.words + kBlock - 1) / kBlock), block(kBlock);
-  const float* corr = (const float*)(uintptr_t)c.ptr[4];
-  if (kind == GH_SOLVER_VANILLA)
-    hipLaunchKernelGGL((k_solver_step<GH_SOLVER_VANILLA>), grid, block, 0, ctx->stream, sb, use, p, corr, tail);
-  else if (kind == GH_SOLVER_RMSPROP)
-    hipLaunchKernelGGL((k_solver_step<GH_SOLVER_RMSPROP>), grid, block, 0, ctx->stream, sb, use, p, corr, tail);
-  else
-    hipLaunchKernelGGL((k_solver_step<GH_SOLVER_ADAM>), grid, block, 0, ctx->stream, sb, use, p, corr, tail);
-  return gh_check_hip(ctx, hipGetLastError(), "solver step launch");
-}
-
-int gh_launch_solver_step(gh_ctx* ctx, const gh_cmd& c) {
-  return gh_launch_solver_steps(ctx, &c, 1, false);
 }
 
 static int stream_blocks(gh_ctx* ctx, int64_t n) {

@@ -259,88 +259,6 @@ __global__ __launch_bounds__(kBlock) void k_bn_bwd_f64(const double* __restrict_
   }
 }
 
-struct SolverPar64 { double eta, eps, l1reg, l2reg, clip, one_per_batch, a, b, corr1, corr2; };
-
-__device__ __forceinline__ double clampd(double v, double lo, double hi) { return v < lo ? lo : (v > hi ? hi : v); }
-
-__device__ __forceinline__ double prep_grad(double g, double w, int use, const SolverPar64& p) {
-  if (use & 1) { const double t = p.l1reg * (double)((w > 0.0) - (w < 0.0)); g = g + t; }
-  if (use & 2) { const double t = w * p.l2reg; g = g + t; }
-  if (use & 8) g = g * p.one_per_batch;
-  if ((use & 4) && p.clip > 0.0) g = clampd(g, -p.clip, p.clip);
-  return g;
-}
-
-// One launch for a run of tensors with the same solver and settings (a model's weights), as in float32: tensor t has
-// the workgroups [first[t], first[t + 1]).  Five tensors of the example's convnet: 25.3 us as five launches, 7.3 as one.
-constexpr int kSolverBatch64 = 8;   // gh_solver_run_length's longest run
-struct SolverBatch64 {
-  double* w[kSolverBatch64]; const double* g[kSolverBatch64]; double* c1[kSolverBatch64]; double* c2[kSolverBatch64];
-  int64_t n[kSolverBatch64];
-  int first[kSolverBatch64 + 1];
-  int count;
-};
-
-template <int KIND>
-__global__ __launch_bounds__(kBlock) void k_solver_step_f64(SolverBatch64 sb, int use, SolverPar64 p, const double* __restrict__ corr, gh_small_copy copy) {
-  if ((int)blockIdx.x >= sb.first[kSolverBatch64]) {
-    const int i = ((int)blockIdx.x - sb.first[kSolverBatch64]) * kBlock + (int)threadIdx.x;
-    if (i < copy.words) copy.dst[i] = copy.src[i];
-    return;
-  }
-  if (KIND == GH_SOLVER_ADAM && corr) { p.corr1 = corr[0]; p.corr2 = corr[1]; }   // see k_solver_step
-  int t = 0;
-#pragma unroll
-  for (int q = 1; q < kSolverBatch64; q++)
-    if (q < sb.count && (int)blockIdx.x >= sb.first[q]) t = q;
-  double* __restrict__ w = sb.w[t];
-  const double* __restrict__ g = sb.g[t];
-  double* __restrict__ c1 = sb.c1[t];
-  double* __restrict__ c2 = sb.c2[t];
-  const int64_t n = sb.n[t], nblk = sb.first[t + 1] - sb.first[t];
-  const double neg_eta = -p.eta;
-  for (int64_t i = (int64_t)((int)blockIdx.x - sb.first[t]) * kBlock + threadIdx.x; i < n; i += nblk * kBlock) {
-    if (KIND == GH_SOLVER_VANILLA) {
-      double gi = prep_grad(g[i], w[i], use, p);
-      gi = gi * neg_eta;
-      w[i] = w[i] + gi;
-    } else if (KIND == GH_SOLVER_RMSPROP) {
-      double gi = g[i];
-      double gt2 = gi * gi;
-      double cw = c1[i] * p.a;
-      gt2 = gt2 * p.b;
-      cw = cw + gt2;
-      c1[i] = cw;
-      if (use & 4) gi = clampd(gi, -p.clip, p.clip);
-      double upd = cw + p.eps;
-      upd = 1.0 / sqrt(upd);
-      gi = gi * neg_eta;
-      upd = upd * gi;
-      if (use & 2) { const double reg = w[i] * p.l2reg; upd = upd - reg; }
-      w[i] = w[i] + upd;
-    } else {
-      const double gi = prep_grad(g[i], w[i], use, p);
-      const double omb1 = 1.0 - p.a, omb2 = 1.0 - p.b;
-      double t1 = gi * omb1;
-      double g2 = gi * gi;
-      g2 = g2 * omb2;
-      const double mb = c1[i] * p.a;
-      t1 = t1 + mb;
-      const double vb = c2[i] * p.b;
-      g2 = g2 + vb;
-      c1[i] = t1;
-      c2[i] = g2;
-      double mh = t1 * p.corr1;
-      double vh = g2 * p.corr2;
-      vh = sqrt(vh);
-      vh = vh + p.eps;
-      mh = mh * neg_eta;
-      mh = mh / vh;
-      w[i] = w[i] + mh;
-    }
-  }
-}
-
 }  // namespace
 
 int gh_launch_relu_bwd_f64(gh_ctx* ctx, const gh_cmd& c) {
@@ -428,42 +346,4 @@ int gh_launch_bn_bwd_f64(gh_ctx* ctx, const gh_cmd& c) {
                      (const double*)(uintptr_t)c.ptr[4], B, (int)C, S, bits_to_double(c.dim[3]),
                      (c.flags & GH_FLAG_BN_EVAL) ? 0 : 1);
   return gh_check_hip(ctx, hipGetLastError(), "batchnorm backward launch");
-}
-
-// One launch for cmds[0..count) (count from gh_solver_run_length), and for the copy behind them.
-int gh_launch_solver_steps_f64(gh_ctx* ctx, const gh_cmd* cmds, int count, bool copy) {
-  const gh_cmd& c = cmds[0];
-  const int kind = (int)gh_fn(c.flags), use = (int)gh_mode(c.flags);
-  SolverPar64 p{bits_to_double(c.dim[1]), bits_to_double(c.dim[2]), bits_to_double(c.dim[3]),
-                bits_to_double(c.dim[4]), bits_to_double(c.dim[5]), bits_to_double(c.dim[6]),
-                bits_to_double(c.dim[7]), bits_to_double(c.dim[8]), bits_to_double(c.dim[9]),
-                bits_to_double(c.dim[10])};
-  SolverBatch64 sb{};
-  int nt = 0, blocks = 0;
-  for (int i = 0; i < count; i++) {
-    const int64_t n = cmds[i].dim[0];
-    if (n == 0) continue;
-    sb.w[nt] = (double*)(uintptr_t)cmds[i].ptr[0];
-    sb.g[nt] = (const double*)(uintptr_t)cmds[i].ptr[1];
-    sb.c1[nt] = (double*)(uintptr_t)cmds[i].ptr[2];
-    sb.c2[nt] = (double*)(uintptr_t)cmds[i].ptr[3];
-    sb.n[nt] = n;
-    sb.first[nt] = blocks;
-    blocks += blocks_for(ctx, n);
-    nt++;
-  }
-  if (nt == 0 && !copy) return GH_OK;
-  for (int i = nt; i <= kSolverBatch64; i++) sb.first[i] = blocks;
-  sb.count = nt;
-  gh_small_copy tail{};
-  if (copy) tail = {(const uint32_t*)(uintptr_t)cmds[count].ptr[1], (uint32_t*)(uintptr_t)cmds[count].ptr[0], (int)(cmds[count].dim[0] / 4)};
-  const dim3 grid((unsigned)(blocks + (tail.words + kBlock - 1) / kBlock)), block(kBlock);
-  const double* corr = (const double*)(uintptr_t)c.ptr[4];
-  if (kind == GH_SOLVER_VANILLA)
-    hipLaunchKernelGGL((k_solver_step_f64<GH_SOLVER_VANILLA>), grid, block, 0, ctx->stream, sb, use, p, corr, tail);
-  else if (kind == GH_SOLVER_RMSPROP)
-    hipLaunchKernelGGL((k_solver_step_f64<GH_SOLVER_RMSPROP>), grid, block, 0, ctx->stream, sb, use, p, corr, tail);
-  else
-    hipLaunchKernelGGL((k_solver_step_f64<GH_SOLVER_ADAM>), grid, block, 0, ctx->stream, sb, use, p, corr, tail);
-  return gh_check_hip(ctx, hipGetLastError(), "solver step launch");
 }

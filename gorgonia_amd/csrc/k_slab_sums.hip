@@ -4,75 +4,17 @@
 // each, of which the additions take one or two.  A training step has one for each layer, and nobody reads a gradient before
 // the solver.  So the sums are put off while the commands behind the gradient, of the kinds that stand between the layers of
 // a backward pass, neither read nor write its result: the slabs lie in 24 MB of the context's that nothing else uses (made for
-// its first submission of several commands with a filter gradient, given back with the context), and the next command of another kind, one that touches a result, or the end of the submission has them added in one launch.
+// its first submission of several commands with a filter gradient, given back with the context), and the next command of another kind, one that touches a result, or the end of the submission has them added in one launch
+// (the solver's steps in theirs, k_solver.hip).
 // us of a training step, a launch for each sum / one: the convnet at batch 128 in float32 229 / 222, the four-block network at
 // batch 8 431 / 424.
 #include <algorithm>
 
-#include "gh_internal.h"
+#include "gh_slab_sums.h"
 
 namespace {
 
-struct Batch {
-  const void* ws[kSlabSums];
-  void* out[kSlabSums];
-  int64_t total[kSlabSums];
-  int slabs[kSlabSums], how[kSlabSums], first[kSlabSums + 1];
-};
-
-// RW results to a workgroup; its 256 / RW thread groups take every G-th slab (reads of a slab are RW values wide), and the
-// groups' sums are added pairwise, neighbours first.
-template <class T, int RW>
-__device__ __forceinline__ void by_groups(const T* __restrict__ ws, int slabs, int64_t total, T* __restrict__ out, int block, T* sh) {
-  constexpr int G = 256 / RW;
-  const int grp = threadIdx.x / RW;
-  const int64_t e = (int64_t)block * RW + threadIdx.x % RW;
-  T sum = (T)0;
-  if (e < total) {
-    int s = grp;
-    for (; s + 3 * G < slabs; s += 4 * G) {   // four loads in flight
-      T v[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) v[u] = ws[(int64_t)(s + u * G) * total + e];
-#pragma unroll
-      for (int u = 0; u < 4; u++) sum = sum + v[u];
-    }
-    for (; s < slabs; s += G) sum = sum + ws[(int64_t)s * total + e];
-  }
-  sh[threadIdx.x] = sum;
-  for (int d = 1; d < G; d <<= 1) {
-    __syncthreads();
-    T v = (T)0;
-    const bool mine = grp % (2 * d) == 0;
-    if (mine) v = sh[threadIdx.x] + sh[threadIdx.x + d * RW];
-    __syncthreads();
-    if (mine) sh[threadIdx.x] = v;
-  }
-  if (grp == 0 && e < total) out[e] = sh[threadIdx.x];
-}
-
-// Many slabs, few results: L lanes share one result.  Lane q adds slabs q, q + L, q + 2 L, ... in that order, then the L
-// sums are combined pairwise, neighbours first.
-template <int L>
-__device__ __forceinline__ void by_lanes(const float* __restrict__ ws, int slabs, int64_t total, float* __restrict__ out, int block) {
-  const int q = threadIdx.x & (L - 1);
-  const int64_t e = ((int64_t)block * 256 + threadIdx.x) / L;
-  float acc = 0.f;
-  if (e < total) {
-    const float* p = ws + (int64_t)q * total + e;
-    int s = q;
-    for (; s + 3 * L < slabs; s += 4 * L) {   // four loads in flight
-      const float v0 = p[0], v1 = p[(int64_t)L * total], v2 = p[2 * (int64_t)L * total], v3 = p[3 * (int64_t)L * total];
-      acc = acc + v0; acc = acc + v1; acc = acc + v2; acc = acc + v3;
-      p += 4 * (int64_t)L * total;
-    }
-    for (; s < slabs; s += L) { acc = acc + p[0]; p += (int64_t)L * total; }
-  }
-  float sum = acc;
-#pragma unroll
-  for (int d = 1; d < L; d <<= 1) sum = sum + __shfl_xor(sum, d, 64);   // commutative per level: every lane ends with the total
-  if (e < total && q == 0) out[e] = sum;
-}
+using namespace slab_sums;
 
 __global__ __launch_bounds__(256) void k_slab_sums(const Batch b) {
   __shared__ double sh[256];
@@ -80,51 +22,19 @@ __global__ __launch_bounds__(256) void k_slab_sums(const Batch b) {
 #pragma unroll
   for (int q = 1; q < kSlabSums; q++)
     if ((int)blockIdx.x >= b.first[q]) t = q;
-  const int block = blockIdx.x - b.first[t], slabs = b.slabs[t];
-  const int64_t total = b.total[t];
-  const float* const ws = (const float*)b.ws[t];
-  float* const out = (float*)b.out[t];
-  switch (b.how[t]) {
-    case kSumGroups64: by_groups<float, 64>(ws, slabs, total, out, block, (float*)sh); break;
-    case kSumGroups16: by_groups<float, 16>(ws, slabs, total, out, block, (float*)sh); break;
-    case kSumGroups64F64: by_groups<double, 64>((const double*)ws, slabs, total, (double*)out, block, sh); break;
-    case kSumGroups16F64: by_groups<double, 16>((const double*)ws, slabs, total, (double*)out, block, sh); break;
-    case kSumLanes16: by_lanes<16>(ws, slabs, total, out, block); break;
-    case kSumLanes4: by_lanes<4>(ws, slabs, total, out, block); break;
-    default: {
-      const int64_t e = (int64_t)block * 256 + threadIdx.x;
-      if (e >= total) break;
-      float acc = ws[e];
-      for (int s = 1; s < slabs; s++) acc = acc + ws[(int64_t)s * total + e];
-      out[e] = acc;
-    }
+  const int block = blockIdx.x - b.first[t];
+  if (b.how[t] == kSumGroups64F64 || b.how[t] == kSumGroups16F64) {
+    double* const out = (double*)b.out[t];
+    workgroup<double>(b, t, block, sh, [&](int64_t e, double sum) { out[e] = sum; });
+  } else {
+    float* const out = (float*)b.out[t];
+    workgroup<float>(b, t, block, sh, [&](int64_t e, float sum) { out[e] = sum; });
   }
 }
-
-int results_of_block(int how) {
-  switch (how) {
-    case kSumGroups64: case kSumGroups64F64: case kSumLanes4: return 64;
-    case kSumGroups16: case kSumGroups16F64: case kSumLanes16: return 16;
-    default: return 256;
-  }
-}
-
-int64_t item(int how) { return how == kSumGroups64F64 || how == kSumGroups16F64 ? 8 : 4; }
 
 int launch(gh_ctx* ctx, const gh_slab_sum* sums, int n) {
-  Batch b{};
-  int blocks = 0;
-  for (int i = 0; i < n; i++) {
-    b.ws[i] = sums[i].ws;
-    b.out[i] = sums[i].out;
-    b.total[i] = sums[i].total;
-    b.slabs[i] = sums[i].slabs;
-    b.how[i] = sums[i].how;
-    b.first[i] = blocks;
-    const int r = results_of_block(sums[i].how);
-    blocks += (int)((sums[i].total + r - 1) / r);
-  }
-  for (int i = n; i <= kSlabSums; i++) b.first[i] = blocks;
+  Batch b;
+  const int blocks = batch_of(sums, n, &b);
   hipLaunchKernelGGL(k_slab_sums, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, b);
   return gh_check_hip(ctx, hipGetLastError(), "slab sum launch");
 }
