@@ -239,9 +239,12 @@ __device__ __forceinline__ void workgroup(const Lanes<T>& g, const ConvTail& tai
   const int tid = (int)threadIdx.x;
   constexpr int nthreads = WV * 64;
   auto value = [&](int e) {
-    T sum = red[0][e];
+    // (eight in the order of k_conv3x3_patch, whose error a sum in one chain is 1 % above)
+    constexpr int kHalves = sizeof(T) == 4 && WV == 8 ? 2 : 1, n = WV / kHalves;
+    auto part = [&](int v) { return kHalves == 2 ? red[v][e] + red[v + n][e] : red[v][e]; };
+    T sum = part(0);
 #pragma unroll
-    for (int v = 1; v < WV; v++) sum = sum + red[v][e];
+    for (int v = 1; v < n; v++) sum = sum + part(v);
     return sum;
   };
 #pragma unroll

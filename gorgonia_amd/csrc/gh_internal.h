@@ -222,7 +222,7 @@ bool gh_conv_pointwise_takes(const gh_cmd& c, int cus);
 bool gh_conv_strip_takes(const gh_cmd& c);
 int gh_launch_conv_strip(gh_ctx* ctx, const gh_cmd& c);
 // 3x3 stride-1 convolution with operands straight from memory, both float types; flip: of an image-gradient command (k_conv_lanes.hip)
-int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, bool whole = false);   // -1: not taken; whole: the other's sums run over all channels
+int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, bool patch = false, bool whole = false);   // -1: not taken; the other: k_conv3x3_patch, one whose sums run over all channels
 int gh_launch_conv_lanes(gh_ctx* ctx, const gh_cmd& c, bool flip, int form);
 int gh_launch_maxpool2d(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_bn_infer(gh_ctx* ctx, const gh_cmd& c);

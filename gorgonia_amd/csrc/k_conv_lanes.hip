@@ -129,6 +129,13 @@ static int quickest(const gh_cmd& c, bool flip, bool f64, int cus, int from, int
 // where they keep it; other_us 0: any shape that a form can take.  It has to be a sixth quicker by the estimates, which
 // are that good.
 //
+// In place of the patch kernel (`patch`) a form of eight wavefronts, whose sums are that kernel's, also where the estimates have it
+// a sixth slower: both are high there, by more for these.  Of 520 drawn gradients and 200 forward passes the rule gives 58 and 20
+// more to it, at 0.54 to 1.0 and 0.73 to 0.92 of the time.  us, before / now, with the launch that mirrors the filters: the gradient of
+// 8 x 32 x 52 x 52 -> 64 16.6 / 13.6, with its filter gradient 39.3 / 31.7; 15 x 64 x 49 x 58 -> 128 77.5 / 64.0; forward 7 x 512 x 8 x 8 ->
+// 1024 50.7 / 39.3, 5 x 256 x 9 x 9 -> 512 25.0 / 22.2.  The form of four wavefronts is quicker for some (6 x 512 x 10 x 10 ->
+// 1024 81.2 / 72.2) and slower for others (8 x 512 x 13 x 13 -> 1024 116 / 145), and its sums are twice as long.
+//
 // float32 where that is not so: a wavefront with a tile of its own and all channels, for few channels and many pixels, where
 // the split forms have one or two quads to a wavefront and the wide-image kernel stages as much as it multiplies.  Only in place
 // of a kernel whose sums run over all channels too (`whole`), since its own are longer than those of one that splits them: the
@@ -137,7 +144,7 @@ static int quickest(const gh_cmd& c, bool flip, bool f64, int cus, int from, int
 // kernel 2.0e-7.  us, before / now: 8 x 16 x 104 x 104 -> 32 22.9 / 15.9, pooled 17.9 / 13.6, its gradient 24.2 / 13.6; 8 x 16 x 104 x 104 -> 16
 // 15.8 / 10.0 and its gradient 17.8 / 8.7; 8 x 32 x 104 x 104 -> 64 46.7 / 39.7 (80 TFLOP/s); 8 x 16 x 208 x 208 -> 32's
 // gradient 45.8 / 36.1; 1 x 16 x 208 x 208 -> 32 pooled 11.0 / 8.7.
-int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, bool whole) {
+int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, bool patch, bool whole) {
   if (getenv("GORGONIA_HIP_CONV_NO_LANES")) return -1;   // tuning switch: the other kernels only
   const bool f64 = gh_dtype_of(c.flags) == GH_F64;
   Lanes<double> g;   // (the narrower of the two in what its offsets reach)
@@ -145,7 +152,12 @@ int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, boo
   double us;
   const int split = quickest(c, flip, f64, cus, 0, f64 && !flip ? 4 : 3, &us);
   if (other_us <= 0 || us < other_us / 1.17) return split;
-  if (f64 || !whole) return -1;
+  if (f64) return -1;
+  if (patch) {
+    const int eight = quickest(c, flip, false, cus, 0, 2, &us);
+    return us < other_us / 0.85 ? eight : -1;
+  }
+  if (!whole) return -1;
   const int form = quickest(c, flip, false, cus, 3, 5, &us);
   return us < other_us / 1.1 ? form : -1;
 }

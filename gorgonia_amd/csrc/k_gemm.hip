@@ -3057,7 +3057,7 @@ static bool conv_sums_whole(const gh_cmd& c) {
 // float32, behind the single-channel, few-channel and small-image kernels, which win where they take a shape.
 static int conv_lanes_form(const gh_cmd& c, int cus) {
   if (c.dim[5] != 3 || c.dim[6] != 3 || gh_conv_rows1_takes(c) || conv_direct_takes(c) || gh_conv_small_takes(c)) return -1;
-  return gh_conv_lanes_form(c, false, cus, conv_others_us(c, cus), conv_sums_whole(c));
+  return gh_conv_lanes_form(c, false, cus, conv_others_us(c, cus), gh_conv_patch_takes(c), conv_sums_whole(c));
 }
 // The image gradient: elsewhere that is a launch that mirrors the filters (4.7 us) and a forward one over dy.
 static int conv_lanes_gradient_form(const gh_cmd& c, int cus) {
@@ -3073,7 +3073,7 @@ static int conv_lanes_gradient_form(const gh_cmd& c, int cus) {
                                                : conv_others_us(f, cus);
   // (a forward form of 3 and more has whole sums as well)
   const int forward = conv_lanes_form(f, cus);
-  return gh_conv_lanes_form(c, true, cus, others + 4.7, conv_sums_whole(f) && (forward < 0 || forward >= 3));
+  return gh_conv_lanes_form(c, true, cus, others + 4.7, !gh_conv_small_takes(f) && gh_conv_patch_takes(f), conv_sums_whole(f) && (forward < 0 || forward >= 3));
 }
 
 static int launch_conv_direct(gh_ctx* ctx, const gh_cmd& c) {
