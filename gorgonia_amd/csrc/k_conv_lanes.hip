@@ -10,7 +10,8 @@
 // offsets do not change from quad to quad (the quad moves a scalar offset), and a value outside the image has an offset
 // that the buffer's range check turns into zero, so the loop holds loads and MFMAs and nothing else: no staging, no
 // barrier, no edge arithmetic.  The loads of a quad are issued in front of the MFMAs of the quad before it.  The
-// wavefronts of a workgroup split the channels of one tile (kSplit), their sums meeting in LDS in wavefront order, or
+// wavefronts of a workgroup split the channels of one tile (kSplit), their sums meeting in LDS in wavefront order (of eight in
+// float32 the upper four first each to the one four below), or
 // own a tile each.  With a pooled result the groups come in pairs, one above the other.
 //
 // With kFlip the same walk is the image gradient: rows are image channels, K runs over the filters, and a lane's nine
