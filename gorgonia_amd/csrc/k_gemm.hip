@@ -1904,8 +1904,10 @@ __global__ __launch_bounds__(256) void k_conv3x3_wgrad_direct(const float* __res
 __global__ __launch_bounds__(256) void k_conv3x3_wgrad_c1(const float* __restrict__ x, const float* __restrict__ dy,
                                                           float* __restrict__ ws, int B, int H, int W, int F, int pad,
                                                           int oh, int ow, unsigned m_ow, unsigned m_pw) {
-  extern __shared__ float img[];   // (H + 2 pad) rows of W + 2 pad
+  extern __shared__ float img[];   // (H + 2 pad) rows of W + 2 pad, and three zeros
   const int PW = W + 2 * pad, PH = H + 2 * pad;
+  float* const zeros = img + PH * PW;
+  if (threadIdx.x < 3) zeros[threadIdx.x] = 0.f;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int f = blockIdx.y * 4 + wave;
   const bool fok = f < F;
@@ -1933,13 +1935,13 @@ __global__ __launch_bounds__(256) void k_conv3x3_wgrad_c1(const float* __restric
       }
 #pragma unroll
       for (int u = 0; u < 8; u++) {
-        const int p = min(p0 + 64 * u, plane - 1);   // (a pixel past the end multiplies a zero)
-        const int oy = (int)__umulhi((unsigned)p, m_ow), ox = p - oy * ow;
-        const float* ip = img + oy * PW + ox;
+        // (a pixel past the end multiplies zeros: zero times an infinity of the last pixel's window would be NaN)
+        const int p = p0 + 64 * u, oy = (int)__umulhi((unsigned)p, m_ow), ox = p - oy * ow, pitch = p < plane ? PW : 0;
+        const float* ip = p < plane ? img + oy * PW + ox : zeros;
 #pragma unroll
         for (int kr = 0; kr < 3; kr++)
 #pragma unroll
-          for (int kc = 0; kc < 3; kc++) acc[kr * 3 + kc] = __builtin_fmaf(g[u], ip[kr * PW + kc], acc[kr * 3 + kc]);
+          for (int kc = 0; kc < 3; kc++) acc[kr * 3 + kc] = __builtin_fmaf(g[u], ip[kr * pitch + kc], acc[kr * 3 + kc]);
       }
     }
   }
@@ -1955,14 +1957,17 @@ __global__ __launch_bounds__(256) void k_conv3x3_wgrad_c1(const float* __restric
 // The same sums with loads ahead, for padded images of up to 1024 values.  What bounds it is what a workgroup waits for one behind
 // the other, so the first dy of an image are asked for with the image, in front of the barriers, each eight's successors before
 // the eight are multiplied, and the next image, kX values a thread, under the current one's sums.  us, slab sum included, before / now:
-// 128 x 28 x 28 -> 32 14.0 / 13.2, 384 of them 31.9 / 23.6, 200 x 28 x 28 -> 10 17.4 / 15.3, 130 x 31 x 29 -> 8 14.5 / 12.8.  Larger images,
-// staged under the barriers, and planes of few pixels gain nothing from it (5 x 110 x 100 -> 6 32.8 / 33.7, 129 x 10 x 9 -> 33 11.9 / 12.3).
+// 128 x 28 x 28 -> 32 14.0 / 13.2, 384 of them 31.9 / 24.0, 200 x 28 x 28 -> 10 17.4 / 15.5, 130 x 31 x 29 -> 8 14.5 / 13.1.  Larger images,
+// staged under the barriers, and planes of few pixels gained nothing from it (5 x 110 x 100 -> 6 32.8 / 33.7, 129 x 10 x 9 -> 33 11.9 / 12.3,
+// both against the kernel above when it moved a pixel past the end inside, which is 29.1 and 11.7 now).
 __global__ __launch_bounds__(256) void k_conv3x3_wgrad_c1_ahead(const float* __restrict__ x, const float* __restrict__ dy,
                                                           float* __restrict__ ws, int B, int H, int W, int F, int pad,
                                                           int oh, int ow, unsigned m_ow, unsigned m_pw) {
   constexpr int kX = 4;
-  extern __shared__ float img[];   // (H + 2 pad) rows of W + 2 pad
+  extern __shared__ float img[];   // (H + 2 pad) rows of W + 2 pad, and three zeros
   const int PW = W + 2 * pad, PH = H + 2 * pad;
+  float* const zeros = img + PH * PW;
+  if (threadIdx.x < 3) zeros[threadIdx.x] = 0.f;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int f = blockIdx.y * 4 + wave;
   const bool fok = f < F;
@@ -1996,14 +2001,14 @@ __global__ __launch_bounds__(256) void k_conv3x3_wgrad_c1_ahead(const float* __r
     if (p0 + lane >= plane) return;
 #pragma unroll
     for (int u = 0; u < 8; u++) {
-      const int q = p0 + lane + 64 * u, p = min(q, plane - 1);   // (a pixel past the end multiplies a zero)
-      const int oy = (int)__umulhi((unsigned)p, m_ow), ox = p - oy * ow;
-      const float* ip = img + oy * PW + ox;
+      // (a pixel past the end multiplies zeros: zero times an infinity of the last pixel's window would be NaN)
+      const int q = p0 + lane + 64 * u, oy = (int)__umulhi((unsigned)q, m_ow), ox = q - oy * ow, pitch = q < plane ? PW : 0;
+      const float* ip = q < plane ? img + oy * PW + ox : zeros;
       const float v = fok && q < plane ? g[u] : 0.f;
 #pragma unroll
       for (int kr = 0; kr < 3; kr++)
 #pragma unroll
-        for (int kc = 0; kc < 3; kc++) acc[kr * 3 + kc] = __builtin_fmaf(v, ip[kr * PW + kc], acc[kr * 3 + kc]);
+        for (int kc = 0; kc < 3; kc++) acc[kr * 3 + kc] = __builtin_fmaf(v, ip[kr * pitch + kc], acc[kr * 3 + kc]);
     }
   };
   float g[8];
@@ -3313,7 +3318,7 @@ int gh_launch_conv2d_bwd_filter(gh_ctx* ctx, const gh_cmd& c) {
       const int PW = g.W + 2 * g.padH;
       float* const wsd = (float*)gh_slab_space(ctx, (int64_t)G1 * F * CKK * 4);
       auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)G1, (unsigned)fby), dim3(256), img_bytes, ctx->stream, xd, dyd, wsd, B, g.H, g.W, F, g.padH, g.oh, g.ow,
+        hipLaunchKernelGGL(kernel, dim3((unsigned)G1, (unsigned)fby), dim3(256), img_bytes + 3 * 4, ctx->stream, xd, dyd, wsd, B, g.H, g.W, F, g.padH, g.oh, g.ow,
                            magic(g.ow), magic(PW));
       };
       if (img_bytes <= 4 * 256 * 4 && g.oh * g.ow >= 256) go(k_conv3x3_wgrad_c1_ahead);

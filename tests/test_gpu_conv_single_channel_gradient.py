@@ -1,10 +1,13 @@
 """The filter gradient over single-channel images (k_conv3x3_wgrad_c1): images fetched ahead and larger ones, whole and partial
-groups of pixels, more images than workgroups and fewer, filters past a workgroup's four, infinities where they belong."""
+groups of pixels, more images than workgroups and fewer, filters past a workgroup's four, infinities and NaN in the last pixel's
+window and in the last pixel, which reach the taps that read them and no other."""
 import numpy as np
 import pytest
 import torch
 
+from gorgonia_amd import _ffi
 from gorgonia_amd import device as D
+from tests.test_gpu_conv_filter_gradient_edges import _compare
 
 pytestmark = pytest.mark.gpu
 
@@ -33,3 +36,17 @@ def test_against_64_bit_sums(ctx, B, H, W, F, pad):
     # 2^-24 of a partial sum, which grows as the square root of its products
     chain = -(-B // 64) * -(-oh * ow // 64) + 12
     assert np.linalg.norm(got - want) <= np.sqrt(chain) * 2.0 ** -24 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("where", ["x", "dy"])
+@pytest.mark.parametrize("B,H,W,F,pad", CASES)
+def test_infinities_and_nan_at_the_end_of_an_image(ctx, B, H, W, F, pad, where, value):
+    rng = np.random.default_rng(B + W)
+    x = rng.standard_normal((B, 1, H, W)).astype(np.float32)
+    dy = rng.standard_normal((B, F, H + 2 * pad - 2, W + 2 * pad - 2)).astype(np.float32)
+    if where == "x":
+        x[B // 2, 0, -1, -1] = value
+    else:
+        dy[B // 2, F // 2, -1, -1] = value
+    _compare(ctx, x, dy, (pad, pad), _ffi.F32)
