@@ -159,6 +159,8 @@ int gh_init(int device, int64_t arena_bytes, gh_ctx** out) {
   }
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) ctx->cu_count = prop.multiProcessorCount;
+  // tuning override: the launchers plan for so many compute units, never for more than there are
+  if (const char* units = getenv("GORGONIA_HIP_COMPUTE_UNITS")) ctx->cu_count = std::max(1, std::min(ctx->cu_count, atoi(units)));
   if (const char* sm = getenv("GORGONIA_HIP_SYNC")) {
     ctx->sync_block = strcmp(sm, "block") == 0;
     ctx->sync_spin = strcmp(sm, "spin") == 0;

@@ -65,6 +65,7 @@ struct gh_held_filter {
   size_t lds = 0;
   alignas(16) unsigned char args[192];
 };
+constexpr int kUnits = 256;   // the MI355X's compute units
 constexpr int kSlabSums = 8;
 constexpr int64_t kSlabSpace = 24ll << 20;
 
@@ -78,7 +79,7 @@ struct gh_ctx {
   bool capturing = false;
   std::vector<gh_graph_slot> graphs;
   hipEvent_t events[64] = {};
-  int cu_count = 256;
+  int cu_count = kUnits;
   // scratch owned by the context (split-K partials, reduction flags)
   void* workspace = nullptr;
   int64_t workspace_bytes = 0;

@@ -130,7 +130,7 @@ static int quickest(const gh_cmd& c, bool flip, bool f64, int cus, int from, int
 // where they keep it; other_us 0: any shape that a form can take.  It has to be a sixth quicker by the estimates, which
 // are that good.
 //
-// In place of the patch kernel (`patch`) a form of eight wavefronts, whose sums are that kernel's, also where the estimates have it
+// In place of the patch kernel (`patch`) a form of eight wavefronts, whose sums are as long as that kernel's, also where the estimates have it
 // a sixth slower: both are high there, by more for these.  Of 520 drawn gradients and 200 forward passes the rule gives 58 and 20
 // more to it, at 0.54 to 1.0 and 0.73 to 0.92 of the time.  us, before / now, with the launch that mirrors the filters: the gradient of
 // 8 x 32 x 52 x 52 -> 64 16.6 / 13.6, with its filter gradient 39.3 / 31.7; 15 x 64 x 49 x 58 -> 128 77.5 / 64.0; forward 7 x 512 x 8 x 8 ->

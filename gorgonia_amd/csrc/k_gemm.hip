@@ -3146,6 +3146,9 @@ static bool conv_sums_whole(const gh_cmd& c) {
 // float32, behind the single-channel, few-channel and small-image kernels, which win where they take a shape.
 static int conv_lanes_form(const gh_cmd& c, int cus) {
   if (c.dim[5] != 3 || c.dim[6] != 3 || gh_conv_rows1_takes(c) || conv_direct_takes(c) || gh_conv_small_takes(c)) return -1;
+  // gh_conv2d_can_pool answers without a device, so where only this kernel can pool (and sums as the plain command does) the choice
+  // between the two is by the MI355X's compute units on every device.
+  if (cus != kUnits && gh_conv_patch_takes(c) && !gh_conv_patch_can_pool(c)) cus = kUnits;
   return gh_conv_lanes_form(c, false, cus, conv_others_us(c, cus), gh_conv_patch_takes(c), conv_sums_whole(c));
 }
 // The image gradient: elsewhere that is a launch that mirrors the filters (4.7 us) and a forward one over dy.

@@ -57,6 +57,27 @@ def test_forward(ctx, B, Cn, H, W, F):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("units", [8, 32, 64, 104, 152, 208])
+def test_pooled_with_other_numbers_of_compute_units(monkeypatch, units):
+    """What gh_conv2d_can_pool accepts, for whatever number of compute units it answers, runs on a device with another number,
+    and has the plain result's bits there too."""
+    monkeypatch.setenv("GORGONIA_HIP_COMPUTE_UNITS", str(units))
+    rng = np.random.default_rng(units)
+    with D.Context() as ctx:
+        for B, Cn, H, W, F in FORWARD:
+            x, w = rng.standard_normal((B, Cn, H, W)).astype(np.float32), rng.standard_normal((F, Cn, 3, 3)).astype(np.float32)
+            at = [ctx.upload(x), ctx.upload(w), ctx.upload(np.full((B, F, H, W), np.nan, np.float32)), ctx.upload(np.full((B, F, H // 2, W // 2), np.nan, np.float32))]
+            plain = D.cmd_conv2d(at[0], at[1], at[2], B, Cn, H, W, F, 3, 3, (1, 1))
+            if _ffi.load().gh_conv2d_can_pool(C.byref(plain)):
+                ctx.run([plain, D.cmd_conv2d(at[0], at[1], at[3], B, Cn, H, W, F, 3, 3, (1, 1), pool2=True)])
+                got = ctx.d2h(at[2], (B, F, H, W))
+                want = got[:, :, :H // 2 * 2, :W // 2 * 2].reshape(B, F, H // 2, 2, W // 2, 2).max(axis=(3, 5))
+                assert_bits_equal(ctx.d2h(at[3], (B, F, H // 2, W // 2)), want)
+            for p in at:
+                ctx.free(p)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,Cn,H,W,F", GRADIENT)
 def test_gradient(ctx, B, Cn, H, W, F):
     rng = np.random.default_rng(B * Cn + H)
