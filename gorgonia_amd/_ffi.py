@@ -101,6 +101,7 @@ SYMBOLS = {
     "gh_gemm_route": (C.c_int, [C.POINTER(GhCmd), C.POINTER(C.c_int)]),
     "gh_runs_straight": (C.c_int, [C.POINTER(GhCmd)]),
     "gh_runs_split": (C.c_int, [C.POINTER(GhCmd)]),
+    "gh_touched_lately": (C.c_int, [_P, C.c_uint64]),
     "gh_gemm_can_softmax": (C.c_int, [C.POINTER(GhCmd)]),
     "gh_sync": (C.c_int, [_P]),
     "gh_graph_begin": (C.c_int, [_P]),

@@ -481,6 +481,7 @@ bool gh_llc_cold(const gh_ctx* ctx, uint64_t p) {
   constexpr uint64_t kWarmWindow = 192ull << 20;
   return !ctx->llc.warm(p, kWarmWindow);
 }
+extern "C" int gh_touched_lately(const gh_ctx* ctx, gh_devptr p) { return ctx && !gh_llc_cold(ctx, p); }
 bool gh_llc_stream(int64_t bytes, bool cold) {
   static const int64_t limit = [] {
     const char* e = getenv("GORGONIA_HIP_EW_STREAM_MIB");   // tuning override

@@ -127,7 +127,7 @@ bool apart(const Span& a, const Span& b) { return a.at + (uint64_t)a.bytes <= b.
 
 }  // namespace
 
-int gh_try_launch_gemm_gradients(gh_ctx* ctx, const gh_cmd* cmds) {
+static int try_launch(gh_ctx* ctx, const gh_cmd* cmds) {
   if (getenv("GORGONIA_HIP_GEMM_APART")) return -1;   // tuning switch: a launch each
   const int w = (cmds[0].flags & GH_FLAG_TRANS_A) ? 0 : 1;
   const gh_cmd &dw = cmds[w], &dx = cmds[1 - w];
@@ -143,6 +143,14 @@ int gh_try_launch_gemm_gradients(gh_ctx* ctx, const gh_cmd* cmds) {
     constexpr bool kDirect = std::decay_t<decltype(p)>::kDirect;
     return with32<false, kDirect>(kx, dx, [&](const auto& q) { return go(ctx, q, p); });
   });
+}
+
+int gh_try_launch_gemm_gradients(gh_ctx* ctx, const gh_cmd* cmds) {
+  const int rc = try_launch(ctx, cmds);
+  if (rc == GH_OK)
+    for (int k = 0; k < 2; k++)
+      for (uint64_t p : cmds[k].ptr) ctx->llc.touch(p, 0, false);
+  return rc;
 }
 
 // Whether cmds[0] and cmds[1] are products of one size of float with the left operand of the one and the right operand of

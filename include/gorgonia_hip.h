@@ -388,6 +388,11 @@ GH_API int gh_runs_straight(const gh_cmd* cmd);
  * instructions that it would run on otherwise.  Host only; 256 compute units, as above. */
 GH_API int gh_runs_split(const gh_cmd* cmd);
 
+/* 1 when the context's account of what the last-level cache holds has the buffer at p as touched lately, by commands
+ * submitted through it.  An elementwise command over large tensors goes past the cache where it has none of its inputs;
+ * the stored bits are the same.  Host only. */
+GH_API int gh_touched_lately(const gh_ctx* ctx, gh_devptr p);
+
 /* 1 when this GEMM command may carry GH_FLAG_GEMM_SOFTMAX: a float32 product of
  * untransposed operands with at most 32 columns and at most 2048 rows, whose
  * rows are whole inside one workgroup.  The stored values are those of the

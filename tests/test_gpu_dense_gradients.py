@@ -80,6 +80,19 @@ def test_result_that_the_other_reads(ctx, which):
         assert_bits_equal(a, b)
 
 
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_operands_are_in_the_cache_account(dt):
+    batch, n_in, n_out = 96, 625, 10
+    rng = np.random.default_rng(7)
+    with D.Context() as ctx:
+        at = [ctx.upload(rng.standard_normal(s).astype(dt)) for s in ((batch, n_in), (batch, n_out), (n_in, n_out), (n_in, n_out), (batch, n_in))]
+        assert not any(ctx.lib.gh_touched_lately(ctx.h, p) for p in at)
+        ctx.run(_commands(*at, batch, n_in, n_out, _ffi.F64 if dt == np.float64 else _ffi.F32))
+        assert all(ctx.lib.gh_touched_lately(ctx.h, p) for p in at)
+        for p in at:
+            ctx.free(p)
+
+
 def test_replayed(ctx):
     batch, n_in, n_out = 128, 1152, 625
     rng = np.random.default_rng(6)
