@@ -279,6 +279,9 @@ int gh_try_launch_solver_sums(gh_ctx* ctx, const gh_cmd* cmds, int count, bool c
     }
   }
   if (!any) return -1;
+  // (as a step by itself is in the account; longer runs never were)
+  if (count + copy == 1)
+    for (uint64_t p : cmds[0].ptr) ctx->llc.touch(p, 0, false);
   const int waits = ctx->pending;
   ctx->pending = 0;
   ctx->slabs_used = 0;

@@ -5,7 +5,7 @@ import pytest
 
 from gorgonia_amd import _ffi
 from gorgonia_amd import device as D
-from tests.test_gpu_slab_sums import LAYERS, _gradient, _same
+from tests.test_gpu_slab_sums import LAYERS, _gradient, _same, _Tensors
 
 pytestmark = pytest.mark.gpu
 
@@ -69,6 +69,19 @@ def test_other_forms(ctx, form):
         second, third = _gradient(t, (64, 32, 14, 14, 64)), _gradient(t, (8, 64, 26, 26, 128))
         return [g, second, third, _step(t, "adam", t.make(n), dw, n), _step(t, "adam", t.make(64 * 32 * 9), second.ptr[2], 64 * 32 * 9)]
     _same(ctx, build)
+
+
+def test_operands_of_one_step_are_in_the_cache_account():
+    layer = (8, 16, 52, 52, 32)
+    n = _size(layer)
+    with D.Context() as ctx:
+        t = _Tensors(ctx, np.float32)
+        gradient = _gradient(t, layer)
+        step = _step(t, "adam", t.make(n), gradient.ptr[2], n)
+        assert not any(ctx.lib.gh_touched_lately(ctx.h, p) for p, _ in t.all)
+        ctx.run([gradient, step])
+        assert all(ctx.lib.gh_touched_lately(ctx.h, p) for p, _ in t.all)
+        t.values()
 
 
 def test_replayed(ctx):
