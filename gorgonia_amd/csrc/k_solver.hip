@@ -205,6 +205,23 @@ int launch(gh_ctx* ctx, const gh_cmd* cmds, int count, bool copy, const gh_slab_
   return gh_check_hip(ctx, hipGetLastError(), "solver step launch");
 }
 
+// Whether step b, of a's solver and type, has to come after step a: one of them writes what the other reads or writes.
+bool follows(const gh_cmd& a, const gh_cmd& b) {
+  const int kind = (int)gh_fn(a.flags), caches = kind == GH_SOLVER_VANILLA ? 0 : kind == GH_SOLVER_RMSPROP ? 1 : 2;
+  const int64_t size = gh_dtype_of(a.flags) == GH_F64 ? 8 : 4;
+  auto meet = [](uint64_t p, int64_t np, uint64_t q, int64_t nq) { return p && q && p < q + (uint64_t)nq && q < p + (uint64_t)np; };
+  auto written = [&](const gh_cmd& x, const gh_cmd& y) {   // by x, and of y's
+    for (int i = 0; i < 2 + caches; i++) {
+      if (i == 1) continue;   // the gradient
+      for (int k = 0; k < 2 + caches; k++)
+        if (meet(x.ptr[i], x.dim[0] * size, y.ptr[k], y.dim[0] * size)) return true;
+      if (kind == GH_SOLVER_ADAM && meet(x.ptr[i], x.dim[0] * size, y.ptr[4], 2 * size)) return true;   // the corrections
+    }
+    return false;
+  };
+  return written(a, b) || written(b, a);
+}
+
 }  // namespace
 
 // How many of the commands cmds[0..n) form one solver launch: consecutive
@@ -216,10 +233,10 @@ int gh_solver_run_length(const gh_cmd* cmds, int n) {
   while (len < n && len < kTensors && cmds[len].opcode == GH_OP_SOLVER_STEP && cmds[len].flags == cmds[0].flags &&
          cmds[len].ptr[4] == cmds[0].ptr[4] && memcmp(cmds[len].f, cmds[0].f, sizeof(cmds[0].f)) == 0 &&
          memcmp(cmds[len].dim + 1, cmds[0].dim + 1, sizeof(cmds[0].dim) - sizeof(cmds[0].dim[0])) == 0) {
-    // a tensor stepped twice keeps its two steps in order: the run ends before the repeat
-    bool repeat = false;
-    for (int j = 0; j < len; j++) repeat = repeat || cmds[j].ptr[0] == cmds[len].ptr[0];
-    if (repeat) break;
+    // steps that have to do with each other keep their order: the run ends before the later one
+    bool later = false;
+    for (int j = 0; j < len; j++) later = later || follows(cmds[j], cmds[len]);
+    if (later) break;
     len++;
   }
   return len;

@@ -71,6 +71,23 @@ def test_other_forms(ctx, form):
     _same(ctx, build)
 
 
+@pytest.mark.parametrize("kind", SETTINGS)
+@pytest.mark.parametrize("form", ["gradient from weights", "weights from gradient", "same cache", "overlap", "the same weights"])
+def test_steps_that_have_to_do_with_each_other(ctx, kind, form):
+    """The second of two steps reads or writes what the first writes, or writes what it reads: in the order of the commands."""
+    n = 300000
+
+    def build(t):
+        first, free = _step(t, kind, t.make(n + 64), t.make(n), n), _step(t, kind, t.make(n), t.make(n), n)
+        w, g = {"gradient from weights": (t.make(n), first.ptr[0]), "weights from gradient": (first.ptr[1], t.make(n)), "same cache": (t.make(n), t.make(n)),
+                "overlap": (first.ptr[0] + 256, t.make(n)), "the same weights": (first.ptr[0], t.make(n))}[form]
+        second = _step(t, kind, w, g, n)
+        if form == "same cache":
+            second.ptr[2] = first.ptr[2]
+        return [first, free, second]
+    _same(ctx, build)
+
+
 def test_operands_of_one_step_are_in_the_cache_account():
     layer = (8, 16, 52, 52, 32)
     n = _size(layer)
