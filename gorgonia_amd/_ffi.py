@@ -101,6 +101,7 @@ SYMBOLS = {
     "gh_gemm_route": (C.c_int, [C.POINTER(GhCmd), C.POINTER(C.c_int)]),
     "gh_runs_straight": (C.c_int, [C.POINTER(GhCmd)]),
     "gh_runs_split": (C.c_int, [C.POINTER(GhCmd)]),
+    "gh_joint_launches": (C.c_int64, [_P, C.c_int, C.POINTER(C.c_int64)]),
     "gh_touched_lately": (C.c_int, [_P, C.c_uint64]),
     "gh_gemm_can_softmax": (C.c_int, [C.POINTER(GhCmd)]),
     "gh_sync": (C.c_int, [_P]),
@@ -116,6 +117,9 @@ SYMBOLS = {
     "gh_event_elapsed_ms": (C.c_int, [_P, C.c_int, C.c_int, C.POINTER(C.c_float)]),
     "gh_version": (C.c_char_p, []),
 }
+
+# enum gh_joint
+JOINT_CONV_GRADIENTS, JOINT_DENSE_GRADIENTS, JOINT_SOLVER_SUMS = range(3)
 
 _lib = None
 

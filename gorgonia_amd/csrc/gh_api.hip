@@ -592,6 +592,12 @@ static int submit_cmds(gh_ctx* ctx, const gh_cmd* cmds, int n) {
   return rc ? rc : late;
 }
 
+int64_t gh_joint_launches(const gh_ctx* ctx, int kind, int64_t* form) {
+  if (!ctx || kind < 0 || kind >= GH_JOINT__COUNT) return -1;
+  if (form) *form = ctx->joint[kind].form;
+  return ctx->joint[kind].launches;
+}
+
 int gh_submit(gh_ctx* ctx, const gh_cmd* cmds, int n) {
   if (!ctx || n < 0 || (n > 0 && !cmds)) return GH_EINVAL;
   if (ctx->err) return ctx->err;

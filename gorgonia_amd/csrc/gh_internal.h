@@ -95,6 +95,7 @@ struct gh_ctx {
   bool defer_sums = false;
   bool hold_filter = false;   // the next filter gradient may be held
   gh_held_filter held;
+  struct { int64_t launches = 0, form = 0; } joint[GH_JOINT__COUNT];   // gh_joint_launches
   // set while gh_submit_noalloc runs: the scratch is the library's fixed array and a
   // plan may not shrink to fit it (results must not depend on the scratch size)
   bool ws_strict = false;

@@ -95,7 +95,10 @@ int go(gh_ctx* ctx, const Lanes<T>& g, int blocks) {
   return GH_OK;
 }
 
-int done(gh_ctx* ctx, int rc) {
+int done(gh_ctx* ctx, int rc, int tm, bool split) {
+  auto& j = ctx->joint[GH_JOINT_CONV_GRADIENTS];
+  j.launches += rc == GH_OK;
+  j.form = 100 * ctx->held.kind + 10 * tm + split;
   ctx->held.kind = kHeldNone;
   return rc ? rc : gh_check_hip(ctx, hipGetLastError(), "convolution gradients launch");
 }
@@ -108,11 +111,11 @@ int gh_try_launch_gradients(gh_ctx* ctx, const conv_lanes::Lanes<float>& g, int 
   using namespace conv_wgrad_small;
   if ((waves == 8) != split || getenv("GORGONIA_HIP_CONV_APART")) return -1;   // tuning switch: a launch each
   switch (ctx->held.kind) {
-    case kHeldSmall: return !split ? -1 : done(ctx, tm == 1 ? go_small<kWide, 1>(ctx, g, blocks) : go_small<kWide, 2>(ctx, g, blocks));
-    case kHeldSmallNarrow: return !split ? -1 : done(ctx, tm == 1 ? go_small<kNarrow, 1>(ctx, g, blocks) : go_small<kNarrow, 2>(ctx, g, blocks));
+    case kHeldSmall: return !split ? -1 : done(ctx, tm == 1 ? go_small<kWide, 1>(ctx, g, blocks) : go_small<kWide, 2>(ctx, g, blocks), tm, split);
+    case kHeldSmallNarrow: return !split ? -1 : done(ctx, tm == 1 ? go_small<kNarrow, 1>(ctx, g, blocks) : go_small<kNarrow, 2>(ctx, g, blocks), tm, split);
     case kHeldF32:
-      if (split) return done(ctx, tm == 1 ? go<float, 2, 4, 8, 1, 4, true>(ctx, g, blocks) : go<float, 2, 4, 8, 2, 4, true>(ctx, g, blocks));
-      return done(ctx, tm == 1 ? go<float, 2, 4, 4, 1, 4, false>(ctx, g, blocks) : go<float, 2, 4, 4, 2, 4, false>(ctx, g, blocks));
+      if (split) return done(ctx, tm == 1 ? go<float, 2, 4, 8, 1, 4, true>(ctx, g, blocks) : go<float, 2, 4, 8, 2, 4, true>(ctx, g, blocks), tm, split);
+      return done(ctx, tm == 1 ? go<float, 2, 4, 4, 1, 4, false>(ctx, g, blocks) : go<float, 2, 4, 4, 2, 4, false>(ctx, g, blocks), tm, split);
   }
   return -1;
 }
@@ -120,8 +123,8 @@ int gh_try_launch_gradients(gh_ctx* ctx, const conv_lanes::Lanes<float>& g, int 
 int gh_try_launch_gradients(gh_ctx* ctx, const conv_lanes::Lanes<double>& g, int waves, int tm, bool split, int blocks) {
   if (waves != 4 || tm != 1 || !split || getenv("GORGONIA_HIP_CONV_APART")) return -1;
   switch (ctx->held.kind) {
-    case kHeldF64: return done(ctx, go<double, 1, 4, 4, 1, 2, true>(ctx, g, blocks));
-    case kHeldF64Narrow: return done(ctx, go<double, 1, 2, 4, 1, 2, true>(ctx, g, blocks));
+    case kHeldF64: return done(ctx, go<double, 1, 4, 4, 1, 2, true>(ctx, g, blocks), tm, split);
+    case kHeldF64Narrow: return done(ctx, go<double, 1, 2, 4, 1, 2, true>(ctx, g, blocks), tm, split);
   }
   return -1;
 }

@@ -127,7 +127,7 @@ bool apart(const Span& a, const Span& b) { return a.at + (uint64_t)a.bytes <= b.
 
 }  // namespace
 
-static int try_launch(gh_ctx* ctx, const gh_cmd* cmds) {
+int gh_try_launch_gemm_gradients(gh_ctx* ctx, const gh_cmd* cmds) {
   if (getenv("GORGONIA_HIP_GEMM_APART")) return -1;   // tuning switch: a launch each
   const int w = (cmds[0].flags & GH_FLAG_TRANS_A) ? 0 : 1;
   const gh_cmd &dw = cmds[w], &dx = cmds[1 - w];
@@ -135,22 +135,24 @@ static int try_launch(gh_ctx* ctx, const gh_cmd* cmds) {
   if (kw.kind == kGemmOther) return -1;
   const gh_gemm_choice kx = gh_choose_gemm(ctx, dx);
   if (kx.kind == kGemmOther) return -1;
+  int rc;
   if (gh_dtype_of(dw.flags) == GH_F64)
-    return with64<true>(kw, dw, [&](const auto& p) {
+    rc = with64<true>(kw, dw, [&](const auto& p) {
       return with64<false>(kx, dx, [&](const auto& q) { return p.all() <= ctx->cu_count ? go(ctx, p, q) : go(ctx, q, p); });
     });
-  return with32<true, false>(kw, dw, [&](const auto& p) {
-    constexpr bool kDirect = std::decay_t<decltype(p)>::kDirect;
-    return with32<false, kDirect>(kx, dx, [&](const auto& q) { return go(ctx, q, p); });
-  });
-}
-
-int gh_try_launch_gemm_gradients(gh_ctx* ctx, const gh_cmd* cmds) {
-  const int rc = try_launch(ctx, cmds);
-  if (rc == GH_OK)
-    for (int k = 0; k < 2; k++)
-      for (uint64_t p : cmds[k].ptr) ctx->llc.touch(p, 0, false);
-  return rc;
+  else
+    rc = with32<true, false>(kw, dw, [&](const auto& p) {
+      constexpr bool kDirect = std::decay_t<decltype(p)>::kDirect;
+      return with32<false, kDirect>(kx, dx, [&](const auto& q) { return go(ctx, q, p); });
+    });
+  if (rc != GH_OK) return rc;
+  for (int k = 0; k < 2; k++)
+    for (uint64_t p : cmds[k].ptr) ctx->llc.touch(p, 0, false);
+  auto& j = ctx->joint[GH_JOINT_DENSE_GRADIENTS];
+  j.launches++;
+  auto digits = [](const gh_gemm_choice& k) { return 10000 * k.kind + 1000 * k.form + 10 * k.waves + k.columns; };
+  j.form = (int64_t)100000 * digits(kw) + digits(kx);
+  return GH_OK;
 }
 
 // Whether cmds[0] and cmds[1] are products of one size of float with the left operand of the one and the right operand of

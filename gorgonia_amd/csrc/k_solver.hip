@@ -302,5 +302,7 @@ int gh_try_launch_solver_sums(gh_ctx* ctx, const gh_cmd* cmds, int count, bool c
   const int waits = ctx->pending;
   ctx->pending = 0;
   ctx->slabs_used = 0;
+  ctx->joint[GH_JOINT_SOLVER_SUMS].launches++;
+  ctx->joint[GH_JOINT_SOLVER_SUMS].form = std::count_if(of_sum, of_sum + kTensors, [](int s) { return s >= 0; });
   return size == 8 ? launch<double>(ctx, cmds, count, copy, ctx->sums, waits, of_sum) : launch<float>(ctx, cmds, count, copy, ctx->sums, waits, of_sum);
 }

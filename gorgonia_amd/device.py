@@ -70,6 +70,11 @@ class Context:
         self.check(self.lib.gh_device_info(self.h, C.byref(d)))
         return d
 
+    def joint_launches(self, kind):
+        """Launches of this context's that ran several commands together (_ffi.JOINT_*), and which kernel the last one was."""
+        form = C.c_int64()
+        return self.lib.gh_joint_launches(self.h, kind, C.byref(form)), form.value
+
     # -- memory -----------------------------------------------------------------
     def malloc(self, nbytes):
         p = C.c_uint64()

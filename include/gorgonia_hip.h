@@ -388,6 +388,21 @@ GH_API int gh_runs_straight(const gh_cmd* cmd);
  * instructions that it would run on otherwise.  Host only; 256 compute units, as above. */
 GH_API int gh_runs_split(const gh_cmd* cmd);
 
+/* How many launches of the context's have run the work of several commands together, of one of these kinds, and in *form (may be
+ * null) which kernel the last of them was; -1 for another kind.  A launch that a graph records counts once.  Host only. */
+enum gh_joint {
+  /* a 3x3 convolution's two gradients (k_conv_gradients.hip): 100 x the filter gradient's kernel (1, 2: small images of more than
+   * and of up to 8 padded columns' pitch; 3: float32; 4, 5: float64 in chunks of 16 and of 8 columns) + 10 x the image gradient's
+   * filter tiles + whether its wavefronts split the channels */
+  GH_JOINT_CONV_GRADIENTS = 0,
+  /* a dense layer's two gradients (k_gemm_gradients.hip): 100000 x the weight gradient's product + the input gradient's, each
+   * 10000 x its kernel (1: k_gemm_direct, 2: a small-output kernel) + 1000 x its form + 10 x its wavefronts + its columns */
+  GH_JOINT_DENSE_GRADIENTS = 1,
+  /* solver steps with the sums of their gradients (k_solver.hip): how many of the sums are a step's */
+  GH_JOINT_SOLVER_SUMS = 2,
+  GH_JOINT__COUNT
+};
+GH_API int64_t gh_joint_launches(const gh_ctx* ctx, int kind, int64_t* form);
 /* 1 when the context's account of what the last-level cache holds has the buffer at p as touched lately, by commands
  * submitted through it.  An elementwise command over large tensors goes past the cache where it has none of its inputs;
  * the stored bits are the same.  Host only. */

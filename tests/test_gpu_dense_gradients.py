@@ -9,13 +9,23 @@ from tests.util import assert_bits_equal
 
 pytestmark = pytest.mark.gpu
 
-# (batch, inputs, outputs): each kernel with each it stands beside, tiles that the sizes fill and do not, the smallest
-# contractions, and products that one launch has no kernel for
-F32 = [(128, 1152, 625), (128, 625, 10), (8, 1152, 625), (8, 625, 10), (31, 1152, 625), (33, 625, 10), (49, 1152, 625), (200, 1152, 625), (64, 784, 300),
-       (64, 300, 100), (64, 100, 10), (37, 99, 41), (17, 530, 513), (16, 33, 600), (100, 47, 515), (5, 7, 9), (4, 16, 4), (300, 1152, 625), (2, 700, 10), (90, 2000, 30),
-       (15, 400, 300), (9, 37, 333), (12, 2500, 140)]
-F64 = [(50, 1152, 625), (50, 625, 10), (8, 1152, 625), (96, 1152, 625), (96, 625, 10), (13, 777, 300), (64, 300, 100), (100, 515, 77), (3, 5, 2), (70, 65, 260),
-       (129, 31, 64), (64, 500, 3000), (40, 1600, 1600), (24, 2000, 2000), (2, 64, 3), (51, 778, 2019)]
+# (batch, inputs, outputs) and the kernel that runs both (gh_joint_launches), None where each has a launch: every pair of kernels that a
+# draw of 13000 found, tiles that the sizes fill and do not, the smallest contractions, and products that one launch has no kernel for
+F32 = {
+    (128, 1152, 625): 1401020162, (128, 625, 10): 2008114010, (8, 1152, 625): 1401010080, (8, 625, 10): None, (31, 1152, 625): 1401020161,
+    (33, 625, 10): 2008114010, (49, 1152, 625): 1401020162, (200, 1152, 625): None, (64, 784, 300): 2008220081, (64, 300, 100): 2008120081,
+    (64, 100, 10): 2008114010, (37, 99, 41): 2008120081, (17, 530, 513): 1401020161, (16, 33, 600): 1401020161, (100, 47, 515): 2008120161,
+    (5, 7, 9): 1401014010, (4, 16, 4): 1401014010, (300, 1152, 625): None, (2, 700, 10): None, (90, 2000, 30): 2008114010,
+    (15, 400, 300): 1401010080, (9, 37, 333): 1401010080, (12, 2500, 140): 1401010080, (84, 751, 705): 1401020162, (66, 2860, 326): 1501010080,
+    (29, 5192, 229): 1501020082, (29, 999, 1092): 1501020161, (46, 2049, 558): 1501020162, (25, 204, 33): 1401020081, (17, 2615, 33): 1401020082,
+    (35, 24, 920): 2008120161, (87, 741, 32): 2008120082, (168, 1414, 35): 2008214010, (45, 1048, 50): 2008220081, (34, 1722, 38): 2008220082,
+    (43, 216, 763): 2008220161, (271, 231, 848): 2008220162, (49, 31, 1): 2008114010}
+F64 = {
+    (50, 1152, 625): 1200020081, (50, 625, 10): 1000010000, (8, 1152, 625): None, (96, 1152, 625): 1200020081, (96, 625, 10): 2004110000,
+    (13, 777, 300): 1000020081, (64, 300, 100): 2004120041, (100, 515, 77): 2004120041, (3, 5, 2): 1000010000, (70, 65, 260): 2004120081,
+    (129, 31, 64): 2004120041, (64, 500, 3000): 1100020081, (40, 1600, 1600): None, (24, 2000, 2000): None, (2, 64, 3): 1000010000,
+    (51, 778, 2019): 1000020081, (2, 4362, 33): 1100010000, (2, 1464, 177): 1100020041, (97, 1954, 713): 1200010000, (3, 2049, 246): 1200020041,
+    (163, 1289, 594): 1300010000, (39, 5223, 141): 1300020041, (106, 1764, 1371): 1400010000, (33, 1158, 1024): 1400020081, (67, 7, 3): 2004110000}
 CASES = [(np.float32,) + c for c in F32] + [(np.float64,) + c for c in F64]
 
 
@@ -43,7 +53,11 @@ def test_both_gradients(ctx, dt, batch, n_in, n_out, input_first):
         if input_first:
             cmds.reverse()
         if together:
+            before = ctx.joint_launches(_ffi.JOINT_DENSE_GRADIENTS)[0]
             ctx.run(cmds)
+            after, form = ctx.joint_launches(_ffi.JOINT_DENSE_GRADIENTS)
+            want = (F32 if dt == np.float32 else F64)[batch, n_in, n_out]
+            assert after - before == (want is not None) and want in (None, form)
         else:
             for c in cmds:
                 ctx.run([c])
@@ -78,6 +92,20 @@ def test_result_that_the_other_reads(ctx, which):
             ctx.free(p)
     for a, b in zip(*got):
         assert_bits_equal(a, b)
+
+
+def test_tuning_switch(ctx, monkeypatch):
+    """GORGONIA_HIP_GEMM_APART: a launch each."""
+    monkeypatch.setenv("GORGONIA_HIP_GEMM_APART", "1")
+    at = [ctx.upload(np.ones(1250, np.float32)) for _ in range(5)]
+    before = ctx.joint_launches(_ffi.JOINT_DENSE_GRADIENTS)
+    ctx.run(_commands(*at, 64, 15, 10, _ffi.F32))
+    assert ctx.joint_launches(_ffi.JOINT_DENSE_GRADIENTS) == before
+    monkeypatch.delenv("GORGONIA_HIP_GEMM_APART")
+    ctx.run(_commands(*at, 64, 15, 10, _ffi.F32))
+    assert ctx.joint_launches(_ffi.JOINT_DENSE_GRADIENTS)[0] == before[0] + 1
+    for p in at:
+        ctx.free(p)
 
 
 @pytest.mark.parametrize("dt", [np.float32, np.float64])

@@ -38,7 +38,10 @@ def test_steps_behind_their_gradients(ctx, kind, code, np_dt):
         steps = [_step(t, kind, t.make(_size(layer)), g.ptr[2], _size(layer), code) for g, layer in zip(grads[1:], LAYERS[1:])]
         steps.insert(3, _step(t, kind, t.make(777), t.make(777), 777, code))
         return grads + steps + [D.cmd_copy(t.make(300), t.make(300), 300 * np_dt().itemsize)]
+    before = ctx.joint_launches(_ffi.JOINT_SOLVER_SUMS)[0]
     _same(ctx, build, np_dt)
+    # six of the seven gradients that have a step waited for it
+    assert ctx.joint_launches(_ffi.JOINT_SOLVER_SUMS) == (before + 1, 6)
 
 
 @pytest.mark.parametrize("form", ["one", "two for one", "part", "weights", "cache", "copy", "other type", "three, two stepped"])
@@ -68,7 +71,11 @@ def test_other_forms(ctx, form):
             return [g, _step(t, "vanilla", t.make(n), dw, n), _step(t, "vanilla", w, g64, n, _ffi.F64)]
         second, third = _gradient(t, (64, 32, 14, 14, 64)), _gradient(t, (8, 64, 26, 26, 128))
         return [g, second, third, _step(t, "adam", t.make(n), dw, n), _step(t, "adam", t.make(64 * 32 * 9), second.ptr[2], 64 * 32 * 9)]
+    before = ctx.joint_launches(_ffi.JOINT_SOLVER_SUMS)[0]
     _same(ctx, build)
+    after, steps = ctx.joint_launches(_ffi.JOINT_SOLVER_SUMS)
+    want = {"one": 1, "other type": 1, "three, two stepped": 2}.get(form)   # steps that took their sum along
+    assert after - before == (want is not None) and want in (None, steps)
 
 
 @pytest.mark.parametrize("kind", SETTINGS)
