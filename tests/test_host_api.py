@@ -203,6 +203,28 @@ def test_tape_program_convnet_fusion():
     m2.Close()
 
 
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_tape_program_keeps_what_two_gradients_read(dt):
+    """A layer's two gradients run in one launch where neither's result lies in what the other reads: no register is given back
+    between the two, so that the second's cannot be one that the first read."""
+    inp = {k: v.astype(dt) for k, v in configs.convnet_inputs(2).items()}
+    onehot = np.eye(10, dtype=dt)[[3, 7]]
+    g, _ = configs.build_convnet_train(inp, onehot, 0.05, read_grads=False, solver="rmsprop")
+    m = G.NewTapeMachine(g, compile_only=True, fuse_activations=True)
+    lines = [l.split("\t", 1)[1] for l in m.program().splitlines() if "\t" in l]
+    m.Close()
+    runs = [i for i, l in enumerate(lines) if l.startswith("execOp")]
+    op = [lines[i].split()[4] for i in runs]
+    pairs = [k for k in range(len(op) - 1) if op[k:k + 2] in (["conv2d.diff.filter", "conv2d.diff.image"], ["matmul", "matmul"])]
+    assert [op[k] for k in pairs] == ["matmul", "matmul", "conv2d.diff.filter", "conv2d.diff.filter"]
+    freed_behind = 0
+    for k in pairs:
+        between, behind = lines[runs[k] + 1:runs[k + 1]], lines[runs[k + 1] + 1:runs[k + 2]]
+        assert all(l.startswith("alloc") for l in between), between
+        freed_behind += sum(l.startswith("free") for l in behind)
+    assert freed_behind >= 2 * len(pairs)
+
+
 def test_apply_refuses_functions_the_engine_does_not_have():
     """Operator kind, binary function and solver numbers are range-checked when the
     node is made (no name table is ever indexed with them); Mod is a real entry."""
