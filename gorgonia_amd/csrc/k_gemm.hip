@@ -1957,9 +1957,9 @@ __global__ __launch_bounds__(256) void k_conv3x3_wgrad_c1(const float* __restric
 // The same sums with loads ahead, for padded images of up to 1024 values.  What bounds it is what a workgroup waits for one behind
 // the other, so the first dy of an image are asked for with the image, in front of the barriers, each eight's successors before
 // the eight are multiplied, and the next image, kX values a thread, under the current one's sums.  us, slab sum included, before / now:
-// 128 x 28 x 28 -> 32 14.0 / 13.2, 384 of them 31.9 / 24.0, 200 x 28 x 28 -> 10 17.4 / 15.5, 130 x 31 x 29 -> 8 14.5 / 13.1.  Larger images,
+// 128 x 28 x 28 -> 32 13.3 / 12.6, 384 of them 30.9 / 22.2, 200 x 28 x 28 -> 10 17.2 / 15.1, 130 x 31 x 29 -> 8 14.2 / 12.8.  Larger images,
 // staged under the barriers, and planes of few pixels gained nothing from it (5 x 110 x 100 -> 6 32.8 / 33.7, 129 x 10 x 9 -> 33 11.9 / 12.3,
-// both against the kernel above when it moved a pixel past the end inside, which is 29.1 and 11.7 now).
+// both against the kernel above when it moved a pixel past the end inside, which is 29.0 and 11.4 now).
 __global__ __launch_bounds__(256) void k_conv3x3_wgrad_c1_ahead(const float* __restrict__ x, const float* __restrict__ dy,
                                                           float* __restrict__ ws, int B, int H, int W, int F, int pad,
                                                           int oh, int ow, unsigned m_ow, unsigned m_pw) {
