@@ -319,7 +319,8 @@ GH_API int gh_validate(const gh_cmd* cmds, int n, char* msg, int msg_len);
  * caller that times one operator by submitting it several times asks here whether it still does. */
 GH_API int gh_elementwise_run(const gh_cmd* cmds, int n);
 /* 1 when this CONV2D command may carry GH_FLAG_CONV_POOL2 (a convolution whose
- * kernel keeps a whole pooling window in one thread), else 0.  Host only.  The
+ * kernel keeps a whole pooling window in one thread), else 0; the answer holds
+ * on a device with any number of compute units.  Host only.  The
  * reference has no fused form: this folds maxpool.CUDADo
  * (ops/nn/maxpool_cuda.go:94-111) into convolution.CUDADo (convolution_cuda.go:95-121). */
 GH_API int gh_conv2d_can_pool(const gh_cmd* conv);
