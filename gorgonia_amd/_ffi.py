@@ -45,6 +45,7 @@ FLAG_GEMM_SOFTMAX = 1 << 27
 FLAG_GEMM_BIAS = 1 << 28
 FLAG_CONV_PRE = 1 << 29
 FLAG_CONV_KEEP = 1 << 30
+FLAG_BN_REMADE = 1 << 31
 
 
 def flag_fn(f):

@@ -557,6 +557,11 @@ static int submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
     }
     // two commands of which the second reads what the first writes are one launch where a kernel takes both
     const bool held = gh_bn_held_pair(ctx, cmds + i, n - i), pair = held || gh_is_pair(cmds + i, n - i);
+    if (cmds[i].opcode == GH_OP_MAXPOOL2D_BWD && (cmds[i].flags & GH_FLAG_BN_REMADE)) {
+      if (!gh_bn_remade_follows(cmds + i, n - i)) return gh_fail(ctx, GH_EINVAL, "cmd " + std::to_string(i) + ": maxpool2d gradient: the batch normalisation's gradient does not follow");
+      if ((rc = gh_flush_sums_before(ctx, cmds[i + 1]))) return rc;
+      if (!held && (rc = gh_launch_bn_remake(ctx, cmds + i))) return rc;
+    }
     if (pair && (rc = gh_flush_sums_before(ctx, cmds[i + 1]))) return rc;
     rc = held ? gh_launch_bn_held_pair(ctx, cmds + i) : pair ? gh_launch_pair(ctx, cmds + i) : dispatch(ctx, cmds[i]);
     if (rc) return rc;

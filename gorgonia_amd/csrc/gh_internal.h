@@ -137,6 +137,8 @@ int gh_flush_sums_before(gh_ctx* ctx, const gh_cmd& c);
 int gh_bn_groups(int64_t n, int64_t S);   // the groups of 256 threads that k_bn_reduce cuts a channel of n values in planes of S into (k_bwd.hip)
 // {BN_TRAIN, MAXPOOL2D} and {MAXPOOL2D_BWD, BN_BWD} in one launch (k_bn_held.hip)
 bool gh_bn_held_pair(const gh_ctx* ctx, const gh_cmd* cmds, int n);
+bool gh_bn_remade_follows(const gh_cmd* c, int n);
+int gh_launch_bn_remake(gh_ctx* ctx, const gh_cmd* c);
 int gh_launch_bn_held_pair(gh_ctx* ctx, const gh_cmd* cmds);
 // a run of elementwise commands in one pass (k_chain.hip): how many commands at the front of cmds one pass can take and is
 // quicker for (0 or >= 2; gh_elementwise_run asks the same), and the launch

@@ -142,6 +142,8 @@ int gh_validate_cmd(const gh_cmd& c, std::string& msg) {
       if (dt > GH_F64) return bad("Unsupported Dtype");
       if (dt == GH_F64 && (c.flags & GH_FLAG_ACT_RELU) && c.opcode == GH_OP_MAXPOOL2D_BWD)
         return bad("maxpool2d gradient: no Rectify on the input for float64");
+      if (c.opcode == GH_OP_MAXPOOL2D_BWD && (c.flags & GH_FLAG_BN_REMADE) && (dt != GH_F32 || !(c.flags & GH_FLAG_ACT_RELU)))
+        return bad("maxpool2d gradient: a batch normalisation is made again for float32 behind a Rectify only");
       return GH_OK;
     }
     case GH_OP_BN_INFER:

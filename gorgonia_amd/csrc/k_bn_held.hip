@@ -19,6 +19,11 @@
 // gradient moves), 8 x 32 x 104 x 104 20.5 / 12.6 and 22.9 / 13.1, 8 x 128 x 26 x 26 14.2 / 9.8 and 13.4 / 7.7,
 // 8 x 16 x 207 x 207 (single loads) 46.6 / 20.9 and 47.3 / 25.9, 2 x 3 x 4 x 4 12.1 / 8.9 and 10.0 / 5.7.  (The forward as the
 // gradient is, its values kept as the pooling's windows lie: 14.8, 9.9 and 7.3, and other sums.)
+// Where the normalised values are read by the pooling and its gradient only (GH_FLAG_BN_REMADE, a training step), the forward
+// leaves them out and the gradient makes them again from what it reads anyway, and passes its own middle result on in registers:
+// 44 MB less of 50 and 94 for 8 x 16 x 208 x 208.  In the step of the four-block network, traced, 21.3 -> 18.8 and 22.9 -> 18.1,
+// 8 x 32 x 104 x 104 13.0 -> 11.9 and 14.5 -> 11.8, 8 x 64 x 52 x 52 10.0 -> 9.1 and 10.6 -> 8.8, 8 x 128 x 26 x 26 9.7 -> 9.4 and
+// 8.1 -> 7.3; the step 408.6 -> 393.5.  What is left is the launch, the first loads and the two waits.
 #include <algorithm>
 #include <cfloat>
 
@@ -191,6 +196,7 @@ struct Cut {
 // The forward sums are k_bn_reduce's to the bit: where one order of additions sends a value to one side of a rectifier's
 // step or a window's maximum and another order to the other, a whole gradient element goes with it.
 // HELD: groups of four images that a thread keeps in registers between its two passes (0: it reads them again).
+// y null: the normalised values are only pooled (GH_FLAG_BN_REMADE).
 template <int COLS, bool EDGES, int HELD>
 __global__ __launch_bounds__(kThreads) void k_bn_train_pool(const float* __restrict__ x, float* __restrict__ y, float* __restrict__ pooled, Planes g, Cut cut, int64_t n,
                                                             BnOut o, u64* page) {
@@ -325,7 +331,7 @@ __global__ __launch_bounds__(kThreads) void k_bn_train_pool(const float* __restr
           const float m = z[r][e] * a;
           z[r][e] = m + b;
         }
-      q.store(g, y + q.at(g, c), z);
+      if (y) q.store(g, y + q.at(g, c), z);
       if (EDGES && !(q.right && q.below)) continue;
       float best[COLS / 2];
 #pragma unroll
@@ -346,8 +352,9 @@ __global__ __launch_bounds__(kThreads) void k_bn_train_pool(const float* __restr
 }
 
 // x: the tensor that was rectified and pooled; dp: the pooled tensor's gradient; dx: the gradient of x; z: the tensor that was
-// normalised; dz its gradient (which may take x's or z's place).
-template <int COLS, bool EDGES, int N>
+// normalised; dz its gradient (which may take x's or z's place).  REMADE: x is z normalised with the saved statistics, made
+// again here in the forward's two operations, and neither x nor dx is touched.
+template <int COLS, bool EDGES, int N, bool REMADE>
 __global__ __launch_bounds__(kThreads) void k_pool_bn_bwd(const float* x, const float* __restrict__ dp, float* __restrict__ dx, const float* z, float* dz, Planes g,
                                                           int64_t n, const float* __restrict__ save_mean, const float* __restrict__ save_var, float eps, u64* page) {
   __shared__ Sums sh;
@@ -356,6 +363,7 @@ __global__ __launch_bounds__(kThreads) void k_pool_bn_bwd(const float* x, const 
   bool claimed = false;
   if (threadIdx.x == 0 && !(g.polls == 0 && (w & 1))) claimed = claim(ch, w);
   const float mean = save_mean[c], vb = save_var[c] / (float)n;
+  const float invstd = 1.0f / sqrtf(vb + eps), shift = -mean * invstd;
   float zv[N][2][COLS], gv[N][2][COLS];
   // unit k of a thread in share `who`
   auto has = [&](int who, int k) { return k * (int)blockDim.x + (int)threadIdx.x < g.per && who * g.per + k * (int)blockDim.x + (int)threadIdx.x < g.units; };
@@ -363,7 +371,7 @@ __global__ __launch_bounds__(kThreads) void k_pool_bn_bwd(const float* x, const 
   auto load = [&](int who, int k, float (&hz)[2][COLS], float (&hg)[2][COLS], float (&d)[COLS / 2]) __attribute__((always_inline)) {
     if (!has(who, k)) return;
     const Unit<COLS, EDGES> t = unit(who, k);
-    t.load(g, x + t.at(g, c), hg);
+    if constexpr (!REMADE) t.load(g, x + t.at(g, c), hg);
     t.load(g, z + t.at(g, c), hz);
     const float* const p = dp + t.pooled(g, c);
     if constexpr (COLS == 4) {
@@ -375,10 +383,18 @@ __global__ __launch_bounds__(kThreads) void k_pool_bn_bwd(const float* x, const 
     }
   };
   float s, dot;
-  auto add = [&](int who, int k, const float (&hz)[2][COLS], float (&hg)[2][COLS], const float (&d)[COLS / 2]) __attribute__((always_inline)) {
-    if (!has(who, k)) return;
-    const Unit<COLS, EDGES> t = unit(who, k);
+  // a unit's gradient of x, where x was (REMADE: is made)
+  auto gradient = [&](const Unit<COLS, EDGES>& t, const float (&hz)[2][COLS], float (&hg)[2][COLS], const float (&d)[COLS / 2]) __attribute__((always_inline)) {
     const bool whole = t.right && t.below;
+    if constexpr (REMADE) {
+#pragma unroll
+      for (int r = 0; r < 2; r++)
+#pragma unroll
+        for (int e = 0; e < COLS; e++) {
+          const float m = hz[r][e] * invstd;
+          hg[r][e] = m + shift;
+        }
+    }
 #pragma unroll
     for (int e = 0; e < COLS / 2; e++) {
       float best = -FLT_MAX;
@@ -396,7 +412,12 @@ __global__ __launch_bounds__(kThreads) void k_pool_bn_bwd(const float* x, const 
         h = whole ? o * relu_mask(h) : 0.0f;
       }
     }
-    t.store(g, dx + t.at(g, c), hg);
+  };
+  auto add = [&](int who, int k, const float (&hz)[2][COLS], float (&hg)[2][COLS], const float (&d)[COLS / 2]) __attribute__((always_inline)) {
+    if (!has(who, k)) return;
+    const Unit<COLS, EDGES> t = unit(who, k);
+    gradient(t, hz, hg, d);
+    if constexpr (!REMADE) t.store(g, dx + t.at(g, c), hg);
     float s4[2][COLS], d4[2][COLS];
 #pragma unroll
     for (int r = 0; r < 2; r++)
@@ -451,7 +472,6 @@ __global__ __launch_bounds__(kThreads) void k_pool_bn_bwd(const float* x, const 
   }
   sum[0] = total(sh, 0, g.G);
   sum[1] = total(sh, 1, g.G);
-  const float invstd = 1.0f / sqrtf(vb + eps);
   float f = sum[1] * invstd;
   f = f * invstd;
   f = f / (float)n;
@@ -474,14 +494,19 @@ __global__ __launch_bounds__(kThreads) void k_pool_bn_bwd(const float* x, const 
     if (!has(w, k)) break;
     finish(unit(w, k), zv[k], gv[k]);
   }
-  for (; more; more &= more - 1) {   // (a thread reads the gradient that it has written)
+  for (; more; more &= more - 1) {   // (a thread reads the gradient that it has written, or makes it again)
     const int who = __builtin_ctzll(more);
 #pragma unroll 1
     for (int k = 0; k < N && has(who, k); k++) {
       const Unit<COLS, EDGES> t = unit(who, k);
-      float hz[2][COLS], hg[2][COLS];
-      t.load(g, z + t.at(g, c), hz);
-      t.load(g, dx + t.at(g, c), hg);
+      float hz[2][COLS], hg[2][COLS], d[COLS / 2];
+      if constexpr (REMADE) {
+        load(who, k, hz, hg, d);
+        gradient(t, hz, hg, d);
+      } else {
+        t.load(g, z + t.at(g, c), hz);
+        t.load(g, dx + t.at(g, c), hg);
+      }
       finish(t, hz, hg);
     }
   }
@@ -632,15 +657,64 @@ int gh_launch_bn_held_pair(gh_ctx* ctx, const gh_cmd* c) {
   u64* const page = (u64*)ctx->bn_page;
   if (fwd) {
     const BnOut o{at<float>(bn.ptr[2]), at<float>(bn.ptr[3]), at<float>(bn.ptr[4]), at<float>(bn.ptr[5]), bn.f[0], bn.f[1]};
+    float* const y = bn.flags & GH_FLAG_BN_REMADE ? nullptr : at<float>(bn.ptr[1]);
     with_held(p, [&](auto COLS, auto EDGES, auto HELD) {
-      hipLaunchKernelGGL((k_bn_train_pool<COLS(), EDGES(), HELD()>), grid, block, 0, ctx->stream, at<const float>(bn.ptr[0]), at<float>(bn.ptr[1]), at<float>(pool.ptr[1]), p.g,
-                         p.cut, count, o, page);
+      hipLaunchKernelGGL((k_bn_train_pool<COLS(), EDGES(), HELD()>), grid, block, 0, ctx->stream, at<const float>(bn.ptr[0]), y, at<float>(pool.ptr[1]), p.g, p.cut, count, o, page);
     });
   } else {
+    const bool remade = pool.flags & GH_FLAG_BN_REMADE;
     with_form(p, [&](auto COLS, auto EDGES, auto UNITS) {
-      hipLaunchKernelGGL((k_pool_bn_bwd<COLS(), EDGES(), UNITS()>), grid, block, 0, ctx->stream, at<const float>(pool.ptr[0]), at<const float>(pool.ptr[1]),
-                         at<float>(pool.ptr[2]), at<const float>(bn.ptr[0]), at<float>(bn.ptr[2]), p.g, count, at<const float>(bn.ptr[3]), at<const float>(bn.ptr[4]), bn.f[0], page);
+      const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, at<const float>(pool.ptr[0]), at<const float>(pool.ptr[1]), at<float>(pool.ptr[2]), at<const float>(bn.ptr[0]),
+                           at<float>(bn.ptr[2]), p.g, count, at<const float>(bn.ptr[3]), at<const float>(bn.ptr[4]), bn.f[0], page);
+      };
+      if (remade) go(k_pool_bn_bwd<COLS(), EDGES(), UNITS(), true>);
+      else go(k_pool_bn_bwd<COLS(), EDGES(), UNITS(), false>);
     });
   }
   return gh_check_hip(ctx, hipGetLastError(), fwd ? "batchnorm statistics launch" : "batchnorm backward launch");
+}
+
+namespace {
+
+// y = z normalised with the saved statistics, one (image, channel) plane per blockIdx.y: the forward's two operations.
+__global__ __launch_bounds__(256) void k_bn_remake(const float* __restrict__ z, float* __restrict__ y, const float* __restrict__ save_mean, const float* __restrict__ save_var, float eps,
+                                                   int64_t BC, int C, int64_t S, int64_t n) {
+  for (int64_t bc = blockIdx.y; bc < BC; bc += gridDim.y) {
+    const int c = (int)(bc % C);
+    const float a = 1.0f / sqrtf(save_var[c] / (float)n + eps), b = -save_mean[c] * a;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < S; i += (int64_t)gridDim.x * 256) {
+      const float m = z[bc * S + i] * a;
+      y[bc * S + i] = m + b;
+    }
+  }
+}
+
+}  // namespace
+
+// (256 compute units, tensors at whole lines: what the tape's tensors have)
+int gh_bn_can_remake(int64_t B, int64_t C, int64_t H, int64_t W) {
+  gh_cmd pool{};
+  pool.flags = GH_FLAG_DTYPE(GH_F32) | GH_FLAG_ACT_RELU;
+  const int64_t dims[12] = {B, C, H, W, 2, 2, 0, 0, 0, 0, 2, 2};
+  std::copy(dims, dims + 12, pool.dim);
+  Plan p;
+  return pools(pool) && plan(pool, true, 0, 0, 256, p) && plan(pool, false, 0, 0, 256, p);
+}
+
+// Whether c[1] is the batch normalisation's gradient that a MAXPOOL2D_BWD command with GH_FLAG_BN_REMADE needs behind it.
+bool gh_bn_remade_follows(const gh_cmd* c, int n) {
+  std::string m;
+  return n >= 2 && c[1].opcode == GH_OP_BN_BWD && gh_dtype_of(c[1].flags) == GH_F32 && !(c[1].flags & GH_FLAG_BN_EVAL) && gh_validate_cmd(c[1], m) == GH_OK &&
+         c[1].ptr[1] == c[0].ptr[2] && c[1].dim[0] == c[0].dim[0] && c[1].dim[1] == c[0].dim[1] && c[1].dim[2] == c[0].dim[2] * c[0].dim[3];
+}
+
+// The tensor that such a pair needs where no kernel takes it whole: into the place that the first command names.
+int gh_launch_bn_remake(gh_ctx* ctx, const gh_cmd* c) {
+  const gh_cmd& bn = c[1];
+  const int64_t BC = bn.dim[0] * bn.dim[1], S = bn.dim[2];
+  const dim3 grid((unsigned)std::min<int64_t>(1024, (S + 1023) / 1024), (unsigned)std::min<int64_t>(BC, 65535));
+  hipLaunchKernelGGL(k_bn_remake, grid, dim3(256), 0, ctx->stream, at<const float>(bn.ptr[0]), at<float>(c[0].ptr[0]), at<const float>(bn.ptr[3]), at<const float>(bn.ptr[4]), bn.f[0], BC,
+                     (int)bn.dim[1], S, bn.dim[0] * S);
+  return gh_check_hip(ctx, hipGetLastError(), "batchnorm launch");
 }

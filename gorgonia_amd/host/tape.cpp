@@ -476,7 +476,7 @@ Status CUDADo(Engine& e, const OpSpec& op, Tensor& prealloc, const std::vector<T
       if (x.dt == Dtype::Other || in[1]->dt != x.dt) return bad("MaxPool2DDiff: Unsupported Dtype");
       gh_cmd c{};
       c.opcode = GH_OP_MAXPOOL2D_BWD;
-      c.flags = (np == 4 ? GH_FLAG_EXPLICIT_PAD : 0) | (op.relu_input ? GH_FLAG_ACT_RELU : 0) | dtype_flag(x.dt);
+      c.flags = (np == 4 ? GH_FLAG_EXPLICIT_PAD : 0) | (op.relu_input ? GH_FLAG_ACT_RELU : 0) | (op.remade ? GH_FLAG_BN_REMADE : 0) | dtype_flag(x.dt);
       c.ptr[0] = x.mem; c.ptr[1] = in[1]->mem; c.ptr[2] = prealloc.mem;
       for (int i = 0; i < 4; i++) c.dim[i] = x.shape[i];
       c.dim[4] = p[0]; c.dim[5] = p[1];
@@ -515,6 +515,7 @@ Status CUDADo(Engine& e, const OpSpec& op, Tensor& prealloc, const std::vector<T
       c.dim[3] = double_bits(op.f0);   // float64: epsilon (and momentum below) as doubles
       if (op.kind == OpKind::BatchNormTrain) {
         c.opcode = GH_OP_BN_TRAIN;
+        if (op.remade) c.flags |= GH_FLAG_BN_REMADE;
         c.ptr[0] = x.mem; c.ptr[1] = prealloc.mem;
         for (int i = 0; i < 4; i++) c.ptr[2 + i] = in[(size_t)(1 + i)]->mem;
         c.f[1] = (float)op.f1;
@@ -765,7 +766,66 @@ int Graph::FuseActivations() {
   fused += fuse_pooled_rectify();
   fused += fuse_first_layer();
   fused += fuse_kept_conv();
+  mark_remade_batchnorm();
   return fused;
+}
+
+// The training pattern around batch statistics:
+//   n = BatchNormTrain(z, ...); p = MaxPool2D(Rectify(n)); ...; dn = MaxPool2DDiff(Rectify(n), g) with RectifyDiff;
+//   dz = BatchNormDiff(z, dn, ...)
+// with n read by nothing but the two and dn by nothing but dz, directly behind it: n is made again from z and the saved
+// statistics where the gradient needs it, and neither n nor dn is stored where one launch does both operators of a pair.
+void Graph::mark_remade_batchnorm() {
+  const size_t N = nodes_.size();
+  std::vector<int> root(N);
+  for (size_t i = 0; i < N; i++) root[i] = nodes_[i].alias_of >= 0 ? root[(size_t)nodes_[i].alias_of] : (int)i;
+  std::vector<std::vector<int>> users(N);
+  for (auto& n : nodes_)
+    if (!n.fused_away)
+      for (int i : n.inputs) users[(size_t)i].push_back(n.id);
+  for (auto& bn : nodes_) {
+    if (bn.fused_away || bn.is_input || bn.read_into || bn.alias_of >= 0 || bn.op.kind != OpKind::BatchNormTrain || bn.dt != Dtype::Float32) continue;
+    if (bn.inputs.size() != 5 || users[(size_t)bn.id].size() != 2) continue;
+    Node *pool = nullptr, *diff = nullptr;
+    for (int u : users[(size_t)bn.id]) {
+      Node& n = nodes_[(size_t)u];
+      if (n.op.kind == OpKind::MaxPool2D && n.op.relu_input && n.inputs.size() == 1) pool = &n;
+      if (n.op.kind == OpKind::MaxPool2DDiff && n.op.relu_input && n.inputs.size() == 2 && n.inputs[0] == bn.id) diff = &n;
+    }
+    if (!pool || !diff || diff->read_into || users[(size_t)diff->id].size() != 1) continue;
+    const Node& dz = nodes_[(size_t)users[(size_t)diff->id][0]];
+    const int z = bn.inputs[0], mean = bn.inputs[3], var = bn.inputs[4];
+    if (dz.op.kind != OpKind::BatchNormDiff || dz.inputs != std::vector<int>{z, diff->id, mean, var} || dz.op.f0 != bn.op.f0) continue;
+    // nothing runs between the two gradients, and nothing writes z or the statistics between the first operator and the last
+    bool clear = dz.id > diff->id && diff->id > bn.id;
+    for (int j = diff->id + 1; j < dz.id && clear; j++) {
+      const Node& n = nodes_[(size_t)j];
+      clear = n.fused_away || n.is_input || n.deferred || (n.alias_of >= 0 && n.op.kind == OpKind::Reshape);
+    }
+    auto touches = [&](int node) {
+      for (int k : {z, mean, var})
+        if (root[(size_t)k] == root[(size_t)node]) return true;
+      return false;
+    };
+    clear = clear && !touches(bn.inputs[1]) && !touches(bn.inputs[2]) && root[(size_t)mean] != root[(size_t)var] && root[(size_t)z] != root[(size_t)mean] &&
+            root[(size_t)z] != root[(size_t)var];
+    for (int j = bn.id + 1; j < dz.id && clear; j++) {
+      const Node& n = nodes_[(size_t)j];
+      if (n.fused_away || n.is_input) continue;
+      if (n.op.kind == OpKind::Set || n.op.kind == OpKind::SolverStep)
+        for (int in : n.inputs) clear = clear && !touches(in);
+      if (n.op.kind == OpKind::BatchNormTrain)
+        for (size_t k = 1; k < n.inputs.size(); k++) clear = clear && !touches(n.inputs[k]);
+    }
+    if (!clear) continue;
+    const auto& q = diff->op.ints;  // kh kw npad pads... sh sw
+    bool plain = q.size() >= 5 && q[0] == 2 && q[1] == 2;
+    for (size_t i = 3; plain && i < q.size(); i++) plain = q[i] == (i >= 3 + (size_t)q[2] ? 2 : 0);
+    const Shape& s = bn.shape;
+    if (!plain || pool->op.ints != q || s.Dims() != 4 || !gh_bn_can_remake(s[0], s[1], s[2], s[3])) continue;
+    bn.op.remade = true;
+    diff->op.remade = true;
+  }
 }
 
 // z = Conv2d(x, w); p = MaxPool2D(z) 2x2/2 (read through a Rectify or not) where other nodes read z as well -
@@ -1421,7 +1481,13 @@ Status TapeMachine::RunAll() {
           ins[k].shape = s.shape;
           inp[k] = &ins[k];
         }
-        st = CUDADo(eng_, n.op, out, inp);
+        if (n.op.remade && (watched || opt_.node_at_a_time)) {   // every value is looked at, or every operator submitted alone
+          OpSpec stored = n.op;
+          stored.remade = false;
+          st = CUDADo(eng_, stored, out, inp);
+        } else {
+          st = CUDADo(eng_, n.op, out, inp);
+        }
         if (!st.ok()) return st.Wrap("PC " + std::to_string(pc) + ": " + op_name(n.op));
         if (moves) {
           regs_[(size_t)in.reg].mem = out.mem;

@@ -90,6 +90,10 @@ struct OpSpec {
   // MaxPool2D / MaxPool2DDiff: input 0 is the value before a Rectify and is read through it; the
   // diff also applies the Rectify's own gradient (it stands for RectifyDiff(z, MaxPool2DDiff(Rectify(z), g)))
   bool relu_input = false;
+  // BatchNormTrain, MaxPool2DDiff: the normalised values between them are read by nothing else but the pool behind the
+  // first, and the second's result by the BatchNormDiff behind it only, which knows what to make them of again
+  // (GH_FLAG_BN_REMADE).
+  bool remade = false;
 };
 
 // Output shape of an op (InferShape of each reference op); error if the inputs
@@ -138,6 +142,7 @@ class Graph {
   // and inputs; the values it stores are bit-identical to the unfused chain's.
   // Returns the number of operators folded away.
   int FuseActivations();
+  void mark_remade_batchnorm();   // part of FuseActivations: normalised values that need not be stored
   int fuse_pooled_rectify();   // part of FuseActivations: the Rectify between a pool and both gradients
   int fuse_first_layer();      // part of FuseActivations: a single-channel first layer folded into the next convolution
   int fuse_rectify_into_pool();   // part of FuseActivations: a Rectify read by nothing but a pool (float64 convolutions have no epilogue)

@@ -135,6 +135,7 @@ enum gh_unaryfn {
 #define GH_FLAG_GEMM_SOFTMAX (1u << 27)   /* GEMM: row SoftMax on the result (after the activation) */
 #define GH_FLAG_CONV_PRE     (1u << 29)   /* CONV2D: the input is made on the fly from single-channel images, see below */
 #define GH_FLAG_CONV_KEEP    (1u << 30)   /* CONV2D with CONV_POOL2: ptr[7] also receives the unpooled result, see below */
+#define GH_FLAG_BN_REMADE    (1u << 31)   /* BN_TRAIN, MAXPOOL2D_BWD: the normalised values need not be stored, see below */
 #define GH_FLAG_GEMM_BIAS    (1u << 28)   /* GEMM (untransposed): ptr[3] = N floats added to every row of the product (before the activation) */
 
 /*
@@ -199,11 +200,18 @@ enum gh_unaryfn {
  *             GH_FLAG_ACT_RELU (float32): x is the value before a Rectify whose result was
  *             pooled; dx = (x>=0) * that gradient taken over x*(x>=0) - MaxPool2DDiff then the
  *             activation's gradient, with their bits, in one pass
+ *             BN_REMADE (float32, with ACT_RELU): x is what a BN_TRAIN command made of the x that the
+ *             BN_BWD command directly behind this one (same B, C, H*W; its dy is this command's dx) is
+ *             given with its statistics.  ptr[0] is memory for such a tensor whose contents do not
+ *             count, the values are made again where they are needed, with the same bits; ptr[0] and
+ *             ptr[2] hold nothing in particular afterwards
  * CONV2D_BWD_DATA   ptr[0]=dy ptr[1]=w ptr[2]=dx ; dims as CONV2D (B,C,H,W describe x / dx)
  * CONV2D_BWD_FILTER ptr[0]=x ptr[1]=dy ptr[2]=dw ; dims as CONV2D
  * BN_TRAIN    ptr[0]=x ptr[1]=y ptr[2]=running_mean ptr[3]=running_var (both updated)
  *             ptr[4]=save_mean ptr[5]=save_var (outputs; save_var is the SUM of squared
  *             deviations, op_nn.go:1536-1541)  dim[0..2]=B,C,S  f[0]=eps f[1]=momentum
+ *             BN_REMADE (float32): y may be left unstored where the MAXPOOL2D command behind this one
+ *             is done in the same launch; nothing else but MAXPOOL2D_BWD with the flag reads it
  * BN_BWD      ptr[0]=x ptr[1]=dy ptr[2]=dx ptr[3]=save_mean ptr[4]=save_var
  *             dim[0..2]=B,C,S  f[0]=eps ; BN_EVAL selects dx = dy/sqrt(save_var/n + eps)
  * SOFTMAX_BWD ptr[0]=y ptr[1]=dy ptr[2]=dx        dim[0]=rows dim[1]=cols
@@ -329,6 +337,9 @@ GH_API int gh_conv2d_can_pool(const gh_cmd* conv);
  * runs the first layer of its convolutional example as three operators with two stored tensors
  * between them (examples/convnet/main.go:86-112); folded, a step has one kernel and one tensor less. */
 GH_API int gh_conv2d_can_pre(const gh_cmd* conv);
+/* 1 where GH_FLAG_BN_REMADE pays for a B x C x H x W tensor: both of its pairs of commands (2x2 / 2 pooling) are one launch
+ * each on 256 compute units.  Host only. */
+GH_API int gh_bn_can_remake(int64_t B, int64_t C, int64_t H, int64_t W);
 /* 1 when gh_submit accepts GH_FLAG_CONV_KEEP on this float32 CONV2D command with CONV_POOL2.  Host only.
  * The reference's training graph stores the convolution's result and runs the activation and the pool
  * as operators of their own (examples/convnet/main.go:86-112); here the convolution stores both. */

@@ -255,3 +255,71 @@ def test_two_contexts_at_once(ctx):
             got = m.all()
             for k in want:
                 assert_bits_equal(got[k], want[k])
+
+
+def _remade(fwd, bwd):
+    fwd[0].flags |= _ffi.FLAG_BN_REMADE
+    bwd[0].flags |= _ffi.FLAG_BN_REMADE
+    return fwd, bwd
+
+
+@pytest.mark.parametrize("polls", [None, 0, 1])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_values_that_are_not_stored(ctx, shape, polls, monkeypatch):
+    """GH_FLAG_BN_REMADE: what is still written has the bits of the commands without it, whatever lay in y's place; "t" as the
+    gradient's place is no pair of one launch, so that the values are made again by a kernel of their own."""
+    for dz in ("dz", "y", "t"):
+        _, want = _run(ctx, shape, 12, dz=dz)
+        if polls is not None:
+            monkeypatch.setenv("GORGONIA_HIP_BN_POLLS", str(polls))
+        with monkeypatch.context() as p:
+            p.setitem(globals(), "_commands", lambda *a, plain=_commands, **kw: _remade(*plain(*a, **kw)))
+            _, got = _run(ctx, shape, 12, dz=dz)
+        monkeypatch.delenv("GORGONIA_HIP_BN_POLLS", raising=False)
+        for k in ("x", "p", "sm", "sv", "rm", "rv", "dp", dz):
+            assert_bits_equal(got[k], want[k], (dz, k))
+
+
+def test_a_command_that_needs_the_one_behind_it(ctx):
+    shape = (2, 3, 4, 4)
+    x, rm, rv, dp = _inputs(shape, 13)
+    m = _Place(ctx, 0, x=x, y=x, p=dp, rm=rm, rv=rv, sm=rm, sv=rv, dp=dp, t=x, dz=x)
+    _, bwd = _remade(*_commands(m, shape))
+    with pytest.raises(D.DeviceError):
+        ctx.run(bwd[:1])
+    ctx.clear_error()
+    ctx.run(bwd)
+    m.all()
+
+
+@pytest.mark.parametrize("read", [None, "n", "dn"])
+def test_on_a_tape(ctx, read):
+    """A graph's normalised values are left out only where nobody else reads them: the same bits as operator by operator."""
+    from gorgonia_amd import graph as G
+    shape = (4, 16, 12, 12)
+    x, rm0, rv0, dp = _inputs(shape, 14)
+
+    def run(machine, **kw):
+        g = G.NewGraph()
+        z = G.LeakyRelu(G.NewTensor(g, x), 0.5)
+        rm, rv, sm, sv = (G.NewTensor(g, v.copy(), resident=True) for v in (rm0, rv0, rm0 * 0, rm0 * 0))
+        n = G.BatchNormTrain(z, rm, rv, sm, sv, momentum=MOMENTUM, epsilon=EPS)
+        a = G.Rectify(n)
+        p = G.MaxPool2D(a, (2, 2), (0, 0), (2, 2))
+        dn = G.RectifyDiff(n, G.MaxPool2DDiff(a, G.HadamardProd(p, G.NewTensor(g, dp)), (2, 2), (0, 0), (2, 2)))
+        dz = G.BatchNormDiff(z, dn, sm, sv, epsilon=EPS)
+        out = {"dz": G.Read(dz), "p": G.Read(p), "rm": G.Read(rm), "rv": G.Read(rv)}
+        if read:
+            out[read] = G.Read({"n": n, "dn": dn}[read])
+        m = machine(g, **kw)
+        for _ in range(3):
+            m.RunAll()
+        got = {k: v.copy() for k, v in out.items()}
+        m.Close()
+        return got
+    fused, apart = run(G.NewTapeMachine, fuse_activations=True), run(G.NewLispMachine)
+    for k in apart:
+        if k == "dz":   # two orders of adding the gradient's sums
+            assert rel_frobenius(fused[k], apart[k].astype(np.float64)) <= U
+        else:
+            assert_bits_equal(fused[k], apart[k], k)
