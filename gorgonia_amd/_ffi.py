@@ -120,7 +120,7 @@ SYMBOLS = {
 }
 
 # enum gh_joint
-JOINT_CONV_GRADIENTS, JOINT_DENSE_GRADIENTS, JOINT_SOLVER_SUMS = range(3)
+JOINT_CONV_GRADIENTS, JOINT_DENSE_GRADIENTS, JOINT_SOLVER_SUMS, JOINT_CONV_ROUNDS = range(4)
 
 _lib = None
 

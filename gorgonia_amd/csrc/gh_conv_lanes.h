@@ -3,6 +3,7 @@
 #pragma once
 #include "gh_conv_common.h"
 #include "gh_internal.h"
+#include "gh_schedule.h"
 
 namespace conv_lanes {
 
@@ -16,6 +17,7 @@ template <> struct Mac<float> {
   static __device__ __forceinline__ float one(__amdgpu_buffer_rsrc_t r, int at, int s) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, at, s, 0));
   }
+  static constexpr int kNine = 3;   // loads of nine()
   static __device__ __forceinline__ void nine(__amdgpu_buffer_rsrc_t r, int at, int s, float (&v)[9]) {
     typedef float V __attribute__((ext_vector_type(4)));
 #pragma unroll
@@ -41,6 +43,7 @@ template <> struct Mac<double> {
   static __device__ __forceinline__ double one(__amdgpu_buffer_rsrc_t r, int at, int s) {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, at, s, 0));
   }
+  static constexpr int kNine = 5;
   static __device__ __forceinline__ void nine(__amdgpu_buffer_rsrc_t r, int at, int s, double (&v)[9]) {
     typedef double V __attribute__((ext_vector_type(2)));
 #pragma unroll
@@ -92,8 +95,6 @@ __device__ __forceinline__ void workgroup(const Lanes<T>& g, const ConvTail& tai
     else { pt = nid / g.ftiles; ft = nid - pt * g.ftiles; }
   }
   const int f0 = ft * 16 * TM, g0 = (kSplit ? pt : pt * WV + wave) * 16 * G;
-  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)g.x, 0, g.x_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)g.w, 0, g.w_bytes, 0x00020000);
   const int HW = g.H * g.W;
   // a group's image, result row and first column
   auto place = [&](int grp, int* b, int* oy, int* ox) {
@@ -126,8 +127,13 @@ __device__ __forceinline__ void workgroup(const Lanes<T>& g, const ConvTail& tai
     }
   }
   const int a_step = (kFlip ? 4 * g.F : 4) * 9 * S, b_step = 4 * HW * S;
+  const int quads = g.C >> 2;
   struct Frag { T a[TM][9]; T b[G][3][V + 2]; };
-  auto load = [&](int quad, Frag& f) {
+  // (a quad past the end: from buffers of no bytes, zeros that nothing is read for)
+  auto load = [&](int quad, Frag& f) __attribute__((always_inline)) {
+    const bool there = quad < quads;
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)g.x, 0, there ? g.x_bytes : 0, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)g.w, 0, there ? g.w_bytes : 0, 0x00020000);
 #pragma unroll
     for (int m = 0; m < TM; m++) U::nine(rw, a_at[m], quad * a_step, f.a[m]);
 #pragma unroll
@@ -164,18 +170,30 @@ __device__ __forceinline__ void workgroup(const Lanes<T>& g, const ConvTail& tai
     if (tail.gamma) bn_gamma = tail.gamma[tf];
     if (tail.beta) bn_beta = tail.beta[tf];
   }
-  const int quads = g.C >> 2;
   constexpr int step = kSplit ? WV : 1;
   const int first = kSplit ? wave : 0;
   if (first < quads) {
-    Frag cur, ahead;
-    load(first, cur);
+    // The loads of a quad are in flight under the MFMAs of the quad before: two sets of operands taken in turn, each load
+    // behind a few MFMAs (gh_schedule.h).  us, before / now: 8 x 32 x 52 x 52 -> 64 14.5 / 12.7, 8 x 32 x 104 x 104 -> 64 36.7 / 33.0, its gradient
+    // 37.0 / 35.0; the gradient of 8 x 128 x 26 x 26 -> 256 31.5 / 28.2, of 8 x 64 x 26 x 26 -> 128 12.9 / 11.9 and beside the filter's 32.6 / 30.7;
+    // float64 4 x 256 x 13 x 13 -> 512 42.2 / 37.8, the gradient of 7 x 64 x 24 x 24 -> 128 13.2 / 11.3.
+    Frag even, odd;
+    int c = first;
+    auto turn = [&](const Frag& now, Frag& next) __attribute__((always_inline)) {
+      c += step;
+      load(c, next);
+      multiply(now);
+      gh_spread_loads<TM * U::kNine + 9 * G, 9 * TM * TN>();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    load(first, even);
     __builtin_amdgcn_s_waitcnt(0x0F70);   // the loop is entered with nothing in flight, so its waits count its own loads only
-    for (int c = first; c < quads; c += step) {
-      load(c + step < quads ? c + step : c, ahead);   // (past the end the last quad again: no branch around the loads)
-      multiply(cur);
-      cur = ahead;
+    const int turns = (quads - first + step - 1) / step;
+    for (int two = turns >> 1; two > 0; two--) {   // (one way out: where paths meet the compiler waits for the worst of them)
+      turn(even, odd);
+      turn(odd, even);
     }
+    if (turns & 1) multiply(even);
   }
 
   float* const tab = (float*)(lds + (kSplit ? WV * TN * 256 * S : 0));

@@ -32,11 +32,34 @@ namespace {
 
 using namespace conv_lanes;
 
-template <class T, int WV, int TM, int V, int G, bool kSplit, bool kFlip, bool kPool>
-__global__ __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(WV == 8 || TM * V * G * sizeof(T) <= 32 ? 2 : 1))) void k_conv3x3_lanes(const Lanes<T> g, const ConvTail tail) {
+// kRounds: a workgroup has every gridDim.x-th tile, of `tiles`.
+template <class T, int WV, int TM, int V, int G, bool kSplit, bool kFlip, bool kPool, bool kRounds>
+__global__ __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(WV == 8 || TM * V * G * sizeof(T) <= 32 ? 2 : 1))) void k_conv3x3_lanes(const Lanes<T> g, const ConvTail tail, int tiles) {
   constexpr int bytes = lds_of<T, WV, TM, V, G, kSplit>(kFlip);
   __shared__ __attribute__((aligned(16))) char lds[bytes ? bytes : 16];
-  workgroup<T, WV, TM, V, G, kSplit, kFlip, kPool>(g, tail, (int)blockIdx.x, (int)gridDim.x, lds);
+  if constexpr (kRounds) {
+    for (int tile = (int)blockIdx.x; tile < tiles; tile += (int)gridDim.x) {
+      if (tile != (int)blockIdx.x) __syncthreads();   // before LDS is written again
+      workgroup<T, WV, TM, V, G, kSplit, kFlip, kPool>(g, tail, tile, tiles, lds);
+    }
+  } else {
+    workgroup<T, WV, TM, V, G, kSplit, kFlip, kPool>(g, tail, (int)blockIdx.x, (int)gridDim.x, lds);
+  }
+}
+
+// Where there are somewhat more tiles than workgroups that the device holds at once, a workgroup for each leaves the last ones to
+// the places that fall free together, two on one compute unit and none on the next: 8 x 128 x 26 x 26 -> 256 pooled, 728 tiles
+// for 512 places, 44.5 us, float64 8 x 32 x 104 x 104 -> 64, 676 for 512, 77.0.  With as many workgroups as places, each with
+// every so many-th tile, the compute units have one more or none: 35.9 and 59.8.  From twice the places on the last round is
+// the smaller part, and the kernel that walks takes some 0.2 us more.
+// How many workgroups of a kernel the device holds at once.
+template <auto kKernel>
+int64_t held_at_once(const gh_ctx* ctx, int threads) {
+  static const int share = [&] {
+    int n = 0;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void*)kKernel, threads, 0) == hipSuccess && n > 0 ? n : 1 << 20;
+  }();
+  return (int64_t)share * ctx->cu_count;
 }
 
 template <class T, int WV, int TM, int V, int G, bool kSplit>
@@ -48,18 +71,27 @@ int launch(gh_ctx* ctx, Lanes<T> g, const ConvTail& tail, bool flip, bool pool) 
   g.ftiles = (g.F + 16 * TM - 1) / (16 * TM);
   g.ptiles = (g.groups + per - 1) / per;
   g.ft_major = g.w_bytes > g.x_bytes;
-  const dim3 grid((unsigned)(g.ftiles * g.ptiles));
-  if constexpr (sizeof(T) == 4) {
-    if (pool) {
-      hipLaunchKernelGGL((k_conv3x3_lanes<T, WV, TM, V, G, kSplit, false, true>), grid, dim3(WV * 64), 0, ctx->stream, g, tail);
-      return gh_check_hip(ctx, hipGetLastError(), "conv3x3 launch");
+  const int tiles = g.ftiles * g.ptiles;
+  const auto go = [&](auto flips, auto pools) {
+    constexpr bool F = decltype(flips)::value, P = decltype(pools)::value;
+    constexpr auto one = k_conv3x3_lanes<T, WV, TM, V, G, kSplit, F, P, false>, rounds = k_conv3x3_lanes<T, WV, TM, V, G, kSplit, F, P, true>;
+    const int64_t held = held_at_once<rounds>(ctx, WV * 64);
+    const bool in_rounds = tiles > held && tiles < 2 * held;
+    if (in_rounds) {
+      ctx->joint[GH_JOINT_CONV_ROUNDS].launches++;
+      ctx->joint[GH_JOINT_CONV_ROUNDS].form = 100 * WV + 10 * TM + kSplit;
     }
+    hipLaunchKernelGGL((in_rounds ? rounds : one), dim3((unsigned)(in_rounds ? held : tiles)), dim3(WV * 64), 0, ctx->stream, g, tail, tiles);
+    return gh_check_hip(ctx, hipGetLastError(), "conv3x3 launch");
+  };
+  using Yes = std::true_type;
+  using No = std::false_type;
+  if constexpr (sizeof(T) == 4) {
+    if (pool) return go(No{}, Yes{});
   }
   if (G == 1 && flip && ctx->held.kind != kHeldNone)
-    if (const int rc = gh_try_launch_gradients(ctx, g, WV, TM, kSplit, (int)grid.x); rc >= 0) return rc;
-  if (flip) hipLaunchKernelGGL((k_conv3x3_lanes<T, WV, TM, V, G, kSplit, true, false>), grid, dim3(WV * 64), 0, ctx->stream, g, tail);
-  else hipLaunchKernelGGL((k_conv3x3_lanes<T, WV, TM, V, G, kSplit, false, false>), grid, dim3(WV * 64), 0, ctx->stream, g, tail);
-  return gh_check_hip(ctx, hipGetLastError(), "conv3x3 launch");
+    if (const int rc = gh_try_launch_gradients(ctx, g, WV, TM, kSplit, tiles); rc >= 0) return rc;
+  return flip ? go(Yes{}, No{}) : go(No{}, No{});
 }
 
 // The geometry of a forward command or (flip) of the convolution that an image-gradient command is; false where the

@@ -412,6 +412,9 @@ enum gh_joint {
   GH_JOINT_DENSE_GRADIENTS = 1,
   /* solver steps with the sums of their gradients (k_solver.hip): how many of the sums are a step's */
   GH_JOINT_SOLVER_SUMS = 2,
+  /* a 3x3 convolution or its image gradient (k_conv_lanes.hip) by workgroups of several tiles each: 100 x the wavefronts of one +
+   * 10 x its filter tiles + whether its wavefronts split the channels */
+  GH_JOINT_CONV_ROUNDS = 3,
   GH_JOINT__COUNT
 };
 GH_API int64_t gh_joint_launches(const gh_ctx* ctx, int kind, int64_t* form);
