@@ -71,12 +71,14 @@ int gh_gemm_direct_form(const gh_cmd& c, int cus, double* us, int* rounds) {
   return best;
 }
 
-// K slices of a form: the wavefronts' shares.  One tile per compute unit has eight wavefronts (float32): with four,
-// a chunk's MFMAs are over before the next chunk's loads are.
+// K slices of a form: the wavefronts' shares.  One tile per compute unit has eight wavefronts: with four, a chunk's MFMAs are over
+// before the next chunk's loads are.  float64, whose MFMAs take twice as long, gains from K = 640 on (us, four / eight: 113 x 1444,
+// K = 1480 21.4 / 14.4, 370 x 661, K = 860 13.3 / 10.5, 1061 x 281, K = 1180 22.1 / 21.5; 777 x 1543, K = 1021 equal) and below loses to the
+// longer meeting (1863 x 388, K = 458 20.6 / 21.2, 764 x 1563, K = 152 13.4 / 14.1).
 static int waves_of(const gh_cmd& c, const Form& f, int cus) {
   if (!f.split) return 1;
   const int64_t tiles = (c.dim[0] + 16 * f.tm - 1) / (16 * f.tm) * ((c.dim[1] + 16 * f.tn - 1) / (16 * f.tn)) * std::max<int64_t>(1, c.dim[6]);
-  return gh_dtype_of(c.flags) != GH_F64 && tiles <= cus ? 8 : 4;
+  return tiles <= cus && (gh_dtype_of(c.flags) != GH_F64 || c.dim[2] >= 640) ? 8 : 4;
 }
 int gh_gemm_direct_slices(const gh_cmd& c, int form, int cus) {
   return waves_of(c, (gh_dtype_of(c.flags) == GH_F64 ? kForms64 : kForms32)[form], cus);
@@ -87,12 +89,13 @@ int gh_launch_gemm_direct(gh_ctx* ctx, const gh_cmd& c, int form) {
   int batch;
   if (gh_dtype_of(c.flags) == GH_F64) {
     const Gemm<double> g = gemm_direct::gemm_of<double>(c, &batch);
+    const bool eight = waves_of(c, kForms64[form], ctx->cu_count) == 8;
     switch (form) {
-      case 0: launch<double, 4, 2, 2>(ctx, g, batch, ta, tb); break;
-      case 1: launch<double, 4, 2, 4>(ctx, g, batch, ta, tb); break;
-      case 2: launch<double, 4, 3, 4>(ctx, g, batch, ta, tb); break;
-      case 3: launch<double, 4, 4, 4>(ctx, g, batch, ta, tb); break;
-      default: launch<double, 4, 5, 4>(ctx, g, batch, ta, tb); break;
+      case 0: eight ? launch<double, 8, 2, 2>(ctx, g, batch, ta, tb) : launch<double, 4, 2, 2>(ctx, g, batch, ta, tb); break;
+      case 1: eight ? launch<double, 8, 2, 4>(ctx, g, batch, ta, tb) : launch<double, 4, 2, 4>(ctx, g, batch, ta, tb); break;
+      case 2: eight ? launch<double, 8, 3, 4>(ctx, g, batch, ta, tb) : launch<double, 4, 3, 4>(ctx, g, batch, ta, tb); break;
+      case 3: eight ? launch<double, 8, 4, 4>(ctx, g, batch, ta, tb) : launch<double, 4, 4, 4>(ctx, g, batch, ta, tb); break;
+      default: eight ? launch<double, 8, 5, 4>(ctx, g, batch, ta, tb) : launch<double, 4, 5, 4>(ctx, g, batch, ta, tb); break;
     }
   } else {
     const Gemm<float> g = gemm_direct::gemm_of<float>(c, &batch);

@@ -42,6 +42,16 @@ def _case(ctx, m, n, k, batch, ta, tb, dt, pad=0, bias=None, act=None):
     return got[:, :, :n], want
 
 
+
+# float64 products of one tile to a compute unit: eight wavefronts from K = 640 on, with whole pairs of chunks for each, one chunk
+# more, one less and a last one that is short
+@pytest.mark.parametrize("m,n,k", [(113, 1444, 1480), (370, 661, 860), (777, 1543, 641), (320, 1300, 1024), (31, 30, 648), (64, 900, 639)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+def test_float64_in_eight_slices(ctx, m, n, k, ta, tb):
+    got, want = _case(ctx, m, n, k, 1, ta, tb, "f64")[:2]
+    assert rel_frobenius(got, want) <= 1e-15 * np.sqrt(k / 8) + 2.0 ** -53 * 8   # a slice's roundings as their root, and eight sums
+
+
 @pytest.mark.parametrize("dt,bar", [("f32", 1e-5), ("f64", 1e-14)])
 @pytest.mark.parametrize("m,n,k,batch", SHAPES)
 def test_product(ctx, m, n, k, batch, dt, bar):
