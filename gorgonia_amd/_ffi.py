@@ -97,6 +97,7 @@ SYMBOLS = {
     "gh_conv2d_can_pool": (C.c_int, [C.POINTER(GhCmd)]),
     "gh_conv2d_can_pre": (C.c_int, [C.POINTER(GhCmd)]),
     "gh_conv2d_can_keep": (C.c_int, [C.POINTER(GhCmd)]),
+    "gh_bn_can_remake": (C.c_int, [C.c_int64] * 4),
     "gh_conv2d_route": (C.c_int, [C.POINTER(GhCmd)]),
     "gh_conv2d_bwd_filter_route": (C.c_int, [C.POINTER(GhCmd)]),
     "gh_gemm_route": (C.c_int, [C.POINTER(GhCmd), C.POINTER(C.c_int)]),
