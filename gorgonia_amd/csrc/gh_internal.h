@@ -172,7 +172,7 @@ int gh_gemm_direct_slices(const gh_cmd& c, int form, int cus);
 int gh_launch_gemm_direct(gh_ctx* ctx, const gh_cmd& c, int form);
 // a dense layer's two gradients in one launch (k_gemm_gradients.hip)
 enum { kGemmOther, kGemmDirect, kGemmSkinny };
-struct gh_gemm_choice { int kind = kGemmOther, form = 0, waves = 0, columns = 0; };   // form: k_gemm_direct's; waves, columns: the small-output kernels'; waves: float32 k_gemm_direct's that share K
+struct gh_gemm_choice { int kind = kGemmOther, form = 0, waves = 0, columns = 0; };   // form: k_gemm_direct's; waves, columns: the small-output kernels'; waves: k_gemm_direct's that share K, of float64 0 for four
 gh_gemm_choice gh_choose_gemm(const gh_ctx* ctx, const gh_cmd& c);
 bool gh_gemm_gradient_pair(const gh_cmd* cmds, int n);
 int gh_try_launch_gemm_gradients(gh_ctx* ctx, const gh_cmd* cmds);   // -1: no kernel has both

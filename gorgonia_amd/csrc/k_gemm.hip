@@ -3063,7 +3063,7 @@ gh_gemm_choice gh_choose_gemm(const gh_ctx* ctx, const gh_cmd& c) {
   if (gh_dtype_of(c.flags) == GH_F64) {
     const int form = gemm64_form(c, cus);
     if (form == kStaged64) return {};
-    if (form >= 0) return {kGemmDirect, form, 0, 0};
+    if (form >= 0) return {kGemmDirect, form, gh_gemm_direct_slices(c, form, cus) == 8 ? 8 : 0, 0};
     if (!skinny64_pairs(c)) return {};
     return {kGemmSkinny, 0, c.dim[2] >= 256 ? 8 : 4, 1};
   }

@@ -25,13 +25,18 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(kWa
   gemm_direct::workgroup<T, kWaves, TM, TN, kSplitK, kTA, kTB>(g, (int)(blockIdx.y * gridDim.x + blockIdx.x), (int)gridDim.x, (int)gridDim.y, (int)blockIdx.z, lds);
 }
 
+template <class T, int W, int TM, int TN, bool kSplitK>
+void launch_along_k(gh_ctx* ctx, const Gemm<T>& g, dim3 grid) {
+  if constexpr (sizeof(T) == 4 || W == 4) hipLaunchKernelGGL((k_gemm_direct<T, W, TM, TN, kSplitK, false, true>), grid, dim3(W * 64), 0, ctx->stream, g);
+}
+
 template <class T, int W, int TM, int TN, bool kSplitK = true>
 void launch(gh_ctx* ctx, const Gemm<T>& g, int batch, bool ta, bool tb) {
   constexpr int rows = 16 * TM * (kSplitK ? 1 : W);
   const dim3 grid((unsigned)((g.N + 16 * TN - 1) / (16 * TN)), (unsigned)((g.M + rows - 1) / rows), (unsigned)batch);
   if (ta && tb) hipLaunchKernelGGL((k_gemm_direct<T, W, TM, TN, kSplitK, true, true>), grid, dim3(W * 64), 0, ctx->stream, g);
   else if (ta) hipLaunchKernelGGL((k_gemm_direct<T, W, TM, TN, kSplitK, true, false>), grid, dim3(W * 64), 0, ctx->stream, g);
-  else if (tb) hipLaunchKernelGGL((k_gemm_direct<T, W, TM, TN, kSplitK, false, true>), grid, dim3(W * 64), 0, ctx->stream, g);
+  else if (tb) launch_along_k<T, W, TM, TN, kSplitK>(ctx, g, grid);
   else hipLaunchKernelGGL((k_gemm_direct<T, W, TM, TN, kSplitK, false, false>), grid, dim3(W * 64), 0, ctx->stream, g);
 }
 
@@ -74,11 +79,13 @@ int gh_gemm_direct_form(const gh_cmd& c, int cus, double* us, int* rounds) {
 // K slices of a form: the wavefronts' shares.  One tile per compute unit has eight wavefronts: with four, a chunk's MFMAs are over
 // before the next chunk's loads are.  float64, whose MFMAs take twice as long, gains from K = 640 on (us, four / eight: 113 x 1444,
 // K = 1480 21.4 / 14.4, 370 x 661, K = 860 13.3 / 10.5, 1061 x 281, K = 1180 22.1 / 21.5; 777 x 1543, K = 1021 equal) and below loses to the
-// longer meeting (1863 x 388, K = 458 20.6 / 21.2, 764 x 1563, K = 152 13.4 / 14.1).
+// longer meeting (1863 x 388, K = 458 20.6 / 21.2, 764 x 1563, K = 152 13.4 / 14.1).  Both operands along K, an input gradient's form,
+// stay with four: 97 x 1954, K = 713 12.1 / 11.8, but 20.0 / 21.5 beside the weight gradient in one launch.
 static int waves_of(const gh_cmd& c, const Form& f, int cus) {
   if (!f.split) return 1;
   const int64_t tiles = (c.dim[0] + 16 * f.tm - 1) / (16 * f.tm) * ((c.dim[1] + 16 * f.tn - 1) / (16 * f.tn)) * std::max<int64_t>(1, c.dim[6]);
-  return tiles <= cus && (gh_dtype_of(c.flags) != GH_F64 || c.dim[2] >= 640) ? 8 : 4;
+  const bool along_k = !(c.flags & GH_FLAG_TRANS_A) && (c.flags & GH_FLAG_TRANS_B);
+  return tiles <= cus && (gh_dtype_of(c.flags) != GH_F64 || (c.dim[2] >= 640 && !along_k)) ? 8 : 4;
 }
 int gh_gemm_direct_slices(const gh_cmd& c, int form, int cus) {
   return waves_of(c, (gh_dtype_of(c.flags) == GH_F64 ? kForms64 : kForms32)[form], cus);

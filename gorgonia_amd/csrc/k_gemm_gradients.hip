@@ -12,7 +12,9 @@
 // here took 0.65 of their time, none more than before.  The input gradient stands first, whose contraction is the longer one
 // (float32 257 x 54 -> 1536 8.5 us, behind the weight gradient 10.3; float64 51 x 778 -> 2019 19.5 and 29.3), but where float64's weight
 // gradient has a compute unit for each of its workgroups: all begin at once, and its larger tiles take longer (50 x 1152 -> 625 12.1 us
-// behind the input gradient, 96 x 1152 -> 625 15.0 and 13.3 in front of it).
+// behind the input gradient, 96 x 1152 -> 625 15.0 and 13.3 in front of it).  A float64 weight gradient in eight slices (640 rows and
+// more) has its four-wavefront input gradient beside it in workgroups of eight: 1448 x 96 -> 1582 38.6 with four / 37.3, 2035 x 129 ->
+// 1529 76.1 / 70.8, but 930 x 142 -> 1859 41.3 / 44.1 and 1610 x 120 -> 1605 35.9 / 37.3; the bits are those of the product alone.
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -103,19 +105,27 @@ int with32(const gh_gemm_choice& k, const gh_cmd& c, Body&& body) {
   return -1;
 }
 
+template <int WV, bool kTA, class Body>
+int direct64(int form, const gh_cmd& c, Body&& body) {
+  if (form == 0) return body(Direct<double, 2, 2, true, kTA, WV>(c));
+  if constexpr (kTA) {
+    switch (form) {
+      case 1: return body(Direct<double, 2, 4, true, kTA, WV>(c));
+      case 2: return body(Direct<double, 3, 4, true, kTA, WV>(c));
+      case 3: return body(Direct<double, 4, 4, true, kTA, WV>(c));
+      case 4: return body(Direct<double, 5, 4, true, kTA, WV>(c));
+    }
+  }
+  return -1;
+}
+
 template <bool kTA, class Body>
 int with64(const gh_gemm_choice& k, const gh_cmd& c, Body&& body) {
   if (k.kind == kGemmDirect) {
-    if (k.form == 0) return body(Direct<double, 2, 2, true, kTA>(c));
-    if constexpr (kTA) {
-      switch (k.form) {
-        case 1: return body(Direct<double, 2, 4, true, kTA>(c));
-        case 2: return body(Direct<double, 3, 4, true, kTA>(c));
-        case 3: return body(Direct<double, 4, 4, true, kTA>(c));
-        case 4: return body(Direct<double, 5, 4, true, kTA>(c));
-      }
-    }
-  } else if (k.kind == kGemmSkinny) {
+    if (k.waves != 8) return direct64<4, kTA>(k.form, c, body);
+    if constexpr (kTA) return direct64<8, kTA>(k.form, c, body);
+  }
+  if (k.kind == kGemmSkinny) {
     if (k.waves == 4) return body(Skinny64<4, kTA>(c));
     if constexpr (!kTA) return body(Skinny64<8, kTA>(c));
   }

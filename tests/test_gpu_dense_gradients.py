@@ -26,7 +26,11 @@ F64 = {
     (129, 31, 64): 2004120041, (64, 500, 3000): 1100020081, (40, 1600, 1600): None, (24, 2000, 2000): None, (2, 64, 3): 1000010000,
     (51, 778, 2019): 1000020081, (2, 4362, 33): 1100010000, (2, 1464, 177): 1100020041, (97, 1954, 713): 1200010000, (3, 2049, 246): 1200020041,
     (163, 1289, 594): 1300010000, (39, 5223, 141): 1300020041, (106, 1764, 1371): 1400010000, (33, 1158, 1024): 1400020081, (67, 7, 3): 2004110000,
-    (2, 362, 80): 1000020041, (37, 877, 931): 1300020081}
+    (2, 362, 80): 1000020041, (37, 877, 931): 1300020081,
+    # weight gradients in eight slices
+    (682, 296, 610): 1008010000, (1448, 96, 1582): 1008020081, (708, 335, 1002): 1108010000, (641, 480, 675): 1108020081,
+    (1578, 133, 3666): 1208010000, (655, 186, 2987): 1208020081, (665, 345, 2324): 1308010000, (730, 251, 3435): 1308020081,
+    (723, 312, 3489): 1408010000, (944, 277, 3673): 1408020081}
 CASES = [(np.float32,) + c for c in F32] + [(np.float64,) + c for c in F64]
 
 
