@@ -42,7 +42,7 @@ HIP_FLAGS = [
     "-I", INCLUDE, "-I", CSRC,
 ]
 
-HIP_SOURCES = ["gh_api.hip", "gh_validate.cpp", "k_elem.hip", "k_chain.hip", "k_pairs.hip", "k_gemm.hip", "k_gemm_direct.hip", "k_gemm_gradients.hip", "k_gemm_thin.hip", "k_gemm_split.hip", "k_conv_small.hip", "k_conv_rows.hip", "k_conv_rows1.hip", "k_conv_patch.hip", "k_conv_wide.hip", "k_conv_strip.hip", "k_conv_pointwise.hip", "k_conv_lanes.hip", "k_conv_wgrad_small.hip", "k_conv_wgrad.hip", "k_conv_gradients.hip", "k_slab_sums.hip", "k_solver.hip", "k_nn.hip", "k_nn64.hip", "k_bwd.hip", "k_bn_held.hip", "k_bwd64.hip"]
+HIP_SOURCES = ["gh_api.hip", "gh_pieces.hip", "gh_validate.cpp", "k_elem.hip", "k_chain.hip", "k_pairs.hip", "k_gemm.hip", "k_gemm_direct.hip", "k_gemm_gradients.hip", "k_gemm_thin.hip", "k_gemm_split.hip", "k_conv_small.hip", "k_conv_rows.hip", "k_conv_rows1.hip", "k_conv_patch.hip", "k_conv_wide.hip", "k_conv_strip.hip", "k_conv_pointwise.hip", "k_conv_lanes.hip", "k_conv_wgrad_small.hip", "k_conv_wgrad.hip", "k_conv_gradients.hip", "k_slab_sums.hip", "k_solver.hip", "k_nn.hip", "k_nn64.hip", "k_bwd.hip", "k_bn_held.hip", "k_bwd64.hip"]
 
 HOST_FLAGS = [
     "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall", "-Wextra",

@@ -61,7 +61,7 @@ int gh_check_hip(gh_ctx* ctx, hipError_t e, const char* what) {
   return gh_fail(ctx, GH_EDEVICE, m);
 }
 
-static bool in_pinned_host(const gh_ctx* ctx, uint64_t p) {
+bool gh_in_pinned_host(const gh_ctx* ctx, uint64_t p) {
   for (const auto& r : ctx->host_ranges)
     if (p >= r.first && p < r.second) return true;
   return false;
@@ -127,6 +127,7 @@ static void drop_ctx(gh_ctx* ctx) {
   if (ctx->workspace) hipFree(ctx->workspace);
   if (ctx->slab_space) hipFree(ctx->slab_space);
   if (ctx->arena) hipFree(ctx->arena);
+  gh_drop_pieces(ctx);
   hipStreamDestroy(ctx->stream);
   delete ctx;
 }
@@ -279,7 +280,7 @@ int gh_memcpy_h2d(gh_ctx* ctx, gh_devptr dst, const void* src, int64_t bytes) {
   if (ctx->err) return ctx->err;
   if (bytes == 0) return GH_OK;
   ctx->idle = false;
-  if (!in_pinned_host(ctx, (uint64_t)(uintptr_t)src)) ctx->runtime_wait = true;
+  if (!gh_in_pinned_host(ctx, (uint64_t)(uintptr_t)src)) ctx->runtime_wait = true;
   return gh_check_hip(ctx,
                       hipMemcpyAsync((void*)(uintptr_t)dst, src, (size_t)bytes,
                                      hipMemcpyHostToDevice, ctx->stream),
@@ -291,7 +292,7 @@ int gh_memcpy_d2h(gh_ctx* ctx, void* dst, gh_devptr src, int64_t bytes) {
   if (ctx->err) return ctx->err;
   if (bytes == 0) return GH_OK;
   ctx->idle = false;
-  if (!in_pinned_host(ctx, (uint64_t)(uintptr_t)dst)) ctx->runtime_wait = true;
+  if (!gh_in_pinned_host(ctx, (uint64_t)(uintptr_t)dst)) ctx->runtime_wait = true;
   return gh_check_hip(ctx,
                       hipMemcpyAsync(dst, (const void*)(uintptr_t)src, (size_t)bytes,
                                      hipMemcpyDeviceToHost, ctx->stream),
@@ -332,7 +333,7 @@ int gh_memcpy_d2d(gh_ctx* ctx, gh_devptr dst, gh_devptr src, int64_t bytes) {
   if (ctx->err) return ctx->err;
   if (bytes == 0) return GH_OK;
   ctx->idle = false;
-  const bool from_host = in_pinned_host(ctx, src);
+  const bool from_host = gh_in_pinned_host(ctx, src);
   if ((from_host || bytes <= kKernelCopyLimit) && ((dst | src | (uint64_t)bytes) & 3) == 0) {
     if (((dst | src) & 15) == 0 && bytes >= 4096) {
       const int64_t n16 = bytes / 16;
@@ -418,7 +419,7 @@ int gh_memcpy_staged(gh_ctx* ctx, gh_devptr dst, void* stage, const void* src, i
   if (ctx->err) return ctx->err;
   if (bytes == 0) return GH_OK;
   const uint64_t from = (uint64_t)(uintptr_t)stage;
-  if (!in_pinned_host(ctx, from) || !in_pinned_host(ctx, from + (uint64_t)bytes - 1)) return gh_fail(ctx, GH_EINVAL, "gh_memcpy_staged: the staging memory is not of gh_host_alloc");
+  if (!gh_in_pinned_host(ctx, from) || !gh_in_pinned_host(ctx, from + (uint64_t)bytes - 1)) return gh_fail(ctx, GH_EINVAL, "gh_memcpy_staged: the staging memory is not of gh_host_alloc");
   if (!ctx->done_word || ctx->capturing || bytes < GH_STAGED_FROM || ((dst | from) & 15) || (bytes & 3)) {
     memcpy(stage, src, (size_t)bytes);
     return gh_memcpy_d2d(ctx, dst, from, bytes);
@@ -498,7 +499,7 @@ int gh_validate(const gh_cmd* cmds, int n, char* msg, int msg_len) {
   return GH_OK;
 }
 
-static int submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
+int gh_submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
   ctx->idle = false;
   for (int i = 0; i < n; i++) {
     std::string m;
@@ -591,7 +592,9 @@ static bool slab_space(gh_ctx* ctx, const gh_cmd* cmds, int n) {
 // Sums of filter-gradient slabs may wait for the commands behind them (k_slab_sums.hip); none waits past the submission.
 static int submit_cmds(gh_ctx* ctx, const gh_cmd* cmds, int n) {
   ctx->defer_sums = n > 1 && !ctx->ws_strict && slab_space(ctx, cmds, n);
-  const int rc = submit_each(ctx, cmds, n);
+  int rc = GH_OK;
+  const int ahead = gh_submit_pieces(ctx, cmds, n, &rc);
+  if (!rc) rc = gh_submit_each(ctx, cmds + ahead, n - ahead);
   ctx->defer_sums = false;
   const int late = gh_flush_sums(ctx);
   return rc ? rc : late;

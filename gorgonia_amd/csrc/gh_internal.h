@@ -68,6 +68,7 @@ struct gh_held_filter {
 constexpr int kUnits = 256;   // the MI355X's compute units
 constexpr int kSlabSums = 8;
 constexpr int64_t kSlabSpace = 24ll << 20;
+constexpr int kPieces = 8;
 
 struct gh_ctx {
   int device = 0;
@@ -107,6 +108,13 @@ struct gh_ctx {
   bool sync_block = false;  // gh_sync waits in the runtime only
   bool sync_spin = false;   // gh_sync never gives up its core: where it would leave the wait to the runtime it asks the stream again and again
   gh_llc_model llc;
+  // uploads in pieces (gh_pieces.hip): the stream that copies them, an event for the work in front, the words they are passed
+  // on by, and how many there have been
+  hipStream_t pieces = nullptr;
+  hipEvent_t pieces_after = nullptr;
+  void* piece_words = nullptr;
+  uint64_t piece_seq = 0;
+  bool no_pieces = false;   // they were not to be had
   // pinned host buffers handed out by gh_host_alloc: [start, end)
   std::vector<std::pair<uint64_t, uint64_t>> host_ranges;
 };
@@ -129,6 +137,12 @@ int gh_validate_cmd(const gh_cmd& c, std::string& msg);
 // inputs lost (`cold`) or not, goes past the cache (k_elem.hip)
 bool gh_llc_cold(const gh_ctx* ctx, uint64_t p);
 bool gh_llc_stream(int64_t bytes, bool cold);
+// a copy out of pinned host memory and the commands behind it in pieces of the batch (gh_pieces.hip): how many commands it
+// has submitted (0: none), *rc what came of them
+int gh_submit_pieces(gh_ctx* ctx, const gh_cmd* cmds, int n, int* rc);
+extern "C" int gh_submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n);
+bool gh_in_pinned_host(const gh_ctx* ctx, uint64_t p);
+void gh_drop_pieces(gh_ctx* ctx);
 // sums of filter-gradient slabs, put off where gh_submit allows it (k_slab_sums.hip)
 void* gh_slab_space(gh_ctx* ctx, int64_t bytes);
 int gh_sum_slabs(gh_ctx* ctx, const gh_slab_sum& s);

@@ -1083,6 +1083,25 @@ Status TapeMachine::Compile() {
       before = i;
     }
   }
+  // The convolutions and poolings behind an uploaded batch may run in pieces of it, for which their values have to lie apart:
+  // what they read is kept until the last of them is done.
+  if (!opt_.node_at_a_time)
+    for (int i = 0; i < N; i++) {
+      const Node& x = nodes[(size_t)i];
+      if (!x.is_input || x.resident || x.shape.Dims() != 4) continue;
+      int at = i, end = -1;
+      std::vector<int> kept;
+      for (;;) {
+        kept.push_back(node_reg_[(size_t)at]);
+        const int next = last_reader[(size_t)root[(size_t)at]];
+        if (next < 0) break;
+        const Node& n = nodes[(size_t)next];
+        if ((n.op.kind != OpKind::Conv2d && n.op.kind != OpKind::MaxPool2D) || n.inputs.empty() || root[(size_t)n.inputs[0]] != root[(size_t)at]) break;
+        at = end = next;
+      }
+      for (int r : kept)
+        if (r >= 0 && reg_last[(size_t)r] >= 0) reg_last[(size_t)r] = std::max(reg_last[(size_t)r], end);
+    }
   // A small result that only the host reads is written by its kernel straight
   // into pinned host memory: no arena register, no staging copy at the end of
   // the segment.

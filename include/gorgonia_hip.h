@@ -415,6 +415,9 @@ enum gh_joint {
   /* a 3x3 convolution or its image gradient (k_conv_lanes.hip) by workgroups of several tiles each: 100 x the wavefronts of one +
    * 10 x its filter tiles + whether its wavefronts split the channels */
   GH_JOINT_CONV_ROUNDS = 3,
+  /* a batch out of pinned host memory in pieces, and the layers behind it piece by piece while the next one comes;
+     form: 100 * the pieces + the layers */
+  GH_JOINT_PIECES = 4,
   GH_JOINT__COUNT
 };
 GH_API int64_t gh_joint_launches(const gh_ctx* ctx, int kind, int64_t* form);
