@@ -12,7 +12,7 @@
 //   * A kernel begins and ends with its caches in order, and that waits for what is under way to and from memory: with 16
 //     workgroups of 1024 threads and 8 loads each, 2 MB under way, a pooling of 4 us took 29.  One load each (128 KB) is as
 //     quick for the bus, and stores that go through to memory leave nothing to be written back.
-// us, whole / in pieces: a detector of nine convolutions, 8 x 3 x 416 x 416 708 / 627, five images 509 / 474, two 231 / 224,
+// us, whole / in pieces: a detector of eight convolutions, 8 x 3 x 416 x 416 708 / 627, five images 509 / 474, two 231 / 224,
 // 8 x 3 x 320 x 320 449 / 416, five of them 310 / 301, 8 x 3 x 224 x 224 250 / 243.
 //
 // Nothing waits for a workgroup that has not begun: a part of a piece is copied by whoever claims it first, the copy's

@@ -17,6 +17,13 @@
 //     image written as zero - so the main loop has no workgroup barrier (there is one in
 //     front of it, behind the shared table of patch cells); the next quad's global loads are
 //     in flight while the current one is multiplied.
+//   * From 128 channels on, with 9 and 11 pixel tiles, the region holds two quads: the next one goes from
+//     registers to its half and the one behind that is loaded among the current one's MFMAs, which then
+//     follow each other without a gap from quad to quad.  With one quad the wavefront's 35 LDS writes, the
+//     first reads behind them and its loads stood between two quads, a fifth of the loop.  Bound: the MFMAs
+//     (82 of the 98 us below) and the first loads and last sums of a workgroup that has a compute unit alone.
+//     us, one quad / two: 8 x 512 x 13 x 13 -> 1024 108.1 / 97.9, 4 x 59.6 / 53.8, 8 x 256 x 13 x 13 -> 512 33.2 / 30.3,
+//     8 x 512 x 12 x 12 -> 1024 90.7 / 82.4, 8 x 128 x 24 x 24 -> 256 28.8 / 27.4.
 //   * With GH_FLAG_CONV_POOL2 the patch has even extents and the N axis enumerates
 //     (pooled pixel, position in the 2x2 window); the epilogue reads a window as four
 //     adjacent columns (scan order and strict > of the pooling kernel, op_nn.go:860-907).
@@ -54,8 +61,28 @@ struct PatchGeom {
 
 constexpr int kWaves = 8;
 constexpr int kSlotsX = 15;   // patch cells each lane stages per quad: 4 planes * PP <= 64 * kSlotsX
+template <int TM>
+constexpr int quad_floats() { return 36 * 16 * TM + 64 * kSlotsX; }   // LDS of a quad where a slot is a word
 
-template <int TM, int TN>
+// A tap's LDS reads one behind each matrix instruction, then its LDS writes (which the compiler keeps behind the reads: they
+// may meet, for all it knows) over the others, its loads over all.
+template <int kReads, int kWrites, int kLoads, int kMacs, int I = 0>
+__device__ __forceinline__ void spread_tap() {
+  if constexpr (I < kMacs) {
+    constexpr int kRest = kMacs - kReads, J = I - kReads;
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    if constexpr (I < kReads) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    if constexpr (J >= 0 && kWrites > 0) {
+      constexpr int w = (J + 1) * kWrites / kRest - J * kWrites / kRest;
+      if constexpr (w > 0) __builtin_amdgcn_sched_group_barrier(0x200, w, 0);
+    }
+    constexpr int l = (I + 1) * kLoads / kMacs - I * kLoads / kMacs;
+    if constexpr (l > 0) __builtin_amdgcn_sched_group_barrier(0x020, l, 0);
+    spread_tap<kReads, kWrites, kLoads, kMacs, I + 1>();
+  }
+}
+
+template <int TM, int TN, bool kTwo>
 __global__ __launch_bounds__(kWaves * 64) void k_conv3x3_patch(const float* __restrict__ x, const float* __restrict__ w,
                                                                float* __restrict__ y, PatchGeom g, ConvTail tail) {
   constexpr int NTH = kWaves * 64;
@@ -71,7 +98,7 @@ __global__ __launch_bounds__(kWaves * 64) void k_conv3x3_patch(const float* __re
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lk = lane >> 4;
-  const int wsize = 36 * SA + 4 * g.PL;           // floats per wavefront region
+  const int wsize = kTwo ? 2 * quad_floats<TM>() : 36 * SA + 4 * g.PL;   // floats per wavefront region
   float* const Aw = lds + wave * wsize;           // [36][SA]
   float* const Pw = Aw + 36 * SA;                 // [4][PL]
   int* const tab = reinterpret_cast<int*>(lds + kWaves * wsize);   // [16 TN] cell of N entry n inside the padded patch
@@ -105,13 +132,15 @@ __global__ __launch_bounds__(kWaves * 64) void k_conv3x3_patch(const float* __re
   bool xin[kSlotsX];
 #pragma unroll
   for (int u = 0; u < kSlotsX; u++) {
-    const int id = min(lane + 64 * u, 4 * g.PP - 1);   // slots past the end repeat the last cell
-    const int pl = mdiv(id, g.mPP), rem = id - pl * g.PP;
+    // with room for two quads a slot is a word of the region, the last of a plane's pitch among them; else slots past the end
+    // repeat the last cell
+    const int id = kTwo ? lane + 64 * u : min(lane + 64 * u, 4 * g.PP - 1);
+    const int pl = kTwo ? min(id / g.PL, 3) : mdiv(id, g.mPP), rem = kTwo ? min(id - pl * g.PL, g.PP - 1) : id - pl * g.PP;
     const int r = mdiv(rem, g.mPW), cc = rem - r * g.PW;
     const int iy = oy0 - g.pad + r, ix = ox0 - g.pad + cc;
     xin[u] = iy >= 0 && iy < g.H && ix >= 0 && ix < g.W;
     xoff[u] = pl * g.HW + min(max(iy, 0), g.H - 1) * g.W + min(max(ix, 0), g.W - 1);
-    xdst[u] = pl * g.PL + rem;
+    xdst[u] = kTwo ? lane + 64 * u : pl * g.PL + rem;
   }
   const float* xq = x + ((int64_t)bimg * g.C + c0) * g.HW;
   f32x4 wv[NWQ];
@@ -180,25 +209,112 @@ __global__ __launch_bounds__(kWaves * 64) void k_conv3x3_patch(const float* __re
 #pragma unroll
     for (int t = 0; t < TN; t++) bf[set][t] = Pw[pb[t][kr] + kc];
   };
-  for (int qd = 0; qd < g.NQ; qd++) {
-    store_quad();                       // this quad: registers to the wavefront's LDS region
-    if (qd + 1 < g.NQ) load_quad();     // the next one is in flight during the MFMAs
-    fetch(0, 0);
-    fetch(1, 1);
+  if constexpr (kTwo) {
+    constexpr int kQuad = quad_floats<TM>();
+    auto fetch_of = [&](int set, int tap, int at) __attribute__((always_inline)) {
+      const int kr = tap / 3, kc = tap % 3;
 #pragma unroll
-    for (int tap = 0; tap < 9; tap++) {
-      if (tap + 2 < 9) fetch((tap + 2) % 3, tap + 2);
+      for (int a = 0; a < TM; a++) af[set][a] = abase[at + tap * SA + a * 16];
 #pragma unroll
-      for (int a = 0; a < TM; a++)
+      for (int t = 0; t < TN; t++) bf[set][t] = Pw[at + pb[t][kr] + kc];
+    };
+    // the filter tile's rows and the wavefront's planes by 32-bit offsets (a row has up to 8192 x 9 values, an image 2^29)
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (int64_t)m0 * g.K), 0, -1, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)(x + ((int64_t)bimg * g.C + c0) * g.HW), 0, -1, 0x00020000);
+    const int wrow = min(wr, g.F - 1 - m0) * g.K * 4, wlane = wrow + wq0 * 16, wlast = wrow + 8 * 16;
+    int qd = min(1, g.NQ - 1);   // the quad that is loaded next (past the last one: that one again)
+    auto load_w = [&](int u) __attribute__((always_inline)) {
+      const bool last = (u + 1) * QL > 8;   // (QL - 1 + u QL, the most, is past the eighth column only here)
+      wv[u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, last ? wlast : wlane + u * QL * 16, (c0 + 4 * qd) * 36, 0));
+    };
+    auto load_x = [&](int u) __attribute__((always_inline)) {
+      xv[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, xoff[u] * 4, 16 * qd * g.HW, 0));
+    };
+    float *const wput = Aw + 4 * wq0 * SA + wr, *const wend = Aw + 32 * SA + wr, *const xput = Pw + lane;
+    auto put_w = [&](int u, int at) __attribute__((always_inline)) {
+      float* const to = ((u + 1) * QL > 8 ? wend : wput + 4 * u * QL * SA) + at;
 #pragma unroll
-        for (int t = 0; t < TN; t++)
-          acc[a][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[tap % 3][a], bf[tap % 3][t], acc[a][t], 0, 0, 0);
+      for (int e = 0; e < 4; e++) to[e * SA] = wv[u][e];
+    };
+    auto put_x = [&](int u, int at) __attribute__((always_inline)) { xput[at + 64 * u] = xin[u] ? xv[u] : 0.f; };
 #pragma unroll
-      for (int i = 0; i < TM * TN; i++) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // DS read
+    for (int u = 0; u < NWQ; u++) put_w(u, 0);
+#pragma unroll
+    for (int u = 0; u < kSlotsX; u++) put_x(u, 0);
+#pragma unroll
+    for (int u = 0; u < NWQ; u++) load_w(u);
+#pragma unroll
+    for (int u = 0; u < kSlotsX; u++) load_x(u);
+    fetch_of(0, 0, 0);
+    fetch_of(1, 1, 0);
+    // One quad out of one half of the region: the next one, loaded, goes to the other half under taps 4 to 6, and the one behind
+    // that is loaded under taps 6 to 8.
+    auto quad = [&](auto half) __attribute__((always_inline)) {
+      constexpr int at = half() * kQuad, next = kQuad - at;
+#pragma unroll
+      for (int tap = 0; tap < 9; tap++) {
+        fetch_of((tap + 2) % 3, (tap + 2) % 9, tap + 2 < 9 ? at : next);
+        if (tap == 4) {
+#pragma unroll
+          for (int u = 0; u < NWQ && u < 3; u++) put_w(u, next);
+        } else if (tap == 5) {
+#pragma unroll
+          for (int u = 3; u < NWQ; u++) put_w(u, next);
+#pragma unroll
+          for (int u = 0; u < 5; u++) put_x(u, next);
+        } else if (tap == 6) {
+#pragma unroll
+          for (int u = 5; u < kSlotsX; u++) put_x(u, next);
+          qd = min(qd + 1, g.NQ - 1);
+#pragma unroll
+          for (int u = 0; u < NWQ; u++) load_w(u);
+        } else if (tap == 7) {
+#pragma unroll
+          for (int u = 0; u < 8; u++) load_x(u);
+        } else if (tap == 8) {
+#pragma unroll
+          for (int u = 8; u < kSlotsX; u++) load_x(u);
+        }
+#pragma unroll
+        for (int a = 0; a < TM; a++)
+#pragma unroll
+          for (int t = 0; t < TN; t++)
+            acc[a][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[tap % 3][a], bf[tap % 3][t], acc[a][t], 0, 0, 0);
+        if (tap == 4) spread_tap<TM + TN, 12, 0, TM * TN>();
+        else if (tap == 5) spread_tap<TM + TN, 4 * (NWQ - 3) + 5, 0, TM * TN>();
+        else if (tap == 6) spread_tap<TM + TN, 10, NWQ, TM * TN>();
+        else if (tap == 7) spread_tap<TM + TN, 0, 8, TM * TN>();
+        else if (tap == 8) spread_tap<TM + TN, 0, 7, TM * TN>();
+        else spread_tap<TM + TN, 0, 0, TM * TN>();
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int two = g.NQ >> 1; two > 0; two--) {
+      quad(std::integral_constant<int, 0>{});
+      quad(std::integral_constant<int, 1>{});
+    }
+    if (g.NQ & 1) quad(std::integral_constant<int, 0>{});
+  } else {
+    for (int qd = 0; qd < g.NQ; qd++) {
+      store_quad();                       // this quad: registers to the wavefront's LDS region
+      if (qd + 1 < g.NQ) load_quad();     // the next one is in flight during the MFMAs
+      fetch(0, 0);
+      fetch(1, 1);
+#pragma unroll
+      for (int tap = 0; tap < 9; tap++) {
+        if (tap + 2 < 9) fetch((tap + 2) % 3, tap + 2);
+#pragma unroll
+        for (int a = 0; a < TM; a++)
+#pragma unroll
+          for (int t = 0; t < TN; t++)
+            acc[a][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[tap % 3][a], bf[tap % 3][t], acc[a][t], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < TM * TN; i++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // DS read
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   }
 
@@ -293,6 +409,7 @@ __global__ __launch_bounds__(kWaves * 64) void k_conv3x3_patch(const float* __re
 struct PatchPlan {
   PatchGeom g;
   int TM, TN;
+  bool two;
   size_t lds;
 };
 
@@ -341,6 +458,7 @@ bool patch_plan_compute(const gh_cmd& c, bool pool, PatchPlan* out) {
   g.tiles_x = (need_w + bTW - 1) / bTW; g.tiles_y = (need_h + bTH - 1) / bTH;
   g.PW = bTW + 2; g.PP = (bTH + 2) * g.PW;
   g.PL = g.PP | 1;   // odd pitch: the four channel planes of a fetch start in different banks
+  if (4 * g.PL > 64 * kSlotsX) g.PL = g.PP;   // 240 cells: they do without it
   g.npix = bTH * bTW;
   const int64_t patches = (int64_t)g.B * g.tiles_x * g.tiles_y;
   if (patches > (1ll << 30)) return false;
@@ -349,7 +467,11 @@ bool patch_plan_compute(const gh_cmd& c, bool pool, PatchPlan* out) {
   g.mTXY = magic_of(g.tiles_x * g.tiles_y); g.mTX = magic_of(g.tiles_x); g.mPP = magic_of(g.PP);
   g.mPW = magic_of(g.PW); g.mTW = magic_of(g.TW); g.mHTW = magic_of(g.HTW); g.mNPIX = magic_of(g.npix);
   g.mNPOOL = magic_of(g.npix / 4);
-  const size_t stage = ((size_t)kWaves * (36 * 16 * TM + 4 * g.PL) + 16 * bTN + 8) * 4;
+  // LDS for two quads to a wavefront, the next one staged under the present one's MFMAs: from 128 channels on (64, which are two
+  // quads: 2 x 64 x 48 x 48 -> 128 11.7 us / 12.3) and for 9 and 11 pixel tiles (with 4 and 7 nothing is gained)
+  out->two = bTN >= 9 && g.NQ >= 4;
+  const size_t quad = out->two ? 2 * (TM == 1 ? quad_floats<1>() : quad_floats<2>()) : 36 * 16 * TM + 4 * g.PL;
+  const size_t stage = ((size_t)kWaves * quad + 16 * bTN + 8) * 4;
   const size_t red = (size_t)4 * 16 * bTN * (16 * TM + 4) * 4;
   size_t lds = stage > red ? stage : red;
   g.epi_off = (int)(lds / 4);
@@ -363,13 +485,13 @@ bool patch_plan(const gh_cmd& c, bool pool, PatchPlan* out) {
   return gh_plan_memo(c, pool, out, [&](PatchPlan* p) { return patch_plan_compute(c, pool, p); });
 }
 
-template <int TM, int TN>
+template <int TM, int TN, bool kTwo>
 int launch_patch(gh_ctx* ctx, const gh_cmd& c, const PatchPlan& p) {
   // more than 64 KB of dynamic LDS has to be allowed per kernel, once
   static std::once_flag once;
   static hipError_t attr_rc = hipSuccess;
   std::call_once(once, [] {
-    attr_rc = hipFuncSetAttribute((const void*)k_conv3x3_patch<TM, TN>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    attr_rc = hipFuncSetAttribute((const void*)k_conv3x3_patch<TM, TN, kTwo>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   160 * 1024);
   });
   if (attr_rc != hipSuccess) return gh_check_hip(ctx, attr_rc, "hipFuncSetAttribute(conv3x3 patch)");
@@ -382,7 +504,7 @@ int launch_patch(gh_ctx* ctx, const gh_cmd& c, const PatchPlan& p) {
   static const bool no_xcd = getenv("GORGONIA_HIP_CONV_PATCH_ORDER") != nullptr;   // tuning switch: "0" patch-major, "1" filter-tile-major
   g.ft_major = (int64_t)g.F * g.K > (int64_t)g.B * g.C * g.HW ? 1 : 0;
   if (no_xcd) g.ft_major = atoi(getenv("GORGONIA_HIP_CONV_PATCH_ORDER")) != 0;
-  hipLaunchKernelGGL((k_conv3x3_patch<TM, TN>), dim3((unsigned)g.nwg), dim3(kWaves * 64), p.lds, ctx->stream,
+  hipLaunchKernelGGL((k_conv3x3_patch<TM, TN, kTwo>), dim3((unsigned)g.nwg), dim3(kWaves * 64), p.lds, ctx->stream,
                      (const float*)(uintptr_t)c.ptr[0], (const float*)(uintptr_t)c.ptr[1],
                      (float*)(uintptr_t)c.ptr[2], g, conv_tail(c));
   return gh_check_hip(ctx, hipGetLastError(), "conv3x3 patch launch");
@@ -396,7 +518,8 @@ bool gh_conv_patch_takes(const gh_cmd& c) {
 }
 
 // What a plain command takes here, in us (fitted to 1 to 8 images, 64 -> 128 at 52 x 52 to 512 -> 1024 at 13 x 13):
-// a workgroup walks its channels at 0.038 us per quad and 16 x 16 results.
+// a workgroup walks its channels at 0.038 us per quad and 16 x 16 results.  (With two quads in LDS it takes 0.033; k_conv3x3_lanes'
+// estimate, to which this one is compared, is as much above its times, and the choice is the quicker kernel as it is.)
 double gh_conv_patch_us(const gh_cmd& c, int cus) {
   PatchPlan p;
   if (!patch_plan(c, false, &p)) return 0;
@@ -425,10 +548,10 @@ int gh_try_launch_conv_patch(gh_ctx* ctx, const gh_cmd& c) {
     return gh_fail(ctx, GH_EINVAL, "conv2d: no fused pooling for this shape (see gh_conv2d_can_pool)");
 #define GH_PATCH_TN(TM_)                                              \
   switch (p.TN) {                                                     \
-    case 4: return launch_patch<TM_, 4>(ctx, c, p);                   \
-    case 7: return launch_patch<TM_, 7>(ctx, c, p);                   \
-    case 9: return launch_patch<TM_, 9>(ctx, c, p);                   \
-    default: return launch_patch<TM_, 11>(ctx, c, p);                 \
+    case 4: return launch_patch<TM_, 4, false>(ctx, c, p);            \
+    case 7: return launch_patch<TM_, 7, false>(ctx, c, p);            \
+    case 9: return p.two ? launch_patch<TM_, 9, true>(ctx, c, p) : launch_patch<TM_, 9, false>(ctx, c, p);     \
+    default: return p.two ? launch_patch<TM_, 11, true>(ctx, c, p) : launch_patch<TM_, 11, false>(ctx, c, p);  \
   }
   if (p.TM == 1) { GH_PATCH_TN(1) }
   GH_PATCH_TN(2)
