@@ -28,7 +28,7 @@ namespace {
 constexpr int kThreads = 1024, kCopiers = 8;
 constexpr int kThrough = 1 | 16;                      // a store's sc0 and sc1 bits: to memory, past the caches
 constexpr int64_t kGiveUp = 400000;                   // ticks of 10 ns, and one more for 100 bytes (GORGONIA_HIP_PIECES_TICKS: fewer)
-constexpr int64_t kLeast = 4000000, kMost = 1 << 30;  // bytes of an upload (the least: two images of 3 x 416 x 416 gain 3 %)
+constexpr int64_t kLeast = GH_PIECES_FROM, kMost = 1 << 30;  // bytes of an upload (the least: two images of 3 x 416 x 416 gain 3 %)
 constexpr int64_t kPieceBytes = 4 << 20;              // (8 x 3 x 416 x 416 in two, three, four and eight: 658, 637, 627 and 674 us)
 constexpr int kHead = 12;
 constexpr int kTries = 6;

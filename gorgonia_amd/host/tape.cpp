@@ -1088,7 +1088,7 @@ Status TapeMachine::Compile() {
   if (!opt_.node_at_a_time)
     for (int i = 0; i < N; i++) {
       const Node& x = nodes[(size_t)i];
-      if (!x.is_input || x.resident || x.shape.Dims() != 4) continue;
+      if (!x.is_input || x.resident || x.shape.Dims() != 4 || x.dt != Dtype::Float32 || x.shape[0] < 2 || bytes_of(x) < GH_PIECES_FROM) continue;
       int at = i, end = -1;
       std::vector<int> kept;
       for (;;) {

@@ -290,6 +290,7 @@ GH_API int gh_memcpy_d2d(gh_ctx* ctx, gh_devptr dst, gh_devptr src, int64_t byte
 /* src (any host memory) to dst by way of `stage` (memory of gh_host_alloc, `bytes` of it): the bus moves what has been
  * copied while the host copies the rest.  Returns when src has been read; `stage` must stay untouched until the next
  * gh_sync(). */
+#define GH_PIECES_FROM 4000000 /* gh_submit: below, a batch is copied whole and the layers behind it follow (GH_JOINT_PIECES) */
 #define GH_STAGED_FROM (128 << 10) /* below, one copy after the other */
 GH_API int gh_memcpy_staged(gh_ctx* ctx, gh_devptr dst, void* stage, const void* src, int64_t bytes);
 
@@ -415,7 +416,7 @@ enum gh_joint {
   /* a 3x3 convolution or its image gradient (k_conv_lanes.hip) by workgroups of several tiles each: 100 x the wavefronts of one +
    * 10 x its filter tiles + whether its wavefronts split the channels */
   GH_JOINT_CONV_ROUNDS = 3,
-  /* a batch out of pinned host memory in pieces, and the layers behind it piece by piece while the next one comes;
+  /* a batch of GH_PIECES_FROM bytes or more out of pinned host memory in pieces, and the layers behind it piece by piece while the next one comes;
      form: 100 * the pieces + the layers */
   GH_JOINT_PIECES = 4,
   GH_JOINT__COUNT
