@@ -556,6 +556,16 @@ int gh_submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
         continue;
       }
     }
+    // a SoftMax, and the scaled tensor and the gradient behind it
+    if (gh_softmax_gradient_follows(cmds + i, n - i)) {
+      for (int j = 1; j < 3; j++)
+        if ((rc = gh_flush_sums_before(ctx, cmds[i + j]))) return rc;
+      if ((rc = (cmds[i].opcode == GH_OP_GEMM ? gh_try_launch_gemm_softmax_gradient : gh_try_launch_softmax_gradient)(ctx, cmds + i)) >= 0) {
+        if (rc) return rc;
+        i += 2;
+        continue;
+      }
+    }
     // two commands of which the second reads what the first writes are one launch where a kernel takes both
     const bool held = gh_bn_held_pair(ctx, cmds + i, n - i), pair = held || gh_is_pair(cmds + i, n - i);
     if (cmds[i].opcode == GH_OP_MAXPOOL2D_BWD && (cmds[i].flags & GH_FLAG_BN_REMADE)) {
@@ -640,16 +650,6 @@ static constexpr auto kPollFor = std::chrono::microseconds(2000);
 // at every 32nd they do not, and the 3 us more of one wait in 32 cannot be told from noise.
 static constexpr uint32_t kRuntimeWaitEvery = 32;
 
-// Waits for everything on the context's stream.  The runtime's own wait puts a barrier packet with a
-// signal behind the last kernel and, where the work takes longer than some tens of microseconds, sleeps
-// until an interrupt: one small kernel and hipStreamSynchronize take 11.3 us, ten take 47.  Here a
-// kernel writes a sequence number to a pinned word behind the last one and the caller's thread polls
-// that word (8.5 and 31 us where the runtime wrote it).  An idle stream is not waited for at all (a tape machine's run asks twice).
-int gh_sync(gh_ctx* ctx) {
-  if (!ctx) return GH_EINVAL;
-  if (ctx->capturing) return gh_fail(ctx, GH_ESTATE, "gh_sync during graph capture");
-  if (ctx->idle) return ctx->err;
-  bool seen = false;
 // The completion word of gh_sync.  What the kernels in front have stored is visible to this one when it begins, and its release
 // takes that along to the host: results lie in coherent pinned memory, which no cache of the device holds back.  Bound: a
 // launch behind the last kernel, 1.3 us; the runtime's own write to a word (hipStreamWriteValue32) sets a barrier of its own
@@ -662,6 +662,16 @@ static bool say_done(gh_ctx* ctx, uint32_t seq) {
   return hipGetLastError() == hipSuccess;
 }
 
+// Waits for everything on the context's stream.  The runtime's own wait puts a barrier packet with a
+// signal behind the last kernel and, where the work takes longer than some tens of microseconds, sleeps
+// until an interrupt: one small kernel and hipStreamSynchronize take 11.3 us, ten take 47.  Here a
+// kernel writes a sequence number to a pinned word behind the last one and the caller's thread polls
+// that word (8.5 and 31 us where the runtime wrote it).  An idle stream is not waited for at all (a tape machine's run asks twice).
+int gh_sync(gh_ctx* ctx) {
+  if (!ctx) return GH_EINVAL;
+  if (ctx->capturing) return gh_fail(ctx, GH_ESTATE, "gh_sync during graph capture");
+  if (ctx->idle) return ctx->err;
+  bool seen = false;
   const uint32_t seq = ctx->done_seq + 1;
   if (ctx->done_word && !ctx->sync_block && !ctx->runtime_wait && !ctx->err && seq % kRuntimeWaitEvery != 0 &&
       say_done(ctx, seq)) {

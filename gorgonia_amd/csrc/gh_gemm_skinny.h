@@ -74,13 +74,15 @@ inline Args64 args64_of(const gh_cmd& c) {
 // transposed views alone reach here with so few columns): one column tile,
 // column indices clamped in the loads and masked in the store.
 //
-// Workgroup id of a grid of gx x gy tiles, slice bz of `slices` of K.  kPlain: no bias and no softmax.
+// Workgroup id of a grid of gx x gy tiles, slice bz of `slices` of K.  kPlain: no bias and no softmax; kGradient
+// (one column tile): a softmax, and `t` behind it.
 template <int WV, int NT>
 constexpr int lds16() { return WV * 16 * 16 * NT * 4; }
 
-template <int WV, int NT, bool TA, bool TB, bool kPlain>
-__device__ __forceinline__ void workgroup16(const Args32& g, int id, int gx, int gy, int bz, int slices, char* lds) {
-  const int M = g.M, N = g.N, K = g.K, lda = g.lda, ldb = g.ldb, ldc = g.ldc, act = g.act, softmax = kPlain ? 0 : g.softmax;
+template <int WV, int NT, bool TA, bool TB, bool kPlain, bool kGradient = false>
+__device__ __forceinline__ void workgroup16(const Args32& g, int id, int gx, int gy, int bz, int slices, char* lds,
+                                            const gh_softmax_gradient<float>& t = {}) {
+  const int M = g.M, N = g.N, K = g.K, lda = g.lda, ldb = g.ldb, ldc = g.ldc, act = g.act, softmax = kPlain ? 0 : kGradient ? 1 : g.softmax;
   const float alpha = g.alpha;
   const float *__restrict__ const A = g.A, *__restrict__ const B = g.B, *__restrict__ const bias = kPlain ? nullptr : g.bias;
   float* __restrict__ C = g.C;
@@ -221,8 +223,22 @@ __device__ __forceinline__ void workgroup16(const Args32& g, int id, int gx, int
     if (e < TILE && col < N) {
       float sum = 0.f;
       for (int j = 0; j < N; j++) sum = sum + sm_e[row * 17 + j];
-      const float inv = 1.0f / sum;
-      C[(int64_t)(m0 + row) * ldc + col] = sm_e[row * 17 + col] * inv;
+      const float inv = 1.0f / sum, y = sm_e[row * 17 + col] * inv;
+      C[(int64_t)(m0 + row) * ldc + col] = y;
+      if constexpr (kGradient) {
+        const int64_t at = (int64_t)(m0 + row) * N + col;
+        const float v = t.x[at] * *t.s;
+        sm_x[row * 17 + col] = v * y;   // (a row's 16 threads are of one wavefront, which is past its reads of sm_x)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        float dot = 0.f;
+        for (int j = 0; j < N; j++) dot = dot + sm_x[row * 17 + j];
+        const float d = v - dot;
+        if (m0 + row >= tile_y * 16) {   // (the last tile's first rows are the one's before it, where x may be g)
+          t.g[at] = v;
+          t.dx[at] = y * d;
+        }
+      }
     }
     return;
   }

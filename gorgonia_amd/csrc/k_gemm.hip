@@ -657,11 +657,20 @@ __global__ __launch_bounds__(WV * 64) void k_gemm_skinny16(const gemm_skinny::Ar
                                                   (int)gridDim.z, lds);
 }
 
+// A classifier's product with its softmax, and behind it the scaled labels and the softmax gradient (k_pairs.hip's arithmetic):
+// the row is in LDS.  Bound: as without them; 128 x 10, K = 625 in a kernel of its own behind this one 4.6 us.
+template <int WV>
+__global__ __launch_bounds__(WV * 64) void k_gemm_softmax_gradient(const gemm_skinny::Args32 g, const gh_softmax_gradient<float> t) {
+  __shared__ __attribute__((aligned(16))) char lds[gemm_skinny::lds16<WV, 1>()];
+  gemm_skinny::workgroup16<WV, 1, false, false, false, true>(g, (int)(blockIdx.y * gridDim.x + blockIdx.x), (int)gridDim.x, (int)gridDim.y, 0, 1, lds, t);
+}
+
 // Adds the slabs of a small-output product cut along K, in slab order, and applies the epilogue: bias, activation,
-// and the row softmax with the arithmetic of the softmax kernel (N <= 32: 32 lanes hold a row).
+// and the row softmax with the arithmetic of the softmax kernel (N <= 32: 32 lanes hold a row); kGradient: and `g` behind that.
+template <bool kGradient>
 __global__ __launch_bounds__(256) void k_skinny_sum(const float* __restrict__ ws, int slabs, int M, int N,
                                                     float* __restrict__ C, int ldc, int act, float alpha,
-                                                    const float* __restrict__ bias, int softmax) {
+                                                    const float* __restrict__ bias, int softmax, const gh_softmax_gradient<float> t) {
   const int64_t total = (int64_t)M * N;
   const int width = softmax ? 32 : N;
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x, row = e / width;
@@ -691,10 +700,22 @@ __global__ __launch_bounds__(256) void k_skinny_sum(const float* __restrict__ ws
     for (int j = 0; j < N; j++) mx = fmaxf(mx, x[r][j]);
     ex[r][col] = mine ? (float)exp((double)(sum - mx)) : 0.f;
     __syncthreads();
-    float t = 0.f;
-    for (int j = 0; j < N; j++) t = t + ex[r][j];
-    const float inv = 1.0f / t;
+    float all = 0.f;
+    for (int j = 0; j < N; j++) all = all + ex[r][j];
+    const float inv = 1.0f / all;
     sum = ex[r][col] * inv;
+    if constexpr (kGradient) {
+      const float v = mine ? t.x[row * N + col] * *t.s : 0.f;
+      x[r][col] = v * sum;   // (read last in front of the barrier above)
+      __syncthreads();
+      float dot = 0.f;
+      for (int j = 0; j < N; j++) dot = dot + x[r][j];
+      const float d = v - dot;
+      if (mine) {
+        t.g[row * N + col] = v;
+        t.dx[row * N + col] = sum * d;
+      }
+    }
   }
   if (mine) C[row * ldc + col] = sum;
 }
@@ -2636,10 +2657,12 @@ static int skinny_slices(const gh_cmd& c, int cus) {
 
 static int launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c, int slices);
 
-static int try_launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c) {
+// `t`: what is behind the product's softmax; only where the product is cut
+static int try_launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c, const gh_softmax_gradient<float>* t = nullptr) {
   if (!gemm_skinny_takes(c, ctx->cu_count)) return -1;
   const int slices = skinny_slices(c, ctx->cu_count);
   const int64_t M = c.dim[0], N = c.dim[1];
+  if (t && (slices == 1 || (int64_t)slices * M * N * 4 > ctx->workspace_bytes)) return -1;
   if (slices > 1 && (int64_t)slices * M * N * 4 > ctx->workspace_bytes) {
     if (int rc = gh_ws_short(ctx, (int64_t)slices * M * N * 4)) return rc;
     return launch_gemm_skinny(ctx, c, 1);
@@ -2652,9 +2675,9 @@ static int try_launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c) {
   if (int rc = launch_gemm_skinny(ctx, part, slices)) return rc;
   const int softmax = (c.flags & GH_FLAG_GEMM_SOFTMAX) ? 1 : 0;
   const int act = (c.flags & GH_FLAG_ACT_RELU) ? 1 : (c.flags & GH_FLAG_ACT_LEAKY) ? 2 : 0;
-  hipLaunchKernelGGL(k_skinny_sum, dim3((unsigned)cdiv(M * (softmax ? 32 : N), 256)), dim3(256), 0, ctx->stream,
+  hipLaunchKernelGGL(t ? k_skinny_sum<true> : k_skinny_sum<false>, dim3((unsigned)cdiv(M * (softmax ? 32 : N), 256)), dim3(256), 0, ctx->stream,
                      (const float*)ctx->workspace, slices, (int)M, (int)N, (float*)(uintptr_t)c.ptr[2], (int)c.dim[5], act, c.f[0],
-                     (c.flags & GH_FLAG_GEMM_BIAS) ? (const float*)(uintptr_t)c.ptr[3] : nullptr, softmax);
+                     (c.flags & GH_FLAG_GEMM_BIAS) ? (const float*)(uintptr_t)c.ptr[3] : nullptr, softmax, t ? *t : gh_softmax_gradient<float>{});
   return gh_check_hip(ctx, hipGetLastError(), "skinny gemm slab sum launch");
 }
 
@@ -2674,10 +2697,16 @@ static Skinny16 skinny16_form(const gh_cmd& c, int cus) {
   return {c.dim[2] >= 512 && !no16 ? 16 : 8, narrow ? 1 : 2};
 }
 
+// Whether an untransposed product is one of the 16-row kernel's.
+static bool skinny_tiles16(const gh_cmd& c, int cus) {
+  const int64_t M = c.dim[0], N = c.dim[1], tiles = cdiv(M, 32) * cdiv(N, 32);
+  const char* force = force_tile();
+  return M >= 16 && (N <= 16 || (N > 32 && tiles * 2 <= cus)) && !(force && !strcmp(force, "32"));
+}
+
 static int launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c, int slices) {
   const bool ta = c.flags & GH_FLAG_TRANS_A, tb = c.flags & GH_FLAG_TRANS_B;
   const int M = (int)c.dim[0], N = (int)c.dim[1], K = (int)c.dim[2];
-  const int64_t tiles = cdiv(M, 32) * cdiv(N, 32);
   const int lda = (int)c.dim[3], ldb = (int)c.dim[4], ldc = (int)c.dim[5];
   const int act = (c.flags & GH_FLAG_ACT_RELU) ? 1 : (c.flags & GH_FLAG_ACT_LEAKY) ? 2 : 0;
   constexpr int WV = 8;  // 512 threads leave each wavefront 256 registers for the grouped loads
@@ -2692,10 +2721,7 @@ static int launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c, int slices) {
   // bits: N <= 16 goes to the 16x16 tiles (softmax in their epilogue), 16 < N <=
   // 32 stays on the 32x32 tile.  Transposed views (the weight and input
   // gradients of a dense layer) only have the 16-row kernel.
-  const char* force = force_tile();
-  const bool transposed = ta || tb;
-  const bool tiles16 = N <= 16 || (N > 32 && tiles * 2 <= ctx->cu_count);
-  if (transposed || (M >= 16 && tiles16 && !(force && !strcmp(force, "32")))) {
+  if (ta || tb || skinny_tiles16(c, ctx->cu_count)) {
     const Skinny16 f = skinny16_form(c, ctx->cu_count);
     const bool narrow = f.columns == 1, wide16 = f.waves == 16;
     const gemm_skinny::Args32 g = gemm_skinny::args32_of(c);
@@ -2730,6 +2756,32 @@ static int launch_gemm_skinny(gh_ctx* ctx, const gh_cmd& c, int slices) {
   else if (vec_b) launch(k_gemm_skinny<WV, false, true>);
   else launch(k_gemm_skinny<WV, false, false>);
   return gh_check_hip(ctx, hipGetLastError(), "skinny gemm launch");
+}
+
+int gh_try_launch_gemm_softmax_gradient(gh_ctx* ctx, const gh_cmd* c) {
+  const gh_cmd& p = c[0];
+  if (gh_dtype_of(p.flags) != GH_F32 || p.dim[0] <= 0 || gh_gemm_thin_takes(p) || !gemm_skinny_takes(p, ctx->cu_count) || p.dim[1] > 32) return -1;
+  const gh_softmax_gradient<float> t = {(const float*)(uintptr_t)c[1].ptr[0], (const float*)(uintptr_t)c[1].ptr[1],
+                                        (float*)(uintptr_t)(c[1].ptr[2] ? c[1].ptr[2] : c[1].ptr[0]), (float*)(uintptr_t)c[2].ptr[2]};
+  int rc, form = 2;
+  if (skinny_slices(p, ctx->cu_count) > 1) {
+    rc = try_launch_gemm_skinny(ctx, p, &t);
+    form = 3;
+  } else {
+    if (!skinny_tiles16(p, ctx->cu_count) || p.dim[1] > 16) return -1;
+    const Skinny16 f = skinny16_form(p, ctx->cu_count);
+    if (f.columns != 1) return -1;
+    const dim3 grid(1, (unsigned)cdiv(p.dim[0], 16));
+    if (f.waves == 16) hipLaunchKernelGGL(k_gemm_softmax_gradient<16>, grid, dim3(16 * 64), 0, ctx->stream, gemm_skinny::args32_of(p), t);
+    else hipLaunchKernelGGL(k_gemm_softmax_gradient<8>, grid, dim3(8 * 64), 0, ctx->stream, gemm_skinny::args32_of(p), t);
+    rc = gh_check_hip(ctx, hipGetLastError(), "gemm and softmax gradient launch");
+  }
+  if (rc < 0) return rc;
+  for (int k = 0; k < 3; k++)
+    for (uint64_t q : c[k].ptr) ctx->llc.touch(q, 0, false);
+  ctx->joint[GH_JOINT_SOFTMAX_GRADIENT].launches++;
+  ctx->joint[GH_JOINT_SOFTMAX_GRADIENT].form = form;
+  return rc;
 }
 
 template <int BM, int BN, int BK>

@@ -8,6 +8,9 @@
 //   * float64 gradient of that pooling and the Rectify gradient behind it, in place or not.
 //   * a tensor times a scalar and the SoftMax gradient that takes it as dy: a wavefront per row.
 //
+//   * a SoftMax in front of these two, of up to 64 columns: the row's values stay in the wavefront's registers.  (A product
+//     with its SoftMax in front of them: k_gemm.hip.)
+//
 // Bound: HBM for large tensors, the launch for small ones.  us, apart / as a pair: Rectify and pooling of 50 x 32 x 28 x 28
 // 10.5 / 4.2 (3.7 TB/s from the caches), of 128 images 18.3 / 9.8 (5.9 TB/s); the gradients 14.5 / 4.6 and 22.6 / 13.1; a
 // float64 training step of the example's network at batch 50 253 / 225.  50 x 10, scaled and SoftMax gradient 5.3 / 3.1,
@@ -155,6 +158,39 @@ __global__ __launch_bounds__(kBlock) void k_scale_softmax_bwd(const T* x, const 
   }
 }
 
+// y = SoftMax(z), g = x s and dx of y and g, with the arithmetic of k_softmax, k_softmax_f64 and the kernel above.  (x and g
+// may be one tensor, and z any of those written: a wavefront reads a row before it writes it.)
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_softmax_gradient(const T* z, T* y, const gh_softmax_gradient<T> t, int64_t rows, int cols) {
+  const int lane = (int)threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int64_t at = row * cols + lane;
+  const bool there = lane < cols;
+  const T v = there ? z[at] : (T)-INFINITY, scaled = there ? t.x[at] * *t.s : (T)0;
+  T mx = there ? fmax((T)-INFINITY, v) : (T)-INFINITY;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
+  const T e = there ? (T)exp((double)(v - mx)) : (T)0;
+  T sum = (T)0;
+  for (int l = 0; l < cols; l++) sum = sum + __shfl(e, l, 64);
+  T mine;
+  if constexpr (sizeof(T) == 8) {
+    mine = e / sum;
+  } else {
+    const T inv = 1.0f / sum;
+    mine = e * inv;
+  }
+  const T p = scaled * mine;
+  T dot = (T)0;
+  for (int l = 0; l < cols; l++) dot = dot + __shfl(p, l, 64);
+  if (!there) return;
+  y[at] = mine;
+  t.g[at] = scaled;
+  const T d = scaled - dot;
+  t.dx[at] = mine * d;
+}
+
 // ---- which commands ---------------------------------------------------------------------
 
 enum { kNone, kReluPool, kPoolReluBwd, kScaleSoftmaxBwd };
@@ -213,6 +249,52 @@ bool gh_is_pair(const gh_cmd* cmds, int n) {
   if (!(a == GH_OP_RELU && b == GH_OP_MAXPOOL2D) && !(a == GH_OP_MAXPOOL2D_BWD && b == GH_OP_RELU_BWD) && !(a == GH_OP_ELEM_BIN && b == GH_OP_SOFTMAX_BWD)) return false;
   std::string m;
   return gh_validate_cmd(cmds[1], m) == GH_OK && kind_of(cmds) != kNone;
+}
+
+// A SOFTMAX, or a GEMM with one: the two commands behind it take its result, and write nothing that it or another row's
+// workgroup reads.
+bool gh_softmax_gradient_follows(const gh_cmd* c, int n) {
+  if (n < 3 || c[1].opcode != GH_OP_ELEM_BIN || c[2].opcode != GH_OP_SOFTMAX_BWD) return false;
+  const bool product = c[0].opcode == GH_OP_GEMM;
+  if (product ? !(c[0].flags & GH_FLAG_GEMM_SOFTMAX) || c[0].dim[6] > 1 || c[0].dim[5] != c[0].dim[1] : c[0].opcode != GH_OP_SOFTMAX) return false;
+  std::string m;
+  if (gh_dtype_of(c[0].flags) != gh_dtype_of(c[1].flags) || gh_validate_cmd(c[1], m) || gh_validate_cmd(c[2], m) || kind_of(c + 1) != kScaleSoftmaxBwd) return false;
+  const gh_cmd &f = c[1], &s = c[2];
+  const int64_t item = gh_dtype_of(f.flags) == GH_F64 ? 8 : 4, bytes = s.dim[0] * s.dim[1] * item;
+  const uint64_t y = c[0].ptr[product ? 2 : 1], g = f.ptr[2] ? f.ptr[2] : f.ptr[0], dx = s.ptr[2];
+  if (s.ptr[0] != y || s.dim[0] != c[0].dim[0] || s.dim[1] != c[0].dim[1]) return false;
+  if (!apart(y, bytes, f.ptr[0], bytes) || !apart(y, bytes, f.ptr[1], item)) return false;
+  if (!product) {
+    const uint64_t z = c[0].ptr[0];
+    for (uint64_t out : {y, g, dx})
+      if (out != z && !apart(out, bytes, z, bytes)) return false;
+    return (z & (uint64_t)(item - 1)) == 0;
+  }
+  const int64_t rows = c[0].dim[0], cols = c[0].dim[1], depth = c[0].dim[2];
+  for (uint64_t out : {g, dx})
+    if (!apart(out, bytes, c[0].ptr[0], ((rows - 1) * c[0].dim[3] + depth) * item) || !apart(out, bytes, c[0].ptr[1], ((depth - 1) * c[0].dim[4] + cols) * item) ||
+        ((c[0].flags & GH_FLAG_GEMM_BIAS) && !apart(out, bytes, c[0].ptr[3], cols * item)))
+      return false;
+  return true;
+}
+
+int gh_try_launch_softmax_gradient(gh_ctx* ctx, const gh_cmd* c) {
+  const int64_t rows = c[0].dim[0];
+  const int cols = (int)c[0].dim[1];
+  if (c[0].dim[1] > 64) return -1;
+  for (int k = 0; k < 3; k++)
+    for (uint64_t p : c[k].ptr) ctx->llc.touch(p, 0, false);
+  auto go = [&](auto* zero) {
+    typedef std::remove_pointer_t<decltype(zero)> T;
+    const gh_softmax_gradient<T> t = {at<const T>(c[1].ptr[0]), at<const T>(c[1].ptr[1]), at<T>(c[1].ptr[2] ? c[1].ptr[2] : c[1].ptr[0]), at<T>(c[2].ptr[2])};
+    hipLaunchKernelGGL(k_softmax_gradient<T>, dim3((unsigned)((rows + kBlock / 64 - 1) / (kBlock / 64))), dim3(kBlock), 0, ctx->stream, at<const T>(c[0].ptr[0]),
+                       at<T>(c[0].ptr[1]), t, rows, cols);
+  };
+  if (gh_dtype_of(c[0].flags) == GH_F64) go((double*)nullptr);
+  else go((float*)nullptr);
+  ctx->joint[GH_JOINT_SOFTMAX_GRADIENT].launches++;
+  ctx->joint[GH_JOINT_SOFTMAX_GRADIENT].form = 1;
+  return gh_check_hip(ctx, hipGetLastError(), "softmax and its gradient launch");
 }
 
 int gh_launch_pair(gh_ctx* ctx, const gh_cmd* c) {

@@ -419,6 +419,9 @@ enum gh_joint {
   /* a batch of GH_PIECES_FROM bytes or more out of pinned host memory in pieces, and the layers behind it piece by piece while the next one comes;
      form: 100 * the pieces + the layers */
   GH_JOINT_PIECES = 4,
+  /* a SoftMax with the scaled tensor and the SoftMax gradient behind it; form: 1 behind a SOFTMAX command, 2 in the product's
+     kernel, 3 in the sum of the product's slabs */
+  GH_JOINT_SOFTMAX_GRADIENT = 5,
   GH_JOINT__COUNT
 };
 GH_API int64_t gh_joint_launches(const gh_ctx* ctx, int kind, int64_t* form);
