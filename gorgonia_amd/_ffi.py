@@ -121,7 +121,7 @@ SYMBOLS = {
 }
 
 # enum gh_joint
-JOINT_CONV_GRADIENTS, JOINT_DENSE_GRADIENTS, JOINT_SOLVER_SUMS, JOINT_CONV_ROUNDS, JOINT_PIECES, JOINT_SOFTMAX_GRADIENT = range(6)
+JOINT_CONV_GRADIENTS, JOINT_DENSE_GRADIENTS, JOINT_SOLVER_SUMS, JOINT_CONV_ROUNDS, JOINT_PIECES, JOINT_SOFTMAX_GRADIENT, JOINT_UNPOOLED = range(7)
 
 _lib = None
 

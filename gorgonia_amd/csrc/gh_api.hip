@@ -538,12 +538,21 @@ int gh_submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
     if (gh_gradient_pair(cmds + i, n - i)) {
       if ((rc = gh_flush_sums_before(ctx, cmds[i + 1]))) return rc;
       const bool first = cmds[i].opcode == GH_OP_CONV2D_BWD_FILTER;
+      gh_unpool unpool;
+      const int behind = gh_unpool_follows(cmds + i, n - i, &unpool);
+      for (int j = 0; j < behind; j++)
+        if ((rc = gh_flush_sums_before(ctx, cmds[i + 2 + j]))) return rc;
+      if (behind) ctx->unpool = unpool;
       ctx->hold_filter = true;
       rc = dispatch(ctx, cmds[first ? i : i + 1]);
       ctx->hold_filter = false;
       if (!rc) rc = dispatch(ctx, cmds[first ? i + 1 : i]);
       const int alone = gh_launch_held(ctx);
+      const bool unpooled = ctx->unpool.done;
+      ctx->unpool = gh_unpool{};
       if (rc || alone) return rc ? rc : alone;
+      for (int j = 0; unpooled && j < behind; j++, i++)
+        for (uint64_t p : cmds[i + 2].ptr) ctx->llc.touch(p, 0, false);
       i++;
       continue;
     }

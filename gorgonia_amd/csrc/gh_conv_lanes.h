@@ -71,6 +71,11 @@ struct Lanes {
   int ftiles, ptiles, ft_major;
 };
 
+// The 2x2 / 2 pooling's gradient behind an image gradient whose result is the pooled values' (2 oh x 2 ow values each), read
+// through a Rectify, and that one's gradient.  float: z; double: a, what was pooled, z in front of its Rectify, and da, the
+// pooling's gradient, where it is not dz.
+template <class T> struct Unpool { const T* a; const T* z; T* da; T* dz; };
+
 // LDS of a workgroup: the wavefronts' sums of 16 filter rows, the filters' constants
 template <class T, int WV, int TM, int V, int G, bool kSplit>
 constexpr int lds_of(bool flip) {
@@ -78,8 +83,9 @@ constexpr int lds_of(bool flip) {
 }
 
 // Workgroup `block` of `blocks`; lds: lds_of bytes.
-template <class T, int WV, int TM, int V, int G, bool kSplit, bool kFlip, bool kPool>
-__device__ __forceinline__ void workgroup(const Lanes<T>& g, const ConvTail& tail, int block, int blocks, char* lds) {
+template <class T, int WV, int TM, int V, int G, bool kSplit, bool kFlip, bool kPool, bool kUnpool = false>
+__device__ __forceinline__ void workgroup(const Lanes<T>& g, const ConvTail& tail, int block, int blocks, char* lds, const Unpool<T>& u = {}) {
+  static_assert(!kUnpool || (kSplit && kFlip && !kPool), "behind an image gradient whose wavefronts share the channels");
   typedef Mac<T> U;
   typedef typename U::acc Acc;
   constexpr int S = (int)sizeof(T), TN = V * G;
@@ -267,6 +273,32 @@ __device__ __forceinline__ void workgroup(const Lanes<T>& g, const ConvTail& tai
   };
 #pragma unroll
   for (int m = 0; m < TM; m++) {
+    // the windows that this thread's results go back to, loaded under the meeting of the wavefronts
+    typedef T Two __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+    constexpr int kWindows = kUnpool ? TN * 256 / nthreads : 1;
+    static_assert(!kUnpool || TN * 256 % nthreads == 0, "whole rounds of windows");
+    [[maybe_unused]] Two z0[kWindows], z1[kWindows], a0[kWindows], a1[kWindows];
+    [[maybe_unused]] int64_t pooled[kWindows];
+    [[maybe_unused]] int column[kWindows];
+    if constexpr (kUnpool) {
+#pragma unroll
+      for (int k = 0; k < kWindows; k++) {
+        const int e = tid + k * nthreads, r = e / (16 * TN), col = e - r * (16 * TN), f = f0 + 16 * m + r, grp = g0 + col / V;
+        pooled[k] = -1;
+        if (f >= g.F || grp >= g.groups) continue;
+        int b, oy, ox;
+        place(grp, &b, &oy, &ox);
+        column[k] = ox + col % V;
+        pooled[k] = (((int64_t)b * g.F + f) * g.oh + oy) * g.ow + column[k];
+        const int64_t at = 4 * pooled[k] - 2 * column[k];   // (row r, column c of ow values: row 2 r, column 2 c of 2 ow)
+        z0[k] = *(const Two*)(u.z + at);
+        z1[k] = *(const Two*)(u.z + at + 2 * g.ow);
+        if constexpr (sizeof(T) == 8) {
+          a0[k] = *(const Two*)(u.a + at);
+          a1[k] = *(const Two*)(u.a + at + 2 * g.ow);
+        }
+      }
+    }
     if (m) __syncthreads();
 #pragma unroll
     for (int n = 0; n < G; n++)
@@ -290,6 +322,41 @@ __device__ __forceinline__ void workgroup(const Lanes<T>& g, const ConvTail& tai
         int b, oy, ox;
         place(grp, &b, &oy, &ox);
         g.y[(((int64_t)b * g.F + f) * (g.rows >> 1) + (oy >> 1)) * (g.cols >> 1) + (ox >> 1) + k] = best;
+      }
+    } else if constexpr (kUnpool) {
+      // scan order, strict > and "0 + dy" of the pooling's gradient, and the Rectify's behind it, as their kernels have them
+#pragma unroll
+      for (int k = 0; k < kWindows; k++) {
+        if (pooled[k] < 0) continue;
+        const int e = tid + k * nthreads;
+        const T own = epilogue(16 * m + e / (16 * TN), value(e));
+        const int64_t at = 4 * pooled[k] - 2 * column[k], row = 2 * (int64_t)g.ow;
+        g.y[pooled[k]] = own;
+        T mask[4], v[4] = {z0[k][0], z0[k][1], z1[k][0], z1[k][1]};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          mask[j] = v[j] >= (T)0 ? (T)1 : (T)0;
+          v[j] = sizeof(T) == 8 ? (j < 2 ? a0[k][j & 1] : a1[k][j & 1]) : v[j] * mask[j];
+        }
+        T best = sizeof(T) == 8 ? (T)-1.7976931348623157e+308 : (T)-3.402823466e+38f;
+        int arg = -1;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (v[j] > best) { best = v[j]; arg = j; }
+        const T back = (T)0 + own;
+        T d[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) d[j] = arg == j ? back : (T)0;
+        if constexpr (sizeof(T) == 8) {
+          if (u.da != u.dz) {
+            *(Two*)(u.da + at) = Two{d[0], d[1]};
+            *(Two*)(u.da + at + row) = Two{d[2], d[3]};
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) d[j] = d[j] * mask[j];
+        *(Two*)(u.dz + at) = Two{d[0], d[1]};
+        *(Two*)(u.dz + at + row) = Two{d[2], d[3]};
       }
     } else {
       for (int e = tid; e < TN * 256; e += nthreads) {

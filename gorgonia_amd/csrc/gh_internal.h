@@ -65,6 +65,9 @@ struct gh_held_filter {
   size_t lds = 0;
   alignas(16) unsigned char args[192];
 };
+// a pooling's gradient that an image gradient's launch takes along (k_conv_gradients.hip); dz 0: none
+struct gh_unpool { uint64_t a = 0, z = 0, da = 0, dz = 0; bool done = false; };
+
 constexpr int kUnits = 256;   // the MI355X's compute units
 constexpr int kSlabSums = 8;
 constexpr int64_t kSlabSpace = 24ll << 20;
@@ -96,6 +99,7 @@ struct gh_ctx {
   bool defer_sums = false;
   bool hold_filter = false;   // the next filter gradient may be held
   gh_held_filter held;
+  gh_unpool unpool;
   struct { int64_t launches = 0, form = 0; } joint[GH_JOINT__COUNT];   // gh_joint_launches
   // set while gh_submit_noalloc runs: the scratch is the library's fixed array and a
   // plan may not shrink to fit it (results must not depend on the scratch size)
@@ -216,6 +220,7 @@ int gh_launch_conv_wgrad(gh_ctx* ctx, const gh_cmd& c);
 // both gradients of a 3x3 convolution in one launch (k_conv_gradients.hip)
 bool gh_gradient_pair(const gh_cmd* cmds, int n);
 int gh_launch_held(gh_ctx* ctx);
+int gh_unpool_follows(const gh_cmd* cmds, int n, gh_unpool* out);
 int gh_launch_held_wgrad(gh_ctx* ctx);         // k_conv_wgrad.hip
 int gh_launch_held_wgrad_small(gh_ctx* ctx);   // k_conv_wgrad_small.hip
 // whether a filter gradient that writes `out` (slabs, or the result itself) may be held: not where it uses the workspace

@@ -15,6 +15,12 @@
 // for a third workgroup to a compute unit, float64's by two meetings of half the LDS, spill and lose what they gain: 96 x 32 x 14 x 14
 // 48.7.  The float32 form that had two filter-gradient workgroups side by side in eight wavefronts spilled, 57 for 35.)
 //
+// Where the convolution's input was pooled (2x2 / 2, even extents), the pooling's gradient and its Rectify's, which take the image
+// gradient value by value, are in the launch as well (gh_unpool_follows): the windows are loaded under the meeting of the wavefronts
+// that share a tile's channels, and the pass over memory runs under the other workgroups' matrix instructions.  Only behind the
+// kernels whose wavefronts share the channels; the others store whole rows from registers.  A training step of the example's network,
+// two such layers: 128 images 184.9 / 181.2, 50 in float64 184.9 / 178.5.
+//
 // gh_submit holds a filter gradient back (gh_held_filter) where an image gradient that has nothing to do with its result
 // stands beside it; the image gradient's launch takes it along, or it is launched by itself behind that.
 #include <algorithm>
@@ -28,6 +34,7 @@
 namespace {
 
 using conv_lanes::Lanes;
+using conv_lanes::Unpool;
 using conv_wgrad::Wg;
 
 // The filter gradient's grid: x, y and all workgroups.
@@ -41,8 +48,9 @@ struct Grid {
   }
 };
 
-template <int kRowPitch, int TM>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_conv3x3_gradients_small(const gh_wgrad_small_args w, const Grid grid, const Lanes<float> g) {
+template <int kRowPitch, int TM, bool kUnpool>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_conv3x3_gradients_small(const gh_wgrad_small_args w, const Grid grid, const Lanes<float> g,
+                                                                                                          const Unpool<float> u) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int b = (int)blockIdx.x;
   if (b < grid.all) {
@@ -50,13 +58,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
     grid.at(b, &bx, &by, &bz);
     conv_wgrad_small::workgroup<kRowPitch>(w.x, w.dy, w.out, w.g, w.slab, bx, by, bz, (float*)lds);
   } else {
-    conv_lanes::workgroup<float, 8, TM, 4, 1, true, true, false>(g, ConvTail{}, b - grid.all, (int)gridDim.x - grid.all, lds);
+    conv_lanes::workgroup<float, 8, TM, 4, 1, true, true, false, kUnpool>(g, ConvTail{}, b - grid.all, (int)gridDim.x - grid.all, lds, u);
   }
 }
 
 // (Where the image gradient's workgroups have eight wavefronts, the filter gradient's use the first four of theirs.)
-template <class T, int TMW, int P, int WV, int TM, int V, bool kSplit>
-__global__ __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 2 : 3))) void k_conv3x3_gradients(const Wg<T> w, const Grid grid, const Lanes<T> g) {
+template <class T, int TMW, int P, int WV, int TM, int V, bool kSplit, bool kUnpool>
+__global__ __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 2 : 3))) void k_conv3x3_gradients(const Wg<T> w, const Grid grid, const Lanes<T> g,
+                                                                                                                          const Unpool<T> u) {
   constexpr int wl = conv_wgrad::lds_of<T, 9>(), ll = conv_lanes::lds_of<T, WV, TM, V, 1, kSplit>(true);
   __shared__ __attribute__((aligned(16))) char lds[wl > ll ? wl : ll];
   const int b = (int)blockIdx.x;
@@ -66,32 +75,43 @@ __global__ __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(sizeof(
     grid.at(b, &bx, &by, &bz);
     conv_wgrad::workgroup<T, TMW, P, 9, false>(w, bx, by, bz, lds);
   } else {
-    conv_lanes::workgroup<T, WV, TM, V, 1, kSplit, true, false>(g, ConvTail{}, b - grid.all, (int)gridDim.x - grid.all, lds);
+    conv_lanes::workgroup<T, WV, TM, V, 1, kSplit, true, false, kUnpool>(g, ConvTail{}, b - grid.all, (int)gridDim.x - grid.all, lds, u);
   }
 }
 
 Grid grid_of(const gh_held_filter& h) { return {(int)h.grid.x, (int)h.grid.y, (int)(h.grid.x * h.grid.y * h.grid.z)}; }
 
-template <int kRowPitch, int TM>
-int go_small(gh_ctx* ctx, const Lanes<float>& g, int blocks) {
+template <class T> Unpool<T> unpool_of(const gh_ctx* ctx) {
+  const gh_unpool& u = ctx->unpool;
+  return {(const T*)(uintptr_t)u.a, (const T*)(uintptr_t)u.z, (T*)(uintptr_t)u.da, (T*)(uintptr_t)u.dz};
+}
+
+template <int kRowPitch, int TM, bool kUnpool>
+int go_small_as(gh_ctx* ctx, const Lanes<float>& g, int blocks) {
   static std::once_flag once;
   static hipError_t attr_rc = hipSuccess;
-  std::call_once(once, [] { attr_rc = hipFuncSetAttribute((const void*)k_conv3x3_gradients_small<kRowPitch, TM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); });
+  std::call_once(once, [] { attr_rc = hipFuncSetAttribute((const void*)k_conv3x3_gradients_small<kRowPitch, TM, kUnpool>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); });
   if (attr_rc != hipSuccess) return gh_check_hip(ctx, attr_rc, "hipFuncSetAttribute(conv3x3 gradients)");
   const Grid grid = grid_of(ctx->held);
   gh_wgrad_small_args w;
   memcpy(&w, ctx->held.args, sizeof w);
   const size_t lds = std::max<size_t>(ctx->held.lds, conv_lanes::lds_of<float, 8, TM, 4, 1, true>(true));
-  hipLaunchKernelGGL((k_conv3x3_gradients_small<kRowPitch, TM>), dim3((unsigned)(grid.all + blocks)), dim3(512), lds, ctx->stream, w, grid, g);
+  hipLaunchKernelGGL((k_conv3x3_gradients_small<kRowPitch, TM, kUnpool>), dim3((unsigned)(grid.all + blocks)), dim3(512), lds, ctx->stream, w, grid, g, unpool_of<float>(ctx));
+  ctx->unpool.done = kUnpool;
   return GH_OK;
 }
+template <int kRowPitch, int TM>
+int go_small(gh_ctx* ctx, const Lanes<float>& g, int blocks) {
+  return ctx->unpool.dz ? go_small_as<kRowPitch, TM, true>(ctx, g, blocks) : go_small_as<kRowPitch, TM, false>(ctx, g, blocks);
+}
 
-template <class T, int TMW, int P, int WV, int TM, int V, bool kSplit>
+template <class T, int TMW, int P, int WV, int TM, int V, bool kSplit, bool kUnpool = false>
 int go(gh_ctx* ctx, const Lanes<T>& g, int blocks) {
   const Grid grid = grid_of(ctx->held);
   Wg<T> w;
   memcpy(&w, ctx->held.args, sizeof w);
-  hipLaunchKernelGGL((k_conv3x3_gradients<T, TMW, P, WV, TM, V, kSplit>), dim3((unsigned)(grid.all + blocks)), dim3(WV * 64), 0, ctx->stream, w, grid, g);
+  hipLaunchKernelGGL((k_conv3x3_gradients<T, TMW, P, WV, TM, V, kSplit, kUnpool>), dim3((unsigned)(grid.all + blocks)), dim3(WV * 64), 0, ctx->stream, w, grid, g, unpool_of<T>(ctx));
+  ctx->unpool.done = kUnpool;
   return GH_OK;
 }
 
@@ -99,6 +119,10 @@ int done(gh_ctx* ctx, int rc, int tm, bool split) {
   auto& j = ctx->joint[GH_JOINT_CONV_GRADIENTS];
   j.launches += rc == GH_OK;
   j.form = 100 * ctx->held.kind + 10 * tm + split;
+  if (ctx->unpool.done) {
+    ctx->joint[GH_JOINT_UNPOOLED].launches += rc == GH_OK;
+    ctx->joint[GH_JOINT_UNPOOLED].form = j.form;
+  }
   ctx->held.kind = kHeldNone;
   return rc ? rc : gh_check_hip(ctx, hipGetLastError(), "convolution gradients launch");
 }
@@ -123,8 +147,8 @@ int gh_try_launch_gradients(gh_ctx* ctx, const conv_lanes::Lanes<float>& g, int 
 int gh_try_launch_gradients(gh_ctx* ctx, const conv_lanes::Lanes<double>& g, int waves, int tm, bool split, int blocks) {
   if (waves != 4 || tm != 1 || !split || getenv("GORGONIA_HIP_CONV_APART")) return -1;
   switch (ctx->held.kind) {
-    case kHeldF64: return done(ctx, go<double, 1, 4, 4, 1, 2, true>(ctx, g, blocks), tm, split);
-    case kHeldF64Narrow: return done(ctx, go<double, 1, 2, 4, 1, 2, true>(ctx, g, blocks), tm, split);
+    case kHeldF64: return done(ctx, ctx->unpool.dz ? go<double, 1, 4, 4, 1, 2, true, true>(ctx, g, blocks) : go<double, 1, 4, 4, 1, 2, true>(ctx, g, blocks), tm, split);
+    case kHeldF64Narrow: return done(ctx, ctx->unpool.dz ? go<double, 1, 2, 4, 1, 2, true, true>(ctx, g, blocks) : go<double, 1, 2, 4, 1, 2, true>(ctx, g, blocks), tm, split);
   }
   return -1;
 }
@@ -156,4 +180,42 @@ bool gh_gradient_pair(const gh_cmd* cmds, int n) {
   const uint64_t dw = f.ptr[2], dx = d.ptr[2];
   return apart(dx, x_of(d), f.ptr[0], x_of(f)) && apart(dx, x_of(d), f.ptr[1], y_of(f)) && apart(dx, x_of(d), dw, w_of(f)) && apart(dw, w_of(f), d.ptr[0], y_of(d)) &&
          apart(dw, w_of(f), d.ptr[1], w_of(d));
+}
+
+// Whether the gradient of a 2x2 / 2 pooling, with its Rectify's, stands behind the two commands of gh_gradient_pair, takes the
+// image gradient's result and lies apart from what the two touch: how many commands it is (float32 1: one command does both; float64
+// 2), or 0.
+int gh_unpool_follows(const gh_cmd* c, int n, gh_unpool* out) {
+  if (n < 3 || c[2].opcode != GH_OP_MAXPOOL2D_BWD) return 0;
+  const gh_cmd &f = c[0].opcode == GH_OP_CONV2D_BWD_FILTER ? c[0] : c[1], &d = c[0].opcode == GH_OP_CONV2D_BWD_FILTER ? c[1] : c[0], &p = c[2];
+  const bool wide = gh_dtype_of(d.flags) == GH_F64;
+  std::string m;
+  if (gh_dtype_of(p.flags) != gh_dtype_of(d.flags) || p.ptr[1] != d.ptr[2] || gh_validate_cmd(p, m)) return 0;
+  if ((p.flags & GH_FLAG_BN_REMADE) || !(p.flags & GH_FLAG_ACT_RELU) != wide) return 0;
+  if (p.dim[0] != d.dim[0] || p.dim[1] != d.dim[1] || p.dim[2] != 2 * d.dim[2] || p.dim[3] != 2 * d.dim[3]) return 0;
+  for (int i : {4, 5, 10, 11}) if (p.dim[i] != 2) return 0;
+  for (int i : {6, 7, 8, 9}) if (p.dim[i] != 0) return 0;
+  const int64_t item = wide ? 8 : 4, whole = p.dim[0] * p.dim[1] * p.dim[2] * p.dim[3] * item;
+  *out = {p.ptr[0], p.ptr[0], p.ptr[2], p.ptr[2], false};
+  if (wide) {
+    if (n < 4 || c[3].opcode != GH_OP_RELU_BWD || gh_dtype_of(c[3].flags) != GH_F64 || c[3].ptr[1] != p.ptr[2] || c[3].dim[0] * item != whole || gh_validate_cmd(c[3], m)) return 0;
+    out->z = c[3].ptr[0];
+    out->dz = c[3].ptr[2];
+    if (out->da != out->dz && !apart(out->da, whole, out->dz, whole)) return 0;
+  }
+  auto x_of = [&](const gh_cmd& k) { return k.dim[0] * k.dim[1] * k.dim[2] * k.dim[3] * item; };
+  auto w_of = [&](const gh_cmd& k) { return k.dim[4] * k.dim[1] * 9 * item; };
+  auto y_of = [&](const gh_cmd& k) {
+    return k.dim[0] * k.dim[4] * gh_conv_out(k.dim[2], 3, k.dim[7], k.dim[9], k.dim[11]) * gh_conv_out(k.dim[3], 3, k.dim[8], k.dim[10], k.dim[12]) * item;
+  };
+  for (uint64_t to : {out->da, out->dz}) {
+    if ((to & (uint64_t)(item - 1)) || !apart(to, whole, d.ptr[0], y_of(d)) || !apart(to, whole, d.ptr[1], w_of(d)) || !apart(to, whole, d.ptr[2], x_of(d)) ||
+        !apart(to, whole, f.ptr[0], x_of(f)) || !apart(to, whole, f.ptr[1], y_of(f)) || !apart(to, whole, f.ptr[2], w_of(f)))
+      return 0;
+    for (uint64_t from : {out->a, out->z})
+      if (!apart(to, whole, from, whole)) return 0;
+  }
+  for (uint64_t from : {out->a, out->z})
+    if ((from & (uint64_t)(item - 1)) || !apart(from, whole, d.ptr[2], x_of(d)) || !apart(from, whole, f.ptr[2], w_of(f))) return 0;
+  return wide ? 2 : 1;
 }

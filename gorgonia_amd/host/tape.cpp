@@ -1083,6 +1083,19 @@ Status TapeMachine::Compile() {
       before = i;
     }
   }
+  // The pooling's gradient behind a convolution's two (and the Rectify's behind it) may run in their launch, and then writes
+  // while they read: what dies with the two is kept until it is done.
+  if (!opt_.node_at_a_time)
+    for (int i = 0; i < N; i++) {
+      const Node& data = nodes[(size_t)i];
+      if (data.fused_away || data.op.kind != OpKind::Conv2dDiffData) continue;
+      int next = last_reader[(size_t)root[(size_t)i]];
+      if (next < 0 || nodes[(size_t)next].op.kind != OpKind::MaxPool2DDiff || nodes[(size_t)next].op.remade) continue;
+      const int behind = last_reader[(size_t)root[(size_t)next]];
+      if (behind > next && nodes[(size_t)behind].op.kind == OpKind::RectifyDiff) next = behind;
+      for (int& last : reg_last)
+        if (last >= i && last < next) last = next;
+    }
   // The convolutions and poolings behind an uploaded batch may run in pieces of it, for which their values have to lie apart:
   // what they read is kept until the last of them is done.
   if (!opt_.node_at_a_time)

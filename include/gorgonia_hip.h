@@ -422,6 +422,8 @@ enum gh_joint {
   /* a SoftMax with the scaled tensor and the SoftMax gradient behind it; form: 1 behind a SOFTMAX command, 2 in the product's
      kernel, 3 in the sum of the product's slabs */
   GH_JOINT_SOFTMAX_GRADIENT = 5,
+  /* a convolution's two gradients with the gradient of the pooling in front of it; form: GH_JOINT_CONV_GRADIENTS's */
+  GH_JOINT_UNPOOLED = 6,
   GH_JOINT__COUNT
 };
 GH_API int64_t gh_joint_launches(const gh_ctx* ctx, int kind, int64_t* form);
