@@ -119,6 +119,7 @@ struct gh_ctx {
   void* piece_words = nullptr;
   uint64_t piece_seq = 0;
   bool no_pieces = false;   // they were not to be had
+  bool beside_copy = false; // a piece's layers are submitted while the next one is copied; cu_count is without the copy's
   // pinned host buffers handed out by gh_host_alloc: [start, end)
   std::vector<std::pair<uint64_t, uint64_t>> host_ranges;
 };

@@ -3196,11 +3196,11 @@ static bool conv_sums_whole(const gh_cmd& c) {
   return plan_tiles(&probe, c.dim[4], c.dim[0] * gh_conv_out(c.dim[2], 3, c.dim[7], 1, 1) * gh_conv_out(c.dim[3], 3, c.dim[8], 1, 1), 9 * c.dim[1], 1, true).splits == 1;
 }
 // float32, behind the single-channel, few-channel and small-image kernels, which win where they take a shape.
-static int conv_lanes_form(const gh_cmd& c, int cus) {
+static int conv_lanes_form(const gh_cmd& c, int cus, bool as_pooled = true) {
   if (c.dim[5] != 3 || c.dim[6] != 3 || gh_conv_rows1_takes(c) || conv_direct_takes(c) || gh_conv_small_takes(c)) return -1;
   // gh_conv2d_can_pool answers without a device, so where only this kernel can pool (and sums as the plain command does) the choice
   // between the two is by the MI355X's compute units on every device.
-  if (cus != kUnits && gh_conv_patch_takes(c) && !gh_conv_patch_can_pool(c)) cus = kUnits;
+  if (as_pooled && cus != kUnits && gh_conv_patch_takes(c) && !gh_conv_patch_can_pool(c)) cus = kUnits;
   return gh_conv_lanes_form(c, false, cus, conv_others_us(c, cus), gh_conv_patch_takes(c), conv_sums_whole(c));
 }
 // The image gradient: elsewhere that is a launch that mirrors the filters (4.7 us) and a forward one over dy.
@@ -3278,7 +3278,7 @@ int gh_launch_conv2d(gh_ctx* ctx, const gh_cmd& c) {
   const int rcs = gh_try_launch_conv_small(ctx, c);
   if (rcs >= 0) return rcs;
   if (gh_conv_strip_takes(c) && gh_conv_wide_takes(c)) return gh_launch_conv_strip(ctx, c);
-  if (const int form = conv_lanes_form(c, ctx->cu_count); form >= 0) return gh_launch_conv_lanes(ctx, c, false, form);
+  if (const int form = conv_lanes_form(c, ctx->cu_count, !ctx->beside_copy || (c.flags & GH_FLAG_CONV_POOL2)); form >= 0) return gh_launch_conv_lanes(ctx, c, false, form);
   const int rcp = gh_try_launch_conv_patch(ctx, c);
   if (rcp >= 0) return rcp;
   const int rcw = gh_try_launch_conv_wide(ctx, c);
