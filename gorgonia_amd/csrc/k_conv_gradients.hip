@@ -18,8 +18,12 @@
 // Where the convolution's input was pooled (2x2 / 2, even extents), the pooling's gradient and its Rectify's, which take the image
 // gradient value by value, are in the launch as well (gh_unpool_follows): the windows are loaded under the meeting of the wavefronts
 // that share a tile's channels, and the pass over memory runs under the other workgroups' matrix instructions.  Only behind the
-// kernels whose wavefronts share the channels; the others store whole rows from registers.  A training step of the example's network,
-// two such layers: 128 images 184.9 / 181.2, 50 in float64 184.9 / 178.5.
+// kernels whose wavefronts share the channels; the others store whole rows from registers.  Bound: the matrix instructions, and the
+// stores of those workgroups that end last.  Beside a small-image filter gradient the image gradient's therefore stand in front where
+// there are more of both than begin at once (two to a compute unit): 128 x 32 x 14 x 14 -> 64 in two launches 25.4 + 7.2 us, in one
+// behind the filter gradient 33.3, in front 31.4; of 128 x 64 x 7 x 7 -> 128, 480 workgroups, 24.4 + 5.3, 25.8, 26.7; float64's are slower in
+// front (50 x 32 x 14 x 14 -> 64 27.8 / 34.1).  (The windows loaded in front of the channels: 35.8, with spilled registers.)
+// A training step of the example's network, two such layers: 128 images 181.0 / 176.2, 50 in float64 181.1 / 175.4, 13 images 132.9 / 128.0.
 //
 // gh_submit holds a filter gradient back (gh_held_filter) where an image gradient that has nothing to do with its result
 // stands beside it; the image gradient's launch takes it along, or it is launched by itself behind that.
@@ -50,9 +54,10 @@ struct Grid {
 
 template <int kRowPitch, int TM, bool kUnpool>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_conv3x3_gradients_small(const gh_wgrad_small_args w, const Grid grid, const Lanes<float> g,
-                                                                                                          const Unpool<float> u) {
+                                                                                                          const Unpool<float> u, const int front) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  const int b = (int)blockIdx.x;
+  int b = (int)blockIdx.x;
+  if (kUnpool && front) b = b < front ? b + grid.all : b - front;   // the image gradient's workgroups stand in front
   if (b < grid.all) {
     int bx, by, bz;
     grid.at(b, &bx, &by, &bz);
@@ -96,7 +101,8 @@ int go_small_as(gh_ctx* ctx, const Lanes<float>& g, int blocks) {
   gh_wgrad_small_args w;
   memcpy(&w, ctx->held.args, sizeof w);
   const size_t lds = std::max<size_t>(ctx->held.lds, conv_lanes::lds_of<float, 8, TM, 4, 1, true>(true));
-  hipLaunchKernelGGL((k_conv3x3_gradients_small<kRowPitch, TM, kUnpool>), dim3((unsigned)(grid.all + blocks)), dim3(512), lds, ctx->stream, w, grid, g, unpool_of<float>(ctx));
+  hipLaunchKernelGGL((k_conv3x3_gradients_small<kRowPitch, TM, kUnpool>), dim3((unsigned)(grid.all + blocks)), dim3(512), lds, ctx->stream, w, grid, g, unpool_of<float>(ctx),
+                     grid.all + blocks > 2 * ctx->cu_count ? blocks : 0);
   ctx->unpool.done = kUnpool;
   return GH_OK;
 }
