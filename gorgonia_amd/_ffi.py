@@ -121,7 +121,7 @@ SYMBOLS = {
 }
 
 # enum gh_joint
-JOINT_CONV_GRADIENTS, JOINT_DENSE_GRADIENTS, JOINT_SOLVER_SUMS, JOINT_CONV_ROUNDS, JOINT_PIECES, JOINT_SOFTMAX_GRADIENT, JOINT_UNPOOLED = range(7)
+JOINT_CONV_GRADIENTS, JOINT_DENSE_GRADIENTS, JOINT_SOLVER_SUMS, JOINT_CONV_ROUNDS, JOINT_PIECES, JOINT_SOFTMAX_GRADIENT, JOINT_UNPOOLED, JOINT_RECTIFIED = range(8)
 
 _lib = None
 

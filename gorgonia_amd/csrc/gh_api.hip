@@ -559,7 +559,18 @@ int gh_submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
     // and so with a dense layer's two gradients
     if (gh_gemm_gradient_pair(cmds + i, n - i)) {
       if ((rc = gh_flush_sums_before(ctx, cmds[i + 1]))) return rc;
-      if ((rc = gh_try_launch_gemm_gradients(ctx, cmds + i)) >= 0) {
+      const bool rectified = gh_rectify_gradient_follows(cmds + i, n - i);
+      if (rectified && (rc = gh_flush_sums_before(ctx, cmds[i + 2]))) return rc;
+      if ((rc = gh_try_launch_gemm_gradients(ctx, cmds + i, rectified)) >= 0) {
+        if (rc) return rc;
+        i += 1 + rectified;
+        continue;
+      }
+    }
+    // a product and its Rectify
+    if (gh_rectify_follows(cmds + i, n - i)) {
+      if ((rc = gh_flush_sums_before(ctx, cmds[i + 1]))) return rc;
+      if ((rc = gh_try_launch_gemm_rectify(ctx, cmds + i)) >= 0) {
         if (rc) return rc;
         i++;
         continue;

@@ -11,6 +11,21 @@
 // same bits: for v < 0 the reference's sum is -0 + v alpha = v alpha, for v >= 0 it is v + 0 = v,
 // and the v * 0 that fmaf adds is a zero of v's sign (which changes neither) unless v is
 // infinite or NaN, where it makes the NaN the reference's inf * 0 makes.
+// A Rectify behind a product (z null) or a Rectify's gradient (z: what it was taken of), value by value into `out`, a tensor of
+// the product's size and layout; where that is the product's own memory, the product is not stored.
+template <class T>
+struct gh_rectify_behind {
+  const T* z = nullptr;
+  T* out = nullptr;
+  // element `at`, in front of the stores: one by one they would wait for each other's loads (out may be what z was loaded from,
+  // for all that the compiler knows; 128 x 10 and 10 x 625 9.9 us so)
+  __device__ __forceinline__ T load(int64_t at) const { return z ? z[at] : (T)0; }
+  __device__ __forceinline__ void store(T* C, int64_t at, T v, T loaded) const {   // v: element `at` of the product C
+    if (out) out[at] = v * ((z ? loaded : v) >= (T)0 ? (T)1 : (T)0);
+    if (out != C) C[at] = v;
+  }
+};
+
 __device__ __forceinline__ float act_apply(float v, int act, float alpha) {
   if (act == 1) return v * (v >= 0.0f ? 1.0f : 0.0f);
   if (act == 3) {

@@ -124,8 +124,8 @@ template <class T, int kWaves, int TN, bool kSplitK>
 constexpr int lds_of() { return kSplitK ? kWaves * TN * 256 * (int)sizeof(T) : 16; }
 
 // Workgroup id of a grid of gx x gy tiles; bz: which product of a batch.
-template <class T, int kWaves, int TM, int TN, bool kSplitK, bool kTA, bool kTB>
-__device__ __forceinline__ void workgroup(const Gemm<T>& g, int id, int gx, int gy, int bz, char* lds) {
+template <class T, int kWaves, int TM, int TN, bool kSplitK, bool kTA, bool kTB, bool kBehind = false>
+__device__ __forceinline__ void workgroup(const Gemm<T>& g, int id, int gx, int gy, int bz, char* lds, const gh_rectify_behind<T>& behind = {}) {
   typedef typename Unit<T>::acc Acc;
   constexpr int KQ = Unit<T>::KQ, KC = 4 * KQ, kThreads = kWaves * 64;
   typedef Operand<T, TM, !kTA> OpA;
@@ -200,16 +200,22 @@ __device__ __forceinline__ void workgroup(const Gemm<T>& g, int id, int gx, int 
     multiply(even);
   }
 
-  auto store = [&](int r, int c, T sum) {
+  auto store = [&](int r, int c, T sum, T loaded) {
     if (r >= g.M || c >= g.N) return;
     if constexpr (sizeof(T) == 4) {
       if (g.bias) sum = sum + g.bias[c];
       sum = act_apply(sum, g.act, g.alpha);
     }
-    C[(int64_t)r * g.ldc + c] = sum;
+    if constexpr (kBehind) behind.store(C, (int64_t)r * g.ldc + c, sum, loaded);
+    else C[(int64_t)r * g.ldc + c] = sum;
+  };
+  auto load = [&](int r, int c) {
+    if constexpr (kBehind) return r < g.M && c < g.N ? behind.load((int64_t)r * g.ldc + c) : (T)0;
+    else return (T)0;
   };
   if constexpr (kSplitK) {
     T (* const red)[TN * 256] = (T (*)[TN * 256])lds;
+    constexpr int kRounds = (TN * 256 + kThreads - 1) / kThreads;
 #pragma unroll
     for (int a = 0; a < TM; a++) {
       if (a) __syncthreads();
@@ -217,23 +223,39 @@ __device__ __forceinline__ void workgroup(const Gemm<T>& g, int id, int gx, int 
       for (int b = 0; b < TN; b++)
 #pragma unroll
         for (int v = 0; v < 4; v++) red[wave][b * 256 + v * 64 + lane] = acc[a][b][v];
+      auto row = [&](int e) { return OpA::row(a, Unit<T>::row((e & 63) >> 4, (e >> 6) & 3), m0, g.M); };
+      auto col = [&](int e) { return OpB::row(e >> 8, e & 15, n0, g.N); };
+      T loaded[kRounds];
+#pragma unroll
+      for (int k = 0; k < kRounds; k++) {
+        const int e = (int)threadIdx.x + k * kThreads;
+        loaded[k] = e < TN * 256 ? load(row(e), col(e)) : (T)0;
+      }
       __syncthreads();
 #pragma unroll
-      for (int e = threadIdx.x; e < TN * 256; e += kThreads) {
+      for (int k = 0; k < kRounds; k++) {
+        const int e = (int)threadIdx.x + k * kThreads;
+        if (e >= TN * 256) break;
         T sum = red[0][e];
 #pragma unroll
         for (int w = 1; w < kWaves; w++) sum = sum + red[w][e];
-        const int l = e & 63, v = (e >> 6) & 3, b = e >> 8;
-        store(OpA::row(a, Unit<T>::row(l >> 4, v), m0, g.M), OpB::row(b, l & 15, n0, g.N), sum);
+        store(row(e), col(e), sum, loaded[k]);
       }
     }
   } else {
+    T loaded[TM][TN][4];
 #pragma unroll
     for (int a = 0; a < TM; a++)
 #pragma unroll
       for (int b = 0; b < TN; b++)
 #pragma unroll
-        for (int v = 0; v < 4; v++) store(OpA::row(a, Unit<T>::row(q, v), m0, g.M), OpB::row(b, i, n0, g.N), acc[a][b][v]);
+        for (int v = 0; v < 4; v++) loaded[a][b][v] = load(OpA::row(a, Unit<T>::row(q, v), m0, g.M), OpB::row(b, i, n0, g.N));
+#pragma unroll
+    for (int a = 0; a < TM; a++)
+#pragma unroll
+      for (int b = 0; b < TN; b++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) store(OpA::row(a, Unit<T>::row(q, v), m0, g.M), OpB::row(b, i, n0, g.N), acc[a][b][v], loaded[a][b][v]);
   }
 }
 

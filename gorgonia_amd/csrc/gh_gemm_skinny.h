@@ -79,9 +79,9 @@ inline Args64 args64_of(const gh_cmd& c) {
 template <int WV, int NT>
 constexpr int lds16() { return WV * 16 * 16 * NT * 4; }
 
-template <int WV, int NT, bool TA, bool TB, bool kPlain, bool kGradient = false>
+template <int WV, int NT, bool TA, bool TB, bool kPlain, bool kGradient = false, bool kBehind = false>
 __device__ __forceinline__ void workgroup16(const Args32& g, int id, int gx, int gy, int bz, int slices, char* lds,
-                                            const gh_softmax_gradient<float>& t = {}) {
+                                            const gh_softmax_gradient<float>& t = {}, const gh_rectify_behind<float>& behind = {}) {
   const int M = g.M, N = g.N, K = g.K, lda = g.lda, ldb = g.ldb, ldc = g.ldc, act = g.act, softmax = kPlain ? 0 : kGradient ? 1 : g.softmax;
   const float alpha = g.alpha;
   const float *__restrict__ const A = g.A, *__restrict__ const B = g.B, *__restrict__ const bias = kPlain ? nullptr : g.bias;
@@ -242,14 +242,28 @@ __device__ __forceinline__ void workgroup16(const Args32& g, int id, int gx, int
     }
     return;
   }
-  for (int e = threadIdx.x; e < TILE; e += WV * 64) {
+  constexpr int kRounds = (TILE + WV * 64 - 1) / (WV * 64);
+  [[maybe_unused]] float loaded[kRounds];
+  if constexpr (kBehind) {
+#pragma unroll
+    for (int k = 0; k < kRounds; k++) {
+      const int e = (int)threadIdx.x + k * WV * 64, col = n0 + e % BN;
+      loaded[k] = e < TILE && col < N ? behind.load((int64_t)(m0 + e / BN) * ldc + col) : 0.0f;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kRounds; k++) {
+    const int e = (int)threadIdx.x + k * WV * 64;
+    if (e >= TILE) break;
     float sum = part[e];
 #pragma unroll
     for (int w = 1; w < WV; w++) sum = sum + part[w * TILE + e];
     const int col = n0 + e % BN;
     if (col >= N) continue;
     if (bias) sum = sum + bias[col];
-    C[(int64_t)(m0 + e / BN) * ldc + col] = act_apply(sum, act, alpha);
+    const int64_t at = (int64_t)(m0 + e / BN) * ldc + col;
+    if constexpr (kBehind) behind.store(C, at, act_apply(sum, act, alpha), loaded[k]);
+    else C[at] = act_apply(sum, act, alpha);
   }
 }
 
@@ -266,8 +280,8 @@ __device__ __forceinline__ void workgroup16(const Args32& g, int id, int gx, int
 template <int WV>
 constexpr int lds64() { return WV * 256 * 8; }
 
-template <int WV, bool AV, bool BV>
-__device__ __forceinline__ void workgroup64(const Args64& g, int bx, int by, int bz, char* lds) {
+template <int WV, bool AV, bool BV, bool kBehind = false>
+__device__ __forceinline__ void workgroup64(const Args64& g, int bx, int by, int bz, char* lds, const gh_rectify_behind<double>& behind = {}) {
   const double* __restrict__ const A = g.A + bz * g.sA;
   const double* __restrict__ const B = g.B + bz * g.sB;
   double* __restrict__ const C = g.C + bz * g.sC;
@@ -340,12 +354,22 @@ __device__ __forceinline__ void workgroup64(const Args64& g, int bx, int by, int
   for (int v = 0; v < 4; v++) part[wave][v * 64 + lane] = acc[v];
   __syncthreads();
   if (wave == 0) {
+    [[maybe_unused]] double loaded[4];
+    if constexpr (kBehind) {
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int i = m0 + 4 * v + lk, j = n0 + lr;
+        loaded[v] = i < M && j < N ? behind.load((int64_t)i * ldc + j) : 0.0;
+      }
+    }
 #pragma unroll
     for (int v = 0; v < 4; v++) {
       double sum = part[0][v * 64 + lane];
       for (int w = 1; w < WV; w++) sum = sum + part[w][v * 64 + lane];
       const int i = m0 + 4 * v + lk, j = n0 + lr;
-      if (i < M && j < N) C[(int64_t)i * ldc + j] = sum;
+      if (i >= M || j >= N) continue;
+      if constexpr (kBehind) behind.store(C, (int64_t)i * ldc + j, sum, loaded[v]);
+      else C[(int64_t)i * ldc + j] = sum;
     }
   }
 }

@@ -168,6 +168,9 @@ bool gh_is_pair(const gh_cmd* cmds, int n);
 // a SoftMax, the tensor times a scalar behind it and the SoftMax gradient that takes both (k_pairs.hip, k_gemm.hip): what is
 // behind the SoftMax's own values, row by row
 template <class T> struct gh_softmax_gradient { const T* x; const T* s; T* g; T* dx; };
+// a product and the Rectify behind it (k_gemm.hip)
+bool gh_rectify_follows(const gh_cmd* cmds, int n);
+int gh_try_launch_gemm_rectify(gh_ctx* ctx, const gh_cmd* cmds);   // -1: no kernel has both
 bool gh_softmax_gradient_follows(const gh_cmd* cmds, int n);
 int gh_try_launch_softmax_gradient(gh_ctx* ctx, const gh_cmd* cmds);        // of a SOFTMAX; -1: no kernel has the three
 int gh_try_launch_gemm_softmax_gradient(gh_ctx* ctx, const gh_cmd* cmds);   // of a GEMM with its SoftMax
@@ -200,7 +203,9 @@ enum { kGemmOther, kGemmDirect, kGemmSkinny };
 struct gh_gemm_choice { int kind = kGemmOther, form = 0, waves = 0, columns = 0; };   // form: k_gemm_direct's; waves, columns: the small-output kernels'; waves: k_gemm_direct's that share K, of float64 0 for four
 gh_gemm_choice gh_choose_gemm(const gh_ctx* ctx, const gh_cmd& c);
 bool gh_gemm_gradient_pair(const gh_cmd* cmds, int n);
-int gh_try_launch_gemm_gradients(gh_ctx* ctx, const gh_cmd* cmds);   // -1: no kernel has both
+// (`rectified`: cmds[2] is a Rectify's gradient and rides along)
+bool gh_rectify_gradient_follows(const gh_cmd* cmds, int n);
+int gh_try_launch_gemm_gradients(gh_ctx* ctx, const gh_cmd* cmds, bool rectified);   // -1: no kernel has both
 // float32 products on the bf16 matrix instructions (k_gemm_split.hip)
 int gh_gemm_split_form(const gh_cmd& c, int cus, double other_us, int other_slices);   // -1: not taken; the other kernel's time and its slices of K
 int gh_launch_gemm_split(gh_ctx* ctx, const gh_cmd& c, int form);

@@ -424,6 +424,9 @@ enum gh_joint {
   GH_JOINT_SOFTMAX_GRADIENT = 5,
   /* a convolution's two gradients with the gradient of the pooling in front of it; form: GH_JOINT_CONV_GRADIENTS's */
   GH_JOINT_UNPOOLED = 6,
+  /* a product and the Rectify of it, both stored; form: 10 * the tiles of 16 columns + the wavefronts, float64 100 + the wavefronts,
+     and a dense layer's gradients with the Rectify's gradient behind them; form 0 */
+  GH_JOINT_RECTIFIED = 7,
   GH_JOINT__COUNT
 };
 GH_API int64_t gh_joint_launches(const gh_ctx* ctx, int kind, int64_t* form);
