@@ -1084,17 +1084,21 @@ Status TapeMachine::Compile() {
     }
   }
   // The pooling's gradient behind a convolution's two (and the Rectify's behind it) may run in their launch, and then writes
-  // while they read: what dies with the two is kept until it is done.
+  // while they read: its memory is taken before what dies with the two is given back.
+  std::vector<std::vector<int>> early((size_t)N);
+  std::vector<char> is_early((size_t)N, 0);
   if (!opt_.node_at_a_time)
     for (int i = 0; i < N; i++) {
       const Node& data = nodes[(size_t)i];
       if (data.fused_away || data.op.kind != OpKind::Conv2dDiffData) continue;
-      int next = last_reader[(size_t)root[(size_t)i]];
+      const int next = last_reader[(size_t)root[(size_t)i]];
       if (next < 0 || nodes[(size_t)next].op.kind != OpKind::MaxPool2DDiff || nodes[(size_t)next].op.remade) continue;
       const int behind = last_reader[(size_t)root[(size_t)next]];
-      if (behind > next && nodes[(size_t)behind].op.kind == OpKind::RectifyDiff) next = behind;
-      for (int& last : reg_last)
-        if (last >= i && last < next) last = next;
+      for (int j : {next, behind > next && nodes[(size_t)behind].op.kind == OpKind::RectifyDiff ? behind : next})
+        if (!inplace[(size_t)j] && !is_early[(size_t)j] && nodes[(size_t)j].alias_of < 0 && !nodes[(size_t)j].read_into) {
+          is_early[(size_t)j] = 1;
+          early[(size_t)i].push_back(j);
+        }
     }
   // The convolutions and poolings behind an uploaded batch may run in pieces of it, for which their values have to lie apart:
   // what they read is kept until the last of them is done.
@@ -1175,10 +1179,17 @@ Status TapeMachine::Compile() {
     } else {
       if (host_out[(size_t)i]) {
         prog_.push_back({InstrKind::AllocHost, i, r, bytes, false});
-      } else if (!inplace[(size_t)i]) {
+      } else if (!inplace[(size_t)i] && !is_early[(size_t)i]) {
         prog_.push_back({InstrKind::Alloc, i, r, bytes, false});
         reg_bytes[(size_t)r] = bytes;
         gpumem_ += bytes;
+      }
+      for (int j : early[(size_t)i]) {
+        const int rj = node_reg_[(size_t)j];
+        const int64_t bj = bytes_of(nodes[(size_t)j]);
+        prog_.push_back({InstrKind::Alloc, j, rj, bj, false});
+        reg_bytes[(size_t)rj] = bj;
+        gpumem_ += bj;
       }
       if (!n.deferred) prog_.push_back({InstrKind::ExecOp, i, r, bytes, inplace[(size_t)i] != 0});
     }
