@@ -666,9 +666,9 @@ int gh_submit_noalloc(gh_ctx* ctx, const gh_cmd* cmds, int n) {
 // How long gh_sync polls its word before it leaves the wait to the runtime (and the core to others).
 static constexpr auto kPollFor = std::chrono::microseconds(2000);
 // The runtime frees what it keeps per launch when it is asked to wait: every so many waits it is.  At
-// every 256th the allocations of a new tape machine paid for the backlog (3.6 -> 5.2 ms for 37 tensors);
-// at every 32nd they do not, and the 3 us more of one wait in 32 cannot be told from noise.
-static constexpr uint32_t kRuntimeWaitEvery = 32;
+// every 32nd the allocations of a new tape machine paid for the backlog (3.6 -> 5 to 6.8 ms for 37 tensors);
+// at every 16th they do not, and the 3 us more of one wait in 16 cannot be told from noise.
+static constexpr uint32_t kRuntimeWaitEvery = 16;
 
 // The completion word of gh_sync.  What the kernels in front have stored is visible to this one when it begins, and its release
 // takes that along to the host: results lie in coherent pinned memory, which no cache of the device holds back.  Bound: a
