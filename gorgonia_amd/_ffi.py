@@ -100,6 +100,7 @@ SYMBOLS = {
     "gh_bn_can_remake": (C.c_int, [C.c_int64] * 4),
     "gh_conv2d_route": (C.c_int, [C.POINTER(GhCmd)]),
     "gh_conv2d_bwd_filter_route": (C.c_int, [C.POINTER(GhCmd)]),
+    "gh_pieces_layers": (C.c_int, [C.POINTER(GhCmd), C.c_int]),
     "gh_gemm_route": (C.c_int, [C.POINTER(GhCmd), C.POINTER(C.c_int)]),
     "gh_runs_straight": (C.c_int, [C.POINTER(GhCmd)]),
     "gh_runs_split": (C.c_int, [C.POINTER(GhCmd)]),

@@ -129,17 +129,19 @@ bool by_image(const gh_cmd& c, Layer* l) {
 }
 
 // The layers behind the upload that run in pieces: as many as take, whole, about half of the upload's time (8 x 3 x 416 x 416:
-// three layers 643 us, four 626, with the fifth 664), each reads what the one in front wrote, nothing else of what they
-// read and write lies together, and the kernels take their shapes with a piece's images, too.
-int head_of(const gh_ctx* ctx, const gh_cmd* cmds, int n, int64_t fewest, int64_t most, Layer* layers) {
+// three layers 643 us, four 626, with the fifth 664), each reads what the one in front wrote, and the kernels take their shapes
+// with a piece's images, too.  A layer's work on the first piece comes before the work of those in front of it on the last: what it
+// writes lies apart from all that they read and write, their filters and constants among it.
+template <class InHost>
+int head_of(const gh_cmd* cmds, int n, int64_t fewest, int64_t most, Layer* layers, InHost&& in_host) {
   const gh_cmd& up = cmds[0];
   const int64_t B = cmds[1].dim[0];
   std::string m;
-  Span spans[kHead + 1];
+  Span values[kHead + 1], constants[5 * kHead];
   uint64_t from = up.ptr[0];
-  spans[0] = Span{from, from + (uint64_t)up.dim[0]};
+  values[0] = Span{from, from + (uint64_t)up.dim[0]};
   double us = 0;
-  int head = 0;
+  int head = 0, held = 0;
   for (; head < kHead && head + 1 < n; head++) {
     const gh_cmd& c = cmds[head + 1];
     Layer& l = layers[head];
@@ -147,14 +149,16 @@ int head_of(const gh_ctx* ctx, const gh_cmd* cmds, int n, int64_t fewest, int64_
     if (head == 0 && B * l.in_bytes != up.dim[0]) break;
     if ((us += l.us) > 0.55 * (double)up.dim[0] / 56e3) break;
     from = c.ptr[l.out];
-    spans[head + 1] = Span{from, from + (uint64_t)(B * l.out_bytes)};
-    bool fits = !gh_in_pinned_host(ctx, from);
-    for (int k = 0; k <= head; k++) fits = fits && !meet(spans[k], spans[head + 1]);
+    values[head + 1] = Span{from, from + (uint64_t)(B * l.out_bytes)};
     if (c.opcode == GH_OP_CONV2D)
       for (int k : {1, 3, 4, 5, 6}) {
         const int64_t bytes = (k == 1 ? c.dim[1] * c.dim[4] * c.dim[5] * c.dim[6] : c.dim[4]) * 4;
-        for (int s = 0; s <= head + 1; s++) fits = fits && !(c.ptr[k] && meet(spans[s], Span{c.ptr[k], c.ptr[k] + (uint64_t)bytes}));
+        if (c.ptr[k]) constants[held++] = Span{c.ptr[k], c.ptr[k] + (uint64_t)bytes};
       }
+    bool fits = !in_host(from);
+    for (int k = 0; k <= head; k++) fits = fits && !meet(values[k], values[head + 1]);
+    for (int k = 0; k < held; k++)
+      for (int s = 0; s <= head + 1; s++) fits = fits && !meet(values[s], constants[k]);
     for (int64_t images : {fewest, most}) {
       gh_cmd part = c;
       part.dim[0] = images;
@@ -163,6 +167,23 @@ int head_of(const gh_ctx* ctx, const gh_cmd* cmds, int n, int64_t fewest, int64_
     if (!fits) break;
   }
   return head;
+}
+
+// How many pieces the commands' batch would be in, 0 where it goes whole.
+int pieces_of(const gh_cmd* cmds, int n) {
+  if (n < 2) return 0;
+  const gh_cmd& up = cmds[0];
+  const int64_t bytes = up.dim[0], B = cmds[1].dim[0];
+  if (up.opcode != GH_OP_MEMCPY_D2D || bytes < kLeast || bytes > kMost || bytes % 4 || B < 2 || ((up.ptr[0] | up.ptr[1]) & 15)) return 0;
+  std::string m;
+  if (gh_validate_cmd(up, m)) return 0;
+  return (int)std::min({B, (int64_t)kPieces, std::max<int64_t>(2, (bytes + kPieceBytes - 1) / kPieceBytes)});
+}
+
+template <class InHost>
+int layers_of(const gh_cmd* cmds, int n, int pieces, Layer* layers, InHost&& in_host) {
+  const int64_t B = cmds[1].dim[0];
+  return head_of(cmds, n, B / pieces, (B + pieces - 1) / pieces, layers, in_host);
 }
 
 // Streams share a few hardware queues, and two of one queue run one behind the other (a batch of 8 then takes 740 us).  Which
@@ -228,18 +249,22 @@ void gh_drop_pieces(gh_ctx* ctx) {
   ctx->piece_words = nullptr;
 }
 
+extern "C" int gh_pieces_layers(const gh_cmd* cmds, int n) {
+  const int pieces = cmds ? pieces_of(cmds, n) : 0;
+  Layer layers[kHead];
+  return pieces ? layers_of(cmds, n, pieces, layers, [](uint64_t) { return false; }) : 0;
+}
+
 int gh_submit_pieces(gh_ctx* ctx, const gh_cmd* cmds, int n, int* rc) {
-  if (n < 2 || ctx->capturing || ctx->ws_strict) return 0;
+  if (ctx->capturing || ctx->ws_strict) return 0;
+  const int pieces = pieces_of(cmds, n);
+  if (!pieces) return 0;
   const gh_cmd& up = cmds[0];
   const int64_t bytes = up.dim[0], B = cmds[1].dim[0];
-  if (up.opcode != GH_OP_MEMCPY_D2D || bytes < kLeast || bytes > kMost || bytes % 4 || B < 2 || ((up.ptr[0] | up.ptr[1]) & 15)) return 0;
   if (!gh_in_pinned_host(ctx, up.ptr[1]) || !gh_in_pinned_host(ctx, up.ptr[1] + (uint64_t)bytes - 1) || gh_in_pinned_host(ctx, up.ptr[0])) return 0;
   if (getenv("GORGONIA_HIP_NO_PIECES")) return 0;   // tuning switch: the upload first
-  std::string m;
-  if (gh_validate_cmd(up, m)) return 0;
-  const int pieces = (int)std::min({B, (int64_t)kPieces, std::max<int64_t>(2, (bytes + kPieceBytes - 1) / kPieceBytes)});
   Layer layers[kHead];
-  const int head = head_of(ctx, cmds, n, B / pieces, (B + pieces - 1) / pieces, layers);
+  const int head = layers_of(cmds, n, pieces, layers, [&](uint64_t p) { return gh_in_pinned_host(ctx, p); });
   bool fresh = false;
   if (head == 0 || !ready(ctx, &fresh)) return 0;
   hipError_t e = hipSuccess;

@@ -290,7 +290,6 @@ GH_API int gh_memcpy_d2d(gh_ctx* ctx, gh_devptr dst, gh_devptr src, int64_t byte
 /* src (any host memory) to dst by way of `stage` (memory of gh_host_alloc, `bytes` of it): the bus moves what has been
  * copied while the host copies the rest.  Returns when src has been read; `stage` must stay untouched until the next
  * gh_sync(). */
-#define GH_PIECES_FROM 4000000 /* gh_submit: below, a batch is copied whole and the layers behind it follow (GH_JOINT_PIECES) */
 #define GH_STAGED_FROM (128 << 10) /* below, one copy after the other */
 GH_API int gh_memcpy_staged(gh_ctx* ctx, gh_devptr dst, void* stage, const void* src, int64_t bytes);
 
@@ -400,6 +399,11 @@ GH_API int gh_runs_straight(const gh_cmd* cmd);
  * values split into three bf16 parts each (k_gemm_split); the queries above then name the kernel of the float32
  * instructions that it would run on otherwise.  Host only; 256 compute units, as above. */
 GH_API int gh_runs_split(const gh_cmd* cmd);
+
+/* How many of the commands behind cmds[0], the copy of a batch, gh_submit runs in pieces of it (GH_JOINT_PIECES), for a copy out
+ * of memory of gh_host_alloc and results in device memory.  Host only; 256 compute units, as above. */
+#define GH_PIECES_FROM 4000000 /* bytes: below, a batch is copied whole and the layers behind it follow */
+GH_API int gh_pieces_layers(const gh_cmd* cmds, int n);
 
 /* How many launches of the context's have run the work of several commands together, of one of these kinds, and in *form (may be
  * null) which kernel the last of them was; -1 for another kind.  A launch that a graph records counts once.  Host only. */
