@@ -129,7 +129,7 @@ bool by_image(const gh_cmd& c, Layer* l) {
 }
 
 // The layers behind the upload that run in pieces: as many as take, whole, about half of the upload's time (8 x 3 x 416 x 416:
-// three layers 643 us, four 626, with the fifth 664), each reads what the one in front wrote, and the kernels take their shapes
+// three layers 643 us, four 626, with the fifth 664), each reads what the one in front wrote, image by image, and the kernels take their shapes
 // with a piece's images, too.  A layer's work on the first piece comes before the work of those in front of it on the last: what it
 // writes lies apart from all that they read and write, their filters and constants among it.
 template <class InHost>
@@ -146,7 +146,7 @@ int head_of(const gh_cmd* cmds, int n, int64_t fewest, int64_t most, Layer* laye
     const gh_cmd& c = cmds[head + 1];
     Layer& l = layers[head];
     if (c.dim[0] != B || gh_validate_cmd(c, m) || !by_image(c, &l) || c.ptr[0] != from) break;
-    if (head == 0 && B * l.in_bytes != up.dim[0]) break;
+    if (head == 0 ? B * l.in_bytes != up.dim[0] : l.in_bytes != layers[head - 1].out_bytes) break;
     if ((us += l.us) > 0.55 * (double)up.dim[0] / 56e3) break;
     from = c.ptr[l.out];
     values[head + 1] = Span{from, from + (uint64_t)(B * l.out_bytes)};

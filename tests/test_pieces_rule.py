@@ -53,3 +53,11 @@ def test_a_result_over_constants(constant):
         conv = D.cmd_conv2d(x, w, y, B, 3, H, W, 16, 3, 3, (1, 1), bn=[bn + 64 * k for k in range(3, 7)])
         return [D.cmd_copy(x, _at(9), BATCH), conv, D.cmd_maxpool2d(y, out, B, 16, H, W, 2, 2, (0, 0, 0, 0), (2, 2))]
     assert _layers(cmds(z)) == 2 and _layers(cmds(bn + 64 * constant + 60)) == 1
+
+
+# the pooled values read as images of more and of fewer values than were written for one, in a command that is valid by itself
+@pytest.mark.parametrize("channels,layers", [(16, 3), (17, 2), (15, 2), (8, 2), (32, 2)])
+def test_images_of_another_size(channels, layers):
+    cmds = _net()
+    cmds[3] = D.cmd_maxpool2d(_at(3), _at(4), B, channels, 112, 112, 2, 2, (0, 0, 0, 0), (2, 2))
+    assert _layers(cmds) == layers
