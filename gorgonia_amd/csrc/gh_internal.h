@@ -119,7 +119,9 @@ struct gh_ctx {
   void* piece_words = nullptr;
   uint64_t piece_seq = 0;
   bool no_pieces = false;   // they were not to be had
-  bool beside_copy = false; // a piece's layers are submitted while the next one is copied; cu_count is without the copy's
+  // while a piece's layers are submitted: the images of the whole batch and the compute units that it would be planned for
+  int64_t whole_images = 0;
+  int whole_units = 0;
   // pinned host buffers handed out by gh_host_alloc: [start, end)
   std::vector<std::pair<uint64_t, uint64_t>> host_ranges;
 };
@@ -215,6 +217,7 @@ int gh_launch_gemm_thin(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_gemv(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_outer(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_conv2d(gh_ctx* ctx, const gh_cmd& c);
+bool gh_conv2d_in_pieces(const gh_cmd& c, int64_t images, int units, int part_units);
 // small-image 3x3 convolution (k_conv_small.hip): -1 when the shape is not one it takes
 int gh_try_launch_conv_small(gh_ctx* ctx, const gh_cmd& c);
 int gh_try_launch_conv_wgrad_small(gh_ctx* ctx, const gh_cmd& c, int* splits, float** slabs);
@@ -258,6 +261,7 @@ bool gh_conv_strip_takes(const gh_cmd& c);
 int gh_launch_conv_strip(gh_ctx* ctx, const gh_cmd& c);
 // 3x3 stride-1 convolution with operands straight from memory, both float types; flip: of an image-gradient command (k_conv_lanes.hip)
 int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, bool patch = false, bool whole = false);   // -1: not taken; the other: k_conv3x3_patch, one whose sums run over all channels
+int gh_conv_lanes_form_like(const gh_cmd& c, int form, int cus);
 int gh_launch_conv_lanes(gh_ctx* ctx, const gh_cmd& c, bool flip, int form);
 int gh_launch_maxpool2d(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_bn_infer(gh_ctx* ctx, const gh_cmd& c);

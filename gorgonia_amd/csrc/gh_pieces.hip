@@ -98,6 +98,9 @@ __global__ __launch_bounds__(kThreads) void k_await_piece(void* dst, const u32x4
 __global__ void k_clear_words(Words* words) { ((unsigned long long*)words)[threadIdx.x] = 0; }
 constexpr int kWordCount = sizeof(Words) / 8;
 
+// the compute units that layers beside the copy are planned for
+int units_beside(int units) { return std::max(1, units - kCopiers); }
+
 struct Span { uint64_t lo, hi; };
 bool meet(const Span& a, const Span& b) { return a.lo < b.hi && b.lo < a.hi; }
 
@@ -129,11 +132,12 @@ bool by_image(const gh_cmd& c, Layer* l) {
 }
 
 // The layers behind the upload that run in pieces: as many as take, whole, about half of the upload's time (8 x 3 x 416 x 416:
-// three layers 643 us, four 626, with the fifth 664), each reads what the one in front wrote, image by image, and the kernels take their shapes
-// with a piece's images, too.  A layer's work on the first piece comes before the work of those in front of it on the last: what it
+// three layers 645 us, with the fourth and its pooling 632), each reads what the one in front wrote, image by image, and the kernels take their shapes
+// with a piece's images, too, and add there as they do for the whole batch: whether a batch goes in pieces (eagerly) or whole (under
+// capture) changes no bits.  A layer's work on the first piece comes before the work of those in front of it on the last: what it
 // writes lies apart from all that they read and write, their filters and constants among it.
 template <class InHost>
-int head_of(const gh_cmd* cmds, int n, int64_t fewest, int64_t most, Layer* layers, InHost&& in_host) {
+int head_of(const gh_cmd* cmds, int n, int64_t fewest, int64_t most, Layer* layers, int units, InHost&& in_host) {
   const gh_cmd& up = cmds[0];
   const int64_t B = cmds[1].dim[0];
   std::string m;
@@ -163,6 +167,8 @@ int head_of(const gh_cmd* cmds, int n, int64_t fewest, int64_t most, Layer* laye
       gh_cmd part = c;
       part.dim[0] = images;
       fits = fits && gh_validate_cmd(part, m) == GH_OK;
+      if (c.opcode == GH_OP_CONV2D)
+        for (int u : {units, units_beside(units)}) fits = fits && gh_conv2d_in_pieces(c, images, units, u);
     }
     if (!fits) break;
   }
@@ -181,9 +187,9 @@ int pieces_of(const gh_cmd* cmds, int n) {
 }
 
 template <class InHost>
-int layers_of(const gh_cmd* cmds, int n, int pieces, Layer* layers, InHost&& in_host) {
+int layers_of(const gh_cmd* cmds, int n, int pieces, Layer* layers, int units, InHost&& in_host) {
   const int64_t B = cmds[1].dim[0];
-  return head_of(cmds, n, B / pieces, (B + pieces - 1) / pieces, layers, in_host);
+  return head_of(cmds, n, B / pieces, (B + pieces - 1) / pieces, layers, units, in_host);
 }
 
 // Streams share a few hardware queues, and two of one queue run one behind the other (a batch of 8 then takes 740 us).  Which
@@ -252,7 +258,7 @@ void gh_drop_pieces(gh_ctx* ctx) {
 extern "C" int gh_pieces_layers(const gh_cmd* cmds, int n) {
   const int pieces = cmds ? pieces_of(cmds, n) : 0;
   Layer layers[kHead];
-  return pieces ? layers_of(cmds, n, pieces, layers, [](uint64_t) { return false; }) : 0;
+  return pieces ? layers_of(cmds, n, pieces, layers, kUnits, [](uint64_t) { return false; }) : 0;
 }
 
 int gh_submit_pieces(gh_ctx* ctx, const gh_cmd* cmds, int n, int* rc) {
@@ -264,7 +270,7 @@ int gh_submit_pieces(gh_ctx* ctx, const gh_cmd* cmds, int n, int* rc) {
   if (!gh_in_pinned_host(ctx, up.ptr[1]) || !gh_in_pinned_host(ctx, up.ptr[1] + (uint64_t)bytes - 1) || gh_in_pinned_host(ctx, up.ptr[0])) return 0;
   if (getenv("GORGONIA_HIP_NO_PIECES")) return 0;   // tuning switch: the upload first
   Layer layers[kHead];
-  const int head = layers_of(cmds, n, pieces, layers, [&](uint64_t p) { return gh_in_pinned_host(ctx, p); });
+  const int head = layers_of(cmds, n, pieces, layers, ctx->cu_count, [&](uint64_t p) { return gh_in_pinned_host(ctx, p); });
   bool fresh = false;
   if (head == 0 || !ready(ctx, &fresh)) return 0;
   hipError_t e = hipSuccess;
@@ -304,12 +310,12 @@ int gh_submit_pieces(gh_ctx* ctx, const gh_cmd* cmds, int n, int* rc) {
     // The copy has kCopiers compute units, so a kernel of one workgroup to each of the device's would run in two rounds: while
     // it is under way the layers are planned without them (8 x 3 x 416 x 416 615 / 599 us, of which a 64 -> 128 convolution of
     // 256 workgroups on two images 28 / 16).
-    const int units = ctx->cu_count;
-    ctx->beside_copy = p + 1 < pieces;
-    if (ctx->beside_copy) ctx->cu_count = std::max(1, units - kCopiers);
+    ctx->whole_images = B;
+    ctx->whole_units = ctx->cu_count;
+    if (p + 1 < pieces) ctx->cu_count = units_beside(ctx->cu_count);
     *rc = gh_submit_each(ctx, part, head);
-    ctx->cu_count = units;
-    ctx->beside_copy = false;
+    ctx->cu_count = ctx->whole_units;
+    ctx->whole_images = 0;
   }
   if (e != hipSuccess && !*rc) *rc = gh_check_hip(ctx, e, "upload in pieces");
   if (*rc) (void)hipStreamSynchronize(ctx->pieces);   // nothing of it is under way behind an error

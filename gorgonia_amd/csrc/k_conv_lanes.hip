@@ -195,6 +195,13 @@ int gh_conv_lanes_form(const gh_cmd& c, bool flip, int cus, double other_us, boo
   return us < other_us / 1.1 ? form : -1;
 }
 
+// The quickest for a float32 forward command of the forms that add as `form` does: eight wavefronts' shares of the channels, four's, or
+// all channels in one chain.
+int gh_conv_lanes_form_like(const gh_cmd& c, int form, int cus) {
+  double us;
+  return form < 2 ? quickest(c, false, false, cus, 0, 2, &us) : form == 2 ? form : quickest(c, false, false, cus, 3, 5, &us);
+}
+
 int gh_launch_conv_lanes(gh_ctx* ctx, const gh_cmd& c, bool flip, int form) {
   const bool pool = !flip && (c.flags & GH_FLAG_CONV_POOL2);
   if (gh_dtype_of(c.flags) == GH_F64) {

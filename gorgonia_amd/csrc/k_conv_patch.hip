@@ -27,6 +27,7 @@
 //   * With GH_FLAG_CONV_POOL2 the patch has even extents and the N axis enumerates
 //     (pooled pixel, position in the 2x2 window); the epilogue reads a window as four
 //     adjacent columns (scan order and strict > of the pooling kernel, op_nn.go:860-907).
+#include <algorithm>
 #include <cstdlib>
 #include <mutex>
 
@@ -413,6 +414,24 @@ struct PatchPlan {
   size_t lds;
 };
 
+// Gives the plan's workgroups 16 tm filters each; whether their LDS fits.
+bool set_filters(PatchPlan* p, int tm) {
+  PatchGeom& g = p->g;
+  const size_t quad = p->two ? 2 * (tm == 1 ? quad_floats<1>() : quad_floats<2>()) : 36 * 16 * tm + 4 * g.PL;
+  const size_t stage = ((size_t)kWaves * quad + 16 * p->TN + 8) * 4;
+  const size_t red = (size_t)4 * 16 * p->TN * (16 * tm + 4) * 4;
+  const size_t lds = std::max(stage, red);
+  g.epi_off = (int)(lds / 4);
+  p->TM = tm;
+  p->lds = lds + (size_t)4 * 16 * tm * 4;
+  return p->lds <= 150 * 1024;
+}
+
+double patch_us(const PatchPlan& p, int tm, int cus) {
+  const int64_t wgs = (int64_t)p.g.B * p.g.tiles_x * p.g.tiles_y * ((p.g.F + 16 * tm - 1) / (16 * tm));
+  return 3.2 + (double)((wgs + cus - 1) / cus) * (4.0 + 0.0377 * tm * p.TN * (p.g.C / 4));
+}
+
 constexpr int kTileMenu[] = {4, 7, 9, 11};   // instantiated N extents (in 16-pixel tiles)
 
 // Geometry and workgroup shape for one command, a function of its shape and of `pool`
@@ -462,22 +481,15 @@ bool patch_plan_compute(const gh_cmd& c, bool pool, PatchPlan* out) {
   g.npix = bTH * bTW;
   const int64_t patches = (int64_t)g.B * g.tiles_x * g.tiles_y;
   if (patches > (1ll << 30)) return false;
-  // 32 filters per workgroup halve the B-operand reads; 16 when that leaves compute units without one
-  const int TM = (F > 16 && patches * ((F + 31) / 32) >= 200) ? 2 : 1;
   g.mTXY = magic_of(g.tiles_x * g.tiles_y); g.mTX = magic_of(g.tiles_x); g.mPP = magic_of(g.PP);
   g.mPW = magic_of(g.PW); g.mTW = magic_of(g.TW); g.mHTW = magic_of(g.HTW); g.mNPIX = magic_of(g.npix);
   g.mNPOOL = magic_of(g.npix / 4);
   // LDS for two quads to a wavefront, the next one staged under the present one's MFMAs: from 128 channels on (64, which are two
   // quads: 2 x 64 x 48 x 48 -> 128 11.7 us / 12.3) and for 9 and 11 pixel tiles (with 4 and 7 nothing is gained)
   out->two = bTN >= 9 && g.NQ >= 4;
-  const size_t quad = out->two ? 2 * (TM == 1 ? quad_floats<1>() : quad_floats<2>()) : 36 * 16 * TM + 4 * g.PL;
-  const size_t stage = ((size_t)kWaves * quad + 16 * bTN + 8) * 4;
-  const size_t red = (size_t)4 * 16 * bTN * (16 * TM + 4) * 4;
-  size_t lds = stage > red ? stage : red;
-  g.epi_off = (int)(lds / 4);
-  lds += (size_t)4 * 16 * TM * 4;
-  out->g = g; out->TM = TM; out->TN = bTN; out->lds = lds;
-  return lds <= 150 * 1024;
+  out->g = g; out->TN = bTN;
+  // 32 filters per workgroup halve the B-operand reads; 16 when that leaves compute units without one
+  return set_filters(out, F > 16 && patches * ((F + 31) / 32) >= 200 ? 2 : 1);
 }
 
 // The plan of a command, remembered per shape (the search over patch shapes costs tens of microseconds).
@@ -523,8 +535,7 @@ bool gh_conv_patch_takes(const gh_cmd& c) {
 double gh_conv_patch_us(const gh_cmd& c, int cus) {
   PatchPlan p;
   if (!patch_plan(c, false, &p)) return 0;
-  const int64_t wgs = (int64_t)p.g.B * p.g.tiles_x * p.g.tiles_y * ((p.g.F + 16 * p.TM - 1) / (16 * p.TM));
-  return 3.2 + (double)((wgs + cus - 1) / cus) * (4.0 + 0.0377 * p.TM * p.TN * (p.g.C / 4));
+  return patch_us(p, p.TM, cus);
 }
 
 // Pooling rides in the epilogue only where the even-sized patches it needs cost about the
@@ -546,6 +557,12 @@ int gh_try_launch_conv_patch(gh_ctx* ctx, const gh_cmd& c) {
   if (!patch_plan(c, false, &p)) return -1;
   if (pool && (!gh_conv_patch_can_pool(c) || !patch_plan(c, true, &p)))
     return gh_fail(ctx, GH_EINVAL, "conv2d: no fused pooling for this shape (see gh_conv2d_can_pool)");
+  // A piece of a batch has some of the compute units: 2 x 64 x 52 x 52 -> 128, 256 workgroups of 16 filters or 128 of 32, on 248 of
+  // them 27 / 23 us (alone on the device 13.7 / 20.5).
+  if (ctx->whole_images && p.g.F > 16) {
+    PatchPlan q = p;
+    if (patch_us(p, 3 - p.TM, ctx->cu_count) < patch_us(p, p.TM, ctx->cu_count) && set_filters(&q, 3 - p.TM)) p = q;
+  }
 #define GH_PATCH_TN(TM_)                                              \
   switch (p.TN) {                                                     \
     case 4: return launch_patch<TM_, 4, false>(ctx, c, p);            \

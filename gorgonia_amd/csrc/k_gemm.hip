@@ -3257,11 +3257,11 @@ static bool conv_sums_whole(const gh_cmd& c) {
   return plan_tiles(&probe, c.dim[4], c.dim[0] * gh_conv_out(c.dim[2], 3, c.dim[7], 1, 1) * gh_conv_out(c.dim[3], 3, c.dim[8], 1, 1), 9 * c.dim[1], 1, true).splits == 1;
 }
 // float32, behind the single-channel, few-channel and small-image kernels, which win where they take a shape.
-static int conv_lanes_form(const gh_cmd& c, int cus, bool as_pooled = true) {
+static int conv_lanes_form(const gh_cmd& c, int cus) {
   if (c.dim[5] != 3 || c.dim[6] != 3 || gh_conv_rows1_takes(c) || conv_direct_takes(c) || gh_conv_small_takes(c)) return -1;
   // gh_conv2d_can_pool answers without a device, so where only this kernel can pool (and sums as the plain command does) the choice
   // between the two is by the MI355X's compute units on every device.
-  if (as_pooled && cus != kUnits && gh_conv_patch_takes(c) && !gh_conv_patch_can_pool(c)) cus = kUnits;
+  if (cus != kUnits && gh_conv_patch_takes(c) && !gh_conv_patch_can_pool(c)) cus = kUnits;
   return gh_conv_lanes_form(c, false, cus, conv_others_us(c, cus), gh_conv_patch_takes(c), conv_sums_whole(c));
 }
 // The image gradient: elsewhere that is a launch that mirrors the filters (4.7 us) and a forward one over dy.
@@ -3324,6 +3324,48 @@ static int launch_conv_direct(gh_ctx* ctx, const gh_cmd& c) {
   return gh_check_hip(ctx, hipGetLastError(), "direct conv launch");
 }
 
+// The kernel of a plain float32 convolution, the order of gh_launch_conv2d without k_conv3x3_lanes: GH_CONV_ROUTE_* or kStrip.
+constexpr int kStrip = 100;
+static int conv_kernel_but_lanes(const gh_cmd& c, int cus) {
+  const int route = gh_conv2d_route(&c);
+  if (route == GH_CONV_ROUTE_ROWS1 || route == GH_CONV_ROUTE_DIRECT || route == GH_CONV_ROUTE_ROWS || route == GH_CONV_ROUTE_SMALL) return route;
+  if (gh_conv_strip_takes(c) && gh_conv_wide_takes(c)) return kStrip;
+  if (route == GH_CONV_ROUTE_PATCH || route == GH_CONV_ROUTE_WIDE) return route;
+  if (gh_conv_pointwise_takes(c, cus)) return GH_CONV_ROUTE_POINTWISE;
+  return route == GH_CONV_ROUTE_POINTWISE ? GH_CONV_ROUTE_GATHER : route;
+}
+
+// Whether `images` of a convolution's images as a command of their own, planned for part_units compute units, have the whole
+// command's bits: on a kernel whose sums do not depend on the number of images (the small-image kernels cut the channels by it, the
+// tiled and the gathering one cut them among workgroups), the same for both.
+bool gh_conv2d_in_pieces(const gh_cmd& c, int64_t images, int units, int part_units) {
+  if (gh_dtype_of(c.flags) != GH_F32 || (c.flags & (GH_FLAG_CONV_PRE | GH_FLAG_CONV_KEEP))) return false;
+  gh_cmd part = c;
+  part.dim[0] = images;
+  const int of_all = conv_kernel_but_lanes(c, units), of_part = conv_kernel_but_lanes(part, part_units);
+  const bool pool = c.flags & GH_FLAG_CONV_POOL2;
+  auto in_front = [](int k) { return k == GH_CONV_ROUTE_ROWS1 || k == GH_CONV_ROUTE_DIRECT || k == GH_CONV_ROUTE_ROWS || k == GH_CONV_ROUTE_SMALL || k == kStrip; };
+  if (!in_front(of_all) && conv_lanes_form(c, units) >= 0) return !in_front(of_part);
+  switch (of_all) {
+    case GH_CONV_ROUTE_ROWS1: case GH_CONV_ROUTE_DIRECT: case GH_CONV_ROUTE_POINTWISE: case kStrip: return of_part == of_all;
+    case GH_CONV_ROUTE_PATCH: return of_part == of_all && (!pool || gh_conv_patch_can_pool(part));
+    case GH_CONV_ROUTE_WIDE: return of_part == of_all && (!pool || gh_conv_wide_can_pool(part));
+  }
+  return false;
+}
+
+// The form for a piece of a batch, -1 where the batch's other kernel has it: the batch's, or the quickest for the piece of those
+// that add as it does.  (k_conv3x3_wide adds as the forms do whose wavefronts have all channels: quad by quad, tap by tap.)
+static int conv_piece_form(const gh_ctx* ctx, const gh_cmd& c) {
+  gh_cmd whole = c;
+  whole.dim[0] = ctx->whole_images;
+  const int form = conv_lanes_form(whole, ctx->whole_units);
+  if (form >= 0) return gh_conv_lanes_form_like(c, form, ctx->cu_count);
+  if (conv_kernel_but_lanes(whole, ctx->whole_units) != GH_CONV_ROUTE_WIDE) return -1;
+  const int own = conv_lanes_form(c, ctx->cu_count);
+  return own >= 3 ? own : -1;
+}
+
 int gh_launch_conv2d(gh_ctx* ctx, const gh_cmd& c) {
   if (gh_dtype_of(c.flags) == GH_F64) return gh_launch_conv2d_f64(ctx, c);
   if (c.flags & GH_FLAG_CONV_PRE) {
@@ -3339,7 +3381,7 @@ int gh_launch_conv2d(gh_ctx* ctx, const gh_cmd& c) {
   const int rcs = gh_try_launch_conv_small(ctx, c);
   if (rcs >= 0) return rcs;
   if (gh_conv_strip_takes(c) && gh_conv_wide_takes(c)) return gh_launch_conv_strip(ctx, c);
-  if (const int form = conv_lanes_form(c, ctx->cu_count, !ctx->beside_copy || (c.flags & GH_FLAG_CONV_POOL2)); form >= 0) return gh_launch_conv_lanes(ctx, c, false, form);
+  if (const int form = ctx->whole_images ? conv_piece_form(ctx, c) : conv_lanes_form(c, ctx->cu_count); form >= 0) return gh_launch_conv_lanes(ctx, c, false, form);
   const int rcp = gh_try_launch_conv_patch(ctx, c);
   if (rcp >= 0) return rcp;
   const int rcw = gh_try_launch_conv_wide(ctx, c);

@@ -74,6 +74,7 @@ HOST_SYMBOLS = {
     "ghh_engine_do_work": (C.c_int, [_P]),
     "ghh_engine_pending": (C.c_int, [_P]),
     "ghh_engine_submit_calls": (C.c_int64, [_P]),
+    "ghh_engine_joint_launches": (C.c_int64, [_P, C.c_int, C.POINTER(C.c_int64)]),
     "ghh_graph_new": (_P, []),
     "ghh_graph_destroy": (None, [_P]),
     "ghh_graph_last_error": (C.c_char_p, [_P]),
@@ -267,6 +268,11 @@ class Engine:
 
     def submit_calls(self):
         return self.lib.ghh_engine_submit_calls(self.h)
+
+    def joint_launches(self, kind):
+        """Context.joint_launches of the engine's context."""
+        form = C.c_int64()
+        return self.lib.ghh_engine_joint_launches(self.h, kind, C.byref(form)), form.value
 
     # Arena
     def Get(self, size):

@@ -173,6 +173,7 @@ int ghh_engine_has_inf(ghh_engine* e, const ghh_tensor* a, int* out) {
 int ghh_engine_do_work(ghh_engine* e) { return ret(e, e->e->DoWork()); }
 int ghh_engine_pending(ghh_engine* e) { return (int)e->e->PendingCommands(); }
 int64_t ghh_engine_submit_calls(ghh_engine* e) { return e->e->SubmitCalls(); }
+int64_t ghh_engine_joint_launches(ghh_engine* e, int kind, int64_t* form) { return e->e->Context() ? gh_joint_launches(e->e->Context(), kind, form) : -1; }
 
 // ---- graph / tape ------------------------------------------------------------------
 ghh_graph* ghh_graph_new(void) { return new ghh_graph(); }

@@ -92,6 +92,8 @@ GH_API int ghh_engine_has_inf(ghh_engine* e, const ghh_tensor* a, int* out);
 GH_API int ghh_engine_do_work(ghh_engine* e);                            /* DoWork / Signal */
 GH_API int ghh_engine_pending(ghh_engine* e);        /* commands recorded, not yet submitted */
 GH_API int64_t ghh_engine_submit_calls(ghh_engine* e);
+/* gh_joint_launches of the engine's context, -1 before Init */
+GH_API int64_t ghh_engine_joint_launches(ghh_engine* e, int kind, int64_t* form);
 
 /* ---- graph + tape machine ------------------------------------------------------ */
 typedef struct ghh_graph ghh_graph;

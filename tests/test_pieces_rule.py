@@ -61,3 +61,13 @@ def test_images_of_another_size(channels, layers):
     cmds = _net()
     cmds[3] = D.cmd_maxpool2d(_at(3), _at(4), B, channels, 112, 112, 2, 2, (0, 0, 0, 0), (2, 2))
     assert _layers(cmds) == layers
+
+
+# kernels that cut the channels by the number of images: gathering, tiled through LDS, small images
+@pytest.mark.parametrize("conv", [D.cmd_conv2d(_at(0), _at(1), _at(2), B, 3, H, W, 64, 16, 16, (0, 0), (16, 16)), D.cmd_conv2d(_at(0), _at(1), _at(2), B, 3, H, W, 16, 5, 5, (2, 2)),
+                                  D.cmd_conv2d(_at(0), _at(1), _at(2), B, 588, 16, 16, 16, 3, 3, (1, 1)), D.cmd_conv2d(_at(0), _at(1), _at(2), 96, 64, 14, 14, 64, 3, 3, (1, 1))])
+def test_kernels_whose_sums_depend_on_the_number_of_images(conv):
+    bytes_ = 4 * conv.dim[0] * conv.dim[1] * conv.dim[2] * conv.dim[3]
+    assert bytes_ >= 4000000 and _layers([D.cmd_copy(_at(0), _at(9), bytes_), conv]) == 0
+    pool = D.cmd_maxpool2d(_at(0), _at(2), *conv.dim[:4], 2, 2, (0, 0), (2, 2))
+    assert _layers([D.cmd_copy(_at(0), _at(9), bytes_), pool]) == 1
