@@ -1100,24 +1100,44 @@ Status TapeMachine::Compile() {
           early[(size_t)i].push_back(j);
         }
     }
-  // The convolutions and poolings behind an uploaded batch may run in pieces of it, for which their values have to lie apart:
-  // what they read is kept until the last of them is done.
+  // The layers behind a lent batch that run in pieces of it (asked with every tensor in a place of its own): what they read,
+  // filters and constants among it, is kept until the last of them is done, so that no result takes its place.
   if (!opt_.node_at_a_time)
     for (int i = 0; i < N; i++) {
       const Node& x = nodes[(size_t)i];
-      if (!x.is_input || x.resident || x.shape.Dims() != 4 || x.dt != Dtype::Float32 || x.shape[0] < 2 || bytes_of(x) < GH_PIECES_FROM) continue;
-      int at = i, end = -1;
-      std::vector<int> kept;
-      for (;;) {
-        kept.push_back(node_reg_[(size_t)at]);
-        const int next = last_reader[(size_t)root[(size_t)at]];
-        if (next < 0) break;
-        const Node& n = nodes[(size_t)next];
+      if (!x.is_input || !x.host_borrowed || x.resident || x.shape.Dims() != 4 || x.dt != Dtype::Float32 || bytes_of(x) < GH_PIECES_FROM) continue;
+      Engine asked;
+      uint64_t place = 0;
+      auto tensor = [&](int node) {
+        Tensor t;
+        t.mem = ++place << 40;
+        t.dt = nodes[(size_t)node].dt;
+        t.shape = nodes[(size_t)node].shape;
+        return t;
+      };
+      Tensor front = tensor(i);
+      asked.RecordCopy(front.mem, tensor(i).mem, bytes_of(x));
+      std::vector<int> layers;
+      int at = i;
+      for (int j = 0; j < N; j++) {
+        const Node& n = nodes[(size_t)j];
+        if (n.fused_away || n.is_input || n.deferred || (n.alias_of >= 0 && n.op.kind == OpKind::Reshape)) continue;
         if ((n.op.kind != OpKind::Conv2d && n.op.kind != OpKind::MaxPool2D) || n.inputs.empty() || root[(size_t)n.inputs[0]] != root[(size_t)at]) break;
-        at = end = next;
+        std::vector<Tensor> ins;
+        for (int in : n.inputs) ins.push_back(tensor(in));
+        ins[0].mem = front.mem;
+        std::vector<Tensor*> inp;
+        for (Tensor& t : ins) inp.push_back(&t);
+        front = tensor(j);
+        if (!CUDADo(asked, n.op, front, inp).ok()) break;
+        layers.push_back(at = j);
       }
-      for (int r : kept)
-        if (r >= 0 && reg_last[(size_t)r] >= 0) reg_last[(size_t)r] = std::max(reg_last[(size_t)r], end);
+      const int kept = gh_pieces_layers(asked.Segment().data(), (int)asked.Segment().size());
+      for (int k = 0; k < kept; k++)
+        for (int in : nodes[(size_t)layers[(size_t)k]].inputs) {
+          int& last = reg_last[(size_t)node_reg_[(size_t)in]];
+          last = std::max(last, layers[(size_t)kept - 1]);
+        }
     }
   // A small result that only the host reads is written by its kernel straight
   // into pinned host memory: no arena register, no staging copy at the end of

@@ -123,3 +123,35 @@ def test_tape(monkeypatch, mode):
     launches, form = m.engine().joint_launches(_ffi.JOINT_PIECES)
     assert form % 100 >= 4 and (launches == 7 if not mode else launches >= 1)   # (the first run uploads the filters as well)
     m.Close()
+
+
+def test_tape_with_filters_that_are_not_resident(monkeypatch):
+    """Filters uploaded in front of a lent batch by each run: their memory is not given to a result that a first piece writes while
+    the next one still reads them."""
+    B, S = 16, 52
+    r = np.random.default_rng(4)
+    x = r.uniform(-1, 1, (B, 64, S, S)).astype(np.float32)
+    ws = [r.standard_normal(s).astype(np.float32) / 24 for s in ((128, 64, 3, 3), (64, 128, 3, 3))]
+
+    def run():
+        g = G.NewGraph()
+        w = [G.NewTensor(g, v) for v in ws]
+        node = G.LetBorrowed(G.NewTensor(g, x))
+        h = G.MaxPool2D(G.Conv2d(node, w[0], (3, 3), (1, 1), (1, 1), (1, 1)), (2, 2), (0, 0), (2, 2))
+        out = G.Read(G.Rectify(G.Conv2d(h, w[1], (3, 3), (1, 1), (1, 1), (1, 1))))
+        m = G.NewTapeMachine(g)
+        m.input(node)[...] = x
+        got = []
+        for k in range(3):
+            G.Let(w[0], ws[0] * np.float32(k + 1))
+            m.RunAll()
+            got.append(out.copy())
+        form = m.engine().joint_launches(_ffi.JOINT_PIECES)
+        m.Close()
+        return got, form
+    got, (launches, form) = run()
+    monkeypatch.setenv("GORGONIA_HIP_NO_PIECES", "1")
+    want, none = run()
+    assert none[0] == 0 and launches == 3 and form % 100 == 3, (launches, form)
+    for g, w in zip(got, want):
+        assert_bits_equal(g, w)

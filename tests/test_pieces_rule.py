@@ -1,8 +1,10 @@
 """Which layers behind the upload of a batch run in pieces of it (gh_pieces.hip), asked without a device."""
+import numpy as np
 import pytest
 
 from gorgonia_amd import _ffi
 from gorgonia_amd import device as D
+from gorgonia_amd import graph as G
 
 B, H, W = 8, 224, 224
 BATCH = 12 * B * H * W
@@ -71,3 +73,41 @@ def test_kernels_whose_sums_depend_on_the_number_of_images(conv):
     assert bytes_ >= 4000000 and _layers([D.cmd_copy(_at(0), _at(9), bytes_), conv]) == 0
     pool = D.cmd_maxpool2d(_at(0), _at(2), *conv.dim[:4], 2, 2, (0, 0), (2, 2))
     assert _layers([D.cmd_copy(_at(0), _at(9), bytes_), pool]) == 1
+
+
+def _program(lend, resident=False, more=0):
+    """What a compiled machine frees behind each operator: input nodes by name; a convolution, 2 + `more` poolings and a Rectify."""
+    g = G.NewGraph()
+    x = G.NewTensor(g, np.zeros((B, 3, H, W), np.float32))
+    w = G.NewTensor(g, np.zeros((16, 3, 3, 3), np.float32), resident=resident)
+    if lend:
+        G.LetBorrowed(x)
+    nodes = [G.Conv2d(x, w, (3, 3), (1, 1), (1, 1), (1, 1))]
+    for _ in range(2 + more):
+        nodes.append(G.MaxPool2D(nodes[-1], (2, 2), (0, 0), (2, 2)))
+    G.Read(G.Rectify(nodes[-1]))
+    m = G.NewTapeMachine(g, compile_only=True)
+    lines, behind, names = [l.split("\t")[1].split() for l in m.program().splitlines() if "\t" in l], [], {}
+    for l in lines:
+        if l[0] == "alloc":
+            names[l[3]] = {x.id: "x", w.id: "w"}.get(int(l[2]), int(l[2]) - nodes[0].id)
+        if l[0] == "execOp":
+            behind.append([])
+        if l[0] == "free" and behind:
+            behind[-1].append(names[l[3]])
+    m.Close()
+    return [sorted(map(str, b)) for b in behind[:3 + more]]
+
+
+def test_a_lent_batch_keeps_what_its_layers_read():
+    """Until the last layer that runs in pieces: behind the second pooling here, and of five layers behind the third."""
+    assert _program(True) == [[], [], ["0", "1", "w", "x"]]
+    assert _program(True, resident=True) == [[], [], ["0", "1", "x"]]
+    far = _program(True, more=3)
+    kept = next(i for i, b in enumerate(far) if b)
+    assert far[kept] == sorted([str(i) for i in range(kept)] + ["w", "x"]) and far[kept + 1:] == [[str(i)] for i in range(kept, 5)]
+
+
+def test_a_batch_bound_with_let_keeps_nothing():
+    """It never runs in pieces: every value goes with its reader."""
+    assert _program(False) == [["w", "x"], ["0"], ["1"]]
