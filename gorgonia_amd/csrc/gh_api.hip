@@ -86,6 +86,7 @@ static uint32_t* take_word() {
   uint32_t* const w = (uint32_t*)(g_words_page + 64 * i);
   *w = 0;
   ((uint64_t*)w)[1] = 0;
+  w[4] = 0;
   return w;
 }
 static void give_word(uint32_t* w) {

@@ -118,7 +118,7 @@ struct gh_ctx {
   hipEvent_t pieces_after = nullptr;
   void* piece_words = nullptr;
   uint64_t piece_seq = 0;
-  bool no_pieces = false;   // they were not to be had
+  bool no_pieces = false;   // they were not to be had, or are given up too often
   // while a piece's layers are submitted: the images of the whole batch and the compute units that it would be planned for
   int64_t whole_images = 0;
   int whole_units = 0;

@@ -16,8 +16,11 @@
 // 8 x 3 x 320 x 320 449 / 416, five of them 310 / 301, 8 x 3 x 224 x 224 250 / 243.
 //
 // Nothing waits for a workgroup that has not begun: a part of a piece is copied by whoever claims it first, the copy's
-// workgroup or, after kGiveUp of the device's clock, the kernel that waits for it (where something runs the streams one after
-// the other, the copy behind).  A part that is claimed is being copied, and waited for without a limit.
+// workgroup or, after some time of the device's clock, the kernel that waits for it (where something runs the streams one after
+// the other, the copy behind: a process has four hardware queues, and the copies of two contexts may each stand behind the other's
+// layers).  That is about three times what the bus takes, and once in an upload: the pieces behind are copied without a wait for
+// who has not begun by then.  A part that is claimed is being copied, and waited for without a limit.  After kMisses such uploads
+// close to each other the context's batches go whole.
 #include <algorithm>
 #include <cstdlib>
 
@@ -27,7 +30,9 @@ namespace {
 
 constexpr int kThreads = 1024, kCopiers = 8;
 constexpr int kThrough = 1 | 16;                      // a store's sc0 and sc1 bits: to memory, past the caches
-constexpr int64_t kGiveUp = 400000;                   // ticks of 10 ns, and one more for 100 bytes (GORGONIA_HIP_PIECES_TICKS: fewer)
+constexpr int64_t kBegin = 20000;                     // ticks of 10 ns for a workgroup to begin, and one more for 200 bytes
+constexpr int64_t kGiveUp = 400000;                   // and to claim a part, and one more for 100 bytes (GORGONIA_HIP_PIECES_TICKS: fewer of both)
+constexpr int kMisses = 3, kWithin = 64;              // uploads that were given up, and how many may lie between two of them
 constexpr int64_t kLeast = GH_PIECES_FROM, kMost = 1 << 30;  // bytes of an upload (the least: two images of 3 x 416 x 416 gain 3 %)
 constexpr int64_t kPieceBytes = 4 << 20;              // (8 x 3 x 416 x 416 in two, three, four and eight: 658, 637, 627 and 674 us)
 constexpr int kHead = 12;
@@ -36,8 +41,9 @@ constexpr int64_t kTryFor = 30000;                    // ticks of 10 ns
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 // Who copies part b of piece p (2 s: the copy's workgroup, 2 s + 1: the kernel that waits), and that it is there (s), for the
-// context's s-th upload.
-struct Words { unsigned long long claim[kPieces][kCopiers], there[kPieces][kCopiers]; };
+// context's s-th upload.  late: the last upload of which a kernel that waits has given something up; missed, misses: the last one
+// that counts, and how many there have been in a row.
+struct Words { unsigned long long claim[kPieces][kCopiers], there[kPieces][kCopiers], late, missed, misses; };
 struct Ends { int n16[kPieces]; };
 
 __device__ __forceinline__ bool claims(unsigned long long* word, unsigned long long seq, int who) {
@@ -69,24 +75,40 @@ __global__ __launch_bounds__(kThreads) void k_copy_pieces(void* dst, const u32x4
 }
 
 __global__ __launch_bounds__(kThreads) void k_await_piece(void* dst, const u32x4* __restrict__ src, int bytes, int from, int to, int tail_words, Words* words,
-                                                          int p, unsigned long long seq, int64_t give_up) {
+                                                          int p, unsigned long long seq, int64_t begin, int64_t give_up, unsigned* misses) {
   __shared__ unsigned long long left;   // the parts that are copied here
   if (threadIdx.x < 64) {
     const int part = threadIdx.x;
     const int64_t t0 = wall_clock64();
+    const bool late = words->late == seq;
     bool waits = part < kCopiers, mine = false, tried = false;
     for (;;) {
       if (waits) waits = __hip_atomic_load(&words->there[p][part], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < seq;
       if (__ballot(waits) == 0) break;
-      if (!tried && (int64_t)wall_clock64() - t0 >= give_up) {   // (of the wavefront: t0 and the clock are the same in all lanes)
-        tried = true;
-        if (waits) mine = claims(&words->claim[p][part], seq, 1);
-        waits = waits && !mine;
+      const int64_t t = (int64_t)wall_clock64() - t0;
+      if (waits && !tried && (late || t >= begin)) {
+        // (a workgroup that has had its part of the first piece comes to this one)
+        const bool begun = __hip_atomic_load(&words->claim[0][part], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 2 * seq;
+        if (!begun || t >= give_up) {
+          tried = true;
+          mine = claims(&words->claim[p][part], seq, 1);
+          waits = !mine;
+        }
       }
       __builtin_amdgcn_s_sleep(2);
     }
     const unsigned long long all = __ballot(mine);
-    if (part == 0) left = all;
+    if (part == 0) {
+      left = all;
+      if (all && !late) {
+        words->late = seq;
+        if (misses) {
+          words->misses = words->missed && seq - words->missed <= kWithin ? words->misses + 1 : 1;
+          words->missed = seq;
+          __hip_atomic_store(misses, (unsigned)words->misses, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+      }
+    }
   }
   __syncthreads();
   if (left == 0) return;
@@ -213,9 +235,13 @@ bool side_by_side(gh_ctx* ctx, hipStream_t s) {
   return hipMemcpyAsync(&seen, word + 1, sizeof seen, hipMemcpyDeviceToHost, ctx->stream) == hipSuccess && hipStreamSynchronize(ctx->stream) == hipSuccess && seen;
 }
 
-// The stream, the event and the words, made for the first upload in pieces.
+// Where the kernels that wait say how many uploads they gave up, behind the completion word on its cache line.
+unsigned* missed(const gh_ctx* ctx) { return ctx->done_word + 4; }
+
+// The stream, the event and the words, made for the first upload in pieces (which so waits for what is on the context's stream).
 bool ready(gh_ctx* ctx, bool* fresh) {
-  if (ctx->pieces || ctx->no_pieces) return ctx->pieces;
+  if (!ctx->done_word || (ctx->pieces && __atomic_load_n(missed(ctx), __ATOMIC_RELAXED) >= (unsigned)kMisses)) ctx->no_pieces = true;
+  if (ctx->pieces || ctx->no_pieces) return !ctx->no_pieces;
   int before = ctx->device;
   (void)hipGetDevice(&before);
   bool ok = hipSetDevice(ctx->device) == hipSuccess && hipMalloc(&ctx->piece_words, sizeof(Words)) == hipSuccess &&
@@ -285,20 +311,25 @@ int gh_submit_pieces(gh_ctx* ctx, const gh_cmd* cmds, int n, int* rc) {
     last[p] = (B * (p + 1) + pieces - 1) / pieces;
     ends.n16[p] = (int)(p == pieces - 1 ? bytes / 16 : (last[p] * (bytes / B) + 15) / 16);
   }
-  int64_t give_up = kGiveUp + bytes / 100;
-  if (const char* ticks = getenv("GORGONIA_HIP_PIECES_TICKS")) give_up = std::max<int64_t>(0, std::min<int64_t>(give_up, atoll(ticks)));
+  int64_t begin = kBegin + bytes / 200, give_up = kGiveUp + bytes / 100;
+  const char* const ticks = getenv("GORGONIA_HIP_PIECES_TICKS");   // tests: the waits given up early, which counts where the copy is late as well
+  const bool late = getenv("GORGONIA_HIP_PIECES_LATE");            // tests: the copy behind the layers
+  if (ticks)
+    for (int64_t* limit : {&begin, &give_up}) *limit = std::max<int64_t>(0, std::min<int64_t>(*limit, atoll(ticks)));
+  unsigned* const misses = ticks && !late ? nullptr : missed(ctx);
   void* const dst = (void*)(uintptr_t)up.ptr[0];
   const u32x4* const src = (const u32x4*)(uintptr_t)up.ptr[1];
   const int tail_words = (int)(bytes % 16 / 4);
   const unsigned long long seq = ++ctx->piece_seq;
-  if (e == hipSuccess) {
+  auto copy = [&] {
     hipLaunchKernelGGL(k_copy_pieces, dim3(kCopiers), dim3(kThreads), 0, ctx->pieces, dst, src, ends, pieces, tail_words, (Words*)ctx->piece_words, seq);
-    e = hipGetLastError();
-  }
+    return hipGetLastError();
+  };
+  if (e == hipSuccess && !late) e = copy();
   for (int p = 0; p < pieces && e == hipSuccess && !*rc; p++) {
     const int64_t first = p ? last[p - 1] : 0;
     hipLaunchKernelGGL(k_await_piece, dim3(1), dim3(kThreads), 0, ctx->stream, dst, src, (int)bytes, p ? ends.n16[p - 1] : 0, ends.n16[p],
-                       p == pieces - 1 ? tail_words : 0, (Words*)ctx->piece_words, p, seq, give_up);
+                       p == pieces - 1 ? tail_words : 0, (Words*)ctx->piece_words, p, seq, begin, give_up, misses);
     if ((e = hipGetLastError()) != hipSuccess) break;
     gh_cmd part[kHead];
     for (int k = 0; k < head; k++) {
@@ -316,6 +347,11 @@ int gh_submit_pieces(gh_ctx* ctx, const gh_cmd* cmds, int n, int* rc) {
     *rc = gh_submit_each(ctx, part, head);
     ctx->cu_count = ctx->whole_units;
     ctx->whole_images = 0;
+  }
+  if (e == hipSuccess && late) {
+    e = hipEventRecord(ctx->pieces_after, ctx->stream);
+    if (e == hipSuccess) e = hipStreamWaitEvent(ctx->pieces, ctx->pieces_after, 0);
+    if (e == hipSuccess) e = copy();
   }
   if (e != hipSuccess && !*rc) *rc = gh_check_hip(ctx, e, "upload in pieces");
   if (*rc) (void)hipStreamSynchronize(ctx->pieces);   // nothing of it is under way behind an error
