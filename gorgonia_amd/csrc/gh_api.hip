@@ -500,12 +500,12 @@ int gh_validate(const gh_cmd* cmds, int n, char* msg, int msg_len) {
   return GH_OK;
 }
 
-int gh_submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
+int gh_submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n, int before) {
   ctx->idle = false;
   for (int i = 0; i < n; i++) {
     std::string m;
     int rc = gh_validate_cmd(cmds[i], m);
-    if (rc) return gh_fail(ctx, rc, "cmd " + std::to_string(i) + ": " + m);
+    if (rc) return gh_fail(ctx, rc, "cmd " + std::to_string(before + i) + ": " + m);
     // solver steps take the sums that wait along where they are their gradients
     if (ctx->pending && cmds[i].opcode == GH_OP_SOLVER_STEP) {
       const int steps = gh_solver_run_length(cmds + i, n - i);
@@ -527,7 +527,7 @@ int gh_submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
     if (run > 1) {
       for (int j = 1; j < run; j++) {
         rc = gh_validate_cmd(cmds[i + j], m);
-        if (rc) return gh_fail(ctx, rc, "cmd " + std::to_string(i + j) + ": " + m);
+        if (rc) return gh_fail(ctx, rc, "cmd " + std::to_string(before + i + j) + ": " + m);
         if ((rc = gh_flush_sums_before(ctx, cmds[i + j]))) return rc;
       }
       rc = solver ? gh_launch_solver_steps(ctx, cmds + i, solver, copy) : gh_launch_chain(ctx, cmds + i, run);
@@ -590,7 +590,7 @@ int gh_submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n) {
     // two commands of which the second reads what the first writes are one launch where a kernel takes both
     const bool held = gh_bn_held_pair(ctx, cmds + i, n - i), pair = held || gh_is_pair(cmds + i, n - i);
     if (cmds[i].opcode == GH_OP_MAXPOOL2D_BWD && (cmds[i].flags & GH_FLAG_BN_REMADE)) {
-      if (!gh_bn_remade_follows(cmds + i, n - i)) return gh_fail(ctx, GH_EINVAL, "cmd " + std::to_string(i) + ": maxpool2d gradient: the batch normalisation's gradient does not follow");
+      if (!gh_bn_remade_follows(cmds + i, n - i)) return gh_fail(ctx, GH_EINVAL, "cmd " + std::to_string(before + i) + ": maxpool2d gradient: the batch normalisation's gradient does not follow");
       if ((rc = gh_flush_sums_before(ctx, cmds[i + 1]))) return rc;
       if (!held && (rc = gh_launch_bn_remake(ctx, cmds + i))) return rc;
     }
@@ -625,7 +625,7 @@ static int submit_cmds(gh_ctx* ctx, const gh_cmd* cmds, int n) {
   ctx->defer_sums = n > 1 && !ctx->ws_strict && slab_space(ctx, cmds, n);
   int rc = GH_OK;
   const int ahead = gh_submit_pieces(ctx, cmds, n, &rc);
-  if (!rc) rc = gh_submit_each(ctx, cmds + ahead, n - ahead);
+  if (!rc) rc = gh_submit_each(ctx, cmds + ahead, n - ahead, ahead);
   ctx->defer_sums = false;
   const int late = gh_flush_sums(ctx);
   return rc ? rc : late;

@@ -147,7 +147,7 @@ bool gh_llc_stream(int64_t bytes, bool cold);
 // a copy out of pinned host memory and the commands behind it in pieces of the batch (gh_pieces.hip): how many commands it
 // has submitted (0: none), *rc what came of them
 int gh_submit_pieces(gh_ctx* ctx, const gh_cmd* cmds, int n, int* rc);
-extern "C" int gh_submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n);
+extern "C" int gh_submit_each(gh_ctx* ctx, const gh_cmd* cmds, int n, int before);   // before: commands of the caller's in front of these, for messages
 bool gh_in_pinned_host(const gh_ctx* ctx, uint64_t p);
 void gh_drop_pieces(gh_ctx* ctx);
 // sums of filter-gradient slabs, put off where gh_submit allows it (k_slab_sums.hip)

@@ -344,7 +344,7 @@ int gh_submit_pieces(gh_ctx* ctx, const gh_cmd* cmds, int n, int* rc) {
     ctx->whole_images = B;
     ctx->whole_units = ctx->cu_count;
     if (p + 1 < pieces) ctx->cu_count = units_beside(ctx->cu_count);
-    *rc = gh_submit_each(ctx, part, head);
+    *rc = gh_submit_each(ctx, part, head, 1);
     ctx->cu_count = ctx->whole_units;
     ctx->whole_images = 0;
   }

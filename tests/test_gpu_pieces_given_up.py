@@ -106,3 +106,27 @@ def test_given_up_once(monkeypatch):
         assert ctx.joint_launches(_ffi.JOINT_PIECES) == (3, 405)
         assert min(took) < 15e-3
         runs.close()
+
+
+def test_a_message_names_the_callers_command(monkeypatch):
+    """Behind the commands that ran in pieces, as where the batch went whole."""
+    with D.Context(0, 0) as ctx:
+        runs = _Runs(ctx, monkeypatch, B=2)
+        chain = runs.chain
+        cmds = [D.cmd_copy(chain.x, runs.host.p.value, chain.nbytes)] + chain.layers
+        for at in (len(cmds), len(cmds) + 1):
+            bad = cmds + [D.cmd_relu(chain.x, chain.x, 16)] * (at - len(cmds)) + [D.cmd_relu(chain.x, 0, 16)]
+            said = []
+            for whole in (False, True):
+                with monkeypatch.context() as p:
+                    if whole:
+                        p.setenv("GORGONIA_HIP_NO_PIECES", "1")
+                    before = ctx.joint_launches(_ffi.JOINT_PIECES)[0]
+                    with pytest.raises(D.DeviceError) as e:
+                        ctx.submit(bad)
+                    assert ctx.joint_launches(_ffi.JOINT_PIECES)[0] - before == (not whole)
+                said.append(str(e.value))
+                ctx.clear_error()
+                ctx.sync()
+            assert said[0] == said[1] and f"cmd {at}:" in said[0], said
+        runs.close()
