@@ -6,11 +6,6 @@
 
 #include "gh_internal.h"
 
-// Epilogue activations in the reference's arithmetic form (nn.go:83-163).
-// act 3 is LeakyRelu for a finite alpha >= 0 in four instructions instead of eight, with the
-// same bits: for v < 0 the reference's sum is -0 + v alpha = v alpha, for v >= 0 it is v + 0 = v,
-// and the v * 0 that fmaf adds is a zero of v's sign (which changes neither) unless v is
-// infinite or NaN, where it makes the NaN the reference's inf * 0 makes.
 // A Rectify behind a product (z null) or a Rectify's gradient (z: what it was taken of), value by value into `out`, a tensor of
 // the product's size and layout; where that is the product's own memory, the product is not stored.
 template <class T>
@@ -26,6 +21,11 @@ struct gh_rectify_behind {
   }
 };
 
+// Epilogue activations in the reference's arithmetic form (nn.go:83-163).
+// act 3 is LeakyRelu for a finite alpha >= 0 in four instructions instead of eight, with the
+// same bits: for v < 0 the reference's sum is -0 + v alpha = v alpha, for v >= 0 it is v + 0 = v,
+// and the v * 0 that fmaf adds is a zero of v's sign (which changes neither) unless v is
+// infinite or NaN, where it makes the NaN the reference's inf * 0 makes.
 __device__ __forceinline__ float act_apply(float v, int act, float alpha) {
   if (act == 1) return v * (v >= 0.0f ? 1.0f : 0.0f);
   if (act == 3) {

@@ -167,16 +167,16 @@ int gh_chain_length(const gh_cmd* cmds, int n);
 int gh_launch_chain(gh_ctx* ctx, const gh_cmd* cmds, int count);
 // two commands in one launch (k_pairs.hip)
 bool gh_is_pair(const gh_cmd* cmds, int n);
-// a SoftMax, the tensor times a scalar behind it and the SoftMax gradient that takes both (k_pairs.hip, k_gemm.hip): what is
-// behind the SoftMax's own values, row by row
-template <class T> struct gh_softmax_gradient { const T* x; const T* s; T* g; T* dx; };
+int gh_launch_pair(gh_ctx* ctx, const gh_cmd* cmds);
 // a product and the Rectify behind it (k_gemm.hip)
 bool gh_rectify_follows(const gh_cmd* cmds, int n);
 int gh_try_launch_gemm_rectify(gh_ctx* ctx, const gh_cmd* cmds);   // -1: no kernel has both
+// a SoftMax, the tensor times a scalar behind it and the SoftMax gradient that takes both (k_pairs.hip, k_gemm.hip): what is
+// behind the SoftMax's own values, row by row
+template <class T> struct gh_softmax_gradient { const T* x; const T* s; T* g; T* dx; };
 bool gh_softmax_gradient_follows(const gh_cmd* cmds, int n);
 int gh_try_launch_softmax_gradient(gh_ctx* ctx, const gh_cmd* cmds);        // of a SOFTMAX; -1: no kernel has the three
 int gh_try_launch_gemm_softmax_gradient(gh_ctx* ctx, const gh_cmd* cmds);   // of a GEMM with its SoftMax
-int gh_launch_pair(gh_ctx* ctx, const gh_cmd* cmds);
 int gh_launch_elem_bin(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_elem_unary(gh_ctx* ctx, const gh_cmd& c);
 int gh_launch_bcast_bin(gh_ctx* ctx, const gh_cmd& c);

@@ -47,11 +47,6 @@ __global__ __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(WV == 8
   }
 }
 
-// Where there are somewhat more tiles than workgroups that the device holds at once, a workgroup for each leaves the last ones to
-// the places that fall free together, two on one compute unit and none on the next: 8 x 128 x 26 x 26 -> 256 pooled, 728 tiles
-// for 512 places, 44.5 us, float64 8 x 32 x 104 x 104 -> 64, 676 for 512, 77.0.  With as many workgroups as places, each with
-// every so many-th tile, the compute units have one more or none: 35.9 and 59.8.  From twice the places on the last round is
-// the smaller part, and the kernel that walks takes some 0.2 us more.
 // How many workgroups of a kernel the device holds at once.
 template <auto kKernel>
 int64_t held_at_once(const gh_ctx* ctx, int threads) {
@@ -62,6 +57,11 @@ int64_t held_at_once(const gh_ctx* ctx, int threads) {
   return (int64_t)share * ctx->cu_count;
 }
 
+// Where there are somewhat more tiles than workgroups that the device holds at once, a workgroup for each leaves the last ones to
+// the places that fall free together, two on one compute unit and none on the next: 8 x 128 x 26 x 26 -> 256 pooled, 728 tiles
+// for 512 places, 44.5 us, float64 8 x 32 x 104 x 104 -> 64, 676 for 512, 77.0.  With as many workgroups as places, each with
+// every so many-th tile, the compute units have one more or none: 35.9 and 59.8.  From twice the places on the last round is
+// the smaller part, and the kernel that walks takes some 0.2 us more.
 template <class T, int WV, int TM, int V, int G, bool kSplit>
 int launch(gh_ctx* ctx, Lanes<T> g, const ConvTail& tail, bool flip, bool pool) {
   constexpr int per = 16 * G * (kSplit ? 1 : WV);

@@ -219,7 +219,8 @@ __global__ __launch_bounds__(kWaves * 64) void k_conv3x3_patch(const float* __re
 #pragma unroll
       for (int t = 0; t < TN; t++) bf[set][t] = Pw[at + pb[t][kr] + kc];
     };
-    // the filter tile's rows and the wavefront's planes by 32-bit offsets (a row has up to 8192 x 9 values, an image 2^29)
+    // the filter tile's rows and the wavefront's planes by 32-bit offsets (a row has up to 8192 x 9 values; the planes are an eighth of an
+    // image's, which has fewer than 2^31 values: fewer than 2^30 bytes)
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (int64_t)m0 * g.K), 0, -1, 0x00020000);
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)(x + ((int64_t)bimg * g.C + c0) * g.HW), 0, -1, 0x00020000);
     const int wrow = min(wr, g.F - 1 - m0) * g.K * 4, wlane = wrow + wq0 * 16, wlast = wrow + 8 * 16;

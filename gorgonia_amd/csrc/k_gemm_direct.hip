@@ -1,12 +1,12 @@
 // Matrix products with operands taken from memory straight into the lanes of the 16x16x4 MFMA.
 //
-// A workgroup owns a tile of 16 TM x 16 TN results and its four wavefronts each sum a quarter of K over the whole
-// tile: chunk w, w + 4, ... of KC = 4 KQ consecutive k.  Lane (i, q) holds, of every row of A and column of B it
+// A workgroup owns a tile of 16 TM x 16 TN results and its wavefronts, four or eight (waves_of), each sum their share of K
+// over the whole tile: chunks 2 w and 2 w + 1 of every 8 or 16, of KC = 4 KQ consecutive k.  Lane (i, q) holds, of every row of A and column of B it
 // feeds, the KQ values k0 + KQ q ... - one 16-byte load where k runs along memory - and MFMA step t takes element
 // t of both, so it does not matter that a step's four k are KQ apart.  Where k does not run along memory, a lane
 // takes V = KQ neighbouring rows (columns) per k instead, also 16 bytes, and its V tiles are interleaved: tile e
-// of a group holds every V-th row.  Nothing is staged and no barrier stands in the loop; the loads of a chunk are
-// issued before the MFMAs of the chunk in front of it.  The wavefronts' sums meet in LDS in wavefront order.
+// of a group holds every V-th row.  Nothing is staged and no barrier stands in the loop; the loads of a chunk
+// stand among the MFMAs of the chunk in front of it.  The wavefronts' sums meet in LDS in wavefront order.
 //
 // Against the LDS-tiled kernels: no tile staging to hide with a second workgroup, so one large tile per compute
 // unit runs at the rate of many, any tile height in steps of 16 is to be had, and a product is cut so that its
