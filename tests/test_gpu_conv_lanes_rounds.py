@@ -12,13 +12,19 @@ from tests.test_gpu_conv_lanes import _forward
 pytestmark = pytest.mark.gpu
 
 # B, C, H, W, F and the numbers of compute units that it is planned for: tiles of whole filters and rows and short of one, one
-# quad to a wavefront, several and none; every form (100 x wavefronts + 10 x filter tiles + whether they split the channels)
-BOTH = [(1, 64, 26, 26, 128, range(4, 60, 3)), (2, 24, 22, 24, 40, range(2, 30, 2)), (3, 16, 40, 41, 32, range(2, 40, 3)), (2, 8, 60, 60, 16, range(4, 40, 4))]
-CASES = [(dt, c) for dt in ("f32", "f64") for c in BOTH] + [("f64", (9, 32, 8, 8, 64, range(1, 20))), ("f32", (2, 128, 26, 26, 256, range(20, 150, 8)))]
+# quad to a wavefront, several and none; and the forms that run so (100 x wavefronts + 10 x filter tiles + whether they split the
+# channels) of the convolution, of it pooled and of the image gradient
+CASES = [("f32", (1, 64, 26, 26, 128, range(4, 60, 3)), {811}, {811}, {811, 821}), ("f32", (2, 24, 22, 24, 40, range(2, 30, 2)), (), (), {811}),
+         ("f32", (3, 16, 40, 41, 32, range(2, 40, 3)), (), (), {811}), ("f32", (2, 8, 60, 60, 16, range(4, 40, 4)), (), (), {811}),
+         ("f32", (2, 128, 26, 26, 256, range(20, 150, 8)), {821}, {821}, {811, 821}), ("f32", (2, 96, 30, 30, 96, range(5, 120, 8)), {421}, {421}, {811, 821}),
+         ("f32", (6, 256, 10, 10, 256, range(20, 256, 16)), {421, 811, 821}, {421, 811, 821}, {811, 821}), ("f32", (10, 32, 104, 104, 64, [256]), {410}, {410}, ()),
+         ("f64", (1, 64, 26, 26, 128, range(4, 60, 3)), {411, 420, 421}, (), {411, 421}), ("f64", (2, 24, 22, 24, 40, range(2, 30, 2)), {411}, (), {411, 421}),
+         ("f64", (3, 16, 40, 41, 32, range(2, 40, 3)), {411, 420}, (), {411}), ("f64", (2, 8, 60, 60, 16, range(4, 40, 4)), {411}, (), ()),
+         ("f64", (9, 32, 8, 8, 64, range(1, 20)), {411, 421}, (), {411, 421})]
 
 
-@pytest.mark.parametrize("dt,case", CASES)
-def test_whole_numbers(monkeypatch, dt, case):
+@pytest.mark.parametrize("dt,case,plain,pooled,gradient", CASES)
+def test_whole_numbers(monkeypatch, dt, case, plain, pooled, gradient):
     B, C, H, W, F, units = case
     np_dt, code = (np.float32, _ffi.F32) if dt == "f32" else (np.float64, _ffi.F64)
     rng = np.random.default_rng(C + H + F)
@@ -46,4 +52,4 @@ def test_whole_numbers(monkeypatch, dt, case):
                 ctx.free(out)
             for p in (px, pw, pdy):
                 ctx.free(p)
-    assert forms, 'no launch of several tiles to a workgroup'
+    assert forms == {("conv2d", p, f) for p, fs in ((False, plain), (True, pooled)) for f in fs} | {("conv2d_bwd_data", False, f) for f in gradient}

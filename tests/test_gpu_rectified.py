@@ -42,12 +42,15 @@ def test_product_and_rectify(ctx, dt, M, N, K, form, shift):
     _check(ctx, lambda q: [D.cmd_gemm(q[0], q[1], q[2], M, N, K, dtype=code), D.cmd_relu(q[2], q[3], M * N, dtype=code)], a, b, none, none, form=form, shift=shift)
 
 
-# batch, inputs, outputs: the small-output and the direct kernels as the input gradient's, float64's in eight wavefronts beside four
-@pytest.mark.parametrize("dt,B,I,O", [(np.float32, 128, 625, 10), (np.float32, 128, 1152, 625), (np.float32, 64, 300, 100), (np.float32, 33, 77, 50), (np.float32, 257, 54, 1536),
-                                      (np.float64, 50, 625, 10), (np.float64, 50, 1152, 625), (np.float64, 96, 65, 33), (np.float64, 1448, 96, 200)])
+# batch, inputs, outputs and whether the gradients are one launch: the small-output and the direct kernels as the input gradient's,
+# float64's direct one beside a weight gradient of eight wavefronts; two launches
+@pytest.mark.parametrize("dt,B,I,O,joint", [
+    (np.float32, 128, 625, 10, True), (np.float32, 128, 1152, 625, True), (np.float32, 64, 300, 100, True), (np.float32, 33, 77, 50, True), (np.float32, 257, 54, 1536, True),
+    (np.float64, 50, 625, 10, True), (np.float64, 50, 1152, 625, True), (np.float64, 96, 65, 33, True), (np.float64, 682, 296, 610, True), (np.float64, 1448, 96, 1582, True),
+    (np.float64, 1448, 96, 200, False)])
 @pytest.mark.parametrize("in_place", [False, True])
 @pytest.mark.parametrize("input_first", [False, True])
-def test_gradients_and_rectify_gradient(ctx, dt, B, I, O, in_place, input_first):
+def test_gradients_and_rectify_gradient(ctx, dt, B, I, O, joint, in_place, input_first):
     rng = np.random.default_rng(B + I + O)
     code = _ffi.F64 if dt == np.float64 else _ffi.F32
     x, dy, w, z = (rng.standard_normal(s).astype(dt) for s in ((B, I), (B, O), (I, O), (B, I)))
@@ -61,8 +64,10 @@ def test_gradients_and_rectify_gradient(ctx, dt, B, I, O, in_place, input_first)
     m = _Memory(ctx, x, dy, w, z, dw, dx, dz)
     ctx.run(commands(m.ptr))
     m.all()
-    joint = ctx.joint_launches(_ffi.JOINT_DENSE_GRADIENTS)[0] > before
-    assert joint or dt == np.float64
+    launches, form = ctx.joint_launches(_ffi.JOINT_DENSE_GRADIENTS)
+    assert launches - before == joint
+    if B == 682:
+        assert form == 1008010000   # (as in test_gpu_dense_gradients.py)
     _check(ctx, commands, x, dy, w, z, dw, dx, dz, form=0 if joint else None)
 
 
