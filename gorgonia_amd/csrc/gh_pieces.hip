@@ -12,8 +12,8 @@
 //   * A kernel begins and ends with its caches in order, and that waits for what is under way to and from memory: with 16
 //     workgroups of 1024 threads and 8 loads each, 2 MB under way, a pooling of 4 us took 29.  One load each (128 KB) is as
 //     quick for the bus, and stores that go through to memory leave nothing to be written back.
-// us, whole / in pieces: a detector of eight convolutions, 8 x 3 x 416 x 416 708 / 627, five images 509 / 474, two 231 / 224,
-// 8 x 3 x 320 x 320 449 / 416, five of them 310 / 301, 8 x 3 x 224 x 224 250 / 243.
+// us, whole / in pieces: a detector of eight convolutions, 8 x 3 x 416 x 416 695 / 619, five images 510 / 474, two 233 / 225,
+// 8 x 3 x 320 x 320 450 / 410, five of them 311 / 299, 8 x 3 x 224 x 224 251 / 240.
 //
 // Nothing waits for a workgroup that has not begun: a part of a piece is copied by whoever claims it first, the copy's
 // workgroup or, after some time of the device's clock, the kernel that waits for it (where something runs the streams one after
@@ -23,6 +23,8 @@
 // close to each other the context's batches go whole.
 #include <algorithm>
 #include <cstdlib>
+#include <cstring>
+#include <mutex>
 
 #include "gh_internal.h"
 
@@ -34,7 +36,7 @@ constexpr int64_t kBegin = 20000;                     // ticks of 10 ns for a wo
 constexpr int64_t kGiveUp = 400000;                   // and to claim a part, and one more for 100 bytes (GORGONIA_HIP_PIECES_TICKS: fewer of both)
 constexpr int kMisses = 3, kWithin = 64;              // uploads that were given up, and how many may lie between two of them
 constexpr int64_t kLeast = GH_PIECES_FROM, kMost = 1 << 30;  // bytes of an upload (the least: two images of 3 x 416 x 416 gain 3 %)
-constexpr int64_t kPieceBytes = 4 << 20;              // (8 x 3 x 416 x 416 in two, three, four and eight: 658, 637, 627 and 674 us)
+constexpr int64_t kPieceBytes = 4 << 20;              // (8 x 3 x 416 x 416 in two, three, four and eight: 637, 635, 618 and 700 us)
 constexpr int kHead = 12;
 constexpr int kTries = 6;
 constexpr int64_t kTryFor = 30000;                    // ticks of 10 ns
@@ -153,8 +155,45 @@ bool by_image(const gh_cmd& c, Layer* l) {
   return false;
 }
 
+// Whether the kernels take a valid command's shape with `fewest` and with `most` of its images, too, and add there as they do for
+// the whole batch.  Asking them all takes 5 to 10 us of host time a layer, in front of a copy of 70 and more; the answers are a
+// function of the shape (and of the switches that take kernels out) and are kept, one for each of kKept places.
+// us of host time for a detector's front, asked / kept: 8 x 3 x 416 x 416 21 / 3, 8 x 3 x 320 x 320 40 / 3.
+constexpr int kKept = 64;
+bool runs_in_pieces(const gh_cmd& c, int64_t fewest, int64_t most, int units) {
+  struct Shape { int64_t dim[16]; int64_t fewest, most, code, units; };
+  struct Place { Shape shape; bool known, fits; };
+  static std::mutex mu;
+  static Place places[kKept] = {};
+  Shape s;
+  memcpy(s.dim, c.dim, sizeof s.dim);
+  s.fewest = fewest;
+  s.most = most;
+  s.code = (int64_t)c.opcode << 32 | c.flags;
+  s.units = (int64_t)units << 2 | (getenv("GORGONIA_HIP_CONV_NO_LANES") ? 2 : 0) | (getenv("GORGONIA_HIP_CONV_NO_STRIP") ? 1 : 0);
+  uint64_t h = 0;
+  for (size_t i = 0; i < sizeof s / 8; i++) h = (h ^ (uint64_t)((const int64_t*)&s)[i]) * 0x9E3779B97F4A7C15ull;
+  Place& p = places[h >> 32 & (kKept - 1)];
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (p.known && memcmp(&p.shape, &s, sizeof s) == 0) return p.fits;
+  }
+  std::string m;
+  bool fits = true;
+  for (int64_t images : {fewest, most}) {
+    gh_cmd part = c;
+    part.dim[0] = images;
+    fits = fits && gh_validate_cmd(part, m) == GH_OK;
+    if (c.opcode == GH_OP_CONV2D)
+      for (int u : {units, units_beside(units)}) fits = fits && gh_conv2d_in_pieces(c, images, units, u);
+  }
+  std::lock_guard<std::mutex> lock(mu);
+  p = Place{s, true, fits};
+  return fits;
+}
+
 // The layers behind the upload that run in pieces: as many as take, whole, about half of the upload's time (8 x 3 x 416 x 416:
-// three layers 645 us, with the fourth and its pooling 632), each reads what the one in front wrote, image by image, and the kernels take their shapes
+// three layers 628 us, with the fourth and its pooling 619), each reads what the one in front wrote, image by image, and the kernels take their shapes
 // with a piece's images, too, and add there as they do for the whole batch: whether a batch goes in pieces (eagerly) or whole (under
 // capture) changes no bits.  A layer's work on the first piece comes before the work of those in front of it on the last: what it
 // writes lies apart from all that they read and write, their filters and constants among it.
@@ -185,14 +224,7 @@ int head_of(const gh_cmd* cmds, int n, int64_t fewest, int64_t most, Layer* laye
     for (int k = 0; k <= head; k++) fits = fits && !meet(values[k], values[head + 1]);
     for (int k = 0; k < held; k++)
       for (int s = 0; s <= head + 1; s++) fits = fits && !meet(values[s], constants[k]);
-    for (int64_t images : {fewest, most}) {
-      gh_cmd part = c;
-      part.dim[0] = images;
-      fits = fits && gh_validate_cmd(part, m) == GH_OK;
-      if (c.opcode == GH_OP_CONV2D)
-        for (int u : {units, units_beside(units)}) fits = fits && gh_conv2d_in_pieces(c, images, units, u);
-    }
-    if (!fits) break;
+    if (!fits || !runs_in_pieces(c, fewest, most, units)) break;
   }
   return head;
 }

@@ -111,3 +111,19 @@ def test_a_lent_batch_keeps_what_its_layers_read():
 def test_a_batch_bound_with_let_keeps_nothing():
     """It never runs in pieces: every value goes with its reader."""
     assert _program(False) == [["w", "x"], ["0"], ["1"]]
+
+
+def test_the_same_answer_when_asked_again(monkeypatch):
+    """More shapes than are kept, each asked at different times and with kernels taken out of the choice."""
+    def ask(c, f, h, b, pool2):
+        y = _at(2)
+        cmds = [D.cmd_copy(_at(0), _at(9), 4 * b * c * h * h), D.cmd_conv2d(_at(0), _at(1), y, b, c, h, h, f, 3, 3, (1, 1), pool2=pool2, act="relu")]
+        return _layers(cmds)
+    shapes = [(c, f, h, -(-4200000 // (4 * c * h * h)) + more, p) for c in (3, 16, 32, 64, 588) for f in (16, 64) for h in (52, 104) for more in (2, 5) for p in (False, True)]
+    first = [ask(*s) for s in shapes]
+    assert len(shapes) > 64 and set(first) == {0, 1}
+    with monkeypatch.context() as p:
+        p.setenv("GORGONIA_HIP_CONV_NO_LANES", "1")
+        without = [ask(*s) for s in shapes]
+    assert without != first
+    assert [ask(*s) for s in shapes] == first and [ask(*s) for s in shapes[::-1]] == first[::-1]
