@@ -157,7 +157,8 @@ bool by_image(const gh_cmd& c, Layer* l) {
 
 // Whether the kernels take a valid command's shape with `fewest` and with `most` of its images, too, and add there as they do for
 // the whole batch.  Asking them all takes 5 to 10 us of host time a layer, in front of a copy of 70 and more; the answers are a
-// function of the shape (and of the switches that take kernels out) and are kept, one for each of kKept places.
+// function of the shape and are kept, one for each of kKept places.  (Tuning switches in the environment: the two named here are asked
+// each time, the others when a shape is first seen.)
 // us of host time for a detector's front, asked / kept: 8 x 3 x 416 x 416 21 / 3, 8 x 3 x 320 x 320 40 / 3.
 constexpr int kKept = 64;
 bool runs_in_pieces(const gh_cmd& c, int64_t fewest, int64_t most, int units) {

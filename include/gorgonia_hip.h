@@ -303,7 +303,9 @@ GH_API int gh_memcpy_staged(gh_ctx* ctx, gh_devptr dst, void* stage, const void*
  * that run in one launch have the bits of the commands one by one, but for a
  * BN_BWD right behind the MAXPOOL2D_BWD whose result it takes: its two sums are
  * added in another order than when it is submitted apart (or in a context
- * beyond a device's 64th), so that the gradient's last bits are others. */
+ * beyond a device's 64th), so that the gradient's last bits are others.  A context's
+ * first submission whose batch goes in pieces (gh_pieces_layers) waits for what is
+ * on its stream. */
 GH_API int gh_submit(gh_ctx* ctx, const gh_cmd* cmds, int n);
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory around a submit - code under HIP graph capture, tight serving loops,
