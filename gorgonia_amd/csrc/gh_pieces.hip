@@ -157,12 +157,18 @@ bool by_image(const gh_cmd& c, Layer* l) {
 
 // Whether the kernels take a valid command's shape with `fewest` and with `most` of its images, too, and add there as they do for
 // the whole batch.  Asking them all takes 5 to 10 us of host time a layer, in front of a copy of 70 and more; the answers are a
-// function of the shape and are kept, one for each of kKept places.  (Tuning switches in the environment: the two named here are asked
-// each time, the others when a shape is first seen.)
+// function of the shape, of the alignment that kernels ask for (k_conv1x1: whole lines of filters) and of the switches that take
+// kernels out, and are kept, one for each of kKept places.  (Other tuning switches are read when a shape is first seen, as for plans.)
 // us of host time for a detector's front, asked / kept: 8 x 3 x 416 x 416 21 / 3, 8 x 3 x 320 x 320 40 / 3.
 constexpr int kKept = 64;
-bool runs_in_pieces(const gh_cmd& c, int64_t fewest, int64_t most, int units) {
-  struct Shape { int64_t dim[16]; int64_t fewest, most, code, units; };
+int64_t switches() {
+  int64_t set = 0;
+  for (const char* name : {"GORGONIA_HIP_CONV_NO_LANES", "GORGONIA_HIP_CONV_NO_STRIP", "GORGONIA_HIP_CONV_NO_DIRECT", "GORGONIA_HIP_CONV_NO_ROWS1", "GORGONIA_HIP_CONV_NO_POINTWISE"})
+    set = set << 1 | (getenv(name) != nullptr);
+  return set;
+}
+bool runs_in_pieces(const gh_cmd& c, int64_t fewest, int64_t most, int units, int64_t set) {
+  struct Shape { int64_t dim[16]; int64_t fewest, most, code, units, aligned; };
   struct Place { Shape shape; bool known, fits; };
   static std::mutex mu;
   static Place places[kKept] = {};
@@ -171,7 +177,8 @@ bool runs_in_pieces(const gh_cmd& c, int64_t fewest, int64_t most, int units) {
   s.fewest = fewest;
   s.most = most;
   s.code = (int64_t)c.opcode << 32 | c.flags;
-  s.units = (int64_t)units << 2 | (getenv("GORGONIA_HIP_CONV_NO_LANES") ? 2 : 0) | (getenv("GORGONIA_HIP_CONV_NO_STRIP") ? 1 : 0);
+  s.units = (int64_t)units << 8 | set;
+  s.aligned = (int64_t)(c.ptr[1] & 15) << 2 | (int64_t)((c.ptr[0] | c.ptr[1] | c.ptr[2]) & 3);
   uint64_t h = 0;
   for (size_t i = 0; i < sizeof s / 8; i++) h = (h ^ (uint64_t)((const int64_t*)&s)[i]) * 0x9E3779B97F4A7C15ull;
   Place& p = places[h >> 32 & (kKept - 1)];
@@ -207,6 +214,7 @@ int head_of(const gh_cmd* cmds, int n, int64_t fewest, int64_t most, Layer* laye
   uint64_t from = up.ptr[0];
   values[0] = Span{from, from + (uint64_t)up.dim[0]};
   double us = 0;
+  const int64_t set = switches();
   int head = 0, held = 0;
   for (; head < kHead && head + 1 < n; head++) {
     const gh_cmd& c = cmds[head + 1];
@@ -225,7 +233,7 @@ int head_of(const gh_cmd* cmds, int n, int64_t fewest, int64_t most, Layer* laye
     for (int k = 0; k <= head; k++) fits = fits && !meet(values[k], values[head + 1]);
     for (int k = 0; k < held; k++)
       for (int s = 0; s <= head + 1; s++) fits = fits && !meet(values[s], constants[k]);
-    if (!fits || !runs_in_pieces(c, fewest, most, units)) break;
+    if (!fits || !runs_in_pieces(c, fewest, most, units, set)) break;
   }
   return head;
 }

@@ -127,3 +127,23 @@ def test_the_same_answer_when_asked_again(monkeypatch):
         without = [ask(*s) for s in shapes]
     assert without != first
     assert [ask(*s) for s in shapes] == first and [ask(*s) for s in shapes[::-1]] == first[::-1]
+
+
+def test_the_answer_for_another_alignment():
+    """A 1x1 convolution runs on k_conv1x1 where its filters lie at whole lines, else on a kernel that cuts the channels by the images."""
+    def ask(w):
+        return _layers([D.cmd_copy(_at(0), _at(9), 4 * 8 * 256 * 28 * 28), D.cmd_conv2d(_at(0), w, _at(2), 8, 256, 28, 28, 64, 1, 1)])
+    assert [ask(_at(1) + off) for off in (0, 4, 8, 16, 4)] == [1, 0, 0, 1, 0]
+
+
+@pytest.mark.parametrize("switch,conv", [("POINTWISE", (8, 256, 28, 28, 64, 1, 1)), ("DIRECT", (1024, 2, 32, 32, 16, 3, 3, (1, 1)))])
+def test_the_answer_with_a_kernel_taken_out(monkeypatch, switch, conv):
+    """The next kernel's cuts the channels by the images; asked before and behind."""
+    def ask():
+        bytes_ = 4 * conv[0] * conv[1] * conv[2] * conv[3]
+        return _layers([D.cmd_copy(_at(0), _at(9), bytes_), D.cmd_conv2d(_at(0), _at(1), _at(2), *conv)])
+    assert ask() == 1
+    with monkeypatch.context() as p:
+        p.setenv("GORGONIA_HIP_CONV_NO_" + switch, "1")
+        assert ask() == 0
+    assert ask() == 1
